@@ -4,10 +4,10 @@
 // decomposition.
 //
 // Column-sliced schedule, for graphs with long windows:
-//   * the column range is cut into S = 8 * P slices and XCD x only ever works on slices x, x + 8,
-//     x + 16, ..., one after the other. The K/V rows of a slice mostly stay in the XCD's 4 MiB L2,
-//     so a row is fetched from the memory side about once per XCD instead of once per window
-//     that names it;
+//   * the column range is cut into slices and an XCD only ever works on one slice (of some of the
+//     heads, for some of the windows: XcdSplit) at a time. The K/V rows of a slice mostly stay in
+//     the XCD's 4 MiB L2, so a row is fetched from the memory side about once per XCD instead of
+//     once per window that names it;
 //   * a wave computes one (window, slice[, head]) unit: the window's TC blocks whose first column
 //     falls into the slice, with (m, l, O) in registers, and writes the unit's partial result to
 //     scratch. A second kernel merges a window's partials (log-sum-exp) and writes its rows;
@@ -37,21 +37,26 @@ using pipe::uniform;
 constexpr int kXcds = 8;
 constexpr int kMaxPhases = 16;
 constexpr int kUnitWaves = 4;  // waves (= units) per workgroup; they do not cooperate
-// the same for the wave-per-window launches of graphs with short windows (measured on the 100k-node
-// 8-head layers: 0.093 / 0.171 ms with two, 0.099 / 0.175 ms with four, 0.121 / 0.197 ms with one)
-constexpr int kShortUnitWaves = 2;
 
-// Partial result of a unit: D/4 + 2 dwords per lane, stored register by register so that every
-// store and load is one coalesced 256-byte row: [o[0][0..3], ..., o[T-1][0..3], m, l][64 lanes].
-// Lane (g, c) holds O[q = c][16j + 4g + i] in o[j][i].
-template <int D>
-constexpr int partial_dwords() {
-  return (D / 4 + 2) * 64;
+// Stages of a wave's LDS ring and waves per SIMD the register allocator is held to.
+// Column-sliced units are runs of dozens of blocks: two stages, as many waves as the rings allow
+// (four workgroups of four waves per CU at D = 32, two up to D = 128, one above). Short windows are
+// two to eight steps, so most of a wave's time is the chain order -> block range -> ids -> rows in
+// front of the first step: one stage, and up to D = 64 the LDS that frees goes to more waves
+// (100k-node 8 x 32 layer 130 -> 112 us, 60k-node 4 x 64 layer 69 -> 51 us, both together with the
+// whole-line stores and the XCD chunks below).
+constexpr int unit_stages(int d, bool sliced) { return sliced && d <= 64 ? 2 : 1; }
+constexpr int unit_waves_per_simd(int d, bool sliced) {
+  return d <= 32 ? (sliced ? 4 : 5) : d <= 64 ? (sliced ? 2 : 4) : d <= 128 ? 2 : 1;
 }
 
-// waves per SIMD the register allocator is held to; the LDS rings allow four workgroups of four
-// waves per CU at D = 32, two up to D = 128 and one above
-constexpr int unit_waves_per_simd(int d) { return d <= 32 ? 4 : d <= 128 ? 2 : 1; }
+// Partial result of a unit: the O^T tiles as the lanes hold them, one coalesced 1 KiB row of 16
+// bytes per lane and tile (lane (g, c) holds O[q = c][16j + 4g + i] in o[j][i]), then m[16] and
+// l[16].
+template <int D>
+constexpr int partial_floats() {
+  return 16 * D + 32;
+}
 
 template <typename ET, int D, bool HEADS>
 __device__ __forceinline__ pipe::Problem<ET> make_problem(const int32_t* sparseAToXidx,
@@ -74,6 +79,56 @@ __device__ __forceinline__ pipe::Problem<ET> make_problem(const int32_t* sparseA
   return pb;
 }
 
+// How the units of a call are dealt to the XCDs. XCD x works on one column slice of one group of
+// heads at a time, for its share of the order's positions:
+//   x = sg + sliceGroups * (hg + headGroups * wg), slice = phase * sliceGroups + sg,
+//   heads hg * headsPerGroup .. + headsPerGroup - 1,
+//   positions [wg * chunk, (wg + 1) * chunk) of every run of windowGroups * chunk positions.
+struct Unit {
+  int pos, head, slice;
+};
+struct XcdSplit {
+  int phases;         // slices an XCD works through, one after the other
+  int sliceGroups;    // slices in work at a time; sliceGroups * headGroups * windowGroups == 8
+  int headGroups;
+  int windowGroups;
+  int headsPerGroup;
+  int chunk;
+  __host__ __device__ int slices() const { return phases * sliceGroups; }
+  // units of one XCD and phase
+  __host__ __device__ int64_t units(int nRW) const {
+    const int64_t run = (int64_t)windowGroups * chunk;
+    return ((int64_t)nRW + run - 1) / run * chunk * headsPerGroup;
+  }
+  // u-th unit of the XCD in the phase: heads innermost (they share ids, bitmaps and lines)
+  __device__ __forceinline__ Unit unit(int xcd, int phase, unsigned u) const {
+    const int sg = xcd & (sliceGroups - 1);  // the group counts are powers of two
+    const int rest = xcd / sliceGroups;
+    const int hg = rest & (headGroups - 1);
+    const int wg = rest / headGroups;
+    const unsigned p = u / (unsigned)headsPerGroup;
+    const unsigned run = p / (unsigned)chunk;
+    Unit r;
+    r.pos = (int)((run * windowGroups + wg) * chunk + (p - run * chunk));
+    r.head = hg * headsPerGroup + (int)(u - p * headsPerGroup);
+    r.slice = phase * sliceGroups + sg;
+    return r;
+  }
+};
+
+// Head groups come first: an XCD that works on some of the heads gathers only their part of the
+// rows, so its share of K + V shrinks without cutting windows into more units. The part stays at
+// least a line of 128 bytes.
+inline XcdSplit split_heads(int d, int heads) {
+  XcdSplit s = {1, 1, 1, kXcds, heads, 1};
+  while (s.headGroups < kXcds && s.headsPerGroup % 2 == 0 && s.headsPerGroup / 2 * d * 2 >= 128) {
+    s.headGroups *= 2;
+    s.windowGroups /= 2;
+    s.headsPerGroup /= 2;
+  }
+  return s;
+}
+
 // probe builds: the partials through the caches instead of past them
 #ifdef F3S_PROBE_PARTIAL_CACHED_STORE
 #define F3S_PARTIAL_STORE(v, p) (*(p) = (v))
@@ -88,12 +143,40 @@ __device__ __forceinline__ pipe::Problem<ET> make_problem(const int32_t* sparseA
 
 template <int D, typename PipeT>
 __device__ __forceinline__ void store_partial(const PipeT& pp, float* __restrict__ dst) {
+  const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int jj = 0; jj < D / 16; jj++)
+    F3S_PARTIAL_STORE(pp.o[jj], reinterpret_cast<float4v*>(dst) + jj * 64 + lane);
+  const float l = pipe::row_sum4(pp.l);  // m is the same in the four lanes of a row already
+  if (lane < 32) F3S_PARTIAL_STORE(lane < 16 ? pp.m : l, dst + 16 * D + lane);
+}
+
+// A window's 16 rows of D floats from the lanes' O^T tiles (already normalised) to memory, through
+// `lds` of the wave (rows_lds_floats<D>() floats): stored as the lanes hold them, a row would leave
+// in pieces of 64 bytes; this way a store instruction fills whole lines.
+template <int D>
+constexpr int rows_lds_floats() {
+  return 16 * (D + 4);
+}
+template <int D>
+__device__ __forceinline__ void store_rows(const float4v (&o)[D / 16], float* lds, int w, int N,
+                                           float* __restrict__ out, int ldOut) {
+  constexpr int LPR = D / 4;  // lanes per row, 16 bytes each
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, c = lane & 15;
 #pragma unroll
-    for (int i = 0; i < 4; i++) F3S_PARTIAL_STORE(pp.o[jj][i], dst + (jj * 4 + i) * 64);
-  F3S_PARTIAL_STORE(pp.m, dst + (D / 4) * 64);
-  F3S_PARTIAL_STORE(pp.l, dst + (D / 4 + 1) * 64);
+  for (int j = 0; j < D / 16; j++)
+    *reinterpret_cast<float4v*>(lds + c * (D + 4) + 16 * j + 4 * g) = o[j];
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int k = 0; k < 16 * LPR / 64; k++) {
+    const int q = (k * 64 + lane) / LPR, cv = (k * 64 + lane) % LPR;
+    const int64_t row = (int64_t)w * 16 + q;
+    if (row < N)
+      store_out(out + row * ldOut + cv * 4,
+                *reinterpret_cast<const float4v*>(lds + q * (D + 4) + cv * 4));
+  }
 }
 
 // One wave per unit, kUnitWaves independent units per workgroup. A unit is
@@ -102,59 +185,52 @@ __device__ __forceinline__ void store_partial(const PipeT& pp, float* __restrict
 //            units of the order); unit = position * nHeads + head; slice = phase * 8 + XCD.
 //   !SLICED: one whole window (of one head, if HEADS); the result is the window's output rows.
 //            Windows of more than maxBlocks TC blocks among the first longPrefix positions of
-//            the order are left to f3s_fwd_kernel, whose four waves share a window and whose
-//            grid covers exactly those positions (with a heavy-first order no long window lies
-//            beyond them; with any other order such a window is simply computed here). Unit u =
-//            position * nHeads + head, so the waves of a workgroup mostly work on the heads of
-//            one window and share its column ids and bitmaps.
+//            the order are left to f3s_fwd_kernel, whose waves share a window and whose grid looks
+//            through exactly those positions (with a heavy-first order no long window lies beyond
+//            them; with any other order such a window is simply computed here). XcdSplit deals
+//            head groups and chunks of the order to the XCDs.
 template <typename ET, int D, bool SOFTMAX, bool SLICED, bool HEADS>
 __global__ __launch_bounds__(kUnitWaves * 64)
-__attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D), unit_waves_per_simd(D)))) void
+__attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D, SLICED),
+                                   unit_waves_per_simd(D, SLICED)))) void
 f3s_fwd_unit_kernel(const int32_t* __restrict__ windowOrder,
                     const int32_t* __restrict__ rowWindowOffset,
                     const int32_t* __restrict__ sparseAToXidx,
                     const uint8_t* __restrict__ bitmapBytes,
-                    const int32_t* __restrict__ sliceStart, int S, int nGroups, int N, int nRW,
-                    int64_t nTcb, const ET* __restrict__ Q, const ET* __restrict__ K,
+                    const int32_t* __restrict__ sliceStart, XcdSplit split, int nGroups, int N,
+                    int nRW, int64_t nTcb, const ET* __restrict__ Q, const ET* __restrict__ K,
                     const ET* __restrict__ V, float scaleLog2, float* __restrict__ partial,
                     float* __restrict__ out, int nHeads, int ldIn, int ldOut, int maxBlocks,
                     int longPrefix, int ldQ) {
-  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false> Pipe;
+  constexpr int STAGES = unit_stages(D, SLICED);
+  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false, STAGES> Pipe;
   constexpr int T = D / 16;
   extern __shared__ __align__(1024) unsigned char smem[];
 
-  const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
-  const int g = lane >> 4;
-  const int c = lane & 15;
 
-  int w, t0, t1, slice = 0, head = 0;
-  if constexpr (SLICED) {
-    const int xcd = blockIdx.x % kXcds;
-    const int j = blockIdx.x / kXcds;
-    const int phase = j / nGroups;
+  // Workgroup b runs on XCD b % 8; its waves take consecutive units of that XCD's list.
+  const int j = blockIdx.x / kXcds;
+  const int phase = j / nGroups;  // 0 if not SLICED
 #ifdef F3S_PROBE_SAME_UNIT
-    // probe: the four waves of a workgroup all compute its first unit, at the same time
-    const int64_t u = (int64_t)(j - phase * nGroups) * (int)(blockDim.x >> 6);
+  // probe: the four waves of a workgroup all compute its first unit, at the same time
+  const unsigned u = (unsigned)(j - phase * nGroups) * kUnitWaves;
 #else
-    const int64_t u = (int64_t)(j - phase * nGroups) * (int)(blockDim.x >> 6) + wave;
+  const unsigned u = (unsigned)(j - phase * nGroups) * kUnitWaves + wave;
 #endif
-    const int pos = HEADS ? (int)(u / nHeads) : (int)u;
-    head = HEADS ? (int)(u - (int64_t)pos * nHeads) : 0;
-    if (pos >= nRW) return;
-    slice = phase * kXcds + xcd;
-    w = uniform(windowOrder ? windowOrder[pos] : pos);
-    if ((unsigned)w >= (unsigned)nRW) return;  // a corrupt order entry must not index out of range
-    t0 = uniform(sliceStart[(int64_t)w * (S + 1) + slice]);
-    t1 = uniform(sliceStart[(int64_t)w * (S + 1) + slice + 1]);
+  const Unit un = split.unit(blockIdx.x % kXcds, phase, u);
+  const int pos = un.pos;
+  const int head = HEADS ? un.head : 0;
+  if (pos >= nRW) return;
+  const int w = uniform(windowOrder ? windowOrder[pos] : pos);
+  if ((unsigned)w >= (unsigned)nRW) return;  // a corrupt order entry must not index out of range
+  int t0, t1;
+  if constexpr (SLICED) {
+    const int64_t at = (int64_t)w * (split.slices() + 1) + un.slice;
+    t0 = uniform(sliceStart[at]);
+    t1 = uniform(sliceStart[at + 1]);
     if (t1 <= t0) return;  // empty unit: nothing is written, the merge skips it
   } else {
-    const int64_t u = (int64_t)blockIdx.x * (int)(blockDim.x >> 6) + wave;
-    const int pos = HEADS ? (int)(u / nHeads) : (int)u;
-    head = HEADS ? (int)(u - (int64_t)pos * nHeads) : 0;
-    if (pos >= nRW) return;
-    w = uniform(windowOrder ? windowOrder[pos] : pos);
-    if ((unsigned)w >= (unsigned)nRW) return;
     t0 = uniform(rowWindowOffset[w]);
     t1 = uniform(rowWindowOffset[w + 1]);
     if (t1 - t0 > maxBlocks && pos < longPrefix) return;  // f3s_fwd_kernel's
@@ -166,29 +242,27 @@ f3s_fwd_unit_kernel(const int32_t* __restrict__ windowOrder,
   const pipe::Problem<ET> pb = make_problem<ET, D, HEADS>(sparseAToXidx, bitmapBytes, Q, K, V, N,
                                                           scaleLog2, ldIn, nTcb, ldQ);
   const unsigned ringAddr =
-      (unsigned)(uintptr_t)(F3S_LDS unsigned char*)smem + (unsigned)wave * pipe::Geo<D>::WAVE_BYTES;
+      (unsigned)(uintptr_t)(F3S_LDS unsigned char*)smem + (unsigned)wave * pipe::Geo<D, STAGES>::WAVE_BYTES;
   Pipe pp;
   pp.init(pb, w, ringAddr, head);
   pp.run(pb, t0, t1);
 
   if constexpr (SLICED) {
     const int64_t wh = (int64_t)w * (HEADS ? nHeads : 1) + head;
-    store_partial<D>(pp, partial + (wh * S + slice) * partial_dwords<D>() + lane);
+    store_partial<D>(pp, partial + (wh * split.slices() + un.slice) * partial_floats<D>());
   } else {
     float inv = 1.0f;
     if constexpr (SOFTMAX) {
       const float lAll = pipe::row_sum4(pp.l);
       inv = (lAll == 0.0f) ? 0.0f : 1.0f / lAll;
     }
-    const int64_t row = (int64_t)w * 16 + c;
-    if (row < N) {
-      float* dst = out + row * (HEADS ? ldOut : D) + head * D + 4 * g;
 #pragma unroll
-      for (int jj = 0; jj < T; jj++) {
-        const float4v v = pp.o[jj] * inv;
-        *reinterpret_cast<float4v*>(dst + 16 * jj) = v;
-      }
-    }
+    for (int jj = 0; jj < T; jj++) pp.o[jj] *= inv;
+    // the wave's ring is free now
+    static_assert(rows_lds_floats<D>() * 4 <= pipe::Geo<D, STAGES>::WAVE_BYTES, "rows fit the ring");
+    store_rows<D>(pp.o,
+                  reinterpret_cast<float*>(smem + (unsigned)wave * pipe::Geo<D, STAGES>::WAVE_BYTES),
+                  w, N, out + (HEADS ? head * D : 0), HEADS ? ldOut : D);
   }
 }
 
@@ -207,17 +281,45 @@ struct SlicedHeader {
 };
 constexpr uint32_t kSlicedMagic = 0xF35C0DE5u;
 
+// Rows of 128 bytes gathered from addresses that are multiples of 256 are served faster than rows
+// from the odd 128-byte lines in between (233k-node graph, d = 64: 1.42 ms with every row on an
+// even line, 1.55 ms with every row on an odd line, 1.48 ms for contiguous rows, which alternate;
+// the L2 hit and miss counts are the same in all three). The single-head call at d = 64 therefore
+// gathers from copies of K and V with a row pitch of 256 bytes, made at the start of the call.
+constexpr int kPaddedRowBytes = 256;
+typedef int pad_chunk __attribute__((ext_vector_type(4)));
+
 // sliceStart[w * (S + 1) + s] = first TC block of window w whose first (smallest) column id is
-// >= s * sliceWidth; entry S is the window's end. One thread per entry, binary search over the
-// window's blocks (their first columns ascend). A block range that does not fit the structure
-// (a mismatched rowWindowOffset) makes the window empty: every entry 0.
+// >= s * sliceWidth; entry S is the window's end. 16 lanes per window look at 16 evenly spaced
+// blocks together, then each finishes one boundary by binary search between two of them (their first
+// columns ascend). Bound by memory: what is left after the first look costs a line or two per step
+// and boundary, 100 MB at 233k nodes. Boundaries interpolated instead of searched read a third of
+// that, but the twentieth of the blocks they leave in the wrong slice slows the unit kernel down by
+// 5 to 14 %. A block range that does not fit the structure (a mismatched rowWindowOffset) makes the
+// window empty: every entry 0.
 // mode 0: part of an attention call, index rebuilt; mode 1: f3s_attention_prepare (index built,
 // header written); mode 2: part of an attention call whose caller says the workspace is prepared:
 // the index is kept if the header confirms it and rebuilt otherwise.
+// Workgroups from setupBlocks on copy K and V instead (if the call wants the copies): the searches
+// are short chains of loads, the copy is bound by memory, and one launch saves the gap of two
+// (233k nodes: 16 + 21 us and the gap apart, 34 us together).
 __global__ __launch_bounds__(256) void sliced_setup_kernel(
     const int32_t* __restrict__ rowWindowOffset, const int32_t* __restrict__ sparseAToXidx, int N,
     int nRW, int S, int sliceWidth, int64_t nTcb, SlicedHeader* __restrict__ hdr, int mode,
-    int32_t* __restrict__ tickets, int32_t* __restrict__ sliceStart) {
+    int32_t* __restrict__ tickets, int32_t* __restrict__ sliceStart, int setupBlocks,
+    const pad_chunk* __restrict__ K, const pad_chunk* __restrict__ V, int64_t chunks,
+    pad_chunk* __restrict__ Kp, pad_chunk* __restrict__ Vp) {
+  if ((int)blockIdx.x >= setupBlocks) {
+    // K and V rows of 128 bytes to a pitch of 256 bytes (one thread per 16 bytes of each)
+    const int64_t i = (int64_t)((int)blockIdx.x - setupBlocks) * blockDim.x + threadIdx.x;
+    if (i >= chunks) return;
+    const int64_t at = (i >> 3) * (kPaddedRowBytes / 16) + (i & 7);
+    const pad_chunk k = __builtin_nontemporal_load(K + i);  // read once, by nobody else
+    const pad_chunk v = __builtin_nontemporal_load(V + i);
+    Kp[at] = k;
+    Vp[at] = v;
+    return;
+  }
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx < kXcds) tickets[idx] = 0;
   if (mode == 2) {
@@ -239,24 +341,37 @@ __global__ __launch_bounds__(256) void sliced_setup_kernel(
       hdr->prepared = 0;  // the index no longer belongs to an earlier f3s_attention_prepare
     }
   }
-  const int per = S + 1;
-  if (idx >= (int64_t)nRW * per) return;
-  const int w = (int)(idx / per), b = (int)(idx % per);
-  int lo = rowWindowOffset[w], hi = rowWindowOffset[w + 1];
-  if (lo < 0 || (int64_t)hi > nTcb || hi < lo) lo = hi = 0;
-  if (b == S) {
-    sliceStart[idx] = hi;
-    return;
+  const int sub = threadIdx.x & 15;
+  const int w = (int)(idx >> 4);
+  int first = 0, end = 0;
+  if (w < nRW) {
+    first = rowWindowOffset[w];
+    end = rowWindowOffset[w + 1];
+    if (first < 0 || (int64_t)end > nTcb || end < first) first = end = 0;
   }
-  const int64_t limit = (int64_t)b * sliceWidth;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (sparseAToXidx[(int64_t)mid * 16] < limit)
-      lo = mid + 1;
-    else
-      hi = mid;
+  const int n = end - first;
+  const int probe = first + (int)((int64_t)sub * n / 16);
+  const int seen = n > 0 ? sparseAToXidx[(int64_t)probe * 16] : 0;
+  int32_t* dst = sliceStart + (int64_t)w * (S + 1);
+  for (int b0 = 0; b0 < S; b0 += 16) {
+    const int64_t limit = (int64_t)(b0 + sub) * sliceWidth;
+    int below = 0;  // of the window's probes in front of this lane's boundary
+#pragma unroll
+    for (int k = 0; k < 16; k++) below += (__shfl(seen, k, 16) < limit) ? 1 : 0;
+    const int left = below > 0 ? below - 1 : 0;
+    // the boundary is the first block of (lo, hi) at or beyond `limit`, or hi
+    int lo = first + (int)((int64_t)left * n / 16) + 1;
+    int hi = first + (int)((int64_t)below * n / 16);
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (sparseAToXidx[(int64_t)mid * 16] < limit)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    if (w < nRW && b0 + sub < S) dst[b0 + sub] = hi;
   }
-  sliceStart[idx] = lo;
+  if (w < nRW && sub == 0) dst[S] = end;
 }
 
 // The resident form: as many workgroups as the GPU holds at once, NW independent waves each.
@@ -278,15 +393,16 @@ __global__ __launch_bounds__(256) void sliced_setup_kernel(
 // for the stores and the returning atomic sit on every unit's path.
 template <typename ET, int D, bool SOFTMAX, bool HEADS, int NW>
 __global__ __launch_bounds__(NW * 64)
-__attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D), unit_waves_per_simd(D)))) void
+__attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D, true),
+                                   unit_waves_per_simd(D, true)))) void
 f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
-                        const int32_t* __restrict__ sliceStart, int P, int nRW, int S, int N,
+                        const int32_t* __restrict__ sliceStart, XcdSplit split, int nRW, int N,
                         int64_t nTcb, int32_t* __restrict__ tickets,
                         const int32_t* __restrict__ sparseAToXidx,
                         const uint8_t* __restrict__ bitmapBytes, const ET* __restrict__ Q,
                         const ET* __restrict__ K, const ET* __restrict__ V, float scaleLog2,
                         float* __restrict__ partial, int nHeads, int ldIn) {
-  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false> Pipe;
+  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false, unit_stages(D, true)> Pipe;
   extern __shared__ __align__(1024) unsigned char smem[];
   __shared__ int sCtl[2];  // slot of this workgroup; next unit of its sequence
 
@@ -312,12 +428,14 @@ f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
   const int x = slot / per;
   const int r = slot - x * per;
   const int heads = HEADS ? nHeads : 1;
-  const int64_t units = (int64_t)P * nRW * heads;  // units of one XCD
+  const int S = split.slices();
+  const int64_t perPhase = split.units(nRW);
+  const int64_t units = perPhase * split.phases;  // units of one XCD
 
   const pipe::Problem<ET> pb = make_problem<ET, D, HEADS>(sparseAToXidx, bitmapBytes, Q, K, V, N,
                                                           scaleLog2, ldIn, nTcb);
   const unsigned ringAddr =
-      (unsigned)(uintptr_t)(F3S_LDS unsigned char*)smem + (unsigned)wave * pipe::Geo<D>::WAVE_BYTES;
+      (unsigned)(uintptr_t)(F3S_LDS unsigned char*)smem + (unsigned)wave * pipe::Geo<D, unit_stages(D, true)>::WAVE_BYTES;
 
   // k-th unit of this workgroup's sequence -> index in the XCD's unit space, -1 past its end,
   // -2 when the sequence is over
@@ -334,14 +452,18 @@ f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
       k = __hip_atomic_fetch_add(&sCtl[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     return unit_index(uniform(k));
   };
-  // unit -> (phase, position of the order, head)
+  auto unit_of = [&](int64_t u) -> Unit {
+    const int phase = (int)(u / perPhase);
+    return split.unit(x, phase, (unsigned)(u - phase * perPhase));
+  };
   auto window_of = [&](int64_t u) -> int {
     if (u < 0) return -1;
-    const int pos = (int)((u / heads) % nRW);
+    const int pos = unit_of(u).pos;
+    if (pos >= nRW) return -1;
     const int w = windowOrder ? windowOrder[pos] : pos;
     return (unsigned)w < (unsigned)nRW ? w : -1;
   };
-  auto slice_of = [&](int64_t u) -> int { return (int)((u / heads) / nRW) * kXcds + x; };
+  auto slice_of = [&](int64_t u) -> int { return unit_of(u).slice; };
 
   // three units in flight: `u` runs, u1 has its window and is fetching its block range, u2 is
   // fetching its window
@@ -364,12 +486,12 @@ f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
     const int w2 = window_of(u2);
     const int wu = uniform(w), t0u = uniform(t0), t1u = uniform(t1);
     if (wu >= 0 && t1u > t0u && t0u >= 0 && (int64_t)t1u <= nTcb) {
-      const int head = HEADS ? (int)(u % heads) : 0;
+      const int head = HEADS ? unit_of(u).head : 0;
       Pipe pp;
       pp.init(pb, wu, ringAddr, head);
       pp.run(pb, t0u, t1u);
       const int64_t wh = (int64_t)wu * heads + head;
-      store_partial<D>(pp, partial + (wh * S + slice_of(u)) * partial_dwords<D>() + lane);
+      store_partial<D>(pp, partial + (wh * S + slice_of(u)) * partial_floats<D>());
     }
     u = u1;
     w = w1;
@@ -381,79 +503,78 @@ f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
 }
 
 // One wave per (window, head): log-sum-exp merge of the unit partials in slice order, then the
-// window's rows. Lane (g, c) holds O[q = c][16j + 4g + i] in O[j * 4 + i], as in the unit
-// kernels. The partials of up to B live slices are requested together.
+// window's rows. Lane (g, c) holds O[q = c][16j + 4g + i] in O[j][i], as in the unit kernels; the
+// partials of up to B live slices are requested together. The rows leave through LDS, as in the
+// unit kernel.
+// Bound by memory: 0.54 GB of partials at 233k nodes and 8 slices. (Lanes that hold O row by row
+// from the start need no LDS, but read the tiles in pieces of 64 bytes: 101 -> 120 us there.)
 template <int D, bool SOFTMAX>
 __global__ __launch_bounds__(256) void f3s_merge_slices_kernel(
     const int32_t* __restrict__ sliceStart, int S, int N, int nRW, int nHeads,
     const float* __restrict__ partial, float* __restrict__ out, int ldOut) {
   constexpr int T = D / 16;
-  constexpr int R = D / 4;  // O registers per lane
   constexpr int B = D <= 64 ? 4 : D <= 128 ? 2 : 1;
+  extern __shared__ __align__(1024) unsigned char smem[];
   const int lane = threadIdx.x & 63;
-  const int64_t wh = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int wave = threadIdx.x >> 6;
+  const int64_t wh = (int64_t)blockIdx.x * 4 + wave;
   if (wh >= (int64_t)nRW * nHeads) return;
   const int w = (int)(wh / nHeads);
   const int head = (int)(wh - (int64_t)w * nHeads);
-  const int g = lane >> 4;
   const int c = lane & 15;
   float M = 0.0f, L = 0.0f;
-  float O[R];
+  float4v O[T];
 #pragma unroll
-  for (int r = 0; r < R; r++) O[r] = 0.0f;
+  for (int j = 0; j < T; j++) O[j] = float4v{0.f, 0.f, 0.f, 0.f};
   const int32_t* ss = sliceStart + (int64_t)w * (S + 1);
-  const float* base = partial + wh * S * partial_dwords<D>() + lane;
+  const float* base = partial + wh * S * partial_floats<D>();
   for (int s0 = 0; s0 < S; s0 += 64) {
     const int s = s0 + lane;
     unsigned long long live = __builtin_amdgcn_ballot_w64(s < S && ss[s + 1] > ss[s]);
     while (live) {
       int sel[B];
-      float v[B][R + 2];
+      float ms[B], ls[B];
+      float4v v[B][T];
 #pragma unroll
       for (int k = 0; k < B; k++) {
         sel[k] = -1;
         if (live) {
           sel[k] = s0 + __builtin_ctzll(live);
           live &= live - 1;
-          const float* src = base + (int64_t)sel[k] * partial_dwords<D>();
+          const float* src = base + (int64_t)sel[k] * partial_floats<D>();
 #pragma unroll
-          for (int r = 0; r < R + (SOFTMAX ? 2 : 0); r++)
-            v[k][r] = F3S_PARTIAL_LOAD(src + r * 64);
+          for (int j = 0; j < T; j++)
+            v[k][j] = F3S_PARTIAL_LOAD(reinterpret_cast<const float4v*>(src) + j * 64 + lane);
+          if constexpr (SOFTMAX) {
+            ms[k] = F3S_PARTIAL_LOAD(src + 16 * D + c);
+            ls[k] = F3S_PARTIAL_LOAD(src + 16 * D + 16 + c);
+          }
         }
       }
 #pragma unroll
       for (int k = 0; k < B; k++) {
         if (sel[k] < 0) continue;
         if constexpr (SOFTMAX) {
-          const float ms = v[k][R], ls = v[k][R + 1];
-          const float mx = fmaxf(M, ms);
-          const float a = pipe::fast_exp2(M - mx), b = pipe::fast_exp2(ms - mx);
+          const float mx = fmaxf(M, ms[k]);
+          const float a = pipe::fast_exp2(M - mx), b = pipe::fast_exp2(ms[k] - mx);
           M = mx;
-          L = fmaf(a, L, b * ls);
+          L = fmaf(a, L, b * ls[k]);
 #pragma unroll
-          for (int r = 0; r < R; r++) O[r] = fmaf(a, O[r], b * v[k][r]);
+          for (int j = 0; j < T; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) O[j][i] = fmaf(a, O[j][i], b * v[k][j][i]);
         } else {
 #pragma unroll
-          for (int r = 0; r < R; r++) O[r] += v[k][r];
+          for (int j = 0; j < T; j++) O[j] += v[k][j];
         }
       }
     }
   }
-  float inv = 1.0f;
-  if constexpr (SOFTMAX) {
-    const float lAll = pipe::row_sum4(L);
-    inv = (lAll == 0.0f) ? 0.0f : 1.0f / lAll;
-  }
-  const int64_t row = (int64_t)w * 16 + c;
-  if (row < N) {
-    float* dst = out + row * ldOut + head * D + 4 * g;
+  const float inv = SOFTMAX ? (L == 0.0f ? 0.0f : 1.0f / L) : 1.0f;
 #pragma unroll
-    for (int jj = 0; jj < T; jj++) {
-      const float4v v4 = {O[jj * 4] * inv, O[jj * 4 + 1] * inv, O[jj * 4 + 2] * inv,
-                          O[jj * 4 + 3] * inv};
-      *reinterpret_cast<float4v*>(dst + 16 * jj) = v4;
-    }
-  }
+  for (int j = 0; j < T; j++) O[j] *= inv;
+  store_rows<D>(O, reinterpret_cast<float*>(smem) + wave * rows_lds_floats<D>(), w, N,
+                out + head * D, ldOut);
 }
 
 // LDS of a workgroup of rings; above 64 KiB the kernel has to be told once
@@ -465,69 +586,48 @@ int allow_lds(KernelT kernel, size_t bytes) {
   return 0;
 }
 
-// Phases P (S = 8 P slices). One slice's K + V rows are held to about 8 MiB: twice an XCD's L2,
-// which already catches 4 of 5 accesses on the 233k-node benchmark graph (P = 1), while more and
+// Phases P (8 P slices of all heads). One slice's K + V rows are held to about 8 MiB: twice an XCD's
+// L2, which already catches 4 of 5 accesses on the 233k-node benchmark graph (P = 1), while more and
 // shorter units cost more than their higher hit rate returns (measured 1.54 / 1.69 / 1.86 ms at
 // P = 1 / 2 / 3). F3S_SLICE_PHASES in the environment overrides the choice.
-int choose_phases(int N, int d) {
+XcdSplit choose_split(int N, int d, int heads) {
   const char* e = getenv("F3S_SLICE_PHASES");  // read per call: tests walk through the phases
   const int forced = e ? atoi(e) : 0;
-  if (forced > 0) return forced > kMaxPhases ? kMaxPhases : forced;
-  const int64_t bytes = (int64_t)N * d * 4;  // K + V
+  if (forced > 0) return {forced > kMaxPhases ? kMaxPhases : forced, kXcds, 1, 1, heads, 1};
+  const int64_t bytes = (int64_t)N * d * heads * 4;  // K + V
   const int64_t perPhase = (int64_t)kXcds * 8 * 1024 * 1024;
   int P = (int)((bytes + perPhase - 1) / perPhase);
   if (P < 1) P = 1;
   if (P > kMaxPhases) P = kMaxPhases;
-  return P;
+  return {P, kXcds, 1, 1, heads, 1};
 }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // byte offsets of the parts of the workspace
 struct SlicedLayout {
-  int P, S;
+  XcdSplit split;
+  int S;
   size_t tickets, sliceStart, partial, total;
   size_t padded;  // 0, or where the copies of K and V with 256-byte rows start (single head, d = 64)
 };
-// Rows of 128 bytes gathered from addresses that are multiples of 256 are served faster than rows
-// from the odd 128-byte lines in between (233k-node graph, d = 64: 1.42 ms with every row on an
-// even line, 1.55 ms with every row on an odd line, 1.48 ms for contiguous rows, which alternate;
-// the L2 hit and miss counts are the same in all three). The single-head call at d = 64 therefore
-// gathers from copies of K and V with a row pitch of 256 bytes, made at the start of the call.
-constexpr int kPaddedRowBytes = 256;
 // nHeads = 0: the single-head layout
 SlicedLayout sliced_layout(int N, int d, int nHeads) {
   const int heads = nHeads > 0 ? nHeads : 1;
   SlicedLayout L;
-  L.P = choose_phases(N, d * heads);
-  L.S = L.P * kXcds;
+  L.split = choose_split(N, d, heads);
+  L.S = L.split.slices();
   const size_t nRW = (size_t)(N + kWinRows - 1) / kWinRows;
   L.tickets = 256;
   L.sliceStart = L.tickets + 256;
   L.partial = L.sliceStart + align256(nRW * (L.S + 1) * sizeof(int32_t));
-  L.total = align256(L.partial + nRW * heads * L.S * (size_t)(d / 4 + 2) * 64 * sizeof(float));
+  L.total = align256(L.partial + nRW * heads * L.S * (size_t)(16 * d + 32) * sizeof(float));
   L.padded = 0;
   if (nHeads == 0 && d == 64) {
     L.padded = L.total;
     L.total += 2 * (size_t)N * kPaddedRowBytes;
   }
   return L;
-}
-
-// K and V rows of 128 bytes copied to a pitch of 256 bytes (one thread per 16 bytes of each)
-typedef int pad_chunk __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256) void pad_rows_kernel(const pad_chunk* __restrict__ K,
-                                                       const pad_chunk* __restrict__ V,
-                                                       int64_t chunks, pad_chunk* __restrict__ Kp,
-                                                       pad_chunk* __restrict__ Vp) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= chunks) return;
-  const int64_t row = i >> 3;
-  const int c = (int)(i & 7);
-  const pad_chunk k = __builtin_nontemporal_load(K + i);  // read once, by nobody else
-  const pad_chunk v = __builtin_nontemporal_load(V + i);
-  Kp[row * (kPaddedRowBytes / 16) + c] = k;
-  Vp[row * (kPaddedRowBytes / 16) + c] = v;
 }
 
 bool padded_rows_requested() {
@@ -548,9 +648,9 @@ int resident_grid(int* grid) {
     if (dev >= 0 && dev < kMaxDev) cusOf[dev] = cus;
   }
   // the rings plus the 1 KiB the two control words cost in front of the 1 KiB-aligned rings
-  constexpr size_t lds = (size_t)NW * pipe::Geo<D>::WAVE_BYTES + 1024;
+  constexpr size_t lds = (size_t)NW * pipe::Geo<D, unit_stages(D, true)>::WAVE_BYTES + 1024;
   int perCu = (int)((160 * 1024) / lds);
-  const int byWaves = unit_waves_per_simd(D) * 4 / NW;
+  const int byWaves = unit_waves_per_simd(D, true) * 4 / NW;
   if (perCu > byWaves) perCu = byWaves;
   if (perCu < 1) perCu = 1;
   int gsz = cus * perCu / kXcds * kXcds;
@@ -570,24 +670,24 @@ int launch_sliced_units(const int32_t* rwo, const int32_t* order, const int32_t*
                         float scaleLog2, float* out, int32_t* tickets, int32_t* sliceStart,
                         float* partial, const SlicedLayout& L, int heads, int ldIn, int ldOut,
                         int64_t nTcb, hipStream_t stream, int ldQ = 0) {
-  constexpr size_t lds = (size_t)kUnitWaves * pipe::Geo<D>::WAVE_BYTES;
+  constexpr size_t lds = (size_t)kUnitWaves * pipe::Geo<D, unit_stages(D, true)>::WAVE_BYTES;
   if (resident_requested()) {
     auto kernel = f3s_fwd_resident_kernel<ET, D, SOFTMAX, HEADS, kUnitWaves>;
     if (int rc = allow_lds(kernel, lds)) return rc;
     int grid = 0;
     if (int rc = resident_grid<D, kUnitWaves>(&grid)) return rc;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kUnitWaves * 64), lds, stream, order,
-                       sliceStart, L.P, nRW, L.S, N, nTcb, tickets, atox, bm, Q, K, V, scaleLog2,
+                       sliceStart, L.split, nRW, N, nTcb, tickets, atox, bm, Q, K, V, scaleLog2,
                        partial, heads, ldIn);
   } else {
     auto kernel = f3s_fwd_unit_kernel<ET, D, SOFTMAX, true, HEADS>;
     if (int rc = allow_lds(kernel, lds)) return rc;
-    const int64_t nGroups = ((int64_t)nRW * heads + kUnitWaves - 1) / kUnitWaves;
-    const int64_t grid = (int64_t)L.P * nGroups * kXcds;
+    const int64_t nGroups = (L.split.units(nRW) + kUnitWaves - 1) / kUnitWaves;
+    const int64_t grid = L.split.phases * nGroups * kXcds;
     if (grid >= ((int64_t)1 << 31))
       return fail(-2, "f3s_attention: too many (window, slice, head) units for one launch");
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kUnitWaves * 64), lds, stream, order, rwo,
-                       atox, bm, sliceStart, L.S, (int)nGroups, N, nRW, nTcb, Q, K, V, scaleLog2,
+                       atox, bm, sliceStart, L.split, (int)nGroups, N, nRW, nTcb, Q, K, V, scaleLog2,
                        partial, out, heads, ldIn, ldOut, 0, 0, ldQ);
   }
   F3S_HIP_CHECK(hipGetLastError());
@@ -607,10 +707,20 @@ int launch_sliced_d(const int32_t* rwo, const int32_t* order, const int32_t* ato
   auto* tickets = reinterpret_cast<int32_t*>(ws + L.tickets);
   auto* sliceStart = reinterpret_cast<int32_t*>(ws + L.sliceStart);
   auto* partial = reinterpret_cast<float*>(ws + L.partial);
-  const int64_t entries = (int64_t)nRW * (S + 1);
-  hipLaunchKernelGGL(sliced_setup_kernel, dim3((unsigned)((entries + 255) / 256)), dim3(256), 0,
-                     stream, rwo, atox, N, nRW, S, sliceWidth, nTcb, hdr, mode, tickets,
-                     sliceStart);
+  const unsigned setupBlocks = (unsigned)(((int64_t)nRW * 16 + 255) / 256);
+  // copies of K and V with 256-byte rows, gathered through the pitched (multi-head) form of the
+  // unit kernel with one head; Q stays where it is
+  const bool padded = mode != 1 && nHeads == 0 && L.padded != 0 && padded_rows_requested() &&
+                      !resident_requested() &&
+                      !gather_needs_wide_offsets(N, kPaddedRowBytes, true);
+  auto* kp = padded ? reinterpret_cast<ET*>(ws + L.padded) : nullptr;
+  auto* vp = padded ? kp + (size_t)N * (kPaddedRowBytes / sizeof(ET)) : nullptr;
+  const int64_t chunks = padded ? (int64_t)N * (D * (int)sizeof(ET) / 16) : 0;
+  hipLaunchKernelGGL(sliced_setup_kernel, dim3(setupBlocks + (unsigned)((chunks + 255) / 256)),
+                     dim3(256), 0, stream, rwo, atox, N, nRW, S, sliceWidth, nTcb, hdr, mode,
+                     tickets, sliceStart, (int)setupBlocks, static_cast<const pad_chunk*>(K),
+                     static_cast<const pad_chunk*>(V), chunks, reinterpret_cast<pad_chunk*>(kp),
+                     reinterpret_cast<pad_chunk*>(vp));
   F3S_HIP_CHECK(hipGetLastError());
   if (mode == 1) return 0;
   const auto* bm = reinterpret_cast<const uint8_t*>(bitmap);
@@ -622,18 +732,7 @@ int launch_sliced_d(const int32_t* rwo, const int32_t* order, const int32_t* ato
     rc = launch_sliced_units<ET, D, SOFTMAX, true>(rwo, order, atox, bm, N, nRW, q, k, v,
                                                    scaleLog2, out, tickets, sliceStart, partial, L,
                                                    heads, ldIn, ldOut, nTcb, stream);
-  } else if (L.padded != 0 && padded_rows_requested() && !resident_requested() &&
-             !gather_needs_wide_offsets(N, kPaddedRowBytes, true)) {
-    // copies of K and V with 256-byte rows, gathered through the pitched (multi-head) form of the
-    // unit kernel with one head; Q stays where it is
-    auto* kp = reinterpret_cast<ET*>(ws + L.padded);
-    auto* vp = kp + (size_t)N * (kPaddedRowBytes / sizeof(ET));
-    const int64_t chunks = (int64_t)N * (D * (int)sizeof(ET) / 16);
-    hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0,
-                       stream, reinterpret_cast<const pad_chunk*>(k),
-                       reinterpret_cast<const pad_chunk*>(v), chunks,
-                       reinterpret_cast<pad_chunk*>(kp), reinterpret_cast<pad_chunk*>(vp));
-    F3S_HIP_CHECK(hipGetLastError());
+  } else if (padded) {
     rc = launch_sliced_units<ET, D, SOFTMAX, true>(
         rwo, order, atox, bm, N, nRW, q, kp, vp, scaleLog2, out, tickets, sliceStart, partial, L, 1,
         kPaddedRowBytes / (int)sizeof(ET), D, nTcb, stream, D);
@@ -644,8 +743,10 @@ int launch_sliced_d(const int32_t* rwo, const int32_t* order, const int32_t* ato
   }
   if (rc != 0) return rc;
   const int64_t merges = (int64_t)nRW * heads;
-  hipLaunchKernelGGL((f3s_merge_slices_kernel<D, SOFTMAX>), dim3((unsigned)((merges + 3) / 4)),
-                     dim3(256), 0, stream, sliceStart, S, N, nRW, heads, partial, out,
+  auto merge = f3s_merge_slices_kernel<D, SOFTMAX>;
+  constexpr size_t mergeLds = (size_t)4 * rows_lds_floats<D>() * sizeof(float);
+  if ((rc = allow_lds(merge, mergeLds)) != 0) return rc;
+  hipLaunchKernelGGL(merge, dim3((unsigned)((merges + 3) / 4)), dim3(256), mergeLds, stream, sliceStart, S, N, nRW, heads, partial, out,
                      nHeads > 0 ? ldOut : D);
   F3S_HIP_CHECK(hipGetLastError());
   return 0;
@@ -698,29 +799,39 @@ int launch_attention_sliced(const int32_t* rowWindowOffset, const int32_t* windo
 
 namespace {
 
+// Positions of the order an XCD takes in a row: windows that follow each other in the order (equal
+// block counts are in window order) often name the same rows, which then come from one L2
+// (60k-node community graph, 4 x 64: 69 -> 52 us; 8, 16 and 64 windows are alike, 256 leave the
+// XCDs unevenly loaded). Only short windows are dealt in chunks: of long ones in heavy-first order
+// the first XCD would get the sixteen heaviest.
+constexpr int kShortChunk = 16;
+
 template <typename ET, int D, bool SOFTMAX>
 int launch_short_d(const int32_t* rwo, const int32_t* order, const int32_t* atox,
                    const uint64_t* bitmap, int N, const void* Q, const void* K, const void* V,
                    float scaleLog2, float* out, int nHeads, int ldIn, int ldOut, int maxBlocks,
                    int longPrefix, int64_t nTcb, hipStream_t stream) {
-  const int64_t nRW = ((int64_t)N + kWinRows - 1) / kWinRows;
-  const int64_t units = nRW * (nHeads > 0 ? nHeads : 1);
-  const dim3 grid((unsigned)((units + kShortUnitWaves - 1) / kShortUnitWaves)),
-      block(kShortUnitWaves * 64);
+  const int nRW = (N + kWinRows - 1) / kWinRows;
+  XcdSplit split = split_heads(D, nHeads > 0 ? nHeads : 1);
+  split.chunk = kShortChunk;
+  const int64_t nGroups = (split.units(nRW) + kUnitWaves - 1) / kUnitWaves;
+  if (nGroups * kXcds >= ((int64_t)1 << 31))
+    return fail(-2, "f3s_attention: too many (window, head) units for one launch");
+  const dim3 grid((unsigned)(nGroups * kXcds)), block(kUnitWaves * 64);
   const auto* bm = reinterpret_cast<const uint8_t*>(bitmap);
   const auto* q = static_cast<const ET*>(Q);
   const auto* k = static_cast<const ET*>(K);
   const auto* v = static_cast<const ET*>(V);
-  constexpr size_t lds = (size_t)kShortUnitWaves * pipe::Geo<D>::WAVE_BYTES;
+  constexpr size_t lds = (size_t)kUnitWaves * pipe::Geo<D, unit_stages(D, false)>::WAVE_BYTES;
   if (nHeads > 0) {
     if (int rc = allow_lds(f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, true>, lds)) return rc;
     hipLaunchKernelGGL((f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, true>), grid, block, lds,
-                       stream, order, rwo, atox, bm, nullptr, 0, 0, N, (int)nRW, nTcb, q, k, v,
+                       stream, order, rwo, atox, bm, nullptr, split, (int)nGroups, N, nRW, nTcb, q, k, v,
                        scaleLog2, nullptr, out, nHeads, ldIn, ldOut, maxBlocks, longPrefix, 0);
   } else {
     if (int rc = allow_lds(f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, false>, lds)) return rc;
     hipLaunchKernelGGL((f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, false>), grid, block, lds,
-                       stream, order, rwo, atox, bm, nullptr, 0, 0, N, (int)nRW, nTcb, q, k, v,
+                       stream, order, rwo, atox, bm, nullptr, split, (int)nGroups, N, nRW, nTcb, q, k, v,
                        scaleLog2, nullptr, out, 1, D, D, maxBlocks, longPrefix, 0);
   }
   F3S_HIP_CHECK(hipGetLastError());

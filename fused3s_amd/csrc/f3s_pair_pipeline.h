@@ -158,7 +158,10 @@ __device__ __forceinline__ void vm_wait() {
 // src/F3S_kernel.cu:601-604,1424,1522). The ring is laid out for DP, the next power of two: a row
 // of the LDS tile is DP elements wide, of which the first D hold data; lanes whose chunk does not
 // exist fetch nothing.
-template <int D>
+// STAGES: pairs of the ring in flight per wave (the kernels choose: two stages where a wave is alone
+// with a long run of blocks, one stage and more waves where runs are short and what has to be
+// hidden is the chain of loads in front of the first gather).
+template <int D, int STAGES>
 struct Geo {
   static_assert(D % 32 == 0 && D >= 32 && D <= 256, "head dimension: a multiple of 32 up to 256");
   static constexpr int DP = D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256;
@@ -172,8 +175,8 @@ struct Geo {
   static constexpr int RPI = 64 / CPR;     // rows per gather instruction
   static constexpr int TILE = 32 * ROW;    // K (or V) rows of one pair
   static constexpr int STAGE = 2 * TILE;   // one pair: K tile, then V tile
-  static constexpr int NS = DP >= 128 ? 1 : 2;  // stages of the ring
-  static constexpr int META_SLOT = 1024;   // metadata of four steps: 512 B ids, 256 B bitmaps
+  static constexpr int NS = STAGES;  // stages of the ring
+  static constexpr int META_SLOT = 768;    // metadata of four steps: 512 B ids, 256 B bitmaps
   static constexpr int META = 2 * META_SLOT;
   static constexpr int WAVE_BYTES = NS * STAGE + META;
 };
@@ -274,9 +277,9 @@ struct Problem {
 // comes from preprocessing with 8-column blocks; two consecutive 16x8 blocks are laid out like
 // one 16x16 block, block indices and counts below are then in 16x8 blocks. WIDE: K or V spans
 // 4 GiB or more (or a pitched layout exceeds the 24-bit multiply): row offsets in 64 bits.
-template <typename ET, int D, bool SOFTMAX, bool HEADS, bool W8, bool WIDE = false>
+template <typename ET, int D, bool SOFTMAX, bool HEADS, bool W8, int STAGES, bool WIDE = false>
 struct PairPipeline {
-  typedef Geo<D> G;
+  typedef Geo<D, STAGES> G;
   typedef typename Vec<ET, 8>::type half8;
   static constexpr int T = G::T;
   static constexpr int KS = G::KS;
@@ -388,7 +391,7 @@ struct PairPipeline {
       if (blk >= t1) blk = t1 - 1;
       src = reinterpret_cast<const char*>(pb.sparseAToXidx) + (blk * IDS_PER_BLOCK + within) * 4;
     } else {
-      const int b = (lane - 32) & 15;  // lanes 48..63 repeat lanes 32..47 (their copy is unused)
+      const int b = (lane - 32) & 15;  // lanes 48..63 fetch nothing
       int64_t blk = first + (b * 16) / BM_BYTES;
       const int within = (b * 16) % BM_BYTES;
       if (blk >= t1) blk = t1 - 1;
@@ -396,15 +399,17 @@ struct PairPipeline {
     }
     F3S_LDS int4v* dst =
         (F3S_LDS int4v*)(uintptr_t)(uniform((int)metaBase) + (k & 1) * G::META_SLOT);
-    __builtin_amdgcn_global_load_lds(reinterpret_cast<const int4v*>(src), dst, 16, 0, 0);
+    if (lane < 48)
+      __builtin_amdgcn_global_load_lds(reinterpret_cast<const int4v*>(src), dst, 16, 0, 0);
   }
 
-  // K and V rows of step p into ring stage `stage` (compile-time), row ids from metadata.
+  // K and V rows of step p into ring stage STAGE_IDX = p % NS, row ids from metadata. The step's
+  // position in its metadata slot is the compile-time Q4 plus the run-time q (one of them 0).
   template <int STAGE_IDX, int Q4>
-  __device__ __forceinline__ void issue_gather(const Problem<ET>& pb, int metaSlot) {
+  __device__ __forceinline__ void issue_gather(const Problem<ET>& pb, int metaSlot, int q) {
     // row ids of this lane's TG slots: groups of four consecutive dwords of the step's 32 ids
     int rows[TG];
-    const unsigned ida = idReadAddr + metaSlot * G::META_SLOT;
+    const unsigned ida = idReadAddr + (unsigned)(metaSlot * G::META_SLOT + q * 128);
     if constexpr (DP == 32) {
       const int2v r = lds_read2_b32<Q4 * 32, Q4 * 32 + 2>(ida);
       lds_wait();
@@ -482,14 +487,15 @@ struct PairPipeline {
   };
 
   template <int STAGE_IDX, int Q4>
-  __device__ __forceinline__ void read_operands(int metaSlot, Operands& op) {
+  __device__ __forceinline__ void read_operands(int metaSlot, int q, Operands& op) {
     constexpr int SO = STAGE_IDX * G::STAGE;
 #pragma unroll
     for (int b = 0; b < 2; b++)
 #pragma unroll
       for (int i = 0; i < KS; i++) op.k[b][i] = lds_read_b128<SO>(kReadAddr[b][i]);
     read_v_tile<SO, 0>(op);
-    op.words = lds_read2_b32<Q4 * 16, Q4 * 16 + 8>(maskReadAddr + metaSlot * G::META_SLOT);
+    op.words = lds_read2_b32<Q4 * 16, Q4 * 16 + 8>(
+        maskReadAddr + (unsigned)(metaSlot * G::META_SLOT + q * 64));
   }
   // tile J of the V operand: 128 bytes (eight chunks) per four tiles beyond tile J % 4
   template <int SO, int J>
@@ -565,8 +571,8 @@ struct PairPipeline {
         b.y = __int_as_float(__float_as_int(s[5]) & keep[5]);
         b.z = __int_as_float(__float_as_int(s[6]) & keep[6]);
         b.w = __int_as_float(__float_as_int(s[7]) & keep[7]);
-        if ((g >> 1) < nValid) *reinterpret_cast<float4*>(dst) = a;
-        if (2 + (g >> 1) < nValid) *reinterpret_cast<float4*>(dst + 256) = b;
+        if ((g >> 1) < nValid) store_out(dst, out_vec{a.x,a.y,a.z,a.w});
+        if (2 + (g >> 1) < nValid) store_out(dst + 256, out_vec{b.x,b.y,b.z,b.w});
       }
     }
     float e[8];
@@ -652,25 +658,25 @@ struct PairPipeline {
     // prologue: metadata of the first four steps, then the first NS gathers
     issue_meta(pb, t0, t1, 0);
     vm_wait<0>();
+    issue_gather<0, 0>(pb, 0, 0);
     if constexpr (NS == 2) {
-      issue_gather<0, 0>(pb, 0);
-      if (nSteps > 1) issue_gather<1, 1>(pb, 0);
-    } else {
-      issue_gather<0, 0>(pb, 0);
+      if (nSteps > 1) issue_gather<1, 1>(pb, 0, 0);
     }
     int p = 0;
     bool metaIssued = false;  // the last first-of-four step requested the next four's metadata
-    // One step; STAGE_IDX = p % NS and Q4 = p % 4 are compile-time. GQ4 = (p + NS) % 4 is the
-    // position of the step whose gather is issued, in metadata slot ((p + NS) / 4) & 1.
+    // One step. NS == 2: STAGE_IDX = p % NS and Q4 = p % 4 are compile-time, the loop is unrolled
+    // by four. NS == 1: Q4 is 0 and the position in the metadata slot a run-time offset (two
+    // scalar instructions), so that the loop is one step long: unrolled by four, its four exits
+    // cost the kernels around it 40 to 70 vector registers.
 #define F3S_PIPE_STEP(STAGE_IDX, Q4)                                                           \
   {                                                                                            \
-    constexpr int GQ4 = (Q4 + NS) % 4;                                                         \
-    const bool more = p + NS < nSteps;                                                         \
+    constexpr int GQ4 = NS == 2 ? (Q4 + NS) % 4 : 0;                                           \
+    const int q = NS == 2 ? Q4 : p & 3;                                                        \
     /* loads issued after this step's gather: the later stages' gathers and, if one of those  \
        steps opened a group of four, its metadata load */                                     \
     if constexpr (NS == 2) {                                                                   \
       if (p + 1 < nSteps) {                                                                    \
-        if (Q4 == 1 && metaIssued) vm_wait<2 * TG + 1>(); else vm_wait<2 * TG>();                \
+        if (Q4 == 1 && metaIssued) vm_wait<2 * TG + 1>(); else vm_wait<2 * TG>();              \
       } else {                                                                                 \
         vm_wait<0>();                                                                          \
       }                                                                                        \
@@ -678,14 +684,16 @@ struct PairPipeline {
       vm_wait<0>();                                                                            \
     }                                                                                          \
     Operands op;                                                                               \
-    F3S_ABL_READ((read_operands<STAGE_IDX, Q4>((p >> 2) & 1, op)));                            \
+    F3S_ABL_READ((read_operands<STAGE_IDX, Q4>((p >> 2) & 1, NS == 2 ? 0 : q, op)));           \
     lds_wait();                                                                                \
     __builtin_amdgcn_sched_barrier(0);                                                         \
-    if constexpr (Q4 == 0) {                                                                   \
+    if (q == 0) {                                                                              \
       metaIssued = (p >> 2) + 1 <= (nSteps - 1) >> 2;                                          \
       if (metaIssued) issue_meta(pb, t0, t1, (p >> 2) + 1);                                    \
     }                                                                                          \
-    if (more) F3S_ABL_GATHER((issue_gather<STAGE_IDX, GQ4>(pb, ((p + NS) >> 2) & 1)));         \
+    if (p + NS < nSteps)                                                                       \
+      F3S_ABL_GATHER((issue_gather<STAGE_IDX, GQ4>(pb, ((p + NS) >> 2) & 1,                    \
+                                                   NS == 2 ? 0 : (p + NS) & 3)));              \
     __builtin_amdgcn_sched_barrier(0);                                                         \
     {                                                                                          \
       const int tFirst = t0 + p * BPS;                                                         \
@@ -697,9 +705,11 @@ struct PairPipeline {
   }
     while (true) {
       F3S_PIPE_STEP(0, 0)
-      F3S_PIPE_STEP(1 % NS, 1)
-      F3S_PIPE_STEP(0, 2)
-      F3S_PIPE_STEP(1 % NS, 3)
+      if constexpr (NS == 2) {
+        F3S_PIPE_STEP(1, 1)
+        F3S_PIPE_STEP(0, 2)
+        F3S_PIPE_STEP(1, 3)
+      }
     }
 #undef F3S_PIPE_STEP
   }

@@ -26,9 +26,28 @@ namespace window {
 using pipe::float4v;
 using pipe::kLog2e;
 
-// Waves per SIMD the register allocator is held to: the LDS rings allow four workgroups per CU at
-// D = 32, two up to D = 128 and one above.
-constexpr int waves_per_simd(int d) { return d <= 32 ? 4 : d <= 128 ? 2 : 1; }
+// Waves and ring stages of a workgroup.
+//   TEAM_SHORT  one workgroup for every window: four waves of one stage. A window's share of a wave is
+//               a few steps, what counts is how many workgroups hide each other's chain of loads in
+//               front of the first gather: five per CU at D = 32 (four were measured alike), three
+//               at D = 64 (two stages allow two: 169k-node R-MAT graph 105 -> 88 us), two up to
+//               D = 128, one above.
+//   TEAM_LONG   the few long windows of a graph of short ones, one workgroup after the other per CU:
+//               as many bytes in flight as one CU's LDS holds, eight waves of two stages up to
+//               D = 64, eight of one stage up to D = 128, four above.
+enum Team { TEAM_SHORT, TEAM_LONG };
+constexpr int team_waves(Team t, int d) { return t == TEAM_LONG && d <= 128 ? 8 : 4; }
+constexpr int team_stages(Team t, int d) { return t == TEAM_LONG && d <= 64 ? 2 : 1; }
+constexpr int waves_per_simd(Team t, int d) {
+  if (d > 128) return 1;
+  return t == TEAM_LONG || d > 64 ? 2 : d > 32 ? 3 : 4;
+}
+
+// LDS of a workgroup: its waves' rings
+constexpr size_t team_lds(Team t, int d) {
+  const int dp = d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : 256;
+  return (size_t)team_waves(t, d) * (team_stages(t, d) * 128 * dp + 2 * 768);
+}
 
 // Constant-rate (100 MHz) timestamp shared by all CUs, and an id of the CU this wave runs on:
 // XCC id in bits 8.., {SE, SH, CU} of HW_ID in bits 0..7. Used only by the timed variant, which
@@ -69,17 +88,21 @@ __global__ void reset_window_cursor_kernel() {
 }
 
 // WIDE: 64-bit row offsets in the K / V gathers.
-template <typename ET, int D, int NWAVES, bool SOFTMAX, bool CLOCKED, bool HEADS, bool W8,
+template <typename ET, int D, Team TEAM, bool SOFTMAX, bool CLOCKED, bool HEADS, bool W8,
           bool WIDE, bool PERSIST = false>
-__global__ __launch_bounds__(NWAVES * 64)
-__attribute__((amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D)))) void f3s_fwd_kernel(
+__global__ __launch_bounds__(team_waves(TEAM, D) * 64)
+__attribute__((amdgpu_waves_per_eu(waves_per_simd(TEAM, D), waves_per_simd(TEAM, D)))) void
+f3s_fwd_kernel(
     const int32_t* __restrict__ rowWindowOffset, const int32_t* __restrict__ windowOrder,
     const int32_t* __restrict__ sparseAToXidx, const uint8_t* __restrict__ bitmapBytes, int N,
     int nRW, int64_t nTcb, const ET* __restrict__ Q, const ET* __restrict__ K,
     const ET* __restrict__ V, float scaleLog2, float* __restrict__ out,
     unsigned long long* __restrict__ cuTimer, int nHeads, int ldIn, int ldOut,
     float* __restrict__ sddmm, int minBlocks, int nPositions) {
-  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, W8, WIDE> Pipe;
+  constexpr int NWAVES = team_waves(TEAM, D);
+  constexpr int WAVE_BYTES = pipe::Geo<D, team_stages(TEAM, D)>::WAVE_BYTES;
+  static_assert(team_lds(TEAM, D) == (size_t)NWAVES * WAVE_BYTES, "what the launch asks for");
+  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, W8, team_stages(TEAM, D), WIDE> Pipe;
   constexpr int T = D / 16;
   constexpr int OSTRIDE = D + 4;
   constexpr int BPS = W8 ? 4 : 2;  // blocks of the structure per pipeline step
@@ -89,20 +112,20 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D)))) void 
 
   static_assert(!PERSIST || (!CLOCKED && !HEADS && !W8), "the persistent form is single-head");
   __shared__ int sNextPos[2];
+  constexpr bool scan = TEAM == TEAM_LONG;
   __shared__ int sUnitCount;
-  __shared__ int sUnitList[NWAVES * 64];
+  __shared__ int sUnitList[scan ? NWAVES * 64 : 1];
   int pos = HEADS ? (int)(blockIdx.x / (unsigned)nHeads) : (int)blockIdx.x;
   int head = HEADS ? (int)(blockIdx.x - (unsigned)pos * (unsigned)nHeads) : 0;
-  // A launch that shares the windows with the wave-per-window kernel (minBlocks >= 0) covers the
-  // (position, head) units of the order's first nPositions positions with a grid of its own
-  // size: thread t of workgroup b looks at unit b + t * gridDim.x, and the workgroup computes
+  // A launch that shares the windows with the wave-per-window kernel (TEAM_LONG, minBlocks >= 0)
+  // covers the (position, head) units of the order's first nPositions positions with a grid of its
+  // own size: thread t of workgroup b looks at unit b + t * gridDim.x, and the workgroup computes
   // the units it finds long, one after the other. When no window is long, which is the usual
-  // case on a graph of short windows, the launch is a thousand workgroups that read a count each
+  // case on a graph of short windows, the launch is a few hundred workgroups that read a count each
   // and leave, instead of one workgroup per unit; in a heavy-first order the long units are the
   // first ones and are dealt out round-robin.
-  const bool scan = !PERSIST && minBlocks >= 0;
   int nMine = 1;
-  if (scan) {
+  if constexpr (scan) {
     if (threadIdx.x == 0) sUnitCount = 0;
     __syncthreads();
     const int heads = HEADS ? nHeads : 1;
@@ -127,7 +150,7 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D)))) void 
   const int g = lane >> 4;
   const int c = lane & 15;
   for (int iter = 0;; iter++) {
-  if (scan) {
+  if constexpr (scan) {
     if (iter >= nMine) break;
     const int u = sUnitList[iter];
     pos = HEADS ? u / nHeads : u;
@@ -165,7 +188,7 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D)))) void 
   pb.nTcb = nTcb;
   pb.sddmm = sddmm;
   const unsigned ringAddr =
-      (unsigned)(uintptr_t)(F3S_LDS unsigned char*)smem + (unsigned)wave * pipe::Geo<D>::WAVE_BYTES;
+      (unsigned)(uintptr_t)(F3S_LDS unsigned char*)smem + (unsigned)wave * WAVE_BYTES;
   Pipe pp;
   pp.init(pb, w, ringAddr, head);
   {
@@ -231,11 +254,11 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D)))) void 
         acc.w += ov.w;
       }
     }
-    *reinterpret_cast<float4*>(out + row * pitchOut + head * D + cv * 4) = acc;
+    store_out(out + row * pitchOut + head * D + cv * 4, out_vec{acc.x, acc.y, acc.z, acc.w});
   }
   } while (false);
   if constexpr (!PERSIST) {
-    if (!scan) break;
+    if constexpr (!scan) break;
   }
   __syncthreads();  // the merge buffers are free again, the next position has arrived
   if constexpr (PERSIST) pos = sNextPos[iter & 1];
@@ -252,7 +275,7 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D)))) void 
   }
 }
 
-// LDS of a workgroup: its waves' rings; above 64 KiB the kernel has to be told
+// above 64 KiB of LDS the kernel has to be told
 template <typename KernelT>
 int allow_lds(KernelT kernel, size_t bytes) {
   if (bytes > 64 * 1024)
@@ -281,60 +304,64 @@ template <typename ET, int D, bool SOFTMAX, bool WIDE>
 int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, const uint64_t* bitmap,
              int N, const void* Q, const void* K, const void* V, float scaleLog2, float* out,
              unsigned long long* cuTimer, HeadLayout hl, hipStream_t stream) {
-  constexpr int NWAVES = 4;
   const int nRW = (N + kWinRows - 1) / kWinRows;
   if (nRW == 0) return 0;
   const auto* bm = reinterpret_cast<const uint8_t*>(bitmap);
   const auto* q = static_cast<const ET*>(Q);
   const auto* k = static_cast<const ET*>(K);
   const auto* v = static_cast<const ET*>(V);
-  const dim3 block(NWAVES * 64);
   const unsigned gw = (unsigned)(hl.gridWindows < nRW ? hl.gridWindows : nRW);
   if (gw == 0) return 0;
-  constexpr size_t lds = (size_t)NWAVES * pipe::Geo<D>::WAVE_BYTES;
-#define F3S_LAUNCH(CLOCKED_, HEADS_, GRID)                                                      \
-  {                                                                                             \
-    auto kernel = f3s_fwd_kernel<ET, D, NWAVES, SOFTMAX, CLOCKED_, HEADS_, false, WIDE>;        \
-    if (int rc = allow_lds(kernel, lds)) return rc;                                             \
-    hipLaunchKernelGGL(kernel, dim3(GRID), block, lds, stream, rwo, order, atox, bm, N, nRW,    \
-                       hl.nTcb, q, k, v, scaleLog2, out, cuTimer, hl.nHeads > 0 ? hl.nHeads : 1,\
-                       hl.nHeads > 0 ? hl.ldIn : D, hl.nHeads > 0 ? hl.ldOut : D,               \
-                       (float*)nullptr, hl.minBlocks, (int)gw);                                 \
+  const int heads = hl.nHeads > 0 ? hl.nHeads : 1;
+  const unsigned units = gw * (unsigned)heads;
+#define F3S_LAUNCH(TEAM_, CLOCKED_, HEADS_, GRID)                                              \
+  {                                                                                            \
+    auto kernel = f3s_fwd_kernel<ET, D, TEAM_, SOFTMAX, CLOCKED_, HEADS_, false, WIDE>;        \
+    constexpr size_t lds = team_lds(TEAM_, D);                                                 \
+    if (int rc = allow_lds(kernel, lds)) return rc;                                            \
+    hipLaunchKernelGGL(kernel, dim3(GRID), dim3(team_waves(TEAM_, D) * 64), lds, stream, rwo,  \
+                       order, atox, bm, N, nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer,     \
+                       heads, hl.nHeads > 0 ? hl.ldIn : D, hl.nHeads > 0 ? hl.ldOut : D,       \
+                       (float*)nullptr, hl.minBlocks, (int)gw);                                \
   }
-  // a launch next to the wave-per-window kernel looks for its units itself (see the kernel):
-  // 256 units per workgroup at most, 1024 workgroups when that is enough
-  const unsigned units = gw * (unsigned)(hl.nHeads > 0 ? hl.nHeads : 1);
-  unsigned scanGrid = (units + NWAVES * 64 - 1) / (NWAVES * 64);
-  if (scanGrid < 1024u) scanGrid = units < 1024u ? units : 1024u;
-  const bool scan = hl.minBlocks >= 0;
-  bool launched = false;
-  if constexpr (!WIDE) {
-    if (hl.nHeads == 0 && !cuTimer && hl.minBlocks < 0 && window_cursor_requested()) {
-      // F3S_WINDOW_PERSISTENT=1: as many workgroups as the GPU holds at once, windows drawn from
-      // a cursor (measured slower than launch order, which therefore stays the default)
-      auto kernel = f3s_fwd_kernel<ET, D, NWAVES, SOFTMAX, false, false, false, false, true>;
+  if (hl.minBlocks >= 0) {
+    // a launch next to the wave-per-window kernel looks for its units itself (see the kernel): one
+    // unit per thread at most, two workgroups per CU (one at a time) when that is enough
+    if constexpr (WIDE) {
+      return fail(-2, "f3s_attention: windows are not shared in the 64-bit form");
+    } else {
+      const unsigned threads = (unsigned)team_waves(TEAM_LONG, D) * 64;
+      unsigned grid = (units + threads - 1) / threads;
+      if (grid < 512u) grid = units < 512u ? units : 512u;
+      if (hl.nHeads > 0) F3S_LAUNCH(TEAM_LONG, false, true, grid)
+      else F3S_LAUNCH(TEAM_LONG, false, false, grid)
+    }
+  } else if (!WIDE && hl.nHeads == 0 && !cuTimer && window_cursor_requested()) {
+    // F3S_WINDOW_PERSISTENT=1: as many workgroups as the GPU holds at once, windows drawn from
+    // a cursor (measured slower than launch order, which therefore stays the default)
+    if constexpr (!WIDE) {
+      auto kernel = f3s_fwd_kernel<ET, D, TEAM_SHORT, SOFTMAX, false, false, false, false, true>;
+      constexpr size_t lds = team_lds(TEAM_SHORT, D);
+      constexpr int threads = team_waves(TEAM_SHORT, D) * 64;
       if (int rc = allow_lds(kernel, lds)) return rc;
       int dev = 0, nCu = 0, perCu = 0;
       F3S_HIP_CHECK(hipGetDevice(&dev));
       F3S_HIP_CHECK(hipDeviceGetAttribute(&nCu, hipDeviceAttributeMultiprocessorCount, dev));
       F3S_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &perCu, reinterpret_cast<const void*>(kernel), NWAVES * 64, lds));
+          &perCu, reinterpret_cast<const void*>(kernel), threads, lds));
       unsigned grid = (unsigned)(nCu * (perCu > 0 ? perCu : 1));
       if (grid > gw) grid = gw;
       hipLaunchKernelGGL(reset_window_cursor_kernel<0>, dim3(1), dim3(1), 0, stream);
-      hipLaunchKernelGGL(kernel, dim3(grid), block, lds, stream, rwo, order, atox, bm, N, nRW,
-                         hl.nTcb, q, k, v, scaleLog2, out, cuTimer, 1, D, D, (float*)nullptr,
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream, rwo, order, atox, bm, N,
+                         nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer, 1, D, D, (float*)nullptr,
                          hl.minBlocks, (int)gw);
-      launched = true;
     }
-  }
-  if (launched) {
   } else if (hl.nHeads > 0) {
-    F3S_LAUNCH(false, true, scan ? scanGrid : units)
+    F3S_LAUNCH(TEAM_SHORT, false, true, units)
   } else if (cuTimer) {
-    F3S_LAUNCH(true, false, scan ? scanGrid : gw)
+    F3S_LAUNCH(TEAM_SHORT, true, false, gw)
   } else {
-    F3S_LAUNCH(false, false, scan ? scanGrid : gw)
+    F3S_LAUNCH(TEAM_SHORT, false, false, gw)
   }
 #undef F3S_LAUNCH
   F3S_HIP_CHECK(hipGetLastError());
@@ -345,13 +372,12 @@ template <int D, bool SOFTMAX, bool WIDE>
 int launch_tcb8(const int32_t* rwo, const int32_t* order, const int32_t* atox,
                 const uint64_t* bitmap, int N, const void* Q, const void* K, const void* V,
                 float scaleLog2, float* out, float* sddmm, int64_t nTcb8, hipStream_t stream) {
-  constexpr int NWAVES = 4;
   const int nRW = (N + kWinRows - 1) / kWinRows;
   if (nRW == 0) return 0;
-  constexpr size_t lds = (size_t)NWAVES * pipe::Geo<D>::WAVE_BYTES;
-  auto kernel = f3s_fwd_kernel<_Float16, D, NWAVES, SOFTMAX, false, false, true, WIDE>;
+  constexpr size_t lds = team_lds(TEAM_SHORT, D);
+  auto kernel = f3s_fwd_kernel<_Float16, D, TEAM_SHORT, SOFTMAX, false, false, true, WIDE>;
   if (int rc = allow_lds(kernel, lds)) return rc;
-  hipLaunchKernelGGL(kernel, dim3(nRW), dim3(NWAVES * 64), lds, stream, rwo, order, atox,
+  hipLaunchKernelGGL(kernel, dim3(nRW), dim3(team_waves(TEAM_SHORT, D) * 64), lds, stream, rwo, order, atox,
                      reinterpret_cast<const uint8_t*>(bitmap), N, nRW, nTcb8,
                      static_cast<const _Float16*>(Q), static_cast<const _Float16*>(K),
                      static_cast<const _Float16*>(V), scaleLog2, out, nullptr, 1, D, D, sddmm, -1,
