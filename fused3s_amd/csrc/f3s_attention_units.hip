@@ -586,20 +586,35 @@ int allow_lds(KernelT kernel, size_t bytes) {
   return 0;
 }
 
-// Phases P (8 P slices of all heads). One slice's K + V rows are held to about 8 MiB: twice an XCD's
-// L2, which already catches 4 of 5 accesses on the 233k-node benchmark graph (P = 1), while more and
-// shorter units cost more than their higher hit rate returns (measured 1.54 / 1.69 / 1.86 ms at
-// P = 1 / 2 / 3). F3S_SLICE_PHASES in the environment overrides the choice.
+// How a column-sliced call's units are dealt to the XCDs: head groups (split_heads), then column
+// slices until a slice's K + V rows (of the group's heads) are at most 8 MiB: twice an XCD's L2,
+// which already catches 4 of 5 accesses on the 233k-node benchmark graph, while more and shorter
+// units cost more than their higher hit rate returns (measured 1.54 / 1.69 / 1.86 ms with 8 / 16 /
+// 24 slices there). XCDs left over share the windows.
+// F3S_SLICE_PHASES = P in the environment forces 8 P slices of all heads.
 XcdSplit choose_split(int N, int d, int heads) {
   const char* e = getenv("F3S_SLICE_PHASES");  // read per call: tests walk through the phases
   const int forced = e ? atoi(e) : 0;
   if (forced > 0) return {forced > kMaxPhases ? kMaxPhases : forced, kXcds, 1, 1, heads, 1};
-  const int64_t bytes = (int64_t)N * d * heads * 4;  // K + V
-  const int64_t perPhase = (int64_t)kXcds * 8 * 1024 * 1024;
-  int P = (int)((bytes + perPhase - 1) / perPhase);
-  if (P < 1) P = 1;
-  if (P > kMaxPhases) P = kMaxPhases;
-  return {P, kXcds, 1, 1, heads, 1};
+  XcdSplit s = split_heads(d, heads);
+  constexpr int64_t kSliceBytes = (int64_t)8 * 1024 * 1024;
+  const int64_t bytes = (int64_t)N * d * s.headsPerGroup * 4;  // K + V of a group's heads
+  int64_t need = (bytes + kSliceBytes - 1) / kSliceBytes;
+  if (need < 2) need = 2;  // one unit per window would be the windows themselves
+  // Slices one after the other keep all XCDs on the same columns at a time, which the memory side
+  // serves faster (100k nodes, 4 x 128: 1.77 -> 1.67 ms; 60k nodes, 4 x 64: 0.87 -> 0.82 ms), as
+  // long as a phase has units for two rounds of waves; with fewer the second phase's heavy windows
+  // start when the first phase's light ones should fill the end (60k nodes, d = 32: 188 -> 206 us).
+  const int64_t waves = 32 * 4 * unit_waves_per_simd(d, true);  // of one XCD
+  if (s.units((N + kWinRows - 1) / kWinRows) < 2 * waves) {
+    while (s.windowGroups > 1 && s.sliceGroups < need) {
+      s.sliceGroups *= 2;
+      s.windowGroups /= 2;
+    }
+  }
+  const int64_t phases = (need + s.sliceGroups - 1) / s.sliceGroups;
+  s.phases = phases > kMaxPhases ? kMaxPhases : (int)phases;
+  return s;
 }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }

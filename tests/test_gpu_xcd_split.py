@@ -1,0 +1,67 @@
+"""How units are dealt to the XCDs: head groups, slice groups, phases and window groups of the
+column-sliced schedule, and the chunks of the wave-per-window launches, at head counts and window
+counts that do not divide evenly. Every (window, head) has to be computed exactly once."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import random_csr
+
+pytestmark = pytest.mark.gpu
+
+
+def on_gpu(oracle_mod, rowPtr, colIdx, N):
+    pre = oracle_mod.preprocess(rowPtr, colIdx, N)
+    t = lambda k: torch.as_tensor(pre[k].astype(np.int32)).cuda()
+    bm = torch.as_tensor(pre["tcbBitMap"].view(np.int64)).cuda().view(torch.uint64)
+    return pre, (t("rowWindowOffset"), t("sortedRowWindows"), t("sparseAToXidx"), bm)
+
+
+def check(oracle_mod, pre, N, heads, d, Q, K, V, got):
+    got = got.cpu().numpy().reshape(N, heads, d)
+    for h in range(heads):
+        want = oracle_mod.attention_ref(pre["rowWindowOffset"], pre["sparseAToXidx"],
+                                        pre["tcbBitMap"], N, Q[:, h].contiguous().cpu().numpy(),
+                                        K[:, h].contiguous().cpu().numpy(),
+                                        V[:, h].contiguous().cpu().numpy(), float(np.sqrt(d)))
+        assert np.abs(got[:, h] - want).max() < 2e-2, h
+        assert np.abs(got[:, h] - want).mean() < 1e-3 * np.abs(want).mean(), h
+
+
+# (1, 64): window groups; (3, 32), (6, 64): heads that split once or not at all; (4, 64): head and
+# slice groups; (8, 64), (8, 128): one head per XCD and two phases
+@pytest.mark.parametrize("heads,d", [(1, 64), (3, 32), (6, 64), (4, 64), (8, 64), (8, 128)])
+@pytest.mark.parametrize("N", [17, 1003])
+def test_sliced(oracle_mod, monkeypatch, N, heads, d):
+    from fused3s_amd import capi
+    print("case sliced split N=%d heads=%d d=%d" % (N, heads, d), flush=True)
+    rng = np.random.default_rng(heads * d)
+    rowPtr, colIdx = random_csr(rng, N, 30, hub=37, empty_frac=0.05)
+    pre, (rwo, order, atox, bm) = on_gpu(oracle_mod, rowPtr, colIdx, N)
+    g = torch.Generator().manual_seed(d)
+    Q, K, V = [torch.randn((N, heads, d), generator=g).half().cuda() for _ in range(3)]
+    monkeypatch.setenv("F3S_SCHEDULE", "sliced")
+    ws = capi.attention_workspace(N, d, "cuda", heads=heads)
+    ws.fill_(0xFF)
+    got = capi.attention_heads(rwo, order, atox, bm, N, Q, K, V, float(np.sqrt(d)), workspace=ws)
+    check(oracle_mod, pre, N, heads, d, Q, K, V, got)
+
+
+# 1025 windows: one more than a whole number of chunks for every number of head groups
+@pytest.mark.parametrize("heads,d", [(1, 32), (3, 64), (4, 64), (8, 32), (2, 128)])
+def test_short_windows(oracle_mod, heads, d):
+    from fused3s_amd import capi
+    N = 16 * 1024 + 3
+    print("case short split heads=%d d=%d" % (heads, d), flush=True)
+    rng = np.random.default_rng(heads + d)
+    deg = rng.poisson(2.0, N)
+    deg[::1999] = 700  # windows for the team of waves
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(deg)
+    colIdx = np.concatenate([np.sort(rng.choice(N, size=k, replace=False)) for k in deg]
+                            ).astype(np.int32)
+    pre, (rwo, order, atox, bm) = on_gpu(oracle_mod, rowPtr, colIdx, N)
+    g = torch.Generator().manual_seed(d)
+    Q, K, V = [torch.randn((N, heads, d), generator=g).half().cuda() for _ in range(3)]
+    got = capi.attention_heads(rwo, order, atox, bm, N, Q, K, V, float(np.sqrt(d)))
+    check(oracle_mod, pre, N, heads, d, Q, K, V, got)
