@@ -4,11 +4,10 @@
 // a global thrust::sort of (window, column) pairs followed by two kernels that walk each
 // window with a single thread. Here a window never leaves its workgroup:
 //
-//   window_rank_radix_kernel / window_rank_small_kernel
-//                        windows of <= 1024 edges, one WAVE per window, no workgroup barrier.
-//                        Graphs of <= 2^22 nodes: stable LSD radix sort of (column, position)
-//                        words in LDS, ranks of the distinct columns scattered back to the
-//                        edges. Larger graphs: bitonic sort of the column ids, ballot / popcount
+//   window_rank_bins_kernel / window_rank_small_kernel
+//                        windows of <= 960 edges, one WAVE per window, no workgroup barrier.
+//                        Graphs of <= 2^22 nodes: (column, position) words sorted by bins of LDS
+//                        counters, ranks of the distinct columns back to the edges. Larger graphs: bitonic sort of the column ids, ballot / popcount
 //                        compaction of the distinct ones, rank by binary search.
 //   window_rank_kernel   larger windows, one workgroup per window. Column ids are OR-ed into an
 //                        LDS bitset (a column range per pass when N exceeds the LDS range), a
@@ -48,12 +47,13 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kRangeMax = 393216;  // columns per bitset pass: 48 KiB of bits + 12 KiB of prefixes
 constexpr int kSortMax = 1024;     // windows up to this many edges are ranked by a per-wave LDS sort
+constexpr int kBinsMax = 960;      // the same on graphs of at most 2^22 nodes (four workgroups per CU)
 // TC blocks held in LDS at once by window_fill_kernel: windows with strictly ascending rows (96
 // bytes of LDS per 16x16 block) and windows with repeated or descending columns (96 bytes as
 // well, but a second pass per chunk)
 constexpr int kFillChunk = 640;
 constexpr int kFillChunkGeneric = 512;
-constexpr int kFillChunkSmall = 128;  // both, for graphs of short windows (one wave each)
+constexpr int kFillChunkLong = 320;  // both, for the long windows of graphs of short ones
 
 // workspace header (bytes 0..255): int64 nTCB, int32 error flag, and the queue of windows too
 // long for the wave-per-window kernel (filled by window_rank_small_kernel, drained by
@@ -102,6 +102,12 @@ __device__ __forceinline__ unsigned wave_inclusive_scan(unsigned v, int /*lane*/
   return v;
 }
 
+// 16 bytes of an output that this call does not read again, past the caches
+__device__ __forceinline__ void store_streaming(uint4* p, const uint4& v) {
+  typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+  __builtin_nontemporal_store(uint4v{v.x, v.y, v.z, v.w}, reinterpret_cast<uint4v*>(p));
+}
+
 // largest r in [0,15] with sRow[r] <= e (sRow[0] <= e < sRow[16])
 __device__ __forceinline__ int row_of_edge(const int* sRow, int e) {
   int r = 0;
@@ -148,6 +154,39 @@ __device__ __forceinline__ void walk_tile_ids(const unsigned long long (&words)[
     while (x) {
       const int p = __builtin_clz(x);
       dst[pos++] = (uint8_t)(32 * q + p);
+      x &= ~(0x80000000u >> p);
+    }
+  }
+}
+
+// Tile ids (row * W + column of every set bit, rows top to bottom, columns left to right) of rows
+// 8 half .. 8 half + 7 of a TC block to dst[pos...]. left, right: those rows of the columns 0-7 and
+// 8-15 (W = 8: left only), MSB first. Brought into row-major order as dwords whose bit 31 - p stands
+// for tile id 8 W half + 32 q + p, two rows of 16 columns or four of 8 in each.
+template <int W>
+__device__ __forceinline__ void walk_half_block(unsigned long long left, unsigned long long right,
+                                                int half, uint8_t* dst, unsigned pos) {
+  constexpr int NQ = W / 4;
+  unsigned rm[NQ];
+  if constexpr (W == 16) {
+#pragma unroll
+    for (int k = 0; k < 2; k++) {  // four rows: the dword from the top
+      const unsigned a = k == 0 ? (unsigned)(left >> 32) : (unsigned)left;
+      const unsigned c = k == 0 ? (unsigned)(right >> 32) : (unsigned)right;
+      rm[2 * k] = __builtin_amdgcn_perm(a, c, 0x07030602u);      // rows +0, +1
+      rm[2 * k + 1] = __builtin_amdgcn_perm(a, c, 0x05010400u);  // rows +2, +3
+    }
+  } else {
+    rm[0] = (unsigned)(left >> 32);
+    rm[1] = (unsigned)left;
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; q++) {
+    unsigned x = rm[q];
+    const int id0 = 8 * W * half + 32 * q;
+    while (x) {
+      const int p = __builtin_clz(x);
+      dst[pos++] = (uint8_t)(id0 + p);
       x &= ~(0x80000000u >> p);
     }
   }
@@ -309,57 +348,11 @@ __device__ __forceinline__ void wave_scatter_in_order(const uint32_t* src, uint3
   }
 }
 
-// The same job for graphs of at most 2^22 nodes, where a column id and the edge's position in
-// the window (< kSortMax = 2^10) fit one 32-bit word: a stable LSD radix sort of those words on
-// the column bits, eight bits per pass, in the wave's LDS slice (histogram with LDS atomics,
-// in-order scatter with wave ballots). The sorted words carry the edge positions along, so the
-// rank of every distinct column is scattered straight back to its edges: no binary search, and
-// a third of the instructions of the bitonic network.
-template <int W>
-__global__ __launch_bounds__(kBlock) void window_rank_radix_kernel(
-    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
-    int colBits, int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
-    int32_t* __restrict__ edgeToRow, WsHeader* __restrict__ hdr, LongQueues queues) {
-  constexpr int WAVES = kBlock / 64;
-  constexpr int IDX_BITS = 10;
-  static_assert(kSortMax <= (1 << IDX_BITS), "edge position must fit IDX_BITS");
-  __shared__ uint32_t sBufA[WAVES][kSortMax];
-  __shared__ uint32_t sBufB[WAVES][kSortMax];
-  __shared__ __align__(16) uint32_t sHist[WAVES][256];
-  __shared__ int sRowW[WAVES][17];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int w = blockIdx.x * WAVES + wave;
-  if (w >= nRW) return;
-  const int r0 = w * 16;
-  int* sRow = sRowW[wave];
-  if (lane < 17) sRow[lane] = rowPtr[min(r0 + lane, N)];
-  wave_lds_sync();
-  const int eS = sRow[0], eE = sRow[16];
-  const int n = eE - eS;
-  if (n == 0) {
-    if (lane == 0) blockPartition[w] = 0;
-    return;
-  }
-  if (n > kSortMax) {  // left to window_rank_kernel, through the queue if there is one
-    if (lane == 0) queue_long_window(queues, hdr, w, n);
-    return;
-  }
-  uint32_t* src = sBufA[wave];
-  uint32_t* dst = sBufB[wave];
-  uint32_t* hist = sHist[wave];
-  const unsigned long long ltMask = (1ull << lane) - 1ull;
-  bool bad = false;
-  for (int i = lane; i < n; i += 64) {
-    uint32_t col = (uint32_t)colIdx[eS + i];
-    if (col >= (uint32_t)N) {
-      bad = true;
-      col = 0;
-    }
-    src[i] = (col << IDX_BITS) | (uint32_t)i;
-    edgeToRow[eS + i] = r0 + row_of_edge(sRow, eS + i);
-  }
-  if (bad) atomicOr(&hdr->error, 1);
+// LSD radix sort of a wave's n words by the colBits bits above IDX_BITS, in LDS: from src through dst
+// and back; returns the buffer that holds the result. hist: 256 counters.
+template <int IDX_BITS>
+__device__ __forceinline__ uint32_t* wave_radix_sort(uint32_t* src, uint32_t* dst, uint32_t* hist,
+                                                     int n, int colBits, int lane) {
   // Digits: the first pass takes eight bits, the stable passes share the rest evenly (22 column
   // bits: 8 + 7 + 7; 18: 8 + 5 + 5), so that a stable pass spends one ballot per bit it needs.
   const int firstBits = colBits < 8 ? colBits : 8;
@@ -411,18 +404,237 @@ __global__ __launch_bounds__(kBlock) void window_rank_radix_kernel(
     dst = t;
     shift += db;
   }
-  // ranks of the distinct columns, scattered to their edges
-  int nUniq = 0;
-  for (int base = 0; base < n; base += 64) {
-    const int i = base + lane;
-    const bool valid = i < n;
-    const uint32_t key = valid ? src[i] : 0u;
-    const bool first = valid && (i == 0 || (src[i - 1] >> IDX_BITS) != (key >> IDX_BITS));
-    const unsigned long long bal = __ballot(first);
-    if (valid)
-      edgeToColumn[eS + (int)(key & ((1u << IDX_BITS) - 1u))] =
-          nUniq + __popcll(bal & (ltMask | (1ull << lane))) - 1;
-    nUniq += __popcll(bal);
+  return src;
+}
+
+// Rows of the edges of a window of at most MAX edges, for one wave that walks the edges in groups of
+// 64. mark: MAX / 32 + 2 words of LDS, 8-byte aligned; bit i is set where a row that is not empty
+// starts at edge i, and nibble k of the last two words names the k-th such row: two instructions
+// count the marks up to a lane, where a search of the row pointers is four dependent LDS reads.
+template <int MAX>
+struct EdgeRows {
+  const uint32_t* mark;
+  unsigned long long names;
+  int rows;  // rows in front of the next group
+
+  // rowStart: lane r holds row r's first edge (from the window's first one), lane 16 their number
+  __device__ __forceinline__ void init(uint32_t* words, int rowStart, int lane) {
+    static_assert(MAX % 64 == 0, "the row names are read as one 64-bit word");
+    if (lane < MAX / 32 + 2) words[lane] = 0u;
+    wave_lds_sync();
+    const int next = __shfl_down(rowStart, 1);
+    const unsigned filled = (unsigned)__ballot(lane < 16 && next > rowStart);
+    if (lane < 16 && ((filled >> lane) & 1u)) {
+      const int k = __popc(filled & ((1u << lane) - 1u));
+      atomicOr(&words[rowStart >> 5], 1u << (rowStart & 31));
+      atomicOr(&words[MAX / 32 + (k >> 3)], (uint32_t)lane << (4 * (k & 7)));
+    }
+    wave_lds_sync();
+    mark = words;
+    names = *reinterpret_cast<const unsigned long long*>(words + MAX / 32);
+    rows = 0;
+  }
+  // row of this lane's edge in the group of 64 from `base` on (groups in order, each once), and
+  // whether the edge is the first of its row
+  __device__ __forceinline__ int next_group(int base, int lane, bool* starts) {
+    const uint2 m = *reinterpret_cast<const uint2*>(mark + (base >> 5));
+    const bool own = (((lane < 32 ? m.x : m.y) >> (lane & 31)) & 1u) != 0u;
+    const int k = rows + (int)__builtin_amdgcn_mbcnt_hi(m.y, __builtin_amdgcn_mbcnt_lo(m.x, 0));
+    rows += __popc(m.x) + __popc(m.y);
+    *starts = own;
+    return (int)(names >> (4 * (k - (own ? 0 : 1)))) & 15;
+  }
+};
+
+// The same job for graphs of at most 2^22 nodes, where a column id and the edge's position in the
+// window (< kBinsMax) fit one 32-bit word. The columns' top ten bits spread the window's
+// edges over 1024 bins (two 16-bit counters per word; one counting pass, one that hands out
+// places), after which an edge shares its bin with one or two others and finds its place by
+// counting the smaller ones. The sorted words carry the edge positions along, so that the rank of
+// every distinct column goes straight back to its edges. A window whose columns crowd into few bins
+// (communities) is sorted by an LSD radix sort of the column bits, whose stable passes cost a
+// ballot per bit: counting the smaller ones takes as many steps as the fullest bin holds.
+//
+// Bound by the issue of vector instructions (a wave of 400 edges is 7 groups of 64), then by LDS
+// latency: the LDS accesses of four groups are in flight together. Four workgroups per CU.
+constexpr int kRankBins = 1024;
+constexpr int kRankCrowd = 24;  // a fuller bin sends the window to the radix sort
+template <int W>
+__global__ __launch_bounds__(kBlock) void window_rank_bins_kernel(
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
+    int colBits, int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
+    int32_t* __restrict__ edgeToRow, WsHeader* __restrict__ hdr, LongQueues queues) {
+  constexpr int WAVES = kBlock / 64;
+  constexpr int IDX_BITS = 10;
+  constexpr int U = 4;  // groups of 64 edges whose LDS accesses are in flight together
+  static_assert(kBinsMax <= (1 << IDX_BITS), "edge position must fit IDX_BITS");
+  __shared__ uint32_t sBufA[WAVES][kBinsMax];
+  __shared__ uint32_t sBufB[WAVES][kBinsMax];
+  __shared__ __align__(16) uint32_t sHist[WAVES][kRankBins / 2];
+  __shared__ __align__(8) uint32_t sMark[WAVES][kBinsMax / 32 + 2];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = blockIdx.x * WAVES + wave;
+  if (w >= nRW) return;
+  const int r0 = w * 16;
+  int rowStart = rowPtr[min(r0 + min(lane, 16), N)];
+  const int eS = __builtin_amdgcn_readlane(rowStart, 0);
+  const int n = __builtin_amdgcn_readlane(rowStart, 16) - eS;
+  rowStart -= eS;
+  if (n == 0) {
+    if (lane == 0) blockPartition[w] = 0;
+    return;
+  }
+  if (n > kBinsMax) {  // left to another kernel, through the queue if there is one
+    if (lane == 0) queue_long_window(queues, hdr, w, n);
+    return;
+  }
+  uint32_t* a = sBufA[wave];
+  uint32_t* b = sBufB[wave];
+  uint32_t* hist = sHist[wave];
+  const unsigned long long leMask = (2ull << lane) - 1ull;
+  const int shift = colBits > 10 ? colBits - 10 : 0;
+  EdgeRows<kBinsMax> edgeRows;
+  edgeRows.init(sMark[wave], rowStart, lane);
+#pragma unroll
+  for (int k = 0; k < kRankBins / 2 / 256; k++)
+    reinterpret_cast<uint4*>(hist)[lane + 64 * k] = make_uint4(0, 0, 0, 0);
+  wave_lds_sync();
+  // ---- rows, and how many edges fall into each bin
+  bool bad = false;
+  for (int base = 0; base < n; base += 64 * U) {
+    uint32_t col[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = base + 64 * u + lane;
+      col[u] = i < n ? (uint32_t)colIdx[eS + i] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (base + 64 * u >= n) break;
+      const int i = base + 64 * u + lane;
+      bool starts;
+      const int row = edgeRows.next_group(base + 64 * u, lane, &starts);
+      if (i < n) {
+        if (col[u] >= (uint32_t)N) {
+          bad = true;
+          col[u] = 0;
+        }
+        edgeToRow[eS + i] = r0 + row;
+        b[i] = col[u];
+        const uint32_t bin = col[u] >> shift;
+        atomicAdd(&hist[bin >> 1], 1u << ((bin & 1u) * 16u));
+      }
+    }
+  }
+  if (bad) atomicOr(&hdr->error, 1);
+  wave_lds_sync();
+  // ---- where each bin starts: lane l owns bins 16 l .. 16 l + 15
+  bool crowded;
+  {
+    uint4* h = reinterpret_cast<uint4*>(hist) + 2 * lane;
+    const uint4 x = h[0], y = h[1];
+    uint32_t v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+    // both counters of a word at once: no sum reaches 2^16
+    uint32_t most = 0, pairs = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      pairs += v[k];
+      most |= v[k] + 0x10001u * (0x7FFFu - kRankCrowd);  // bit 15 of a half: more than kRankCrowd
+    }
+    crowded = __ballot((most & 0x80008000u) != 0u) != 0ull;
+    const uint32_t total = (pairs & 0xFFFFu) + (pairs >> 16);
+    uint32_t run = wave_inclusive_scan(total, lane) - total;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const uint32_t lo = run + (v[k] & 0xFFFFu);
+      const uint32_t start = run | (lo << 16);
+      run = lo + (v[k] >> 16);
+      v[k] = start;
+    }
+    if (!crowded) {
+      h[0] = make_uint4(v[0], v[1], v[2], v[3]);
+      h[1] = make_uint4(v[4], v[5], v[6], v[7]);
+    }
+  }
+  wave_lds_sync();
+  const uint32_t* sorted = b;
+  if (!crowded) {
+    // ---- into the bins; afterwards hist[bin] is where the bin ends
+    for (int base = 0; base < n; base += 64 * U) {
+      uint32_t col[U], old[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) col[u] = b[min(base + 64 * u + lane, n - 1)];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const uint32_t bin = col[u] >> shift;
+        if (base + 64 * u + lane < n)
+          old[u] = atomicAdd(&hist[bin >> 1], 1u << ((bin & 1u) * 16u));
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int i = base + 64 * u + lane;
+        const uint32_t bin = col[u] >> shift;
+        if (i < n)
+          a[(old[u] >> ((bin & 1u) * 16u)) & 0xFFFFu] = (col[u] << IDX_BITS) | (uint32_t)i;
+      }
+    }
+    wave_lds_sync();
+    // ---- each edge's place inside its bin
+    const uint16_t* binEnd = reinterpret_cast<const uint16_t*>(hist);
+    for (int base = 0; base < n; base += 64 * U) {
+      uint32_t key[U];
+      int end[U], q[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) key[u] = a[min(base + 64 * u + lane, n - 1)];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const uint32_t bin = key[u] >> (IDX_BITS + shift);
+        end[u] = binEnd[bin];
+        q[u] = bin == 0u ? 0 : (int)binEnd[max(bin, 1u) - 1u];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (base + 64 * u >= n) break;
+        int at = q[u];
+        if (end[u] - q[u] > 1)
+          for (int k = q[u]; k < end[u]; k++) at += a[k] < key[u] ? 1 : 0;
+        if (base + 64 * u + lane < n) b[at] = key[u];
+      }
+    }
+  } else {
+    for (int i = lane; i < n; i += 64) a[i] = (b[i] << IDX_BITS) | (uint32_t)i;
+    wave_lds_sync();
+    sorted = wave_radix_sort<IDX_BITS>(a, b, hist, n, colBits, lane);
+  }
+  wave_lds_sync();
+  // ---- ranks of the distinct columns, collected in edge order and written as whole lines
+  uint32_t* rankOf = sorted == b ? a : b;
+  int nUniq = 0, lastCol = -1;
+  for (int base = 0; base < n; base += 64 * U) {
+    uint32_t key[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) key[u] = sorted[min(base + 64 * u + lane, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (base + 64 * u >= n) break;
+      const bool valid = base + 64 * u + lane < n;
+      const int col = (int)(key[u] >> IDX_BITS);
+      const int left = __builtin_amdgcn_update_dpp(lastCol, col, 0x138, 0xf, 0xf, false);
+      lastCol = __builtin_amdgcn_readlane(col, 63);
+      const unsigned long long bal = __ballot(valid && left != col);
+      if (valid)
+        rankOf[key[u] & ((1u << IDX_BITS) - 1u)] = (uint32_t)(nUniq + __popcll(bal & leMask) - 1);
+      nUniq += __popcll(bal);
+    }
+  }
+  wave_lds_sync();
+  for (int base = 0; base < n; base += 64 * U) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = base + 64 * u + lane;
+      if (i < n) edgeToColumn[eS + i] = (int)rankOf[i];
+    }
   }
   if (lane == 0) blockPartition[w] = (nUniq + W - 1) / W;
 }
@@ -433,7 +645,7 @@ __global__ __launch_bounds__(TB) void window_rank_kernel(
     int nPasses, int32_t* __restrict__ blockPartition,
     int32_t* __restrict__ edgeToColumn,
     int32_t* __restrict__ edgeToRow, WsHeader* __restrict__ hdr,
-    const int32_t* __restrict__ bigList) {
+    const int32_t* __restrict__ bigList, int shortMax) {
   extern __shared__ __align__(16) uint32_t smem[];
   uint32_t* bits = smem;                 // range/32 words
   uint32_t* pref = smem + (range >> 5);  // range/128 group prefixes
@@ -460,7 +672,7 @@ __global__ __launch_bounds__(TB) void window_rank_kernel(
   if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
   __syncthreads();
   const int eS = sRow[0], eE = sRow[16];
-  if (!bigList && eE - eS <= kSortMax) break;  // ranked by window_rank_small_kernel
+  if (!bigList && eE - eS <= shortMax) break;  // ranked by one wave
   const int nGroups = range >> 7;
   unsigned uniqueBefore = 0;
   for (int pass = 0; pass < nPasses; pass++) {
@@ -542,11 +754,11 @@ __global__ __launch_bounds__(TB) void window_rank_kernel(
   }
 }
 
-// Windows of kSortMax < edges <= kMedMax on graphs whose column range needs several bitset passes
+// Windows of kBinsMax (kSortMax) < edges <= kMedMax on graphs whose column range needs several bitset passes
 // (N > kRangeMax): one workgroup per queued window sorts the window's column ids, compacts the
 // distinct ones and ranks every edge by binary search, instead of several passes over a 48 KiB
 // bitset that such a window fills with a few thousand bits. The sort is the wave-level LSD radix
-// sort of window_rank_radix_kernel widened to a workgroup: eight bits per pass, every wave on its
+// sort of wave_radix_sort widened to a workgroup: eight bits per pass, every wave on its
 // own contiguous quarter of the keys (histogram with LDS atomics, one thread per digit turns the
 // per-wave counts into start positions, in-order scatter with wave ballots), two LDS buffers.
 // Two sizes: windows of up to kMedMax edges (256 threads, 32 KiB of buffers, four workgroups per
@@ -1280,8 +1492,7 @@ __device__ __forceinline__ void fill_one_window(
     int E, const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
     const WsHeader* __restrict__ hdr, int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
-    int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap, int minBlocks,
-    int maxBlocks) {
+    int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
   constexpr int WPT = 16 * W / 64;  // bitmap words per TC block
   constexpr int LOGW = (W == 16) ? 4 : 3;
   constexpr int FAST_BYTES = TC * (WPT * 8 + W * 4);
@@ -1304,8 +1515,7 @@ __device__ __forceinline__ void fill_one_window(
   if (w == 0 && tid == 0) tcblockOffset[rowWindowOffset[nRW]] = E;
   const int base = rowWindowOffset[w];
   const int nb = rowWindowOffset[w + 1] - base;
-  // a launch may be one of two that share the windows by length: [minBlocks, maxBlocks]
-  if (nb == 0 || nb < minBlocks || nb > maxBlocks) return;
+  if (nb == 0) return;
   const int r0 = w * 16;
   if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
   __syncthreads();
@@ -1428,48 +1638,224 @@ __device__ __forceinline__ void fill_one_window(
   }
 }
 
+// Windows of at most kBinsMax edges: one wave per window, everything in its LDS slice. Every edge sets
+// its bit in the window's bitmaps and drops its column into the ids; two lanes per TC block then walk
+// the set bits row by row (a block of a sparse graph has 17, most of a walk's time is the fullest
+// dword among the lanes), and bitmaps, ids and tile ids leave as whole words. Bound by the issue of
+// vector instructions; five workgroups of four waves per CU.
+constexpr int kFillWaves = 4;
+template <int W>
+__global__ __launch_bounds__(kFillWaves * 64) void window_fill_short_kernel(
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
+    const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
+    const WsHeader* __restrict__ hdr, int32_t* __restrict__ tcblockRowid,
+    uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
+    int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
+  constexpr int WPT = 16 * W / 64;
+  constexpr int LOGW = (W == 16) ? 4 : 3;
+  constexpr int MAXB = (kBinsMax + W - 1) / W;  // TC blocks of a window at most
+  constexpr int U = 4;  // groups of 64 edges in flight together
+  __shared__ __align__(16) unsigned long long sBm[kFillWaves][MAXB * WPT];
+  __shared__ __align__(16) uint32_t sIds[kFillWaves][MAXB * W];
+  __shared__ __align__(16) uint8_t sTile[kFillWaves][kBinsMax + 8];
+  __shared__ __align__(8) uint32_t sMark[kFillWaves][kBinsMax / 32 + 2];
+  static_assert(MAXB * 8 <= MAXB * W, "edges per (block, row), two counters per word, fit sIds");
+  if (hdr && hdr->error) return;  // edgeToColumn is incomplete
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = blockIdx.x * kFillWaves + wave;
+  if (w >= nRW) return;
+  int rowStart = rowPtr[min(w * 16 + min(lane, 16), N)];
+  const int base = __builtin_amdgcn_readfirstlane(rowWindowOffset[w]);
+  const int nb = __builtin_amdgcn_readfirstlane(rowWindowOffset[w + 1]) - base;
+  const int eS = __builtin_amdgcn_readlane(rowStart, 0);
+  const int n = __builtin_amdgcn_readlane(rowStart, 16) - eS;
+  rowStart -= eS;
+  if (w == nRW - 1 && lane == 0) tcblockOffset[base + nb] = E;
+  if (n == 0 || n > kBinsMax || nb > MAXB) return;  // long ones: window_fill_long_kernel
+  unsigned long long* bm = sBm[wave];
+  uint32_t* ids = sIds[wave];
+  EdgeRows<kBinsMax> edgeRows;
+  edgeRows.init(sMark[wave], rowStart, lane);
+  for (int i = lane; i < nb * WPT / 2; i += 64)
+    reinterpret_cast<uint4*>(bm)[i] = make_uint4(0, 0, 0, 0);
+  for (int i = nb * W - W + lane; i < nb * W; i += 64) ids[i] = 0u;  // unused slots hold 0
+  wave_lds_sync();
+  bool rough = false;  // some row's columns do not strictly ascend
+  int before = -1;
+  for (int e0 = 0; e0 < n; e0 += 64 * U) {
+    int rank[U], col[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = min(e0 + 64 * u + lane, n - 1);
+      rank[u] = edgeToColumn[eS + i];
+      col[u] = colIdx[eS + i];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (e0 + 64 * u >= n) break;
+      bool starts;
+      const int row = edgeRows.next_group(e0 + 64 * u, lane, &starts);
+      const int left = __builtin_amdgcn_update_dpp(before, col[u], 0x138, 0xf, 0xf, false);
+      before = __builtin_amdgcn_readlane(col[u], 63);
+      if (e0 + 64 * u + lane < n && (unsigned)rank[u] < (unsigned)(nb * W)) {
+        rough = rough || (!starts && left >= col[u]);
+        ids[rank[u]] = (uint32_t)col[u];
+        // word and bit of (rank, row): see window_rank_fill_kernel
+        const int byte = 7 - (row & 7);
+        atomicOr(&reinterpret_cast<unsigned*>(bm)[(rank[u] >> 3) * 4 + (row >> 3) * 2 + (byte >> 2)],
+                 (0x80u << (8 * (byte & 3))) >> (rank[u] & 7));
+      }
+    }
+  }
+  wave_lds_sync();
+  for (int i = lane; i < nb * WPT / 2; i += 64)
+    store_streaming(reinterpret_cast<uint4*>(bitmap + (int64_t)base * WPT) + i,
+                    reinterpret_cast<const uint4*>(bm)[i]);
+  for (int i = lane; i < nb * W / 4; i += 64)
+    store_streaming(reinterpret_cast<uint4*>(sparseAToXidx + (int64_t)base * W) + i,
+                    reinterpret_cast<const uint4*>(ids)[i]);
+  if (__ballot(rough) == 0ull) {
+    uint8_t* stage = sTile[wave];
+    const unsigned skew = (unsigned)((uintptr_t)(tcblocktileId + eS) & 3u);
+    unsigned carry = 0;
+    for (int k = 0; k < 2 * nb; k += 64) {
+      const int t = (k + lane) >> 1, half = lane & 1;
+      unsigned long long left = 0, right = 0;
+      if (t < nb) {
+        left = bm[t * WPT + half];
+        if constexpr (W == 16) right = bm[t * WPT + 2 + half];
+      }
+      const unsigned nnz = __popcll(left) + __popcll(right);
+      const unsigned incl = wave_inclusive_scan(nnz, lane);
+      const unsigned at = carry + incl - nnz;
+      carry += (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
+      if (t < nb && half == 0) {
+        tcblockOffset[base + t] = eS + (int)at;
+        tcblockRowid[base + t] = w;
+      }
+      walk_half_block<W>(left, right, half, stage, at + skew);
+    }
+    wave_lds_sync();
+    uint8_t* dst = tcblocktileId + eS - skew;  // the dword that holds the window's first tile id
+    const int end = n + (int)skew;
+    for (int i = 4 * lane; i < end; i += 256) {
+      if (i >= (int)skew && i + 4 <= end) {
+        *reinterpret_cast<uint32_t*>(dst + i) = *reinterpret_cast<const uint32_t*>(stage + i);
+      } else {
+        for (int j = 0; j < 4; j++)
+          if (i + j >= (int)skew && i + j < end) dst[i + j] = stage[i + j];
+      }
+    }
+    return;
+  }
+  // Repeated or descending columns: tile ids sit in edge order inside a block. The edges of every
+  // (block, row) are counted (two 16-bit counters per word, where the ids were), the counts turned
+  // into places and the rows replayed in order (src/utils.cu:173-224).
+  uint32_t* cnt = ids;
+  wave_lds_sync();
+  for (int i = lane; i < nb * 8; i += 64) cnt[i] = 0u;
+  wave_lds_sync();
+  edgeRows.rows = 0;
+  for (int e0 = 0; e0 < n; e0 += 64) {
+    bool starts;
+    const int row = edgeRows.next_group(e0, lane, &starts);
+    if (e0 + lane < n) {
+      const int c = (edgeToColumn[eS + e0 + lane] >> LOGW) * 16 + row;
+      atomicAdd(&cnt[c >> 1], 1u << ((c & 1) * 16));
+    }
+  }
+  wave_lds_sync();
+  unsigned carry = 0;
+  for (int k = 0; k < nb; k += 64) {
+    const int t = k + lane;
+    unsigned nnz = 0;
+    for (int q = 0; q < 8; q++) {
+      const uint32_t v = t < nb ? cnt[t * 8 + q] : 0u;
+      nnz += (v & 0xFFFFu) + (v >> 16);
+    }
+    const unsigned incl = wave_inclusive_scan(nnz, lane);
+    unsigned run = carry + incl - nnz;
+    carry += (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
+    if (t < nb) {
+      tcblockOffset[base + t] = eS + (int)run;
+      tcblockRowid[base + t] = w;
+      for (int q = 0; q < 8; q++) {
+        const uint32_t v = cnt[t * 8 + q], lo = run + (v & 0xFFFFu);
+        cnt[t * 8 + q] = run | (lo << 16);
+        run = lo + (v >> 16);
+      }
+    }
+  }
+  wave_lds_sync();
+  const unsigned long long ltMask = (1ull << lane) - 1ull;
+  for (int row = 0; row < 16; row++) {
+    const int rs = __builtin_amdgcn_readlane(rowStart, row);
+    const int re = __builtin_amdgcn_readlane(rowStart, row + 1);
+    for (int e0 = rs; e0 < re; e0 += 64) {
+      const bool valid = e0 + lane < re;
+      const int rank = valid ? edgeToColumn[eS + e0 + lane] : 0;
+      const int t = rank >> LOGW;
+      unsigned long long peers = __ballot(valid);  // lanes whose edges fall into the same block
+      for (int bit = 0; (MAXB >> bit) != 0; bit++) {
+        const unsigned long long bal = __ballot((t >> bit) & 1);
+        peers &= ((t >> bit) & 1) ? bal : ~bal;
+      }
+      const int c = t * 16 + row, sh = (c & 1) * 16;
+      if (valid)
+        tcblocktileId[eS + ((cnt[c >> 1] >> sh) & 0xFFFFu) + __popcll(peers & ltMask)] =
+            (uint8_t)(row * W + (rank & (W - 1)));
+      wave_lds_sync();
+      // the row's blocks have a word each: the last lane of a block moves its counter
+      if (valid && (peers >> lane) == 1ull)
+        atomicAdd(&cnt[c >> 1], (uint32_t)__popcll(peers) << sh);
+      wave_lds_sync();
+    }
+  }
+}
+
 template <int W, int TB, int TC, int TCG>
 __global__ __launch_bounds__(TB) void window_fill_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E,
     const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
     const WsHeader* __restrict__ hdr, int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
-    int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap, int minBlocks,
-    int maxBlocks) {
+    int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
   fill_one_window<W, TB, TC, TCG>((int)blockIdx.x, (int)gridDim.x, rowPtr, colIdx, N, E,
                                   edgeToColumn, rowWindowOffset, hdr, tcblockRowid, tcblocktileId,
-                                  tcblockOffset, sparseAToXidx, bitmap, minBlocks, maxBlocks);
+                                  tcblockOffset, sparseAToXidx, bitmap);
 }
 
-// The few long windows of a graph of short ones (more than minBlocks - 1 TC blocks): a grid of a
-// few hundred workgroups looks through the block counts, 256 windows at a time per workgroup,
-// and fills the long ones it finds one after the other. One workgroup per window, as
-// window_fill_kernel has it, would start a hundred thousand workgroups of 60 KiB of LDS each to
-// find that nearly all of them have nothing to do.
+// The windows that window_fill_short_kernel leaves out: thread t of workgroup b looks at window
+// b + t * gridDim.x (and so on), and the workgroup fills the long ones it finds one after the other,
+// so that long windows are dealt out evenly wherever they lie. One workgroup per window instead
+// would start a hundred thousand workgroups of 30 KiB of LDS each to find that nearly all of them
+// have nothing to do. 320 TC blocks of LDS at a time: five workgroups per CU.
 template <int W, int TB, int TC, int TCG>
 __global__ __launch_bounds__(TB) void window_fill_long_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
     const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
     const WsHeader* __restrict__ hdr, int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
-    int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap, int minBlocks) {
-  static_assert(TB == 256, "one candidate window per thread and round");
+    int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
   __shared__ int sList[TB];
   __shared__ int sListLen;
-  for (int base = (int)blockIdx.x * TB; base < nRW; base += (int)gridDim.x * TB) {
-    __syncthreads();  // the list of the 256 windows before these has been worked through
+  const int stride = (int)gridDim.x;
+  for (int64_t first = blockIdx.x; first < nRW; first += (int64_t)TB * stride) {
+    __syncthreads();  // the list before this one has been worked through
     if (threadIdx.x == 0) sListLen = 0;
     __syncthreads();
-    const int w = base + (int)threadIdx.x;
-    if (w < nRW && rowWindowOffset[w + 1] - rowWindowOffset[w] >= minBlocks)
-      sList[atomicAdd(&sListLen, 1)] = w;
+    const int64_t w = first + (int64_t)threadIdx.x * stride;
+    if (w < nRW &&
+        rowPtr[min((int)w * 16 + 16, N)] - rowPtr[(int)w * 16] > kBinsMax)
+      sList[atomicAdd(&sListLen, 1)] = (int)w;
     __syncthreads();
     const int len = sListLen;
     for (int k = 0; k < len; k++) {
       __syncthreads();  // the window before this one has left the LDS arrays
       fill_one_window<W, TB, TC, TCG>(sList[k], nRW, rowPtr, colIdx, N, E, edgeToColumn,
                                       rowWindowOffset, hdr, tcblockRowid, tcblocktileId,
-                                      tcblockOffset, sparseAToXidx, bitmap, minBlocks, 0x7FFFFFFF);
+                                      tcblockOffset, sparseAToXidx, bitmap);
     }
   }
 }
@@ -1934,6 +2320,9 @@ size_t preprocess_workspace_bytes(int N, int /*E*/) {
 
 namespace {
 
+// long windows on average: a workgroup per window instead of a wave
+bool long_windows(int nRW, int64_t E) { return E >= (int64_t)nRW * 2048; }
+
 // Scan of the block counts and the window order, after the kernels that write blockPartition.
 int enqueue_finalize(int N, int W, const int32_t* blockPartition, int32_t* rowWindowOffset,
                      int32_t* sortedRowWindows, char* ws, hipStream_t stream) {
@@ -1998,7 +2387,7 @@ int enqueue_count(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, in
     const int nPasses = (N + range - 1) / range;
     const size_t lds = (size_t)(range / 32 + range / 128) * sizeof(uint32_t);
     const int smallGrid = (nRW + kBlock / 64 - 1) / (kBlock / 64);
-    const bool big = (int64_t)E >= (int64_t)nRW * 2048;  // long windows on average
+    const bool big = long_windows(nRW, E);
     int32_t* queue = big ? nullptr : valsTmp;
     // queued windows of a few thousand edges on a graph that needs several bitset passes are
     // sorted (window_rank_sort_kernel) instead of walking every pass; the others go to the
@@ -2012,11 +2401,11 @@ int enqueue_count(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, in
     while (colBits < 31 && ((int64_t)1 << colBits) < (int64_t)N) colBits++;
     if (colBits <= 22) {
       if (W == 16)
-        hipLaunchKernelGGL(window_rank_radix_kernel<16>, dim3(smallGrid), dim3(kBlock), 0, stream,
+        hipLaunchKernelGGL(window_rank_bins_kernel<16>, dim3(smallGrid), dim3(kBlock), 0, stream,
                            rowPtr, colIdx, N, nRW, colBits, blockPartition, edgeToColumn,
                            edgeToRow, hdr, queues);
       else
-        hipLaunchKernelGGL(window_rank_radix_kernel<8>, dim3(smallGrid), dim3(kBlock), 0, stream,
+        hipLaunchKernelGGL(window_rank_bins_kernel<8>, dim3(smallGrid), dim3(kBlock), 0, stream,
                            rowPtr, colIdx, N, nRW, colBits, blockPartition, edgeToColumn,
                            edgeToRow, hdr, queues);
     } else if (W == 16) {
@@ -2058,7 +2447,7 @@ int enqueue_count(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, in
 #define F3S_RANK(WW, TBB)                                                                     \
   hipLaunchKernelGGL((window_rank_kernel<WW, TBB>), dim3(rankGrid), dim3(TBB), lds, stream,   \
                      rowPtr, colIdx, N, range, nPasses, blockPartition,                       \
-                     edgeToColumn, edgeToRow, hdr, queue)
+                     edgeToColumn, edgeToRow, hdr, queue, colBits <= 22 ? kBinsMax : kSortMax)
     // the queue lives in the buffer finalize_count_kernel later uses for its values and is
     // drained by at most two workgroups per CU (2048 of them took 25 us to find an empty queue)
     const int rankGrid = big ? nRW : (nRW < 512 ? nRW : 512);
@@ -2174,41 +2563,30 @@ int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int
                  int32_t* sparseAToXidx, uint64_t* bitmap, hipStream_t stream) {
   const int nRW = (N + kWinRows - 1) / kWinRows;
   auto bm = reinterpret_cast<unsigned long long*>(bitmap);
-  // Windows with thousands of edges get eight waves and 512 TC blocks of LDS at a time. Graphs
-  // of short windows get one wave per window and 128 blocks of LDS, so that a CU works on a
-  // dozen windows at once instead of three with most of their waves idle; their few windows of
-  // more than 128 blocks are left to a second launch with four waves per window.
-#define F3S_FILL(WW, TBB, TCC, TCG, LO, HI)                                                    \
-  hipLaunchKernelGGL((window_fill_kernel<WW, TBB, TCC, TCG>), dim3(nRW), dim3(TBB), 0, stream, \
-                     rowPtr, colIdx, N, E, edgeToColumn, rowWindowOffset, hdr, tcblockRowid,   \
-                     tcblocktileId, tcblockOffset, sparseAToXidx, bm, LO, HI)
-  // the long windows of a graph of short ones: at most two workgroups per CU look for them
-#define F3S_FILL_LONG(WW)                                                                       \
-  hipLaunchKernelGGL((window_fill_long_kernel<WW, 256, kFillChunk, kFillChunkGeneric>),         \
-                     dim3((unsigned)min(512, (nRW + 255) / 256)), dim3(256), 0, stream, rowPtr, \
-                     colIdx, N, E, nRW, edgeToColumn, rowWindowOffset, hdr, tcblockRowid,       \
-                     tcblocktileId, tcblockOffset, sparseAToXidx, bm, kFillChunkSmall + 1)
-  const bool big = (int64_t)E >= (int64_t)nRW * 2048;
-  constexpr int kAll = 0x7FFFFFFF;
-  if (W == 16) {
-    if (big) {
-      F3S_FILL(16, 512, kFillChunk, kFillChunkGeneric, 0, kAll);
-    } else {
-      F3S_FILL(16, 64, kFillChunkSmall, kFillChunkSmall, 0, kFillChunkSmall);
-      F3S_HIP_CHECK(hipGetLastError());
-      F3S_FILL_LONG(16);
-    }
-  } else {
-    if (big) {
-      F3S_FILL(8, 512, kFillChunk, kFillChunkGeneric, 0, kAll);
-    } else {
-      F3S_FILL(8, 64, kFillChunkSmall, kFillChunkSmall, 0, kFillChunkSmall);
-      F3S_HIP_CHECK(hipGetLastError());
-      F3S_FILL_LONG(8);
-    }
-  }
+  // Graphs of windows with thousands of edges: eight waves per window. Others: a wave per window of
+  // at most kBinsMax edges, and at most five workgroups per CU for the longer ones.
+#define F3S_FILL(WW)                                                                            \
+  do {                                                                                          \
+    if (long_windows(nRW, E)) {                                                                 \
+      hipLaunchKernelGGL((window_fill_kernel<WW, 512, kFillChunk, kFillChunkGeneric>),          \
+                         dim3(nRW), dim3(512), 0, stream, rowPtr, colIdx, N, E, edgeToColumn,   \
+                         rowWindowOffset, hdr, tcblockRowid, tcblocktileId, tcblockOffset,      \
+                         sparseAToXidx, bm);                                                    \
+    } else {                                                                                    \
+      hipLaunchKernelGGL((window_fill_short_kernel<WW>),                                        \
+                         dim3((unsigned)((nRW + kFillWaves - 1) / kFillWaves)),                 \
+                         dim3(kFillWaves * 64), 0, stream, rowPtr, colIdx, N, E, nRW,           \
+                         edgeToColumn, rowWindowOffset, hdr, tcblockRowid, tcblocktileId,       \
+                         tcblockOffset, sparseAToXidx, bm);                                     \
+      F3S_HIP_CHECK(hipGetLastError());                                                         \
+      hipLaunchKernelGGL((window_fill_long_kernel<WW, 256, kFillChunkLong, kFillChunkLong>),    \
+                         dim3((unsigned)min(1280, nRW)), dim3(256), 0, stream, rowPtr, colIdx,  \
+                         N, E, nRW, edgeToColumn, rowWindowOffset, hdr, tcblockRowid,           \
+                         tcblocktileId, tcblockOffset, sparseAToXidx, bm);                      \
+    }                                                                                           \
+  } while (0)
+  if (W == 16) F3S_FILL(16); else F3S_FILL(8);
 #undef F3S_FILL
-#undef F3S_FILL_LONG
   F3S_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -2262,7 +2640,7 @@ int launch_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E
         reinterpret_cast<uintptr_t>(edgeToRow) | reinterpret_cast<uintptr_t>(sparseAToXidx) |
         reinterpret_cast<uintptr_t>(tcblocktileId)) & 15u) == 0;
   // long windows, one bitset pass: the kernels that keep a window's bitset in LDS for both phases
-  const bool fused = nRW > 0 && (int64_t)E >= (int64_t)nRW * 2048 && N <= kRangeMax && aligned16;
+  const bool fused = nRW > 0 && long_windows(nRW, E) && N <= kRangeMax && aligned16;
   if (fused) {
     const int range = ((N + 127) / 128) * 128;
     const int bitsetBytes = ((3 * (range / 64) + 3) & ~3) * 4;  // bitset + per-word prefixes

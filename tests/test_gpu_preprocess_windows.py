@@ -1,0 +1,67 @@
+"""Preprocessing at the window sizes where its kernels change hands or fill up: groups of 64 edges,
+the most a wave takes, the sort kernels' capacities, and columns that spread evenly, crowd into a few
+bins, repeat or descend. Bit-exact against the oracle, through the one call and through count + fill."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ["rowWindowOffset", "sortedRowWindows", "tcblockRowid", "tcblocktileId", "tcblockOffset",
+        "sparseAToXidx", "blockPartition", "edgeToColumn", "edgeToRow"]
+
+
+def window_rows(rng, n, N, columns):
+    """16 rows with n edges in all (some rows empty), columns per `columns`."""
+    share = rng.random(16) * (rng.random(16) > 0.2)
+    share[rng.integers(16)] += 0.5
+    cuts = np.sort(rng.choice(16, size=n, p=share / share.sum()))
+    rows = []
+    for r in range(16):
+        k = int((cuts == r).sum())
+        if columns == "crowded":
+            lo = N // 3
+            pool = np.concatenate([np.arange(lo, min(N, lo + max(300, 2 * n // 8))),
+                                   rng.integers(0, N, 20)])
+            cols = rng.choice(np.unique(pool), size=min(k, 200), replace=False)
+            cols = np.concatenate([cols, rng.choice(N, size=k - len(cols), replace=False)])
+        else:
+            cols = rng.choice(N, size=k, replace=k > N)
+        cols = np.unique(cols) if columns != "rough" else cols
+        if columns == "rough" and k > 2:
+            cols[k // 2] = cols[0]  # unsorted, with a repeated column
+        rows.append(cols.astype(np.int32))
+    return rows
+
+
+def build(rng, sizes, N, columns):
+    rows = [r for n in sizes for r in window_rows(rng, n, N, columns)]
+    rows += [np.zeros(0, np.int32)] * (N - len(rows))
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum([len(r) for r in rows])
+    return rowPtr, np.concatenate(rows).astype(np.int32)
+
+
+SIZES = [0, 1, 2, 63, 64, 65, 255, 256, 257, 700, 958, 959, 960, 961, 962, 1023, 1024, 1025, 1100,
+         2048, 4095, 4096, 4097, 5000]
+
+
+@pytest.mark.parametrize("W", [16, 8])
+@pytest.mark.parametrize("columns", ["even", "crowded", "rough"])
+# 1000: fewer columns than bins; 40 000: one bitset pass; 400 003: sort kernels for the long windows
+@pytest.mark.parametrize("N", [1000, 40_000, 400_003])
+def test_window_sizes(oracle_mod, N, columns, W):
+    from fused3s_amd import capi
+    print("case window sizes N=%d %s W=%d" % (N, columns, W), flush=True)
+    rng = np.random.default_rng(N + W)
+    sizes = SIZES + ([16_384, 16_385, 20_000] if N > 1000 else [])
+    rowPtr, colIdx = build(rng, sizes, N, columns)
+    want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, W)
+    rp, ci = torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda()
+    for two_phase in (False, True):
+        got = capi.preprocess(rp, ci, N, 16, W, two_phase=two_phase)
+        assert got["blockCount"] == want["blockCount"]
+        for k in KEYS:
+            assert np.array_equal(got[k].cpu().numpy(), want[k]), (k, two_phase)
+        bm = got["tcbBitMap"].cpu().view(torch.int64).numpy().view(np.uint64)
+        assert np.array_equal(bm, want["tcbBitMap"]), two_phase
