@@ -7,31 +7,38 @@
 //   window_rank_bins_kernel / window_rank_small_kernel
 //                        windows of <= 960 edges, one WAVE per window, no workgroup barrier.
 //                        Graphs of <= 2^22 nodes: (column, position) words sorted by bins of LDS
-//                        counters, ranks of the distinct columns back to the edges. Larger graphs: bitonic sort of the column ids, ballot / popcount
-//                        compaction of the distinct ones, rank by binary search.
+//                        counters, ranks of the distinct columns back to the edges. Larger graphs:
+//                        bitonic sort of the column ids, ballot / popcount compaction of the
+//                        distinct ones, rank by binary search.
+//   window_rank_sort_kernel
+//                        windows of up to 32k edges where the columns take several bitset passes,
+//                        one workgroup per window: sorted by bins as well.
 //   window_rank_kernel   larger windows, one workgroup per window. Column ids are OR-ed into an
 //                        LDS bitset (a column range per pass when N exceeds the LDS range), a
 //                        wave64 popcount prefix scan turns the bitset into ranks, and every edge
 //                        reads its compacted column index back: the sorted unique column list
 //                        (reference: sort + inplace_deduplication + binarysearch,
 //                        src/utils.cu:102-153,281-289) is never materialised.
-//   finalize_count_kernel one workgroup, every wave on its own chunk of the windows: inclusive
-//                        scan of the per-window block counts (src/utils.cu:293-300) and a stable
-//                        LSD radix sort of the windows by descending block count
-//                        (src/utils.cu:400-436), ranks from wave ballots.
+//   window_scan_kernel, finalize_count_kernel, finalize_*_kernel
+//                        scan of the per-window block counts (src/utils.cu:293-300) and stable LSD
+//                        radix sort of the windows by descending block count
+//                        (src/utils.cu:400-436), ranks from wave ballots: one workgroup, or many on
+//                        graphs of many windows.
 //   window_count_kernel, window_rank_fill_kernel
 //                        graphs of long windows through the one-call entry: block counts, then
 //                        ranks, rows, ids, bitmaps and tile ids of a window while its bitset sits
 //                        in LDS.
-//   window_fill_kernel   one workgroup (or one wave, on graphs of short windows) per window:
-//                        bitmaps and per-(row, block) edge counts are accumulated in LDS, a scan
-//                        yields the per-block offsets, and the tile ids are written per block
-//                        from its bitmap when the window's rows ascend, else placed edge by edge
-//                        in CSR order (src/utils.cu:173-224, 23-36, 53-65).
+//   window_fill_kernel, window_fill_short_kernel, window_fill_long_kernel
+//                        one workgroup (or one wave, for short windows) per window: bitmaps and
+//                        per-(row, block) edge counts are accumulated in LDS, a scan yields the
+//                        per-block offsets, and the tile ids are written per block from its bitmap
+//                        when the window's rows ascend, else placed edge by edge in CSR order
+//                        (src/utils.cu:173-224, 23-36, 53-65).
 //
 // All results are bit-identical to the reference's algorithm with edgeToRow[e] = row(e).
 
 #include <mutex>
+#include <vector>
 
 #include "f3s_common.h"
 
@@ -44,48 +51,48 @@ static __device__ __align__(256) unsigned char scratch[kF3sStaticScratchBytes];
 namespace f3s {
 namespace {
 
-constexpr int kBlock = 256;
 constexpr int kRangeMax = 393216;  // columns per bitset pass: 48 KiB of bits + 12 KiB of prefixes
 constexpr int kSortMax = 1024;     // windows up to this many edges are ranked by a per-wave LDS sort
-constexpr int kBinsMax = 960;      // the same on graphs of at most 2^22 nodes (four workgroups per CU)
+constexpr int kBinsMax = 960;      // the same on graphs of at most 2^22 nodes (16 waves per CU)
 // TC blocks held in LDS at once by window_fill_kernel: windows with strictly ascending rows (96
 // bytes of LDS per 16x16 block) and windows with repeated or descending columns (96 bytes as
 // well, but a second pass per chunk)
 constexpr int kFillChunk = 640;
 constexpr int kFillChunkGeneric = 512;
-constexpr int kFillChunkLong = 320;  // both, for the long windows of graphs of short ones
+// both, for the long windows of graphs of short ones: of up to kFillMid edges, and longer (or all)
+constexpr int kFillChunkMid = 320, kFillChunkLong = 1280;
+constexpr int kFillMid = 4096;
+constexpr int kFillFewLong = 4096;
 
-// workspace header (bytes 0..255): int64 nTCB, int32 error flag, and the queue of windows too
-// long for the wave-per-window kernel (filled by window_rank_small_kernel, drained by
-// window_rank_kernel)
+// workspace header (bytes 0..255)
 struct WsHeader {
-  long long nTcb;
-  int error;
-  int nBig;     // entries in the queue of the bitset kernel (window_rank_kernel)
-  int nextBig;  // next entry to hand out
+  int error;    // graphs of long windows: a column index outside [0, N) was met
   int maxCount; // largest per-window block count (multi-workgroup finalize)
-  int nMed, nextMed;      // queue of window_rank_sort_kernel, windows of up to kMedMax edges
-  int nLarge, nextLarge;  // the same for its launch over the windows of up to kLargeMax edges
+};
+// Where phase 1 leaves its result: a device array of the caller's, or pinned host memory that the
+// host reads when the stream is done, without a copy (a copy to pageable memory costs 7 us more).
+struct ResultPtr {
+  long long* nTcb;
+  int* error;  // 0 before the first kernel; a kernel that meets a column outside [0, N) stores 1
 };
 
-// Where the wave-per-window kernels leave the windows that are too long for them: one queue per
-// kernel that takes such windows, chosen by the window's edge count. big == nullptr: no queues
-// (every long window is found by its own workgroup). medMax == 0: everything goes to `big`.
-struct LongQueues {
-  int32_t* med;
-  int32_t* large;
-  int32_t* big;
-  int medMax, largeMax;
-};
-__device__ __forceinline__ void queue_long_window(const LongQueues& q, WsHeader* hdr, int w,
-                                                  int nEdges) {
-  if (!q.big) return;
-  if (nEdges <= q.medMax)
-    q.med[atomicAdd(&hdr->nMed, 1)] = w;
-  else if (nEdges <= q.largeMax)
-    q.large[atomicAdd(&hdr->nLarge, 1)] = w;
-  else
-    q.big[atomicAdd(&hdr->nBig, 1)] = w;
+// The windows of more than minEdges and at most maxEdges edges are few and lie anywhere: thread t of
+// workgroup b of `stride` looks at window b + t * stride (of those from `first` on), so that they are dealt out
+// evenly without a queue. list: one entry per thread, in LDS. Returns their number; every thread of
+// the workgroup calls this.
+__device__ __forceinline__ int find_windows(const int32_t* __restrict__ rowPtr, int N, int nRW,
+                                            int64_t first, int stride, int minEdges,
+                                            int maxEdges, int* list, int* listLen) {
+  __syncthreads();  // the list before this one has been worked through
+  if (threadIdx.x == 0) *listLen = 0;
+  __syncthreads();
+  const int64_t w = first + blockIdx.x + (int64_t)threadIdx.x * stride;
+  if (w < nRW) {
+    const int n = rowPtr[min((int)w * 16 + 16, N)] - rowPtr[(int)w * 16];
+    if (n > minEdges && n <= maxEdges) list[atomicAdd(listLen, 1)] = (int)w;
+  }
+  __syncthreads();
+  return *listLen;
 }
 constexpr size_t kWsHeaderBytes = 256;
 
@@ -205,20 +212,17 @@ __device__ __forceinline__ void wave_lds_sync() {
 // lane row), compacts the distinct ones with ballot + popcount prefixes, and ranks every edge by
 // binary search in the distinct list.
 template <int W>
-__global__ __launch_bounds__(kBlock) void window_rank_small_kernel(
+__global__ __launch_bounds__(64) void window_rank_small_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
     int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
-    int32_t* __restrict__ edgeToRow, WsHeader* __restrict__ hdr, LongQueues queues) {
-  constexpr int WAVES = kBlock / 64;
-  __shared__ uint32_t sKeys[WAVES][kSortMax];
-  __shared__ uint32_t sUniq[WAVES][kSortMax];
-  __shared__ int sRowW[WAVES][17];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int w = blockIdx.x * WAVES + wave;
-  if (w >= nRW) return;
+    int32_t* __restrict__ edgeToRow, int* __restrict__ error) {
+  __shared__ uint32_t sKeys[kSortMax];
+  __shared__ uint32_t sUniq[kSortMax];
+  __shared__ int sRowW[17];
+  const int lane = threadIdx.x;
+  const int w = blockIdx.x;
   const int r0 = w * 16;
-  int* sRow = sRowW[wave];
+  int* sRow = sRowW;
   if (lane < 17) sRow[lane] = rowPtr[min(r0 + lane, N)];
   wave_lds_sync();
   const int eS = sRow[0], eE = sRow[16];
@@ -227,12 +231,9 @@ __global__ __launch_bounds__(kBlock) void window_rank_small_kernel(
     if (lane == 0) blockPartition[w] = 0;
     return;
   }
-  if (n > kSortMax) {  // left to window_rank_kernel, through the queue if there is one
-    if (lane == 0) queue_long_window(queues, hdr, w, n);
-    return;
-  }
-  uint32_t* keys = sKeys[wave];
-  uint32_t* uniq = sUniq[wave];
+  if (n > kSortMax) return;  // left to another kernel
+  uint32_t* keys = sKeys;
+  uint32_t* uniq = sUniq;
   int P = 64;
   while (P < n) P <<= 1;
   bool bad = false;
@@ -247,7 +248,7 @@ __global__ __launch_bounds__(kBlock) void window_rank_small_kernel(
     }
     keys[i] = k;
   }
-  if (bad) atomicOr(&hdr->error, 1);
+  if (bad) *error = 1;
   wave_lds_sync();
   for (int k = 2; k <= P; k <<= 1) {
     for (int j = k >> 1; j > 0; j >>= 1) {
@@ -456,26 +457,25 @@ struct EdgeRows {
 // ballot per bit: counting the smaller ones takes as many steps as the fullest bin holds.
 //
 // Bound by the issue of vector instructions (a wave of 400 edges is 7 groups of 64), then by LDS
-// latency: the LDS accesses of four groups are in flight together. Four workgroups per CU.
+// latency: the LDS accesses of four groups are in flight together. Workgroups of one wave, 16 per CU:
+// a workgroup of four kept the LDS of three windows until the longest of them was done (61M edges:
+// 432 instead of 332 us).
 constexpr int kRankBins = 1024;
 constexpr int kRankCrowd = 24;  // a fuller bin sends the window to the radix sort
 template <int W>
-__global__ __launch_bounds__(kBlock) void window_rank_bins_kernel(
+__global__ __launch_bounds__(64) void window_rank_bins_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
     int colBits, int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
-    int32_t* __restrict__ edgeToRow, WsHeader* __restrict__ hdr, LongQueues queues) {
-  constexpr int WAVES = kBlock / 64;
+    int32_t* __restrict__ edgeToRow, int* __restrict__ error) {
   constexpr int IDX_BITS = 10;
   constexpr int U = 4;  // groups of 64 edges whose LDS accesses are in flight together
   static_assert(kBinsMax <= (1 << IDX_BITS), "edge position must fit IDX_BITS");
-  __shared__ uint32_t sBufA[WAVES][kBinsMax];
-  __shared__ uint32_t sBufB[WAVES][kBinsMax];
-  __shared__ __align__(16) uint32_t sHist[WAVES][kRankBins / 2];
-  __shared__ __align__(8) uint32_t sMark[WAVES][kBinsMax / 32 + 2];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int w = blockIdx.x * WAVES + wave;
-  if (w >= nRW) return;
+  __shared__ uint32_t sBufA[kBinsMax];
+  __shared__ uint32_t sBufB[kBinsMax];
+  __shared__ __align__(16) uint32_t sHist[kRankBins / 2];
+  __shared__ __align__(8) uint32_t sMark[kBinsMax / 32 + 2];
+  const int lane = threadIdx.x;
+  const int w = blockIdx.x;
   const int r0 = w * 16;
   int rowStart = rowPtr[min(r0 + min(lane, 16), N)];
   const int eS = __builtin_amdgcn_readlane(rowStart, 0);
@@ -485,17 +485,14 @@ __global__ __launch_bounds__(kBlock) void window_rank_bins_kernel(
     if (lane == 0) blockPartition[w] = 0;
     return;
   }
-  if (n > kBinsMax) {  // left to another kernel, through the queue if there is one
-    if (lane == 0) queue_long_window(queues, hdr, w, n);
-    return;
-  }
-  uint32_t* a = sBufA[wave];
-  uint32_t* b = sBufB[wave];
-  uint32_t* hist = sHist[wave];
+  if (n > kBinsMax) return;  // left to another kernel
+  uint32_t* a = sBufA;
+  uint32_t* b = sBufB;
+  uint32_t* hist = sHist;
   const unsigned long long leMask = (2ull << lane) - 1ull;
   const int shift = colBits > 10 ? colBits - 10 : 0;
   EdgeRows<kBinsMax> edgeRows;
-  edgeRows.init(sMark[wave], rowStart, lane);
+  edgeRows.init(sMark, rowStart, lane);
 #pragma unroll
   for (int k = 0; k < kRankBins / 2 / 256; k++)
     reinterpret_cast<uint4*>(hist)[lane + 64 * k] = make_uint4(0, 0, 0, 0);
@@ -527,7 +524,7 @@ __global__ __launch_bounds__(kBlock) void window_rank_bins_kernel(
       }
     }
   }
-  if (bad) atomicOr(&hdr->error, 1);
+  if (bad) *error = 1;
   wave_lds_sync();
   // ---- where each bin starts: lane l owns bins 16 l .. 16 l + 15
   bool crowded;
@@ -639,40 +636,37 @@ __global__ __launch_bounds__(kBlock) void window_rank_bins_kernel(
   if (lane == 0) blockPartition[w] = (nUniq + W - 1) / W;
 }
 
-template <int W, int TB>
+// SCAN: the grid is a fixed number of workgroups that look for the windows of more than minEdges
+// edges (graphs of mostly short windows); else workgroup b takes window b, if it is that long.
+template <int W, int TB, bool SCAN>
 __global__ __launch_bounds__(TB) void window_rank_kernel(
-    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int range,
-    int nPasses, int32_t* __restrict__ blockPartition,
-    int32_t* __restrict__ edgeToColumn,
-    int32_t* __restrict__ edgeToRow, WsHeader* __restrict__ hdr,
-    const int32_t* __restrict__ bigList, int shortMax) {
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
+    int range, int nPasses, int minEdges, int32_t* __restrict__ blockPartition,
+    int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
+    int* __restrict__ error) {
   extern __shared__ __align__(16) uint32_t smem[];
   uint32_t* bits = smem;                 // range/32 words
   uint32_t* pref = smem + (range >> 5);  // range/128 group prefixes
   __shared__ int sRow[17];
   __shared__ unsigned sWaveTot[TB / 64];
-  __shared__ int sTake;
+  __shared__ int sList[SCAN ? TB : 1];
+  __shared__ int sListLen;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  // Two ways to find work. With a queue (graphs of mostly short windows) the grid is a fixed
-  // number of workgroups that drain it: an empty queue ends the kernel at once instead of one
-  // workgroup per window holding this kernel's large LDS allocation. Without one (graphs of long
-  // windows, where the appends to the queue would cost more than they save) workgroup b takes
-  // window b.
-  const int nBig = bigList ? hdr->nBig : 1;
-  while (true) {
-  __syncthreads();  // the previous window's reads of sRow / sTake are done
-  if (tid == 0) sTake = bigList ? atomicAdd(&hdr->nextBig, 1) : 0;
-  __syncthreads();
-  if (sTake >= nBig) break;
-  const int w = bigList ? bigList[sTake] : (int)blockIdx.x;
+  for (int64_t first = 0; first < (SCAN ? nRW : 1); first += (int64_t)TB * gridDim.x) {
+  int found = 1;
+  if constexpr (SCAN)
+    found = find_windows(rowPtr, N, nRW, first, (int)gridDim.x, minEdges, 0x7FFFFFFF, sList, &sListLen);
+  for (int k = 0; k < found; k++) {
+  __syncthreads();  // the previous window's reads of sRow are done
+  const int w = SCAN ? sList[k] : (int)blockIdx.x;
   const int r0 = w * 16;
   if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
   __syncthreads();
   const int eS = sRow[0], eE = sRow[16];
-  if (!bigList && eE - eS <= shortMax) break;  // ranked by one wave
+  if (eE - eS <= minEdges) break;  // ranked by one wave
   const int nGroups = range >> 7;
   unsigned uniqueBefore = 0;
   for (int pass = 0; pass < nPasses; pass++) {
@@ -688,10 +682,10 @@ __global__ __launch_bounds__(TB) void window_rank_kernel(
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         if (e0 + u * TB >= eE) continue;
-        const int col = cols[u];
+        int col = cols[u];
         if ((unsigned)col >= (unsigned)N) {
-          atomicOr(&hdr->error, 1);
-          continue;
+          *error = 1;
+          col = 0;
         }
         const unsigned rel = (unsigned)(col - lo);
         if (rel < (unsigned)range) atomicOr(&bits[rel >> 5], 1u << (rel & 31));
@@ -726,9 +720,10 @@ __global__ __launch_bounds__(TB) void window_rank_kernel(
       for (int u = 0; u < 4; u++) cols[u] = (e0 + u * TB < eE) ? colIdx[e0 + u * TB] : -1;
 #pragma unroll
       for (int u = 0; u < 4; u++) {
-        const int col = cols[u];
+        if (e0 + u * TB >= eE) continue;
+        const int col = (unsigned)cols[u] < (unsigned)N ? cols[u] : 0;
         const unsigned rel = (unsigned)(col - lo);
-        if ((unsigned)col < (unsigned)N && rel < (unsigned)range) {
+        if (rel < (unsigned)range) {
           // rank = set bits below this one: group prefix, then the whole 128-bit group read at
           // once and masked
           const unsigned wd = rel >> 5;
@@ -750,75 +745,225 @@ __global__ __launch_bounds__(TB) void window_rank_kernel(
   }
   for (int e = eS + tid; e < eE; e += TB) edgeToRow[e] = r0 + row_of_edge(sRow, e);
   if (tid == 0) blockPartition[w] = (int)((uniqueBefore + W - 1) / W);
-  if (!bigList) break;
+  }
   }
 }
 
-// Windows of kBinsMax (kSortMax) < edges <= kMedMax on graphs whose column range needs several bitset passes
-// (N > kRangeMax): one workgroup per queued window sorts the window's column ids, compacts the
-// distinct ones and ranks every edge by binary search, instead of several passes over a 48 KiB
-// bitset that such a window fills with a few thousand bits. The sort is the wave-level LSD radix
-// sort of wave_radix_sort widened to a workgroup: eight bits per pass, every wave on its
-// own contiguous quarter of the keys (histogram with LDS atomics, one thread per digit turns the
-// per-wave counts into start positions, in-order scatter with wave ballots), two LDS buffers.
-// Two sizes: windows of up to kMedMax edges (256 threads, 32 KiB of buffers, four workgroups per
-// CU), and the handful of windows of up to kLargeMax edges (1024 threads, 128 KiB), which would
-// otherwise each walk the bitset passes alone at the end of the phase.
+// Windows too long for a wave on graphs whose column range needs several bitset passes (N >
+// kRangeMax): one workgroup sorts the window's column ids, marks the distinct ones and finds every
+// edge's rank, instead of several passes over a 48 KiB bitset that such a window fills with a few
+// thousand bits. The sort is that of window_rank_bins_kernel widened to a workgroup, with eight bins
+// per thread; an edge then finds its column in its bin. Windows whose columns crowd into few bins
+// take an LSD radix sort, eight bits per pass, every wave on its own contiguous part of the keys, and
+// a binary search per edge. (Radix sort and search for all: 163 instead of 128 us for the 4 272 such
+// windows of a 61M-edge graph.)
+// Two sizes: windows of up to kMedMax edges (256 threads, 36 KiB of LDS, four workgroups per CU), and
+// the handful of windows of up to kLargeMax edges (1024 threads, 144 KiB), which would otherwise each
+// walk the bitset passes alone at the end of the phase.
 constexpr int kMedThreads = 256;
 constexpr int kMedItems = 16;
 constexpr int kMedMax = kMedThreads * kMedItems;
 constexpr int kLargeThreads = 1024;
 constexpr int kLargeItems = 16;
 constexpr int kLargeMax = kLargeThreads * kLargeItems;
+constexpr int kSortCrowd = 32;  // a fuller bin sends the window to the radix sort
+template <int ITEMS, int THREADS>
+constexpr size_t rank_sort_lds() {
+  return ((size_t)2 * THREADS * ITEMS + 4 * THREADS) * sizeof(uint32_t);
+}
 
-// takes the windows of `queue` (each of at most THREADS * ITEMS edges)
+// takes the windows of more than minEdges and at most THREADS * ITEMS edges
 template <int W, int ITEMS, int THREADS>
 __global__ __launch_bounds__(THREADS) void window_rank_sort_kernel(
-    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int colBits,
-    int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
-    int32_t* __restrict__ edgeToRow, WsHeader* __restrict__ hdr,
-    const int32_t* __restrict__ queue, const int* __restrict__ queueLen,
-    int* __restrict__ nextEntry) {
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
+    int colBits, int minEdges, int32_t* __restrict__ blockPartition,
+    int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
+    int* __restrict__ error) {
   constexpr int WAVES = THREADS / 64;
   constexpr int CAP = THREADS * ITEMS;
+  constexpr int BIN_BITS = THREADS == 256 ? 11 : 13;
+  constexpr int U = 4;  // edges of a thread in flight together
+  static_assert((1 << BIN_BITS) == 8 * THREADS, "eight bins per thread");
   static_assert(THREADS >= 256 && THREADS % 256 == 0, "the first 256 threads own one digit each");
-  extern __shared__ __align__(16) uint32_t sBufDyn[];  // two buffers of CAP keys
+  // two buffers of CAP keys, then the bins' 16-bit counters or the radix sort's digit counters
+  extern __shared__ __align__(16) uint32_t sBufDyn[];
   uint32_t* const sBuf0 = sBufDyn;
   uint32_t* const sBuf1 = sBufDyn + CAP;
-  __shared__ uint32_t sHist[WAVES][256];
+  uint32_t* const sBins = sBufDyn + 2 * CAP;
+  uint32_t (*const sHist)[256] = reinterpret_cast<uint32_t (*)[256]>(sBins);
   __shared__ int sRow[17];
   __shared__ unsigned sWaveTot[WAVES];
-  __shared__ int sTake;
+  __shared__ int sCrowded;
+  __shared__ int sList[THREADS];
+  __shared__ int sListLen;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const unsigned long long ltMask = (1ull << lane) - 1ull;
-  const int nQueued = *queueLen;
-  while (true) {
+  const int shiftBins = colBits > BIN_BITS ? colBits - BIN_BITS : 0;
+  for (int64_t first = 0; first < nRW; first += (int64_t)THREADS * gridDim.x) {
+  const int found = find_windows(rowPtr, N, nRW, first, (int)gridDim.x, minEdges, CAP, sList, &sListLen);
+  for (int taken = 0; taken < found; taken++) {
     __syncthreads();
-    if (tid == 0) sTake = atomicAdd(nextEntry, 1);
-    __syncthreads();
-    if (sTake >= nQueued) break;
-    const int w = queue[sTake];
+    const int w = sList[taken];
     const int r0 = w * 16;
     if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
+    if (tid == 0) sCrowded = 0;
+    reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(0, 0, 0, 0);
     __syncthreads();
     const int eS = sRow[0], eE = sRow[16];
     const int n = eE - eS;
-    if (n > CAP) continue;  // cannot happen: the queue holds what fits
     bool bad = false;
-    for (int i = tid; i < n; i += THREADS) {
-      unsigned k = (unsigned)colIdx[eS + i];
-      if (k >= (unsigned)N) {
-        bad = true;
-        k = 0u;
+    for (int i0 = tid; i0 < n; i0 += U * THREADS) {
+      unsigned k[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) k[u] = (unsigned)colIdx[eS + min(i0 + u * THREADS, n - 1)];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (i0 + u * THREADS >= n) break;
+        if (k[u] >= (unsigned)N) {
+          bad = true;
+          k[u] = 0u;
+        }
+        sBuf0[i0 + u * THREADS] = k[u];
+        const unsigned bin = k[u] >> shiftBins;
+        atomicAdd(&sBins[bin >> 1], 1u << ((bin & 1u) * 16u));
       }
-      sBuf0[i] = k;
     }
-    if (bad) atomicOr(&hdr->error, 1);
-    // wave v sorts the keys [cb, ce) of every pass's input into their places of its output
+    if (bad) *error = 1;
+    __syncthreads();
+    {
+      const uint4 x = reinterpret_cast<const uint4*>(sBins)[tid];
+      uint32_t v[4] = {x.x, x.y, x.z, x.w};
+      uint32_t total = 0, most = 0;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        total += (v[k] & 0xFFFFu) + (v[k] >> 16);
+        most = max(most, max(v[k] & 0xFFFFu, v[k] >> 16));
+      }
+      if (most > (uint32_t)kSortCrowd) sCrowded = 1;
+      const unsigned incl = wave_inclusive_scan(total, lane);
+      if (lane == 63) sWaveTot[wave] = incl;
+      __syncthreads();
+      unsigned run = incl - total;
+#pragma unroll
+      for (int u = 0; u < WAVES; u++)
+        if (u < wave) run += sWaveTot[u];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const uint32_t mid = run + (v[k] & 0xFFFFu);
+        const uint32_t start = run | (mid << 16);
+        run = mid + (v[k] >> 16);
+        v[k] = start;
+      }
+      if (!sCrowded) reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(v[0], v[1], v[2], v[3]);
+    }
+    __syncthreads();
+    // the wave's contiguous part of the keys
     const int chunk = ((n + THREADS - 1) / THREADS) * 64;
     const int cb = min(n, wave * chunk), ce = min(n, cb + chunk);
+    if (!sCrowded) {
+      // into the bins; afterwards a bin's counter says where it ends
+      for (int i0 = tid; i0 < n; i0 += U * THREADS) {
+        uint32_t col[U], old[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) col[u] = sBuf0[min(i0 + u * THREADS, n - 1)];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const uint32_t bin = col[u] >> shiftBins;
+          if (i0 + u * THREADS < n)
+            old[u] = atomicAdd(&sBins[bin >> 1], 1u << ((bin & 1u) * 16u));
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const uint32_t half = ((col[u] >> shiftBins) & 1u) * 16u;
+          if (i0 + u * THREADS < n) sBuf1[(old[u] >> half) & 0xFFFFu] = col[u];
+        }
+      }
+      __syncthreads();
+      const uint16_t* binEnd = reinterpret_cast<const uint16_t*>(sBins);
+      for (int i0 = tid; i0 < n; i0 += U * THREADS) {
+        uint32_t key[U];
+        int end[U], at[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) key[u] = sBuf1[min(i0 + u * THREADS, n - 1)];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const uint32_t bin = key[u] >> shiftBins;
+          end[u] = binEnd[bin];
+          at[u] = bin == 0u ? 0 : (int)binEnd[max(bin, 1u) - 1u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int i = i0 + u * THREADS;
+          if (i >= n) break;
+          const int begin = at[u];
+          if (end[u] - begin > 1)
+            for (int q = begin; q < end[u]; q++) {
+              const uint32_t other = sBuf1[q];
+              at[u] += (other < key[u] || (other == key[u] && q < i)) ? 1 : 0;
+            }
+          sBuf0[at[u]] = key[u];
+        }
+      }
+      __syncthreads();
+      // ranks of the sorted keys, next to them in the other buffer
+      unsigned cnt = 0;
+      for (int base = cb; base < ce; base += 64) {
+        const int i = base + lane;
+        cnt += (unsigned)__popcll(__ballot(i < ce && (i == 0 || sBuf0[i - 1] != sBuf0[i])));
+      }
+      if (lane == 0) sWaveTot[wave] = cnt;
+      __syncthreads();
+      unsigned rank = 0, nUniq = 0;
+#pragma unroll
+      for (int v = 0; v < WAVES; v++) {
+        const unsigned x = sWaveTot[v];
+        if (v < wave) rank += x;
+        nUniq += x;
+      }
+      for (int base = cb; base < ce; base += 64) {
+        const int i = base + lane;
+        const unsigned long long bal =
+            __ballot(i < ce && (i == 0 || sBuf0[i - 1] != sBuf0[i]));
+        if (i < ce) sBuf1[i] = rank + (unsigned)__popcll(bal & (ltMask | (1ull << lane))) - 1u;
+        rank += (unsigned)__popcll(bal);
+      }
+      __syncthreads();
+      for (int i0 = tid; i0 < n; i0 += U * THREADS) {
+        uint32_t col[U];
+        int end[U], q[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          col[u] = (uint32_t)colIdx[eS + min(i0 + u * THREADS, n - 1)];
+          if (col[u] >= (uint32_t)N) col[u] = 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const uint32_t bin = col[u] >> shiftBins;
+          end[u] = binEnd[bin];
+          q[u] = bin == 0u ? 0 : (int)binEnd[max(bin, 1u) - 1u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int e = eS + i0 + u * THREADS;
+          if (e >= eE) break;
+          // the first of the bin's sorted columns that is not below this one: the column itself
+          while (q[u] < end[u] - 1) {
+            const int mid = (q[u] + end[u] - 1) >> 1;
+            if (sBuf0[mid] < col[u])
+              q[u] = mid + 1;
+            else
+              end[u] = mid + 1;
+          }
+          edgeToColumn[e] = (int)sBuf1[q[u]];
+          edgeToRow[e] = r0 + row_of_edge(sRow, e);
+        }
+      }
+      if (tid == 0) blockPartition[w] = (int)((nUniq + W - 1) / W);
+      continue;
+    }
+    // wave v sorts the keys [cb, ce) of every pass's input into their places of its output
     uint32_t* src = sBuf0;
     uint32_t* dst = sBuf1;
     uint32_t* hist = sHist[wave];
@@ -916,6 +1061,7 @@ __global__ __launch_bounds__(THREADS) void window_rank_sort_kernel(
     }
     if (tid == 0) blockPartition[w] = (int)((nUniq + W - 1) / W);
   }
+  }
 }
 
 // ------------------------------------------------- scan + window ordering
@@ -925,19 +1071,63 @@ constexpr int kFinBlock = 1024;
 constexpr int kFinSingleMax = 16384;
 constexpr int kFinIdBits = 14;
 
-__global__ __launch_bounds__(kFinBlock) void finalize_count_kernel(
-    const int32_t* __restrict__ blockPartition, int nRW, int32_t* __restrict__ rowWindowOffset,
-    int32_t* __restrict__ sortedRowWindows, WsHeader* __restrict__ hdr) {
-  // One workgroup; every wave owns a contiguous chunk of the windows and walks it on its own
-  // (wave-level scans and ballots only), so a pass over the array costs a handful of block
-  // barriers instead of several per 1024 elements. The sort's two buffers are in LDS
-  // (2 * kFinSingleMax words of dynamic LDS): a (key, window) pair is one word, key above
-  // kFinIdBits bits of window id.
-  extern __shared__ __align__(16) uint32_t finLds[];
-  uint32_t* bufA = finLds;
-  uint32_t* bufB = finLds + kFinSingleMax;
+// Exclusive prefix of the block counts into rowWindowOffset and their total, by one workgroup: every
+// wave owns a contiguous chunk of the windows, all of its loads in flight together.
+__device__ __forceinline__ void scan_windows(const int32_t* __restrict__ blockPartition, int nRW,
+                                             int32_t* __restrict__ rowWindowOffset,
+                                             long long* __restrict__ nTcb) {
   constexpr int NW = kFinBlock / 64;
+  constexpr int G = kFinSingleMax / kFinBlock;  // groups of 64 windows per wave at most
   __shared__ unsigned sWaveSum[NW];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int chunk = (((nRW + NW - 1) / NW) + 63) & ~63;
+  const int cBegin = min(wave * chunk, nRW);
+  const int cEnd = min(cBegin + chunk, nRW);
+  unsigned v[G], sum = 0;
+#pragma unroll
+  for (int k = 0; k < G; k++) {
+    const int i = cBegin + 64 * k + lane;
+    v[k] = i < cEnd ? (unsigned)blockPartition[i] : 0u;
+  }
+#pragma unroll
+  for (int k = 0; k < G; k++) sum += v[k];
+  sum = wave_inclusive_scan(sum, lane);
+  if (lane == 63) sWaveSum[wave] = sum;
+  __syncthreads();
+  unsigned carry = 0, total = 0;
+#pragma unroll
+  for (int k = 0; k < NW; k++) {
+    const unsigned t = sWaveSum[k];
+    if (k < wave) carry += t;
+    total += t;
+  }
+#pragma unroll
+  for (int k = 0; k < G; k++) {
+    if (64 * k >= chunk) break;
+    const int i = cBegin + 64 * k + lane;
+    const unsigned incl = wave_inclusive_scan(v[k], lane);
+    if (i < cEnd) rowWindowOffset[i + 1] = (int)(carry + incl);
+    carry += (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
+  }
+  if (threadIdx.x == 0) {
+    rowWindowOffset[0] = 0;
+    *nTcb = (long long)total;
+  }
+}
+
+// Windows by descending block count, ties ascending, by one workgroup of kFinBlock threads; every
+// wave owns a contiguous chunk of the windows and walks it on its own (wave-level scans and ballots
+// only), so a pass over the array costs a handful of block barriers instead of several per 1024
+// elements. lds: order_lds_words(nRW) words; a (key, window) pair is one word, key above kFinIdBits
+// bits of window id.
+constexpr size_t order_lds_words(int nRW) { return 2 * (size_t)((nRW + 3) & ~3); }
+__device__ __forceinline__ void order_windows(const int32_t* __restrict__ blockPartition, int nRW,
+                                              int32_t* __restrict__ sortedRowWindows,
+                                              uint32_t* lds) {
+  uint32_t* bufA = lds;
+  uint32_t* bufB = lds + ((nRW + 3) & ~3);
+  constexpr int NW = kFinBlock / 64;
   __shared__ int sWaveMax[NW];
   constexpr int DB = 6;               // digit bits per sorting pass: one bin per lane
   constexpr int NB = 1 << DB;
@@ -950,11 +1140,12 @@ __global__ __launch_bounds__(kFinBlock) void finalize_count_kernel(
   const int cBegin = min(wave * chunk, nRW);
   const int cEnd = min(cBegin + chunk, nRW);
 
-  // ---- the counts into LDS first, every thread's loads in flight together: each later pass
-  // walks its chunk group by group, and a global load per group would cost its full latency
-  // every time
+  // ---- the counts into LDS first, every thread's loads in flight together (each later pass walks
+  // its chunk group by group, and a global load per group would cost its full latency every time),
+  // and their maximum
   {
     constexpr int U = 4;
+    int mx = 0;
     for (int i0 = tid; i0 < nRW; i0 += U * kFinBlock) {
       int v[U];
 #pragma unroll
@@ -966,50 +1157,17 @@ __global__ __launch_bounds__(kFinBlock) void finalize_count_kernel(
       for (int u = 0; u < U; u++) {
         const int i = i0 + u * kFinBlock;
         if (i < nRW) bufB[i] = (uint32_t)v[u];
+        mx = max(mx, v[u]);
       }
     }
-  }
-  __syncthreads();
-  // ---- inclusive scan of the block counts into rowWindowOffset[1..], and their maximum
-  {
-    unsigned sum = 0;
-    int mx = 0;
-    for (int i = cBegin + lane; i < cEnd; i += 64) {
-      const int v = (int)bufB[i];
-      sum += (unsigned)v;
-      mx = max(mx, v);
-    }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      sum += __shfl_xor(sum, off);
-      mx = max(mx, __shfl_xor(mx, off));
-    }
-    if (lane == 0) {
-      sWaveSum[wave] = sum;
-      sWaveMax[wave] = mx;
-    }
+    for (int off = 32; off > 0; off >>= 1) mx = max(mx, __shfl_xor(mx, off));
+    if (lane == 0) sWaveMax[wave] = mx;
   }
   __syncthreads();
-  unsigned carry = 0, total = 0;
   int maxC = 0;
 #pragma unroll
-  for (int k = 0; k < NW; k++) {
-    const unsigned t = sWaveSum[k];
-    if (k < wave) carry += t;
-    total += t;
-    maxC = max(maxC, sWaveMax[k]);
-  }
-  for (int base = cBegin; base < cEnd; base += 64) {
-    const int i = base + lane;
-    const unsigned v = (i < cEnd) ? bufB[i] : 0u;
-    const unsigned incl = wave_inclusive_scan(v, lane);
-    if (i < cEnd) rowWindowOffset[i + 1] = (int)(carry + incl);
-    carry += __shfl(incl, 63);
-  }
-  if (tid == 0) {
-    rowWindowOffset[0] = 0;
-    hdr->nTcb = (long long)total;
-  }
+  for (int k = 0; k < NW; k++) maxC = max(maxC, sWaveMax[k]);
 
   // ---- stable sort by descending count == stable ascending LSD radix sort of (maxC - count),
   // six bits per pass
@@ -1091,6 +1249,20 @@ __global__ __launch_bounds__(kFinBlock) void finalize_count_kernel(
         sortedRowWindows[i] = (int)(dst[i] & ((1u << kFinIdBits) - 1u));
     }
   }
+}
+
+__global__ __launch_bounds__(kFinBlock) void window_scan_kernel(
+    const int32_t* __restrict__ blockPartition, int nRW, int32_t* __restrict__ rowWindowOffset,
+    long long* __restrict__ nTcb) {
+  scan_windows(blockPartition, nRW, rowWindowOffset, nTcb);
+}
+
+__global__ __launch_bounds__(kFinBlock) void finalize_count_kernel(
+    const int32_t* __restrict__ blockPartition, int nRW, int32_t* __restrict__ rowWindowOffset,
+    int32_t* __restrict__ sortedRowWindows, long long* __restrict__ nTcb) {
+  extern __shared__ __align__(16) uint32_t finLds[];
+  scan_windows(blockPartition, nRW, rowWindowOffset, nTcb);
+  order_windows(blockPartition, nRW, sortedRowWindows, finLds);
 }
 
 // ---- the same scan + stable sort spread over many workgroups, for graphs with many windows.
@@ -1186,7 +1358,7 @@ __global__ __launch_bounds__(256) void finalize_scan_kernel(
     const int32_t* __restrict__ blockPartition, int nRW, int totalWaves,
     const unsigned* __restrict__ waveSum, const int* __restrict__ waveMax,
     int32_t* __restrict__ rowWindowOffset, unsigned* __restrict__ hist,
-    WsHeader* __restrict__ hdr) {
+    WsHeader* __restrict__ hdr, long long* __restrict__ nTcb) {
   __shared__ unsigned sBins[4][kFinBins];
   const int lane = threadIdx.x & 63;
   const int gw = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -1216,7 +1388,7 @@ __global__ __launch_bounds__(256) void finalize_scan_kernel(
   }
   if (gw == 0 && lane == 0) {
     rowWindowOffset[0] = 0;
-    hdr->nTcb = (long long)total;
+    *nTcb = (long long)total;
     hdr->maxCount = maxC;
   }
   fin_histogram(blockPartition, true, maxC, c, 0, lane, sBins[threadIdx.x >> 6],
@@ -1486,19 +1658,21 @@ __device__ __forceinline__ void fill_window_generic(
 // row by row (src/utils.cu:213-223 walks the edges in exactly that order), and bitmaps and ids
 // leave LDS as contiguous runs. A window with a repeated or descending column is handed to
 // fill_window_generic. TC blocks of LDS at a time on the short way, TCG on the general one.
+// LDS of fill_one_window: sRaw
+template <int W>
+constexpr size_t fill_lds_bytes(int tc, int tcg) {
+  const size_t fast = (size_t)tc * (2 * W + 4 * W), generic = (size_t)tcg * (64 + 2 * W);
+  return fast > generic ? fast : generic;
+}
 template <int W, int TB, int TC, int TCG>
 __device__ __forceinline__ void fill_one_window(
     int w, int nRW, const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N,
     int E, const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
-    const WsHeader* __restrict__ hdr, int32_t* __restrict__ tcblockRowid,
+    unsigned char* sRaw, int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
     int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
   constexpr int WPT = 16 * W / 64;  // bitmap words per TC block
   constexpr int LOGW = (W == 16) ? 4 : 3;
-  constexpr int FAST_BYTES = TC * (WPT * 8 + W * 4);
-  constexpr int GEN_BYTES = TCG * (16 * 4 + WPT * 8);
-  constexpr int RAW_BYTES = FAST_BYTES > GEN_BYTES ? FAST_BYTES : GEN_BYTES;
-  __shared__ __align__(16) unsigned char sRaw[RAW_BYTES];
   __shared__ int sRow[17];
   __shared__ unsigned sWaveTot[TB / 64];
   __shared__ unsigned sUnsorted;  // bit r: row r's columns are not strictly ascending
@@ -1508,9 +1682,6 @@ __device__ __forceinline__ void fill_one_window(
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  // launched right behind phase 1 (no host in between): a column index outside [0, N) left
-  // edgeToColumn unwritten, so nothing here may run
-  if (hdr && hdr->error) return;
   if (tid == 0) sUnsorted = 0u;
   if (w == 0 && tid == 0) tcblockOffset[rowWindowOffset[nRW]] = E;
   const int base = rowWindowOffset[w];
@@ -1642,29 +1813,26 @@ __device__ __forceinline__ void fill_one_window(
 // its bit in the window's bitmaps and drops its column into the ids; two lanes per TC block then walk
 // the set bits row by row (a block of a sparse graph has 17, most of a walk's time is the fullest
 // dword among the lanes), and bitmaps, ids and tile ids leave as whole words. Bound by the issue of
-// vector instructions; five workgroups of four waves per CU.
-constexpr int kFillWaves = 4;
+// vector instructions. Workgroups of one wave, 22 per CU (of four: 260 instead of 220 us for the 149k
+// such windows of a 61M-edge graph).
 template <int W>
-__global__ __launch_bounds__(kFillWaves * 64) void window_fill_short_kernel(
+__global__ __launch_bounds__(64) void window_fill_short_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
     const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
-    const WsHeader* __restrict__ hdr, int32_t* __restrict__ tcblockRowid,
+    int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
     int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
   constexpr int WPT = 16 * W / 64;
   constexpr int LOGW = (W == 16) ? 4 : 3;
   constexpr int MAXB = (kBinsMax + W - 1) / W;  // TC blocks of a window at most
   constexpr int U = 4;  // groups of 64 edges in flight together
-  __shared__ __align__(16) unsigned long long sBm[kFillWaves][MAXB * WPT];
-  __shared__ __align__(16) uint32_t sIds[kFillWaves][MAXB * W];
-  __shared__ __align__(16) uint8_t sTile[kFillWaves][kBinsMax + 8];
-  __shared__ __align__(8) uint32_t sMark[kFillWaves][kBinsMax / 32 + 2];
+  __shared__ __align__(16) unsigned long long sBm[MAXB * WPT];
+  __shared__ __align__(16) uint32_t sIds[MAXB * W];
+  __shared__ __align__(16) uint8_t sTile[kBinsMax + 8];
+  __shared__ __align__(8) uint32_t sMark[kBinsMax / 32 + 2];
   static_assert(MAXB * 8 <= MAXB * W, "edges per (block, row), two counters per word, fit sIds");
-  if (hdr && hdr->error) return;  // edgeToColumn is incomplete
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int w = blockIdx.x * kFillWaves + wave;
-  if (w >= nRW) return;
+  const int lane = threadIdx.x;
+  const int w = blockIdx.x;
   int rowStart = rowPtr[min(w * 16 + min(lane, 16), N)];
   const int base = __builtin_amdgcn_readfirstlane(rowWindowOffset[w]);
   const int nb = __builtin_amdgcn_readfirstlane(rowWindowOffset[w + 1]) - base;
@@ -1673,10 +1841,10 @@ __global__ __launch_bounds__(kFillWaves * 64) void window_fill_short_kernel(
   rowStart -= eS;
   if (w == nRW - 1 && lane == 0) tcblockOffset[base + nb] = E;
   if (n == 0 || n > kBinsMax || nb > MAXB) return;  // long ones: window_fill_long_kernel
-  unsigned long long* bm = sBm[wave];
-  uint32_t* ids = sIds[wave];
+  unsigned long long* bm = sBm;
+  uint32_t* ids = sIds;
   EdgeRows<kBinsMax> edgeRows;
-  edgeRows.init(sMark[wave], rowStart, lane);
+  edgeRows.init(sMark, rowStart, lane);
   for (int i = lane; i < nb * WPT / 2; i += 64)
     reinterpret_cast<uint4*>(bm)[i] = make_uint4(0, 0, 0, 0);
   for (int i = nb * W - W + lane; i < nb * W; i += 64) ids[i] = 0u;  // unused slots hold 0
@@ -1716,7 +1884,7 @@ __global__ __launch_bounds__(kFillWaves * 64) void window_fill_short_kernel(
     store_streaming(reinterpret_cast<uint4*>(sparseAToXidx + (int64_t)base * W) + i,
                     reinterpret_cast<const uint4*>(ids)[i]);
   if (__ballot(rough) == 0ull) {
-    uint8_t* stage = sTile[wave];
+    uint8_t* stage = sTile;
     const unsigned skew = (unsigned)((uintptr_t)(tcblocktileId + eS) & 3u);
     unsigned carry = 0;
     for (int k = 0; k < 2 * nb; k += 64) {
@@ -1818,44 +1986,48 @@ template <int W, int TB, int TC, int TCG>
 __global__ __launch_bounds__(TB) void window_fill_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E,
     const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
-    const WsHeader* __restrict__ hdr, int32_t* __restrict__ tcblockRowid,
+    int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
     int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
+  extern __shared__ __align__(16) unsigned char sRawDyn[];
   fill_one_window<W, TB, TC, TCG>((int)blockIdx.x, (int)gridDim.x, rowPtr, colIdx, N, E,
-                                  edgeToColumn, rowWindowOffset, hdr, tcblockRowid, tcblocktileId,
+                                  edgeToColumn, rowWindowOffset, sRawDyn, tcblockRowid, tcblocktileId,
                                   tcblockOffset, sparseAToXidx, bitmap);
 }
 
-// The windows that window_fill_short_kernel leaves out: thread t of workgroup b looks at window
-// b + t * gridDim.x (and so on), and the workgroup fills the long ones it finds one after the other,
-// so that long windows are dealt out evenly wherever they lie. One workgroup per window instead
-// would start a hundred thousand workgroups of 30 KiB of LDS each to find that nearly all of them
-// have nothing to do. 320 TC blocks of LDS at a time: five workgroups per CU.
-template <int W, int TB, int TC, int TCG>
+// The windows that window_fill_short_kernel leaves out, of more than minEdges and at most maxEdges
+// edges (find_windows). Two sizes: 256 threads and 320 TC blocks of LDS at a time for windows of up to
+// kFillMid edges (five workgroups per CU), 1024 threads and 1280 blocks for longer ones, which would
+// otherwise each keep one small workgroup busy long after the others are done (31 700 edges:
+// 190 us). On graphs of few windows the large workgroups take both.
+// ORDER: the last workgroup writes the window order meanwhile, which no other kernel of the call waits for.
+template <int W, int TB, int TC, bool ORDER>
 __global__ __launch_bounds__(TB) void window_fill_long_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
     const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
-    const WsHeader* __restrict__ hdr, int32_t* __restrict__ tcblockRowid,
+    int minEdges, int maxEdges, const int32_t* __restrict__ blockPartition,
+    int32_t* __restrict__ sortedRowWindows, int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
     int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
+  extern __shared__ __align__(16) unsigned char sRawDyn[];
   __shared__ int sList[TB];
   __shared__ int sListLen;
-  const int stride = (int)gridDim.x;
-  for (int64_t first = blockIdx.x; first < nRW; first += (int64_t)TB * stride) {
-    __syncthreads();  // the list before this one has been worked through
-    if (threadIdx.x == 0) sListLen = 0;
-    __syncthreads();
-    const int64_t w = first + (int64_t)threadIdx.x * stride;
-    if (w < nRW &&
-        rowPtr[min((int)w * 16 + 16, N)] - rowPtr[(int)w * 16] > kBinsMax)
-      sList[atomicAdd(&sListLen, 1)] = (int)w;
-    __syncthreads();
-    const int len = sListLen;
-    for (int k = 0; k < len; k++) {
+  if constexpr (ORDER) {
+    static_assert(TB == kFinBlock, "the order is one such workgroup's work");
+    if (blockIdx.x == gridDim.x - 1) {
+      order_windows(blockPartition, nRW, sortedRowWindows, reinterpret_cast<uint32_t*>(sRawDyn));
+      return;
+    }
+  }
+  const int stride = (int)gridDim.x - (ORDER ? 1 : 0);
+  for (int64_t first = 0; first < nRW; first += (int64_t)TB * stride) {
+    const int found = find_windows(rowPtr, N, nRW, first, stride, minEdges, maxEdges, sList,
+                                   &sListLen);
+    for (int k = 0; k < found; k++) {
       __syncthreads();  // the window before this one has left the LDS arrays
-      fill_one_window<W, TB, TC, TCG>(sList[k], nRW, rowPtr, colIdx, N, E, edgeToColumn,
-                                      rowWindowOffset, hdr, tcblockRowid, tcblocktileId,
-                                      tcblockOffset, sparseAToXidx, bitmap);
+      fill_one_window<W, TB, TC, TC>(sList[k], nRW, rowPtr, colIdx, N, E, edgeToColumn,
+                                     rowWindowOffset, sRawDyn, tcblockRowid, tcblocktileId,
+                                     tcblockOffset, sparseAToXidx, bitmap);
     }
   }
 }
@@ -1945,7 +2117,7 @@ __device__ __forceinline__ bool set_column_bits(const int32_t* __restrict__ colI
 template <int W, int TB>
 __global__ __launch_bounds__(TB) void window_count_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int range,
-    int32_t* __restrict__ blockPartition, WsHeader* __restrict__ hdr) {
+    int32_t* __restrict__ blockPartition, WsHeader* __restrict__ hdr, int* __restrict__ error) {
   extern __shared__ __align__(16) uint32_t smem[];
   uint32_t* bits = smem;  // range/32 words
   __shared__ unsigned sWaveTot[TB / 64];
@@ -1963,7 +2135,10 @@ __global__ __launch_bounds__(TB) void window_count_kernel(
     reinterpret_cast<uint4*>(bits)[i] = make_uint4(0, 0, 0, 0);
   lds_barrier();
   const EdgeSplit sp = split_edges(eS, eE);
-  if (!set_column_bits<TB, 4>(colIdx, eS, eE, sp, (unsigned)N, bits)) atomicOr(&hdr->error, 1);
+  if (!set_column_bits<TB, 4>(colIdx, eS, eE, sp, (unsigned)N, bits)) {
+    hdr->error = 1;  // window_rank_fill_kernel asks here, the host over there
+    *error = 1;
+  }
   lds_barrier();
   unsigned cnt = 0;
   for (int gi = tid; gi < nGroups; gi += TB) {
@@ -2289,17 +2464,7 @@ __global__ void set_tail_kernel(int32_t* tcblockOffset, long long nTcb, int E) {
   tcblockOffset[nTcb] = E;
 }
 
-__global__ void clear_header_kernel(WsHeader* hdr) {
-  hdr->nTcb = 0;
-  hdr->error = 0;
-  hdr->nBig = 0;
-  hdr->nextBig = 0;
-  hdr->maxCount = 0;
-  hdr->nMed = 0;
-  hdr->nextMed = 0;
-  hdr->nLarge = 0;
-  hdr->nextLarge = 0;
-}
+__global__ void clear_error_kernel(int* error) { *error = 0; }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -2323,9 +2488,18 @@ namespace {
 // long windows on average: a workgroup per window instead of a wave
 bool long_windows(int nRW, int64_t E) { return E >= (int64_t)nRW * 2048; }
 
+// Kernels of more than 64 KiB of LDS have to be told.
+template <typename KernelT>
+int allow_lds(KernelT kernel, size_t bytes) {
+  if (bytes > 64 * 1024)
+    F3S_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  return 0;
+}
+
 // Scan of the block counts and the window order, after the kernels that write blockPartition.
 int enqueue_finalize(int N, int W, const int32_t* blockPartition, int32_t* rowWindowOffset,
-                     int32_t* sortedRowWindows, char* ws, hipStream_t stream) {
+                     int32_t* sortedRowWindows, char* ws, long long* nTcb, hipStream_t stream) {
   const int nRW = (N + kWinRows - 1) / kWinRows;
   WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
   const size_t seg = align256((size_t)nRW * sizeof(int32_t));
@@ -2334,11 +2508,10 @@ int enqueue_finalize(int N, int W, const int32_t* blockPartition, int32_t* rowWi
   int32_t* valsTmp = reinterpret_cast<int32_t*>(ws + kWsHeaderBytes + 2 * seg);
   const int finWaves = finalize_waves(nRW);
   if (finWaves == 0) {
-    constexpr int ldsBytes = 2 * kFinSingleMax * (int)sizeof(uint32_t);
-    F3S_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&finalize_count_kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, ldsBytes));
-    hipLaunchKernelGGL(finalize_count_kernel, dim3(1), dim3(kFinBlock), ldsBytes, stream,
-                       blockPartition, nRW, rowWindowOffset, sortedRowWindows, hdr);
+    const size_t lds = order_lds_words(nRW) * sizeof(uint32_t);
+    if (int rc = allow_lds(finalize_count_kernel, lds)) return rc;
+    hipLaunchKernelGGL(finalize_count_kernel, dim3(1), dim3(kFinBlock), lds, stream,
+                       blockPartition, nRW, rowWindowOffset, sortedRowWindows, nTcb);
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
   }
@@ -2349,7 +2522,7 @@ int enqueue_finalize(int N, int W, const int32_t* blockPartition, int32_t* rowWi
   hipLaunchKernelGGL(finalize_partials_kernel, grid, block, 0, stream, blockPartition, nRW,
                      finWaves, waveSum, waveMax);
   hipLaunchKernelGGL(finalize_scan_kernel, grid, block, 0, stream, blockPartition, nRW, finWaves,
-                     waveSum, waveMax, rowWindowOffset, hist, hdr);
+                     waveSum, waveMax, rowWindowOffset, hist, hdr, nTcb);
   // a window holds at most ceil(N / W) blocks: that bounds the passes that can be needed
   int maxBits = 0;
   while ((((int64_t)N + W - 1) / W >> maxBits) != 0) maxBits++;
@@ -2365,102 +2538,142 @@ int enqueue_finalize(int N, int W, const int32_t* blockPartition, int32_t* rowWi
   return 0;
 }
 
+// Workgroups that look for the windows of more than minEdges edges: one for each that there can be, so
+// that the device deals them out as workgroups end (a fixed 1024 of them met up to 13 of the 4 272
+// windows of a 61M-edge graph, 4.2 on average: 200 instead of 149 us), within `most`.
+unsigned long_grid(int nRW, int E, int minEdges, int most) {
+  int grid = E / (minEdges + 1) + 1;
+  if (grid > nRW) grid = nRW;
+  return (unsigned)(grid > most ? most : grid);
+}
+
+// Enqueues the kernels that rank the windows' columns and count their TC blocks.
+template <int W>
+int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
+                 int32_t* blockPartition, int32_t* edgeToColumn, int32_t* edgeToRow, int* error,
+                 hipStream_t stream) {
+  const int nRW = (N + kWinRows - 1) / kWinRows;
+  if (nRW == 0) return 0;
+  int range = ((N + 127) / 128) * 128;
+  if (range > kRangeMax) range = kRangeMax;
+  const int nPasses = (N + range - 1) / range;
+  const size_t lds = (size_t)(range / 32 + range / 128) * sizeof(uint32_t);
+  // short windows: packed (column, position) words when the column ids leave room for the
+  // position, else the bitonic network on bare column ids
+  int colBits = 0;
+  while (colBits < 31 && ((int64_t)1 << colBits) < (int64_t)N) colBits++;
+  int shortMax = kBinsMax;
+  if (colBits <= 22) {
+    hipLaunchKernelGGL(window_rank_bins_kernel<W>, dim3(nRW), dim3(64), 0, stream, rowPtr,
+                       colIdx, N, nRW, colBits, blockPartition, edgeToColumn, edgeToRow, error);
+  } else {
+    shortMax = kSortMax;
+    hipLaunchKernelGGL(window_rank_small_kernel<W>, dim3(nRW), dim3(64), 0, stream,
+                       rowPtr, colIdx, N, nRW, blockPartition, edgeToColumn, edgeToRow, error);
+  }
+  F3S_HIP_CHECK(hipGetLastError());
+  if (long_windows(nRW, E)) {
+    hipLaunchKernelGGL((window_rank_kernel<W, 512, false>), dim3(nRW), dim3(512), lds, stream,
+                       rowPtr, colIdx, N, nRW, range, nPasses, shortMax, blockPartition,
+                       edgeToColumn, edgeToRow, error);
+    F3S_HIP_CHECK(hipGetLastError());
+    return 0;
+  }
+  // The longer ones, which each kernel looks for. On a graph that needs several bitset passes,
+  // windows of a few thousand edges are sorted instead of walking every pass: up to kMedMax edges
+  // with four workgroups per CU, then the few windows up to kLargeMax with one.
+  int minEdges = shortMax;
+  if (nPasses >= 2) {
+    auto med = window_rank_sort_kernel<W, kMedItems, kMedThreads>;
+    auto large = window_rank_sort_kernel<W, kLargeItems, kLargeThreads>;
+    constexpr size_t medLds = rank_sort_lds<kMedItems, kMedThreads>();
+    constexpr size_t largeLds = rank_sort_lds<kLargeItems, kLargeThreads>();
+    if (int rc = allow_lds(med, medLds)) return rc;
+    if (int rc = allow_lds(large, largeLds)) return rc;
+    hipLaunchKernelGGL(med, dim3(long_grid(nRW, E, minEdges, 8192)), dim3(kMedThreads), medLds,
+                       stream, rowPtr, colIdx, N, nRW, colBits, minEdges, blockPartition,
+                       edgeToColumn, edgeToRow, error);
+    hipLaunchKernelGGL(large, dim3(long_grid(nRW, E, kMedMax, 1024)), dim3(kLargeThreads),
+                       largeLds, stream, rowPtr, colIdx, N, nRW, colBits, kMedMax, blockPartition,
+                       edgeToColumn, edgeToRow, error);
+    F3S_HIP_CHECK(hipGetLastError());
+    minEdges = kLargeMax;
+  }
+  // sixteen waves per window: what counts is how soon the longest one is done (169k-node R-MAT graph,
+  // windows of up to 12 500 edges: 31 us with four)
+  hipLaunchKernelGGL((window_rank_kernel<W, 1024, true>), dim3(long_grid(nRW, E, minEdges, 512)),
+                     dim3(1024), lds, stream, rowPtr, colIdx, N, nRW, range, nPasses, minEdges,
+                     blockPartition, edgeToColumn, edgeToRow, error);
+  F3S_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W,
+                 int32_t* blockPartition, int32_t* edgeToColumn, int32_t* edgeToRow, int* error,
+                 hipStream_t stream) {
+  return W == 16 ? enqueue_rank<16>(rowPtr, colIdx, N, E, blockPartition, edgeToColumn, edgeToRow,
+                                    error, stream)
+                 : enqueue_rank<8>(rowPtr, colIdx, N, E, blockPartition, edgeToColumn, edgeToRow,
+                                   error, stream);
+}
+
 // Enqueues every kernel of phase 1 on `stream`; `ws` is device scratch of
-// preprocess_workspace_bytes(N, E) bytes whose header ends up holding the TC-block total and the
-// error flag.
+// preprocess_workspace_bytes(N, E) bytes.
 int enqueue_count(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W,
                   int32_t* blockPartition, int32_t* edgeToColumn, int32_t* edgeToRow,
                   int32_t* rowWindowOffset, int32_t* sortedRowWindows, char* ws,
-                  hipStream_t stream) {
-  const int nRW = (N + kWinRows - 1) / kWinRows;
-  WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
-  const size_t seg = align256((size_t)nRW * sizeof(int32_t));
-  // the three buffers the window order later sorts in hold the queues of long windows until then
-  int32_t* keysA = reinterpret_cast<int32_t*>(ws + kWsHeaderBytes);
-  int32_t* keysB = reinterpret_cast<int32_t*>(ws + kWsHeaderBytes + seg);
-  int32_t* valsTmp = reinterpret_cast<int32_t*>(ws + kWsHeaderBytes + 2 * seg);
-
-  hipLaunchKernelGGL(clear_header_kernel, dim3(1), dim3(1), 0, stream, hdr);
-  if (nRW > 0) {
-    int range = ((N + 127) / 128) * 128;
-    if (range > kRangeMax) range = kRangeMax;
-    const int nPasses = (N + range - 1) / range;
-    const size_t lds = (size_t)(range / 32 + range / 128) * sizeof(uint32_t);
-    const int smallGrid = (nRW + kBlock / 64 - 1) / (kBlock / 64);
-    const bool big = long_windows(nRW, E);
-    int32_t* queue = big ? nullptr : valsTmp;
-    // queued windows of a few thousand edges on a graph that needs several bitset passes are
-    // sorted (window_rank_sort_kernel) instead of walking every pass; the others go to the
-    // bitset kernel
-    const bool sortMedium = queue != nullptr && nPasses >= 2;
-    const LongQueues queues = {keysA, keysB, queue, sortMedium ? kMedMax : 0,
-                               sortMedium ? kLargeMax : 0};
-    // short windows: radix sort of packed (column, position) words when the column ids leave
-    // room for the position, else the bitonic network on bare column ids
-    int colBits = 0;
-    while (colBits < 31 && ((int64_t)1 << colBits) < (int64_t)N) colBits++;
-    if (colBits <= 22) {
-      if (W == 16)
-        hipLaunchKernelGGL(window_rank_bins_kernel<16>, dim3(smallGrid), dim3(kBlock), 0, stream,
-                           rowPtr, colIdx, N, nRW, colBits, blockPartition, edgeToColumn,
-                           edgeToRow, hdr, queues);
-      else
-        hipLaunchKernelGGL(window_rank_bins_kernel<8>, dim3(smallGrid), dim3(kBlock), 0, stream,
-                           rowPtr, colIdx, N, nRW, colBits, blockPartition, edgeToColumn,
-                           edgeToRow, hdr, queues);
-    } else if (W == 16) {
-      hipLaunchKernelGGL(window_rank_small_kernel<16>, dim3(smallGrid), dim3(kBlock), 0, stream,
-                         rowPtr, colIdx, N, nRW, blockPartition, edgeToColumn, edgeToRow, hdr,
-                         queues);
-    } else {
-      hipLaunchKernelGGL(window_rank_small_kernel<8>, dim3(smallGrid), dim3(kBlock), 0, stream,
-                         rowPtr, colIdx, N, nRW, blockPartition, edgeToColumn, edgeToRow, hdr,
-                         queues);
-    }
-    F3S_HIP_CHECK(hipGetLastError());
-    if (sortMedium) {
-      // two launches: up to kMedMax edges with 32 KiB of sort buffers (four workgroups per CU),
-      // then the few windows up to kLargeMax with 128 KiB (one per CU)
-#define F3S_SORT(WW, ITEMS, THREADS, GRID, QUEUE, LEN, COUNTER)                                 \
-  do {                                                                                          \
-    constexpr size_t ldsSort = (size_t)2 * THREADS * ITEMS * sizeof(uint32_t);                  \
-    if (ldsSort > 48 * 1024)                                                                    \
-      F3S_HIP_CHECK(hipFuncSetAttribute(                                                        \
-          reinterpret_cast<const void*>(&window_rank_sort_kernel<WW, ITEMS, THREADS>),          \
-          hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsSort));                           \
-    hipLaunchKernelGGL((window_rank_sort_kernel<WW, ITEMS, THREADS>), dim3(GRID), dim3(THREADS),\
-                       ldsSort, stream, rowPtr, colIdx, N, colBits, blockPartition,             \
-                       edgeToColumn, edgeToRow, hdr, QUEUE, LEN, COUNTER);                      \
-    F3S_HIP_CHECK(hipGetLastError());                                                           \
-  } while (0)
-      const int medGrid = nRW < 1024 ? nRW : 1024;
-      const int largeGrid = nRW < 256 ? nRW : 256;
-      if (W == 16) {
-        F3S_SORT(16, kMedItems, kMedThreads, medGrid, keysA, &hdr->nMed, &hdr->nextMed);
-        F3S_SORT(16, kLargeItems, kLargeThreads, largeGrid, keysB, &hdr->nLarge, &hdr->nextLarge);
-      } else {
-        F3S_SORT(8, kMedItems, kMedThreads, medGrid, keysA, &hdr->nMed, &hdr->nextMed);
-        F3S_SORT(8, kLargeItems, kLargeThreads, largeGrid, keysB, &hdr->nLarge, &hdr->nextLarge);
-      }
-#undef F3S_SORT
-    }
-#define F3S_RANK(WW, TBB)                                                                     \
-  hipLaunchKernelGGL((window_rank_kernel<WW, TBB>), dim3(rankGrid), dim3(TBB), lds, stream,   \
-                     rowPtr, colIdx, N, range, nPasses, blockPartition,                       \
-                     edgeToColumn, edgeToRow, hdr, queue, colBits <= 22 ? kBinsMax : kSortMax)
-    // the queue lives in the buffer finalize_count_kernel later uses for its values and is
-    // drained by at most two workgroups per CU (2048 of them took 25 us to find an empty queue)
-    const int rankGrid = big ? nRW : (nRW < 512 ? nRW : 512);
-    if (W == 16) {
-      if (big) F3S_RANK(16, 512); else F3S_RANK(16, 256);
-    } else {
-      if (big) F3S_RANK(8, 512); else F3S_RANK(8, 256);
-    }
-#undef F3S_RANK
-    F3S_HIP_CHECK(hipGetLastError());
-  }
-  return enqueue_finalize(N, W, blockPartition, rowWindowOffset, sortedRowWindows, ws, stream);
+                  const ResultPtr& result, hipStream_t stream) {
+  if (int rc = enqueue_rank(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
+                            result.error, stream))
+    return rc;
+  return enqueue_finalize(N, W, blockPartition, rowWindowOffset, sortedRowWindows, ws, result.nTcb,
+                          stream);
 }
+
+// Pinned host memory for the results of calls that wait for the device: a slot per call in progress,
+// taken from pages of 64 slots that stay with the library (one page unless more than 64 host
+// threads preprocess at a time).
+struct HostResult {
+  long long nTcb;
+  int error;
+  int pad[13];
+};
+static_assert(sizeof(HostResult) == 64, "a line of its own");
+class HostResultLease {
+ public:
+  int take() {
+    std::lock_guard<std::mutex> lock(mutex_());
+    auto& free = free_();
+    if (free.empty()) {
+      void* page = nullptr;
+      F3S_HIP_CHECK(hipHostMalloc(&page, 64 * sizeof(HostResult), hipHostMallocPortable));
+      for (int i = 0; i < 64; i++) free.push_back(static_cast<HostResult*>(page) + i);
+    }
+    slot_ = free.back();
+    free.pop_back();
+    slot_->nTcb = 0;
+    slot_->error = 0;
+    return 0;
+  }
+  ~HostResultLease() {
+    if (!slot_) return;
+    std::lock_guard<std::mutex> lock(mutex_());
+    free_().push_back(slot_);
+  }
+  ResultPtr pointers() const { return {&slot_->nTcb, &slot_->error}; }
+  // after the stream is done
+  const volatile HostResult& value() const { return *slot_; }
+
+ private:
+  static std::mutex& mutex_() {
+    static std::mutex m;
+    return m;
+  }
+  static std::vector<HostResult*>& free_() {
+    static std::vector<HostResult*> v;
+    return v;
+  }
+  HostResult* slot_ = nullptr;
+};
 
 int check_count_args(const char* who, int N, int E, int H, int W) {
   if (H != 16 || (W != 16 && W != 8))
@@ -2480,15 +2693,18 @@ int launch_preprocess_count(const int32_t* rowPtr, const int32_t* colIdx, int N,
   if (wsBytes < preprocess_workspace_bytes(N, E))
     return fail(-2, "f3s_preprocess_count: workspace %zu B < required %zu B", wsBytes,
                 preprocess_workspace_bytes(N, E));
-  char* ws = static_cast<char*>(workspace);
-  if (int rc = enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
-                             rowWindowOffset, sortedRowWindows, ws, stream))
-    return rc;
-  WsHeader host;
-  F3S_HIP_CHECK(hipMemcpyAsync(&host, ws, sizeof(WsHeader), hipMemcpyDeviceToHost, stream));
-  F3S_HIP_CHECK(hipStreamSynchronize(stream));
-  if (host.error) return fail(-4, "f3s_preprocess_count: column index outside [0, %d)", N);
-  *nTcbHost = host.nTcb;
+  HostResultLease result;
+  if (int rc = result.take()) return rc;
+  int rc = enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
+                         rowWindowOffset, sortedRowWindows, static_cast<char*>(workspace),
+                         result.pointers(), stream);
+  // also after a failed launch: the slot must not be written to any more when it is given back
+  const hipError_t done = hipStreamSynchronize(stream);
+  if (rc != 0) return rc;
+  F3S_HIP_CHECK(done);
+  if (result.value().error)
+    return fail(-4, "f3s_preprocess_count: column index outside [0, %d)", N);
+  *nTcbHost = result.value().nTcb;
   return 0;
 }
 
@@ -2518,10 +2734,9 @@ int static_scratch(char** out) {
   return 0;
 }
 
-__global__ void publish_result_kernel(const WsHeader* __restrict__ hdr,
-                                      long long* __restrict__ result) {
-  result[0] = hdr->nTcb;
-  result[1] = (long long)hdr->error;
+__global__ void clear_result_kernel(long long* result) {
+  result[0] = 0;
+  result[1] = 0;
 }
 
 }  // namespace
@@ -2540,55 +2755,91 @@ int launch_preprocess_count_static(const int32_t* rowPtr, const int32_t* colIdx,
                 N, preprocess_workspace_bytes(N, E), kStaticScratchBytes);
   char* ws = nullptr;
   if (int rc = static_scratch(&ws)) return rc;
-  // every kernel below starts from a header it clears itself and overwrites whatever else it
-  // reads of the buffer, so nothing of an earlier call survives into this one
-  if (int rc = enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
-                             rowWindowOffset, sortedRowWindows, ws, stream))
-    return rc;
-  hipLaunchKernelGGL(publish_result_kernel, dim3(1), dim3(1), 0, stream,
-                     reinterpret_cast<const WsHeader*>(ws),
-                     reinterpret_cast<long long*>(resultDev));
+  // every kernel below overwrites whatever it reads of the buffer, so nothing of an earlier call
+  // survives into this one
+  auto* result = reinterpret_cast<long long*>(resultDev);
+  hipLaunchKernelGGL(clear_result_kernel, dim3(1), dim3(1), 0, stream, result);
   F3S_HIP_CHECK(hipGetLastError());
-  return 0;
+  // the error flag is the low half of the second value
+  return enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
+                       rowWindowOffset, sortedRowWindows, ws,
+                       {result, reinterpret_cast<int*>(result + 1)}, stream);
 }
 
 namespace {
 
-// Enqueues phase 2. `hdr` (may be null) is the header phase 1 left on the device: with it the
-// kernels do nothing after a column index error, so that phase 2 can follow phase 1 on the stream
-// without the host in between.
-int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W,
-                 const int32_t* edgeToColumn, const int32_t* rowWindowOffset, const WsHeader* hdr,
-                 int32_t* tcblockRowid, uint8_t* tcblocktileId, int32_t* tcblockOffset,
-                 int32_t* sparseAToXidx, uint64_t* bitmap, hipStream_t stream) {
+// Enqueues phase 2. With sortedRowWindows (not null, at most kFinSingleMax windows) the last launch
+// writes the window order too, from blockPartition.
+template <int W>
+int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
+                 const int32_t* edgeToColumn, const int32_t* rowWindowOffset,
+                 const int32_t* blockPartition, int32_t* sortedRowWindows, int32_t* tcblockRowid,
+                 uint8_t* tcblocktileId, int32_t* tcblockOffset, int32_t* sparseAToXidx,
+                 uint64_t* bitmap, hipStream_t stream) {
   const int nRW = (N + kWinRows - 1) / kWinRows;
   auto bm = reinterpret_cast<unsigned long long*>(bitmap);
-  // Graphs of windows with thousands of edges: eight waves per window. Others: a wave per window of
-  // at most kBinsMax edges, and at most five workgroups per CU for the longer ones.
-#define F3S_FILL(WW)                                                                            \
+  // Graphs of windows with thousands of edges: eight waves per window.
+  if (long_windows(nRW, E)) {
+    auto kernel = window_fill_kernel<W, 512, kFillChunk, kFillChunkGeneric>;
+    constexpr size_t lds = fill_lds_bytes<W>(kFillChunk, kFillChunkGeneric);
+    hipLaunchKernelGGL(kernel, dim3(nRW), dim3(512), lds, stream, rowPtr, colIdx, N, E,
+                       edgeToColumn, rowWindowOffset, tcblockRowid, tcblocktileId, tcblockOffset,
+                       sparseAToXidx, bm);
+    F3S_HIP_CHECK(hipGetLastError());
+    return 0;
+  }
+  hipLaunchKernelGGL((window_fill_short_kernel<W>),
+                     dim3(nRW), dim3(64),
+                     0, stream, rowPtr, colIdx, N, E, nRW, edgeToColumn, rowWindowOffset,
+                     tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bm);
+  F3S_HIP_CHECK(hipGetLastError());
+  // few long windows (at most kFillFewLong, and as windows have at most half of kBinsMax edges on
+  // average, commonly far fewer): the large workgroups take all of them, which saves a launch
+  // (169k-node R-MAT graph: 20 us instead of 15 + 20; 60k nodes of 50 neighbours, 800 edges per
+  // window: 103 us for the call, against 118 this way)
+  int minEdges = kBinsMax;
+  const bool few = E / kBinsMax <= kFillFewLong && E / nRW <= kBinsMax / 2;
+  if (!few) {
+    auto mid = window_fill_long_kernel<W, 256, kFillChunkMid, false>;
+    constexpr size_t lds = fill_lds_bytes<W>(kFillChunkMid, kFillChunkMid);
+    hipLaunchKernelGGL(mid, dim3(long_grid(nRW, E, minEdges, 8192)), dim3(256), lds, stream, rowPtr, colIdx, N, E, nRW,
+                       edgeToColumn, rowWindowOffset, minEdges, kFillMid, blockPartition,
+                       sortedRowWindows, tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx,
+                       bm);
+    F3S_HIP_CHECK(hipGetLastError());
+    minEdges = kFillMid;
+  }
+  size_t lds = fill_lds_bytes<W>(kFillChunkLong, kFillChunkLong);
+  const unsigned grid = long_grid(nRW, E, minEdges, 255);
+  if (sortedRowWindows) {
+    const size_t order = order_lds_words(nRW) * sizeof(uint32_t);
+    if (lds < order) lds = order;
+  }
+#define F3S_LONG(ORDER_, GRID)                                                                  \
   do {                                                                                          \
-    if (long_windows(nRW, E)) {                                                                 \
-      hipLaunchKernelGGL((window_fill_kernel<WW, 512, kFillChunk, kFillChunkGeneric>),          \
-                         dim3(nRW), dim3(512), 0, stream, rowPtr, colIdx, N, E, edgeToColumn,   \
-                         rowWindowOffset, hdr, tcblockRowid, tcblocktileId, tcblockOffset,      \
-                         sparseAToXidx, bm);                                                    \
-    } else {                                                                                    \
-      hipLaunchKernelGGL((window_fill_short_kernel<WW>),                                        \
-                         dim3((unsigned)((nRW + kFillWaves - 1) / kFillWaves)),                 \
-                         dim3(kFillWaves * 64), 0, stream, rowPtr, colIdx, N, E, nRW,           \
-                         edgeToColumn, rowWindowOffset, hdr, tcblockRowid, tcblocktileId,       \
-                         tcblockOffset, sparseAToXidx, bm);                                     \
-      F3S_HIP_CHECK(hipGetLastError());                                                         \
-      hipLaunchKernelGGL((window_fill_long_kernel<WW, 256, kFillChunkLong, kFillChunkLong>),    \
-                         dim3((unsigned)min(1280, nRW)), dim3(256), 0, stream, rowPtr, colIdx,  \
-                         N, E, nRW, edgeToColumn, rowWindowOffset, hdr, tcblockRowid,           \
-                         tcblocktileId, tcblockOffset, sparseAToXidx, bm);                      \
-    }                                                                                           \
+    auto kernel = window_fill_long_kernel<W, 1024, kFillChunkLong, ORDER_>;                     \
+    if (int rc = allow_lds(kernel, lds)) return rc;                                             \
+    hipLaunchKernelGGL(kernel, dim3(GRID), dim3(1024), lds, stream, rowPtr, colIdx, N, E, nRW,  \
+                       edgeToColumn, rowWindowOffset, minEdges, 0x7FFFFFFF, blockPartition,     \
+                       sortedRowWindows, tcblockRowid, tcblocktileId, tcblockOffset,            \
+                       sparseAToXidx, bm);                                                      \
   } while (0)
-  if (W == 16) F3S_FILL(16); else F3S_FILL(8);
-#undef F3S_FILL
+  if (sortedRowWindows) F3S_LONG(true, grid + 1); else F3S_LONG(false, grid);
+#undef F3S_LONG
   F3S_HIP_CHECK(hipGetLastError());
   return 0;
+}
+int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W,
+                 const int32_t* edgeToColumn, const int32_t* rowWindowOffset,
+                 const int32_t* blockPartition, int32_t* sortedRowWindows, int32_t* tcblockRowid,
+                 uint8_t* tcblocktileId, int32_t* tcblockOffset, int32_t* sparseAToXidx,
+                 uint64_t* bitmap, hipStream_t stream) {
+  return W == 16 ? enqueue_fill<16>(rowPtr, colIdx, N, E, edgeToColumn, rowWindowOffset,
+                                    blockPartition, sortedRowWindows, tcblockRowid, tcblocktileId,
+                                    tcblockOffset, sparseAToXidx, bitmap, stream)
+                 : enqueue_fill<8>(rowPtr, colIdx, N, E, edgeToColumn, rowWindowOffset,
+                                   blockPartition, sortedRowWindows, tcblockRowid, tcblocktileId,
+                                   tcblockOffset, sparseAToXidx, bitmap, stream);
 }
 
 }  // namespace
@@ -2607,8 +2858,8 @@ int launch_preprocess_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, 
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
   }
-  return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, nullptr, tcblockRowid,
-                      tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
+  return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, nullptr, nullptr,
+                      tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
 }
 
 // ------------------------------------------------------- both phases behind one call
@@ -2617,6 +2868,79 @@ int64_t preprocess_capacity(int N, int64_t E, int W) {
   const int64_t nRW = ((int64_t)N + kWinRows - 1) / kWinRows;
   return (E + W - 1) / W + nRW;
 }
+
+namespace {
+
+// Both phases, with nothing of the host in between.
+int enqueue_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W,
+                       int32_t* blockPartition, int32_t* edgeToColumn, int32_t* edgeToRow,
+                       int32_t* rowWindowOffset, int32_t* sortedRowWindows, int32_t* tcblockRowid,
+                       uint8_t* tcblocktileId, int32_t* tcblockOffset, int32_t* sparseAToXidx,
+                       uint64_t* bitmap, char* ws, const ResultPtr& result, hipStream_t stream) {
+  const int nRW = (N + kWinRows - 1) / kWinRows;
+  const bool aligned16 =
+      ((reinterpret_cast<uintptr_t>(colIdx) | reinterpret_cast<uintptr_t>(edgeToColumn) |
+        reinterpret_cast<uintptr_t>(edgeToRow) | reinterpret_cast<uintptr_t>(sparseAToXidx) |
+        reinterpret_cast<uintptr_t>(tcblocktileId)) & 15u) == 0;
+  // long windows, one bitset pass: the kernels that keep a window's bitset in LDS for both phases
+  if (nRW > 0 && long_windows(nRW, E) && N <= kRangeMax && aligned16) {
+    WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
+    const int range = ((N + 127) / 128) * 128;
+    const int bitsetBytes = ((3 * (range / 64) + 3) & ~3) * 4;  // bitset + per-word prefixes
+    // two workgroups of twelve waves per CU (registers allow no more): half of the CU's LDS each
+    int chunkBytes = (160 * 1024) / 2 - 1024 - bitsetBytes;
+    chunkBytes &= ~255;
+    const size_t ldsCount = (size_t)(range / 32) * 4;
+    const size_t ldsFill = (size_t)bitsetBytes + chunkBytes;
+    hipLaunchKernelGGL(clear_error_kernel, dim3(1), dim3(1), 0, stream, &hdr->error);
+#define F3S_ONECALL(WW)                                                                        \
+  do {                                                                                         \
+    auto rankFill = window_rank_fill_kernel<WW, kRankFillThreads>;                             \
+    if (int rc = allow_lds(rankFill, ldsFill)) return rc;                                      \
+    hipLaunchKernelGGL((window_count_kernel<WW, 512>), dim3(nRW), dim3(512), ldsCount, stream, \
+                       rowPtr, colIdx, N, range, blockPartition, hdr, result.error);           \
+    F3S_HIP_CHECK(hipGetLastError());                                                          \
+    if (int rc = enqueue_finalize(N, W, blockPartition, rowWindowOffset, sortedRowWindows, ws, \
+                                  result.nTcb, stream))                                        \
+      return rc;                                                                               \
+    hipLaunchKernelGGL(rankFill, dim3(nRW), dim3(kRankFillThreads), ldsFill, stream, rowPtr,   \
+                       colIdx, N, E, range, chunkBytes, rowWindowOffset, sortedRowWindows,     \
+                       hdr, edgeToColumn, edgeToRow, tcblockRowid, tcblocktileId,              \
+                       tcblockOffset, sparseAToXidx,                                           \
+                       reinterpret_cast<unsigned long long*>(bitmap));                         \
+    F3S_HIP_CHECK(hipGetLastError());                                                          \
+  } while (0)
+    if (W == 16) F3S_ONECALL(16); else F3S_ONECALL(8);
+#undef F3S_ONECALL
+    return 0;
+  }
+  // Graphs whose windows one workgroup can order: the scan alone stands between the phases, and the
+  // order is made beside the fill (as its own launch in between it took 23 us of the 219 of a call on
+  // 169k nodes).
+  if (nRW > 0 && finalize_waves(nRW) == 0 && !long_windows(nRW, E)) {
+    if (int rc = enqueue_rank(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
+                              result.error, stream))
+      return rc;
+    hipLaunchKernelGGL(window_scan_kernel, dim3(1), dim3(kFinBlock), 0, stream, blockPartition, nRW,
+                       rowWindowOffset, result.nTcb);
+    F3S_HIP_CHECK(hipGetLastError());
+    return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, blockPartition,
+                        sortedRowWindows, tcblockRowid, tcblocktileId, tcblockOffset,
+                        sparseAToXidx, bitmap, stream);
+  }
+  if (int rc = enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
+                             rowWindowOffset, sortedRowWindows, ws, result, stream))
+    return rc;
+  if (nRW == 0) {
+    hipLaunchKernelGGL(set_tail_kernel, dim3(1), dim3(1), 0, stream, tcblockOffset, 0ll, E);
+    F3S_HIP_CHECK(hipGetLastError());
+    return 0;
+  }
+  return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, nullptr, nullptr,
+                      tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
+}
+
+}  // namespace
 
 int launch_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int H, int W,
                       int32_t* blockPartition, int32_t* edgeToColumn, int32_t* edgeToRow,
@@ -2632,64 +2956,18 @@ int launch_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E
     return fail(-2, "f3s_preprocess: block arrays sized for %lld TC blocks, the bound for this "
                     "graph is %lld (f3s_preprocess_capacity)",
                 (long long)capacity, (long long)preprocess_capacity(N, E, W));
-  char* ws = static_cast<char*>(workspace);
-  WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
-  const int nRW = (N + kWinRows - 1) / kWinRows;
-  const bool aligned16 =
-      ((reinterpret_cast<uintptr_t>(colIdx) | reinterpret_cast<uintptr_t>(edgeToColumn) |
-        reinterpret_cast<uintptr_t>(edgeToRow) | reinterpret_cast<uintptr_t>(sparseAToXidx) |
-        reinterpret_cast<uintptr_t>(tcblocktileId)) & 15u) == 0;
-  // long windows, one bitset pass: the kernels that keep a window's bitset in LDS for both phases
-  const bool fused = nRW > 0 && long_windows(nRW, E) && N <= kRangeMax && aligned16;
-  if (fused) {
-    const int range = ((N + 127) / 128) * 128;
-    const int bitsetBytes = ((3 * (range / 64) + 3) & ~3) * 4;  // bitset + per-word prefixes
-    // two workgroups of twelve waves per CU (registers allow no more): half of the CU's LDS each
-    int chunkBytes = (160 * 1024) / 2 - 1024 - bitsetBytes;
-    chunkBytes &= ~255;
-    const size_t ldsCount = (size_t)(range / 32) * 4;
-    const size_t ldsFill = (size_t)bitsetBytes + chunkBytes;
-    hipLaunchKernelGGL(clear_header_kernel, dim3(1), dim3(1), 0, stream, hdr);
-#define F3S_ONECALL(WW)                                                                        \
-  do {                                                                                         \
-    if (ldsFill > 64 * 1024)                                                                   \
-      F3S_HIP_CHECK(hipFuncSetAttribute(                                                       \
-          reinterpret_cast<const void*>(&window_rank_fill_kernel<WW, kRankFillThreads>),                    \
-          hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsFill));                          \
-    hipLaunchKernelGGL((window_count_kernel<WW, 512>), dim3(nRW), dim3(512), ldsCount, stream, \
-                       rowPtr, colIdx, N, range, blockPartition, hdr);                      \
-    F3S_HIP_CHECK(hipGetLastError());                                                          \
-    if (int rc = enqueue_finalize(N, W, blockPartition, rowWindowOffset, sortedRowWindows, ws, \
-                                  stream))                                                     \
-      return rc;                                                                               \
-    hipLaunchKernelGGL((window_rank_fill_kernel<WW, kRankFillThreads>), dim3(nRW),            \
-                       dim3(kRankFillThreads), ldsFill,                                          \
-                       stream, rowPtr, colIdx, N, E, range, chunkBytes, rowWindowOffset,       \
-                       sortedRowWindows, hdr,                                                  \
-                       edgeToColumn, edgeToRow, tcblockRowid, tcblocktileId, tcblockOffset,    \
-                       sparseAToXidx, reinterpret_cast<unsigned long long*>(bitmap));          \
-    F3S_HIP_CHECK(hipGetLastError());                                                          \
-  } while (0)
-    if (W == 16) F3S_ONECALL(16); else F3S_ONECALL(8);
-#undef F3S_ONECALL
-  } else {
-    if (int rc = enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
-                               rowWindowOffset, sortedRowWindows, ws, stream))
-      return rc;
-    if (nRW == 0) {
-      hipLaunchKernelGGL(set_tail_kernel, dim3(1), dim3(1), 0, stream, tcblockOffset, 0ll, E);
-      F3S_HIP_CHECK(hipGetLastError());
-    } else if (int rc = enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, hdr,
-                                     tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx,
-                                     bitmap, stream)) {
-      return rc;
-    }
-  }
-  WsHeader host;
-  F3S_HIP_CHECK(hipMemcpyAsync(&host, ws, sizeof(WsHeader), hipMemcpyDeviceToHost, stream));
-  F3S_HIP_CHECK(hipStreamSynchronize(stream));
-  if (host.error) return fail(-4, "f3s_preprocess: column index outside [0, %d)", N);
-  *nTcbHost = host.nTcb;
+  HostResultLease result;
+  if (int rc = result.take()) return rc;
+  const int rc = enqueue_preprocess(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn,
+                                    edgeToRow, rowWindowOffset, sortedRowWindows, tcblockRowid,
+                                    tcblocktileId, tcblockOffset, sparseAToXidx, bitmap,
+                                    static_cast<char*>(workspace), result.pointers(), stream);
+  // also after a failed launch: the slot must not be written to any more when it is given back
+  const hipError_t done = hipStreamSynchronize(stream);
+  if (rc != 0) return rc;
+  F3S_HIP_CHECK(done);
+  if (result.value().error) return fail(-4, "f3s_preprocess: column index outside [0, %d)", N);
+  *nTcbHost = result.value().nTcb;
   return 0;
 }
 
