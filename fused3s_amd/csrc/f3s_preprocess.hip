@@ -20,10 +20,13 @@
 //                        (reference: sort + inplace_deduplication + binarysearch,
 //                        src/utils.cu:102-153,281-289) is never materialised.
 //   window_scan_kernel, finalize_count_kernel, finalize_*_kernel
-//                        scan of the per-window block counts (src/utils.cu:293-300) and stable LSD
-//                        radix sort of the windows by descending block count
-//                        (src/utils.cu:400-436), ranks from wave ballots: one workgroup, or many on
-//                        graphs of many windows.
+//                        scan of the per-window block counts (src/utils.cu:293-300) and the windows
+//                        by descending block count (src/utils.cu:400-436): places from a histogram
+//                        of the counts, or on graphs of many windows a stable LSD radix sort.
+//   window_rank_all_kernel, window_fill_all_kernel
+//                        the two phases on graphs of up to 16384 windows that are not all long: the
+//                        wave per short window, the workgroup per long one and the order of the
+//                        windows side by side in one launch each.
 //   window_count_kernel, window_rank_fill_kernel
 //                        graphs of long windows through the one-call entry: block counts, then
 //                        ranks, rows, ids, bitmaps and tile ids of a window while its bitset sits
@@ -462,20 +465,21 @@ struct EdgeRows {
 // 432 instead of 332 us).
 constexpr int kRankBins = 1024;
 constexpr int kRankCrowd = 24;  // a fuller bin sends the window to the radix sort
+struct alignas(16) RankBinsLds {  // of one wave
+  uint32_t hist[kRankBins / 2];
+  uint32_t bufA[kBinsMax], bufB[kBinsMax];
+  uint32_t mark[kBinsMax / 32 + 2];
+};
 template <int W>
-__global__ __launch_bounds__(64) void window_rank_bins_kernel(
-    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
-    int colBits, int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
-    int32_t* __restrict__ edgeToRow, int* __restrict__ error) {
+__device__ __forceinline__ void rank_window_by_bins(
+    int w, const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N,
+    int colBits, RankBinsLds& lds, int32_t* __restrict__ blockPartition,
+    int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
+    int* __restrict__ error) {
   constexpr int IDX_BITS = 10;
   constexpr int U = 4;  // groups of 64 edges whose LDS accesses are in flight together
   static_assert(kBinsMax <= (1 << IDX_BITS), "edge position must fit IDX_BITS");
-  __shared__ uint32_t sBufA[kBinsMax];
-  __shared__ uint32_t sBufB[kBinsMax];
-  __shared__ __align__(16) uint32_t sHist[kRankBins / 2];
-  __shared__ __align__(8) uint32_t sMark[kBinsMax / 32 + 2];
-  const int lane = threadIdx.x;
-  const int w = blockIdx.x;
+  const int lane = threadIdx.x & 63;
   const int r0 = w * 16;
   int rowStart = rowPtr[min(r0 + min(lane, 16), N)];
   const int eS = __builtin_amdgcn_readlane(rowStart, 0);
@@ -486,13 +490,13 @@ __global__ __launch_bounds__(64) void window_rank_bins_kernel(
     return;
   }
   if (n > kBinsMax) return;  // left to another kernel
-  uint32_t* a = sBufA;
-  uint32_t* b = sBufB;
-  uint32_t* hist = sHist;
+  uint32_t* a = lds.bufA;
+  uint32_t* b = lds.bufB;
+  uint32_t* hist = lds.hist;
   const unsigned long long leMask = (2ull << lane) - 1ull;
   const int shift = colBits > 10 ? colBits - 10 : 0;
   EdgeRows<kBinsMax> edgeRows;
-  edgeRows.init(sMark, rowStart, lane);
+  edgeRows.init(lds.mark, rowStart, lane);
 #pragma unroll
   for (int k = 0; k < kRankBins / 2 / 256; k++)
     reinterpret_cast<uint4*>(hist)[lane + 64 * k] = make_uint4(0, 0, 0, 0);
@@ -635,38 +639,36 @@ __global__ __launch_bounds__(64) void window_rank_bins_kernel(
   }
   if (lane == 0) blockPartition[w] = (nUniq + W - 1) / W;
 }
+template <int W>
+__global__ __launch_bounds__(64) void window_rank_bins_kernel(
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int colBits,
+    int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
+    int32_t* __restrict__ edgeToRow, int* __restrict__ error) {
+  __shared__ RankBinsLds lds;
+  rank_window_by_bins<W>((int)blockIdx.x, rowPtr, colIdx, N, colBits, lds, blockPartition,
+                         edgeToColumn, edgeToRow, error);
+}
 
-// SCAN: the grid is a fixed number of workgroups that look for the windows of more than minEdges
-// edges (graphs of mostly short windows); else workgroup b takes window b, if it is that long.
-template <int W, int TB, bool SCAN>
-__global__ __launch_bounds__(TB) void window_rank_kernel(
-    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
-    int range, int nPasses, int minEdges, int32_t* __restrict__ blockPartition,
+// One window by the whole workgroup, every edge's column against a bitset in LDS: range / 32 words
+// of bits, then range / 128 group prefixes. Every thread of the workgroup calls this.
+template <int W, int TB>
+__device__ __forceinline__ void rank_window_by_bitset(
+    int w, const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N,
+    int range, int nPasses, int minEdges, uint32_t* bits, int32_t* __restrict__ blockPartition,
     int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
     int* __restrict__ error) {
-  extern __shared__ __align__(16) uint32_t smem[];
-  uint32_t* bits = smem;                 // range/32 words
-  uint32_t* pref = smem + (range >> 5);  // range/128 group prefixes
+  uint32_t* pref = bits + (range >> 5);
   __shared__ int sRow[17];
   __shared__ unsigned sWaveTot[TB / 64];
-  __shared__ int sList[SCAN ? TB : 1];
-  __shared__ int sListLen;
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  for (int64_t first = 0; first < (SCAN ? nRW : 1); first += (int64_t)TB * gridDim.x) {
-  int found = 1;
-  if constexpr (SCAN)
-    found = find_windows(rowPtr, N, nRW, first, (int)gridDim.x, minEdges, 0x7FFFFFFF, sList, &sListLen);
-  for (int k = 0; k < found; k++) {
   __syncthreads();  // the previous window's reads of sRow are done
-  const int w = SCAN ? sList[k] : (int)blockIdx.x;
   const int r0 = w * 16;
   if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
   __syncthreads();
   const int eS = sRow[0], eE = sRow[16];
-  if (eE - eS <= minEdges) break;  // ranked by one wave
+  if (eE - eS <= minEdges) return;  // ranked by one wave
   const int nGroups = range >> 7;
   unsigned uniqueBefore = 0;
   for (int pass = 0; pass < nPasses; pass++) {
@@ -738,15 +740,78 @@ __global__ __launch_bounds__(TB) void window_rank_kernel(
           }
           edgeToColumn[e0 + u * TB] = (int)rank;
         }
+        if (pass == 0) edgeToRow[e0 + u * TB] = r0 + row_of_edge(sRow, e0 + u * TB);
       }
     }
     uniqueBefore = carry;
     __syncthreads();
   }
-  for (int e = eS + tid; e < eE; e += TB) edgeToRow[e] = r0 + row_of_edge(sRow, e);
   if (tid == 0) blockPartition[w] = (int)((uniqueBefore + W - 1) / W);
+}
+
+// SCAN: the grid is a fixed number of workgroups that look for the windows of more than minEdges
+// edges (graphs of mostly short windows); else workgroup b takes window b, if it is that long.
+template <int W, int TB, bool SCAN>
+__global__ __launch_bounds__(TB) void window_rank_kernel(
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
+    int range, int nPasses, int minEdges, int32_t* __restrict__ blockPartition,
+    int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
+    int* __restrict__ error) {
+  extern __shared__ __align__(16) uint32_t smem[];
+  if constexpr (SCAN) {
+    __shared__ int sList[TB];
+    __shared__ int sListLen;
+    for (int64_t first = 0; first < nRW; first += (int64_t)TB * gridDim.x) {
+      const int found = find_windows(rowPtr, N, nRW, first, (int)gridDim.x, minEdges, 0x7FFFFFFF,
+                                     sList, &sListLen);
+      for (int k = 0; k < found; k++)
+        rank_window_by_bitset<W, TB>(sList[k], rowPtr, colIdx, N, range, nPasses, minEdges, smem,
+                                     blockPartition, edgeToColumn, edgeToRow, error);
+    }
+  } else {
+    rank_window_by_bitset<W, TB>((int)blockIdx.x, rowPtr, colIdx, N, range, nPasses, minEdges,
+                                 smem, blockPartition, edgeToColumn, edgeToRow, error);
   }
+}
+
+// Graphs of up to kFinSingleMax windows, most of them short: both kinds of window in one launch. The
+// first longGroups workgroups look for the windows of more than kBinsMax edges and take one at a
+// time with all of their waves, each wave of the others takes one window. One launch after the other
+// meant that everything waited for the longest window twice (169k-node R-MAT graph, windows of up to
+// 12 500 edges: 29 + 23 us; together 39 us with four waves, 44 with eight, which keep more LDS until
+// the last of them is done).
+constexpr int kRankAllThreads = 256;
+template <int W>
+__global__ __launch_bounds__(kRankAllThreads) void window_rank_all_kernel(
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
+    int colBits, int range, int longGroups, int32_t* __restrict__ blockPartition,
+    int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
+    int* __restrict__ error) {
+  extern __shared__ __align__(16) uint32_t smem[];
+  constexpr int NW = kRankAllThreads / 64;
+  if ((int)blockIdx.x >= longGroups) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int w = ((int)blockIdx.x - longGroups) * NW + wave;
+    if (w < nRW)
+      rank_window_by_bins<W>(w, rowPtr, colIdx, N, colBits,
+                             reinterpret_cast<RankBinsLds*>(smem)[wave], blockPartition,
+                             edgeToColumn, edgeToRow, error);
+    return;
   }
+  __shared__ int sList[kRankAllThreads];
+  __shared__ int sListLen;
+  for (int64_t first = 0; first < nRW; first += (int64_t)kRankAllThreads * longGroups) {
+    const int found = find_windows(rowPtr, N, nRW, first, longGroups, kBinsMax, 0x7FFFFFFF, sList,
+                                   &sListLen);
+    for (int k = 0; k < found; k++)
+      rank_window_by_bitset<W, kRankAllThreads>(sList[k], rowPtr, colIdx, N, range, 1, kBinsMax, smem,
+                                              blockPartition, edgeToColumn, edgeToRow, error);
+  }
+}
+constexpr size_t rank_all_lds(int range) {
+  const size_t bins = (kRankAllThreads / 64) * sizeof(RankBinsLds);
+  const size_t bitset = (size_t)(range / 32 + range / 128) * sizeof(uint32_t);
+  return bins > bitset ? bins : bitset;
 }
 
 // Windows too long for a wave on graphs whose column range needs several bitset passes (N >
@@ -1066,10 +1131,8 @@ __global__ __launch_bounds__(THREADS) void window_rank_sort_kernel(
 
 // ------------------------------------------------- scan + window ordering
 constexpr int kFinBlock = 1024;
-// windows the single-workgroup kernel takes: a window id fits kFinIdBits bits and a block count
-// (at most 16 * kFinSingleMax / 8 + 1) the rest of a 32-bit word
+// windows up to which one workgroup scans the counts and order_chunk orders them
 constexpr int kFinSingleMax = 16384;
-constexpr int kFinIdBits = 14;
 
 // Exclusive prefix of the block counts into rowWindowOffset and their total, by one workgroup: every
 // wave owns a contiguous chunk of the windows, all of its loads in flight together.
@@ -1116,139 +1179,97 @@ __device__ __forceinline__ void scan_windows(const int32_t* __restrict__ blockPa
   }
 }
 
-// Windows by descending block count, ties ascending, by one workgroup of kFinBlock threads; every
-// wave owns a contiguous chunk of the windows and walks it on its own (wave-level scans and ballots
-// only), so a pass over the array costs a handful of block barriers instead of several per 1024
-// elements. lds: order_lds_words(nRW) words; a (key, window) pair is one word, key above kFinIdBits
-// bits of window id.
-constexpr size_t order_lds_words(int nRW) { return 2 * (size_t)((nRW + 3) & ~3); }
-__device__ __forceinline__ void order_windows(const int32_t* __restrict__ blockPartition, int nRW,
-                                              int32_t* __restrict__ sortedRowWindows,
-                                              uint32_t* lds) {
-  uint32_t* bufA = lds;
-  uint32_t* bufB = lds + ((nRW + 3) & ~3);
-  constexpr int NW = kFinBlock / 64;
-  __shared__ int sWaveMax[NW];
-  constexpr int DB = 6;               // digit bits per sorting pass: one bin per lane
-  constexpr int NB = 1 << DB;
-  static_assert(NB == 64, "the start computation gives every lane one bin");
-  __shared__ unsigned sCnt[NW][NB];   // per wave: elements per digit, then its running position
+// Positions of windows first .. first + TB - 1 (first: a multiple of TB) in the order by descending
+// block count, ties ascending, into sortedRowWindows, by one workgroup: the counts of all windows
+// become a histogram in LDS (low half of a word: windows with that many blocks, high half: those in
+// front of `first`), its sums from the top the places. No workgroup waits for another one, and
+// nRW / TB of them share the work (a radix sort by one workgroup of 1024 threads took 21 us for
+// 10 584 windows, 30 us for 14 561). Counts from nBins - 1 on share the last bin; the few windows
+// that have so many compare themselves with all others. hist: nBins words, a multiple of TB.
+template <int TB>
+__device__ __forceinline__ void order_chunk(const int32_t* __restrict__ blockPartition, int nRW,
+                                            int first, int nBins,
+                                            int32_t* __restrict__ sortedRowWindows,
+                                            uint32_t* hist) {
+  static_assert(kFinSingleMax < 0x8000, "two counters of windows per word");
+  constexpr int NW = TB / 64;
+  constexpr int U = 4;
+  __shared__ unsigned sBinTot[NW];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int chunk = (((nRW + NW - 1) / NW) + 63) & ~63;
-  const int cBegin = min(wave * chunk, nRW);
-  const int cEnd = min(cBegin + chunk, nRW);
-
-  // ---- the counts into LDS first, every thread's loads in flight together (each later pass walks
-  // its chunk group by group, and a global load per group would cost its full latency every time),
-  // and their maximum
-  {
-    constexpr int U = 4;
-    int mx = 0;
-    for (int i0 = tid; i0 < nRW; i0 += U * kFinBlock) {
-      int v[U];
+  const int top = nBins - 1;
+  for (int i = tid; i < nBins; i += TB) hist[i] = 0u;
+  __syncthreads();
+  for (int i0 = 0; i0 < nRW; i0 += U * TB) {
+    int c[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int i = i0 + u * kFinBlock;
-        v[u] = i < nRW ? blockPartition[i] : 0;
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int i = i0 + u * kFinBlock;
-        if (i < nRW) bufB[i] = (uint32_t)v[u];
-        mx = max(mx, v[u]);
-      }
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + u * TB + tid;
+      c[u] = i < nRW ? min(blockPartition[i], top) : -1;
     }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) mx = max(mx, __shfl_xor(mx, off));
-    if (lane == 0) sWaveMax[wave] = mx;
+    for (int u = 0; u < U; u++) {
+      // counts cluster, and lanes that name the same bin are served one after the other: the lanes
+      // that agree with the group's first one are counted with one ballot and added once
+      const int c0 = __builtin_amdgcn_readfirstlane(c[u]);
+      const unsigned one = i0 + u * TB + wave * 64 < first ? 0x10001u : 1u;
+      const unsigned long long same = __ballot(c[u] == c0);
+      if (c[u] >= 0 && c[u] != c0) atomicAdd(&hist[c[u]], one);
+      if (c0 >= 0 && lane == 0) atomicAdd(&hist[c0], one * (unsigned)__popcll(same));
+    }
   }
   __syncthreads();
-  int maxC = 0;
+  {  // where each bin's windows of this chunk start; thread t owns nBins / TB bins from the top
+    const int per = nBins / TB;
+    unsigned total = 0;
+    for (int k = 0; k < per; k++) total += hist[top - (tid * per + k)] & 0xFFFFu;
+    const unsigned incl = wave_inclusive_scan(total, lane);
+    if (lane == 63) sBinTot[wave] = incl;
+    __syncthreads();
+    unsigned run = incl - total;
 #pragma unroll
-  for (int k = 0; k < NW; k++) maxC = max(maxC, sWaveMax[k]);
-
-  // ---- stable sort by descending count == stable ascending LSD radix sort of (maxC - count),
-  // six bits per pass
-  int nBits = 0;
-  while ((maxC >> nBits) != 0) nBits++;
-  const int nPass = (nBits + DB - 1) / DB;
-  if (nPass == 0) {
-    for (int i = tid; i < nRW; i += kFinBlock) sortedRowWindows[i] = i;
-    return;
+    for (int k = 0; k < NW; k++) run += k < wave ? sBinTot[k] : 0u;
+    for (int k = 0; k < per; k++) {
+      const uint32_t v = hist[top - (tid * per + k)];
+      hist[top - (tid * per + k)] = run + (v >> 16);
+      run += v & 0xFFFFu;
+    }
   }
-  const unsigned long long ltMask = (1ull << lane) - 1ull;
-  for (int pass = 0; pass < nPass; pass++) {
-    const int shift = kFinIdBits + pass * DB;
-    const bool last = pass == nPass - 1;
-    uint32_t* dst = (pass & 1) ? bufB : bufA;
-    const uint32_t* src = (pass & 1) ? bufA : bufB;
-    __syncthreads();  // the previous pass's writes are visible, its use of sCnt is over
-    sCnt[wave][lane] = 0;
-    // peers = lanes of this 64-element group with the same digit (one ballot per digit bit)
-    auto digit_peers = [&](bool valid, int dgt) {
-      unsigned long long peers = __ballot(valid);
-#pragma unroll
-      for (int b = 0; b < DB; b++) {
-        const unsigned long long bal = __ballot((dgt >> b) & 1);
-        peers &= ((dgt >> b) & 1) ? bal : ~bal;
-      }
-      return peers;
-    };
-    auto load_key = [&](int i) -> unsigned {
-      if (i >= cEnd) return 0u;
-      // the first pass finds the counts themselves in bufB
-      return pass == 0 ? ((unsigned)(maxC - (int)src[i]) << kFinIdBits) | (unsigned)i : src[i];
-    };
-    // histogram of the wave's chunk: LDS atomics (the whole workgroup shares one CU's vector
-    // ALUs, and a ballot per digit bit costs far more instructions than the atomic's conflicts)
-    // Counts cluster (most windows of a skewed graph share a digit), and lanes that name the same
-    // bin are served one after the other: the lanes that agree with the group's first one are
-    // counted with one ballot and added once.
+  const int i = first + tid;
+  const int count = i < nRW ? blockPartition[i] : -1;
+  const bool binned = count >= 0 && count < top;
+  unsigned long long peers = __ballot(binned);
+  for (int b = 0; (top >> b) != 0; b++) {
+    const unsigned long long bal = __ballot((count >> b) & 1);
+    peers &= ((count >> b) & 1) ? bal : ~bal;
+  }
+  for (int turn = 0; turn < NW; turn++) {  // ties go by window: one wave after the other
+    __syncthreads();
+    if (wave != turn) continue;
+    const unsigned at = binned ? hist[count] : 0u;
     wave_lds_sync();
-    for (int base = cBegin; base < cEnd; base += 64) {
-      const int i = base + lane;
-      const bool valid = i < cEnd;
-      const int dgt = (int)(load_key(i) >> shift) & (NB - 1);
-      const int d0 = __builtin_amdgcn_readfirstlane(dgt);
-      const unsigned long long same = __ballot(valid && dgt == d0);
-      if (valid && dgt != d0) atomicAdd(&sCnt[wave][dgt], 1u);
-      if (lane == 0) atomicAdd(&sCnt[wave][d0], (unsigned)__popcll(same));
-    }
-    __syncthreads();
-    // start of (digit = lane, wave): all smaller digits, then the same digit in earlier waves
-    unsigned digitTotal = 0, before = 0;
-#pragma unroll
-    for (int k = 0; k < NW; k++) {
-      const unsigned cnt = sCnt[k][lane];
-      digitTotal += cnt;
-      if (k < wave) before += cnt;
-    }
-    const unsigned start = wave_inclusive_scan(digitTotal, lane) - digitTotal + before;
-    __syncthreads();
-    sCnt[wave][lane] = start;
-    // scatter, in order (the next group's key is in flight during this one's)
-    unsigned keyNext = load_key(cBegin + lane);
-    for (int base = cBegin; base < cEnd; base += 64) {
-      const int i = base + lane;
-      const bool valid = i < cEnd;
-      const unsigned key = keyNext;
-      keyNext = load_key(i + 64);
-      const int dgt = (int)(key >> shift) & (NB - 1);
-      const unsigned long long peers = digit_peers(valid, dgt);
-      if (valid) dst[sCnt[wave][dgt] + __popcll(peers & ltMask)] = key;
-      // the last peer moves the digit's running position (the wave's LDS accesses stay in order)
-      if (valid && (peers >> lane) == 1ull) sCnt[wave][dgt] += __popcll(peers);
-    }
-    if (last) {
-      // the order leaves LDS as whole lines: scattered 4-byte stores from the last pass would
-      // all go through this one CU's address unit, 64 lines per instruction
-      __syncthreads();
-      for (int i = tid; i < nRW; i += kFinBlock)
-        sortedRowWindows[i] = (int)(dst[i] & ((1u << kFinIdBits) - 1u));
+    if (binned) {
+      sortedRowWindows[at + __popcll(peers & ((1ull << lane) - 1ull))] = i;
+      if ((peers >> lane) == 1ull) hist[count] = at + (unsigned)__popcll(peers);
     }
   }
+  for (unsigned long long left = __ballot(count >= top); left != 0ull; left &= left - 1ull) {
+    const int src = __builtin_ctzll(left);
+    const int c = __builtin_amdgcn_readlane(count, src), w = first + wave * 64 + src;
+    unsigned before = 0;
+    for (int k = lane; k < nRW; k += 64) {
+      const int x = blockPartition[k];
+      before += (x > c || (x == c && k < w)) ? 1u : 0u;
+    }
+    before = wave_inclusive_scan(before, lane);
+    if (lane == 63) sortedRowWindows[before] = w;
+  }
+}
+// bins for the counts that the windows of a graph can have, within 16 KiB
+constexpr int order_bins(int N, int W) {
+  const int bins = ((N / W + 2) + 1023) & ~1023;
+  return bins < 4096 ? bins : 4096;
 }
 
 __global__ __launch_bounds__(kFinBlock) void window_scan_kernel(
@@ -1257,17 +1278,22 @@ __global__ __launch_bounds__(kFinBlock) void window_scan_kernel(
   scan_windows(blockPartition, nRW, rowWindowOffset, nTcb);
 }
 
+// workgroup 0 scans the counts, each of the others orders kFinBlock windows
 __global__ __launch_bounds__(kFinBlock) void finalize_count_kernel(
-    const int32_t* __restrict__ blockPartition, int nRW, int32_t* __restrict__ rowWindowOffset,
-    int32_t* __restrict__ sortedRowWindows, long long* __restrict__ nTcb) {
+    const int32_t* __restrict__ blockPartition, int nRW, int nBins,
+    int32_t* __restrict__ rowWindowOffset, int32_t* __restrict__ sortedRowWindows,
+    long long* __restrict__ nTcb) {
   extern __shared__ __align__(16) uint32_t finLds[];
-  scan_windows(blockPartition, nRW, rowWindowOffset, nTcb);
-  order_windows(blockPartition, nRW, sortedRowWindows, finLds);
+  if (blockIdx.x == 0)
+    scan_windows(blockPartition, nRW, rowWindowOffset, nTcb);
+  else
+    order_chunk<kFinBlock>(blockPartition, nRW, ((int)blockIdx.x - 1) * kFinBlock, nBins,
+                           sortedRowWindows, finLds);
 }
 
 // ---- the same scan + stable sort spread over many workgroups, for graphs with many windows.
 // Every WAVE of the grid owns a contiguous chunk of the windows (chunks in wave order), exactly as
-// the waves of finalize_count_kernel do; what that kernel exchanges through LDS and block barriers
+// the waves of scan_windows do; what they exchange through LDS and block barriers
 // goes through small global arrays and kernel boundaries here:
 //   finalize_partials_kernel   per-wave sum and maximum of the block counts
 //   finalize_scan_kernel       rowWindowOffset of the chunk (carry = sums of the earlier waves),
@@ -1666,8 +1692,8 @@ constexpr size_t fill_lds_bytes(int tc, int tcg) {
 }
 template <int W, int TB, int TC, int TCG>
 __device__ __forceinline__ void fill_one_window(
-    int w, int nRW, const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N,
-    int E, const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
+    int w, int base, int nb, const int32_t* __restrict__ rowPtr,
+    const int32_t* __restrict__ colIdx, int N, int E, const int32_t* __restrict__ edgeToColumn,
     unsigned char* sRaw, int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
     int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
@@ -1683,9 +1709,6 @@ __device__ __forceinline__ void fill_one_window(
   const int lane = tid & 63;
   const int wave = tid >> 6;
   if (tid == 0) sUnsorted = 0u;
-  if (w == 0 && tid == 0) tcblockOffset[rowWindowOffset[nRW]] = E;
-  const int base = rowWindowOffset[w];
-  const int nb = rowWindowOffset[w + 1] - base;
   if (nb == 0) return;
   const int r0 = w * 16;
   if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
@@ -1816,35 +1839,35 @@ __device__ __forceinline__ void fill_one_window(
 // vector instructions. Workgroups of one wave, 22 per CU (of four: 260 instead of 220 us for the 149k
 // such windows of a 61M-edge graph).
 template <int W>
-__global__ __launch_bounds__(64) void window_fill_short_kernel(
-    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
-    const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
-    int32_t* __restrict__ tcblockRowid,
-    uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
-    int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
+struct alignas(16) FillShortLds {  // of one wave
+  static constexpr int MAXB = (kBinsMax + W - 1) / W;  // TC blocks of a window at most
+  unsigned long long bm[MAXB * (16 * W / 64)];
+  uint32_t ids[MAXB * W];
+  uint8_t tile[kBinsMax + 8];
+  alignas(8) uint32_t mark[kBinsMax / 32 + 2];
+};
+template <int W>
+__device__ __forceinline__ void fill_short_window(
+    int w, int base, int nb, const int32_t* __restrict__ rowPtr,
+    const int32_t* __restrict__ colIdx, int N, const int32_t* __restrict__ edgeToColumn,
+    FillShortLds<W>& lds, int32_t* __restrict__ tcblockRowid, uint8_t* __restrict__ tcblocktileId,
+    int32_t* __restrict__ tcblockOffset, int32_t* __restrict__ sparseAToXidx,
+    unsigned long long* __restrict__ bitmap) {
   constexpr int WPT = 16 * W / 64;
   constexpr int LOGW = (W == 16) ? 4 : 3;
-  constexpr int MAXB = (kBinsMax + W - 1) / W;  // TC blocks of a window at most
+  constexpr int MAXB = FillShortLds<W>::MAXB;
   constexpr int U = 4;  // groups of 64 edges in flight together
-  __shared__ __align__(16) unsigned long long sBm[MAXB * WPT];
-  __shared__ __align__(16) uint32_t sIds[MAXB * W];
-  __shared__ __align__(16) uint8_t sTile[kBinsMax + 8];
-  __shared__ __align__(8) uint32_t sMark[kBinsMax / 32 + 2];
-  static_assert(MAXB * 8 <= MAXB * W, "edges per (block, row), two counters per word, fit sIds");
-  const int lane = threadIdx.x;
-  const int w = blockIdx.x;
+  static_assert(MAXB * 8 <= MAXB * W, "edges per (block, row), two counters per word, fit ids");
+  const int lane = threadIdx.x & 63;
   int rowStart = rowPtr[min(w * 16 + min(lane, 16), N)];
-  const int base = __builtin_amdgcn_readfirstlane(rowWindowOffset[w]);
-  const int nb = __builtin_amdgcn_readfirstlane(rowWindowOffset[w + 1]) - base;
   const int eS = __builtin_amdgcn_readlane(rowStart, 0);
   const int n = __builtin_amdgcn_readlane(rowStart, 16) - eS;
   rowStart -= eS;
-  if (w == nRW - 1 && lane == 0) tcblockOffset[base + nb] = E;
-  if (n == 0 || n > kBinsMax || nb > MAXB) return;  // long ones: window_fill_long_kernel
-  unsigned long long* bm = sBm;
-  uint32_t* ids = sIds;
+  if (n == 0 || n > kBinsMax || nb > MAXB) return;  // long ones: fill_one_window
+  unsigned long long* bm = lds.bm;
+  uint32_t* ids = lds.ids;
   EdgeRows<kBinsMax> edgeRows;
-  edgeRows.init(sMark, rowStart, lane);
+  edgeRows.init(lds.mark, rowStart, lane);
   for (int i = lane; i < nb * WPT / 2; i += 64)
     reinterpret_cast<uint4*>(bm)[i] = make_uint4(0, 0, 0, 0);
   for (int i = nb * W - W + lane; i < nb * W; i += 64) ids[i] = 0u;  // unused slots hold 0
@@ -1884,7 +1907,7 @@ __global__ __launch_bounds__(64) void window_fill_short_kernel(
     store_streaming(reinterpret_cast<uint4*>(sparseAToXidx + (int64_t)base * W) + i,
                     reinterpret_cast<const uint4*>(ids)[i]);
   if (__ballot(rough) == 0ull) {
-    uint8_t* stage = sTile;
+    uint8_t* stage = lds.tile;
     const unsigned skew = (unsigned)((uintptr_t)(tcblocktileId + eS) & 3u);
     unsigned carry = 0;
     for (int k = 0; k < 2 * nb; k += 64) {
@@ -1982,6 +2005,22 @@ __global__ __launch_bounds__(64) void window_fill_short_kernel(
   }
 }
 
+template <int W>
+__global__ __launch_bounds__(64) void window_fill_short_kernel(
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
+    const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
+    int32_t* __restrict__ tcblockRowid, uint8_t* __restrict__ tcblocktileId,
+    int32_t* __restrict__ tcblockOffset, int32_t* __restrict__ sparseAToXidx,
+    unsigned long long* __restrict__ bitmap) {
+  __shared__ FillShortLds<W> lds;
+  const int w = blockIdx.x;
+  const int base = __builtin_amdgcn_readfirstlane(rowWindowOffset[w]);
+  const int nb = __builtin_amdgcn_readfirstlane(rowWindowOffset[w + 1]) - base;
+  if (w == nRW - 1 && threadIdx.x == 0) tcblockOffset[base + nb] = E;
+  fill_short_window<W>(w, base, nb, rowPtr, colIdx, N, edgeToColumn, lds, tcblockRowid,
+                       tcblocktileId, tcblockOffset, sparseAToXidx, bitmap);
+}
+
 template <int W, int TB, int TC, int TCG>
 __global__ __launch_bounds__(TB) void window_fill_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E,
@@ -1990,46 +2029,141 @@ __global__ __launch_bounds__(TB) void window_fill_kernel(
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
     int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
   extern __shared__ __align__(16) unsigned char sRawDyn[];
-  fill_one_window<W, TB, TC, TCG>((int)blockIdx.x, (int)gridDim.x, rowPtr, colIdx, N, E,
-                                  edgeToColumn, rowWindowOffset, sRawDyn, tcblockRowid, tcblocktileId,
-                                  tcblockOffset, sparseAToXidx, bitmap);
+  const int w = blockIdx.x;
+  if (w == 0 && threadIdx.x == 0) tcblockOffset[rowWindowOffset[gridDim.x]] = E;
+  const int base = rowWindowOffset[w];
+  fill_one_window<W, TB, TC, TCG>(w, base, rowWindowOffset[w + 1] - base, rowPtr, colIdx, N, E,
+                                  edgeToColumn, sRawDyn, tcblockRowid, tcblocktileId, tcblockOffset,
+                                  sparseAToXidx, bitmap);
 }
 
 // The windows that window_fill_short_kernel leaves out, of more than minEdges and at most maxEdges
 // edges (find_windows). Two sizes: 256 threads and 320 TC blocks of LDS at a time for windows of up to
 // kFillMid edges (five workgroups per CU), 1024 threads and 1280 blocks for longer ones, which would
 // otherwise each keep one small workgroup busy long after the others are done (31 700 edges:
-// 190 us). On graphs of few windows the large workgroups take both.
-// ORDER: the last workgroup writes the window order meanwhile, which no other kernel of the call waits for.
-template <int W, int TB, int TC, bool ORDER>
+// 190 us).
+template <int W, int TB, int TC>
 __global__ __launch_bounds__(TB) void window_fill_long_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
     const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
-    int minEdges, int maxEdges, const int32_t* __restrict__ blockPartition,
-    int32_t* __restrict__ sortedRowWindows, int32_t* __restrict__ tcblockRowid,
+    int minEdges, int maxEdges, int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
     int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
   extern __shared__ __align__(16) unsigned char sRawDyn[];
   __shared__ int sList[TB];
   __shared__ int sListLen;
-  if constexpr (ORDER) {
-    static_assert(TB == kFinBlock, "the order is one such workgroup's work");
-    if (blockIdx.x == gridDim.x - 1) {
-      order_windows(blockPartition, nRW, sortedRowWindows, reinterpret_cast<uint32_t*>(sRawDyn));
-      return;
-    }
-  }
-  const int stride = (int)gridDim.x - (ORDER ? 1 : 0);
-  for (int64_t first = 0; first < nRW; first += (int64_t)TB * stride) {
-    const int found = find_windows(rowPtr, N, nRW, first, stride, minEdges, maxEdges, sList,
+  for (int64_t first = 0; first < nRW; first += (int64_t)TB * gridDim.x) {
+    const int found = find_windows(rowPtr, N, nRW, first, (int)gridDim.x, minEdges, maxEdges, sList,
                                    &sListLen);
     for (int k = 0; k < found; k++) {
       __syncthreads();  // the window before this one has left the LDS arrays
-      fill_one_window<W, TB, TC, TC>(sList[k], nRW, rowPtr, colIdx, N, E, edgeToColumn,
-                                     rowWindowOffset, sRawDyn, tcblockRowid, tcblocktileId,
+      const int w = sList[k], base = rowWindowOffset[w];
+      fill_one_window<W, TB, TC, TC>(w, base, rowWindowOffset[w + 1] - base, rowPtr, colIdx, N, E,
+                                     edgeToColumn, sRawDyn, tcblockRowid, tcblocktileId,
                                      tcblockOffset, sparseAToXidx, bitmap);
     }
   }
+}
+
+// Sum of counts[0 .. n) by the whole workgroup; every thread calls this and gets the sum.
+template <int TB>
+__device__ __forceinline__ int sum_counts(const int32_t* __restrict__ counts, int n) {
+  __shared__ unsigned sSum[TB / 64];
+  unsigned sum = 0;
+  for (int i = threadIdx.x; i < n; i += TB) sum += (unsigned)counts[i];
+  sum = wave_inclusive_scan(sum, threadIdx.x & 63);
+  __syncthreads();  // the reads of the call before this one are done
+  if ((threadIdx.x & 63) == 63) sSum[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  unsigned total = 0;
+#pragma unroll
+  for (int k = 0; k < TB / 64; k++) total += sSum[k];
+  return (int)total;
+}
+
+// Phase 2 of a graph of up to kFinSingleMax windows, most of them short, in one launch like
+// window_rank_all_kernel: workgroups that look for the long windows, then some that make the window
+// order (unless orderGroups is 0), which nothing else of the call waits for, then those of the short
+// windows. 169k-node R-MAT graph: 17 + 25 us as two launches, 29 us together; with four waves and half the
+// blocks of a long window at a time 52 us, with sixteen and twice as many 37 us.
+// SELF: no scan was launched before; every workgroup adds up the counts in front of its windows itself
+// and the short ones' write rowWindowOffset and the total. That is one launch (4 us) less where the sums
+// are short, a few counts per thread: up to kSelfScanMax windows.
+constexpr int kFillAllThreads = 512;
+constexpr int kFillAllChunk = 576;  // TC blocks: 54 KiB of LDS, as much as the short windows take
+constexpr int kSelfScanMax = 2048;
+template <int W, bool SELF>
+__global__ __launch_bounds__(kFillAllThreads) void window_fill_all_kernel(
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
+    const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ blockPartition,
+    int longGroups, int orderGroups, int nBins, int32_t* __restrict__ rowWindowOffset,
+    int32_t* __restrict__ sortedRowWindows, long long* __restrict__ nTcb,
+    int32_t* __restrict__ tcblockRowid, uint8_t* __restrict__ tcblocktileId,
+    int32_t* __restrict__ tcblockOffset, int32_t* __restrict__ sparseAToXidx,
+    unsigned long long* __restrict__ bitmap) {
+  extern __shared__ __align__(16) unsigned char sRawDyn[];
+  constexpr int TB = kFillAllThreads, NW = TB / 64;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = (int)blockIdx.x - longGroups - orderGroups;
+  if (group >= 0) {
+    const int w = group * NW + wave;
+    int base, nb;
+    if constexpr (SELF) {
+      base = sum_counts<TB>(blockPartition, group * NW);
+      if (w >= nRW) return;
+      const unsigned c = lane <= wave ? (unsigned)blockPartition[group * NW + lane] : 0u;
+      nb = __builtin_amdgcn_readlane((int)c, wave);
+      base += __builtin_amdgcn_readlane((int)wave_inclusive_scan(c, lane), 63) - nb;
+      if (lane == 0) {
+        if (w == 0) rowWindowOffset[0] = 0;
+        rowWindowOffset[w + 1] = base + nb;
+        if (w == nRW - 1) *nTcb = base + nb;
+      }
+    } else {
+      if (w >= nRW) return;
+      base = __builtin_amdgcn_readfirstlane(rowWindowOffset[w]);
+      nb = __builtin_amdgcn_readfirstlane(rowWindowOffset[w + 1]) - base;
+    }
+    if (w == nRW - 1 && lane == 0) tcblockOffset[base + nb] = E;
+    fill_short_window<W>(w, base, nb, rowPtr, colIdx, N, edgeToColumn,
+                         reinterpret_cast<FillShortLds<W>*>(sRawDyn)[wave], tcblockRowid,
+                         tcblocktileId, tcblockOffset, sparseAToXidx, bitmap);
+    return;
+  }
+  if ((int)blockIdx.x >= longGroups) {
+    order_chunk<TB>(blockPartition, nRW, ((int)blockIdx.x - longGroups) * TB, nBins,
+                    sortedRowWindows, reinterpret_cast<uint32_t*>(sRawDyn));
+    return;
+  }
+  __shared__ int sList[TB];
+  __shared__ int sListLen;
+  for (int64_t first = 0; first < nRW; first += (int64_t)TB * longGroups) {
+    const int found = find_windows(rowPtr, N, nRW, first, longGroups, kBinsMax, 0x7FFFFFFF, sList,
+                                   &sListLen);
+    for (int k = 0; k < found; k++) {
+      __syncthreads();  // the window before this one has left the LDS arrays
+      const int w = sList[k];
+      int base, nb;
+      if constexpr (SELF) {
+        base = sum_counts<TB>(blockPartition, w);
+        nb = blockPartition[w];
+      } else {
+        base = rowWindowOffset[w];
+        nb = rowWindowOffset[w + 1] - base;
+      }
+      fill_one_window<W, TB, kFillAllChunk, kFillAllChunk>(
+          w, base, nb, rowPtr, colIdx, N, E, edgeToColumn, sRawDyn, tcblockRowid, tcblocktileId,
+          tcblockOffset, sparseAToXidx, bitmap);
+    }
+  }
+}
+template <int W>
+constexpr size_t fill_all_lds(int nBins) {
+  size_t lds = (kFillAllThreads / 64) * sizeof(FillShortLds<W>);
+  if (lds < fill_lds_bytes<W>(kFillAllChunk, kFillAllChunk))
+    lds = fill_lds_bytes<W>(kFillAllChunk, kFillAllChunk);
+  return lds > nBins * sizeof(uint32_t) ? lds : nBins * sizeof(uint32_t);
 }
 
 // ------------------------------------------------------------------ both phases, one call
@@ -2508,10 +2642,11 @@ int enqueue_finalize(int N, int W, const int32_t* blockPartition, int32_t* rowWi
   int32_t* valsTmp = reinterpret_cast<int32_t*>(ws + kWsHeaderBytes + 2 * seg);
   const int finWaves = finalize_waves(nRW);
   if (finWaves == 0) {
-    const size_t lds = order_lds_words(nRW) * sizeof(uint32_t);
-    if (int rc = allow_lds(finalize_count_kernel, lds)) return rc;
-    hipLaunchKernelGGL(finalize_count_kernel, dim3(1), dim3(kFinBlock), lds, stream,
-                       blockPartition, nRW, rowWindowOffset, sortedRowWindows, nTcb);
+    const int nBins = order_bins(N, W);
+    hipLaunchKernelGGL(finalize_count_kernel,
+                       dim3(1 + (unsigned)((nRW + kFinBlock - 1) / kFinBlock)), dim3(kFinBlock),
+                       nBins * sizeof(uint32_t), stream, blockPartition, nRW, nBins,
+                       rowWindowOffset, sortedRowWindows, nTcb);
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
   }
@@ -2547,6 +2682,17 @@ unsigned long_grid(int nRW, int E, int minEdges, int most) {
   return (unsigned)(grid > most ? most : grid);
 }
 
+// Graphs whose short and long windows share a launch in both phases. Above kFinSingleMax windows the
+// workgroups of one wave are the better ones: with more than four rounds of windows on every CU the
+// LDS that a finished wave keeps until its workgroup ends costs more than the overlap gives.
+bool one_launch(int nRW, int64_t E) { return nRW <= kFinSingleMax && !long_windows(nRW, E); }
+// Their workgroups for windows of more than kBinsMax edges: where such windows are the exception two per CU
+// (with one for each that there can be, most look in vain and the short windows wait for their
+// slots), else as above.
+unsigned all_long_groups(int nRW, int E) {
+  return long_grid(nRW, E, kBinsMax, E / nRW <= kBinsMax / 2 ? 512 : kFinSingleMax);
+}
+
 // Enqueues the kernels that rank the windows' columns and count their TC blocks.
 template <int W>
 int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
@@ -2562,10 +2708,21 @@ int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
   // position, else the bitonic network on bare column ids
   int colBits = 0;
   while (colBits < 31 && ((int64_t)1 << colBits) < (int64_t)N) colBits++;
+  if (one_launch(nRW, E)) {
+    const unsigned groups = all_long_groups(nRW, E);
+    const size_t ldsAll = rank_all_lds(range);
+    if (int rc = allow_lds(window_rank_all_kernel<W>, ldsAll)) return rc;
+    hipLaunchKernelGGL(window_rank_all_kernel<W>,
+                       dim3(groups + (unsigned)((nRW + kRankAllThreads / 64 - 1) / (kRankAllThreads / 64))),
+                       dim3(kRankAllThreads), ldsAll, stream, rowPtr, colIdx, N, nRW, colBits, range,
+                       (int)groups, blockPartition, edgeToColumn, edgeToRow, error);
+    F3S_HIP_CHECK(hipGetLastError());
+    return 0;
+  }
   int shortMax = kBinsMax;
   if (colBits <= 22) {
     hipLaunchKernelGGL(window_rank_bins_kernel<W>, dim3(nRW), dim3(64), 0, stream, rowPtr,
-                       colIdx, N, nRW, colBits, blockPartition, edgeToColumn, edgeToRow, error);
+                       colIdx, N, colBits, blockPartition, edgeToColumn, edgeToRow, error);
   } else {
     shortMax = kSortMax;
     hipLaunchKernelGGL(window_rank_small_kernel<W>, dim3(nRW), dim3(64), 0, stream,
@@ -2768,14 +2925,15 @@ int launch_preprocess_count_static(const int32_t* rowPtr, const int32_t* colIdx,
 
 namespace {
 
-// Enqueues phase 2. With sortedRowWindows (not null, at most kFinSingleMax windows) the last launch
-// writes the window order too, from blockPartition.
+// Enqueues phase 2. With sortedRowWindows (not null: at most kFinSingleMax windows, and mostly short
+// ones) the window order is written too, from blockPartition; with nTcb (not null: at most
+// kSelfScanMax of them) rowWindowOffset and the total as well.
 template <int W>
 int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
-                 const int32_t* edgeToColumn, const int32_t* rowWindowOffset,
-                 const int32_t* blockPartition, int32_t* sortedRowWindows, int32_t* tcblockRowid,
-                 uint8_t* tcblocktileId, int32_t* tcblockOffset, int32_t* sparseAToXidx,
-                 uint64_t* bitmap, hipStream_t stream) {
+                 const int32_t* edgeToColumn, int32_t* rowWindowOffset,
+                 const int32_t* blockPartition, int32_t* sortedRowWindows, long long* nTcb,
+                 int32_t* tcblockRowid, uint8_t* tcblocktileId, int32_t* tcblockOffset,
+                 int32_t* sparseAToXidx, uint64_t* bitmap, hipStream_t stream) {
   const int nRW = (N + kWinRows - 1) / kWinRows;
   auto bm = reinterpret_cast<unsigned long long*>(bitmap);
   // Graphs of windows with thousands of edges: eight waves per window.
@@ -2788,58 +2946,60 @@ int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
   }
-  hipLaunchKernelGGL((window_fill_short_kernel<W>),
-                     dim3(nRW), dim3(64),
-                     0, stream, rowPtr, colIdx, N, E, nRW, edgeToColumn, rowWindowOffset,
-                     tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bm);
+  if (one_launch(nRW, E)) {
+    const unsigned longGroups = all_long_groups(nRW, E);
+    const unsigned orderGroups =
+        sortedRowWindows ? (unsigned)((nRW + kFillAllThreads - 1) / kFillAllThreads) : 0;
+    constexpr int NW = kFillAllThreads / 64;
+    const unsigned grid = longGroups + orderGroups + (unsigned)((nRW + NW - 1) / NW);
+    const int nBins = order_bins(N, W);
+    const size_t lds = fill_all_lds<W>(nBins);
+    auto kernel = nTcb ? window_fill_all_kernel<W, true> : window_fill_all_kernel<W, false>;
+    if (int rc = allow_lds(kernel, lds)) return rc;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kFillAllThreads), lds, stream, rowPtr, colIdx, N, E,
+                       nRW, edgeToColumn, blockPartition, (int)longGroups, (int)orderGroups, nBins,
+                       rowWindowOffset, sortedRowWindows, nTcb, tcblockRowid, tcblocktileId,
+                       tcblockOffset, sparseAToXidx, bm);
+    F3S_HIP_CHECK(hipGetLastError());
+    return 0;
+  }
+  hipLaunchKernelGGL((window_fill_short_kernel<W>), dim3(nRW), dim3(64), 0, stream, rowPtr, colIdx, N,
+                     E, nRW, edgeToColumn, rowWindowOffset, tcblockRowid, tcblocktileId,
+                     tcblockOffset, sparseAToXidx, bm);
   F3S_HIP_CHECK(hipGetLastError());
   // few long windows (at most kFillFewLong, and as windows have at most half of kBinsMax edges on
   // average, commonly far fewer): the large workgroups take all of them, which saves a launch
-  // (169k-node R-MAT graph: 20 us instead of 15 + 20; 60k nodes of 50 neighbours, 800 edges per
-  // window: 103 us for the call, against 118 this way)
   int minEdges = kBinsMax;
   const bool few = E / kBinsMax <= kFillFewLong && E / nRW <= kBinsMax / 2;
   if (!few) {
-    auto mid = window_fill_long_kernel<W, 256, kFillChunkMid, false>;
+    auto mid = window_fill_long_kernel<W, 256, kFillChunkMid>;
     constexpr size_t lds = fill_lds_bytes<W>(kFillChunkMid, kFillChunkMid);
-    hipLaunchKernelGGL(mid, dim3(long_grid(nRW, E, minEdges, 8192)), dim3(256), lds, stream, rowPtr, colIdx, N, E, nRW,
-                       edgeToColumn, rowWindowOffset, minEdges, kFillMid, blockPartition,
-                       sortedRowWindows, tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx,
-                       bm);
+    hipLaunchKernelGGL(mid, dim3(long_grid(nRW, E, minEdges, 8192)), dim3(256), lds, stream, rowPtr,
+                       colIdx, N, E, nRW, edgeToColumn, rowWindowOffset, minEdges, kFillMid,
+                       tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bm);
     F3S_HIP_CHECK(hipGetLastError());
     minEdges = kFillMid;
   }
-  size_t lds = fill_lds_bytes<W>(kFillChunkLong, kFillChunkLong);
-  const unsigned grid = long_grid(nRW, E, minEdges, 255);
-  if (sortedRowWindows) {
-    const size_t order = order_lds_words(nRW) * sizeof(uint32_t);
-    if (lds < order) lds = order;
-  }
-#define F3S_LONG(ORDER_, GRID)                                                                  \
-  do {                                                                                          \
-    auto kernel = window_fill_long_kernel<W, 1024, kFillChunkLong, ORDER_>;                     \
-    if (int rc = allow_lds(kernel, lds)) return rc;                                             \
-    hipLaunchKernelGGL(kernel, dim3(GRID), dim3(1024), lds, stream, rowPtr, colIdx, N, E, nRW,  \
-                       edgeToColumn, rowWindowOffset, minEdges, 0x7FFFFFFF, blockPartition,     \
-                       sortedRowWindows, tcblockRowid, tcblocktileId, tcblockOffset,            \
-                       sparseAToXidx, bm);                                                      \
-  } while (0)
-  if (sortedRowWindows) F3S_LONG(true, grid + 1); else F3S_LONG(false, grid);
-#undef F3S_LONG
+  auto kernel = window_fill_long_kernel<W, 1024, kFillChunkLong>;
+  constexpr size_t lds = fill_lds_bytes<W>(kFillChunkLong, kFillChunkLong);
+  if (int rc = allow_lds(kernel, lds)) return rc;
+  hipLaunchKernelGGL(kernel, dim3(long_grid(nRW, E, minEdges, 255)), dim3(1024), lds, stream, rowPtr,
+                     colIdx, N, E, nRW, edgeToColumn, rowWindowOffset, minEdges, 0x7FFFFFFF,
+                     tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bm);
   F3S_HIP_CHECK(hipGetLastError());
   return 0;
 }
 int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W,
-                 const int32_t* edgeToColumn, const int32_t* rowWindowOffset,
-                 const int32_t* blockPartition, int32_t* sortedRowWindows, int32_t* tcblockRowid,
-                 uint8_t* tcblocktileId, int32_t* tcblockOffset, int32_t* sparseAToXidx,
-                 uint64_t* bitmap, hipStream_t stream) {
+                 const int32_t* edgeToColumn, int32_t* rowWindowOffset,
+                 const int32_t* blockPartition, int32_t* sortedRowWindows, long long* nTcb,
+                 int32_t* tcblockRowid, uint8_t* tcblocktileId, int32_t* tcblockOffset,
+                 int32_t* sparseAToXidx, uint64_t* bitmap, hipStream_t stream) {
   return W == 16 ? enqueue_fill<16>(rowPtr, colIdx, N, E, edgeToColumn, rowWindowOffset,
-                                    blockPartition, sortedRowWindows, tcblockRowid, tcblocktileId,
-                                    tcblockOffset, sparseAToXidx, bitmap, stream)
+                                    blockPartition, sortedRowWindows, nTcb, tcblockRowid,
+                                    tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream)
                  : enqueue_fill<8>(rowPtr, colIdx, N, E, edgeToColumn, rowWindowOffset,
-                                   blockPartition, sortedRowWindows, tcblockRowid, tcblocktileId,
-                                   tcblockOffset, sparseAToXidx, bitmap, stream);
+                                   blockPartition, sortedRowWindows, nTcb, tcblockRowid,
+                                   tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
 }
 
 }  // namespace
@@ -2858,8 +3018,9 @@ int launch_preprocess_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, 
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
   }
-  return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, nullptr, nullptr,
-                      tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
+  // the offsets are only read: without nTcb nothing writes them
+  return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, const_cast<int32_t*>(rowWindowOffset),
+                      nullptr, nullptr, nullptr, tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
 }
 
 // ------------------------------------------------------- both phases behind one call
@@ -2914,19 +3075,21 @@ int enqueue_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int 
 #undef F3S_ONECALL
     return 0;
   }
-  // Graphs whose windows one workgroup can order: the scan alone stands between the phases, and the
-  // order is made beside the fill (as its own launch in between it took 23 us of the 219 of a call on
-  // 169k nodes).
-  if (nRW > 0 && finalize_waves(nRW) == 0 && !long_windows(nRW, E)) {
+  // At most the scan stands between the phases; the order is made beside the fill (as its own launch in
+  // between it took 23 us of the 219 of a call on 169k nodes).
+  if (nRW > 0 && one_launch(nRW, E)) {
     if (int rc = enqueue_rank(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
                               result.error, stream))
       return rc;
-    hipLaunchKernelGGL(window_scan_kernel, dim3(1), dim3(kFinBlock), 0, stream, blockPartition, nRW,
-                       rowWindowOffset, result.nTcb);
-    F3S_HIP_CHECK(hipGetLastError());
+    const bool self = nRW <= kSelfScanMax;
+    if (!self) {
+      hipLaunchKernelGGL(window_scan_kernel, dim3(1), dim3(kFinBlock), 0, stream, blockPartition,
+                         nRW, rowWindowOffset, result.nTcb);
+      F3S_HIP_CHECK(hipGetLastError());
+    }
     return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, blockPartition,
-                        sortedRowWindows, tcblockRowid, tcblocktileId, tcblockOffset,
-                        sparseAToXidx, bitmap, stream);
+                        sortedRowWindows, self ? result.nTcb : nullptr, tcblockRowid,
+                        tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
   }
   if (int rc = enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
                              rowWindowOffset, sortedRowWindows, ws, result, stream))
@@ -2937,7 +3100,7 @@ int enqueue_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int 
     return 0;
   }
   return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, nullptr, nullptr,
-                      tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
+                      nullptr, tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
 }
 
 }  // namespace

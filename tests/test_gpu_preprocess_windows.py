@@ -65,3 +65,33 @@ def test_window_sizes(oracle_mod, N, columns, W):
             assert np.array_equal(got[k].cpu().numpy(), want[k]), (k, two_phase)
         bm = got["tcbBitMap"].cpu().view(torch.int64).numpy().view(np.uint64)
         assert np.array_equal(bm, want["tcbBitMap"]), two_phase
+
+
+# Windows on both sides of 2048 (each workgroup adds up the counts in front of it, or a scan is
+# launched) and of 16 384 (one launch per phase, or one per kind of window), counts that tie, counts
+# beyond the last bin of the window order, and graphs without edges
+@pytest.mark.parametrize("nRW,edges,wide", [(1, 0, 0), (8, 5, 0), (9, 20, 1), (2047, 3, 1),
+                                            (2048, 2, 2), (2049, 2, 2), (16_384, 1, 2),
+                                            (16_385, 1, 2)])
+@pytest.mark.parametrize("W", [16, 8])
+def test_window_counts(oracle_mod, nRW, edges, wide, W):
+    from fused3s_amd import capi
+    print("case window counts nRW=%d edges=%d wide=%d W=%d" % (nRW, edges, wide, W), flush=True)
+    rng = np.random.default_rng(nRW + W)
+    N = 16 * nRW - 5
+    degree = rng.integers(0, edges + 1, N) if edges else np.zeros(N, np.int64)
+    for k in range(wide):  # 40 000 edges: more than 4095 blocks of 8 columns
+        degree[16 * int(rng.integers(nRW - 1))] = min(N, 40_000)
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(degree)
+    colIdx = np.concatenate([np.sort(rng.choice(N, size=int(k), replace=False)) if k > 100 else
+                             np.sort(rng.integers(0, N, int(k))) for k in degree]).astype(np.int32)
+    want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, W)
+    rp, ci = torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda()
+    for two_phase in (False, True):
+        got = capi.preprocess(rp, ci, N, 16, W, two_phase=two_phase)
+        assert got["blockCount"] == want["blockCount"]
+        for k in KEYS:
+            assert np.array_equal(got[k].cpu().numpy(), want[k]), (k, two_phase)
+        bm = got["tcbBitMap"].cpu().view(torch.int64).numpy().view(np.uint64)
+        assert np.array_equal(bm, want["tcbBitMap"]), two_phase
