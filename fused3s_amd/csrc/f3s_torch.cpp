@@ -108,8 +108,8 @@ preprocess_gpu(torch::Tensor edgeList, torch::Tensor nodePointer, int num_nodes,
                             reinterpret_cast<uint64_t*>(tcbBitMap.data_ptr()), current_stream()),
         "f3s_preprocess_fill");
   } else {
-    // one call: the nTCB-sized arrays are allocated for the bound on the block total and returned as
-    // views of their first nTcb entries, so the host waits for the device once, at the end
+    // one call: the nTCB-sized arrays are allocated for the bound on the block total and cut to
+    // their first nTcb entries, so the host waits for the device once, at the end
     TORCH_CHECK(blockSize_h == 16 && (blockSize_w == 16 || blockSize_w == 8),
                 "preprocess_gpu: block ", blockSize_h, "x", blockSize_w,
                 " unsupported (16x16 or 16x8)");
@@ -128,12 +128,16 @@ preprocess_gpu(torch::Tensor edgeList, torch::Tensor nodePointer, int num_nodes,
                        reinterpret_cast<uint64_t*>(tcbBitMap.data_ptr()), workspace.data_ptr(),
                        wsBytes, &nTcb, current_stream()),
         "f3s_preprocess");
-    tcblockRowid = tcblockRowid.narrow(0, 0, nTcb);
-    tcblockOffset = tcblockOffset.narrow(0, 0, nTcb + 1);
-    sparseAToXidx = sparseAToXidx.narrow(0, 0, nTcb * blockSize_w);
-    tcbBitMap = tcbBitMap.narrow(0, 0, nTcb * bmWords);
+    // nobody else holds them yet, so their sizes are set where a view would go through the dispatcher
+    auto shorten = [](torch::Tensor& t, int64_t n) {
+      t.unsafeGetTensorImpl()->set_sizes_contiguous({n});
+    };
+    shorten(tcblockRowid, nTcb);
+    shorten(tcblockOffset, nTcb + 1);
+    shorten(sparseAToXidx, nTcb * blockSize_w);
+    shorten(tcbBitMap, nTcb * bmWords);
     if (nTcb * 2 < cap) {
-      // rows of a window that share columns: far fewer blocks than the bound. The views would keep
+      // rows of a window that share columns: far fewer blocks than the bound. They would keep
       // the whole allocation alive for as long as the caller keeps the structure, so it gets
       // exact-size copies instead (at most half of what was allocated is copied).
       tcblockRowid = tcblockRowid.clone();
@@ -177,25 +181,41 @@ void write_cu_time(const torch::Tensor& timer, int64_t nBlocks, const std::strin
     out << (double)kv.second.first / 1e5 << " " << (double)kv.second.second / 1e5 << std::endl;
 }
 
+// The two events of a call, destroyed whichever way it ends. Nobody waits for the start event, so
+// its packet does without the write-back that makes results visible outside of the GPU (1.6 us).
+struct TimingEvents {
+  hipEvent_t start = nullptr, stop = nullptr;
+  TimingEvents() {
+    TORCH_CHECK(hipEventCreateWithFlags(&start, hipEventDisableSystemFence) == hipSuccess &&
+                hipEventCreate(&stop) == hipSuccess);
+  }
+  ~TimingEvents() {
+    if (start) (void)hipEventDestroy(start);
+    if (stop) (void)hipEventDestroy(stop);
+  }
+};
+
 // Runs `launch(stream)` on PyTorch's current stream between two events, blocks on the stop event
-// like the reference's launchers (src/F3S_kernel.cu:436-451) and returns the elapsed ms.
+// like the reference's launchers (src/F3S_kernel.cu:436-451) and returns the tensors that they
+// return: {time in ms (0-d CPU fp32), out, scores}, an empty one when there are no scores. What the
+// host still has to make it makes while the GPU works: a call on a small graph is mostly latency
+// (2 708 nodes, a kernel of 4 us: 22.4 -> 20.5 us).
 template <typename F>
-float timed_launch(const char* what, F&& launch) {
+std::vector<torch::Tensor> timed_launch(const char* what, const torch::Tensor& out,
+                                        torch::Tensor scores, F&& launch) {
   hipStream_t stream = at::hip::getCurrentHIPStream().stream();
-  hipEvent_t start, stop;
-  TORCH_CHECK(hipEventCreate(&start) == hipSuccess && hipEventCreate(&stop) == hipSuccess);
-  TORCH_CHECK(hipEventRecord(start, stream) == hipSuccess);
+  TimingEvents events;
+  TORCH_CHECK(hipEventRecord(events.start, stream) == hipSuccess);
   const int rc = launch(static_cast<void*>(stream));
-  hipError_t e1 = hipEventRecord(stop, stream);
-  hipError_t e2 = hipEventSynchronize(stop);
-  float ms = 0.f;
-  hipError_t e3 = hipEventElapsedTime(&ms, start, stop);
-  (void)hipEventDestroy(start);
-  (void)hipEventDestroy(stop);
+  hipError_t e1 = hipEventRecord(events.stop, stream);
+  auto time = torch::empty({}, torch::TensorOptions().dtype(torch::kFloat32));
+  if (!scores.defined()) scores = torch::empty({0}, out.options());
+  hipError_t e2 = hipEventSynchronize(events.stop);
+  hipError_t e3 = hipEventElapsedTime(time.data_ptr<float>(), events.start, events.stop);
   check_status(rc, what);
   TORCH_CHECK(e1 == hipSuccess && e2 == hipSuccess && e3 == hipSuccess, "HIP event timing failed: ",
               hipGetErrorString(e2 != hipSuccess ? e2 : (e1 != hipSuccess ? e1 : e3)));
-  return ms;
+  return {time, out, scores};
 }
 
 struct Launch {
@@ -276,7 +296,6 @@ std::vector<torch::Tensor> run_1tb1rw(const torch::Tensor& rowWindowOffset,
   c10::DeviceGuard guard(Q.device());
   auto f32 = torch::TensorOptions().dtype(torch::kFloat32).device(Q.device());
   auto out = torch::empty({(int64_t)nNodes, d}, f32);
-  auto sddmmResult = torch::zeros({0}, f32);
   torch::Tensor timer;
   unsigned long long* timerPtr = nullptr;
   if (L.timerFile) {
@@ -290,7 +309,7 @@ std::vector<torch::Tensor> run_1tb1rw(const torch::Tensor& rowWindowOffset,
   const size_t wsBytes = sliced ? f3s_attention_workspace_bytes(nNodes, (int)d) : 0;
   WorkspaceLease lease(sliced, wsBytes, Q.device());
   torch::Tensor& workspace = lease.tensor;
-  const float ms = timed_launch("f3s_attention_fwd", [&](void* stream) {
+  auto result = timed_launch("f3s_attention_fwd", out, {}, [&](void* stream) {
     return f3s_attention_fwd(
         rowWindowOffset.data_ptr<int>(), L.order ? L.order->data_ptr<int>() : nullptr,
         sparseAToXidx.data_ptr<int>(), reinterpret_cast<const uint64_t*>(tcbBitMap.data_ptr()),
@@ -299,8 +318,7 @@ std::vector<torch::Tensor> run_1tb1rw(const torch::Tensor& rowWindowOffset,
         sliced ? workspace.data_ptr() : nullptr, wsBytes, 0, stream);
   });
   if (L.timerFile) write_cu_time(timer, nRW, L.timerFile);
-  auto time = torch::tensor(ms, torch::TensorOptions().dtype(torch::kFloat32));
-  return {time, out, sddmmResult};
+  return result;
 }
 
 // Multi-head call, beyond the reference's surface: its graph-transformer callers run
@@ -343,7 +361,7 @@ std::vector<torch::Tensor> f3sMultiHeadScaleQK(torch::Tensor rowWindowOffset,
   const size_t wsBytes =
       sliced ? f3s_attention_heads_workspace_bytes(nNodes, (int)nHeads, (int)d) : 0;
   WorkspaceLease lease(sliced, wsBytes, Q.device());
-  const float ms = timed_launch("f3s_attention_fwd_heads", [&](void* stream) {
+  return timed_launch("f3s_attention_fwd_heads", out, {}, [&](void* stream) {
     return f3s_attention_fwd_heads(
         rowWindowOffset.data_ptr<int>(), sortedRowWindows.data_ptr<int>(),
         sparseAToXidx.data_ptr<int>(), reinterpret_cast<const uint64_t*>(tcbBitMap.data_ptr()),
@@ -351,8 +369,6 @@ std::vector<torch::Tensor> f3sMultiHeadScaleQK(torch::Tensor rowWindowOffset,
         K.data_ptr(), V.data_ptr(), Q.stride(0), scalingFactor, 1, out.data_ptr<float>(),
         out.stride(0), sliced ? lease.tensor.data_ptr() : nullptr, wsBytes, 0, stream);
   });
-  auto time = torch::tensor(ms, torch::TensorOptions().dtype(torch::kFloat32));
-  return {time, out, torch::zeros({0}, f32)};
 }
 
 // F3S.f3s_1tb1rw (src/F3S.cpp:145-183)
@@ -437,15 +453,13 @@ std::vector<torch::Tensor> f3s1tb1tcb(torch::Tensor rowWindowOffset, torch::Tens
   auto f32 = torch::TensorOptions().dtype(torch::kFloat32).device(Q.device());
   auto out = torch::empty({(int64_t)nNodes, d}, f32);
   auto sddmmResult = torch::empty({saveSddmmResult ? nTcb * 128 : 0}, f32);
-  const float ms = timed_launch("f3s_attention_fwd_tcb8", [&](void* stream) {
+  return timed_launch("f3s_attention_fwd_tcb8", out, sddmmResult, [&](void* stream) {
     return f3s_attention_fwd_tcb8(
         rowWindowOffset.data_ptr<int>(), nullptr, sparseAToXidx.data_ptr<int>(),
         reinterpret_cast<const uint64_t*>(tcbBitMap.data_ptr()), nNodes, nTcb, (int)d,
         Q.data_ptr(), K.data_ptr(), V.data_ptr(), applySoftmax ? 1 : 0, out.data_ptr<float>(),
         saveSddmmResult ? sddmmResult.data_ptr<float>() : nullptr, stream);
   });
-  auto time = torch::tensor(ms, torch::TensorOptions().dtype(torch::kFloat32));
-  return {time, out, sddmmResult};
 }
 
 }  // namespace
