@@ -19,7 +19,8 @@ EXPORTS = ["f3s_abi_version", "f3s_last_error", "f3s_preprocess_workspace_bytes"
            "f3s_attention_fwd_tcb8", "f3s_attention_uses_workspace",
            "f3s_preprocess_static_scratch_bytes", "f3s_preprocess_count_static",
            "f3s_preprocess_capacity", "f3s_preprocess", "f3s_attention_prepare",
-           "f3s_attention_heads_workspace_bytes", "f3s_attention_uses_wide_offsets"]
+           "f3s_attention_heads_workspace_bytes", "f3s_attention_uses_wide_offsets",
+           "f3s_window_order"]
 
 
 def lib():
@@ -71,6 +72,8 @@ def lib():
         L.f3s_attention_fwd_tcb8.restype = ci
         L.f3s_attention_fwd_tcb8.argtypes = [vp, vp, vp, vp, ci, ctypes.c_int64, ci, vp, vp, vp,
                                              ci, vp, vp, vp]
+        L.f3s_window_order.restype = ci
+        L.f3s_window_order.argtypes = [vp, ci, vp, vp]
         _lib = L
     return _lib
 

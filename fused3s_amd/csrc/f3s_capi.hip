@@ -122,6 +122,12 @@ int f3s_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, i
                                 static_cast<hipStream_t>(stream));
 }
 
+int f3s_window_order(const int32_t* rowWindowOffset, int nRW, int32_t* order, void* stream) {
+  if (nRW > 0 && (!rowWindowOffset || !order))
+    return f3s::fail(-1, "f3s_window_order: null pointer");
+  return f3s::launch_window_order(rowWindowOffset, nRW, order, static_cast<hipStream_t>(stream));
+}
+
 size_t f3s_attention_workspace_bytes(int N, int d) {
   if (N < 0) N = 0;
   if (d < 32) d = 32;

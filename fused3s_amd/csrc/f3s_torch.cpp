@@ -218,6 +218,24 @@ std::vector<torch::Tensor> timed_launch(const char* what, const torch::Tensor& o
   return {time, out, scores};
 }
 
+// Whether a call that came without a window order makes one (f3s_window_order: two launches' time,
+// 5 to 15 us), so that a long window that is far down the list does not start last. Neither the
+// number of windows nor of blocks says how skewed a graph is, so the lines are where no measured
+// graph lost (natural -> own order, in us):
+// - blocks of 16 columns: windows of 32 blocks and more on average (50k nodes, 4.1M edges, d = 96:
+//   192 -> 148; 180k nodes, 40M edges, d = 64: 842 -> 647), from 1024 windows and 128M products of
+//   block columns and d (35k nodes, 3M edges, d = 64, 192M: 106 -> 92; 12k nodes, 3M edges, 750
+//   windows: 49 -> 50). Graphs of shorter windows gain when skewed (R-MAT, 169k nodes: 124 -> 103)
+//   and lose when not (200k nodes, d = 128: 292 -> 300), and stay as they are.
+// - blocks of 8 columns, by a workgroup per window: from 64M products (R-MAT, 65k nodes, d = 128:
+//   122 -> 103; 149k nodes, d = 64: 137 -> 123; below, 24k nodes, d = 128: 53 -> 55).
+bool order_pays(int64_t nRW, int64_t nTCB, int W, int64_t d) {
+  const int64_t products = nTCB * W * d;
+  if (nRW > 16384) return false;  // more than f3s_window_order takes
+  if (W == 8) return products >= (64ll << 20);
+  return nRW >= 1024 && nTCB >= 32 * nRW && products >= (128ll << 20);
+}
+
 struct Launch {
   const torch::Tensor* order;  // nullptr = natural window order
   float scalingFactor;
@@ -309,9 +327,19 @@ std::vector<torch::Tensor> run_1tb1rw(const torch::Tensor& rowWindowOffset,
   const size_t wsBytes = sliced ? f3s_attention_workspace_bytes(nNodes, (int)d) : 0;
   WorkspaceLease lease(sliced, wsBytes, Q.device());
   torch::Tensor& workspace = lease.tensor;
+  // per-CU times are those of the order that was asked for
+  torch::Tensor ownOrder;
+  if (!L.order && !L.timerFile && order_pays(nRW, sparseAToXidx.numel() / 16, 16, d))
+    ownOrder = torch::empty({nRW}, f32.dtype(torch::kInt32));
+  const int* order = L.order ? L.order->data_ptr<int>()
+                             : (ownOrder.defined() ? ownOrder.data_ptr<int>() : nullptr);
   auto result = timed_launch("f3s_attention_fwd", out, {}, [&](void* stream) {
+    if (ownOrder.defined())
+      if (int rc = f3s_window_order(rowWindowOffset.data_ptr<int>(), (int)nRW,
+                                    ownOrder.data_ptr<int>(), stream))
+        return rc;
     return f3s_attention_fwd(
-        rowWindowOffset.data_ptr<int>(), L.order ? L.order->data_ptr<int>() : nullptr,
+        rowWindowOffset.data_ptr<int>(), order,
         sparseAToXidx.data_ptr<int>(), reinterpret_cast<const uint64_t*>(tcbBitMap.data_ptr()),
         nNodes, sparseAToXidx.numel() / 16, (int)d, dtype, Q.data_ptr(), K.data_ptr(),
         V.data_ptr(), L.scalingFactor, L.applySoftmax ? 1 : 0, out.data_ptr<float>(), timerPtr,
@@ -453,9 +481,16 @@ std::vector<torch::Tensor> f3s1tb1tcb(torch::Tensor rowWindowOffset, torch::Tens
   auto f32 = torch::TensorOptions().dtype(torch::kFloat32).device(Q.device());
   auto out = torch::empty({(int64_t)nNodes, d}, f32);
   auto sddmmResult = torch::empty({saveSddmmResult ? nTcb * 128 : 0}, f32);
+  torch::Tensor order;
+  if (order_pays(nRW, nTcb, 8, d)) order = torch::empty({nRW}, f32.dtype(torch::kInt32));
   return timed_launch("f3s_attention_fwd_tcb8", out, sddmmResult, [&](void* stream) {
+    if (order.defined())
+      if (int rc = f3s_window_order(rowWindowOffset.data_ptr<int>(), (int)nRW,
+                                    order.data_ptr<int>(), stream))
+        return rc;
     return f3s_attention_fwd_tcb8(
-        rowWindowOffset.data_ptr<int>(), nullptr, sparseAToXidx.data_ptr<int>(),
+        rowWindowOffset.data_ptr<int>(), order.defined() ? order.data_ptr<int>() : nullptr,
+        sparseAToXidx.data_ptr<int>(),
         reinterpret_cast<const uint64_t*>(tcbBitMap.data_ptr()), nNodes, nTcb, (int)d,
         Q.data_ptr(), K.data_ptr(), V.data_ptr(), applySoftmax ? 1 : 0, out.data_ptr<float>(),
         saveSddmmResult ? sddmmResult.data_ptr<float>() : nullptr, stream);

@@ -249,3 +249,42 @@ def test_1tb1tcb_call_sequence(oracle_mod, d):
         assert np.abs(got_s - want_s).max() <= 1e-5 * max(1.0, np.abs(want_s).max())
         t2, out2, empty = F3S.f3s_1tb1tcb(rwo, atox, bitmap, N, Qd, Kd, Vd, softmax, False)
         assert empty.numel() == 0 and torch.equal(out2, out)
+
+
+@pytest.mark.parametrize("W,edges,ordered", [(16, 70, False), (16, 170, True), (8, 40, False),
+                                             (8, 90, True)])
+def test_calls_without_a_window_order(oracle_mod, W, edges, ordered):
+    """On both sides of the line from which such a call makes an order of its own (as `ordered` says):
+    windows that are empty, ordinary and far down the list long ones."""
+    from fused3s_amd import F3S
+    print("case no window order W=%d edges=%d" % (W, edges), flush=True)
+    N, d = 16_384 + 21, 64
+    nRW = (N + 15) // 16
+    rng = np.random.default_rng(edges)
+    deg = np.full(N, edges)
+    deg[rng.random(N) < 0.05] = 0
+    deg[12_000:12_016] = 1500
+    deg[-3:] = 900
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(deg)
+    colIdx = np.concatenate([np.sort(rng.choice(N, size=k, replace=False)) for k in deg])
+    res, *_ = preprocess_like_the_reference(F3S, rowPtr, colIdx.astype(np.int32), N, W)
+    rwo, order, _, _, _, atox, bm, count = res
+    line = (128 << 20) if W == 16 else (64 << 20)
+    assert (count * W * d >= line) == ordered
+    Q, K, V = (torch.rand((N, d), device="cuda", generator=torch.Generator("cuda").manual_seed(i))
+               .half() for i in range(3))
+    if W == 16:
+        out = F3S.f3s_1tb1rw(rwo, atox, bm, N, Q, K, V, 8, True, False)[1]
+    else:
+        out = F3S.f3s_1tb1tcb(rwo, atox, bm, N, Q, K, V, True, False)[1]
+    rows = np.concatenate([np.arange(0, N, 257), np.arange(11_990, 12_020), np.arange(N - 20, N)])
+    Qh, Kh, Vh = (x.float().cpu().numpy() for x in (Q, K, V))
+    for r in rows:
+        c = colIdx[rowPtr[r]:rowPtr[r + 1]]
+        want = np.zeros(d, np.float32)
+        if len(c):
+            s = Kh[c] @ Qh[r]
+            p = np.exp(s - s.max())
+            want = (p / p.sum()) @ Vh[c]
+        np.testing.assert_allclose(out[r].cpu().numpy(), want, atol=MAX_ABS, rtol=1e-2)

@@ -95,3 +95,24 @@ def test_window_counts(oracle_mod, nRW, edges, wide, W):
             assert np.array_equal(got[k].cpu().numpy(), want[k]), (k, two_phase)
         bm = got["tcbBitMap"].cpu().view(torch.int64).numpy().view(np.uint64)
         assert np.array_equal(bm, want["tcbBitMap"]), two_phase
+
+
+@pytest.mark.parametrize("nRW", [1, 511, 512, 513, 2048, 4097, 16_384])
+def test_window_order_alone(nRW):
+    """Long windows first, equal counts by window; from 512 blocks on, 64 bins an octave."""
+    from fused3s_amd import capi
+    print("case window order nRW=%d" % nRW, flush=True)
+    rng = np.random.default_rng(nRW)
+    count = rng.integers(0, 40, nRW)
+    far = rng.random(nRW) < 0.1
+    count[far] = rng.choice([511, 512, 513, 1023, 1024, 5000, 100_000], size=int(far.sum()))
+    rwo = torch.zeros(nRW + 1, dtype=torch.int32, device="cuda")
+    rwo[1:] = torch.as_tensor(np.cumsum(count), device="cuda")
+    order = torch.full((nRW,), -1, dtype=torch.int32, device="cuda")
+    rc = capi.lib().f3s_window_order(capi._ptr(rwo), nRW, capi._ptr(order), capi._stream())
+    assert rc == 0, capi.lib().f3s_last_error()
+    bucket = np.where(count < 512, count, 0)
+    for octave in range(9, 17):
+        inside = (count >> octave) == 1
+        bucket[inside] = 512 + (octave - 9) * 64 + ((count[inside] >> (octave - 6)) & 63)
+    np.testing.assert_array_equal(order.cpu().numpy(), np.argsort(-bucket, kind="stable"))
