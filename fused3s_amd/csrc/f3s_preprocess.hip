@@ -1881,6 +1881,7 @@ __device__ __forceinline__ void fill_short_window(
   const int n = __builtin_amdgcn_readlane(rowStart, 16) - eS;
   rowStart -= eS;
   if (n == 0 || n > kBinsMax || nb > MAXB) return;  // long ones: fill_one_window
+  if (nb < 1) return;  // no block to write: every column of the window lay outside [0, N)
   unsigned long long* bm = lds.bm;
   uint32_t* ids = lds.ids;
   EdgeRows<kBinsMax> edgeRows;

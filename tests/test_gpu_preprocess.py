@@ -294,6 +294,34 @@ def test_out_of_range_column_is_an_error():
         capi.preprocess(rowPtr.cuda(), cols.cuda(), N)
 
 
+# 1 and 40 edges: a wave per window; 1000: ranked by a wave, filled by a workgroup
+@pytest.mark.parametrize("W", [16, 8])
+@pytest.mark.parametrize("edges", [1, 40, 1000])
+@pytest.mark.parametrize("N", [50_000, (1 << 22) + 21])
+def test_window_of_out_of_range_columns_only(oracle_mod, N, edges, W):
+    """A window none of whose columns exists has no TC block where columns are compacted by sorting
+    (N > 2^22): the fill has nothing to write for it. The call reports the column, and the next call
+    on the mended columns is right."""
+    from fused3s_amd import capi
+    print("case bad window N=%d edges=%d W=%d" % (N, edges, W), flush=True)
+    rng = np.random.default_rng(N + edges)
+    deg = np.zeros(N, np.int64)
+    deg[::N // 50] = 5
+    bad = 16 * (N // 32)
+    deg[bad:bad + 16] = 0
+    deg[bad + 3] = edges
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(deg)
+    colIdx = rng.integers(0, N, int(rowPtr[-1])).astype(np.int32)
+    broken = colIdx.copy()
+    broken[rowPtr[bad]:rowPtr[bad + 16]] = [N + k if k % 2 else -1 - k for k in range(edges)]
+    rp, ci = torch.as_tensor(rowPtr).cuda(), torch.as_tensor(broken).cuda()
+    for two_phase in (False, True):
+        with pytest.raises(RuntimeError, match="column index"):
+            capi.preprocess(rp, ci, N, 16, W, two_phase=two_phase)
+    compare_preprocess(run_gpu(rowPtr, colIdx, N, W), oracle_mod.preprocess(rowPtr, colIdx, N, 16, W))
+
+
 @pytest.mark.parametrize("name,scale", [("cfg1_gnm_2708", 1.0), ("cfg2_rmat_169k", 1.0),
                                         ("cfg3_chunglu_233k", 0.02), ("cfg5_sbm_100k", 1.0)])
 def test_benchmark_shapes_bit_exact(oracle_mod, name, scale):
