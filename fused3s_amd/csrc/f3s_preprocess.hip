@@ -1300,7 +1300,9 @@ __global__ __launch_bounds__(kOrderOnlyThreads) void window_order_kernel(
     const int32_t* __restrict__ rowWindowOffset, int nRW, int32_t* __restrict__ order) {
   __shared__ uint32_t hist[kOrderOnlyBins];
   auto blocks = [=](int i) {
-    const int c = rowWindowOffset[i + 1] - rowWindowOffset[i];
+    // offsets that descend (not from preprocessing) stand for an empty window, as in the attention
+    // kernels: every window has its place, whatever the caller's offsets hold
+    const int c = max((int)((unsigned)rowWindowOffset[i + 1] - (unsigned)rowWindowOffset[i]), 0);
     const int octave = 31 - __builtin_clz((unsigned)c | 1u);
     return c < 512 ? c : 512 + (octave - 9) * 64 + ((c >> (octave - 6)) & 63);
   };

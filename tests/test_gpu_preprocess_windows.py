@@ -116,3 +116,50 @@ def test_window_order_alone(nRW):
         inside = (count >> octave) == 1
         bucket[inside] = 512 + (octave - 9) * 64 + ((count[inside] >> (octave - 6)) & 63)
     np.testing.assert_array_equal(order.cpu().numpy(), np.argsort(-bucket, kind="stable"))
+
+
+@pytest.mark.parametrize("nRW", [1, 65, 513, 2049, 16_384])
+def test_window_order_of_descending_offsets(nRW):
+    """Offsets that did not come from preprocessing: a window whose range is negative counts as empty,
+    and the order is still a permutation of all windows."""
+    from fused3s_amd import capi
+    print("case descending offsets nRW=%d" % nRW, flush=True)
+    rng = np.random.default_rng(nRW)
+    offsets = rng.integers(-2**31, 2**31, nRW + 1) if nRW == 65 else rng.integers(0, 500, nRW + 1)
+    rwo = torch.as_tensor(offsets.astype(np.int32)).cuda()
+    order = torch.full((nRW,), -1, dtype=torch.int32, device="cuda")
+    rc = capi.lib().f3s_window_order(capi._ptr(rwo), nRW, capi._ptr(order), capi._stream())
+    assert rc == 0, capi.lib().f3s_last_error()
+    got = order.cpu().numpy()
+    np.testing.assert_array_equal(np.sort(got), np.arange(nRW))
+    if nRW != 65:
+        count = np.maximum(np.diff(offsets), 0)
+        np.testing.assert_array_equal(got, np.argsort(-count, kind="stable"))
+
+
+def test_call_without_order_on_descending_offsets(oracle_mod):
+    """A call that makes its own order (1040 windows of 33 blocks, d = 256) writes zeros to the rows of a
+    window whose offsets descend, as the call with a given order does."""
+    from fused3s_amd import F3S
+    print("case own order, descending offsets", flush=True)
+    nRW, blocks, d = 1040, 33, 256
+    N = 16 * nRW
+    rng = np.random.default_rng(3)
+    atox = np.sort(rng.integers(0, N, (nRW, blocks * 16)), axis=1).astype(np.int32)
+    bitmap = rng.integers(0, 2**63, nRW * blocks * 4, dtype=np.uint64)
+    rwo = np.arange(nRW + 1) * blocks
+    broken = rwo.copy()
+    broken[500] = 0  # window 499 descends, window 500 spans the first 501 windows' blocks
+    Q, K, V = [torch.rand((N, d), dtype=torch.float32).half().cuda() for _ in range(3)]
+    dev = lambda a: torch.as_tensor(a).cuda()
+    at, bm = dev(atox.reshape(-1)), dev(bitmap.view(np.int64)).view(torch.uint64)
+    out = []
+    for offsets in (rwo, broken):
+        spoiled = torch.full((N, d), float("nan"), device="cuda")
+        del spoiled  # the memory the call's result is likely to get
+        out.append(F3S.f3s_1tb1rw(dev(offsets.astype(np.int32)), at, bm, N, Q, K, V, 8, True,
+                                  False)[1].cpu().numpy())
+    assert not out[1][499 * 16:500 * 16].any()
+    keep = np.ones(N, bool)
+    keep[499 * 16:501 * 16] = False
+    assert np.isfinite(out[1]).all() and np.array_equal(out[0][keep], out[1][keep])
