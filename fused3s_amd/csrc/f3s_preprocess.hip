@@ -1971,8 +1971,9 @@ __device__ __forceinline__ void fill_short_window(
   for (int e0 = 0; e0 < n; e0 += 64) {
     bool starts;
     const int row = edgeRows.next_group(e0, lane, &starts);
-    if (e0 + lane < n) {
-      const int c = (edgeToColumn[eS + e0 + lane] >> LOGW) * 16 + row;
+    const int rank = e0 + lane < n ? edgeToColumn[eS + e0 + lane] : -1;
+    if ((unsigned)rank < (unsigned)(nb * W)) {
+      const int c = (rank >> LOGW) * 16 + row;
       atomicAdd(&cnt[c >> 1], 1u << ((c & 1) * 16));
     }
   }
@@ -2004,8 +2005,8 @@ __device__ __forceinline__ void fill_short_window(
     const int rs = __builtin_amdgcn_readlane(rowStart, row);
     const int re = __builtin_amdgcn_readlane(rowStart, row + 1);
     for (int e0 = rs; e0 < re; e0 += 64) {
-      const bool valid = e0 + lane < re;
-      const int rank = valid ? edgeToColumn[eS + e0 + lane] : 0;
+      const int rank = e0 + lane < re ? edgeToColumn[eS + e0 + lane] : -1;
+      const bool valid = (unsigned)rank < (unsigned)(nb * W);
       const int t = rank >> LOGW;
       unsigned long long peers = __ballot(valid);  // lanes whose edges fall into the same block
       for (int bit = 0; (MAXB >> bit) != 0; bit++) {

@@ -322,6 +322,52 @@ def test_window_of_out_of_range_columns_only(oracle_mod, N, edges, W):
     compare_preprocess(run_gpu(rowPtr, colIdx, N, W), oracle_mod.preprocess(rowPtr, colIdx, N, 16, W))
 
 
+# 300 edges: a wave per window; 1500: a workgroup
+@pytest.mark.parametrize("W", [16, 8])
+@pytest.mark.parametrize("edges", [300, 1500])
+def test_fill_leaves_out_ranks_beyond_the_window(oracle_mod, edges, W):
+    """f3s_preprocess_fill with ranks that name no block of their window, in a window whose rows hold
+    repeated columns (tile ids are placed edge by edge): the edges are left out, the other windows
+    are as without them."""
+    from fused3s_amd import capi
+    print("case bad ranks edges=%d W=%d" % (edges, W), flush=True)
+    rng = np.random.default_rng(edges + W)
+    N = 16 * 40
+    deg = np.full(N, 4)
+    bad = 16 * 20
+    deg[bad:bad + 16] = edges // 16
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(deg)
+    colIdx = rng.integers(0, N, int(rowPtr[-1])).astype(np.int32)  # unsorted, repeated
+    want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, W)
+    dev = lambda a: torch.as_tensor(a.astype(np.int32)).cuda()
+    e2c = want["edgeToColumn"].copy()
+    lo, hi = rowPtr[bad], rowPtr[bad + 16]
+    nb = int(want["blockPartition"][20])
+    e2c[lo:hi:7] = np.resize([-1, -2**31, 2**31 - 1, nb * W, nb * W + 4099], len(e2c[lo:hi:7]))
+    E, nT = len(colIdx), int(want["blockCount"])
+    rp, ci, ranks, rwo = dev(rowPtr), dev(colIdx), dev(e2c), dev(want["rowWindowOffset"])
+    i32 = dict(dtype=torch.int32, device="cuda")
+    rowid, toff = torch.empty(nT, **i32), torch.empty(nT + 1, **i32)
+    atox = torch.empty(nT * W, **i32)
+    guard = 1 << 17  # tile ids beyond the last edge: nothing may be written there
+    tile = torch.full((E + guard,), 0xA5, dtype=torch.uint8, device="cuda")
+    bm = torch.empty(nT * W // 4, dtype=torch.uint64, device="cuda")
+    p = capi._ptr
+    rc = capi.lib().f3s_preprocess_fill(p(rp), p(ci), N, E, 16, W, p(ranks), p(rwo), nT, p(rowid),
+                                        p(tile), p(toff), p(atox), p(bm), capi._stream())
+    assert rc == 0, capi.lib().f3s_last_error()
+    tile = tile.cpu().numpy()
+    assert (tile[E:] == 0xA5).all()
+    first, last = want["rowWindowOffset"][20], want["rowWindowOffset"][21]
+    for got, ref, a, b in ((tile[:E], want["tcblocktileId"], lo, hi),
+                           (rowid.cpu().numpy(), want["tcblockRowid"], first, first),
+                           (atox.cpu().numpy(), want["sparseAToXidx"], first * W, last * W),
+                           (bm.cpu().view(torch.int64).numpy().view(np.uint64), want["tcbBitMap"],
+                            first * W // 4, last * W // 4)):
+        assert np.array_equal(got[:a], ref[:a]) and np.array_equal(got[b:], ref[b:])
+
+
 @pytest.mark.parametrize("name,scale", [("cfg1_gnm_2708", 1.0), ("cfg2_rmat_169k", 1.0),
                                         ("cfg3_chunglu_233k", 0.02), ("cfg5_sbm_100k", 1.0)])
 def test_benchmark_shapes_bit_exact(oracle_mod, name, scale):
