@@ -1184,9 +1184,14 @@ __device__ __forceinline__ void scan_windows(const int32_t* __restrict__ blockPa
 // become a histogram in LDS (low half of a word: windows with that many blocks, high half: those in
 // front of `first`), its sums from the top the places. No workgroup waits for another one, and
 // nRW / TB of them share the work (a radix sort by one workgroup of 1024 threads took 21 us for
-// 10 584 windows, 30 us for 14 561). Counts from nBins - 1 on share the last bin; the few windows
-// that have so many compare themselves with all others. hist: nBins words, a multiple of TB.
-// blocks(i): window i's count.
+// 10 584 windows, 30 us for 14 561). hist: nBins words, a multiple of TB. blocks(i): window i's count,
+// not negative.
+// Counts from nBins - 1 on share the last bin; while it holds any, another round orders the windows
+// of the next nBins - 1 counts, so a call takes as many rounds as its largest count asks for (at most
+// nine: 32 769 blocks of 8 columns, 4096 bins); nearly every graph takes one. Wide windows that compare
+// themselves with all others instead, one after the other in a wave, are slow where there are many:
+// 100 000 nodes of 2 500 edges, 8-column blocks, 6 245 of 6 250 windows: a preprocessing call of 7.54
+// instead of 7.01 ms; 262 000 nodes of 2 200 edges: 17.01 instead of 15.03 ms.
 template <int TB, typename BlocksOf>
 __device__ __forceinline__ void order_chunk(const BlocksOf& blocks, int nRW, int first, int nBins,
                                             int32_t* __restrict__ sortedRowWindows,
@@ -1199,71 +1204,65 @@ __device__ __forceinline__ void order_chunk(const BlocksOf& blocks, int nRW, int
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int top = nBins - 1;
-  for (int i = tid; i < nBins; i += TB) hist[i] = 0u;
-  __syncthreads();
-  for (int i0 = 0; i0 < nRW; i0 += U * TB) {
-    int c[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int i = i0 + u * TB + tid;
-      c[u] = i < nRW ? min(blocks(i), top) : -1;
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      // counts cluster, and lanes that name the same bin are served one after the other: the lanes
-      // that agree with the group's first one are counted with one ballot and added once
-      const int c0 = __builtin_amdgcn_readfirstlane(c[u]);
-      const unsigned one = i0 + u * TB + wave * 64 < first ? 0x10001u : 1u;
-      const unsigned long long same = __ballot(c[u] == c0);
-      if (c[u] >= 0 && c[u] != c0) atomicAdd(&hist[c[u]], one);
-      if (c0 >= 0 && lane == 0) atomicAdd(&hist[c0], one * (unsigned)__popcll(same));
-    }
-  }
-  __syncthreads();
-  {  // where each bin's windows of this chunk start; thread t owns nBins / TB bins from the top
-    const int per = nBins / TB;
-    unsigned total = 0;
-    for (int k = 0; k < per; k++) total += hist[top - (tid * per + k)] & 0xFFFFu;
-    const unsigned incl = wave_inclusive_scan(total, lane);
-    if (lane == 63) sBinTot[wave] = incl;
+  const int count = first + tid < nRW ? blocks(first + tid) : -1;
+  for (int low = 0;; low += top) {  // windows of low .. low + top - 1 blocks
+    for (int i = tid; i < nBins; i += TB) hist[i] = 0u;
     __syncthreads();
-    unsigned run = incl - total;
+    for (int i0 = 0; i0 < nRW; i0 += U * TB) {
+      int c[U];
 #pragma unroll
-    for (int k = 0; k < NW; k++) run += k < wave ? sBinTot[k] : 0u;
-    for (int k = 0; k < per; k++) {
-      const uint32_t v = hist[top - (tid * per + k)];
-      hist[top - (tid * per + k)] = run + (v >> 16);
-      run += v & 0xFFFFu;
+      for (int u = 0; u < U; u++) {
+        const int i = i0 + u * TB + tid;
+        c[u] = i < nRW ? min(blocks(i) - low, top) : -1;
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        // counts cluster, and lanes that name the same bin are served one after the other: the lanes
+        // that agree with the group's first one are counted with one ballot and added once
+        const int c0 = __builtin_amdgcn_readfirstlane(c[u]);
+        const unsigned one = i0 + u * TB + wave * 64 < first ? 0x10001u : 1u;
+        const unsigned long long same = __ballot(c[u] == c0);
+        if (c[u] >= 0 && c[u] != c0) atomicAdd(&hist[c[u]], one);
+        if (c0 >= 0 && lane == 0) atomicAdd(&hist[c0], one * (unsigned)__popcll(same));
+      }
     }
-  }
-  const int i = first + tid;
-  const int count = i < nRW ? blocks(i) : -1;
-  const bool binned = count >= 0 && count < top;
-  unsigned long long peers = __ballot(binned);
-  for (int b = 0; (top >> b) != 0; b++) {
-    const unsigned long long bal = __ballot((count >> b) & 1);
-    peers &= ((count >> b) & 1) ? bal : ~bal;
-  }
-  for (int turn = 0; turn < NW; turn++) {  // ties go by window: one wave after the other
     __syncthreads();
-    if (wave != turn) continue;
-    const unsigned at = binned ? hist[count] : 0u;
-    wave_lds_sync();
-    if (binned) {
-      sortedRowWindows[at + __popcll(peers & ((1ull << lane) - 1ull))] = i;
-      if ((peers >> lane) == 1ull) hist[count] = at + (unsigned)__popcll(peers);
+    const bool wider = (hist[top] & 0xFFFFu) != 0u;  // windows left for the rounds to come
+    {  // where each bin's windows of this chunk start; thread t owns nBins / TB bins from the top
+      const int per = nBins / TB;
+      unsigned total = 0;
+      for (int k = 0; k < per; k++) total += hist[top - (tid * per + k)] & 0xFFFFu;
+      const unsigned incl = wave_inclusive_scan(total, lane);
+      if (lane == 63) sBinTot[wave] = incl;
+      __syncthreads();
+      unsigned run = incl - total;
+#pragma unroll
+      for (int k = 0; k < NW; k++) run += k < wave ? sBinTot[k] : 0u;
+      for (int k = 0; k < per; k++) {
+        const uint32_t v = hist[top - (tid * per + k)];
+        hist[top - (tid * per + k)] = run + (v >> 16);
+        run += v & 0xFFFFu;
+      }
     }
-  }
-  for (unsigned long long left = __ballot(count >= top); left != 0ull; left &= left - 1ull) {
-    const int src = __builtin_ctzll(left);
-    const int c = __builtin_amdgcn_readlane(count, src), w = first + wave * 64 + src;
-    unsigned before = 0;
-    for (int k = lane; k < nRW; k += 64) {
-      const int x = blocks(k);
-      before += (x > c || (x == c && k < w)) ? 1u : 0u;
+    const int bin = count - low;
+    const bool binned = bin >= 0 && bin < top;
+    unsigned long long peers = __ballot(binned);
+    for (int b = 0; (top >> b) != 0; b++) {
+      const unsigned long long bal = __ballot((bin >> b) & 1);
+      peers &= ((bin >> b) & 1) ? bal : ~bal;
     }
-    before = wave_inclusive_scan(before, lane);
-    if (lane == 63) sortedRowWindows[before] = w;
+    for (int turn = 0; turn < NW; turn++) {  // ties go by window: one wave after the other
+      __syncthreads();
+      if (wave != turn) continue;
+      const unsigned at = binned ? hist[bin] : 0u;
+      wave_lds_sync();
+      if (binned) {
+        sortedRowWindows[at + __popcll(peers & ((1ull << lane) - 1ull))] = first + tid;
+        if ((peers >> lane) == 1ull) hist[bin] = at + (unsigned)__popcll(peers);
+      }
+    }
+    if (!wider) return;
+    __syncthreads();  // the bins are free again
   }
 }
 // bins for the counts that the windows of a graph can have, within 16 KiB
@@ -1292,8 +1291,8 @@ __global__ __launch_bounds__(kFinBlock) void finalize_count_kernel(
 }
 
 // The order alone, for attention calls without one. It only has to start the long windows first, so
-// counts of 512 blocks and more share 64 bins an octave: 1024 bins in all, and no window compares
-// itself with all others (below 131 000 blocks). 4 to 6 us.
+// counts of 512 blocks and more share 64 bins an octave: 1024 bins in all, one round below
+// 131 000 blocks. 4 to 6 us.
 constexpr int kOrderOnlyBins = 1024;
 constexpr int kOrderOnlyThreads = 512;
 __global__ __launch_bounds__(kOrderOnlyThreads) void window_order_kernel(

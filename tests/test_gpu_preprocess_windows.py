@@ -97,6 +97,40 @@ def test_window_counts(oracle_mod, nRW, edges, wide, W):
         assert np.array_equal(bm, want["tcbBitMap"]), two_phase
 
 
+# The order's histogram has 4096 bins: windows of 4095 blocks and more take further rounds. Counts at
+# the rounds' edges, ties of more than a wave, rounds that no window falls into, and one window that
+# spans every node
+@pytest.mark.parametrize("W,counts", [
+    (8, [4093, 4094, 4095, 4096, 8189, 8190, 8191, 12_284, 12_285, 16_375, 0, 1]),
+    (8, [16_375]),
+    (8, [4095] * 70 + [4094, 4100]),
+    (16, [4094, 4095, 4096, 8186]),
+])
+def test_window_order_of_wide_windows(oracle_mod, W, counts):
+    from fused3s_amd import capi
+    print("case wide windows W=%d counts=%s" % (W, counts[:12]), flush=True)
+    N = 131_000
+    rng = np.random.default_rng(len(counts) + W)
+    rows = [np.sort(rng.choice(N, size=3, replace=False)).astype(np.int32) for _ in range(N)]
+    at = rng.choice(N // 16, size=len(counts), replace=False)
+    if len(counts) > 64:
+        at = np.arange(100, 100 + len(counts))
+    for w, blocks in zip(at, counts):
+        cols = np.sort(rng.choice(N, size=blocks * W, replace=False)).astype(np.int32)
+        for r in range(16):
+            rows[16 * w + r] = cols[r::16]
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum([len(r) for r in rows])
+    colIdx = np.concatenate(rows)
+    want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, W)
+    assert sorted(counts) == sorted(want["blockPartition"][at])
+    rp, ci = torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda()
+    for two_phase in (False, True):
+        got = capi.preprocess(rp, ci, N, 16, W, two_phase=two_phase)
+        for k in KEYS:
+            assert np.array_equal(got[k].cpu().numpy(), want[k]), (k, two_phase)
+
+
 @pytest.mark.parametrize("nRW", [1, 511, 512, 513, 2048, 4097, 16_384])
 def test_window_order_alone(nRW):
     """Long windows first, equal counts by window; from 512 blocks on, 64 bins an octave."""
