@@ -26,21 +26,41 @@ namespace window {
 using pipe::float4v;
 using pipe::kLog2e;
 
-// Waves and ring stages of a workgroup.
-//   TEAM_SHORT  one workgroup for every window: four waves of one stage. A window's share of a wave is
-//               a few steps, what counts is how many workgroups hide each other's chain of loads in
-//               front of the first gather: five per CU at D = 32 (four were measured alike), three
-//               at D = 64 (two stages allow two: 169k-node R-MAT graph 105 -> 88 us), two up to
-//               D = 128, one above.
+// Waves and ring stages of a workgroup. Bound by the latency of the gathers and of the chain of loads
+// in front of the first one, so what counts is the pairs in flight on a CU, and how long the longest
+// window takes alone.
+//   TEAM_SHORT  one workgroup for every window: four waves of one stage. Four workgroups per CU at
+//               D = 32, three at D = 64 (two stages allow two), two up to D = 128, one above.
+//   TEAM_PAIRS  the same with two stages at D = 32, where they cost no workgroup (see two_stages).
 //   TEAM_LONG   the few long windows of a graph of short ones, one workgroup after the other per CU:
 //               as many bytes in flight as one CU's LDS holds, eight waves of two stages up to
 //               D = 64, eight of one stage up to D = 128, four above.
-enum Team { TEAM_SHORT, TEAM_LONG };
+enum Team { TEAM_SHORT, TEAM_PAIRS, TEAM_LONG };
 constexpr int team_waves(Team t, int d) { return t == TEAM_LONG && d <= 128 ? 8 : 4; }
-constexpr int team_stages(Team t, int d) { return t == TEAM_LONG && d <= 64 ? 2 : 1; }
+constexpr int team_stages(Team t, int d) { return t != TEAM_SHORT && d <= 64 ? 2 : 1; }
 constexpr int waves_per_simd(Team t, int d) {
   if (d > 128) return 1;
   return t == TEAM_LONG || d > 64 ? 2 : d > 32 ? 3 : 4;
+}
+
+// Whether TEAM_PAIRS takes the windows rather than TEAM_SHORT (nTcb16: blocks of 16 columns, of all
+// heads). At D = 32 four workgroups fit a CU either way and the second stage halves what the longest
+// window of a skewed graph waits for; with windows long on average, or many heads, all CUs are busy to
+// the end and the shorter loop of one stage wins. One -> two stages in us, windows in heavy-first order:
+//   17 to 30 blocks a window: R-MAT 65 521 nodes 48.6 -> 40.8, 169 343 nodes 78.9 -> 65.8 and 105 ->
+//   85.7, 600 000 nodes 239 -> 241; 38 to 57: 100 000 nodes 74.0 -> 67.6, 200 000 nodes 224 -> 227;
+//   86 to 90: 30 000 nodes 45.1 -> 41.8, with 4 heads 143 -> 148; uniform and community graphs of 5 to
+//   20: within 2 %.
+//   124 to 132: 52.4 -> 50.8, with 4 heads 196 -> 204; 160 to 180: 62.8 -> 63.3 and 121 -> 128;
+//   337 to 387: 44.2 -> 47.1, 108 -> 114 (233 000 nodes, 448: 2217 -> 2079, the one exception).
+// At D = 64 a second stage costs the third workgroup: windows of 160 to 390 blocks 0 to 14 % slower,
+// R-MAT of 10 blocks a window up to 25 % (169 343 nodes 69 -> 85), uniform graphs 10 to 24 %. Against
+// that, R-MAT of 20 to 29 blocks and up to 100 000 nodes would gain (65 521 nodes 53.6 -> 47.7 and
+// 65.2 -> 54.0), but a less skewed graph of the same size and block count loses (40 000 nodes 29.8 ->
+// 32.4), and sizes do not tell the two apart.
+constexpr int kTwoStageBlocks = 96;
+inline bool two_stages(int d, int64_t nTcb16, int nRW) {
+  return d <= 32 && nTcb16 < (int64_t)kTwoStageBlocks * nRW;
 }
 
 // LDS of a workgroup: its waves' rings
@@ -356,12 +376,19 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
                          nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer, 1, D, D, (float*)nullptr,
                          hl.minBlocks, (int)gw);
     }
-  } else if (hl.nHeads > 0) {
-    F3S_LAUNCH(TEAM_SHORT, false, true, units)
-  } else if (cuTimer) {
-    F3S_LAUNCH(TEAM_SHORT, true, false, gw)
   } else {
-    F3S_LAUNCH(TEAM_SHORT, false, false, gw)
+    constexpr Team kPairs = D <= 32 ? TEAM_PAIRS : TEAM_SHORT;  // no second kernel above D = 32
+    const bool pairs = two_stages(D, hl.nTcb * heads, nRW);
+    if (hl.nHeads > 0) {
+      if (pairs) F3S_LAUNCH(kPairs, false, true, units)
+      else F3S_LAUNCH(TEAM_SHORT, false, true, units)
+    } else if (cuTimer) {
+      if (pairs) F3S_LAUNCH(kPairs, true, false, gw)
+      else F3S_LAUNCH(TEAM_SHORT, true, false, gw)
+    } else {
+      if (pairs) F3S_LAUNCH(kPairs, false, false, gw)
+      else F3S_LAUNCH(TEAM_SHORT, false, false, gw)
+    }
   }
 #undef F3S_LAUNCH
   F3S_HIP_CHECK(hipGetLastError());
@@ -374,8 +401,12 @@ int launch_tcb8(const int32_t* rwo, const int32_t* order, const int32_t* atox,
                 float scaleLog2, float* out, float* sddmm, int64_t nTcb8, hipStream_t stream) {
   const int nRW = (N + kWinRows - 1) / kWinRows;
   if (nRW == 0) return 0;
-  constexpr size_t lds = team_lds(TEAM_SHORT, D);
-  auto kernel = f3s_fwd_kernel<_Float16, D, TEAM_SHORT, SOFTMAX, false, false, true, WIDE>;
+  constexpr Team kPairs = D <= 32 ? TEAM_PAIRS : TEAM_SHORT;
+  const bool pairs = two_stages(D, nTcb8 / 2, nRW);
+  const size_t lds = pairs ? team_lds(kPairs, D) : team_lds(TEAM_SHORT, D);
+  auto kernel = pairs ? f3s_fwd_kernel<_Float16, D, kPairs, SOFTMAX, false, false, true, WIDE>
+                      : f3s_fwd_kernel<_Float16, D, TEAM_SHORT, SOFTMAX, false, false, true, WIDE>;
+  static_assert(team_waves(kPairs, D) == team_waves(TEAM_SHORT, D), "one launch for both");
   if (int rc = allow_lds(kernel, lds)) return rc;
   hipLaunchKernelGGL(kernel, dim3(nRW), dim3(team_waves(TEAM_SHORT, D) * 64), lds, stream, rwo, order, atox,
                      reinterpret_cast<const uint8_t*>(bitmap), N, nRW, nTcb8,
