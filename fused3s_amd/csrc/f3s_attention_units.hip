@@ -35,7 +35,7 @@ using pipe::float4v;
 using pipe::uniform;
 
 constexpr int kXcds = 8;
-constexpr int kMaxPhases = 16;
+constexpr int kMaxPhases = 16;  // slices that an XCD works through one after the other (choose_split)
 constexpr int kUnitWaves = 4;  // waves (= units) per workgroup; they do not cooperate
 
 // Stages of a wave's LDS ring and waves per SIMD the register allocator is held to.
@@ -591,6 +591,15 @@ int allow_lds(KernelT kernel, size_t bytes) {
 // which already catches 4 of 5 accesses on the 233k-node benchmark graph, while more and shorter
 // units cost more than their higher hit rate returns (measured 1.54 / 1.69 / 1.86 ms with 8 / 16 /
 // 24 slices there). XCDs left over share the windows.
+// No more than kMaxPhases slices are worked through one after the other: from 128 MiB of K + V per
+// group of heads on (524 000 nodes at d = 64, 262 000 at 128, 131 000 at 256) slices get wider than
+// 8 MiB instead. Every slice more is a partial result more per window, to be written and merged, and on
+// large graphs that outweighs the L2 hits. With the cap against without, in ms (and GB of workspace):
+// 200 000 nodes, 141 blocks a window, d = 256: 3.05 (3.1) against 3.80 (4.8); 600 000, 290, d = 128:
+// 6.93 (4.7) against 8.46 (10.8); 1 000 000, 99, d = 128: 6.98 (7.8) against 16.7 (30); 1 200 000, 99,
+// d = 64: 4.38 against 7.68; 300 000, 555, 2 x 128: 9.14 against 9.45; 400 000, 747, d = 128: 8.39
+// against 8.75; 262 144, 899: alike. A cap of 8 is slower on long windows (the 747: 9.71) and faster on
+// short ones (the 99: 5.79).
 // F3S_SLICE_PHASES = P in the environment forces 8 P slices of all heads.
 XcdSplit choose_split(int N, int d, int heads) {
   const char* e = getenv("F3S_SLICE_PHASES");  // read per call: tests walk through the phases

@@ -47,6 +47,40 @@ def test_sliced(oracle_mod, monkeypatch, N, heads, d):
     check(oracle_mod, pre, N, heads, d, Q, K, V, got)
 
 
+# K + V of a group of heads that would take 18 and 17 slices of 8 MiB: 16 wider ones are used. Columns at
+# every slice edge, and a window that names all slices
+@pytest.mark.parametrize("heads,d,N", [(0, 256, 140_003), (2, 128, 270_011)])
+def test_sixteen_slices(oracle_mod, monkeypatch, heads, d, N):
+    from fused3s_amd import capi
+    print("case sixteen slices heads=%d d=%d" % (heads, d), flush=True)
+    nRW, width = (N + 15) // 16, (N + 15) // 16  # slices of N / 16 columns, rounded up
+    rng = np.random.default_rng(d)
+    edge = np.concatenate([np.arange(1, 16) * width + k for k in (-1, 0, 1)])
+    deg = rng.integers(0, 3, N)
+    deg[5] = 4000
+    deg[100:100 + len(edge)] = 1
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(deg)
+    colIdx = rng.integers(0, N, int(rowPtr[-1])).astype(np.int32)
+    colIdx[rowPtr[5]:rowPtr[6]] = np.sort(rng.choice(N, size=4000, replace=False))
+    colIdx[rowPtr[100]:rowPtr[100 + len(edge)]] = edge
+    pre, (rwo, order, atox, bm) = on_gpu(oracle_mod, rowPtr, colIdx, N)
+    g = torch.Generator().manual_seed(d)
+    Q, K, V = [torch.randn((N, max(heads, 1), d), generator=g).half().cuda() for _ in range(3)]
+    monkeypatch.setenv("F3S_SCHEDULE", "sliced")
+    monkeypatch.delenv("F3S_SLICE_PHASES", raising=False)
+    ws = capi.attention_workspace(N, d, "cuda", heads=heads)
+    per_slice = nRW * max(heads, 1) * (16 * d + 32) * 4  # bytes of partial results
+    assert 16 <= ws.numel() / per_slice < 17
+    ws.fill_(0xFF)
+    if heads:
+        got = capi.attention_heads(rwo, order, atox, bm, N, Q, K, V, float(np.sqrt(d)), workspace=ws)
+    else:
+        got = capi.attention(rwo, order, atox, bm, N, *[t[:, 0].contiguous() for t in (Q, K, V)],
+                             float(np.sqrt(d)), workspace=ws)
+    check(oracle_mod, pre, N, max(heads, 1), d, Q, K, V, got)
+
+
 # 1025 windows: one more than a whole number of chunks for every number of head groups
 @pytest.mark.parametrize("heads,d", [(1, 32), (3, 64), (4, 64), (8, 32), (2, 128)])
 def test_short_windows(oracle_mod, heads, d):
