@@ -182,7 +182,7 @@ __device__ __forceinline__ void store_rows(const float4v (&o)[D / 16], float* ld
 // One wave per unit, kUnitWaves independent units per workgroup. A unit is
 //   SLICED:  the TC blocks of one (window, column slice[, head]); the result is a partial
 //            (m, l, O). Workgroup b: XCD b % 8, then (phase, group of kUnitWaves consecutive
-//            units of the order); unit = position * nHeads + head; slice = phase * 8 + XCD.
+//            units of that XCD and phase); which position, head and slice a unit is: XcdSplit.
 //   !SLICED: one whole window (of one head, if HEADS); the result is the window's output rows.
 //            Windows of more than maxBlocks TC blocks among the first longPrefix positions of
 //            the order are left to f3s_fwd_kernel, whose waves share a window and whose grid looks

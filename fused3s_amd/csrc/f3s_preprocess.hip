@@ -5,14 +5,14 @@
 // window with a single thread. Here a window never leaves its workgroup:
 //
 //   window_rank_bins_kernel / window_rank_small_kernel
-//                        windows of <= 960 edges, one WAVE per window, no workgroup barrier.
-//                        Graphs of <= 2^22 nodes: (column, position) words sorted by bins of LDS
-//                        counters, ranks of the distinct columns back to the edges. Larger graphs:
-//                        bitonic sort of the column ids, ballot / popcount compaction of the
-//                        distinct ones, rank by binary search.
+//                        short windows, one WAVE per window, no workgroup barrier. Graphs of
+//                        <= 2^22 nodes, windows of <= 960 edges: (column, position) words sorted by
+//                        bins of LDS counters, ranks of the distinct columns back to the edges.
+//                        Larger graphs, <= 1024 edges: bitonic sort of the column ids, ballot /
+//                        popcount compaction of the distinct ones, rank by binary search.
 //   window_rank_sort_kernel
-//                        windows of up to 32k edges where the columns take several bitset passes,
-//                        one workgroup per window: sorted by bins as well.
+//                        windows of up to 16 384 edges where the columns take several bitset
+//                        passes, one workgroup per window: sorted by bins as well.
 //   window_rank_kernel   larger windows, one workgroup per window. Column ids are OR-ed into an
 //                        LDS bitset (a column range per pass when N exceeds the LDS range), a
 //                        wave64 popcount prefix scan turns the bitset into ranks, and every edge

@@ -189,10 +189,11 @@ int f3s_attention_fwd(const int32_t* rowWindowOffset, const int32_t* windowOrder
 /*
  * Bytes of device scratch f3s_attention_fwd / f3s_attention_fwd_heads can use for a graph of N
  * nodes at head dimension d (a header, the slice boundaries of every window, plus one partial
- * (m, l, O) per window, head and slice: about 4.6 KB * ceil(N/16) * slices at d = 64; for the
- * single-head call at d = 64 also 512 * N bytes for copies of K and V with 256-byte rows, which
- * the call makes itself and gathers from instead: rows that start on even 128-byte lines are
- * served faster than rows on the odd lines in between). The reference's launchers
+ * (m, l, O) of 64 d + 128 bytes per window, head and slice; for the single-head call at d = 64 also
+ * 512 * N bytes for copies of K and V with 256-byte rows, which the call makes itself and gathers
+ * from instead: rows that start on even 128-byte lines are served faster than rows on the odd lines
+ * in between). Slices are two or more, about one per 8 MiB of a group of heads' K + V rows up to
+ * sixteen, so the size does not grow with N alone: ask for every N and d. The reference's launchers
  * (src/F3S_kernel.cu:581-671) need no scratch; passing workspace = NULL keeps that behaviour.
  */
 size_t f3s_attention_workspace_bytes(int N, int d);
@@ -275,7 +276,8 @@ int f3s_attention_fwd_tcb8(const int32_t* rowWindowOffset, const int32_t* window
  * this one windows of 512 blocks and more that differ by less than 1.6 % may change places).
  *
  *   rowWindowOffset [nRW+1]   from preprocessing; nRW at most 16384
- *   order [nRW]               out: a permutation of the windows
+ *   order [nRW]               out: a permutation of the windows (offsets that descend count as an
+ *                             empty window)
  * Asynchronous on `stream`.
  */
 int f3s_window_order(const int32_t* rowWindowOffset, int nRW, int32_t* order, void* stream);

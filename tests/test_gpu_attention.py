@@ -139,8 +139,8 @@ def test_end_to_end_hip_preprocess_then_attention(oracle_mod):
 @pytest.mark.parametrize("persistent", ["0", "1"])
 @pytest.mark.parametrize("phases", [2, 3])
 def test_column_sliced_schedule_with_several_phases(oracle_mod, monkeypatch, phases, persistent):
-    """16 and 24 column slices (two and three per XCD, which the library only picks by itself above
-    64 MiB of K + V) through the launch-ordered kernel and through the queue-based one."""
+    """16 and 24 column slices of all heads, two and three per XCD (forced: the library's own choice is
+    another deal of at most 16), through the launch-ordered kernel and through the resident one."""
     print("case sliced phases=%d persistent=%s" % (phases, persistent), flush=True)
     from fused3s_amd import synth
     monkeypatch.setenv("F3S_SLICE_PHASES", str(phases))

@@ -227,7 +227,7 @@ def test_multi_pass_bitset_large_n(oracle_mod):
 
 def test_more_than_4m_nodes_takes_the_bitonic_short_window_kernel(oracle_mod):
     """Above 2^22 nodes a column id and an edge position no longer share a 32-bit word, so short
-    windows are ranked by the bitonic kernel instead of the radix one; long windows (a hub row)
+    windows are ranked by the bitonic kernel instead of the bins; long windows (a hub row)
     and the multi-pass bitset are in the same graph."""
     print("case 5m_nodes", flush=True)
     N = 5_000_011

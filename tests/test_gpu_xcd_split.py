@@ -49,10 +49,11 @@ def test_sliced(oracle_mod, monkeypatch, N, heads, d):
 
 # K + V of a group of heads that would take 18 and 17 slices of 8 MiB: 16 wider ones are used. Columns at
 # every slice edge, and a window that names all slices
+@pytest.mark.parametrize("persistent", ["0", "1"])
 @pytest.mark.parametrize("heads,d,N", [(0, 256, 140_003), (2, 128, 270_011)])
-def test_sixteen_slices(oracle_mod, monkeypatch, heads, d, N):
+def test_sixteen_slices(oracle_mod, monkeypatch, heads, d, N, persistent):
     from fused3s_amd import capi
-    print("case sixteen slices heads=%d d=%d" % (heads, d), flush=True)
+    print("case sixteen slices heads=%d d=%d persistent=%s" % (heads, d, persistent), flush=True)
     nRW, width = (N + 15) // 16, (N + 15) // 16  # slices of N / 16 columns, rounded up
     rng = np.random.default_rng(d)
     edge = np.concatenate([np.arange(1, 16) * width + k for k in (-1, 0, 1)])
@@ -68,6 +69,7 @@ def test_sixteen_slices(oracle_mod, monkeypatch, heads, d, N):
     g = torch.Generator().manual_seed(d)
     Q, K, V = [torch.randn((N, max(heads, 1), d), generator=g).half().cuda() for _ in range(3)]
     monkeypatch.setenv("F3S_SCHEDULE", "sliced")
+    monkeypatch.setenv("F3S_SLICED_PERSISTENT", persistent)
     monkeypatch.delenv("F3S_SLICE_PHASES", raising=False)
     ws = capi.attention_workspace(N, d, "cuda", heads=heads)
     per_slice = nRW * max(heads, 1) * (16 * d + 32) * 4  # bytes of partial results
