@@ -385,12 +385,13 @@ __global__ __launch_bounds__(256) void sliced_setup_kernel(
 //     from a counter in LDS. No device-wide atomic is on the path of a unit.
 //   * The window of the unit after next and the block range of the next unit are requested before
 //     the current unit runs, so they have arrived when it ends.
-// Measured on the 233k-node benchmark graph at d = 64: 1.51 ms against 1.45 ms for the launch-order
-// kernel (static shares leave a tail that the hardware's dispatch of fresh workgroups does not),
-// so this form is the one to ask for (F3S_SLICED_PERSISTENT=1) where workgroups are not dealt
-// round-robin to the XCDs. A variant in which the wave that finishes a window's last unit merges
-// its partials (an arrival counter per window, partials written through) took 1.92 ms: the wait
-// for the stores and the returning atomic sit on every unit's path.
+// Measured on the 233k-node benchmark graph at d = 64: 1.58 ms against 1.46 ms for the launch-order
+// kernel (static shares leave a tail that the hardware's dispatch of fresh workgroups does not; and
+// this form gathers from the rows in place, which costs the other 0.02 ms), so it is the one to ask for
+// (F3S_SLICED_PERSISTENT=1) where workgroups are not dealt round-robin to the XCDs. A variant in which
+// the wave that finishes a window's last unit merges its partials (an arrival counter per window,
+// partials written through) took 1.92 ms: the wait for the stores and the returning atomic sit on
+// every unit's path.
 template <typename ET, int D, bool SOFTMAX, bool HEADS, int NW>
 __global__ __launch_bounds__(NW * 64)
 __attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D, true),
@@ -626,6 +627,20 @@ XcdSplit choose_split(int N, int d, int heads) {
   return s;
 }
 
+// The same slices for the resident form. Its waves move on to the next phase one by one, so an XCD's
+// L2 has to hold two slices while they do: as few phases as the slices divide into evenly, the XCDs on
+// different slices instead. (Unevenly some XCDs would have nothing to do in the last phase: 3 slices in
+// groups of 4 0.48 instead of 0.43 ms.) 233k-node graph, d = 64, 8 slices: 1.82 -> 1.58 ms; 34k nodes,
+// 8 x 32, 2 slices: 1.27 -> 1.16 ms.
+XcdSplit resident_split(XcdSplit s) {
+  while (s.windowGroups > 1 && s.phases % 2 == 0) {
+    s.sliceGroups *= 2;
+    s.windowGroups /= 2;
+    s.phases /= 2;
+  }
+  return s;
+}
+
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // byte offsets of the parts of the workspace
@@ -701,7 +716,7 @@ int launch_sliced_units(const int32_t* rwo, const int32_t* order, const int32_t*
     int grid = 0;
     if (int rc = resident_grid<D, kUnitWaves>(&grid)) return rc;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kUnitWaves * 64), lds, stream, order,
-                       sliceStart, L.split, nRW, N, nTcb, tickets, atox, bm, Q, K, V, scaleLog2,
+                       sliceStart, resident_split(L.split), nRW, N, nTcb, tickets, atox, bm, Q, K, V, scaleLog2,
                        partial, heads, ldIn);
   } else {
     auto kernel = f3s_fwd_unit_kernel<ET, D, SOFTMAX, true, HEADS>;

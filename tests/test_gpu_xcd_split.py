@@ -83,6 +83,39 @@ def test_sixteen_slices(oracle_mod, monkeypatch, heads, d, N, persistent):
     check(oracle_mod, pre, N, max(heads, 1), d, Q, K, V, got)
 
 
+# The resident form deals the same slices in as few phases as they divide into: 3 (three phases as in
+# launch order), 4 (one phase; with four heads in two), 5 and 6 slices
+@pytest.mark.parametrize("heads,d,N", [(0, 64, 70_001), (0, 128, 60_013), (4, 64, 100_003),
+                                       (0, 128, 81_003), (2, 64, 180_001)])
+def test_resident_deals_the_same_slices(oracle_mod, monkeypatch, heads, d, N):
+    from fused3s_amd import capi
+    print("case resident deal heads=%d d=%d N=%d" % (heads, d, N), flush=True)
+    rng = np.random.default_rng(N)
+    deg = rng.poisson(1.0, N)
+    deg[::5003] = 900
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(deg)
+    colIdx = rng.integers(0, N, int(rowPtr[-1])).astype(np.int32)
+    pre, (rwo, order, atox, bm) = on_gpu(oracle_mod, rowPtr, colIdx, N)
+    g = torch.Generator().manual_seed(N)
+    Q, K, V = [torch.randn((N, max(heads, 1), d), generator=g).half().cuda() for _ in range(3)]
+    monkeypatch.setenv("F3S_SCHEDULE", "sliced")
+    ws = capi.attention_workspace(N, d, "cuda", heads=heads)
+    got = []
+    for persistent in ("0", "1"):
+        monkeypatch.setenv("F3S_SLICED_PERSISTENT", persistent)
+        ws.fill_(0xFF)
+        if heads:
+            got.append(capi.attention_heads(rwo, order, atox, bm, N, Q, K, V, float(np.sqrt(d)),
+                                            workspace=ws))
+        else:
+            got.append(capi.attention(rwo, order, atox, bm, N,
+                                      *[t[:, 0].contiguous() for t in (Q, K, V)],
+                                      float(np.sqrt(d)), workspace=ws))
+    assert torch.equal(got[0], got[1])
+    check(oracle_mod, pre, N, max(heads, 1), d, Q, K, V, got[1])
+
+
 # 1025 windows: one more than a whole number of chunks for every number of head groups
 @pytest.mark.parametrize("heads,d", [(1, 32), (3, 64), (4, 64), (8, 32), (2, 128)])
 def test_short_windows(oracle_mod, heads, d):
