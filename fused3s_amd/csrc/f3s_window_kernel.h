@@ -43,24 +43,31 @@ constexpr int waves_per_simd(Team t, int d) {
   return t == TEAM_LONG || d > 64 ? 2 : d > 32 ? 3 : 4;
 }
 
-// Whether TEAM_PAIRS takes the windows rather than TEAM_SHORT (nTcb16: blocks of 16 columns, of all
-// heads). At D = 32 four workgroups fit a CU either way and the second stage halves what the longest
-// window of a skewed graph waits for; with windows long on average, or many heads, all CUs are busy to
-// the end and the shorter loop of one stage wins. One -> two stages in us, windows in heavy-first order:
-//   17 to 30 blocks a window: R-MAT 65 521 nodes 48.6 -> 40.8, 169 343 nodes 78.9 -> 65.8 and 105 ->
-//   85.7, 600 000 nodes 239 -> 241; 38 to 57: 100 000 nodes 74.0 -> 67.6, 200 000 nodes 224 -> 227;
-//   86 to 90: 30 000 nodes 45.1 -> 41.8, with 4 heads 143 -> 148; uniform and community graphs of 5 to
-//   20: within 2 %.
-//   124 to 132: 52.4 -> 50.8, with 4 heads 196 -> 204; 160 to 180: 62.8 -> 63.3 and 121 -> 128;
-//   337 to 387: 44.2 -> 47.1, 108 -> 114 (233 000 nodes, 448: 2217 -> 2079, the one exception).
-// At D = 64 a second stage costs the third workgroup: windows of 160 to 390 blocks 0 to 14 % slower,
-// R-MAT of 10 blocks a window up to 25 % (169 343 nodes 69 -> 85), uniform graphs 10 to 24 %. Against
-// that, R-MAT of 20 to 29 blocks and up to 100 000 nodes would gain (65 521 nodes 53.6 -> 47.7 and
-// 65.2 -> 54.0), but a less skewed graph of the same size and block count loses (40 000 nodes 29.8 ->
-// 32.4), and sizes do not tell the two apart.
-constexpr int kTwoStageBlocks = 96;
-inline bool two_stages(int d, int64_t nTcb16, int nRW) {
-  return d <= 32 && nTcb16 < (int64_t)kTwoStageBlocks * nRW;
+// Whether TEAM_PAIRS takes the windows rather than TEAM_SHORT (nTcb16: blocks of 16 columns). At D = 32
+// four workgroups fit a CU either way, so the second stage only has to pay for its longer loop.
+// One -> two stages in us, heavy-first order, one head unless stated. It pays
+// - where blocks are few and the longest window of a skewed graph decides. 17 to 30 blocks a window:
+//   R-MAT 65 521 nodes 48.6 -> 40.8, 169 343 nodes 78.9 -> 65.8 and 105 -> 85.7, 600 000 nodes 239 -> 241;
+//   38 to 57: 100 000 nodes 74.0 -> 67.6, 200 000 nodes 224 -> 227; 86 to 90: 30 000 nodes 45.1 -> 41.8,
+//   with 4 heads 143 -> 148; uniform and community graphs of 5 to 20: within 2 %.
+// - where windows are long, many, and the rows come from beyond the L2s (K + V of 20 MB): 100 000 nodes,
+//   423 blocks, 4 heads 3364 -> 2662; 140 000, 274, 4 heads 3194 -> 2897; 180 000, 434 1458 -> 1351;
+//   233 000, 448 2155 -> 2068, 8 heads 23 100 -> 21 200; 400 000, 239, 4 heads 10 168 -> 9 828.
+// In between all CUs are busy to the end, mostly with rows from the L2s: 124 to 132 blocks 52.4 -> 50.8,
+// with 4 heads 196 -> 204; 160 to 180 62.8 -> 63.3 and 127 -> 134; 337 to 387 44.2 -> 47.1 and 108 -> 114;
+// 100 000 nodes, 121 177 -> 188, 4 heads 889 -> 922; 233 000 nodes, 188 882 -> 900; 30 000 nodes, 387,
+// 8 heads 1154 -> 1175.
+// At D = 64 a second stage costs the third workgroup: windows of 160 to 390 blocks 0 to 14 % slower, up
+// to 2 % faster on 100 000 nodes and more; R-MAT of 10 blocks a window up to 25 % slower (169 343 nodes
+// 69 -> 85), uniform graphs 10 to 24 %. Against that, R-MAT of 20 to 29 blocks and up to 100 000 nodes
+// would gain (65 521 nodes 53.6 -> 47.7 and 65.2 -> 54.0), but a less skewed graph of the same size and
+// block count loses (40 000 nodes 29.8 -> 32.4), and sizes do not tell the two apart.
+inline bool two_stages(int d, int64_t nTcb16, int heads, int N) {
+  if (d > 32) return false;
+  const int64_t nRW = ((int64_t)N + kWinRows - 1) / kWinRows;
+  if (nTcb16 * heads < 96 * nRW) return true;
+  return nRW >= 2048 && nTcb16 >= 160 * nRW && nTcb16 * heads >= 400 * nRW &&
+         (int64_t)N * d * heads * 4 >= (int64_t)20 << 20;
 }
 
 // LDS of a workgroup: its waves' rings
@@ -378,7 +385,7 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
     }
   } else {
     constexpr Team kPairs = D <= 32 ? TEAM_PAIRS : TEAM_SHORT;  // no second kernel above D = 32
-    const bool pairs = two_stages(D, hl.nTcb * heads, nRW);
+    const bool pairs = two_stages(D, hl.nTcb, heads, N);
     if (hl.nHeads > 0) {
       if (pairs) F3S_LAUNCH(kPairs, false, true, units)
       else F3S_LAUNCH(TEAM_SHORT, false, true, units)
@@ -402,7 +409,7 @@ int launch_tcb8(const int32_t* rwo, const int32_t* order, const int32_t* atox,
   const int nRW = (N + kWinRows - 1) / kWinRows;
   if (nRW == 0) return 0;
   constexpr Team kPairs = D <= 32 ? TEAM_PAIRS : TEAM_SHORT;
-  const bool pairs = two_stages(D, nTcb8 / 2, nRW);
+  const bool pairs = two_stages(D, nTcb8 / 2, 1, N);
   const size_t lds = pairs ? team_lds(kPairs, D) : team_lds(TEAM_SHORT, D);
   auto kernel = pairs ? f3s_fwd_kernel<_Float16, D, kPairs, SOFTMAX, false, false, true, WIDE>
                       : f3s_fwd_kernel<_Float16, D, TEAM_SHORT, SOFTMAX, false, false, true, WIDE>;

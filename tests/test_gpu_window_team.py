@@ -1,5 +1,6 @@
-"""Where the workgroup-per-window kernel changes from two ring stages to one at d = 32: graphs of one TC
-block fewer than 96 a window and head on average, and of exactly 96, through every entry that runs it."""
+"""Where the workgroup-per-window kernel changes between one ring stage and two at d = 32: graphs of one
+TC block fewer than 96 a window and head on average, and of exactly 96, through every entry that runs it;
+and long windows of 20 MB of K + V, of one block fewer than 160 a window and of exactly 160."""
 import numpy as np
 import pytest
 import torch
@@ -73,3 +74,29 @@ def test_both_sides_of_the_line(oracle_mod, tmp_path, monkeypatch, missing, soft
                                V.cuda(), applySoftmax=softmax)
     for h in range(heads):
         close(got[:, h * d:(h + 1) * d], reference(oracle_mod.attention_ref, pre, h), "head %d" % h)
+
+
+@pytest.mark.parametrize("missing", [1, 0])
+def test_long_windows_of_many_heads(oracle_mod, missing):
+    from fused3s_amd import capi
+    print("case window team, long windows missing=%d" % missing, flush=True)
+    nRW, blocks, heads, d = 2048, 160, 8, 32
+    N = 16 * nRW
+    rng = np.random.default_rng(missing)
+    atox = np.sort(np.argpartition(rng.random((nRW, 4096)), blocks * 16, axis=1)[:, :blocks * 16])
+    atox = (atox * 8 + rng.integers(0, 8, atox.shape)).astype(np.int32).reshape(-1)
+    bitmap = rng.integers(0, 2**63, nRW * blocks * 4, dtype=np.uint64)
+    bitmap &= rng.integers(0, 2**63, len(bitmap), dtype=np.uint64)
+    rwo = (np.arange(nRW + 1) * blocks).astype(np.int32)
+    rwo[-1] -= missing
+    atox, bitmap = atox[:rwo[-1] * 16], bitmap[:rwo[-1] * 4]
+    g = torch.Generator().manual_seed(missing)
+    Q, K, V = [torch.randn((N, heads, d), generator=g).half() for _ in range(3)]
+    dev = lambda a: torch.as_tensor(a).cuda()
+    got = capi.attention_heads(dev(rwo), None, dev(atox), dev(bitmap.view(np.int64)).view(torch.uint64),
+                               N, Q.cuda(), K.cuda(), V.cuda(), float(np.sqrt(d))).cpu().numpy()
+    for h in (0, 7):
+        want = oracle_mod.attention_ref(rwo, atox, bitmap, N, *[t[:, h].contiguous().numpy()
+                                                                for t in (Q, K, V)], float(np.sqrt(d)))
+        assert np.abs(got[:, h * d:(h + 1) * d] - want).max() < 2e-2, h
+        assert np.abs(got[:, h * d:(h + 1) * d] - want).mean() < 1e-3 * np.abs(want).mean(), h
