@@ -136,13 +136,20 @@ def bucketed_order(pre, N, buckets):
     return torch.argsort(key, stable=True).to(torch.int32)
 
 
-def recorded_traffic(config, schedule, scale, natural_order):
+# switches of the library that change which kernels a call runs, or what they move
+KERNEL_SWITCHES = ("F3S_AMD_LIB", "F3S_PAD_ROWS", "F3S_SLICE_PHASES", "F3S_SLICED_PERSISTENT",
+                   "F3S_WINDOW_PERSISTENT", "F3S_SHORT_WINDOWS")
+
+
+def recorded_traffic(config, schedule, scale, changed):
     """HBM-side bytes per attention call as rocprofv3 counted them in an EARLIER run (FETCH_SIZE
     and WRITE_SIZE, scaled by what the same counters read for a plain copy): counters cannot be
     read from inside this process, so the figure is a record, labelled with the profile summary
-    it comes from, and is only given for the workload and schedule it was taken on."""
+    it comes from, and is only given for the workload and schedule it was taken on: not for an
+    experiment with another order or layout (changed), nor under a switch of the library."""
     path = os.path.join(ROOT, "profiles", "traffic_recorded.json")
-    if scale != 1.0 or natural_order or not os.path.exists(path):
+    if (scale != 1.0 or changed or any(os.environ.get(v) for v in KERNEL_SWITCHES) or
+            not os.path.exists(path)):
         return None
     for rec in json.load(open(path)).get("records", []):
         if rec.get("config") == config and rec.get("schedule") == schedule:
@@ -363,7 +370,9 @@ def run_config(name, args, dev, headline):
         "schedule": schedule,
         "sanity": sanity,
         "roofline": roofline,
-        "traffic_recorded": recorded_traffic(name, schedule, scale_graph, natural),
+        "traffic_recorded": recorded_traffic(name, schedule, scale_graph,
+                                             natural or bool(layout) or
+                                             (headline and args.column_buckets > 0)),
     }
     if result["traffic_recorded"] is not None:
         # HBM-side bytes per call of the same kernels on the same workload, from the record
