@@ -41,7 +41,6 @@
 // All results are bit-identical to the reference's algorithm with edgeToRow[e] = row(e).
 
 #include <mutex>
-#include <vector>
 
 #include "f3s_common.h"
 
@@ -2809,49 +2808,53 @@ int enqueue_count(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, in
 
 // Pinned host memory for the results of calls that wait for the device: a slot per call in progress,
 // taken from pages of 64 slots that stay with the library (one page unless more than 64 host
-// threads preprocess at a time).
+// threads preprocess at a time). The free slots are a list through the slots themselves, so that
+// neither taking one nor giving it back can run out of host memory and throw through the C ABI.
 struct HostResult {
   long long nTcb;
   int error;
-  int pad[13];
+  HostResult* next;  // of the free list
+  int pad[10];
 };
 static_assert(sizeof(HostResult) == 64, "a line of its own");
 class HostResultLease {
  public:
   int take() {
-    std::lock_guard<std::mutex> lock(mutex_());
-    auto& free = free_();
-    if (free.empty()) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    if (!free_) {
       void* page = nullptr;
       F3S_HIP_CHECK(hipHostMalloc(&page, 64 * sizeof(HostResult), hipHostMallocPortable));
-      for (int i = 0; i < 64; i++) free.push_back(static_cast<HostResult*>(page) + i);
+      for (int i = 0; i < 64; i++) give_back(static_cast<HostResult*>(page) + i);
     }
-    slot_ = free.back();
-    free.pop_back();
+    slot_ = free_;
+    free_ = slot_->next;
     slot_->nTcb = 0;
     slot_->error = 0;
     return 0;
   }
   ~HostResultLease() {
     if (!slot_) return;
-    std::lock_guard<std::mutex> lock(mutex_());
-    free_().push_back(slot_);
+    std::lock_guard<std::mutex> lock(mutex_);
+    give_back(slot_);
   }
+  // The host could not wait for the stream (a stream under capture, a lost device): kernels that hold
+  // the slot's address may still run, so nobody else gets it.
+  void abandon() { slot_ = nullptr; }
   ResultPtr pointers() const { return {&slot_->nTcb, &slot_->error}; }
   // after the stream is done
   const volatile HostResult& value() const { return *slot_; }
 
  private:
-  static std::mutex& mutex_() {
-    static std::mutex m;
-    return m;
+  static void give_back(HostResult* slot) {  // under the lock
+    slot->next = free_;
+    free_ = slot;
   }
-  static std::vector<HostResult*>& free_() {
-    static std::vector<HostResult*> v;
-    return v;
-  }
+  static std::mutex mutex_;
+  static HostResult* free_;
   HostResult* slot_ = nullptr;
 };
+std::mutex HostResultLease::mutex_;
+HostResult* HostResultLease::free_ = nullptr;
 
 int check_count_args(const char* who, int N, int E, int H, int W) {
   if (H != 16 || (W != 16 && W != 8))
@@ -2878,6 +2881,7 @@ int launch_preprocess_count(const int32_t* rowPtr, const int32_t* colIdx, int N,
                          result.pointers(), stream);
   // also after a failed launch: the slot must not be written to any more when it is given back
   const hipError_t done = hipStreamSynchronize(stream);
+  if (done != hipSuccess) result.abandon();
   if (rc != 0) return rc;
   F3S_HIP_CHECK(done);
   if (result.value().error)
@@ -3160,6 +3164,7 @@ int launch_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E
                                     static_cast<char*>(workspace), result.pointers(), stream);
   // also after a failed launch: the slot must not be written to any more when it is given back
   const hipError_t done = hipStreamSynchronize(stream);
+  if (done != hipSuccess) result.abandon();
   if (rc != 0) return rc;
   F3S_HIP_CHECK(done);
   if (result.value().error) return fail(-4, "f3s_preprocess: column index outside [0, %d)", N);

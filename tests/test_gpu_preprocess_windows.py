@@ -197,3 +197,45 @@ def test_call_without_order_on_descending_offsets(oracle_mod):
     keep = np.ones(N, bool)
     keep[499 * 16:501 * 16] = False
     assert np.isfinite(out[1]).all() and np.array_equal(out[0][keep], out[1][keep])
+
+
+def test_threads_and_streams(oracle_mod):
+    """Eight host threads preprocess graphs of their own on streams of their own at the same time: each
+    gets its own total and, for a graph with a column that does not exist, its own error."""
+    import threading
+
+    from fused3s_amd import capi
+    print("case threads", flush=True)
+    graphs = []
+    for k in range(8):
+        rng = np.random.default_rng(k)
+        N = 500 + 700 * k
+        rowPtr, colIdx = build(rng, [int(n) for n in rng.integers(0, 300, N // 16)], N, "even")
+        if k == 5:
+            colIdx[len(colIdx) // 2] = N
+        want = None if k == 5 else oracle_mod.preprocess(rowPtr, colIdx, N, 16, 16)
+        graphs.append((N, torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda(), want))
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(k):
+        N, rp, ci, want = graphs[k]
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for turn in range(10):
+                try:
+                    got = capi.preprocess(rp, ci, N, two_phase=bool(turn % 2))
+                except RuntimeError as e:
+                    if want is not None or "column index" not in str(e):
+                        wrong.append((k, turn, str(e)))
+                    continue
+                torch.cuda.current_stream().synchronize()
+                if want is None or got["blockCount"] != want["blockCount"] or not np.array_equal(
+                        got["sparseAToXidx"].cpu().numpy(), want["sparseAToXidx"]):
+                    wrong.append((k, turn))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong
