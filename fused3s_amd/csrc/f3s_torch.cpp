@@ -185,7 +185,7 @@ void write_cu_time(const torch::Tensor& timer, int64_t nBlocks, const std::strin
 // its packet does without the write-back that makes results visible outside of the GPU (1.6 us).
 struct TimingEvents {
   hipEvent_t start = nullptr, stop = nullptr;
-  TimingEvents() {
+  void create() {  // not in a constructor: an object whose constructor throws is not destroyed
     TORCH_CHECK(hipEventCreateWithFlags(&start, hipEventDisableSystemFence) == hipSuccess &&
                 hipEventCreate(&stop) == hipSuccess);
   }
@@ -205,6 +205,7 @@ std::vector<torch::Tensor> timed_launch(const char* what, const torch::Tensor& o
                                         torch::Tensor scores, F&& launch) {
   hipStream_t stream = at::hip::getCurrentHIPStream().stream();
   TimingEvents events;
+  events.create();
   TORCH_CHECK(hipEventRecord(events.start, stream) == hipSuccess);
   const int rc = launch(static_cast<void*>(stream));
   hipError_t e1 = hipEventRecord(events.stop, stream);
