@@ -41,6 +41,7 @@
 // All results are bit-identical to the reference's algorithm with edgeToRow[e] = row(e).
 
 #include <mutex>
+#include <type_traits>
 
 #include "f3s_common.h"
 
@@ -110,6 +111,8 @@ __device__ __forceinline__ unsigned wave_inclusive_scan(unsigned v, int /*lane*/
   v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
   return v;
 }
+
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // 16 bytes of an output that this call does not read again, past the caches
 __device__ __forceinline__ void store_streaming(uint4* p, const uint4& v) {
@@ -2194,10 +2197,16 @@ constexpr size_t fill_all_lds(int nBins) {
 // never read back and the column ids are read from memory once (the second and third reads of a
 // window's 30 KB come from the L2).
 //
-// Neither kernel is bound by memory (on a 115 M-edge graph the vector ALUs are busy about half of
-// the time and HBM a quarter), so they are written for few instructions per edge: a window's edges are split into whole groups of four consecutive edges
-// from a 4-aligned index (no per-edge range checks, 16-byte loads and stores) and at most six
-// edges at the window's two ends, which single threads handle one by one.
+// Neither kernel is bound by memory alone: on a 115 M-edge graph of 233 k nodes the second one takes
+// 577 us for 2.2 GB that it cannot do without, and the vector ALUs are busy half of that. So both are
+// written for few instructions per edge: a window's edges are split into whole groups of four
+// consecutive edges from a 4-aligned index (no per-edge range checks, 16-byte loads and stores) and at
+// most six edges at the window's two ends, which single threads handle one by one, as they do the
+// (at most fifteen) groups in which a row starts. On that graph: such groups out of the main loop, ids
+// collected in LDS instead of enumerated from the bitset, 16-bit prefixes (which make the room for
+// them) and the first loads in front of the clearing 738 -> 610 us; outputs past the caches, which
+// leaves the column ids there for their second and third reading, 610 -> 577 us and the count kernel
+// 129 -> 88 us.
 
 // Workgroup barrier that orders LDS traffic only: unlike __syncthreads() it does not wait for the
 // wave's outstanding global loads and stores, which then overlap the next phase. For phases that
@@ -2229,43 +2238,46 @@ __device__ __forceinline__ int loose_edge(const EdgeSplit& sp, int eS, int eE, i
   return (i < 6 && e < eE) ? e : -1;
 }
 
-// Sets the bits of the window's column ids in `bits` (32-bit words). Returns false (for the
-// calling thread) when it met a column outside [0, N). U groups per thread and step, loads first.
+// The groups of a thread's step, from e0 on: U of them, TB apart. A group past the end repeats the first
+// one (its bits are set already).
+template <int TB, int U>
+__device__ __forceinline__ void load_groups(const int32_t* __restrict__ colIdx, const EdgeSplit& sp,
+                                            int e0, int4 (&c)[U]) {
+#pragma unroll
+  for (int g = 0; g < U; g++) {
+    const int e = e0 + 4 * g * TB < sp.gB ? e0 + 4 * g * TB : e0;
+    c[g] = *reinterpret_cast<const int4*>(colIdx + e);
+  }
+}
+
+// Sets the bits of the window's column ids in `bits` (32-bit words). c: the thread's first step, which
+// the caller has requested before it cleared the bits. Returns false (for the calling thread) when it
+// met a column outside [0, N); such a column sets the bit of N - 1.
 template <int TB, int U>
 __device__ __forceinline__ bool set_column_bits(const int32_t* __restrict__ colIdx, int eS, int eE,
-                                                const EdgeSplit& sp, unsigned N, uint32_t* bits) {
+                                                const EdgeSplit& sp, unsigned N, uint32_t* bits,
+                                                int4 (&c)[U]) {
   const int tid = threadIdx.x;
-  bool ok = true;
-  for (int e0 = sp.gA + 4 * tid; e0 < sp.gB; e0 += 4 * U * TB) {
-    int4 c[U];
+  unsigned most = 0;
+  const auto set = [&](unsigned col) {
+    most = max(most, col);
+    col = min(col, N - 1u);
+    atomicOr(&bits[col >> 5], 1u << (col & 31));
+  };
+  for (int e0 = sp.gA + 4 * tid; e0 < sp.gB;) {
 #pragma unroll
     for (int g = 0; g < U; g++) {
-      // a group past the end repeats the first one (its bits are set already)
-      const int e = e0 + 4 * g * TB < sp.gB ? e0 + 4 * g * TB : e0;
-      c[g] = *reinterpret_cast<const int4*>(colIdx + e);
+      set((unsigned)c[g].x);
+      set((unsigned)c[g].y);
+      set((unsigned)c[g].z);
+      set((unsigned)c[g].w);
     }
-#pragma unroll
-    for (int g = 0; g < U; g++) {
-      const unsigned col[4] = {(unsigned)c[g].x, (unsigned)c[g].y, (unsigned)c[g].z,
-                               (unsigned)c[g].w};
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        if (col[u] < N)
-          atomicOr(&bits[col[u] >> 5], 1u << (col[u] & 31));
-        else
-          ok = false;
-      }
-    }
+    e0 += 4 * U * TB;
+    if (e0 < sp.gB) load_groups<TB, U>(colIdx, sp, e0, c);
   }
   const int e = loose_edge(sp, eS, eE, tid);
-  if (e >= 0) {
-    const unsigned c = (unsigned)colIdx[e];
-    if (c < N)
-      atomicOr(&bits[c >> 5], 1u << (c & 31));
-    else
-      ok = false;
-  }
-  return ok;
+  if (e >= 0) set((unsigned)colIdx[e]);
+  return most < N;
 }
 
 template <int W, int TB>
@@ -2284,12 +2296,14 @@ __global__ __launch_bounds__(TB) void window_count_kernel(
     if (tid == 0) blockPartition[w] = 0;
     return;
   }
+  const EdgeSplit sp = split_edges(eS, eE);
+  int4 c[4];
+  if (sp.gA + 4 * tid < sp.gB) load_groups<TB, 4>(colIdx, sp, sp.gA + 4 * tid, c);
   const int nGroups = range >> 7;
   for (int i = tid; i < nGroups; i += TB)
     reinterpret_cast<uint4*>(bits)[i] = make_uint4(0, 0, 0, 0);
   lds_barrier();
-  const EdgeSplit sp = split_edges(eS, eE);
-  if (!set_column_bits<TB, 4>(colIdx, eS, eE, sp, (unsigned)N, bits)) {
+  if (!set_column_bits<TB, 4>(colIdx, eS, eE, sp, (unsigned)N, bits, c)) {
     hdr->error = 1;  // window_rank_fill_kernel asks here, the host over there
     *error = 1;
   }
@@ -2313,11 +2327,15 @@ __global__ __launch_bounds__(TB) void window_count_kernel(
 constexpr int kRankFillThreads = 768;
 // 64-bit bitset words per thread of window_rank_fill_kernel at the largest column range
 constexpr int kRankFillPerMax = (kRangeMax / 64 + kRankFillThreads - 1) / kRankFillThreads;
+// bytes of bitset and prefixes (16 bits per 64-bit word), a multiple of 16
+constexpr int rank_fill_bitset_bytes(int range) { return (range / 64 * 10 + 15) & ~15; }
 
-// Dynamic LDS: bitset (range/64 64-bit words) | set bits before each word (range/64 32-bit words)
-// | chunkBytes of TC-block bitmaps. A window with a repeated or descending column is handed to
-// fill_window_generic once its edgeToColumn entries are written, with the whole of the dynamic LDS
-// as that routine's arrays.
+// Dynamic LDS: bitset (range/64 64-bit words) | set bits before each word (range/64 16-bit words)
+// | chunkBytes: the window's TC-block bitmaps, then the low halves of its column ids, in rank order; a
+// window with more blocks than both have room for there (or whose prefixes need more than 16 bits, see
+// `big`) takes its blocks in chunks of bitmaps and enumerates its ids from the bitset. A window with a
+// repeated or descending column is handed to fill_window_generic once its edgeToColumn entries are
+// written, with the whole of the dynamic LDS as that routine's arrays.
 template <int W, int TB>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6, 6)))
 void window_rank_fill_kernel(
@@ -2332,23 +2350,25 @@ void window_rank_fill_kernel(
   constexpr int LOGW = (W == 16) ? 4 : 3;
   constexpr int NWAVE = TB / 64;
   constexpr int PER = kRankFillPerMax;
+  constexpr int HIGH = (kRangeMax + 65535) >> 16;  // values of a column id's upper half
   static_assert(TB == kRankFillThreads, "PER is computed for this workgroup size");
   extern __shared__ __align__(16) uint32_t smem[];
   const int nW64 = range >> 6;  // even: range is a multiple of 128
   unsigned long long* bits64 = reinterpret_cast<unsigned long long*>(smem);
   uint32_t* bits = smem;
-  uint32_t* pref = smem + 2 * nW64;
-  const int bitsetWords = (3 * nW64 + 3) & ~3;  // 32-bit words of bitset + prefixes, 16-byte padded
-  unsigned long long* sBm = reinterpret_cast<unsigned long long*>(smem + bitsetWords);
-  const int TC = chunkBytes / (WPT * 8);
+  uint16_t* pref = reinterpret_cast<uint16_t*>(smem + 2 * nW64);
+  const int bitsetBytes = rank_fill_bitset_bytes(range);
+  unsigned long long* sBm = reinterpret_cast<unsigned long long*>(smem + bitsetBytes / 4);
   __shared__ int sRow[17];
   __shared__ unsigned sWaveTot[NWAVE];
-  __shared__ unsigned sTot[PER * NWAVE];  // set bits per (round, wave), then their exclusive scan
+  __shared__ unsigned sTot[PER * NWAVE];     // set bits per (round, wave)
+  __shared__ unsigned sBefore[PER * NWAVE];  // and in front of it
+  __shared__ unsigned sHigh[HIGH];        // distinct columns below 65536 h
   __shared__ unsigned sUnsorted;          // bit r: row r's columns are not strictly ascending
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = uniform(tid >> 6);
   // windows start in the heavy-first order that the scan kernel has just written: the longest
   // ones first, so that none of them is still running alone when the others are done
   const int w = order[blockIdx.x];
@@ -2357,59 +2377,70 @@ void window_rank_fill_kernel(
   const int base = rowWindowOffset[w];
   const int nb = rowWindowOffset[w + 1] - base;
   const int r0 = w * 16;
-  if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
-  if (tid == 0) sUnsorted = 0u;
-  for (int i = tid; i < (nW64 >> 1); i += TB)
-    reinterpret_cast<uint4*>(bits)[i] = make_uint4(0, 0, 0, 0);
-  lds_barrier();
-  const int eS = sRow[0], eE = sRow[16];
+  const int eS = rowPtr[min(r0, N)], eE = rowPtr[min(r0 + 16, N)];
   if (eE <= eS) return;
   const EdgeSplit sp = split_edges(eS, eE);
-
-  // ---- the window's distinct columns as a bitset (validated by window_count_kernel)
-  set_column_bits<TB, 2>(colIdx, eS, eE, sp, (unsigned)N, bits);
+  constexpr int U = 2;  // groups of a thread in flight together
+  {
+    // ---- the window's distinct columns as a bitset (validated by window_count_kernel)
+    int4 c[U];
+    if (sp.gA + 4 * tid < sp.gB) load_groups<TB, U>(colIdx, sp, sp.gA + 4 * tid, c);
+    if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
+    if (tid < HIGH) sHigh[tid] = 0xFFFFFFFFu;
+    if (tid == 0) sUnsorted = 0u;
+    for (int i = tid; i < (nW64 >> 1); i += TB)
+      reinterpret_cast<uint4*>(bits)[i] = make_uint4(0, 0, 0, 0);
+    lds_barrier();
+    set_column_bits<TB, U>(colIdx, eS, eE, sp, (unsigned)N, bits, c);
+  }
   lds_barrier();
 
-  // ---- set bits before every 64-bit word; the compacted column ids, which are the set bits in
-  // ascending order. Thread t owns the words t, t + TB, ... (neighbouring lanes, neighbouring
-  // words): a wave-level scan per round, one scan of the (round, wave) totals by the first wave.
+  // ---- set bits before every 64-bit word. Thread t owns the words t, t + TB, ... (neighbouring lanes,
+  // neighbouring words): a wave-level scan per round, then every wave scans the (round, wave) totals.
   const int per = (nW64 + TB - 1) / TB;  // <= PER
+  unsigned before[PER];  // within the wave's 64 words
 #pragma unroll
   for (int k = 0; k < PER; k++) {
     if (k < per) {
       const int i = k * TB + tid;
       const unsigned cnt = i < nW64 ? (unsigned)__popcll(bits64[i]) : 0u;
       const unsigned incl = wave_inclusive_scan(cnt, lane);
-      if (i < nW64) pref[i] = incl - cnt;  // within the wave's 64 words for now
+      before[k] = incl - cnt;
       if (lane == 63) sTot[k * NWAVE + wave] = incl;
     }
   }
   lds_barrier();
-  if (wave == 0) {
-    // exclusive scan of the per * NWAVE totals in (round, wave) order, two per lane
+  unsigned pairIncl, pairBoth, pairFirst;  // lane l: pair l of the totals
+  {
     static_assert(PER * NWAVE <= 128, "two totals per lane");
     const int n = per * NWAVE;
-    const unsigned a = (2 * lane < n) ? sTot[2 * lane] : 0u;
-    const unsigned b = (2 * lane + 1 < n) ? sTot[2 * lane + 1] : 0u;
-    const unsigned inc = wave_inclusive_scan(a + b, lane);
-    if (2 * lane < n) sTot[2 * lane] = inc - a - b;
-    if (2 * lane + 1 < n) sTot[2 * lane + 1] = inc - b;
-    if (lane == 63) sWaveTot[0] = inc;
+    pairFirst = (2 * lane < n) ? sTot[2 * lane] : 0u;
+    const unsigned second = (2 * lane + 1 < n) ? sTot[2 * lane + 1] : 0u;
+    pairBoth = pairFirst + second;
+    pairIncl = wave_inclusive_scan(pairBoth, lane);
+    if (wave == 0 && 2 * lane < n) sBefore[2 * lane] = pairIncl - pairBoth;
+    if (wave == 0 && 2 * lane + 1 < n) sBefore[2 * lane + 1] = pairIncl - second;
   }
-  lds_barrier();
-  const unsigned nCols = sWaveTot[0];
-  {
-    int32_t* idDst = sparseAToXidx + (int64_t)base * W;
-    char* idBytes = reinterpret_cast<char*>(idDst);
-    for (int k = 0; k < per; k++) {
+  const unsigned nCols = (unsigned)__builtin_amdgcn_readlane((int)pairIncl, 63);
+  // more distinct columns than a 16-bit prefix can name: the prefixes stay relative to their wave's 64
+  // words and sBefore is added on every use
+  const bool big = nCols > 0xFFFFu;
+  const bool idsInLds = nb * (WPT * 8 + W * 2) <= chunkBytes && !big;
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    if (k < per) {
       const int i = k * TB + tid;
-      if (i < nW64) {
-        unsigned pos = sTot[k * NWAVE + wave] + pref[i];
-        pref[i] = pos;
-#ifdef F3S_PROBE_PRE_NO_IDS
-        continue;
-#endif
-        // 32 bits at a time, with a 32-bit byte offset from the window's first id slot
+      const int at = k * NWAVE + wave;
+      unsigned front = (unsigned)__builtin_amdgcn_readlane((int)(pairIncl - pairBoth), at >> 1);
+      if (at & 1) front += (unsigned)__builtin_amdgcn_readlane((int)pairFirst, at >> 1);
+      const unsigned pos = front + before[k];
+      if (i < nW64) pref[i] = (uint16_t)(big ? before[k] : pos);
+      if (idsInLds) {
+        if ((i & 1023) == 0 && i < nW64) sHigh[i >> 10] = pos;
+      } else if (i < nW64) {
+        // the compacted column ids, which are the set bits in ascending order, 32 bits at a time, with a
+        // 32-bit byte offset from the window's first id slot
+        char* idBytes = reinterpret_cast<char*>(sparseAToXidx + (int64_t)base * W);
         const unsigned long long x = bits64[i];
         unsigned off = pos * 4u;
 #pragma unroll
@@ -2424,30 +2455,28 @@ void window_rank_fill_kernel(
         }
       }
     }
-    // the slots that the last block leaves unused hold 0
-    for (int i = (int)nCols + tid; i < nb * W; i += TB) idDst[i] = 0;
   }
+  if (!idsInLds)  // the slots that the last block leaves unused hold 0
+    for (int i = (int)nCols + tid; i < nb * W; i += TB) sparseAToXidx[(int64_t)base * W + i] = 0;
 
-  // ---- ranks, rows and bitmaps. The first chunk of TC blocks also writes edgeToColumn /
-  // edgeToRow; a window with more blocks ranks its edges again per chunk (the bitset stays in
-  // LDS).
-  auto rank_of = [&](int col) -> int {
+  // ---- ranks, rows and bitmaps. The first chunk of TC blocks also writes edgeToColumn / edgeToRow;
+  // a window of several chunks ranks its edges again per chunk (the bitset stays in LDS).
+  const auto rank_of = [&](int col) -> int {
     const unsigned wd = (unsigned)col >> 6;
-    const unsigned long long below = bits64[wd] & ((1ull << (col & 63)) - 1ull);
-    return (int)(pref[wd] + (unsigned)__popcll(below));
+    const unsigned long long upTo = bits64[wd] << (~col & 63);  // the column's own bit on top
+    unsigned rank = pref[wd] + (unsigned)__popcll(upTo) - 1u;
+    if (big) rank += sBefore[wd >> 6];
+    return (int)rank;
   };
-  unsigned carry = (unsigned)eS;  // absolute edge position where the next TC block starts
   unsigned* sBmWords = reinterpret_cast<unsigned*>(sBm);
-  const int stageBytes = ((bitsetWords * 4) / NWAVE) & ~15;
-  for (int tc0 = 0; tc0 < nb; tc0 += TC) {
-    const int nt = min(TC, nb - tc0);
-    const bool lastChunk = tc0 + TC >= nb;
-    const bool first = tc0 == 0;
-    lds_barrier();  // ranks are read after the prefixes are written (and the previous chunk is out)
-    for (int i = tid; i < nt * WPT; i += TB) sBm[i] = 0ull;
-    lds_barrier();
-    // one edge: rank, row, bit (the window's loose ends and groups that straddle rows)
-    auto one_edge = [&](int e, int col, int r) {
+  // the window's edges against the blocks [tc0, tc0 + nt): bitmap bits, with `ids` the ids' low halves
+  // as well, and edgeToColumn / edgeToRow where tc0 = 0. ids: one chunk holds all blocks.
+  const auto rank_edges = [&](auto ids, int tc0, int nt) {
+    constexpr bool IDS = decltype(ids)::value;
+    const bool first = IDS || tc0 == 0;
+    uint16_t* sId = reinterpret_cast<uint16_t*>(sBm + nt * WPT);
+    // one edge: rank, row, bit (the window's loose ends and the groups that straddle rows)
+    const auto one_edge = [&](int e, int col, int r) {
       const int ec = rank_of(col);
       if (first) {
         edgeToColumn[e] = ec;
@@ -2455,33 +2484,36 @@ void window_rank_fill_kernel(
         if (e > sRow[r] && colIdx[e - 1] >= col) atomicOr(&sUnsorted, 1u << r);
       }
       const int t = (ec >> LOGW) - tc0;
-      if ((unsigned)t < (unsigned)nt) {
+      if (IDS || (unsigned)t < (unsigned)nt) {
         const int cl = ec & (W - 1);
         const int sub = (cl >> 3) * (W / 8) + (r >> 3);
         const int key = (t * WPT + sub) * 8 + 7 - (r & 7);
         atomicOr(&sBmWords[key >> 2], (0x80u >> (cl & 7)) << (8 * (key & 3)));
+        if constexpr (IDS) sId[ec] = (uint16_t)col;
       }
     };
-    // a whole group of four edges
-    auto group = [&](int e0, const int4& c4, int left) {
+    // a whole group of four edges of one row; left: the column in front of it
+    const auto group = [&](int e0, const int4& c4, int left) {
       const int cols[4] = {c4.x, c4.y, c4.z, c4.w};
       const int r = row_of_edge(sRow, e0);
-      if (e0 + 3 >= sRow[r + 1]) {  // the group straddles rows
-#pragma unroll
-        for (int u = 0; u < 4; u++) one_edge(e0 + u, cols[u], row_of_edge(sRow, e0 + u));
-        return;
-      }
+      if (e0 + 3 >= sRow[r + 1]) return;  // it straddles rows: edge by edge below
       int ecs[4];
 #pragma unroll
       for (int u = 0; u < 4; u++) ecs[u] = rank_of(cols[u]);
       if (first) {
 #ifndef F3S_PROBE_PRE_NO_EDGE_STORES
-        *reinterpret_cast<int4*>(edgeToColumn + e0) = make_int4(ecs[0], ecs[1], ecs[2], ecs[3]);
-        *reinterpret_cast<int4*>(edgeToRow + e0) = make_int4(r0 + r, r0 + r, r0 + r, r0 + r);
+        store_streaming(reinterpret_cast<uint4*>(edgeToColumn + e0),
+                        make_uint4(ecs[0], ecs[1], ecs[2], ecs[3]));
+        store_streaming(reinterpret_cast<uint4*>(edgeToRow + e0),
+                        make_uint4(r0 + r, r0 + r, r0 + r, r0 + r));
 #endif
         const bool bad = (e0 > sRow[r] && left >= cols[0]) || cols[0] >= cols[1] ||
                          cols[1] >= cols[2] || cols[2] >= cols[3];
         if (bad) atomicOr(&sUnsorted, 1u << r);
+      }
+      if constexpr (IDS) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) sId[ecs[u]] = (uint16_t)cols[u];
       }
       // Bits of one row. A TC block's bitmap is WPT 64-bit words, one per 8x8 sub-block (column
       // halves first); byte 7 - r%8 of a word is row r%8, MSB first. With rank = 16 t + cl (or
@@ -2498,7 +2530,7 @@ void window_rank_fill_kernel(
       for (int u = 0; u < 4; u++) {
         word[u] = (ecs[u] >> 3) * 4 + wordBias;
         m[u] = rowBit >> (ecs[u] & 7);
-        if ((unsigned)((ecs[u] >> LOGW) - tc0) >= (unsigned)nt) m[u] = 0u;
+        if (!IDS && (unsigned)((ecs[u] >> LOGW) - tc0) >= (unsigned)nt) m[u] = 0u;
       }
 #pragma unroll
       for (int u = 1; u < 4; u++) {
@@ -2509,30 +2541,60 @@ void window_rank_fill_kernel(
       }
 #pragma unroll
       for (int u = 0; u < 4; u++)
-        if (m[u]) atomicOr(&sBmWords[word[u]], m[u]);
+        if (m[u])
+          atomicOr(&sBmWords[word[u]], m[u]);
     };
-    // two groups per thread and step, loads first
+    // two groups per thread and step, loads first. A group's left neighbour is the last edge of the lane
+    // before, whose group lies directly in front; the wave's first lane fetches its own.
 #ifdef F3S_PROBE_PRE_NO_FILL
     if (nb < 0)
 #endif
-    for (int e0 = sp.gA + 4 * tid; e0 < sp.gB; e0 += 8 * TB) {
-      const int e1 = e0 + 4 * TB;
-      const bool two = e1 < sp.gB;
-      const int4 a = *reinterpret_cast<const int4*>(colIdx + e0);
-      int4 b = a;
-      if (two) b = *reinterpret_cast<const int4*>(colIdx + e1);
-      int leftA = -1, leftB = -1;
-      if (first) {
-        if (e0 > eS) leftA = colIdx[e0 - 1];
-        if (two) leftB = colIdx[e1 - 1];
+    for (int e0 = sp.gA + 4 * tid; e0 < sp.gB; e0 += 4 * U * TB) {
+      int4 c[U];
+      load_groups<TB, U>(colIdx, sp, e0, c);
+      int left[U];
+#pragma unroll
+      for (int g = 0; g < U; g++) {
+        const int e = e0 + 4 * g * TB;
+        left[g] = -1;
+        if (first && lane == 0 && e > eS && e < sp.gB) left[g] = colIdx[e - 1];
       }
-      group(e0, a, leftA);
-      if (two) group(e1, b, leftB);
+#pragma unroll
+      for (int g = 0; g < U; g++) {
+        left[g] = __builtin_amdgcn_update_dpp(left[g], c[g].w, 0x138, 0xf, 0xf, false);  // wave_shr:1
+        if (e0 + 4 * g * TB < sp.gB) group(e0 + 4 * g * TB, c[g], left[g]);
+      }
     }
-    {
-      const int e = loose_edge(sp, eS, eE, tid);
+    // Edge by edge: the groups with a row boundary inside (lanes 4 k - 4 .. 4 k - 1 of the first wave take
+    // the group around the start of row k, unless row k - 1 starts inside it too) and the loose ends
+    // (the second wave). Inside the loop above such a group would hold up its whole wave.
+    if (tid < 128) {
+      int e = -1;
+      if (tid < 64) {
+        const int k = (tid >> 2) + 1;
+        const int start = sRow[k];
+        const int g = start & ~3;
+        if (k < 16 && start != g && g >= sp.gA && g < sp.gB && sRow[k - 1] <= g) e = g + (tid & 3);
+      } else {
+        e = loose_edge(sp, eS, eE, tid - 64);
+      }
       if (e >= 0) one_edge(e, colIdx[e], row_of_edge(sRow, e));
     }
+  };
+
+  unsigned carry = (unsigned)eS;  // absolute edge position where the next TC block starts
+  const int stageBytes = (bitsetBytes / NWAVE) & ~15;
+  const int TC = idsInLds ? nb : chunkBytes / (WPT * 8);
+  for (int tc0 = 0; tc0 < nb; tc0 += TC) {
+    const int nt = min(TC, nb - tc0);
+    const bool lastChunk = tc0 + TC >= nb;
+    if (tc0 > 0) lds_barrier();  // the previous chunk is out
+    for (int i = tid; i < nt * WPT; i += TB) sBm[i] = 0ull;
+    lds_barrier();  // ranks are read after the prefixes are written
+    if (idsInLds)
+      rank_edges(std::true_type{}, 0, nt);
+    else
+      rank_edges(std::false_type{}, tc0, nt);
     lds_barrier();
     if (sUnsorted != 0u) break;  // known after the first pass over the window's edges
     for (int tb = 0; tb < nt; tb += TB) {
@@ -2595,7 +2657,40 @@ void window_rank_fill_kernel(
     }
     {
       unsigned long long* bmDst = bitmap + ((int64_t)base + tc0) * WPT;
-      for (int i = tid; i < nt * WPT; i += TB) bmDst[i] = sBm[i];
+      for (int i = tid; i < nt * WPT; i += TB) __builtin_nontemporal_store(sBm[i], bmDst + i);
+    }
+    if (idsInLds) {
+      // The ids, four per thread and step, their upper halves from the ranks at which those change (mostly
+      // not within a wave's step); the slots that the last block leaves unused hold 0.
+      const uint2* lows = reinterpret_cast<const uint2*>(sBm + nt * WPT);
+      uint4* idDst = reinterpret_cast<uint4*>(sparseAToXidx + (int64_t)base * W);
+      unsigned from[HIGH];
+#pragma unroll
+      for (int h = 1; h < HIGH; h++) from[h] = (unsigned)uniform((int)sHigh[h]);
+      for (int i = tid; i < nt * (W / 4); i += TB) {
+        const uint2 low = lows[i];
+        const unsigned first = 4u * i, last = first + 3u;
+        unsigned high = 0, highLast = 0;
+#pragma unroll
+        for (int h = 1; h < HIGH; h++) {
+          high += first >= from[h] ? 1u : 0u;
+          highLast += last >= from[h] ? 1u : 0u;
+        }
+        high <<= 16;
+        uint4 id = make_uint4((low.x & 0xFFFFu) | high, (low.x >> 16) | high,
+                              (low.y & 0xFFFFu) | high, (low.y >> 16) | high);
+        if (high != highLast << 16 || last >= nCols) {
+          unsigned v[4] = {low.x & 0xFFFFu, low.x >> 16, low.y & 0xFFFFu, low.y >> 16};
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+#pragma unroll
+            for (int h = 1; h < HIGH; h++) v[u] += first + u >= from[h] ? 0x10000u : 0u;
+            if (first + u >= nCols) v[u] = 0u;
+          }
+          id = make_uint4(v[0], v[1], v[2], v[3]);
+        }
+        store_streaming(idDst + i, id);
+      }
     }
   }
   if (sUnsorted != 0u) {
@@ -2604,7 +2699,7 @@ void window_rank_fill_kernel(
     __syncthreads();
     if (tid == 0) sUnsorted = 0u;
     __syncthreads();
-    const int dynBytes = bitsetWords * 4 + chunkBytes;
+    const int dynBytes = bitsetBytes + chunkBytes;
     const int tcg = dynBytes / (64 + WPT * 8);
     unsigned* gCnt = reinterpret_cast<unsigned*>(smem);                                // [tcg*16]
     unsigned long long* gBm = reinterpret_cast<unsigned long long*>(smem + tcg * 16);  // [tcg*WPT]
@@ -3084,7 +3179,7 @@ int enqueue_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int 
   if (nRW > 0 && long_windows(nRW, E) && N <= kRangeMax && aligned16) {
     WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
     const int range = ((N + 127) / 128) * 128;
-    const int bitsetBytes = ((3 * (range / 64) + 3) & ~3) * 4;  // bitset + per-word prefixes
+    const int bitsetBytes = rank_fill_bitset_bytes(range);
     // two workgroups of twelve waves per CU (registers allow no more): half of the CU's LDS each
     int chunkBytes = (160 * 1024) / 2 - 1024 - bitsetBytes;
     chunkBytes &= ~255;

@@ -97,6 +97,55 @@ def test_window_counts(oracle_mod, nRW, edges, wide, W):
         assert np.array_equal(bm, want["tcbBitMap"]), two_phase
 
 
+def split_columns(rng, cols, lengths):
+    """16 ascending rows of the given lengths over `cols`, which together name every one of them."""
+    cols = np.sort(cols)
+    rows = [np.sort(rng.choice(cols, size=min(k, len(cols)), replace=False)) for k in lengths]
+    at = int(np.argmax(lengths))
+    missing = np.setdiff1d(cols, np.concatenate(rows))
+    rows[at] = np.union1d(rows[at], missing)
+    return [r.astype(np.int32) for r in rows]
+
+
+# Graphs of long windows keep a window's ids in LDS beside its bitmaps where both fit (up to 940 blocks of
+# 16 columns at this N), as 16-bit halves whose upper ones change at multiples of 65 536, and count with
+# 16-bit prefixes up to 65 535 distinct columns: windows on both sides of each, rows that start at every
+# place of a group of four edges, several of them in one group, and a window of repeated columns.
+@pytest.mark.parametrize("W", [16, 8])
+def test_long_windows_ids_and_prefixes(oracle_mod, W):
+    from fused3s_amd import capi
+    print("case long windows, ids and prefixes W=%d" % W, flush=True)
+    rng = np.random.default_rng(41 + W)
+    N = 131_200
+    even = lambda n: rng.choice(N, size=n, replace=False)
+    ends = np.concatenate([np.arange(101), np.arange(N - 99, N)])
+    about = np.concatenate([np.arange(65_530, 65_541), np.arange(131_069, 131_076)])
+    windows = [split_columns(rng, even(n), [n // 8] * 16) for n in (15_039, 15_040, 15_041)]
+    windows += [split_columns(rng, even(n), [n // 2] * 16) for n in (65_535, 65_536, 65_537)]
+    windows += [split_columns(rng, ends, [k % 4 for k in range(15)] + [150])]
+    windows += [split_columns(rng, about, [1, 0, 2, 1, 1, 1, 3, 0, 0, 1, 5, 2, 2, 1, 1, 18])]
+    windows += [split_columns(rng, even(40), [1] * 16), split_columns(rng, even(3), [0] * 15 + [3])]
+    rough = split_columns(rng, even(9_000), [1_000] * 16)
+    rough[7][500] = rough[7][2]
+    windows += [rough]
+    nRW = (N + 15) // 16
+    while sum(len(r) for rows in windows for r in rows) < 2048 * nRW:  # every second column, 16 rows
+        windows += [[np.flatnonzero(rng.random(N) < 0.5).astype(np.int32) for _ in range(16)]]
+    rows = [r for w in windows for r in w]
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:len(rows) + 1] = np.cumsum([len(r) for r in rows])
+    rowPtr[len(rows) + 1:] = rowPtr[len(rows)]
+    colIdx = np.concatenate(rows).astype(np.int32)
+    want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, W)
+    assert list(want["blockPartition"][:6]) == [-(-n // W) for n in (15_039, 15_040, 15_041, 65_535,
+                                                                    65_536, 65_537)]
+    got = capi.preprocess(torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda(), N, 16, W)
+    for k in KEYS:
+        assert np.array_equal(got[k].cpu().numpy(), want[k]), k
+    assert np.array_equal(got["tcbBitMap"].cpu().view(torch.int64).numpy().view(np.uint64),
+                          want["tcbBitMap"])
+
+
 # The order's histogram has 4096 bins: windows of 4095 blocks and more take further rounds. Counts at
 # the rounds' edges, ties of more than a wave, rounds that no window falls into, and one window that
 # spans every node
