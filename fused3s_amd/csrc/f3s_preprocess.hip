@@ -22,7 +22,8 @@
 //   window_scan_kernel, finalize_count_kernel, finalize_*_kernel
 //                        scan of the per-window block counts (src/utils.cu:293-300) and the windows
 //                        by descending block count (src/utils.cu:400-436): places from a histogram
-//                        of the counts, or on graphs of many windows a stable LSD radix sort.
+//                        of the counts, or on graphs of very many windows (and in the count / fill
+//                        calls of graphs of many) a stable LSD radix sort.
 //   window_rank_all_kernel, window_fill_all_kernel
 //                        the two phases on graphs of up to 16384 windows that are not all long: the
 //                        wave per short window, the workgroup per long one and the order of the
@@ -67,10 +68,32 @@ constexpr int kFillChunkMid = 320, kFillChunkLong = 1280;
 constexpr int kFillMid = 4096;
 constexpr int kFillFewLong = 4096;
 
+// The windows that the kernels with a wave per window leave to larger workgroups, as those kernels meet
+// them: `mid` of up to midMax edges from the front of an array of nRW entries, `large` of more from its
+// back. The counts lie in the workspace header and are cleared before phase 1.
+struct LongLists {
+  int mid, large;
+};
+struct LongQueue {
+  LongLists* counts;  // null: no lists, nobody asks for them (or they are looked for, find_windows)
+  int32_t* list;
+  int nRW;
+  int midMax;
+  __device__ __forceinline__ void add(int w, int edges) const {
+    if (edges <= midMax)
+      list[atomicAdd(&counts->mid, 1)] = w;
+    else
+      list[nRW - 1 - atomicAdd(&counts->large, 1)] = w;
+  }
+  __device__ __forceinline__ int size(bool large) const { return large ? counts->large : counts->mid; }
+  __device__ __forceinline__ int at(bool large, int k) const { return list[large ? nRW - 1 - k : k]; }
+};
+
 // workspace header (bytes 0..255)
 struct WsHeader {
   int error;    // graphs of long windows: a column index outside [0, N) was met
   int maxCount; // largest per-window block count (multi-workgroup finalize)
+  LongLists rank, fill;
 };
 // Where phase 1 leaves its result: a device array of the caller's, or pinned host memory that the
 // host reads when the stream is done, without a copy (a copy to pageable memory costs 7 us more).
@@ -219,7 +242,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 template <int W>
 __global__ __launch_bounds__(64) void window_rank_small_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
-    int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
+    LongQueue queue, int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
     int32_t* __restrict__ edgeToRow, int* __restrict__ error) {
   __shared__ uint32_t sKeys[kSortMax];
   __shared__ uint32_t sUniq[kSortMax];
@@ -236,7 +259,10 @@ __global__ __launch_bounds__(64) void window_rank_small_kernel(
     if (lane == 0) blockPartition[w] = 0;
     return;
   }
-  if (n > kSortMax) return;  // left to another kernel
+  if (n > kSortMax) {  // left to another kernel
+    if (lane == 0 && queue.counts) queue.add(w, n);
+    return;
+  }
   uint32_t* keys = sKeys;
   uint32_t* uniq = sUniq;
   int P = 64;
@@ -475,7 +501,7 @@ struct alignas(16) RankBinsLds {  // of one wave
 template <int W>
 __device__ __forceinline__ void rank_window_by_bins(
     int w, const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N,
-    int colBits, RankBinsLds& lds, int32_t* __restrict__ blockPartition,
+    int colBits, const LongQueue& queue, RankBinsLds& lds, int32_t* __restrict__ blockPartition,
     int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
     int* __restrict__ error) {
   constexpr int IDX_BITS = 10;
@@ -491,7 +517,10 @@ __device__ __forceinline__ void rank_window_by_bins(
     if (lane == 0) blockPartition[w] = 0;
     return;
   }
-  if (n > kBinsMax) return;  // left to another kernel
+  if (n > kBinsMax) {  // left to another kernel
+    if (lane == 0 && queue.counts) queue.add(w, n);
+    return;
+  }
   uint32_t* a = lds.bufA;
   uint32_t* b = lds.bufB;
   uint32_t* hist = lds.hist;
@@ -644,10 +673,10 @@ __device__ __forceinline__ void rank_window_by_bins(
 template <int W>
 __global__ __launch_bounds__(64) void window_rank_bins_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int colBits,
-    int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
+    LongQueue queue, int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
     int32_t* __restrict__ edgeToRow, int* __restrict__ error) {
   __shared__ RankBinsLds lds;
-  rank_window_by_bins<W>((int)blockIdx.x, rowPtr, colIdx, N, colBits, lds, blockPartition,
+  rank_window_by_bins<W>((int)blockIdx.x, rowPtr, colIdx, N, colBits, queue, lds, blockPartition,
                          edgeToColumn, edgeToRow, error);
 }
 
@@ -751,25 +780,20 @@ __device__ __forceinline__ void rank_window_by_bitset(
   if (tid == 0) blockPartition[w] = (int)((uniqueBefore + W - 1) / W);
 }
 
-// SCAN: the grid is a fixed number of workgroups that look for the windows of more than minEdges
-// edges (graphs of mostly short windows); else workgroup b takes window b, if it is that long.
-template <int W, int TB, bool SCAN>
+// LISTED: the large windows of the queue, of which those of more than minEdges edges are taken (graphs of
+// mostly short windows); else workgroup b takes window b, if it is that long.
+template <int W, int TB, bool LISTED>
 __global__ __launch_bounds__(TB) void window_rank_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
-    int range, int nPasses, int minEdges, int32_t* __restrict__ blockPartition,
+    int range, int nPasses, int minEdges, LongQueue queue, int32_t* __restrict__ blockPartition,
     int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
     int* __restrict__ error) {
   extern __shared__ __align__(16) uint32_t smem[];
-  if constexpr (SCAN) {
-    __shared__ int sList[TB];
-    __shared__ int sListLen;
-    for (int64_t first = 0; first < nRW; first += (int64_t)TB * gridDim.x) {
-      const int found = find_windows(rowPtr, N, nRW, first, (int)gridDim.x, minEdges, 0x7FFFFFFF,
-                                     sList, &sListLen);
-      for (int k = 0; k < found; k++)
-        rank_window_by_bitset<W, TB>(sList[k], rowPtr, colIdx, N, range, nPasses, minEdges, smem,
-                                     blockPartition, edgeToColumn, edgeToRow, error);
-    }
+  if constexpr (LISTED) {
+    const int listed = queue.size(true);
+    for (int k = blockIdx.x; k < listed; k += (int)gridDim.x)
+      rank_window_by_bitset<W, TB>(queue.at(true, k), rowPtr, colIdx, N, range, nPasses, minEdges, smem,
+                                   blockPartition, edgeToColumn, edgeToRow, error);
   } else {
     rank_window_by_bitset<W, TB>((int)blockIdx.x, rowPtr, colIdx, N, range, nPasses, minEdges,
                                  smem, blockPartition, edgeToColumn, edgeToRow, error);
@@ -795,7 +819,7 @@ __global__ __launch_bounds__(kRankAllThreads) void window_rank_all_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int w = ((int)blockIdx.x - longGroups) * NW + wave;
     if (w < nRW)
-      rank_window_by_bins<W>(w, rowPtr, colIdx, N, colBits,
+      rank_window_by_bins<W>(w, rowPtr, colIdx, N, colBits, LongQueue{nullptr, nullptr, 0, 0},
                              reinterpret_cast<RankBinsLds*>(smem)[wave], blockPartition,
                              edgeToColumn, edgeToRow, error);
     return;
@@ -824,6 +848,9 @@ constexpr size_t rank_all_lds(int range) {
 // take an LSD radix sort, eight bits per pass, every wave on its own contiguous part of the keys, and
 // a binary search per edge. (Radix sort and search for all: 163 instead of 128 us for the 4 272 such
 // windows of a 61M-edge graph.)
+// The windows come from the lists that the kernel for short windows has made: where every workgroup looked
+// for its own, some met five and some none (4 272 windows dealt to 8 192 workgroups: 133 instead of
+// 96 us; window_fill_long_kernel 68 instead of 45 us).
 // Two sizes: windows of up to kMedMax edges (256 threads, 36 KiB of LDS, four workgroups per CU), and
 // the handful of windows of up to kLargeMax edges (1024 threads, 144 KiB), which would otherwise each
 // walk the bitset passes alone at the end of the phase.
@@ -839,11 +866,11 @@ constexpr size_t rank_sort_lds() {
   return ((size_t)2 * THREADS * ITEMS + 4 * THREADS) * sizeof(uint32_t);
 }
 
-// takes the windows of more than minEdges and at most THREADS * ITEMS edges
-template <int W, int ITEMS, int THREADS>
+// takes the mid windows of the queue, or (LARGE) the large ones of at most THREADS * ITEMS edges
+template <int W, int ITEMS, int THREADS, bool LARGE>
 __global__ __launch_bounds__(THREADS) void window_rank_sort_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
-    int colBits, int minEdges, int32_t* __restrict__ blockPartition,
+    int colBits, LongQueue queue, int32_t* __restrict__ blockPartition,
     int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
     int* __restrict__ error) {
   constexpr int WAVES = THREADS / 64;
@@ -861,19 +888,17 @@ __global__ __launch_bounds__(THREADS) void window_rank_sort_kernel(
   __shared__ int sRow[17];
   __shared__ unsigned sWaveTot[WAVES];
   __shared__ int sCrowded;
-  __shared__ int sList[THREADS];
-  __shared__ int sListLen;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const unsigned long long ltMask = (1ull << lane) - 1ull;
   const int shiftBins = colBits > BIN_BITS ? colBits - BIN_BITS : 0;
-  for (int64_t first = 0; first < nRW; first += (int64_t)THREADS * gridDim.x) {
-  const int found = find_windows(rowPtr, N, nRW, first, (int)gridDim.x, minEdges, CAP, sList, &sListLen);
-  for (int taken = 0; taken < found; taken++) {
-    __syncthreads();
-    const int w = sList[taken];
+  const int listed = queue.size(LARGE);
+  for (int taken = blockIdx.x; taken < listed; taken += (int)gridDim.x) {
+    const int w = queue.at(LARGE, taken);
     const int r0 = w * 16;
+    if (LARGE && rowPtr[min(r0 + 16, N)] - rowPtr[r0] > CAP) continue;  // window_rank_kernel's
+    __syncthreads();  // the window before this one has left the LDS arrays
     if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
     if (tid == 0) sCrowded = 0;
     reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(0, 0, 0, 0);
@@ -1128,7 +1153,6 @@ __global__ __launch_bounds__(THREADS) void window_rank_sort_kernel(
     }
     if (tid == 0) blockPartition[w] = (int)((nUniq + W - 1) / W);
   }
-  }
 }
 
 // ------------------------------------------------- scan + window ordering
@@ -1188,52 +1212,80 @@ __device__ __forceinline__ void scan_windows(const int32_t* __restrict__ blockPa
 // nRW / TB of them share the work (a radix sort by one workgroup of 1024 threads took 21 us for
 // 10 584 windows, 30 us for 14 561). hist: nBins words, a multiple of TB. blocks(i): window i's count,
 // not negative.
+// ROWS: more windows than 16 bits count, so the two halves are words of their own, hist 2 nBins of them;
+// and the histogram of the first nBins - 1 counts is added up from `rows`, one per TB windows
+// (finalize_partials_kernel): one after the other for all windows, the LDS additions of 153 000 windows
+// take 60 us, of 64 lanes a handful of distinct counts.
 // Counts from nBins - 1 on share the last bin; while it holds any, another round orders the windows
 // of the next nBins - 1 counts, so a call takes as many rounds as its largest count asks for (at most
 // nine: 32 769 blocks of 8 columns, 4096 bins); nearly every graph takes one. Wide windows that compare
 // themselves with all others instead, one after the other in a wave, are slow where there are many:
 // 100 000 nodes of 2 500 edges, 8-column blocks, 6 245 of 6 250 windows: a preprocessing call of 7.54
 // instead of 7.01 ms; 262 000 nodes of 2 200 edges: 17.01 instead of 15.03 ms.
-template <int TB, typename BlocksOf>
+template <int TB, bool ROWS = false, typename BlocksOf>
 __device__ __forceinline__ void order_chunk(const BlocksOf& blocks, int nRW, int first, int nBins,
-                                            int32_t* __restrict__ sortedRowWindows,
-                                            uint32_t* hist) {
+                                            int32_t* __restrict__ sortedRowWindows, uint32_t* hist,
+                                            const uint16_t* __restrict__ rows = nullptr) {
   static_assert(kFinSingleMax < 0x8000, "two counters of windows per word");
   constexpr int NW = TB / 64;
-  constexpr int U = 4;
+  constexpr int U = 4;  // counts of a thread in flight together
   __shared__ unsigned sBinTot[NW];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int top = nBins - 1;
   const int count = first + tid < nRW ? blocks(first + tid) : -1;
+  uint32_t* const ahead = ROWS ? hist + nBins : hist;  // windows in front of `first`, then the places
+  const auto windows_in = [&](int bin) { return ROWS ? hist[bin] : hist[bin] & 0xFFFFu; };
   for (int low = 0;; low += top) {  // windows of low .. low + top - 1 blocks
-    for (int i = tid; i < nBins; i += TB) hist[i] = 0u;
-    __syncthreads();
-    for (int i0 = 0; i0 < nRW; i0 += U * TB) {
-      int c[U];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int i = i0 + u * TB + tid;
-        c[u] = i < nRW ? min(blocks(i) - low, top) : -1;
+    if (ROWS && low == 0) {
+      const int nRows = (nRW + TB - 1) / TB, own = first / TB;
+      for (int b = tid; b < nBins; b += TB) {
+        unsigned all = 0, front = 0;
+#pragma unroll 16
+        for (int r = 0; r < nRows; r++) {
+          const unsigned n = rows[(size_t)r * nBins + b];
+          all += n;
+          front += r < own ? n : 0u;
+        }
+        hist[b] = all;
+        ahead[b] = front;
       }
+    } else {
+      for (int i = tid; i < (ROWS ? 2 : 1) * nBins; i += TB) hist[i] = 0u;
+      __syncthreads();
+      for (int i0 = 0; i0 < nRW; i0 += U * TB) {
+        int c[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        // counts cluster, and lanes that name the same bin are served one after the other: the lanes
-        // that agree with the group's first one are counted with one ballot and added once
-        const int c0 = __builtin_amdgcn_readfirstlane(c[u]);
-        const unsigned one = i0 + u * TB + wave * 64 < first ? 0x10001u : 1u;
-        const unsigned long long same = __ballot(c[u] == c0);
-        if (c[u] >= 0 && c[u] != c0) atomicAdd(&hist[c[u]], one);
-        if (c0 >= 0 && lane == 0) atomicAdd(&hist[c0], one * (unsigned)__popcll(same));
+        for (int u = 0; u < U; u++) {
+          const int i = i0 + u * TB + tid;
+          c[u] = i < nRW ? min(blocks(i) - low, top) : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          // counts cluster, and lanes that name the same bin are served one after the other: the lanes
+          // that agree with the group's first one are counted with one ballot and added once
+          const int c0 = __builtin_amdgcn_readfirstlane(c[u]);
+          const bool front = i0 + u * TB + wave * 64 < first;
+          const unsigned one = !ROWS && front ? 0x10001u : 1u;
+          const unsigned long long same = __ballot(c[u] == c0);
+          if (c[u] >= 0 && c[u] != c0) {
+            atomicAdd(&hist[c[u]], one);
+            if (ROWS && front) atomicAdd(&ahead[c[u]], 1u);
+          }
+          if (c0 >= 0 && lane == 0) {
+            atomicAdd(&hist[c0], one * (unsigned)__popcll(same));
+            if (ROWS && front) atomicAdd(&ahead[c0], (unsigned)__popcll(same));
+          }
+        }
       }
     }
     __syncthreads();
-    const bool wider = (hist[top] & 0xFFFFu) != 0u;  // windows left for the rounds to come
+    const bool wider = windows_in(top) != 0u;  // windows left for the rounds to come
     {  // where each bin's windows of this chunk start; thread t owns nBins / TB bins from the top
       const int per = nBins / TB;
       unsigned total = 0;
-      for (int k = 0; k < per; k++) total += hist[top - (tid * per + k)] & 0xFFFFu;
+      for (int k = 0; k < per; k++) total += windows_in(top - (tid * per + k));
       const unsigned incl = wave_inclusive_scan(total, lane);
       if (lane == 63) sBinTot[wave] = incl;
       __syncthreads();
@@ -1241,9 +1293,10 @@ __device__ __forceinline__ void order_chunk(const BlocksOf& blocks, int nRW, int
 #pragma unroll
       for (int k = 0; k < NW; k++) run += k < wave ? sBinTot[k] : 0u;
       for (int k = 0; k < per; k++) {
-        const uint32_t v = hist[top - (tid * per + k)];
-        hist[top - (tid * per + k)] = run + (v >> 16);
-        run += v & 0xFFFFu;
+        const int b = top - (tid * per + k);
+        const uint32_t in = windows_in(b);
+        ahead[b] = run + (ROWS ? ahead[b] : hist[b] >> 16);
+        run += in;
       }
     }
     const int bin = count - low;
@@ -1256,11 +1309,11 @@ __device__ __forceinline__ void order_chunk(const BlocksOf& blocks, int nRW, int
     for (int turn = 0; turn < NW; turn++) {  // ties go by window: one wave after the other
       __syncthreads();
       if (wave != turn) continue;
-      const unsigned at = binned ? hist[bin] : 0u;
+      const unsigned at = binned ? ahead[bin] : 0u;
       wave_lds_sync();
       if (binned) {
         sortedRowWindows[at + __popcll(peers & ((1ull << lane) - 1ull))] = first + tid;
-        if ((peers >> lane) == 1ull) hist[bin] = at + (unsigned)__popcll(peers);
+        if ((peers >> lane) == 1ull) ahead[bin] = at + (unsigned)__popcll(peers);
       }
     }
     if (!wider) return;
@@ -1352,28 +1405,47 @@ __device__ __forceinline__ int fin_passes(int maxC) {
   return (nBits + kFinDigitBits - 1) / kFinDigitBits;
 }
 
+// With rows (not null: a wave's chunk is 512 windows then): the histogram of every kOrderRowWindows
+// windows' counts as well, counts from kOrderRowBins - 1 on in the last bin, for order_chunk.
+constexpr int kOrderRowWindows = 1024, kOrderRowBins = 1024;
 __global__ __launch_bounds__(256) void finalize_partials_kernel(
     const int32_t* __restrict__ blockPartition, int nRW, int totalWaves,
-    unsigned* __restrict__ waveSum, int* __restrict__ waveMax) {
+    unsigned* __restrict__ waveSum, int* __restrict__ waveMax, uint16_t* __restrict__ rows) {
+  constexpr int ROWS = 2048 / kOrderRowWindows;  // of a workgroup
+  __shared__ uint32_t sHist[ROWS][kOrderRowBins];
   const int lane = threadIdx.x & 63;
-  const int gw = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (gw >= totalWaves) return;
-  const FinChunk c = fin_chunk(nRW, totalWaves, gw);
+  const int wave = threadIdx.x >> 6;
+  const int gw = blockIdx.x * 4 + wave;
+  const FinChunk c = fin_chunk(nRW, totalWaves, gw);  // empty if gw >= totalWaves
+  if (rows) {
+    for (int i = threadIdx.x; i < ROWS * kOrderRowBins; i += 256) sHist[0][i] = 0u;
+    __syncthreads();
+  }
   unsigned sum = 0;
   int mx = 0;
   for (int i = c.begin + lane; i < c.end; i += 64) {
     const int v = blockPartition[i];
     sum += (unsigned)v;
     mx = max(mx, v);
+    if (rows) atomicAdd(&sHist[wave * ROWS / 4][min(v, kOrderRowBins - 1)], 1u);
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     sum += __shfl_xor(sum, off);
     mx = max(mx, __shfl_xor(mx, off));
   }
-  if (lane == 0) {
+  if (lane == 0 && gw < totalWaves) {
     waveSum[gw] = sum;
     waveMax[gw] = mx;
+  }
+  if (rows) {
+    __syncthreads();
+    const int nRows = (nRW + kOrderRowWindows - 1) / kOrderRowWindows;
+    for (int r = 0; r < ROWS; r++) {
+      const int row = (int)blockIdx.x * ROWS + r;
+      for (int i = threadIdx.x; row < nRows && i < kOrderRowBins; i += 256)
+        rows[(size_t)row * kOrderRowBins + i] = (uint16_t)sHist[r][i];
+    }
   }
 }
 
@@ -1437,8 +1509,9 @@ __global__ __launch_bounds__(256) void finalize_scan_kernel(
     *nTcb = (long long)total;
     hdr->maxCount = maxC;
   }
-  fin_histogram(blockPartition, true, maxC, c, 0, lane, sBins[threadIdx.x >> 6],
-                hist + (size_t)gw * kFinBins);
+  if (hist)  // null: the order is not made here
+    fin_histogram(blockPartition, true, maxC, c, 0, lane, sBins[threadIdx.x >> 6],
+                  hist + (size_t)gw * kFinBins);
 }
 
 __global__ __launch_bounds__(256) void finalize_histogram_kernel(
@@ -1870,7 +1943,7 @@ template <int W>
 __device__ __forceinline__ void fill_short_window(
     int w, int base, int nb, const int32_t* __restrict__ rowPtr,
     const int32_t* __restrict__ colIdx, int N, const int32_t* __restrict__ edgeToColumn,
-    FillShortLds<W>& lds, int32_t* __restrict__ tcblockRowid, uint8_t* __restrict__ tcblocktileId,
+    const LongQueue& queue, FillShortLds<W>& lds, int32_t* __restrict__ tcblockRowid, uint8_t* __restrict__ tcblocktileId,
     int32_t* __restrict__ tcblockOffset, int32_t* __restrict__ sparseAToXidx,
     unsigned long long* __restrict__ bitmap) {
   constexpr int WPT = 16 * W / 64;
@@ -1883,6 +1956,7 @@ __device__ __forceinline__ void fill_short_window(
   const int eS = __builtin_amdgcn_readlane(rowStart, 0);
   const int n = __builtin_amdgcn_readlane(rowStart, 16) - eS;
   rowStart -= eS;
+  if (n > kBinsMax && queue.counts && lane == 0) queue.add(w, n);
   if (n == 0 || n > kBinsMax || nb > MAXB) return;  // long ones: fill_one_window
   if (nb < 1) return;  // no block to write: every column of the window lay outside [0, N)
   unsigned long long* bm = lds.bm;
@@ -2031,7 +2105,7 @@ template <int W>
 __global__ __launch_bounds__(64) void window_fill_short_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
     const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
-    int32_t* __restrict__ tcblockRowid, uint8_t* __restrict__ tcblocktileId,
+    LongQueue queue, int32_t* __restrict__ tcblockRowid, uint8_t* __restrict__ tcblocktileId,
     int32_t* __restrict__ tcblockOffset, int32_t* __restrict__ sparseAToXidx,
     unsigned long long* __restrict__ bitmap) {
   __shared__ FillShortLds<W> lds;
@@ -2039,7 +2113,7 @@ __global__ __launch_bounds__(64) void window_fill_short_kernel(
   const int base = __builtin_amdgcn_readfirstlane(rowWindowOffset[w]);
   const int nb = __builtin_amdgcn_readfirstlane(rowWindowOffset[w + 1]) - base;
   if (w == nRW - 1 && threadIdx.x == 0) tcblockOffset[base + nb] = E;
-  fill_short_window<W>(w, base, nb, rowPtr, colIdx, N, edgeToColumn, lds, tcblockRowid,
+  fill_short_window<W>(w, base, nb, rowPtr, colIdx, N, edgeToColumn, queue, lds, tcblockRowid,
                        tcblocktileId, tcblockOffset, sparseAToXidx, bitmap);
 }
 
@@ -2059,31 +2133,54 @@ __global__ __launch_bounds__(TB) void window_fill_kernel(
                                   sparseAToXidx, bitmap);
 }
 
-// The windows that window_fill_short_kernel leaves out, of more than minEdges and at most maxEdges
-// edges (find_windows). Two sizes: 256 threads and 320 TC blocks of LDS at a time for windows of up to
-// kFillMid edges (five workgroups per CU), 1024 threads and 1280 blocks for longer ones, which would
+// The windows that window_fill_short_kernel leaves out: those of its queue (the large ones if LARGE, else
+// the mid ones), or, where the caller has no memory for one, those of more than minEdges and at most
+// maxEdges edges (find_windows). Two sizes: 256 threads and 320 TC blocks of LDS at a time for windows of
+// up to kFillMid edges (five workgroups per CU), 1024 threads and 1280 blocks for longer ones, which would
 // otherwise each keep one small workgroup busy long after the others are done (31 700 edges:
 // 190 us).
-template <int W, int TB, int TC>
+// LARGE: the first orderGroups workgroups order the windows instead, TB of them each: the launch holds a
+// handful of windows, so most of the CUs would be idle, and nothing else of the call waits for the
+// order.
+template <int W, int TB, int TC, bool LARGE>
 __global__ __launch_bounds__(TB) void window_fill_long_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int E, int nRW,
     const int32_t* __restrict__ edgeToColumn, const int32_t* __restrict__ rowWindowOffset,
-    int minEdges, int maxEdges, int32_t* __restrict__ tcblockRowid,
+    LongQueue queue, int minEdges, int maxEdges, int orderGroups,
+    const int32_t* __restrict__ blockPartition, const uint16_t* __restrict__ orderRows,
+    int32_t* __restrict__ sortedRowWindows, int32_t* __restrict__ tcblockRowid,
     uint8_t* __restrict__ tcblocktileId, int32_t* __restrict__ tcblockOffset,
     int32_t* __restrict__ sparseAToXidx, unsigned long long* __restrict__ bitmap) {
   extern __shared__ __align__(16) unsigned char sRawDyn[];
   __shared__ int sList[TB];
   __shared__ int sListLen;
-  for (int64_t first = 0; first < nRW; first += (int64_t)TB * gridDim.x) {
-    const int found = find_windows(rowPtr, N, nRW, first, (int)gridDim.x, minEdges, maxEdges, sList,
-                                   &sListLen);
-    for (int k = 0; k < found; k++) {
-      __syncthreads();  // the window before this one has left the LDS arrays
-      const int w = sList[k], base = rowWindowOffset[w];
-      fill_one_window<W, TB, TC, TC>(w, base, rowWindowOffset[w + 1] - base, rowPtr, colIdx, N, E,
-                                     edgeToColumn, sRawDyn, tcblockRowid, tcblocktileId,
-                                     tcblockOffset, sparseAToXidx, bitmap);
+  if constexpr (LARGE) {
+    if ((int)blockIdx.x < orderGroups) {
+      static_assert(TB == kOrderRowWindows, "a row of the histogram per workgroup");
+      order_chunk<TB, true>([=](int i) { return blockPartition[i]; }, nRW, (int)blockIdx.x * TB,
+                            kOrderRowBins, sortedRowWindows, reinterpret_cast<uint32_t*>(sRawDyn),
+                            orderRows);
+      return;
     }
+  }
+  const int group = (int)blockIdx.x - (LARGE ? orderGroups : 0);
+  const int groups = (int)gridDim.x - (LARGE ? orderGroups : 0);
+  const auto fill = [&](int w) {
+    __syncthreads();  // the window before this one has left the LDS arrays
+    const int base = rowWindowOffset[w];
+    fill_one_window<W, TB, TC, TC>(w, base, rowWindowOffset[w + 1] - base, rowPtr, colIdx, N, E,
+                                   edgeToColumn, sRawDyn, tcblockRowid, tcblocktileId, tcblockOffset,
+                                   sparseAToXidx, bitmap);
+  };
+  if (queue.counts) {
+    const int listed = queue.size(LARGE);
+    for (int k = group; k < listed; k += groups) fill(queue.at(LARGE, k));
+    return;
+  }
+  for (int64_t first = 0; first < nRW; first += (int64_t)TB * groups) {
+    const int found = find_windows(rowPtr, N, nRW, first + group - (int)blockIdx.x, groups, minEdges,
+                                   maxEdges, sList, &sListLen);
+    for (int k = 0; k < found; k++) fill(sList[k]);
   }
 }
 
@@ -2149,6 +2246,7 @@ __global__ __launch_bounds__(kFillAllThreads) void window_fill_all_kernel(
     }
     if (w == nRW - 1 && lane == 0) tcblockOffset[base + nb] = E;
     fill_short_window<W>(w, base, nb, rowPtr, colIdx, N, edgeToColumn,
+                         LongQueue{nullptr, nullptr, 0, 0},
                          reinterpret_cast<FillShortLds<W>*>(sRawDyn)[wave], tcblockRowid,
                          tcblocktileId, tcblockOffset, sparseAToXidx, bitmap);
     return;
@@ -2713,7 +2811,7 @@ __global__ void set_tail_kernel(int32_t* tcblockOffset, long long nTcb, int E) {
   tcblockOffset[nTcb] = E;
 }
 
-__global__ void clear_error_kernel(int* error) { *error = 0; }
+__global__ void clear_header_kernel(WsHeader* hdr) { *hdr = WsHeader{}; }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -2746,9 +2844,11 @@ int allow_lds(KernelT kernel, size_t bytes) {
   return 0;
 }
 
-// Scan of the block counts and the window order, after the kernels that write blockPartition.
+// Scan of the block counts and (unless it is made beside the fill, see order_beside_fill) the window
+// order, after the kernels that write blockPartition.
 int enqueue_finalize(int N, int W, const int32_t* blockPartition, int32_t* rowWindowOffset,
-                     int32_t* sortedRowWindows, char* ws, long long* nTcb, hipStream_t stream) {
+                     int32_t* sortedRowWindows, bool order, char* ws, long long* nTcb,
+                     hipStream_t stream) {
   const int nRW = (N + kWinRows - 1) / kWinRows;
   WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
   const size_t seg = align256((size_t)nRW * sizeof(int32_t));
@@ -2770,9 +2870,12 @@ int enqueue_finalize(int N, int W, const int32_t* blockPartition, int32_t* rowWi
   unsigned* hist = waveSum + 2 * (size_t)finWaves;
   const dim3 grid((unsigned)((finWaves + 3) / 4)), block(256);
   hipLaunchKernelGGL(finalize_partials_kernel, grid, block, 0, stream, blockPartition, nRW,
-                     finWaves, waveSum, waveMax);
+                     finWaves, waveSum, waveMax,
+                     order ? nullptr : reinterpret_cast<uint16_t*>(keysB));
   hipLaunchKernelGGL(finalize_scan_kernel, grid, block, 0, stream, blockPartition, nRW, finWaves,
-                     waveSum, waveMax, rowWindowOffset, hist, hdr, nTcb);
+                     waveSum, waveMax, rowWindowOffset, order ? hist : nullptr, hdr, nTcb);
+  F3S_HIP_CHECK(hipGetLastError());
+  if (!order) return 0;
   // a window holds at most ceil(N / W) blocks: that bounds the passes that can be needed
   int maxBits = 0;
   while ((((int64_t)N + W - 1) / W >> maxBits) != 0) maxBits++;
@@ -2808,10 +2911,21 @@ unsigned all_long_groups(int nRW, int E) {
   return long_grid(nRW, E, kBinsMax, E / nRW <= kBinsMax / 2 ? 512 : kFinSingleMax);
 }
 
-// Enqueues the kernels that rank the windows' columns and count their TC blocks.
+// Above kFinSingleMax windows the order is made in the last launch of the fill, where most CUs are idle:
+// nRW / 1024 workgroups add up the rows of a histogram that the scan's first kernel leaves. A radix sort
+// between the phases is five launches; a call's time in us with it and without: 17 000 windows 153 ->
+// 117, 69 000 250 -> 212, 153 000 815 -> 763, 262 000 625 -> 573, 500 000 2140 -> 2077. Beyond, the
+// workgroups' readings (nRW^2 / 512 bytes) grow faster than the sort.
+constexpr int kOrderBesideMax = 524288;
+bool order_beside_fill(int nRW, int64_t E) {
+  return nRW > kFinSingleMax && nRW <= kOrderBesideMax && !long_windows(nRW, E);
+}
+
+// Enqueues the kernels that rank the windows' columns and count their TC blocks. sortedRowWindows holds
+// the lists of long windows until the order is written.
 template <int W>
-int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
-                 int32_t* blockPartition, int32_t* edgeToColumn, int32_t* edgeToRow, int* error,
+int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, char* ws,
+                 int32_t* sortedRowWindows, int32_t* blockPartition, int32_t* edgeToColumn, int32_t* edgeToRow, int* error,
                  hipStream_t stream) {
   const int nRW = (N + kWinRows - 1) / kWinRows;
   if (nRW == 0) return 0;
@@ -2835,38 +2949,44 @@ int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
     return 0;
   }
   int shortMax = kBinsMax;
+  WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
+  LongQueue queue = {nullptr, nullptr, 0, 0};
+  if (!long_windows(nRW, E)) {
+    queue = {&hdr->rank, sortedRowWindows, nRW, nPasses >= 2 ? kMedMax : 0};
+    hipLaunchKernelGGL(clear_header_kernel, dim3(1), dim3(1), 0, stream, hdr);
+  }
   if (colBits <= 22) {
     hipLaunchKernelGGL(window_rank_bins_kernel<W>, dim3(nRW), dim3(64), 0, stream, rowPtr,
-                       colIdx, N, colBits, blockPartition, edgeToColumn, edgeToRow, error);
+                       colIdx, N, colBits, queue, blockPartition, edgeToColumn, edgeToRow, error);
   } else {
     shortMax = kSortMax;
-    hipLaunchKernelGGL(window_rank_small_kernel<W>, dim3(nRW), dim3(64), 0, stream,
-                       rowPtr, colIdx, N, nRW, blockPartition, edgeToColumn, edgeToRow, error);
+    hipLaunchKernelGGL(window_rank_small_kernel<W>, dim3(nRW), dim3(64), 0, stream, rowPtr, colIdx, N,
+                       nRW, queue, blockPartition, edgeToColumn, edgeToRow, error);
   }
   F3S_HIP_CHECK(hipGetLastError());
   if (long_windows(nRW, E)) {
     hipLaunchKernelGGL((window_rank_kernel<W, 512, false>), dim3(nRW), dim3(512), lds, stream,
-                       rowPtr, colIdx, N, nRW, range, nPasses, shortMax, blockPartition,
+                       rowPtr, colIdx, N, nRW, range, nPasses, shortMax, queue, blockPartition,
                        edgeToColumn, edgeToRow, error);
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
   }
-  // The longer ones, which each kernel looks for. On a graph that needs several bitset passes,
+  // The longer ones, from the lists. On a graph that needs several bitset passes,
   // windows of a few thousand edges are sorted instead of walking every pass: up to kMedMax edges
   // with four workgroups per CU, then the few windows up to kLargeMax with one.
   int minEdges = shortMax;
   if (nPasses >= 2) {
-    auto med = window_rank_sort_kernel<W, kMedItems, kMedThreads>;
-    auto large = window_rank_sort_kernel<W, kLargeItems, kLargeThreads>;
+    auto med = window_rank_sort_kernel<W, kMedItems, kMedThreads, false>;
+    auto large = window_rank_sort_kernel<W, kLargeItems, kLargeThreads, true>;
     constexpr size_t medLds = rank_sort_lds<kMedItems, kMedThreads>();
     constexpr size_t largeLds = rank_sort_lds<kLargeItems, kLargeThreads>();
     if (int rc = allow_lds(med, medLds)) return rc;
     if (int rc = allow_lds(large, largeLds)) return rc;
     hipLaunchKernelGGL(med, dim3(long_grid(nRW, E, minEdges, 8192)), dim3(kMedThreads), medLds,
-                       stream, rowPtr, colIdx, N, nRW, colBits, minEdges, blockPartition,
-                       edgeToColumn, edgeToRow, error);
+                       stream, rowPtr, colIdx, N, nRW, colBits, queue, blockPartition, edgeToColumn,
+                       edgeToRow, error);
     hipLaunchKernelGGL(large, dim3(long_grid(nRW, E, kMedMax, 1024)), dim3(kLargeThreads),
-                       largeLds, stream, rowPtr, colIdx, N, nRW, colBits, kMedMax, blockPartition,
+                       largeLds, stream, rowPtr, colIdx, N, nRW, colBits, queue, blockPartition,
                        edgeToColumn, edgeToRow, error);
     F3S_HIP_CHECK(hipGetLastError());
     minEdges = kLargeMax;
@@ -2874,31 +2994,31 @@ int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
   // sixteen waves per window: what counts is how soon the longest one is done (169k-node R-MAT graph,
   // windows of up to 12 500 edges: 31 us with four)
   hipLaunchKernelGGL((window_rank_kernel<W, 1024, true>), dim3(long_grid(nRW, E, minEdges, 512)),
-                     dim3(1024), lds, stream, rowPtr, colIdx, N, nRW, range, nPasses, minEdges,
+                     dim3(1024), lds, stream, rowPtr, colIdx, N, nRW, range, nPasses, minEdges, queue,
                      blockPartition, edgeToColumn, edgeToRow, error);
   F3S_HIP_CHECK(hipGetLastError());
   return 0;
 }
-int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W,
-                 int32_t* blockPartition, int32_t* edgeToColumn, int32_t* edgeToRow, int* error,
-                 hipStream_t stream) {
-  return W == 16 ? enqueue_rank<16>(rowPtr, colIdx, N, E, blockPartition, edgeToColumn, edgeToRow,
-                                    error, stream)
-                 : enqueue_rank<8>(rowPtr, colIdx, N, E, blockPartition, edgeToColumn, edgeToRow,
-                                   error, stream);
+int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W, char* ws,
+                 int32_t* sortedRowWindows, int32_t* blockPartition, int32_t* edgeToColumn,
+                 int32_t* edgeToRow, int* error, hipStream_t stream) {
+  return W == 16 ? enqueue_rank<16>(rowPtr, colIdx, N, E, ws, sortedRowWindows, blockPartition,
+                                    edgeToColumn, edgeToRow, error, stream)
+                 : enqueue_rank<8>(rowPtr, colIdx, N, E, ws, sortedRowWindows, blockPartition,
+                                   edgeToColumn, edgeToRow, error, stream);
 }
 
-// Enqueues every kernel of phase 1 on `stream`; `ws` is device scratch of
-// preprocess_workspace_bytes(N, E) bytes.
+// Enqueues every kernel of phase 1 on `stream`, the window order only if `order`; `ws` is device scratch
+// of preprocess_workspace_bytes(N, E) bytes.
 int enqueue_count(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W,
                   int32_t* blockPartition, int32_t* edgeToColumn, int32_t* edgeToRow,
-                  int32_t* rowWindowOffset, int32_t* sortedRowWindows, char* ws,
+                  int32_t* rowWindowOffset, int32_t* sortedRowWindows, bool order, char* ws,
                   const ResultPtr& result, hipStream_t stream) {
-  if (int rc = enqueue_rank(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
-                            result.error, stream))
+  if (int rc = enqueue_rank(rowPtr, colIdx, N, E, W, ws, sortedRowWindows, blockPartition,
+                            edgeToColumn, edgeToRow, result.error, stream))
     return rc;
-  return enqueue_finalize(N, W, blockPartition, rowWindowOffset, sortedRowWindows, ws, result.nTcb,
-                          stream);
+  return enqueue_finalize(N, W, blockPartition, rowWindowOffset, sortedRowWindows, order, ws,
+                          result.nTcb, stream);
 }
 
 // Pinned host memory for the results of calls that wait for the device: a slot per call in progress,
@@ -2972,7 +3092,7 @@ int launch_preprocess_count(const int32_t* rowPtr, const int32_t* colIdx, int N,
   HostResultLease result;
   if (int rc = result.take()) return rc;
   int rc = enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
-                         rowWindowOffset, sortedRowWindows, static_cast<char*>(workspace),
+                         rowWindowOffset, sortedRowWindows, true, static_cast<char*>(workspace),
                          result.pointers(), stream);
   // also after a failed launch: the slot must not be written to any more when it is given back
   const hipError_t done = hipStreamSynchronize(stream);
@@ -3039,19 +3159,19 @@ int launch_preprocess_count_static(const int32_t* rowPtr, const int32_t* colIdx,
   F3S_HIP_CHECK(hipGetLastError());
   // the error flag is the low half of the second value
   return enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
-                       rowWindowOffset, sortedRowWindows, ws,
+                       rowWindowOffset, sortedRowWindows, true, ws,
                        {result, reinterpret_cast<int*>(result + 1)}, stream);
 }
 
 namespace {
 
-// Enqueues phase 2. With sortedRowWindows (not null: at most kFinSingleMax windows, and mostly short
-// ones) the window order is written too, from blockPartition; with nTcb (not null: at most
-// kSelfScanMax of them) rowWindowOffset and the total as well.
+// Enqueues phase 2. With sortedRowWindows (not null: order_beside_fill) the window order is written
+// too, from blockPartition; with nTcb (not null: at most kSelfScanMax windows) rowWindowOffset and the
+// total as well. ws: the workspace of phase 1, or null (the long windows are then looked for).
 template <int W>
 int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
                  const int32_t* edgeToColumn, int32_t* rowWindowOffset,
-                 const int32_t* blockPartition, int32_t* sortedRowWindows, long long* nTcb,
+                 const int32_t* blockPartition, int32_t* sortedRowWindows, long long* nTcb, char* ws,
                  int32_t* tcblockRowid, uint8_t* tcblocktileId, int32_t* tcblockOffset,
                  int32_t* sparseAToXidx, uint64_t* bitmap, hipStream_t stream) {
   const int nRW = (N + kWinRows - 1) / kWinRows;
@@ -3083,42 +3203,52 @@ int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
   }
-  hipLaunchKernelGGL((window_fill_short_kernel<W>), dim3(nRW), dim3(64), 0, stream, rowPtr, colIdx, N,
-                     E, nRW, edgeToColumn, rowWindowOffset, tcblockRowid, tcblocktileId,
-                     tcblockOffset, sparseAToXidx, bm);
-  F3S_HIP_CHECK(hipGetLastError());
   // few long windows (at most kFillFewLong, and as windows have at most half of kBinsMax edges on
   // average, commonly far fewer): the large workgroups take all of them, which saves a launch
-  int minEdges = kBinsMax;
   const bool few = E / kBinsMax <= kFillFewLong && E / nRW <= kBinsMax / 2;
+  LongQueue queue = {nullptr, nullptr, 0, 0};
+  if (ws)  // phase 1 has cleared the counts and is done with the keys behind the header
+    queue = {&reinterpret_cast<WsHeader*>(ws)->fill, reinterpret_cast<int32_t*>(ws + kWsHeaderBytes), nRW,
+             few ? 0 : kFillMid};
+  hipLaunchKernelGGL((window_fill_short_kernel<W>), dim3(nRW), dim3(64), 0, stream, rowPtr, colIdx, N,
+                     E, nRW, edgeToColumn, rowWindowOffset, queue, tcblockRowid, tcblocktileId,
+                     tcblockOffset, sparseAToXidx, bm);
+  F3S_HIP_CHECK(hipGetLastError());
+  int minEdges = kBinsMax;
   if (!few) {
-    auto mid = window_fill_long_kernel<W, 256, kFillChunkMid>;
+    auto mid = window_fill_long_kernel<W, 256, kFillChunkMid, false>;
     constexpr size_t lds = fill_lds_bytes<W>(kFillChunkMid, kFillChunkMid);
     hipLaunchKernelGGL(mid, dim3(long_grid(nRW, E, minEdges, 8192)), dim3(256), lds, stream, rowPtr,
-                       colIdx, N, E, nRW, edgeToColumn, rowWindowOffset, minEdges, kFillMid,
-                       tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bm);
+                       colIdx, N, E, nRW, edgeToColumn, rowWindowOffset, queue, minEdges, kFillMid, 0,
+                       nullptr, nullptr, nullptr, tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bm);
     F3S_HIP_CHECK(hipGetLastError());
     minEdges = kFillMid;
   }
-  auto kernel = window_fill_long_kernel<W, 1024, kFillChunkLong>;
+  auto kernel = window_fill_long_kernel<W, 1024, kFillChunkLong, true>;
   constexpr size_t lds = fill_lds_bytes<W>(kFillChunkLong, kFillChunkLong);
+  static_assert(lds >= 2 * kOrderRowBins * sizeof(uint32_t), "order_chunk's arrays");
+  const size_t seg = align256((size_t)nRW * sizeof(int32_t));
   if (int rc = allow_lds(kernel, lds)) return rc;
-  hipLaunchKernelGGL(kernel, dim3(long_grid(nRW, E, minEdges, 255)), dim3(1024), lds, stream, rowPtr,
-                     colIdx, N, E, nRW, edgeToColumn, rowWindowOffset, minEdges, 0x7FFFFFFF,
-                     tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bm);
+  const unsigned orderGroups =
+      sortedRowWindows ? (unsigned)((nRW + kOrderRowWindows - 1) / kOrderRowWindows) : 0;
+  hipLaunchKernelGGL(kernel, dim3(orderGroups + long_grid(nRW, E, minEdges, 255)), dim3(1024), lds,
+                     stream, rowPtr, colIdx, N, E, nRW, edgeToColumn, rowWindowOffset, queue, minEdges,
+                     0x7FFFFFFF, (int)orderGroups, blockPartition,
+                     reinterpret_cast<const uint16_t*>(ws + kWsHeaderBytes + seg), sortedRowWindows, tcblockRowid,
+                     tcblocktileId, tcblockOffset, sparseAToXidx, bm);
   F3S_HIP_CHECK(hipGetLastError());
   return 0;
 }
 int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, int W,
                  const int32_t* edgeToColumn, int32_t* rowWindowOffset,
-                 const int32_t* blockPartition, int32_t* sortedRowWindows, long long* nTcb,
+                 const int32_t* blockPartition, int32_t* sortedRowWindows, long long* nTcb, char* ws,
                  int32_t* tcblockRowid, uint8_t* tcblocktileId, int32_t* tcblockOffset,
                  int32_t* sparseAToXidx, uint64_t* bitmap, hipStream_t stream) {
   return W == 16 ? enqueue_fill<16>(rowPtr, colIdx, N, E, edgeToColumn, rowWindowOffset,
-                                    blockPartition, sortedRowWindows, nTcb, tcblockRowid,
+                                    blockPartition, sortedRowWindows, nTcb, ws, tcblockRowid,
                                     tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream)
                  : enqueue_fill<8>(rowPtr, colIdx, N, E, edgeToColumn, rowWindowOffset,
-                                   blockPartition, sortedRowWindows, nTcb, tcblockRowid,
+                                   blockPartition, sortedRowWindows, nTcb, ws, tcblockRowid,
                                    tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
 }
 
@@ -3140,7 +3270,8 @@ int launch_preprocess_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, 
   }
   // the offsets are only read: without nTcb nothing writes them
   return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, const_cast<int32_t*>(rowWindowOffset),
-                      nullptr, nullptr, nullptr, tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
+                      nullptr, nullptr, nullptr, nullptr, tcblockRowid, tcblocktileId, tcblockOffset,
+                      sparseAToXidx, bitmap, stream);
 }
 
 int launch_window_order(const int32_t* rowWindowOffset, int nRW, int32_t* order,
@@ -3185,7 +3316,7 @@ int enqueue_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int 
     chunkBytes &= ~255;
     const size_t ldsCount = (size_t)(range / 32) * 4;
     const size_t ldsFill = (size_t)bitsetBytes + chunkBytes;
-    hipLaunchKernelGGL(clear_error_kernel, dim3(1), dim3(1), 0, stream, &hdr->error);
+    hipLaunchKernelGGL(clear_header_kernel, dim3(1), dim3(1), 0, stream, hdr);
 #define F3S_ONECALL(WW)                                                                        \
   do {                                                                                         \
     auto rankFill = window_rank_fill_kernel<WW, kRankFillThreads>;                             \
@@ -3193,8 +3324,8 @@ int enqueue_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int 
     hipLaunchKernelGGL((window_count_kernel<WW, 512>), dim3(nRW), dim3(512), ldsCount, stream, \
                        rowPtr, colIdx, N, range, blockPartition, hdr, result.error);           \
     F3S_HIP_CHECK(hipGetLastError());                                                          \
-    if (int rc = enqueue_finalize(N, W, blockPartition, rowWindowOffset, sortedRowWindows, ws, \
-                                  result.nTcb, stream))                                        \
+    if (int rc = enqueue_finalize(N, W, blockPartition, rowWindowOffset, sortedRowWindows,     \
+                                  true, ws, result.nTcb, stream))                              \
       return rc;                                                                               \
     hipLaunchKernelGGL(rankFill, dim3(nRW), dim3(kRankFillThreads), ldsFill, stream, rowPtr,   \
                        colIdx, N, E, range, chunkBytes, rowWindowOffset, sortedRowWindows,     \
@@ -3210,8 +3341,8 @@ int enqueue_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int 
   // At most the scan stands between the phases; the order is made beside the fill (as its own launch in
   // between it took 23 us of the 219 of a call on 169k nodes).
   if (nRW > 0 && one_launch(nRW, E)) {
-    if (int rc = enqueue_rank(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
-                              result.error, stream))
+    if (int rc = enqueue_rank(rowPtr, colIdx, N, E, W, ws, sortedRowWindows, blockPartition,
+                              edgeToColumn, edgeToRow, result.error, stream))
       return rc;
     const bool self = nRW <= kSelfScanMax;
     if (!self) {
@@ -3220,19 +3351,21 @@ int enqueue_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int 
       F3S_HIP_CHECK(hipGetLastError());
     }
     return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, blockPartition,
-                        sortedRowWindows, self ? result.nTcb : nullptr, tcblockRowid,
+                        sortedRowWindows, self ? result.nTcb : nullptr, ws, tcblockRowid,
                         tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
   }
+  const bool beside = order_beside_fill(nRW, E);
   if (int rc = enqueue_count(rowPtr, colIdx, N, E, W, blockPartition, edgeToColumn, edgeToRow,
-                             rowWindowOffset, sortedRowWindows, ws, result, stream))
+                             rowWindowOffset, sortedRowWindows, !beside, ws, result, stream))
     return rc;
   if (nRW == 0) {
     hipLaunchKernelGGL(set_tail_kernel, dim3(1), dim3(1), 0, stream, tcblockOffset, 0ll, E);
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
   }
-  return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, nullptr, nullptr,
-                      nullptr, tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bitmap, stream);
+  return enqueue_fill(rowPtr, colIdx, N, E, W, edgeToColumn, rowWindowOffset, blockPartition,
+                      beside ? sortedRowWindows : nullptr, nullptr, ws, tcblockRowid, tcblocktileId,
+                      tcblockOffset, sparseAToXidx, bitmap, stream);
 }
 
 }  // namespace

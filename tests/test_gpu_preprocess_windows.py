@@ -146,6 +146,37 @@ def test_long_windows_ids_and_prefixes(oracle_mod, W):
                           want["tcbBitMap"])
 
 
+# Above 16 384 windows the order of the one call comes from rows of a histogram, one per 1024 windows (up to
+# 524 288 of them), whose last bin is 1023 blocks and more; long windows go through lists, mid and large
+# ones (one bitset pass: all of them large): windows on both sides of each, ties across rows
+@pytest.mark.parametrize("nRW", [16_385, 17_407, 17_408, 17_409, 18_432, 24_576, 24_577, 40_000,
+                                 524_288, 524_289])
+def test_order_beside_the_fill(oracle_mod, nRW):
+    from fused3s_amd import capi
+    print("case order beside the fill nRW=%d" % nRW, flush=True)
+    rng = np.random.default_rng(nRW)
+    N, W = 16 * nRW - 3, 8
+    degree = np.zeros(N, np.int64)
+    degree[rng.choice(N, 50_000, replace=False)] = rng.integers(1, 40, 50_000)
+    wide = np.array([1022, 1023, 1024, 1024, 2045, 2046, 2047, 120, 121, 512, 513]) * 8
+    at = np.concatenate([[0, 1023, 1024, nRW - 2], rng.choice(nRW - 2, len(wide) - 4, replace=False)])
+    for w, n in zip(at, wide):
+        degree[16 * w:16 * w + 16] = 0
+        degree[16 * w] = n
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(degree)
+    colIdx = rng.integers(0, N, int(rowPtr[-1])).astype(np.int32)
+    for w, n in zip(at, wide):
+        if degree[16 * w] == n:
+            colIdx[rowPtr[16 * w]:rowPtr[16 * w + 1]] = np.sort(rng.choice(N, int(n), replace=False))
+    want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, W)
+    rp, ci = torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda()
+    for two_phase in (False, True):
+        got = capi.preprocess(rp, ci, N, 16, W, two_phase=two_phase)
+        for k in KEYS:
+            assert np.array_equal(got[k].cpu().numpy(), want[k]), (k, two_phase)
+
+
 # The order's histogram has 4096 bins: windows of 4095 blocks and more take further rounds. Counts at
 # the rounds' edges, ties of more than a wave, rounds that no window falls into, and one window that
 # spans every node
