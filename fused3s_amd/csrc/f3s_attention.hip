@@ -52,6 +52,17 @@ int attention_uses_workspace(int N, int64_t nTcb, int d, int dtype) {
   return nRW >= 2048 && nTcb >= 64 * nRW;
 }
 
+// Single-head calls on small structures of narrow rows are over before their slices pay, with or without a
+// workspace (window against sliced, us): d = 64: 50 000 nodes, 76 blocks a window 63 against 83; 70 000,
+// 93: 106 against 119; 100 000, 66: 120 against 145; 50 000, 178: 118 against 121; from 750 000 blocks
+// sliced is faster (100 000, 121: 219 against 193). d = 32: 50 000, 76: 47 against 54; 40 000, 100: 48
+// against 54; 100 000, 66: 99 against 92. Of several heads even small ones pay (40 000, 73, 4 x 32: 152
+// against 126).
+bool windows_suffice(int64_t nTcb, int d) {
+  if (getenv("F3S_SCHEDULE") || getenv("F3S_SLICE_PHASES")) return false;  // asked for
+  return nTcb < (d <= 32 ? 260000 : d <= 64 ? 450000 : 0);
+}
+
 int launch_attention(const int32_t* rowWindowOffset, const int32_t* windowOrder,
                      const int32_t* sparseAToXidx, const uint64_t* bitmap, int N, int64_t nTcb,
                      int d, int dtype, const void* Q, const void* K, const void* V,
@@ -71,7 +82,8 @@ int launch_attention(const int32_t* rowWindowOffset, const int32_t* windowOrder,
   if (gather_needs_wide_offsets(N, (int64_t)d * 2, false))
     return launch_window_wide(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q,
                               K, V, scaleLog2, applySoftmax, out, cuTimer, 0, d, d, nTcb, stream);
-  if (workspace && !cuTimer && attention_uses_workspace(N, nTcb, d, dtype))
+  if (workspace && !cuTimer && attention_uses_workspace(N, nTcb, d, dtype) &&
+      !windows_suffice(nTcb, d))
     return launch_attention_sliced(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, 0, d, d, prepared ? 2 : 0, stream);

@@ -34,8 +34,7 @@ namespace {
 using pipe::float4v;
 using pipe::uniform;
 
-constexpr int kXcds = 8;
-constexpr int kMaxPhases = 16;  // slices that an XCD works through one after the other (choose_split)
+constexpr int kMaxPhases = 16;  // slices that an XCD works through one after the other at most
 constexpr int kUnitWaves = 4;  // waves (= units) per workgroup; they do not cooperate
 
 // Stages of a wave's LDS ring and waves per SIMD the register allocator is held to.
@@ -120,13 +119,8 @@ struct XcdSplit {
 // rows, so its share of K + V shrinks without cutting windows into more units. The part stays at
 // least a line of 128 bytes.
 inline XcdSplit split_heads(int d, int heads) {
-  XcdSplit s = {1, 1, 1, kXcds, heads, 1};
-  while (s.headGroups < kXcds && s.headsPerGroup % 2 == 0 && s.headsPerGroup / 2 * d * 2 >= 128) {
-    s.headGroups *= 2;
-    s.windowGroups /= 2;
-    s.headsPerGroup /= 2;
-  }
-  return s;
+  const int groups = head_groups(d, heads);
+  return {1, 1, groups, kXcds / groups, heads / groups, 1};
 }
 
 // probe builds: the partials through the caches instead of past them
@@ -587,42 +581,60 @@ int allow_lds(KernelT kernel, size_t bytes) {
   return 0;
 }
 
-// How a column-sliced call's units are dealt to the XCDs: head groups (split_heads), then column
-// slices until a slice's K + V rows (of the group's heads) are at most 8 MiB: twice an XCD's L2,
-// which already catches 4 of 5 accesses on the 233k-node benchmark graph, while more and shorter
-// units cost more than their higher hit rate returns (measured 1.54 / 1.69 / 1.86 ms with 8 / 16 /
-// 24 slices there). XCDs left over share the windows.
-// No more than kMaxPhases slices are worked through one after the other: from 128 MiB of K + V per
-// group of heads on (524 000 nodes at d = 64, 262 000 at 128, 131 000 at 256) slices get wider than
-// 8 MiB instead. Every slice more is a partial result more per window, to be written and merged, and on
-// large graphs that outweighs the L2 hits. With the cap against without, in ms (and GB of workspace):
-// 200 000 nodes, 141 blocks a window, d = 256: 3.05 (3.1) against 3.80 (4.8); 600 000, 290, d = 128:
-// 6.93 (4.7) against 8.46 (10.8); 1 000 000, 99, d = 128: 6.98 (7.8) against 16.7 (30); 1 200 000, 99,
-// d = 64: 4.38 against 7.68; 300 000, 555, 2 x 128: 9.14 against 9.45; 400 000, 747, d = 128: 8.39
-// against 8.75; 262 144, 899: alike. A cap of 8 is slower on long windows (the 747: 9.71) and faster on
-// short ones (the 99: 5.79).
+// Slices of a column-sliced call: how many bytes of K + V (of a group's heads) a slice should have at
+// most, and what a window's blocks have to be worth for another slice, in parts of a hundred. A slice more
+// brings a slice's rows closer to the size of an XCD's L2, and costs every window a partial result more
+// (64 d + 128 bytes, written and merged) and a unit's start. From sweeps of 2 to 16 slices over power-law
+// graphs of 40 000 to 200 000 nodes and 60 to 430 blocks a window, fp16, 1 to 8 heads:
+// - the best number grows with the square root of the blocks per window (d = 128, K + V of 102 MB: 4, 6
+//   and 8 slices at 67, 123 and 276 blocks);
+// - short rows want smaller slices (d = 32: 8 x 32, 270 blocks: 2.37 ms with 8 MiB, 1.96 ms with 2 MiB), long
+//   ones, whose kernels run one wave per SIMD and spend more on arithmetic, larger ones (d = 192, 154 MB,
+//   67 blocks: 2.02 ms with 16 slices, 1.01 ms with 2).
+// With the blocks per window left out (8 MiB slices, at most sixteen) against now, in us: 100 000 nodes,
+// 66 blocks, d = 192 733 -> 493; 200 000, 67: d = 128 857 -> 644, d = 256 2365 -> 1376; 200 000, 123, d = 256
+// 2842 -> 2161; 200 000, 276, d = 192 3986 -> 3137; 100 000, 270, 8 x 32 2369 -> 1937; 200 000, 141, 4 x 128
+// 5267 -> 4353; 1 000 000, 99, d = 128 6993 -> 5658; 233 000, 450, d = 64 1481 -> 1478.
+constexpr int64_t slice_bytes(int d) {
+  return (d <= 32 ? 3 : d <= 128 ? 8 : d < 256 ? 25 : 20) * (int64_t)1024 * 1024;
+}
+constexpr int64_t slice_weight(int d) { return d <= 32 ? 55 : d <= 128 ? 45 : d < 256 ? 30 : 40; }
+
+// How the units are dealt to the XCDs: head groups (split_heads), then column slices; XCDs left over share
+// the windows. nTcb < 0: the most slices that any number of blocks asks for (the size of the workspace),
+// 8 MiB each above d = 32.
 // F3S_SLICE_PHASES = P in the environment forces 8 P slices of all heads.
-XcdSplit choose_split(int N, int d, int heads) {
+XcdSplit choose_split(int N, int d, int heads, int64_t nTcb) {
   const char* e = getenv("F3S_SLICE_PHASES");  // read per call: tests walk through the phases
   const int forced = e ? atoi(e) : 0;
   if (forced > 0) return {forced > kMaxPhases ? kMaxPhases : forced, kXcds, 1, 1, heads, 1};
   XcdSplit s = split_heads(d, heads);
-  constexpr int64_t kSliceBytes = (int64_t)8 * 1024 * 1024;
+  const int64_t nRW = (N + kWinRows - 1) / kWinRows;
   const int64_t bytes = (int64_t)N * d * s.headsPerGroup * 4;  // K + V of a group's heads
-  int64_t need = (bytes + kSliceBytes - 1) / kSliceBytes;
+  const int64_t most = nTcb < 0 && d > 32 ? slice_bytes(64) : slice_bytes(d);
+  int64_t need = (bytes + most - 1) / most;
+  if (nTcb >= 0 && nRW > 0) {  // (weight / 100) sqrt(blocks per window), rounded
+    int64_t worth = 2;
+    while ((2 * worth + 1) * (2 * worth + 1) * 2500 * nRW <= slice_weight(d) * slice_weight(d) * nTcb)
+      worth++;
+    if (need > worth) need = worth;
+  }
   if (need < 2) need = 2;  // one unit per window would be the windows themselves
   // Slices one after the other keep all XCDs on the same columns at a time, which the memory side
   // serves faster (100k nodes, 4 x 128: 1.77 -> 1.67 ms; 60k nodes, 4 x 64: 0.87 -> 0.82 ms), as
   // long as a phase has units for two rounds of waves; with fewer the second phase's heavy windows
   // start when the first phase's light ones should fill the end (60k nodes, d = 32: 188 -> 206 us).
+  // The slices at a time are a power of two, the nearest one rather than the next (50k nodes, d = 96:
+  // 123 us with 4 slices, 146 with 8).
   const int64_t waves = 32 * 4 * unit_waves_per_simd(d, true);  // of one XCD
-  if (s.units((N + kWinRows - 1) / kWinRows) < 2 * waves) {
-    while (s.windowGroups > 1 && s.sliceGroups < need) {
+  if (s.units(nRW) < 2 * waves) {
+    while (s.windowGroups > 1 && (nTcb < 0 ? s.sliceGroups < need : 3 * s.sliceGroups <= 2 * need)) {
       s.sliceGroups *= 2;
       s.windowGroups /= 2;
     }
   }
-  const int64_t phases = (need + s.sliceGroups - 1) / s.sliceGroups;
+  int64_t phases = (need + (nTcb < 0 ? s.sliceGroups - 1 : s.sliceGroups / 2)) / s.sliceGroups;
+  if (phases < 1) phases = 1;
   s.phases = phases > kMaxPhases ? kMaxPhases : (int)phases;
   return s;
 }
@@ -650,11 +662,11 @@ struct SlicedLayout {
   size_t tickets, sliceStart, partial, total;
   size_t padded;  // 0, or where the copies of K and V with 256-byte rows start (single head, d = 64)
 };
-// nHeads = 0: the single-head layout
-SlicedLayout sliced_layout(int N, int d, int nHeads) {
+// nHeads = 0: the single-head layout. nTcb < 0: the largest that any structure of N nodes asks for.
+SlicedLayout sliced_layout(int N, int d, int nHeads, int64_t nTcb) {
   const int heads = nHeads > 0 ? nHeads : 1;
   SlicedLayout L;
-  L.split = choose_split(N, d, heads);
+  L.split = choose_split(N, d, heads, nTcb);
   L.S = L.split.slices();
   const size_t nRW = (size_t)(N + kWinRows - 1) / kWinRows;
   L.tickets = 256;
@@ -794,7 +806,7 @@ int launch_sliced_d(const int32_t* rwo, const int32_t* order, const int32_t* ato
 }  // namespace
 
 size_t attention_sliced_workspace_bytes(int N, int d, int nHeads) {
-  return sliced_layout(N, d, nHeads).total;
+  return sliced_layout(N, d, nHeads, -1).total;
 }
 
 // mode 0 / 2: an attention call (2: on a prepared workspace); mode 1: f3s_attention_prepare
@@ -807,7 +819,7 @@ int launch_attention_sliced(const int32_t* rowWindowOffset, const int32_t* windo
                             int mode, hipStream_t stream) {
   if (!head_dim_supported(d))
     return fail(-2, "f3s_attention: head dim %d unsupported (a multiple of 32 up to 256)", d);
-  const SlicedLayout L = sliced_layout(N, d, nHeads);
+  const SlicedLayout L = sliced_layout(N, d, nHeads, nTcb);
   if (wsBytes < L.total)
     return fail(-2, "f3s_attention: workspace %zu B < required %zu B", wsBytes, L.total);
   char* ws = static_cast<char*>(workspace);

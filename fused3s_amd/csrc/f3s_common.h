@@ -23,6 +23,19 @@ inline int gather_needs_wide_offsets(int64_t N, int64_t pitchBytes, bool pitched
   return 0;
 }
 
+constexpr int kXcds = 8;
+
+// Groups of heads that the XCDs are dealt: as many as leave a group at least a line of 128 bytes of a
+// row, a power of two up to the number of XCDs.
+inline int head_groups(int d, int heads) {
+  int groups = 1, perGroup = heads;
+  while (groups < kXcds && perGroup % 2 == 0 && perGroup / 2 * d * 2 >= 128) {
+    groups *= 2;
+    perGroup /= 2;
+  }
+  return groups;
+}
+
 // 16 bytes of an output nobody reads before the kernel ends, past the caches: an output that is
 // still dirty in the L2s when a kernel ends is written back then, with the GPU idle (a call with
 // 43 MB of output: 119 -> 105 us; one with 217 MB: 155 -> 121 us). Only for stores that fill whole

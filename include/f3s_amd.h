@@ -169,7 +169,8 @@ int f3s_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, i
  *                                  With it, graphs for which f3s_attention_uses_workspace()
  *                                  returns 1 are computed by the column-sliced schedule: per
  *                                  (window, column slice) partial results that a second kernel
- *                                  merges in slice order. Results agree with the default
+ *                                  merges in slice order (small structures at d <= 64 are
+ *                                  computed as without it). Results agree with the default
  *                                  schedule within the tolerance of the summation order.
  *                                  Ignored with cuTimer. Calls that share a workspace must not
  *                                  overlap. Its contents need not be initialised.
@@ -192,8 +193,9 @@ int f3s_attention_fwd(const int32_t* rowWindowOffset, const int32_t* windowOrder
  * (m, l, O) of 64 d + 128 bytes per window, head and slice; for the single-head call at d = 64 also
  * 512 * N bytes for copies of K and V with 256-byte rows, which the call makes itself and gathers
  * from instead: rows that start on even 128-byte lines are served faster than rows on the odd lines
- * in between). Slices are two or more, about one per 8 MiB of a group of heads' K + V rows up to
- * sixteen, so the size does not grow with N alone: ask for every N and d. The reference's launchers
+ * in between). Room is for as many slices as any structure of N nodes is cut into: two or more, about
+ * one per 8 MiB (3 MiB at d = 32) of a group of heads' K + V rows up to sixteen, so the size does not
+ * grow with N alone: ask for every N and d. The reference's launchers
  * (src/F3S_kernel.cu:581-671) need no scratch; passing workspace = NULL keeps that behaviour.
  */
 size_t f3s_attention_workspace_bytes(int N, int d);

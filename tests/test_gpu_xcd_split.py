@@ -116,6 +116,76 @@ def test_resident_deals_the_same_slices(oracle_mod, monkeypatch, heads, d, N):
     check(oracle_mod, pre, N, max(heads, 1), d, Q, K, V, got[1])
 
 
+# The number of slices follows from the blocks per window: of 2 048 windows, the first `long` name
+# `blocks` blocks each (2.5, 4.5 and 8 slices' worth on average at d = 128; K + V of 17 and 134 MB bound
+# it, one or four slices at a time). A prepared workspace of one structure serves a call on another, whose
+# slices are other ones.
+@pytest.mark.parametrize("heads,d,N", [(0, 128, 32_771), (0, 256, 131_101), (2, 32, 32_771),
+                                       (4, 128, 65_551)])
+def test_slices_by_blocks_per_window(oracle_mod, monkeypatch, heads, d, N):
+    from fused3s_amd import capi
+    print("case slices by blocks heads=%d d=%d N=%d" % (heads, d, N), flush=True)
+    monkeypatch.setenv("F3S_SCHEDULE", "sliced")
+    monkeypatch.delenv("F3S_SLICE_PHASES", raising=False)
+    g = torch.Generator().manual_seed(N)
+    Q, K, V = [torch.randn((N, max(heads, 1), d), generator=g).half().cuda() for _ in range(3)]
+    ws = capi.attention_workspace(N, d, "cuda", heads=heads)
+    structures = []
+    for per_window in (3, 90, 300):  # blocks of 16 distinct columns
+        rng = np.random.default_rng(per_window)
+        long = min((N + 15) // 16 - 2, 40)
+        rowPtr = np.zeros(N + 1, np.int32)
+        deg = np.zeros(N, np.int64)
+        deg[:16 * long:16] = min(N, 16 * per_window * ((N + 15) // 16) // long)
+        deg[N // 2:] = 1
+        rowPtr[1:] = np.cumsum(deg)
+        cols = [np.sort(rng.choice(N, size=k, replace=False)) for k in deg[:16 * long:16]]
+        colIdx = np.concatenate(cols + [rng.integers(0, N, int(deg[N // 2:].sum()))])
+        structures.append(on_gpu(oracle_mod, rowPtr, colIdx.astype(np.int32), N))
+    for prepared_for, (pre, (rwo, order, atox, bm)) in zip((0, 0, 2), structures):
+        ws.fill_(0xFF)
+        base = structures[prepared_for][1]
+        capi.attention_prepare(base[0], base[2], N, d, ws, heads=heads)
+        if heads:
+            got = capi.attention_heads(rwo, order, atox, bm, N, Q, K, V, float(np.sqrt(d)),
+                                       workspace=ws, prepared=True)
+        else:
+            got = capi.attention(rwo, order, atox, bm, N, *[t[:, 0].contiguous() for t in (Q, K, V)],
+                                 float(np.sqrt(d)), workspace=ws, prepared=True)
+        check(oracle_mod, pre, N, max(heads, 1), d, Q, K, V, got)
+
+
+# Single-head calls at d <= 64 on structures of fewer blocks than 260 000 (d = 32) or 450 000 (d = 64) leave
+# their workspace alone, those of more use it
+@pytest.mark.parametrize("d,blocks", [(32, 259_000), (32, 261_000), (64, 449_000), (64, 451_000),
+                                      (96, 200_000)])
+def test_small_single_head_calls_leave_the_workspace(oracle_mod, monkeypatch, d, blocks):
+    from fused3s_amd import capi
+    print("case small single head d=%d blocks=%d" % (d, blocks), flush=True)
+    monkeypatch.delenv("F3S_SCHEDULE", raising=False)
+    monkeypatch.delenv("F3S_SLICE_PHASES", raising=False)
+    N = 16 * 2048 - 3
+    rng = np.random.default_rng(blocks)
+    long = 300
+    deg = np.ones(N, np.int64)
+    deg[:16 * long:16] = min(N, 16 * blocks // long)
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(deg)
+    colIdx = np.concatenate([np.sort(rng.choice(N, size=k, replace=False)) if k > 1 else
+                             rng.integers(0, N, 1) for k in deg]).astype(np.int32)
+    pre, (rwo, order, atox, bm) = on_gpu(oracle_mod, rowPtr, colIdx, N)
+    limit = {32: 260_000, 64: 450_000}.get(d, 0)
+    assert pre["blockCount"] >= 64 * 2048
+    g = torch.Generator().manual_seed(d)
+    Q, K, V = [torch.randn((N, 1, d), generator=g).half().cuda() for _ in range(3)]
+    ws = capi.attention_workspace(N, d, "cuda", nTCB=atox.numel() // 16)
+    ws.fill_(0xFF)
+    got = capi.attention(rwo, order, atox, bm, N, *[t[:, 0].contiguous() for t in (Q, K, V)],
+                         float(np.sqrt(d)), workspace=ws)
+    assert bool((ws == 0xFF).all()) == (pre["blockCount"] < limit)
+    check(oracle_mod, pre, N, 1, d, Q, K, V, got)
+
+
 # 1025 windows: one more than a whole number of chunks for every number of head groups
 @pytest.mark.parametrize("heads,d", [(1, 32), (3, 64), (4, 64), (8, 32), (2, 128)])
 def test_short_windows(oracle_mod, heads, d):
