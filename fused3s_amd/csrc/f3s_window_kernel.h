@@ -91,9 +91,13 @@ __device__ __forceinline__ unsigned cu_key() {
 
 // HEADS = false: Q/K/V are [N, D] contiguous, one workgroup per window (blockIdx.x = position in
 // the window order). HEADS = true: Q/K/V are [N, nHeads, D] with a row pitch of ldIn elements,
-// out is [N, nHeads * D] with a row pitch of ldOut floats, and blockIdx.x = position * nHeads +
-// head, so that the workgroups of one window's heads are dispatched together and share the
-// window's column ids and bitmaps (and the neighbouring pieces of its K/V rows) in L2.
+// out is [N, nHeads * D] with a row pitch of ldOut floats. Workgroup b runs on XCD b % 8; the XCDs are
+// dealt groups of heads (split_heads: of at least a line of a row) and, 8 / headGroups of them to a
+// group, the positions of the order, the heads of a position one after the other: an XCD gathers one
+// group's part of the rows, and whole lines of it. With blockIdx.x = position * nHeads + head the two
+// heads of a line came from two XCDs, each of which fetched all of it (bf16, 200 000 nodes, 48 blocks a
+// window, 4 x 32: 823 -> 472 us; R-MAT of 1 000 000 nodes and 25 blocks, 2 x 32: 1203 -> 836 us; 40 000
+// nodes, 19 blocks, 8 x 32: 111 -> 100 us; wider heads are dealt as before).
 // W8 = true: the structure comes from preprocessing with 8-column blocks (the reference's
 // 1tb1tcb path, src/F3S_kernel.cu:677-877). Column ids and bitmap words of two consecutive 16x8
 // blocks are laid out exactly like one 16x16 block, so the same pipeline runs over four 16x8
@@ -124,7 +128,7 @@ f3s_fwd_kernel(
     const int32_t* __restrict__ sparseAToXidx, const uint8_t* __restrict__ bitmapBytes, int N,
     int nRW, int64_t nTcb, const ET* __restrict__ Q, const ET* __restrict__ K,
     const ET* __restrict__ V, float scaleLog2, float* __restrict__ out,
-    unsigned long long* __restrict__ cuTimer, int nHeads, int ldIn, int ldOut,
+    unsigned long long* __restrict__ cuTimer, int nHeads, int headGroups, int ldIn, int ldOut,
     float* __restrict__ sddmm, int minBlocks, int nPositions) {
   constexpr int NWAVES = team_waves(TEAM, D);
   constexpr int WAVE_BYTES = pipe::Geo<D, team_stages(TEAM, D)>::WAVE_BYTES;
@@ -142,8 +146,15 @@ f3s_fwd_kernel(
   constexpr bool scan = TEAM == TEAM_LONG;
   __shared__ int sUnitCount;
   __shared__ int sUnitList[scan ? NWAVES * 64 : 1];
-  int pos = HEADS ? (int)(blockIdx.x / (unsigned)nHeads) : (int)blockIdx.x;
-  int head = HEADS ? (int)(blockIdx.x - (unsigned)pos * (unsigned)nHeads) : 0;
+  int pos = (int)blockIdx.x, head = 0;
+  if constexpr (HEADS && !scan) {
+    const unsigned perGroup = (unsigned)nHeads / (unsigned)headGroups;
+    const unsigned xcd = blockIdx.x % kXcds, u = blockIdx.x / kXcds, p = u / perGroup;
+    const unsigned shares = kXcds / (unsigned)headGroups;  // of the positions
+    pos = (int)(p * shares + xcd / (unsigned)headGroups);
+    head = (int)(xcd % (unsigned)headGroups * perGroup + (u - p * perGroup));
+    if (pos >= nPositions) return;
+  }
   // A launch that shares the windows with the wave-per-window kernel (TEAM_LONG, minBlocks >= 0)
   // covers the (position, head) units of the order's first nPositions positions with a grid of its
   // own size: thread t of workgroup b looks at unit b + t * gridDim.x, and the workgroup computes
@@ -341,6 +352,9 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
   if (gw == 0) return 0;
   const int heads = hl.nHeads > 0 ? hl.nHeads : 1;
   const unsigned units = gw * (unsigned)heads;
+  const int headGroups = head_groups(D, heads);
+  const unsigned shares = kXcds / (unsigned)headGroups;
+  const unsigned headGrid = (gw + shares - 1) / shares * (heads / headGroups) * kXcds;
 #define F3S_LAUNCH(TEAM_, CLOCKED_, HEADS_, GRID)                                              \
   {                                                                                            \
     auto kernel = f3s_fwd_kernel<ET, D, TEAM_, SOFTMAX, CLOCKED_, HEADS_, false, WIDE>;        \
@@ -348,7 +362,8 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
     if (int rc = allow_lds(kernel, lds)) return rc;                                            \
     hipLaunchKernelGGL(kernel, dim3(GRID), dim3(team_waves(TEAM_, D) * 64), lds, stream, rwo,  \
                        order, atox, bm, N, nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer,     \
-                       heads, hl.nHeads > 0 ? hl.ldIn : D, hl.nHeads > 0 ? hl.ldOut : D,       \
+                       heads, headGroups, hl.nHeads > 0 ? hl.ldIn : D,                         \
+                       hl.nHeads > 0 ? hl.ldOut : D,                                           \
                        (float*)nullptr, hl.minBlocks, (int)gw);                                \
   }
   if (hl.minBlocks >= 0) {
@@ -380,15 +395,15 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
       if (grid > gw) grid = gw;
       hipLaunchKernelGGL(reset_window_cursor_kernel<0>, dim3(1), dim3(1), 0, stream);
       hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream, rwo, order, atox, bm, N,
-                         nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer, 1, D, D, (float*)nullptr,
+                         nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer, 1, 1, D, D, (float*)nullptr,
                          hl.minBlocks, (int)gw);
     }
   } else {
     constexpr Team kPairs = D <= 32 ? TEAM_PAIRS : TEAM_SHORT;  // no second kernel above D = 32
     const bool pairs = two_stages(D, hl.nTcb, heads, N);
     if (hl.nHeads > 0) {
-      if (pairs) F3S_LAUNCH(kPairs, false, true, units)
-      else F3S_LAUNCH(TEAM_SHORT, false, true, units)
+      if (pairs) F3S_LAUNCH(kPairs, false, true, headGrid)
+      else F3S_LAUNCH(TEAM_SHORT, false, true, headGrid)
     } else if (cuTimer) {
       if (pairs) F3S_LAUNCH(kPairs, true, false, gw)
       else F3S_LAUNCH(TEAM_SHORT, true, false, gw)
@@ -418,7 +433,7 @@ int launch_tcb8(const int32_t* rwo, const int32_t* order, const int32_t* atox,
   hipLaunchKernelGGL(kernel, dim3(nRW), dim3(team_waves(TEAM_SHORT, D) * 64), lds, stream, rwo, order, atox,
                      reinterpret_cast<const uint8_t*>(bitmap), N, nRW, nTcb8,
                      static_cast<const _Float16*>(Q), static_cast<const _Float16*>(K),
-                     static_cast<const _Float16*>(V), scaleLog2, out, nullptr, 1, D, D, sddmm, -1,
+                     static_cast<const _Float16*>(V), scaleLog2, out, nullptr, 1, 1, D, D, sddmm, -1,
                      nRW);
   F3S_HIP_CHECK(hipGetLastError());
   return 0;

@@ -186,6 +186,25 @@ def test_small_single_head_calls_leave_the_workspace(oracle_mod, monkeypatch, d,
     check(oracle_mod, pre, N, 1, d, Q, K, V, got)
 
 
+# The window kernel deals the XCDs groups of heads: every (window, head) exactly once, for head counts that
+# split into one to eight groups or not at all, and one window more or less than a share of them
+@pytest.mark.parametrize("heads,d", [(2, 32), (3, 32), (4, 32), (6, 32), (16, 32), (5, 64), (12, 64),
+                                     (16, 64), (4, 96), (7, 128)])
+@pytest.mark.parametrize("N", [16, 16 * 7 + 1, 16 * 9])
+def test_window_kernel_head_groups(oracle_mod, monkeypatch, heads, d, N):
+    from fused3s_amd import capi
+    print("case window head groups heads=%d d=%d N=%d" % (heads, d, N), flush=True)
+    monkeypatch.setenv("F3S_SCHEDULE", "window")
+    rng = np.random.default_rng(heads + N)
+    pre, (rwo, order, atox, bm) = on_gpu(oracle_mod, *random_csr(rng, N, 9, empty_frac=0.1), N)
+    g = torch.Generator().manual_seed(d)
+    Q, K, V = [torch.randn((N, heads, d), generator=g).half().cuda() for _ in range(3)]
+    out = torch.full((N, heads * d), float("nan"), device="cuda")
+    for od in (order, None):
+        got = capi.attention_heads(rwo, od, atox, bm, N, Q, K, V, float(np.sqrt(d)), out=out.clone())
+        check(oracle_mod, pre, N, heads, d, Q, K, V, got)
+
+
 # 1025 windows: one more than a whole number of chunks for every number of head groups
 @pytest.mark.parametrize("heads,d", [(1, 32), (3, 64), (4, 64), (8, 32), (2, 128)])
 def test_short_windows(oracle_mod, heads, d):
