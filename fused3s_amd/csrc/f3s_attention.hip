@@ -52,15 +52,19 @@ int attention_uses_workspace(int N, int64_t nTcb, int d, int dtype) {
   return nRW >= 2048 && nTcb >= 64 * nRW;
 }
 
-// Single-head calls on small structures of narrow rows are over before their slices pay, with or without a
-// workspace (window against sliced, us): d = 64: 50 000 nodes, 76 blocks a window 63 against 83; 70 000,
-// 93: 106 against 119; 100 000, 66: 120 against 145; 50 000, 178: 118 against 121; from 750 000 blocks
-// sliced is faster (100 000, 121: 219 against 193). d = 32: 50 000, 76: 47 against 54; 40 000, 100: 48
-// against 54; 100 000, 66: 99 against 92. Of several heads even small ones pay (40 000, 73, 4 x 32: 152
-// against 126).
-bool windows_suffice(int64_t nTcb, int d) {
+// Calls on small structures of narrow rows are over before their slices pay, with or without a workspace
+// (window against sliced, us; nodes, blocks a window). One head, d = 64: 50 000, 76 63 against 83; 70 000,
+// 93 106 against 119; 100 000, 66 120 against 145; 50 000, 178 118 against 121; from 750 000 blocks sliced
+// is faster (100 000, 121: 219 against 193). d = 32: 50 000, 76 47 against 54; 40 000, 100 48 against 54;
+// 100 000, 66 99 against 92. Several heads, d = 64: 40 000, 73: 2 heads 90 against 104, 4 heads 175
+// against 183; 100 000, 66: 241 against 233, 505 against 464. Pairs of 32: 100 000, 61: 4 heads 231
+// against 302, 8 heads 474 against 551; 100 000, 121: 459 against 468, 959 against 879.
+bool windows_suffice(int64_t nTcb, int d, int nHeads) {
   if (getenv("F3S_SCHEDULE") || getenv("F3S_SLICE_PHASES")) return false;  // asked for
-  return nTcb < (d <= 32 ? 260000 : d <= 64 ? 450000 : 0);
+  if (d > 64) return false;
+  if (nHeads <= 1) return nTcb < (d <= 32 ? 260000 : 450000);
+  if (d == 32) return heads_in_pairs(d, nHeads) && nTcb < 600000;
+  return nTcb < 250000;
 }
 
 int launch_attention(const int32_t* rowWindowOffset, const int32_t* windowOrder,
@@ -83,7 +87,7 @@ int launch_attention(const int32_t* rowWindowOffset, const int32_t* windowOrder,
     return launch_window_wide(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q,
                               K, V, scaleLog2, applySoftmax, out, cuTimer, 0, d, d, nTcb, stream);
   if (workspace && !cuTimer && attention_uses_workspace(N, nTcb, d, dtype) &&
-      !windows_suffice(nTcb, d))
+      !windows_suffice(nTcb, d, 0))
     return launch_attention_sliced(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, 0, d, d, prepared ? 2 : 0, stream);
@@ -174,7 +178,7 @@ int launch_attention_heads(const int32_t* rowWindowOffset, const int32_t* window
     return launch_window_wide(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q,
                               K, V, scaleLog2, applySoftmax, out, nullptr, nHeads, (int)ldIn,
                               (int)ldOut, nTcb, stream);
-  if (workspace && attention_uses_workspace(N, nTcb, d, dtype))
+  if (workspace && attention_uses_workspace(N, nTcb, d, dtype) && !windows_suffice(nTcb, d, nHeads))
     return launch_attention_sliced(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, nHeads, (int)ldIn, (int)ldOut, prepared ? 2 : 0, stream);

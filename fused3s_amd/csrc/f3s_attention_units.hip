@@ -135,14 +135,21 @@ inline XcdSplit split_heads(int d, int heads) {
 #define F3S_PARTIAL_LOAD(p) __builtin_nontemporal_load(p)
 #endif
 
-template <int D, typename PipeT>
-__device__ __forceinline__ void store_partial(const PipeT& pp, float* __restrict__ dst) {
+// of NH heads of D / NH features each, whose partials lie `stride` floats apart
+template <int D, int NH, typename PipeT>
+__device__ __forceinline__ void store_partial(const PipeT& pp, float* __restrict__ dst,
+                                              int64_t stride) {
+  constexpr int TH = D / NH / 16;
   const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int jj = 0; jj < D / 16; jj++)
-    F3S_PARTIAL_STORE(pp.o[jj], reinterpret_cast<float4v*>(dst) + jj * 64 + lane);
-  const float l = pipe::row_sum4(pp.l);  // m is the same in the four lanes of a row already
-  if (lane < 32) F3S_PARTIAL_STORE(lane < 16 ? pp.m : l, dst + 16 * D + lane);
+  for (int h = 0; h < NH; h++) {
+#pragma unroll
+    for (int jj = 0; jj < TH; jj++)
+      F3S_PARTIAL_STORE(pp.o[h * TH + jj], reinterpret_cast<float4v*>(dst) + jj * 64 + lane);
+    const float l = pipe::row_sum4(pp.l[h]);  // m is the same in the four lanes of a row already
+    if (lane < 32) F3S_PARTIAL_STORE(lane < 16 ? pp.m[h] : l, dst + 16 * (D / NH) + lane);
+    dst += stride;
+  }
 }
 
 // A window's 16 rows of D floats from the lanes' O^T tiles (already normalised) to memory, through
@@ -183,7 +190,8 @@ __device__ __forceinline__ void store_rows(const float4v (&o)[D / 16], float* ld
 //            through exactly those positions (with a heavy-first order no long window lies beyond
 //            them; with any other order such a window is simply computed here). XcdSplit deals
 //            head groups and chunks of the order to the XCDs.
-template <typename ET, int D, bool SOFTMAX, bool SLICED, bool HEADS>
+// NH = 2: D = 64 stands for two heads of 32; split counts such pairs, nHeads heads.
+template <typename ET, int D, bool SOFTMAX, bool SLICED, bool HEADS, int NH = 1>
 __global__ __launch_bounds__(kUnitWaves * 64)
 __attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D, SLICED),
                                    unit_waves_per_simd(D, SLICED)))) void
@@ -197,8 +205,8 @@ f3s_fwd_unit_kernel(const int32_t* __restrict__ windowOrder,
                     float* __restrict__ out, int nHeads, int ldIn, int ldOut, int maxBlocks,
                     int longPrefix, int ldQ) {
   constexpr int STAGES = unit_stages(D, SLICED);
-  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false, STAGES> Pipe;
-  constexpr int T = D / 16;
+  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false, STAGES, false, NH> Pipe;
+  constexpr int TH = D / NH / 16;
   extern __shared__ __align__(1024) unsigned char smem[];
 
   const int wave = uniform(threadIdx.x >> 6);
@@ -242,16 +250,20 @@ f3s_fwd_unit_kernel(const int32_t* __restrict__ windowOrder,
   pp.run(pb, t0, t1);
 
   if constexpr (SLICED) {
-    const int64_t wh = (int64_t)w * (HEADS ? nHeads : 1) + head;
-    store_partial<D>(pp, partial + (wh * split.slices() + un.slice) * partial_floats<D>());
+    const int64_t wh = (int64_t)w * (HEADS ? nHeads : 1) + head * NH;
+    const int64_t stride = (int64_t)split.slices() * partial_floats<D / NH>();
+    store_partial<D, NH>(pp, partial + wh * stride + un.slice * partial_floats<D / NH>(), stride);
   } else {
-    float inv = 1.0f;
-    if constexpr (SOFTMAX) {
-      const float lAll = pipe::row_sum4(pp.l);
-      inv = (lAll == 0.0f) ? 0.0f : 1.0f / lAll;
-    }
 #pragma unroll
-    for (int jj = 0; jj < T; jj++) pp.o[jj] *= inv;
+    for (int h = 0; h < NH; h++) {
+      float inv = 1.0f;
+      if constexpr (SOFTMAX) {
+        const float lAll = pipe::row_sum4(pp.l[h]);
+        inv = (lAll == 0.0f) ? 0.0f : 1.0f / lAll;
+      }
+#pragma unroll
+      for (int jj = 0; jj < TH; jj++) pp.o[h * TH + jj] *= inv;
+    }
     // the wave's ring is free now
     static_assert(rows_lds_floats<D>() * 4 <= pipe::Geo<D, STAGES>::WAVE_BYTES, "rows fit the ring");
     store_rows<D>(pp.o,
@@ -386,7 +398,7 @@ __global__ __launch_bounds__(256) void sliced_setup_kernel(
 // the wave that finishes a window's last unit merges its partials (an arrival counter per window,
 // partials written through) took 1.92 ms: the wait for the stores and the returning atomic sit on
 // every unit's path.
-template <typename ET, int D, bool SOFTMAX, bool HEADS, int NW>
+template <typename ET, int D, bool SOFTMAX, bool HEADS, int NW, int NH = 1>
 __global__ __launch_bounds__(NW * 64)
 __attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D, true),
                                    unit_waves_per_simd(D, true)))) void
@@ -397,7 +409,7 @@ f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
                         const uint8_t* __restrict__ bitmapBytes, const ET* __restrict__ Q,
                         const ET* __restrict__ K, const ET* __restrict__ V, float scaleLog2,
                         float* __restrict__ partial, int nHeads, int ldIn) {
-  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false, unit_stages(D, true)> Pipe;
+  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false, unit_stages(D, true), false, NH> Pipe;
   extern __shared__ __align__(1024) unsigned char smem[];
   __shared__ int sCtl[2];  // slot of this workgroup; next unit of its sequence
 
@@ -485,8 +497,9 @@ f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
       Pipe pp;
       pp.init(pb, wu, ringAddr, head);
       pp.run(pb, t0u, t1u);
-      const int64_t wh = (int64_t)wu * heads + head;
-      store_partial<D>(pp, partial + (wh * S + slice_of(u)) * partial_floats<D>());
+      const int64_t wh = (int64_t)wu * heads + head * NH;
+      const int64_t stride = (int64_t)S * partial_floats<D / NH>();
+      store_partial<D, NH>(pp, partial + wh * stride + slice_of(u) * partial_floats<D / NH>(), stride);
     }
     u = u1;
     w = w1;
@@ -607,15 +620,18 @@ constexpr int64_t slice_weight(int d) { return d <= 32 ? 55 : d <= 128 ? 45 : d 
 XcdSplit choose_split(int N, int d, int heads, int64_t nTcb) {
   const char* e = getenv("F3S_SLICE_PHASES");  // read per call: tests walk through the phases
   const int forced = e ? atoi(e) : 0;
-  if (forced > 0) return {forced > kMaxPhases ? kMaxPhases : forced, kXcds, 1, 1, heads, 1};
-  XcdSplit s = split_heads(d, heads);
+  const int units = heads_in_pairs(d, heads) ? heads / 2 : heads;  // that a window and slice are
+  if (forced > 0) return {forced > kMaxPhases ? kMaxPhases : forced, kXcds, 1, 1, units, 1};
+  const int dUnit = heads / units * d;  // columns of a row that a unit gathers
+  XcdSplit s = split_heads(dUnit, units);
   const int64_t nRW = (N + kWinRows - 1) / kWinRows;
-  const int64_t bytes = (int64_t)N * d * s.headsPerGroup * 4;  // K + V of a group's heads
-  const int64_t most = nTcb < 0 && d > 32 ? slice_bytes(64) : slice_bytes(d);
+  // K + V of a group's heads
+  const int64_t bytes = (int64_t)N * dUnit * s.headsPerGroup * 4;
+  const int64_t most = nTcb < 0 && dUnit > 32 ? slice_bytes(64) : slice_bytes(dUnit);
   int64_t need = (bytes + most - 1) / most;
   if (nTcb >= 0 && nRW > 0) {  // (weight / 100) sqrt(blocks per window), rounded
     int64_t worth = 2;
-    while ((2 * worth + 1) * (2 * worth + 1) * 2500 * nRW <= slice_weight(d) * slice_weight(d) * nTcb)
+    while ((2 * worth + 1) * (2 * worth + 1) * 2500 * nRW <= slice_weight(dUnit) * slice_weight(dUnit) * nTcb)
       worth++;
     if (need > worth) need = worth;
   }
@@ -626,7 +642,7 @@ XcdSplit choose_split(int N, int d, int heads, int64_t nTcb) {
   // start when the first phase's light ones should fill the end (60k nodes, d = 32: 188 -> 206 us).
   // The slices at a time are a power of two, the nearest one rather than the next (50k nodes, d = 96:
   // 123 us with 4 slices, 146 with 8).
-  const int64_t waves = 32 * 4 * unit_waves_per_simd(d, true);  // of one XCD
+  const int64_t waves = 32 * 4 * unit_waves_per_simd(dUnit, true);  // of one XCD
   if (s.units(nRW) < 2 * waves) {
     while (s.windowGroups > 1 && (nTcb < 0 ? s.sliceGroups < need : 3 * s.sliceGroups <= 2 * need)) {
       s.sliceGroups *= 2;
@@ -715,7 +731,7 @@ bool resident_requested() {
   return e && e[0] == '1';
 }
 
-template <typename ET, int D, bool SOFTMAX, bool HEADS>
+template <typename ET, int D, bool SOFTMAX, bool HEADS, int NH = 1>
 int launch_sliced_units(const int32_t* rwo, const int32_t* order, const int32_t* atox,
                         const uint8_t* bm, int N, int nRW, const ET* Q, const ET* K, const ET* V,
                         float scaleLog2, float* out, int32_t* tickets, int32_t* sliceStart,
@@ -723,7 +739,7 @@ int launch_sliced_units(const int32_t* rwo, const int32_t* order, const int32_t*
                         int64_t nTcb, hipStream_t stream, int ldQ = 0) {
   constexpr size_t lds = (size_t)kUnitWaves * pipe::Geo<D, unit_stages(D, true)>::WAVE_BYTES;
   if (resident_requested()) {
-    auto kernel = f3s_fwd_resident_kernel<ET, D, SOFTMAX, HEADS, kUnitWaves>;
+    auto kernel = f3s_fwd_resident_kernel<ET, D, SOFTMAX, HEADS, kUnitWaves, NH>;
     if (int rc = allow_lds(kernel, lds)) return rc;
     int grid = 0;
     if (int rc = resident_grid<D, kUnitWaves>(&grid)) return rc;
@@ -731,7 +747,7 @@ int launch_sliced_units(const int32_t* rwo, const int32_t* order, const int32_t*
                        sliceStart, resident_split(L.split), nRW, N, nTcb, tickets, atox, bm, Q, K, V, scaleLog2,
                        partial, heads, ldIn);
   } else {
-    auto kernel = f3s_fwd_unit_kernel<ET, D, SOFTMAX, true, HEADS>;
+    auto kernel = f3s_fwd_unit_kernel<ET, D, SOFTMAX, true, HEADS, NH>;
     if (int rc = allow_lds(kernel, lds)) return rc;
     const int64_t nGroups = (L.split.units(nRW) + kUnitWaves - 1) / kUnitWaves;
     const int64_t grid = L.split.phases * nGroups * kXcds;
@@ -779,7 +795,11 @@ int launch_sliced_d(const int32_t* rwo, const int32_t* order, const int32_t* ato
   const auto* k = static_cast<const ET*>(K);
   const auto* v = static_cast<const ET*>(V);
   int rc;
-  if (nHeads > 0) {
+  if (D == 32 && heads_in_pairs(D, nHeads)) {
+    rc = launch_sliced_units<ET, D == 32 ? 64 : D, SOFTMAX, true, D == 32 ? 2 : 1>(
+        rwo, order, atox, bm, N, nRW, q, k, v, scaleLog2, out, tickets, sliceStart, partial, L, heads,
+        ldIn, ldOut, nTcb, stream);
+  } else if (nHeads > 0) {
     rc = launch_sliced_units<ET, D, SOFTMAX, true>(rwo, order, atox, bm, N, nRW, q, k, v,
                                                    scaleLog2, out, tickets, sliceStart, partial, L,
                                                    heads, ldIn, ldOut, nTcb, stream);
@@ -857,13 +877,19 @@ namespace {
 // the first XCD would get the sixteen heaviest.
 constexpr int kShortChunk = 16;
 
-template <typename ET, int D, bool SOFTMAX>
+// NH = 2: D = 64 stands for two heads of 32
+template <typename ET, int D, bool SOFTMAX, int NH = 1>
 int launch_short_d(const int32_t* rwo, const int32_t* order, const int32_t* atox,
                    const uint64_t* bitmap, int N, const void* Q, const void* K, const void* V,
                    float scaleLog2, float* out, int nHeads, int ldIn, int ldOut, int maxBlocks,
                    int longPrefix, int64_t nTcb, hipStream_t stream) {
+  if constexpr (D == 32) {
+    if (heads_in_pairs(D, nHeads))
+      return launch_short_d<ET, 64, SOFTMAX, 2>(rwo, order, atox, bitmap, N, Q, K, V, scaleLog2, out,
+                                                nHeads, ldIn, ldOut, maxBlocks, longPrefix, nTcb, stream);
+  }
   const int nRW = (N + kWinRows - 1) / kWinRows;
-  XcdSplit split = split_heads(D, nHeads > 0 ? nHeads : 1);
+  XcdSplit split = split_heads(D, nHeads > 0 ? nHeads / NH : 1);
   split.chunk = kShortChunk;
   const int64_t nGroups = (split.units(nRW) + kUnitWaves - 1) / kUnitWaves;
   if (nGroups * kXcds >= ((int64_t)1 << 31))
@@ -874,12 +900,13 @@ int launch_short_d(const int32_t* rwo, const int32_t* order, const int32_t* atox
   const auto* k = static_cast<const ET*>(K);
   const auto* v = static_cast<const ET*>(V);
   constexpr size_t lds = (size_t)kUnitWaves * pipe::Geo<D, unit_stages(D, false)>::WAVE_BYTES;
-  if (nHeads > 0) {
-    if (int rc = allow_lds(f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, true>, lds)) return rc;
-    hipLaunchKernelGGL((f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, true>), grid, block, lds,
+  if (NH > 1 || nHeads > 0) {
+    auto kernel = f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, true, NH>;
+    if (int rc = allow_lds(kernel, lds)) return rc;
+    hipLaunchKernelGGL(kernel, grid, block, lds,
                        stream, order, rwo, atox, bm, nullptr, split, (int)nGroups, N, nRW, nTcb, q, k, v,
                        scaleLog2, nullptr, out, nHeads, ldIn, ldOut, maxBlocks, longPrefix, 0);
-  } else {
+  } else if constexpr (NH == 1) {
     if (int rc = allow_lds(f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, false>, lds)) return rc;
     hipLaunchKernelGGL((f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, false>), grid, block, lds,
                        stream, order, rwo, atox, bm, nullptr, split, (int)nGroups, N, nRW, nTcb, q, k, v,

@@ -36,6 +36,10 @@ inline int head_groups(int d, int heads) {
   return groups;
 }
 
+// Whether a multi-head call computes its heads two at a time: 32-wide heads share the 128-byte lines of
+// K and V rows in pairs. nHeads = 0: the single-head layout.
+inline bool heads_in_pairs(int d, int nHeads) { return d == 32 && nHeads > 0 && nHeads % 2 == 0; }
+
 // 16 bytes of an output nobody reads before the kernel ends, past the caches: an output that is
 // still dirty in the L2s when a kernel ends is written back then, with the GPU idle (a call with
 // 43 MB of output: 119 -> 105 us; one with 217 MB: 155 -> 121 us). Only for stores that fill whole

@@ -277,8 +277,18 @@ struct Problem {
 // comes from preprocessing with 8-column blocks; two consecutive 16x8 blocks are laid out like
 // one 16x16 block, block indices and counts below are then in 16x8 blocks. WIDE: K or V spans
 // 4 GiB or more (or a pitched layout exceeds the 24-bit multiply): row offsets in 64 bits.
-template <typename ET, int D, bool SOFTMAX, bool HEADS, bool W8, int STAGES, bool WIDE = false>
+// NH = 2: the D = 64 features of a row are two heads of 32 next to each other. Rows are gathered, and
+// operands read, as one head's of 64; scores, softmax (m, l) and the two halves of O are each head's
+// own, with the arithmetic of a D = 32 pipeline in the same order (bit-identical). Two 32-wide heads one
+// by one ask for every 128-byte line twice, half of it each, and run the chain of ids, bitmaps and rows
+// twice: that chain is most of a short window's time, and the vector memory path what bounds long ones
+// (bf16: 100k-node community layer of 6 blocks a window, 8 x 32 111.5 -> 97.1 us a call; R-MAT 150 000
+// nodes, 8 x 32 365 -> 260 us, power-law 50 000 nodes, 382 blocks, 8 x 32 1490 -> 1068 us; both with
+// head groups dealt to the XCDs, which by itself made the former 295 us).
+template <typename ET, int D, bool SOFTMAX, bool HEADS, bool W8, int STAGES, bool WIDE = false,
+          int NH = 1>
 struct PairPipeline {
+  static_assert(NH == 1 || (NH == 2 && D == 64 && HEADS && !W8), "two heads of 32");
   typedef Geo<D, STAGES> G;
   typedef typename Vec<ET, 8>::type half8;
   static constexpr int T = G::T;
@@ -294,8 +304,8 @@ struct PairPipeline {
   static constexpr bool SPLIT_P = sizeof(ET) == 2 && !__is_same(ET, _Float16);  // bf16
 
   // running state
-  float m, l;
-  float4v o[T];
+  float m[NH], l[NH];
+  float4v o[T];  // NH tiles' worth of each head, one after the other
 
   // loop-invariant per-lane values
   half8 qf[KS];
@@ -316,8 +326,8 @@ struct PairPipeline {
     c = lane & 15;
     ring = ringAddr;
     metaBase = ringAddr + NS * G::STAGE;
-    m = 0.0f;
-    l = 0.0f;
+#pragma unroll
+    for (int h = 0; h < NH; h++) m[h] = l[h] = 0.0f;
 #pragma unroll
     for (int j = 0; j < T; j++) o[j] = float4v{0.f, 0.f, 0.f, 0.f};
     {
@@ -531,11 +541,14 @@ struct PairPipeline {
     for (int b = 0; b < 2; b++)
 #pragma unroll
       for (int i = 0; i < KS; i++) pin(op.k[b][i]);
-    float4v sA = {0.f, 0.f, 0.f, 0.f}, sB = {0.f, 0.f, 0.f, 0.f};
+    float4v sA[NH], sB[NH];
+#pragma unroll
+    for (int h = 0; h < NH; h++) sA[h] = sB[h] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < KS; i++) {
-      sA = mfma_16x16x32<ET>(__builtin_bit_cast(half8, op.k[0][i]), qf[i], sA);
-      sB = mfma_16x16x32<ET>(__builtin_bit_cast(half8, op.k[1][i]), qf[i], sB);
+      constexpr int KH = KS / NH;  // k-steps of a head
+      sA[i / KH] = mfma_16x16x32<ET>(__builtin_bit_cast(half8, op.k[0][i]), qf[i], sA[i / KH]);
+      sB[i / KH] = mfma_16x16x32<ET>(__builtin_bit_cast(half8, op.k[1][i]), qf[i], sB[i / KH]);
     }
     pin(op.words);
     int wordA = op.words[0], wordB = op.words[1];
@@ -552,6 +565,20 @@ struct PairPipeline {
       keep[i] = __builtin_amdgcn_sbfe(wordA, keepPos[i], 1);  // 0 or -1
       keep[4 + i] = __builtin_amdgcn_sbfe(wordB, keepPos[i], 1);
     }
+#pragma unroll
+    for (int j = 0; j < T; j++) {
+      pin(op.v[j][0]);
+      pin(op.v[j][1]);
+    }
+#pragma unroll
+    for (int h = 0; h < NH; h++) one_head(pb, op, sA[h], sB[h], keep, h, tFirst, nValid);
+  }
+
+  // softmax and second product of head h
+  __device__ __forceinline__ void one_head(const Problem<ET>& pb, Operands& op, const float4v& sA,
+                                           const float4v& sB, const int (&keep)[8], int h, int tFirst,
+                                           int nValid) {
+    constexpr int TH = T / NH;  // output tiles of a head
     float s[8];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -578,7 +605,7 @@ struct PairPipeline {
     float e[8];
     if constexpr (SOFTMAX) {
       // fast path: exponentials against the current maximum, masked ones cleared afterwards
-      const float negM = -m;
+      const float negM = -m[h];
       float sum = 0.0f;
 #pragma unroll
       for (int i = 0; i < 8; i++) {
@@ -594,26 +621,26 @@ struct PairPipeline {
       // that is exactly zero (masked or not): redo the step the careful way
       if (__builtin_amdgcn_ballot_w64(!(sum <= kLazyLimit) || zmin == 0.0f) != 0ull) {
         float sc[8];
-        float mx = m;
+        float mx = m[h];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
           sc[i] = __int_as_float(__float_as_int(s[i]) & keep[i]) * pb.scaleLog2;
           mx = fmaxf(mx, sc[i]);
         }
         mx = row_max4(mx);
-        const float alpha = fast_exp2(m - mx);
-        m = mx;
+        const float alpha = fast_exp2(m[h] - mx);
+        m[h] = mx;
         sum = 0.0f;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
           e[i] = (sc[i] == 0.0f) ? 0.0f : fast_exp2(sc[i] - mx);
           sum += e[i];
         }
-        l *= alpha;
+        l[h] *= alpha;
 #pragma unroll
-        for (int j = 0; j < T; j++) o[j] *= alpha;
+        for (int j = 0; j < TH; j++) o[h * TH + j] *= alpha;
       }
-      l += sum;
+      l[h] += sum;
     } else {
 #pragma unroll
       for (int i = 0; i < 8; i++) e[i] = __int_as_float(__float_as_int(s[i]) & keep[i]);
@@ -621,17 +648,12 @@ struct PairPipeline {
     half8 pf;
 #pragma unroll
     for (int i = 0; i < 8; i++) pf[i] = (ET)e[i];
-#pragma unroll
-    for (int j = 0; j < T; j++) {
-      pin(op.v[j][0]);
-      pin(op.v[j][1]);
-    }
     if constexpr (SPLIT_P) {
       half8 pt;
 #pragma unroll
       for (int i = 0; i < 8; i++) pt[i] = (ET)(e[i] - (float)pf[i]);
 #pragma unroll
-      for (int j = 0; j < T; j++) {
+      for (int j = h * TH; j < (h + 1) * TH; j++) {
         const half8 va = __builtin_bit_cast(
             half8, __builtin_shufflevector(op.v[j][0], op.v[j][1], 0, 1, 2, 3, 4, 5, 6, 7));
         o[j] = mfma_16x16x32<ET>(va, pf, o[j]);
@@ -639,7 +661,7 @@ struct PairPipeline {
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < T; j++) {
+      for (int j = h * TH; j < (h + 1) * TH; j++) {
         const half8 va = __builtin_bit_cast(
             half8, __builtin_shufflevector(op.v[j][0], op.v[j][1], 0, 1, 2, 3, 4, 5, 6, 7));
         o[j] = mfma_16x16x32<ET>(va, pf, o[j]);

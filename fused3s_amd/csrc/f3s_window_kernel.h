@@ -119,8 +119,9 @@ __global__ void reset_window_cursor_kernel() {
 }
 
 // WIDE: 64-bit row offsets in the K / V gathers.
+// NH = 2: D = 64 stands for two heads of 32; nHeads and headGroups count such pairs.
 template <typename ET, int D, Team TEAM, bool SOFTMAX, bool CLOCKED, bool HEADS, bool W8,
-          bool WIDE, bool PERSIST = false>
+          bool WIDE, bool PERSIST = false, int NH = 1>
 __global__ __launch_bounds__(team_waves(TEAM, D) * 64)
 __attribute__((amdgpu_waves_per_eu(waves_per_simd(TEAM, D), waves_per_simd(TEAM, D)))) void
 f3s_fwd_kernel(
@@ -133,7 +134,7 @@ f3s_fwd_kernel(
   constexpr int NWAVES = team_waves(TEAM, D);
   constexpr int WAVE_BYTES = pipe::Geo<D, team_stages(TEAM, D)>::WAVE_BYTES;
   static_assert(team_lds(TEAM, D) == (size_t)NWAVES * WAVE_BYTES, "what the launch asks for");
-  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, W8, team_stages(TEAM, D), WIDE> Pipe;
+  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, W8, team_stages(TEAM, D), WIDE, NH> Pipe;
   constexpr int T = D / 16;
   constexpr int OSTRIDE = D + 4;
   constexpr int BPS = W8 ? 4 : 2;  // blocks of the structure per pipeline step
@@ -241,14 +242,17 @@ f3s_fwd_kernel(
   // ---- merge the waves' partial (m, l, O) and write the window's rows. The merge buffers reuse
   // the rings' memory once every wave has left its loop.
   __syncthreads();
-  float* sM = reinterpret_cast<float*>(smem);                    // [NWAVES][16]
-  float* sL = sM + NWAVES * 16;                                  // [NWAVES][16]
-  float* sO = sL + NWAVES * 16;                                  // [NWAVES][16][OSTRIDE]
-  float l = pp.l;
-  if constexpr (SOFTMAX) l = pipe::row_sum4(l);
-  if (g == 0) {
-    sM[wave * 16 + c] = pp.m;
-    sL[wave * 16 + c] = l;
+  float* sM = reinterpret_cast<float*>(smem);                    // [NH][NWAVES][16]
+  float* sL = sM + NH * NWAVES * 16;                             // [NH][NWAVES][16]
+  float* sO = sL + NH * NWAVES * 16;                             // [NWAVES][16][OSTRIDE]
+#pragma unroll
+  for (int h = 0; h < NH; h++) {
+    float l = pp.l[h];
+    if constexpr (SOFTMAX) l = pipe::row_sum4(l);
+    if (g == 0) {
+      sM[(h * NWAVES + wave) * 16 + c] = pp.m[h];
+      sL[(h * NWAVES + wave) * 16 + c] = l;
+    }
   }
 #pragma unroll
   for (int j = 0; j < T; j++)
@@ -263,14 +267,15 @@ f3s_fwd_kernel(
     if (row >= N) continue;
     float4 acc = {0.f, 0.f, 0.f, 0.f};
     if constexpr (SOFTMAX) {
-      float mAll = sM[q];
+      const int ml = (NH > 1 ? cv / (VEC_PER_ROW / NH) * NWAVES * 16 : 0) + q;  // of this head and row
+      float mAll = sM[ml];
 #pragma unroll
-      for (int v = 1; v < NWAVES; v++) mAll = fmaxf(mAll, sM[v * 16 + q]);
+      for (int v = 1; v < NWAVES; v++) mAll = fmaxf(mAll, sM[v * 16 + ml]);
       float lAll = 0.0f;
 #pragma unroll
       for (int v = 0; v < NWAVES; v++) {
-        const float f = pipe::fast_exp2(sM[v * 16 + q] - mAll);
-        lAll = fmaf(f, sL[v * 16 + q], lAll);
+        const float f = pipe::fast_exp2(sM[v * 16 + ml] - mAll);
+        lAll = fmaf(f, sL[v * 16 + ml], lAll);
         const float4 ov = *reinterpret_cast<const float4*>(&sO[(v * 16 + q) * OSTRIDE + cv * 4]);
         acc.x = fmaf(f, ov.x, acc.x);
         acc.y = fmaf(f, ov.y, acc.y);
@@ -338,12 +343,30 @@ struct HeadLayout {
   int64_t nTcb;     // TC blocks of the structure (bounds every window's block range)
 };
 
-template <typename ET, int D, bool SOFTMAX, bool WIDE>
+// 32-wide heads are computed one by one where there is little to do: the longest window decides there, and
+// one workgroup takes longer for two of its heads (us; blocks times pairs of heads). One pair: R-MAT 57 000
+// 35 -> 43, 88 000 59 -> 63, uniform 39 000 24 -> 26, power-law 75 000 56 -> 64, 72 000 35 -> 28; from
+// 118 000 on no measured graph lost (52 -> 44, 69 -> 60, 79 -> 75, 223 -> 177, 836 -> 682). Two pairs: R-MAT
+// 30 000 29 -> 34, 55 000 33 -> 32, 60 000 44 -> 44, power-law 68 000 33 -> 28, uniform 78 000 58 -> 40. Four:
+// R-MAT 60 000 38 -> 39, uniform 55 000 33 -> 28, R-MAT 110 000 59 -> 48.
+inline bool pairs_pay(int64_t nTcb, int pairs) {
+  return nTcb * pairs >= (pairs == 1 ? 100000 : 50000);
+}
+
+// NH = 2: D = 64 stands for two heads of 32, hl.nHeads for the number of pairs.
+template <typename ET, int D, bool SOFTMAX, bool WIDE, int NH = 1>
 int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, const uint64_t* bitmap,
              int N, const void* Q, const void* K, const void* V, float scaleLog2, float* out,
              unsigned long long* cuTimer, HeadLayout hl, hipStream_t stream) {
   const int nRW = (N + kWinRows - 1) / kWinRows;
   if (nRW == 0) return 0;
+  if constexpr (D == 32) {
+    if (heads_in_pairs(D, hl.nHeads) && pairs_pay(hl.nTcb, hl.nHeads / 2)) {
+      hl.nHeads /= 2;
+      return launch_d<ET, 64, SOFTMAX, WIDE, 2>(rwo, order, atox, bitmap, N, Q, K, V, scaleLog2, out,
+                                                cuTimer, hl, stream);
+    }
+  }
   const auto* bm = reinterpret_cast<const uint8_t*>(bitmap);
   const auto* q = static_cast<const ET*>(Q);
   const auto* k = static_cast<const ET*>(K);
@@ -357,7 +380,8 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
   const unsigned headGrid = (gw + shares - 1) / shares * (heads / headGroups) * kXcds;
 #define F3S_LAUNCH(TEAM_, CLOCKED_, HEADS_, GRID)                                              \
   {                                                                                            \
-    auto kernel = f3s_fwd_kernel<ET, D, TEAM_, SOFTMAX, CLOCKED_, HEADS_, false, WIDE>;        \
+    auto kernel = f3s_fwd_kernel<ET, D, TEAM_, SOFTMAX, CLOCKED_, HEADS_, false, WIDE, false,  \
+                                 HEADS_ ? NH : 1>;                                             \
     constexpr size_t lds = team_lds(TEAM_, D);                                                 \
     if (int rc = allow_lds(kernel, lds)) return rc;                                            \
     hipLaunchKernelGGL(kernel, dim3(GRID), dim3(team_waves(TEAM_, D) * 64), lds, stream, rwo,  \
@@ -375,13 +399,15 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
       const unsigned threads = (unsigned)team_waves(TEAM_LONG, D) * 64;
       unsigned grid = (units + threads - 1) / threads;
       if (grid < 512u) grid = units < 512u ? units : 512u;
-      if (hl.nHeads > 0) F3S_LAUNCH(TEAM_LONG, false, true, grid)
-      else F3S_LAUNCH(TEAM_LONG, false, false, grid)
+      if (NH > 1 || hl.nHeads > 0) F3S_LAUNCH(TEAM_LONG, false, true, grid)
+      else if constexpr (NH == 1) F3S_LAUNCH(TEAM_LONG, false, false, grid)
     }
+  } else if (NH > 1) {
+    F3S_LAUNCH(TEAM_SHORT, false, true, headGrid)
   } else if (!WIDE && hl.nHeads == 0 && !cuTimer && window_cursor_requested()) {
     // F3S_WINDOW_PERSISTENT=1: as many workgroups as the GPU holds at once, windows drawn from
     // a cursor (measured slower than launch order, which therefore stays the default)
-    if constexpr (!WIDE) {
+    if constexpr (!WIDE && NH == 1) {
       auto kernel = f3s_fwd_kernel<ET, D, TEAM_SHORT, SOFTMAX, false, false, false, false, true>;
       constexpr size_t lds = team_lds(TEAM_SHORT, D);
       constexpr int threads = team_waves(TEAM_SHORT, D) * 64;
@@ -398,7 +424,7 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
                          nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer, 1, 1, D, D, (float*)nullptr,
                          hl.minBlocks, (int)gw);
     }
-  } else {
+  } else if constexpr (NH == 1) {
     constexpr Team kPairs = D <= 32 ? TEAM_PAIRS : TEAM_SHORT;  // no second kernel above D = 32
     const bool pairs = two_stages(D, hl.nTcb, heads, N);
     if (hl.nHeads > 0) {

@@ -205,6 +205,47 @@ def test_window_kernel_head_groups(oracle_mod, monkeypatch, heads, d, N):
         check(oracle_mod, pre, N, heads, d, Q, K, V, got)
 
 
+# 32-wide heads two at a time: bit-identical to head by head through every schedule (windows, with and
+# without natural order; short windows with long ones beside them; column slices in both forms), on rows of
+# a pitch that shifts the pairs off the 128-byte lines, scores far above the running maximum in one head
+# of a pair only, and scores that are exactly 0
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads", [2, 4, 6, 16])
+@pytest.mark.parametrize("kind", ["window", "short", "sliced", "resident"])
+def test_pairs_of_heads_are_bit_identical(oracle_mod, monkeypatch, kind, heads, dtype):
+    from fused3s_amd import capi
+    print("case pairs of heads %s heads=%d %s" % (kind, heads, dtype), flush=True)
+    rng = np.random.default_rng(heads)
+    d, N = 32, 16 * (1100 if kind == "short" else 300 if kind != "window" else
+                     2000 if heads == 2 else 1000) + 5
+    deg = rng.poisson(2.0 if kind == "short" else 60.0, N)
+    deg[::1999] = 900
+    rows = [np.unique(rng.integers(0, N, k)) for k in deg]
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum([len(r) for r in rows])
+    pre, (rwo, order, atox, bm) = on_gpu(oracle_mod, rowPtr, np.concatenate(rows).astype(np.int32), N)
+    # enough for the window kernel to take pairs
+    assert kind != "window" or pre["blockCount"] * (heads // 2) >= (100_000 if heads == 2 else 50_000)
+    monkeypatch.setenv("F3S_SCHEDULE", "window" if kind in ("window", "short") else "sliced")
+    monkeypatch.setenv("F3S_SLICED_PERSISTENT", "1" if kind == "resident" else "0")
+    g = torch.Generator().manual_seed(heads)
+    store = torch.randn((3, N, heads * d + 8), generator=g)
+    store[0, ::7, d:2 * d] *= 40.0  # scores of head 1 far above the others'
+    store[0, 3::11, :d] = 0.0
+    store = store.to(dtype).cuda()
+    Q, K, V = [store[k, :, :heads * d].unflatten(1, (heads, d)) for k in range(3)]
+    monkeypatch.setenv("F3S_SLICE_PHASES", "1")  # as many slices for one head as for all
+    scratch = lambda n: None if kind in ("window", "short") else capi.attention_workspace(
+        N, d, "cuda", heads=n)
+    for od in (order, None) if kind == "window" else (order,):
+        got = capi.attention_heads(rwo, od, atox, bm, N, Q, K, V, float(np.sqrt(d)),
+                                   workspace=scratch(heads))
+        one = [capi.attention_heads(rwo, od, atox, bm, N, *[t[:, h:h + 1] for t in (Q, K, V)],
+                                    float(np.sqrt(d)), workspace=scratch(1)) for h in range(heads)]
+        assert torch.isfinite(got).all()
+        assert torch.equal(got, torch.cat(one, dim=1))
+
+
 # 1025 windows: one more than a whole number of chunks for every number of head groups
 @pytest.mark.parametrize("heads,d", [(1, 32), (3, 64), (4, 64), (8, 32), (2, 128)])
 def test_short_windows(oracle_mod, heads, d):
