@@ -57,7 +57,7 @@ namespace {
 
 constexpr int kRangeMax = 393216;  // columns per bitset pass: 48 KiB of bits + 12 KiB of prefixes
 constexpr int kSortMax = 1024;     // windows up to this many edges are ranked by a per-wave LDS sort
-constexpr int kBinsMax = 960;      // the same on graphs of at most 2^22 nodes (16 waves per CU)
+constexpr int kBinsMax = 960;      // the same on graphs of at most 2^22 nodes (26 waves per CU)
 // TC blocks held in LDS at once by window_fill_kernel: windows with strictly ascending rows (96
 // bytes of LDS per 16x16 block) and windows with repeated or descending columns (96 bytes as
 // well, but a second pass per chunk)
@@ -380,16 +380,17 @@ __device__ __forceinline__ void wave_scatter_in_order(const uint32_t* src, uint3
   }
 }
 
-// LSD radix sort of a wave's n words by the colBits bits above IDX_BITS, in LDS: from src through dst
-// and back; returns the buffer that holds the result. hist: 256 counters.
-template <int IDX_BITS>
-__device__ __forceinline__ uint32_t* wave_radix_sort(uint32_t* src, uint32_t* dst, uint32_t* hist,
-                                                     int n, int colBits, int lane) {
+// LSD radix sort of a wave's n words in `buf` (LDS) by the colBits bits above IDX_BITS: every pass holds
+// the words in registers, G groups of 64 at most, while it scatters them back. hist: 256 counters.
+template <int IDX_BITS, int G>
+__device__ __forceinline__ void wave_radix_sort(uint32_t* buf, uint32_t* hist, int n, int colBits,
+                                                int lane) {
   // Digits: the first pass takes eight bits, the stable passes share the rest evenly (22 column
   // bits: 8 + 7 + 7; 18: 8 + 5 + 5), so that a stable pass spends one ballot per bit it needs.
   const int firstBits = colBits < 8 ? colBits : 8;
   const int restBits = colBits - firstBits;
   const int nStable = (restBits + 7) / 8;
+  const unsigned long long ltMask = (1ull << lane) - 1ull;
   int shift = IDX_BITS;
   for (int pass = 0; pass <= nStable; pass++) {
     const int db = pass == 0 ? firstBits
@@ -397,8 +398,18 @@ __device__ __forceinline__ uint32_t* wave_radix_sort(uint32_t* src, uint32_t* ds
     const unsigned mask = (1u << db) - 1u;
 #pragma unroll
     for (int k = 0; k < 4; k++) hist[lane + 64 * k] = 0;
+    uint32_t key[G];
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      if (64 * u >= n) break;
+      key[u] = buf[min(64 * u + lane, n - 1)];
+    }
     wave_lds_sync();
-    for (int i = lane; i < n; i += 64) atomicAdd(&hist[(src[i] >> shift) & mask], 1u);
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      if (64 * u >= n) break;
+      if (64 * u + lane < n) atomicAdd(&hist[(key[u] >> shift) & mask], 1u);
+    }
     wave_lds_sync();
     {
       // exclusive scan of the 256 counts: lane l owns bins 4l .. 4l+3
@@ -409,34 +420,32 @@ __device__ __forceinline__ uint32_t* wave_radix_sort(uint32_t* src, uint32_t* ds
           make_uint4(excl, excl + c.x, excl + c.x + c.y, excl + c.x + c.y + c.z);
     }
     wave_lds_sync();
-    if (pass == 0) {
-      // The first pass need not be stable: words with the same digit are put in order by the
-      // later passes or name the same column, and equal columns only have to end up next to
-      // each other. A returning LDS atomic hands out the places, a tenth of the instructions
-      // of the in-order scatter below.
-      for (int i = lane; i < n; i += 64) {
-        const uint32_t key = src[i];
-        dst[atomicAdd(&hist[(key >> shift) & mask], 1u)] = key;
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      if (64 * u >= n) break;
+      const bool valid = 64 * u + lane < n;
+      const unsigned dgt = (key[u] >> shift) & mask;
+      if (pass == 0) {
+        // The first pass need not be stable: words with the same digit are put in order by the
+        // later passes or name the same column, and equal columns only have to end up next to
+        // each other. A returning LDS atomic hands out the places, a tenth of the instructions
+        // of the in-order scatter.
+        if (valid) buf[atomicAdd(&hist[dgt], 1u)] = key[u];
+        continue;
       }
-    } else {
-      switch (db) {
-        case 1: wave_scatter_in_order<1>(src, dst, hist, n, shift, lane); break;
-        case 2: wave_scatter_in_order<2>(src, dst, hist, n, shift, lane); break;
-        case 3: wave_scatter_in_order<3>(src, dst, hist, n, shift, lane); break;
-        case 4: wave_scatter_in_order<4>(src, dst, hist, n, shift, lane); break;
-        case 5: wave_scatter_in_order<5>(src, dst, hist, n, shift, lane); break;
-        case 6: wave_scatter_in_order<6>(src, dst, hist, n, shift, lane); break;
-        case 7: wave_scatter_in_order<7>(src, dst, hist, n, shift, lane); break;
-        default: wave_scatter_in_order<8>(src, dst, hist, n, shift, lane); break;
+      unsigned long long peers = __ballot(valid);
+      for (int b = 0; b < db; b++) {
+        const bool bit = (dgt >> b) & 1u;
+        const unsigned long long bal = __ballot(bit);
+        peers &= bit ? bal : ~bal;
       }
+      if (valid) buf[hist[dgt] + __popcll(peers & ltMask)] = key[u];
+      // the last peer advances the digit's position; the wave's LDS operations stay in order
+      if (valid && (peers >> lane) == 1ull) hist[dgt] += __popcll(peers);
     }
     wave_lds_sync();
-    uint32_t* t = src;
-    src = dst;
-    dst = t;
     shift += db;
   }
-  return src;
 }
 
 // Rows of the edges of a window of at most MAX edges, for one wave that walks the edges in groups of
@@ -487,15 +496,15 @@ struct EdgeRows {
 // (communities) is sorted by an LSD radix sort of the column bits, whose stable passes cost a
 // ballot per bit: counting the smaller ones takes as many steps as the fullest bin holds.
 //
-// Bound by the issue of vector instructions (a wave of 400 edges is 7 groups of 64), then by LDS
-// latency: the LDS accesses of four groups are in flight together. Workgroups of one wave, 16 per CU:
-// a workgroup of four kept the LDS of three windows until the longest of them was done (61M edges:
-// 432 instead of 332 us).
+// One LDS buffer: between its passes a window's words are in registers (fifteen groups of 64 at most),
+// so that a pass can scatter into the buffer it has read. 6 KiB and 67 registers: 26 waves per CU, where two
+// buffers allowed 16 (preprocessing of a 61M-edge graph, 149k such windows: 789 -> 745 us; of a
+// 2.8M-edge R-MAT graph: 112 -> 108).
 constexpr int kRankBins = 1024;
 constexpr int kRankCrowd = 24;  // a fuller bin sends the window to the radix sort
 struct alignas(16) RankBinsLds {  // of one wave
   uint32_t hist[kRankBins / 2];
-  uint32_t bufA[kBinsMax], bufB[kBinsMax];
+  uint32_t buf[kBinsMax];
   uint32_t mark[kBinsMax / 32 + 2];
 };
 template <int W>
@@ -505,8 +514,10 @@ __device__ __forceinline__ void rank_window_by_bins(
     int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
     int* __restrict__ error) {
   constexpr int IDX_BITS = 10;
-  constexpr int U = 4;  // groups of 64 edges whose LDS accesses are in flight together
+  constexpr int G = kBinsMax / 64;  // groups of 64 edges
+  constexpr int U = 4;  // groups whose LDS accesses are in flight together where they wait for each other
   static_assert(kBinsMax <= (1 << IDX_BITS), "edge position must fit IDX_BITS");
+  static_assert(kBinsMax % 64 == 0, "whole groups");
   const int lane = threadIdx.x & 63;
   const int r0 = w * 16;
   int rowStart = rowPtr[min(r0 + min(lane, 16), N)];
@@ -521,11 +532,16 @@ __device__ __forceinline__ void rank_window_by_bins(
     if (lane == 0 && queue.counts) queue.add(w, n);
     return;
   }
-  uint32_t* a = lds.bufA;
-  uint32_t* b = lds.bufB;
+  uint32_t* buf = lds.buf;
   uint32_t* hist = lds.hist;
   const unsigned long long leMask = (2ull << lane) - 1ull;
   const int shift = colBits > 10 ? colBits - 10 : 0;
+  uint32_t col[G];  // columns, later (column, position) words, of edges 64 u + lane
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    if (64 * u >= n) break;
+    col[u] = (uint32_t)colIdx[eS + min(64 * u + lane, n - 1)];
+  }
   EdgeRows<kBinsMax> edgeRows;
   edgeRows.init(lds.mark, rowStart, lane);
 #pragma unroll
@@ -534,29 +550,20 @@ __device__ __forceinline__ void rank_window_by_bins(
   wave_lds_sync();
   // ---- rows, and how many edges fall into each bin
   bool bad = false;
-  for (int base = 0; base < n; base += 64 * U) {
-    uint32_t col[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int i = base + 64 * u + lane;
-      col[u] = i < n ? (uint32_t)colIdx[eS + i] : 0u;
+  for (int u = 0; u < G; u++) {
+    if (64 * u >= n) break;
+    const int i = 64 * u + lane;
+    bool starts;
+    const int row = edgeRows.next_group(64 * u, lane, &starts);
+    if (col[u] >= (uint32_t)N) {
+      bad = true;
+      col[u] = 0;
     }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (base + 64 * u >= n) break;
-      const int i = base + 64 * u + lane;
-      bool starts;
-      const int row = edgeRows.next_group(base + 64 * u, lane, &starts);
-      if (i < n) {
-        if (col[u] >= (uint32_t)N) {
-          bad = true;
-          col[u] = 0;
-        }
-        edgeToRow[eS + i] = r0 + row;
-        b[i] = col[u];
-        const uint32_t bin = col[u] >> shift;
-        atomicAdd(&hist[bin >> 1], 1u << ((bin & 1u) * 16u));
-      }
+    const uint32_t bin = col[u] >> shift;
+    if (i < n) {
+      edgeToRow[eS + i] = r0 + row;
+      atomicAdd(&hist[bin >> 1], 1u << ((bin & 1u) * 16u));
     }
   }
   if (bad) *error = 1;
@@ -590,83 +597,91 @@ __device__ __forceinline__ void rank_window_by_bins(
     }
   }
   wave_lds_sync();
-  const uint32_t* sorted = b;
   if (!crowded) {
     // ---- into the bins; afterwards hist[bin] is where the bin ends
-    for (int base = 0; base < n; base += 64 * U) {
-      uint32_t col[U], old[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) col[u] = b[min(base + 64 * u + lane, n - 1)];
+    for (int u0 = 0; u0 < G; u0 += U) {
+      if (64 * u0 >= n) break;
+      uint32_t old[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
+      for (int u = u0; u < min(u0 + U, G); u++) {
         const uint32_t bin = col[u] >> shift;
-        if (base + 64 * u + lane < n)
-          old[u] = atomicAdd(&hist[bin >> 1], 1u << ((bin & 1u) * 16u));
+        if (64 * u + lane < n) old[u - u0] = atomicAdd(&hist[bin >> 1], 1u << ((bin & 1u) * 16u));
       }
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int i = base + 64 * u + lane;
-        const uint32_t bin = col[u] >> shift;
-        if (i < n)
-          a[(old[u] >> ((bin & 1u) * 16u)) & 0xFFFFu] = (col[u] << IDX_BITS) | (uint32_t)i;
+      for (int u = u0; u < min(u0 + U, G); u++) {
+        const int i = 64 * u + lane;
+        const uint32_t half = ((col[u] >> shift) & 1u) * 16u;
+        if (i < n) buf[(old[u - u0] >> half) & 0xFFFFu] = (col[u] << IDX_BITS) | (uint32_t)i;
       }
     }
     wave_lds_sync();
     // ---- each edge's place inside its bin
     const uint16_t* binEnd = reinterpret_cast<const uint16_t*>(hist);
-    for (int base = 0; base < n; base += 64 * U) {
-      uint32_t key[U];
+    uint32_t at[G];
+#pragma unroll
+    for (int u0 = 0; u0 < G; u0 += U) {
+      if (64 * u0 >= n) break;
       int end[U], q[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) key[u] = a[min(base + 64 * u + lane, n - 1)];
+      for (int u = u0; u < min(u0 + U, G); u++) col[u] = buf[min(64 * u + lane, n - 1)];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const uint32_t bin = key[u] >> (IDX_BITS + shift);
-        end[u] = binEnd[bin];
-        q[u] = bin == 0u ? 0 : (int)binEnd[max(bin, 1u) - 1u];
+      for (int u = u0; u < min(u0 + U, G); u++) {
+        const uint32_t bin = col[u] >> (IDX_BITS + shift);
+        end[u - u0] = binEnd[bin];
+        q[u - u0] = bin == 0u ? 0 : (int)binEnd[max(bin, 1u) - 1u];
       }
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (base + 64 * u >= n) break;
-        int at = q[u];
-        if (end[u] - q[u] > 1)
-          for (int k = q[u]; k < end[u]; k++) at += a[k] < key[u] ? 1 : 0;
-        if (base + 64 * u + lane < n) b[at] = key[u];
+      for (int u = u0; u < min(u0 + U, G); u++) {
+        int place = q[u - u0];
+        if (end[u - u0] - q[u - u0] > 1)
+          for (int k = q[u - u0]; k < end[u - u0]; k++) place += buf[k] < col[u] ? 1 : 0;
+        at[u] = (uint32_t)place;
       }
     }
-  } else {
-    for (int i = lane; i < n; i += 64) a[i] = (b[i] << IDX_BITS) | (uint32_t)i;
     wave_lds_sync();
-    sorted = wave_radix_sort<IDX_BITS>(a, b, hist, n, colBits, lane);
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      if (64 * u >= n) break;
+      if (64 * u + lane < n) buf[at[u]] = col[u];
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      if (64 * u >= n) break;
+      const int i = 64 * u + lane;
+      if (i < n) buf[i] = (col[u] << IDX_BITS) | (uint32_t)i;
+    }
+    wave_lds_sync();
+    wave_radix_sort<IDX_BITS, G>(buf, hist, n, colBits, lane);
   }
   wave_lds_sync();
   // ---- ranks of the distinct columns, collected in edge order and written as whole lines
-  uint32_t* rankOf = sorted == b ? a : b;
-  int nUniq = 0, lastCol = -1;
-  for (int base = 0; base < n; base += 64 * U) {
-    uint32_t key[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) key[u] = sorted[min(base + 64 * u + lane, n - 1)];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (base + 64 * u >= n) break;
-      const bool valid = base + 64 * u + lane < n;
-      const int col = (int)(key[u] >> IDX_BITS);
-      const int left = __builtin_amdgcn_update_dpp(lastCol, col, 0x138, 0xf, 0xf, false);
-      lastCol = __builtin_amdgcn_readlane(col, 63);
-      const unsigned long long bal = __ballot(valid && left != col);
-      if (valid)
-        rankOf[key[u] & ((1u << IDX_BITS) - 1u)] = (uint32_t)(nUniq + __popcll(bal & leMask) - 1);
-      nUniq += __popcll(bal);
-    }
+  for (int u = 0; u < G; u++) {
+    if (64 * u >= n) break;
+    col[u] = buf[min(64 * u + lane, n - 1)];
   }
   wave_lds_sync();
-  for (int base = 0; base < n; base += 64 * U) {
+  int nUniq = 0, lastCol = -1;
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int i = base + 64 * u + lane;
-      if (i < n) edgeToColumn[eS + i] = (int)rankOf[i];
-    }
+  for (int u = 0; u < G; u++) {
+    if (64 * u >= n) break;
+    const bool valid = 64 * u + lane < n;
+    const int c = (int)(col[u] >> IDX_BITS);
+    const int left = __builtin_amdgcn_update_dpp(lastCol, c, 0x138, 0xf, 0xf, false);
+    lastCol = __builtin_amdgcn_readlane(c, 63);
+    const unsigned long long bal = __ballot(valid && left != c);
+    if (valid)
+      buf[col[u] & ((1u << IDX_BITS) - 1u)] = (uint32_t)(nUniq + __popcll(bal & leMask) - 1);
+    nUniq += __popcll(bal);
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    if (64 * u >= n) break;
+    const int i = 64 * u + lane;
+    if (i < n) edgeToColumn[eS + i] = (int)buf[i];
   }
   if (lane == 0) blockPartition[w] = (nUniq + W - 1) / W;
 }
