@@ -381,7 +381,8 @@ __device__ __forceinline__ void wave_scatter_in_order(const uint32_t* src, uint3
 }
 
 // LSD radix sort of a wave's n words in `buf` (LDS) by the colBits bits above IDX_BITS: every pass holds
-// the words in registers, G groups of 64 at most, while it scatters them back. hist: 256 counters.
+// the words in registers, G groups of 64 at most, while it scatters them back. hist: 256 counters. buf: 64 G
+// words.
 template <int IDX_BITS, int G>
 __device__ __forceinline__ void wave_radix_sort(uint32_t* buf, uint32_t* hist, int n, int colBits,
                                                 int lane) {
@@ -402,13 +403,13 @@ __device__ __forceinline__ void wave_radix_sort(uint32_t* buf, uint32_t* hist, i
 #pragma unroll
     for (int u = 0; u < G; u++) {
       if (64 * u >= n) break;
-      key[u] = buf[min(64 * u + lane, n - 1)];
+      key[u] = buf[64 * u + lane];
     }
     wave_lds_sync();
 #pragma unroll
     for (int u = 0; u < G; u++) {
       if (64 * u >= n) break;
-      if (64 * u + lane < n) atomicAdd(&hist[(key[u] >> shift) & mask], 1u);
+      if (lane < n - 64 * u) atomicAdd(&hist[(key[u] >> shift) & mask], 1u);
     }
     wave_lds_sync();
     {
@@ -423,7 +424,7 @@ __device__ __forceinline__ void wave_radix_sort(uint32_t* buf, uint32_t* hist, i
 #pragma unroll
     for (int u = 0; u < G; u++) {
       if (64 * u >= n) break;
-      const bool valid = 64 * u + lane < n;
+      const bool valid = lane < n - 64 * u;
       const unsigned dgt = (key[u] >> shift) & mask;
       if (pass == 0) {
         // The first pass need not be stable: words with the same digit are put in order by the
@@ -487,40 +488,340 @@ struct EdgeRows {
   }
 };
 
+// EdgeRows where only the rows are asked for: bit i - 1 is set where a row that is not empty starts at edge
+// i > 0, so that the set bits below a lane are the rows that started before its edge, without the first one.
+template <int MAX>
+struct RowMarks {
+  uint32_t words;  // lane l holds word l of the marks
+  unsigned long long names;
+  int rows;
+
+  // rowStart, mark: as for EdgeRows
+  __device__ __forceinline__ void init(uint32_t* mark, int rowStart, int lane) {
+    static_assert(MAX % 64 == 0 && MAX / 32 + 2 <= 64, "whole groups, a word per lane");
+    if (lane < MAX / 32 + 2) mark[lane] = 0u;
+    wave_lds_sync();
+    const int next = __shfl_down(rowStart, 1);
+    const unsigned filled = (unsigned)__ballot(lane < 16 && next > rowStart);
+    if (lane < 16 && ((filled >> lane) & 1u)) {
+      const int k = __popc(filled & ((1u << lane) - 1u));
+      if (k > 0) atomicOr(&mark[(rowStart - 1) >> 5], 1u << ((rowStart - 1) & 31));
+      atomicOr(&mark[MAX / 32 + (k >> 3)], (uint32_t)lane << (4 * (k & 7)));
+    }
+    wave_lds_sync();
+    words = mark[min(lane, MAX / 32 + 1)];
+    names = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)words, MAX / 32) |
+            (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)words, MAX / 32 + 1) << 32;
+    rows = 0;
+  }
+  // row of this lane's edge in group u of 64 (groups in order, each once)
+  __device__ __forceinline__ int next_group(int u) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)words, 2 * u);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)words, 2 * u + 1);
+    const int k = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, rows));
+    rows += __popc(lo) + __popc(hi);
+    return (int)(names >> (4 * k)) & 15;
+  }
+};
+
 // The same job for graphs of at most 2^22 nodes, where a column id and the edge's position in the
 // window (< kBinsMax) fit one 32-bit word. The columns' top ten bits spread the window's
 // edges over 1024 bins (two 16-bit counters per word; one counting pass, one that hands out
 // places), after which an edge shares its bin with one or two others and finds its place by
-// counting the smaller ones. The sorted words carry the edge positions along, so that the rank of
+// comparing itself with its neighbours. The sorted words carry the edge positions along, so that the rank of
 // every distinct column goes straight back to its edges. A window whose columns crowd into few bins
-// (communities) is sorted by an LSD radix sort of the column bits, whose stable passes cost a
-// ballot per bit: counting the smaller ones takes as many steps as the fullest bin holds.
+// (communities) is binned again, more finely around its middle; only one that crowds there too takes an LSD
+// radix sort of the column bits, whose stable passes cost a ballot per bit.
 //
-// One LDS buffer: between its passes a window's words are in registers (fifteen groups of 64 at most),
-// so that a pass can scatter into the buffer it has read. 6 KiB and 67 registers: 26 waves per CU, where two
-// buffers allowed 16 (preprocessing of a 61M-edge graph, 149k such windows: 789 -> 745 us; of a
-// 2.8M-edge R-MAT graph: 112 -> 108).
+// Bound by the issue of vector instructions: 885 of them for a window of 400 edges when every group of 64
+// edges guarded its lanes, looked up its bins' ends and walked them. Groups that are known to be whole (by the
+// window's size, six sizes) need no guards and immediate offsets, and the neighbours need no bin's ends. One
+// LDS buffer: between its passes a window's words are in registers, so that a pass can scatter into the
+// buffer it has read; 6 KiB and 71 registers, 26 waves per CU, where two buffers allowed 16. Preprocessing of
+// a 61M-edge graph (149k such windows) 789 -> 646 us, of a 2.8M-edge R-MAT graph 112 -> 104, of community
+// graphs of 15k to 200k nodes 53 -> 52 to 209 -> 163.
 constexpr int kRankBins = 1024;
-constexpr int kRankCrowd = 24;  // a fuller bin sends the window to the radix sort
+// A fuller bin makes a window a crowded one. At 12 R-MAT graphs, whose hub columns repeat up to 16 times, take
+// that route: 2.8M edges 104 -> 121 us, 61M edges 646 -> 840; at 36 and 48 communities walk fuller bins: 60k
+// nodes 58 -> 59 and 60.
+constexpr int kRankCrowd = 24;
+constexpr int kRankNear = 3;    // neighbours on each side that every word is compared with
+constexpr int kRankStep = 4;    // ... and how many more at a time where bins are fuller
+constexpr int kRankPad = 32;
+static_assert(kRankPad >= kRankCrowd + kRankStep, "neighbours of the first and the last word");
 struct alignas(16) RankBinsLds {  // of one wave
-  uint32_t hist[kRankBins / 2];
-  uint32_t buf[kBinsMax];
+  uint32_t hist[kRankBins / 2];  // word i: bin i in the low half, bin 512 + i in the high one
+  // the window's words from kRankPad on: words below them all in front, words above them all behind the last
+  uint32_t words[kRankPad + kBinsMax + kRankPad];
   uint32_t mark[kBinsMax / 32 + 2];
 };
+
+constexpr int kRankIdxBits = 10;
+static_assert(kBinsMax <= (1 << kRankIdxBits), "edge position must fit kRankIdxBits");
+
+// Ranks of the distinct columns of n sorted words, collected in edge order and written as whole lines. Here and
+// in rank_window_groups 64 (G - P) < n <= 64 G: the first G - P groups of 64 edges are whole, and only the
+// others look at the edge's number.
+template <int W, int G, int P>
+__device__ __forceinline__ void rank_sorted_words(int w, uint32_t* buf, int n, int lane,
+                                                  int32_t* __restrict__ blockPartition,
+                                                  int32_t* __restrict__ ranks) {
+  uint32_t word[G];
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    if (u >= G - P && 64 * u >= n) continue;
+    word[u] = buf[64 * u + lane];
+  }
+  wave_lds_sync();
+  int nUniq = 0;
+  uint32_t last = ~(uint32_t)__builtin_amdgcn_readfirstlane((int)word[0]);
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    if (u >= G - P && 64 * u >= n) continue;
+    const bool valid = u < G - P || lane < n - 64 * u;
+    const uint32_t left =
+        (uint32_t)__builtin_amdgcn_update_dpp((int)last, (int)word[u], 0x138, 0xf, 0xf, false);
+    last = (uint32_t)__builtin_amdgcn_readlane((int)word[u], 63);
+    const bool first = (left ^ word[u]) >= (1u << kRankIdxBits) && valid;
+    const unsigned long long firsts = __ballot(first);
+    const int below = (int)__builtin_amdgcn_mbcnt_hi(
+        (unsigned)(firsts >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)firsts, nUniq));
+    if (valid) buf[word[u] & ((1u << kRankIdxBits) - 1u)] = (uint32_t)(below - (first ? 0 : 1));
+    nUniq += __popcll(firsts);
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    if (u >= G - P && 64 * u >= n) continue;
+    if (u < G - P || lane < n - 64 * u) ranks[64 * u + lane] = (int)buf[64 * u + lane];
+  }
+  if (lane == 0) blockPartition[w] = (nUniq + W - 1) / W;
+}
+
+// Counts of the bins into where each starts; whether some bin holds more than kRankCrowd. Lane l owns words
+// 8 l .. 8 l + 7, both halves at once: no sum reaches 2^16.
+__device__ __forceinline__ bool rank_bin_starts(uint32_t* hist, int lane) {
+  uint4* h = reinterpret_cast<uint4*>(hist) + 2 * lane;
+  const uint4 x = h[0], y = h[1];
+  uint32_t v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+  uint32_t total = 0, full = 0;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    full |= v[k] + 0x10001u * (0x7FFFu - kRankCrowd);  // bit 15 of a half: more than kRankCrowd
+    total += v[k];
+  }
+  const uint32_t incl = wave_inclusive_scan(total, lane);
+  uint32_t run = incl - total + ((uint32_t)__builtin_amdgcn_readlane((int)incl, 63) << 16);
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const uint32_t start = run;
+    run += v[k];
+    v[k] = start;
+  }
+  h[0] = make_uint4(v[0], v[1], v[2], v[3]);
+  h[1] = make_uint4(v[4], v[5], v[6], v[7]);
+  const bool crowded = __ballot((full & 0x80008000u) != 0u) != 0ull;
+  wave_lds_sync();
+  return crowded;
+}
+
+// Place of word i of the words that are in their bins' order: inside its bin, later ones that are smaller move
+// it up, earlier ones that are larger move it down, and words of other bins do neither. Three neighbours on
+// each side are enough for bins of four; a group with a fuller bin goes on until no lane's next neighbour is
+// of its bin. sameBin: words of one bin differ by less in their exclusive or. WHOLE: the group and the one
+// before it are all words of the window, and the one behind it is not its end.
+template <bool WHOLE>
+__device__ __forceinline__ int rank_place(const uint32_t* buf, int u, int lane, int n, uint32_t word,
+                                          uint32_t sameBin) {
+  uint32_t up = 0, down = 0;
+  int place = 64 * u + lane;
+  const uint32_t* at = buf + place;
+#pragma unroll
+  for (int k = 1; k <= kRankNear; k++) {
+    up = at[k];
+    down = at[-k];
+    place += up < word ? 1 : 0;
+    place -= down > word ? 1 : 0;
+  }
+  for (int k = kRankNear; k < kRankCrowd; k += kRankStep) {
+    bool more = (up ^ word) < sameBin || (down ^ word) < sameBin;
+    if constexpr (!WHOLE)
+      more = ((up ^ word) < sameBin && lane < n - 64 * u - k) ||
+             ((down ^ word) < sameBin && lane >= k - 64 * u && lane < n - 64 * u);
+    if (__ballot(more) == 0ull) break;
+#pragma unroll
+    for (int j = 1; j <= kRankStep; j++) {
+      up = at[k + j];
+      down = at[-k - j];
+      place += up < word ? 1 : 0;
+      place -= down > word ? 1 : 0;
+    }
+  }
+  return place;
+}
+
+// False where columns crowd into few bins: the rows are written, the unsorted words are in lds.words and the
+// rest is left to the caller.
+template <int W, int G, int P>
+__device__ __forceinline__ bool rank_window_groups(
+    int w, const int32_t* __restrict__ cols, int n, int rowStart, int N, int colBits, RankBinsLds& lds,
+    int32_t* __restrict__ blockPartition, int32_t* __restrict__ ranks, int32_t* __restrict__ rows,
+    int* __restrict__ error) {
+  const int lane = threadIdx.x & 63;
+  const int shift = colBits > 10 ? colBits - 10 : 0;
+  uint32_t* buf = lds.words + kRankPad;
+  uint32_t* hist = lds.hist;
+  uint32_t col[G];  // columns, later (column, position) words, of edges 64 u + lane
+#pragma unroll
+  for (int u = 0; u < G; u++)
+    col[u] = (uint32_t)cols[u < G - P ? 64 * u + lane : min(64 * u + lane, n - 1)];
+  auto valid = [&](int u) { return u < G - P || lane < n - 64 * u; };
+  RowMarks<kBinsMax> marks;
+  marks.init(lds.mark, rowStart, lane);
+#pragma unroll
+  for (int k = 0; k < kRankBins / 2 / 256; k++)
+    reinterpret_cast<uint4*>(hist)[lane + 64 * k] = make_uint4(0, 0, 0, 0);
+  if (lane < kRankPad) {
+    lds.words[lane] = 0u;
+    buf[n + lane] = 0xFFFFFFFFu;
+  }
+  wave_lds_sync();
+  // ---- rows
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    const int row = marks.next_group(u);
+    if (valid(u)) rows[64 * u + lane] = w * 16 + row;
+  }
+  // ---- how many edges fall into each bin
+  uint32_t most = 0;
+#pragma unroll
+  for (int u = 0; u < G; u++) most = max(most, col[u]);
+  if (__ballot(most >= (uint32_t)N) != 0ull) {
+    *error = 1;
+#pragma unroll
+    for (int u = 0; u < G; u++) col[u] = col[u] < (uint32_t)N ? col[u] : 0u;
+  }
+  const uint32_t upper = 512u << shift;  // first column of the bins in high halves
+#pragma unroll
+  for (int u = 0; u < G; u++)
+    if (valid(u)) atomicAdd(&hist[(col[u] >> shift) & 511u], col[u] < upper ? 1u : 0x10000u);
+  wave_lds_sync();
+  const bool crowded = rank_bin_starts(hist, lane);
+  if (crowded) {
+#pragma unroll
+    for (int u = 0; u < G; u++)
+      if (valid(u)) buf[64 * u + lane] = (col[u] << kRankIdxBits) | (uint32_t)(64 * u + lane);
+    wave_lds_sync();
+    return false;
+  }
+  // ---- into the bins
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    const uint32_t half = col[u] < upper ? 0u : 16u;
+    if (valid(u)) {
+      const uint32_t old = atomicAdd(&hist[(col[u] >> shift) & 511u], 1u << half);
+      buf[(old >> half) & 0xFFFFu] = (col[u] << kRankIdxBits) | (uint32_t)(64 * u + lane);
+    }
+  }
+  wave_lds_sync();
+  // ---- from the bins' order to the columns'
+  const uint32_t sameBin = 1u << (kRankIdxBits + shift);
+  uint32_t at[G];
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    col[u] = buf[64 * u + lane];
+    at[u] = (uint32_t)(u > 0 && u < G - P - 1 ? rank_place<true>(buf, u, lane, n, col[u], sameBin)
+                                              : rank_place<false>(buf, u, lane, n, col[u], sameBin));
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int u = 0; u < G; u++)
+    if (valid(u)) buf[at[u]] = col[u];
+  wave_lds_sync();
+  rank_sorted_words<W, G, P>(w, buf, n, lane, blockPartition, ranks);
+  return true;
+}
+
+// The rest of a window whose columns crowd into few bins, as those of a community do: half of the bins are spread
+// over the columns around the window's middle edge (512 of them, or four bins' worth), the others over
+// what lies below and above. Columns that crowd there as well take the radix sort.
+template <int W, int G>
+__device__ __forceinline__ void rank_crowded_window(int w, int n, int colBits, RankBinsLds& lds, int lane,
+                                                    int32_t* __restrict__ blockPartition,
+                                                    int32_t* __restrict__ ranks) {
+  const int shift = colBits > 10 ? colBits - 10 : 0;
+  uint32_t* buf = lds.words + kRankPad;
+  uint32_t* hist = lds.hist;
+  // the last bin that starts at or before the middle edge
+  uint32_t bin = 0;
+#pragma unroll
+  for (int k = 0; k < kRankBins / 128; k++) {
+    const uint32_t v = hist[lane + 64 * k];
+    bin += __popcll(__ballot((v & 0xFFFFu) <= (uint32_t)n / 2)) + __popcll(__ballot((v >> 16) <= (uint32_t)n / 2));
+  }
+  bin -= 1u;
+  const int fine = shift > 7 ? shift - 7 : 0;
+  const uint32_t span = 512u << fine;
+  const uint32_t middle = (2u * bin + 1u) << shift >> 1;
+  const uint32_t from = (middle > span / 2 ? middle - span / 2 : 0u) >> fine << fine;
+  wave_lds_sync();
+#pragma unroll
+  for (int k = 0; k < kRankBins / 2 / 256; k++)
+    reinterpret_cast<uint4*>(hist)[lane + 64 * k] = make_uint4(0, 0, 0, 0);
+  wave_lds_sync();
+  // bins 0..255: below, 256..767: around the middle, 768..1023: above
+  auto bin_of = [&](uint32_t c) {
+    const uint32_t coarse = (c >> (shift + 2)) + (c < from ? 0u : 768u);
+    return c - from < span ? 256u + ((c - from) >> fine) : coarse;
+  };
+  uint32_t word[G], at[G];
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    if (64 * u >= n) continue;
+    word[u] = buf[64 * u + lane];
+    const uint32_t b = bin_of(word[u] >> kRankIdxBits);
+    if (lane < n - 64 * u) atomicAdd(&hist[b & 511u], b < 512u ? 1u : 0x10000u);
+  }
+  wave_lds_sync();
+  if (rank_bin_starts(hist, lane)) {
+    wave_radix_sort<kRankIdxBits, G>(buf, hist, n, colBits, lane);
+  } else {
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      if (64 * u >= n) continue;
+      const uint32_t b = bin_of(word[u] >> kRankIdxBits);
+      const uint32_t half = b < 512u ? 0u : 16u;
+      if (lane < n - 64 * u)
+        buf[(atomicAdd(&hist[b & 511u], 1u << half) >> half) & 0xFFFFu] = word[u];
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      if (64 * u >= n) continue;
+      word[u] = buf[64 * u + lane];
+      const bool middleBin = (word[u] >> kRankIdxBits) - from < span;
+      const uint32_t sameBin = 1u << (kRankIdxBits + (middleBin ? fine : shift + 2));
+      at[u] = (uint32_t)rank_place<false>(buf, u, lane, n, word[u], sameBin);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      if (64 * u >= n) continue;
+      if (lane < n - 64 * u) buf[at[u]] = word[u];
+    }
+    wave_lds_sync();
+  }
+  rank_sorted_words<W, G, G>(w, buf, n, lane, blockPartition, ranks);
+}
+
 template <int W>
 __device__ __forceinline__ void rank_window_by_bins(
     int w, const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N,
     int colBits, const LongQueue& queue, RankBinsLds& lds, int32_t* __restrict__ blockPartition,
     int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
     int* __restrict__ error) {
-  constexpr int IDX_BITS = 10;
-  constexpr int G = kBinsMax / 64;  // groups of 64 edges
-  constexpr int U = 4;  // groups whose LDS accesses are in flight together where they wait for each other
-  static_assert(kBinsMax <= (1 << IDX_BITS), "edge position must fit IDX_BITS");
-  static_assert(kBinsMax % 64 == 0, "whole groups");
   const int lane = threadIdx.x & 63;
-  const int r0 = w * 16;
-  int rowStart = rowPtr[min(r0 + min(lane, 16), N)];
+  int rowStart = rowPtr[min(w * 16 + min(lane, 16), N)];
   const int eS = __builtin_amdgcn_readlane(rowStart, 0);
   const int n = __builtin_amdgcn_readlane(rowStart, 16) - eS;
   rowStart -= eS;
@@ -532,158 +833,30 @@ __device__ __forceinline__ void rank_window_by_bins(
     if (lane == 0 && queue.counts) queue.add(w, n);
     return;
   }
-  uint32_t* buf = lds.buf;
-  uint32_t* hist = lds.hist;
-  const unsigned long long leMask = (2ull << lane) - 1ull;
-  const int shift = colBits > 10 ? colBits - 10 : 0;
-  uint32_t col[G];  // columns, later (column, position) words, of edges 64 u + lane
-#pragma unroll
-  for (int u = 0; u < G; u++) {
-    if (64 * u >= n) break;
-    col[u] = (uint32_t)colIdx[eS + min(64 * u + lane, n - 1)];
-  }
-  EdgeRows<kBinsMax> edgeRows;
-  edgeRows.init(lds.mark, rowStart, lane);
-#pragma unroll
-  for (int k = 0; k < kRankBins / 2 / 256; k++)
-    reinterpret_cast<uint4*>(hist)[lane + 64 * k] = make_uint4(0, 0, 0, 0);
-  wave_lds_sync();
-  // ---- rows, and how many edges fall into each bin
-  bool bad = false;
-#pragma unroll
-  for (int u = 0; u < G; u++) {
-    if (64 * u >= n) break;
-    const int i = 64 * u + lane;
-    bool starts;
-    const int row = edgeRows.next_group(64 * u, lane, &starts);
-    if (col[u] >= (uint32_t)N) {
-      bad = true;
-      col[u] = 0;
-    }
-    const uint32_t bin = col[u] >> shift;
-    if (i < n) {
-      edgeToRow[eS + i] = r0 + row;
-      atomicAdd(&hist[bin >> 1], 1u << ((bin & 1u) * 16u));
-    }
-  }
-  if (bad) *error = 1;
-  wave_lds_sync();
-  // ---- where each bin starts: lane l owns bins 16 l .. 16 l + 15
-  bool crowded;
-  {
-    uint4* h = reinterpret_cast<uint4*>(hist) + 2 * lane;
-    const uint4 x = h[0], y = h[1];
-    uint32_t v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-    // both counters of a word at once: no sum reaches 2^16
-    uint32_t most = 0, pairs = 0;
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      pairs += v[k];
-      most |= v[k] + 0x10001u * (0x7FFFu - kRankCrowd);  // bit 15 of a half: more than kRankCrowd
-    }
-    crowded = __ballot((most & 0x80008000u) != 0u) != 0ull;
-    const uint32_t total = (pairs & 0xFFFFu) + (pairs >> 16);
-    uint32_t run = wave_inclusive_scan(total, lane) - total;
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const uint32_t lo = run + (v[k] & 0xFFFFu);
-      const uint32_t start = run | (lo << 16);
-      run = lo + (v[k] >> 16);
-      v[k] = start;
-    }
-    if (!crowded) {
-      h[0] = make_uint4(v[0], v[1], v[2], v[3]);
-      h[1] = make_uint4(v[4], v[5], v[6], v[7]);
-    }
-  }
-  wave_lds_sync();
-  if (!crowded) {
-    // ---- into the bins; afterwards hist[bin] is where the bin ends
-#pragma unroll
-    for (int u0 = 0; u0 < G; u0 += U) {
-      if (64 * u0 >= n) break;
-      uint32_t old[U];
-#pragma unroll
-      for (int u = u0; u < min(u0 + U, G); u++) {
-        const uint32_t bin = col[u] >> shift;
-        if (64 * u + lane < n) old[u - u0] = atomicAdd(&hist[bin >> 1], 1u << ((bin & 1u) * 16u));
-      }
-#pragma unroll
-      for (int u = u0; u < min(u0 + U, G); u++) {
-        const int i = 64 * u + lane;
-        const uint32_t half = ((col[u] >> shift) & 1u) * 16u;
-        if (i < n) buf[(old[u - u0] >> half) & 0xFFFFu] = (col[u] << IDX_BITS) | (uint32_t)i;
-      }
-    }
-    wave_lds_sync();
-    // ---- each edge's place inside its bin
-    const uint16_t* binEnd = reinterpret_cast<const uint16_t*>(hist);
-    uint32_t at[G];
-#pragma unroll
-    for (int u0 = 0; u0 < G; u0 += U) {
-      if (64 * u0 >= n) break;
-      int end[U], q[U];
-#pragma unroll
-      for (int u = u0; u < min(u0 + U, G); u++) col[u] = buf[min(64 * u + lane, n - 1)];
-#pragma unroll
-      for (int u = u0; u < min(u0 + U, G); u++) {
-        const uint32_t bin = col[u] >> (IDX_BITS + shift);
-        end[u - u0] = binEnd[bin];
-        q[u - u0] = bin == 0u ? 0 : (int)binEnd[max(bin, 1u) - 1u];
-      }
-#pragma unroll
-      for (int u = u0; u < min(u0 + U, G); u++) {
-        int place = q[u - u0];
-        if (end[u - u0] - q[u - u0] > 1)
-          for (int k = q[u - u0]; k < end[u - u0]; k++) place += buf[k] < col[u] ? 1 : 0;
-        at[u] = (uint32_t)place;
-      }
-    }
-    wave_lds_sync();
-#pragma unroll
-    for (int u = 0; u < G; u++) {
-      if (64 * u >= n) break;
-      if (64 * u + lane < n) buf[at[u]] = col[u];
-    }
+  const int32_t* cols = colIdx + eS;
+  int32_t *ranks = edgeToColumn + eS, *rows = edgeToRow + eS;
+  bool done;
+#define F3S_RANK_GROUPS(G, P)                                                                       \
+  rank_window_groups<W, G, P>(w, cols, n, rowStart, N, colBits, lds, blockPartition, ranks, rows, error)
+  if (n <= 64 * 2) {
+    done = F3S_RANK_GROUPS(2, 2);
+  } else if (n <= 64 * 4) {
+    done = F3S_RANK_GROUPS(4, 2);
+  } else if (n <= 64 * 6) {
+    done = F3S_RANK_GROUPS(6, 2);
+  } else if (n <= 64 * 8) {
+    done = F3S_RANK_GROUPS(8, 2);
+  } else if (n <= 64 * 11) {
+    done = F3S_RANK_GROUPS(11, 3);
   } else {
-#pragma unroll
-    for (int u = 0; u < G; u++) {
-      if (64 * u >= n) break;
-      const int i = 64 * u + lane;
-      if (i < n) buf[i] = (col[u] << IDX_BITS) | (uint32_t)i;
-    }
-    wave_lds_sync();
-    wave_radix_sort<IDX_BITS, G>(buf, hist, n, colBits, lane);
+    done = F3S_RANK_GROUPS(15, 4);
   }
-  wave_lds_sync();
-  // ---- ranks of the distinct columns, collected in edge order and written as whole lines
-#pragma unroll
-  for (int u = 0; u < G; u++) {
-    if (64 * u >= n) break;
-    col[u] = buf[min(64 * u + lane, n - 1)];
-  }
-  wave_lds_sync();
-  int nUniq = 0, lastCol = -1;
-#pragma unroll
-  for (int u = 0; u < G; u++) {
-    if (64 * u >= n) break;
-    const bool valid = 64 * u + lane < n;
-    const int c = (int)(col[u] >> IDX_BITS);
-    const int left = __builtin_amdgcn_update_dpp(lastCol, c, 0x138, 0xf, 0xf, false);
-    lastCol = __builtin_amdgcn_readlane(c, 63);
-    const unsigned long long bal = __ballot(valid && left != c);
-    if (valid)
-      buf[col[u] & ((1u << IDX_BITS) - 1u)] = (uint32_t)(nUniq + __popcll(bal & leMask) - 1);
-    nUniq += __popcll(bal);
-  }
-  wave_lds_sync();
-#pragma unroll
-  for (int u = 0; u < G; u++) {
-    if (64 * u >= n) break;
-    const int i = 64 * u + lane;
-    if (i < n) edgeToColumn[eS + i] = (int)buf[i];
-  }
-  if (lane == 0) blockPartition[w] = (nUniq + W - 1) / W;
+#undef F3S_RANK_GROUPS
+  if (done) return;
+  if (n <= 64 * 4)
+    rank_crowded_window<W, 4>(w, n, colBits, lds, lane, blockPartition, ranks);
+  else
+    rank_crowded_window<W, kBinsMax / 64>(w, n, colBits, lds, lane, blockPartition, ranks);
 }
 template <int W>
 __global__ __launch_bounds__(64) void window_rank_bins_kernel(

@@ -97,6 +97,51 @@ def test_window_counts(oracle_mod, nRW, edges, wide, W):
         assert np.array_equal(bm, want["tcbBitMap"]), two_phase
 
 
+# A window whose columns crowd into few of its bins is binned again around its middle edge, and sorted where
+# that crowds as well. Communities at both ends of the columns and in the middle, two far apart, one column
+# in many edges, bins filled to the limit of 24 and beyond; the last column of 2^22 is a word of ones
+@pytest.mark.parametrize("N", [900, 15_000, 400_003, 1 << 22])
+def test_crowded_windows(oracle_mod, N):
+    from fused3s_amd import capi
+    print("case crowded windows N=%d" % N, flush=True)
+    rng = np.random.default_rng(N)
+
+    def around(at, n, width):
+        at = min(max(0, at), N - width)
+        return at + rng.integers(0, width, n)
+
+    bits = max(1, (N - 1).bit_length() - 10)
+    windows = []
+    for n in (25, 64, 65, 128, 129, 250, 256, 257, 500, 704, 705, 960):
+        width = min(N, 200 + n // 4)
+        for at in (0, N // 2, N - width):
+            windows.append(around(at, n, width))                                  # one community
+            windows.append(np.where(rng.random(n) < 0.15, rng.integers(0, N, n), around(at, n, width)))
+        windows.append(np.where(rng.random(n) < 0.5, around(0, n, width), around(N - width, n, width)))
+        windows.append(np.full(n, N - 1))                                         # sorted after both attempts
+        windows.append(np.where(rng.random(n) < 0.3, N - 1, rng.integers(0, N, n)))
+        for k in (23, 24, 25):                                                    # bins of just that many edges
+            lo = (N // 3 >> bits) << bits
+            spread = rng.integers(0, N, n)
+            spread[:min(n, k)] = lo + np.arange(min(n, k)) % (1 << bits)
+            windows.append(spread)
+    degree = np.zeros(N, np.int64)
+    columns = []
+    for w, cols in enumerate(windows[:(N + 15) // 16]):
+        rows = np.sort(rng.integers(0, 16, len(cols)))
+        rows = np.minimum(rows, N - 1 - 16 * w)
+        order = np.lexsort((cols, rows)) if w % 4 else np.argsort(rows, kind="stable")
+        degree[16 * w:16 * w + 16] += np.bincount(rows, minlength=16)[:min(16, N - 16 * w)]
+        columns.append(cols[order])
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(degree)
+    colIdx = np.concatenate(columns).astype(np.int32)
+    want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, 16)
+    got = capi.preprocess(torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda(), N, 16, 16)
+    for k in KEYS:
+        assert np.array_equal(got[k].cpu().numpy(), want[k]), k
+
+
 def split_columns(rng, cols, lengths):
     """16 ascending rows of the given lengths over `cols`, which together name every one of them."""
     cols = np.sort(cols)
