@@ -992,17 +992,15 @@ __global__ __launch_bounds__(TB) void window_rank_kernel(
 // first longGroups workgroups look for the windows of more than kBinsMax edges and take one at a
 // time with all of their waves, each wave of the others takes one window. One launch after the other
 // meant that everything waited for the longest window twice (169k-node R-MAT graph, windows of up to
-// 12 500 edges: 29 + 23 us; together 39 us with four waves, 44 with eight, which keep more LDS until
-// the last of them is done).
-constexpr int kRankAllThreads = 256;
-template <int W>
-__global__ __launch_bounds__(kRankAllThreads) void window_rank_all_kernel(
+// 12 500 edges: 29 + 23 us).
+template <int W, int TB>
+__global__ __launch_bounds__(TB) void window_rank_all_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
     int colBits, int range, int longGroups, int32_t* __restrict__ blockPartition,
     int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
     int* __restrict__ error) {
   extern __shared__ __align__(16) uint32_t smem[];
-  constexpr int NW = kRankAllThreads / 64;
+  constexpr int NW = TB / 64;
   if ((int)blockIdx.x >= longGroups) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int w = ((int)blockIdx.x - longGroups) * NW + wave;
@@ -1012,22 +1010,16 @@ __global__ __launch_bounds__(kRankAllThreads) void window_rank_all_kernel(
                              edgeToColumn, edgeToRow, error);
     return;
   }
-  __shared__ int sList[kRankAllThreads];
+  __shared__ int sList[TB];
   __shared__ int sListLen;
-  for (int64_t first = 0; first < nRW; first += (int64_t)kRankAllThreads * longGroups) {
+  for (int64_t first = 0; first < nRW; first += (int64_t)TB * longGroups) {
     const int found = find_windows(rowPtr, N, nRW, first, longGroups, kBinsMax, 0x7FFFFFFF, sList,
                                    &sListLen);
     for (int k = 0; k < found; k++)
-      rank_window_by_bitset<W, kRankAllThreads>(sList[k], rowPtr, colIdx, N, range, 1, kBinsMax, smem,
-                                              blockPartition, edgeToColumn, edgeToRow, error);
+      rank_window_by_bitset<W, TB>(sList[k], rowPtr, colIdx, N, range, 1, kBinsMax, smem, blockPartition,
+                                   edgeToColumn, edgeToRow, error);
   }
 }
-constexpr size_t rank_all_lds(int range) {
-  const size_t bins = (kRankAllThreads / 64) * sizeof(RankBinsLds);
-  const size_t bitset = (size_t)(range / 32 + range / 128) * sizeof(uint32_t);
-  return bins > bitset ? bins : bitset;
-}
-
 // Windows too long for a wave on graphs whose column range needs several bitset passes (N >
 // kRangeMax): one workgroup sorts the window's column ids, marks the distinct ones and finds every
 // edge's rank, instead of several passes over a 48 KiB bitset that such a window fills with a few
@@ -3109,6 +3101,34 @@ bool order_beside_fill(int nRW, int64_t E) {
   return nRW > kFinSingleMax && nRW <= kOrderBesideMax && !long_windows(nRW, E);
 }
 
+// Eight waves or four: of eight, the few long windows of a skewed graph are done sooner, and where there are
+// several rounds of short ones the chip starts fewer workgroups; four keep LDS for the rest of a workgroup
+// less long and take more long windows at once where those are many (four -> eight waves, call in us; R-MAT
+// of 130k nodes and 200, 340, 420 edges a window: 86 -> 83, 109 -> 99, 118 -> 104; power-law, 250k nodes, 340:
+// 138 -> 119; even, 250k nodes, 260: 91 -> 89; but even, 65k nodes, 260: 60.6 -> 62, power-law, 130k
+// nodes, 700: 124 -> 129).
+constexpr int64_t kRankWideEdges = 1250000;
+constexpr int kRankWideWindows = 8000;
+bool rank_all_wide(int nRW, int64_t E) {
+  return E / nRW <= kBinsMax / 2 && (E >= kRankWideEdges || nRW >= kRankWideWindows);
+}
+template <int W, int TB>
+int launch_rank_all(const int32_t* rowPtr, const int32_t* colIdx, int N, int nRW, int colBits, int range,
+                    unsigned longGroups, int32_t* blockPartition, int32_t* edgeToColumn,
+                    int32_t* edgeToRow, int* error, hipStream_t stream) {
+  constexpr int NW = TB / 64;
+  const size_t bins = NW * sizeof(RankBinsLds);
+  const size_t bitset = (size_t)(range / 32 + range / 128) * sizeof(uint32_t);
+  const size_t lds = bins > bitset ? bins : bitset;
+  auto kernel = window_rank_all_kernel<W, TB>;
+  if (int rc = allow_lds(kernel, lds)) return rc;
+  hipLaunchKernelGGL(kernel, dim3(longGroups + (unsigned)((nRW + NW - 1) / NW)), dim3(TB), lds, stream, rowPtr,
+                     colIdx, N, nRW, colBits, range, (int)longGroups, blockPartition, edgeToColumn,
+                     edgeToRow, error);
+  F3S_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
 // Enqueues the kernels that rank the windows' columns and count their TC blocks. sortedRowWindows holds
 // the lists of long windows until the order is written.
 template <int W>
@@ -3127,14 +3147,9 @@ int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, cha
   while (colBits < 31 && ((int64_t)1 << colBits) < (int64_t)N) colBits++;
   if (one_launch(nRW, E)) {
     const unsigned groups = all_long_groups(nRW, E);
-    const size_t ldsAll = rank_all_lds(range);
-    if (int rc = allow_lds(window_rank_all_kernel<W>, ldsAll)) return rc;
-    hipLaunchKernelGGL(window_rank_all_kernel<W>,
-                       dim3(groups + (unsigned)((nRW + kRankAllThreads / 64 - 1) / (kRankAllThreads / 64))),
-                       dim3(kRankAllThreads), ldsAll, stream, rowPtr, colIdx, N, nRW, colBits, range,
-                       (int)groups, blockPartition, edgeToColumn, edgeToRow, error);
-    F3S_HIP_CHECK(hipGetLastError());
-    return 0;
+    auto launch = rank_all_wide(nRW, E) ? launch_rank_all<W, 512> : launch_rank_all<W, 256>;
+    return launch(rowPtr, colIdx, N, nRW, colBits, range, groups, blockPartition, edgeToColumn, edgeToRow,
+                  error, stream);
   }
   int shortMax = kBinsMax;
   WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
