@@ -2109,14 +2109,13 @@ __device__ __forceinline__ void fill_one_window(
 // its bit in the window's bitmaps and drops its column into the ids; two lanes per TC block then walk
 // the set bits row by row (a block of a sparse graph has 17, most of a walk's time is the fullest
 // dword among the lanes), and bitmaps, ids and tile ids leave as whole words. Bound by the issue of
-// vector instructions. Workgroups of one wave, 22 per CU (of four: 260 instead of 220 us for the 149k
+// vector instructions. Workgroups of one wave, 27 per CU (of four: 260 instead of 220 us for the 149k
 // such windows of a 61M-edge graph).
 template <int W>
 struct alignas(16) FillShortLds {  // of one wave
   static constexpr int MAXB = (kBinsMax + W - 1) / W;  // TC blocks of a window at most
   unsigned long long bm[MAXB * (16 * W / 64)];
-  uint32_t ids[MAXB * W];
-  uint8_t tile[kBinsMax + 8];
+  uint32_t ids[MAXB * W];  // later the tile ids, kBinsMax + 8 bytes
   alignas(8) uint32_t mark[kBinsMax / 32 + 2];
 };
 template <int W>
@@ -2182,7 +2181,9 @@ __device__ __forceinline__ void fill_short_window(
     store_streaming(reinterpret_cast<uint4*>(sparseAToXidx + (int64_t)base * W) + i,
                     reinterpret_cast<const uint4*>(ids)[i]);
   if (__ballot(rough) == 0ull) {
-    uint8_t* stage = lds.tile;
+    static_assert(kBinsMax + 8 <= sizeof(lds.ids), "tile ids where the ids were");
+    uint8_t* stage = reinterpret_cast<uint8_t*>(ids);
+    wave_lds_sync();  // the ids are out
     const unsigned skew = (unsigned)((uintptr_t)(tcblocktileId + eS) & 3u);
     unsigned carry = 0;
     for (int k = 0; k < 2 * nb; k += 64) {
@@ -2383,13 +2384,19 @@ __device__ __forceinline__ int sum_counts(const int32_t* __restrict__ counts, in
 // Phase 2 of a graph of up to kFinSingleMax windows, most of them short, in one launch like
 // window_rank_all_kernel: workgroups that look for the long windows, then some that make the window
 // order (unless orderGroups is 0), which nothing else of the call waits for, then those of the short
-// windows. 169k-node R-MAT graph: 17 + 25 us as two launches, 29 us together; with four waves and half the
-// blocks of a long window at a time 52 us, with sixteen and twice as many 37 us.
+// windows. 169k-node R-MAT graph: 17 + 25 us as two launches, 29 us together. Eight waves: preprocessing
+// calls on 34 R-MAT, power-law and even graphs take up to 23 % longer with four and 28 % with sixteen.
+// As many blocks of a long window at a time as let three workgroups share a CU (53 760 bytes of LDS each),
+// which the short windows' LDS does too since a window's tile ids are staged where its ids were (two
+// workgroups and 576 blocks before: power-law, 50k nodes, 1300 edges a window: 107 -> 98 us, 250k nodes, 700:
+// 195 -> 173; R-MAT, 250k nodes, 200: 115 -> 109; power-law, 130k nodes, 100, whose longest windows fall
+// between 528 and 576 blocks: 74 -> 78).
 // SELF: no scan was launched before; every workgroup adds up the counts in front of its windows itself
 // and the short ones' write rowWindowOffset and the total. That is one launch (4 us) less where the sums
 // are short, a few counts per thread: up to kSelfScanMax windows.
 constexpr int kFillAllThreads = 512;
-constexpr int kFillAllChunk = 576;  // TC blocks: 54 KiB of LDS, as much as the short windows take
+template <int W>
+constexpr int kFillAllChunk = W == 16 ? 528 : 640;
 constexpr int kSelfScanMax = 2048;
 template <int W, bool SELF>
 __global__ __launch_bounds__(kFillAllThreads) void window_fill_all_kernel(
@@ -2453,7 +2460,7 @@ __global__ __launch_bounds__(kFillAllThreads) void window_fill_all_kernel(
         base = rowWindowOffset[w];
         nb = rowWindowOffset[w + 1] - base;
       }
-      fill_one_window<W, TB, kFillAllChunk, kFillAllChunk>(
+      fill_one_window<W, TB, kFillAllChunk<W>, kFillAllChunk<W>>(
           w, base, nb, rowPtr, colIdx, N, E, edgeToColumn, sRawDyn, tcblockRowid, tcblocktileId,
           tcblockOffset, sparseAToXidx, bitmap);
     }
@@ -2462,8 +2469,8 @@ __global__ __launch_bounds__(kFillAllThreads) void window_fill_all_kernel(
 template <int W>
 constexpr size_t fill_all_lds(int nBins) {
   size_t lds = (kFillAllThreads / 64) * sizeof(FillShortLds<W>);
-  if (lds < fill_lds_bytes<W>(kFillAllChunk, kFillAllChunk))
-    lds = fill_lds_bytes<W>(kFillAllChunk, kFillAllChunk);
+  if (lds < fill_lds_bytes<W>(kFillAllChunk<W>, kFillAllChunk<W>))
+    lds = fill_lds_bytes<W>(kFillAllChunk<W>, kFillAllChunk<W>);
   return lds > nBins * sizeof(uint32_t) ? lds : nBins * sizeof(uint32_t);
 }
 
@@ -3084,11 +3091,17 @@ unsigned long_grid(int nRW, int E, int minEdges, int most) {
 // workgroups of one wave are the better ones: with more than four rounds of windows on every CU the
 // LDS that a finished wave keeps until its workgroup ends costs more than the overlap gives.
 bool one_launch(int nRW, int64_t E) { return nRW <= kFinSingleMax && !long_windows(nRW, E); }
-// Their workgroups for windows of more than kBinsMax edges: where such windows are the exception two per CU
-// (with one for each that there can be, most look in vain and the short windows wait for their
-// slots), else as above.
+// Their workgroups for windows of more than kBinsMax edges, one for each that there can be; where such windows
+// are the exception 512 or 1024, as most look in vain and the short windows wait for their slots. 1024, so
+// that fewer meet two long ones, where long windows are to be expected (512 -> 1024, means of six orders of
+// the nodes; R-MAT, 130k nodes, 420 edges a window: 110 -> 103 us, power-law, 250k nodes, 420: 136 -> 125;
+// even, 65k nodes, 200, none of them long: 59.4 -> 61).
+constexpr int64_t kLongGroupsEdges = 1250000;
 unsigned all_long_groups(int nRW, int E) {
-  return long_grid(nRW, E, kBinsMax, E / nRW <= kBinsMax / 2 ? 512 : kFinSingleMax);
+  const int mean = E / nRW;
+  const int most = mean > kBinsMax / 2 ? kFinSingleMax
+                   : mean >= kBinsMax / 4 && E >= kLongGroupsEdges ? 1024 : 512;
+  return long_grid(nRW, E, kBinsMax, most);
 }
 
 // Above kFinSingleMax windows the order is made in the last launch of the fill, where most CUs are idle:

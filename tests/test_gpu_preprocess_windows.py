@@ -143,7 +143,8 @@ def test_crowded_windows(oracle_mod, N):
 
 
 # One launch ranks the short and the long windows of up to 16 384: workgroups of eight waves from 8000
-# windows or 1.25M edges on, of at most 480 edges a window, of four otherwise
+# windows or 1.25M edges on, of at most 480 edges a window, of four otherwise; the long ones are filled 528
+# blocks of 16 columns or 640 of 8 at a time
 @pytest.mark.parametrize("nRW,edges", [(7999, 60), (8000, 60), (2600, 479), (2606, 480), (2600, 482), (16_384, 20)])
 @pytest.mark.parametrize("W", [16, 8])
 def test_waves_of_the_one_launch(oracle_mod, nRW, edges, W):
@@ -151,14 +152,18 @@ def test_waves_of_the_one_launch(oracle_mod, nRW, edges, W):
     print("case one launch nRW=%d edges=%d W=%d" % (nRW, edges, W), flush=True)
     rng = np.random.default_rng(nRW + edges)
     N, E = 16 * nRW - 5, nRW * edges
-    degree = np.bincount(rng.integers(0, N - 400, E - 8000), minlength=N)
-    degree[[0, 17, 8000, N - 1]] += [961, 3000, 3039, 1000]  # long windows among the short ones
+    wide = {16: 528 * 16, 48: 528 * 16 + 1, 4000: 640 * 8, 4032: 640 * 8 + 1, N - 1: 961, 8000: 3039}
+    degree = np.bincount(rng.integers(5000, N - 400, E - sum(wide.values())), minlength=N)
+    for r, n in wide.items():
+        degree[r] += n  # long windows among the short ones
     rowPtr = np.zeros(N + 1, np.int32)
     rowPtr[1:] = np.cumsum(degree)
     row = np.repeat(np.arange(N), degree)
     colIdx = rng.integers(0, N, E)
     colIdx = colIdx[np.lexsort((colIdx, row))].astype(np.int32)
     assert rowPtr[-1] == E
+    for r in wide:
+        colIdx[rowPtr[r]:rowPtr[r + 1]] = np.sort(rng.choice(N, degree[r], replace=False))
     want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, W)
     got = capi.preprocess(torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda(), N, 16, W)
     for k in KEYS:
