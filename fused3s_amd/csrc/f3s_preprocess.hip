@@ -356,27 +356,40 @@ __global__ __launch_bounds__(64) void window_rank_small_kernel(
   if (lane == 0) blockPartition[w] = (nUniq + W - 1) / W;
 }
 
-// One stable pass of a wave's LSD radix sort on a DB-bit digit: hist holds the first place of
-// every digit; a lane's place is that plus the number of lanes before it in its group of 64 with
-// the same digit (one ballot per digit bit).
-template <int DB>
-__device__ __forceinline__ void wave_scatter_in_order(const uint32_t* src, uint32_t* dst,
-                                                      uint32_t* hist, int n, int shift, int lane) {
+// A wave's n words, groups of 64 in key[], into buf at the places that hist holds for the values of their
+// `bits` bits above `shift`, in order: a lane's place is that plus the number of lanes before it in its
+// group with the same value (one ballot per bit).
+template <int G>
+__device__ __forceinline__ void wave_scatter_in_order(const uint32_t (&key)[G], uint32_t* buf, uint32_t* hist,
+                                                      int n, int shift, int bits, int lane) {
   const unsigned long long ltMask = (1ull << lane) - 1ull;
-  for (int base = 0; base < n; base += 64) {
-    const int i = base + lane;
-    const bool valid = i < n;
-    const uint32_t key = valid ? src[i] : 0u;
-    const unsigned dgt = (key >> shift) & ((1u << DB) - 1u);
-    unsigned long long peers = __ballot(valid);
 #pragma unroll
-    for (int b = 0; b < DB; b++) {
-      const unsigned long long bal = __ballot((dgt >> b) & 1u);
-      peers &= ((dgt >> b) & 1u) ? bal : ~bal;
+  for (int u = 0; u < G; u++) {
+    if (64 * u >= n) break;
+    const bool valid = lane < n - 64 * u;
+    const unsigned dgt = (key[u] >> shift) & ((1u << bits) - 1u);
+    unsigned long long peers = __ballot(valid);
+    for (int b = 0; b < bits; b++) {
+      const bool bit = (dgt >> b) & 1u;
+      const unsigned long long bal = __ballot(bit);
+      peers &= bit ? bal : ~bal;
     }
-    if (valid) dst[hist[dgt] + __popcll(peers & ltMask)] = key;
-    // the last peer advances the digit's position; the wave's LDS operations stay in order
+    if (valid) buf[hist[dgt] + __popcll(peers & ltMask)] = key[u];
+    // the last peer advances the value's position; the wave's LDS operations stay in order
     if (valid && (peers >> lane) == 1ull) hist[dgt] += __popcll(peers);
+  }
+}
+
+// The same where the order does not matter: words with the same value are put in order by the later
+// passes of a sort or name the same column, and equal columns only have to end up next to each other. A
+// returning LDS atomic hands out the places, a tenth of the instructions.
+template <int G>
+__device__ __forceinline__ void wave_scatter(const uint32_t (&key)[G], uint32_t* buf, uint32_t* hist, int n,
+                                             int shift, int bits, int lane) {
+#pragma unroll
+  for (int u = 0; u < G; u++) {
+    if (64 * u >= n) break;
+    if (lane < n - 64 * u) buf[atomicAdd(&hist[(key[u] >> shift) & ((1u << bits) - 1u)], 1u)] = key[u];
   }
 }
 
@@ -391,7 +404,6 @@ __device__ __forceinline__ void wave_radix_sort(uint32_t* buf, uint32_t* hist, i
   const int firstBits = colBits < 8 ? colBits : 8;
   const int restBits = colBits - firstBits;
   const int nStable = (restBits + 7) / 8;
-  const unsigned long long ltMask = (1ull << lane) - 1ull;
   int shift = IDX_BITS;
   for (int pass = 0; pass <= nStable; pass++) {
     const int db = pass == 0 ? firstBits
@@ -421,29 +433,10 @@ __device__ __forceinline__ void wave_radix_sort(uint32_t* buf, uint32_t* hist, i
           make_uint4(excl, excl + c.x, excl + c.x + c.y, excl + c.x + c.y + c.z);
     }
     wave_lds_sync();
-#pragma unroll
-    for (int u = 0; u < G; u++) {
-      if (64 * u >= n) break;
-      const bool valid = lane < n - 64 * u;
-      const unsigned dgt = (key[u] >> shift) & mask;
-      if (pass == 0) {
-        // The first pass need not be stable: words with the same digit are put in order by the
-        // later passes or name the same column, and equal columns only have to end up next to
-        // each other. A returning LDS atomic hands out the places, a tenth of the instructions
-        // of the in-order scatter.
-        if (valid) buf[atomicAdd(&hist[dgt], 1u)] = key[u];
-        continue;
-      }
-      unsigned long long peers = __ballot(valid);
-      for (int b = 0; b < db; b++) {
-        const bool bit = (dgt >> b) & 1u;
-        const unsigned long long bal = __ballot(bit);
-        peers &= bit ? bal : ~bal;
-      }
-      if (valid) buf[hist[dgt] + __popcll(peers & ltMask)] = key[u];
-      // the last peer advances the digit's position; the wave's LDS operations stay in order
-      if (valid && (peers >> lane) == 1ull) hist[dgt] += __popcll(peers);
-    }
+    if (pass == 0)
+      wave_scatter<G>(key, buf, hist, n, shift, db, lane);
+    else
+      wave_scatter_in_order<G>(key, buf, hist, n, shift, db, lane);
     wave_lds_sync();
     shift += db;
   }
@@ -1020,59 +1013,162 @@ __global__ __launch_bounds__(TB) void window_rank_all_kernel(
                                    edgeToColumn, edgeToRow, error);
   }
 }
+
 // Windows too long for a wave on graphs whose column range needs several bitset passes (N >
-// kRangeMax): one workgroup sorts the window's column ids, marks the distinct ones and finds every
-// edge's rank, instead of several passes over a 48 KiB bitset that such a window fills with a few
-// thousand bits. The sort is that of window_rank_bins_kernel widened to a workgroup, with eight bins
-// per thread; an edge then finds its column in its bin. Windows whose columns crowd into few bins
-// take an LSD radix sort, eight bits per pass, every wave on its own contiguous part of the keys, and
-// a binary search per edge. (Radix sort and search for all: 163 instead of 128 us for the 4 272 such
-// windows of a 61M-edge graph.)
+// kRangeMax): one workgroup ranks the window's column ids among each other, instead of several passes over
+// a 48 KiB bitset that such a window fills with a few thousand bits. The columns go into eight bins per
+// thread, as in rank_window_groups; a thread keeps its columns and where it put them, finds their places
+// among the sorted ones from their neighbours and marks the first of every column in a bitset of places, in
+// which a rank is a count. Bound by latency, so by the waves that LDS and registers leave: 24 per CU, where
+// the sorted columns in a second buffer, searched again by every edge, allowed 16 (4 272 such windows of a
+// 61M-edge graph: preprocessing 635 -> 615 us). Windows whose columns crowd into few bins
+// take an LSD radix sort, eight bits per pass, and a binary search per edge.
 // The windows come from the lists that the kernel for short windows has made: where every workgroup looked
 // for its own, some met five and some none (4 272 windows dealt to 8 192 workgroups: 133 instead of
 // 96 us; window_fill_long_kernel 68 instead of 45 us).
-// Two sizes: windows of up to kMedMax edges (256 threads, 36 KiB of LDS, four workgroups per CU), and
-// the handful of windows of up to kLargeMax edges (1024 threads, 144 KiB), which would otherwise each
-// walk the bitset passes alone at the end of the phase.
-constexpr int kMedThreads = 256;
-constexpr int kMedItems = 16;
+// Two sizes: windows of up to kMedMax edges (512 threads, 26 KiB of LDS; 256 threads of 16 edges
+// do not fit 80 registers), and the handful of windows of up to kLargeMax edges (1024
+// threads, 85 KiB), which would otherwise each walk the bitset passes alone at the end of the phase.
+constexpr int kMedThreads = 512;
+constexpr int kMedItems = 8;
 constexpr int kMedMax = kMedThreads * kMedItems;
 constexpr int kLargeThreads = 1024;
 constexpr int kLargeItems = 16;
 constexpr int kLargeMax = kLargeThreads * kLargeItems;
 constexpr int kSortCrowd = 32;  // a fuller bin sends the window to the radix sort
+constexpr int kSortPad = 64;
+static_assert(kSortPad >= kSortCrowd + kRankStep, "neighbours of the first and the last key");
 template <int ITEMS, int THREADS>
 constexpr size_t rank_sort_lds() {
-  return ((size_t)2 * THREADS * ITEMS + 4 * THREADS) * sizeof(uint32_t);
+  return ((size_t)THREADS * ITEMS + 2 * kSortPad + 4 * THREADS + 2 * (THREADS * ITEMS / 32)) * sizeof(uint32_t);
+}
+
+// The n distinct ones of a workgroup's keys, ascending, in sKeys and their number in *sUniq: an LSD radix
+// sort, eight bits per pass, every wave on its own contiguous part of the keys, which it holds in registers
+// while it scatters them back. Key u * THREADS + thread is key[u] of the thread. Every thread of the
+// workgroup calls this.
+template <int ITEMS, int THREADS>
+__device__ __forceinline__ void rank_crowded_keys(const uint32_t (&key)[ITEMS], uint32_t* sKeys, uint32_t* sHist,
+                                                  unsigned* sWaveTot, int n, int keyBits, int* sUniq) {
+  constexpr int WAVES = THREADS / 64;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+  for (int u = 0; u < ITEMS; u++)
+    if (tid < n - u * THREADS) sKeys[u * THREADS + tid] = key[u];
+  // wave v sorts the keys [cb, cb + part) of every pass's input into their places of its output
+  const int chunk = ((n + THREADS - 1) / THREADS) * 64;
+  const int cb = min(n, wave * chunk), part = min(n - cb, chunk);
+  uint32_t* hist = sHist + 256 * wave;
+  uint32_t mine[ITEMS];
+  for (int shift = 0; shift < keyBits; shift += 8) {
+    __syncthreads();  // the keys of this pass are in place
+#pragma unroll
+    for (int u = 0; u < ITEMS; u++) {
+      if (64 * u >= part) continue;
+      mine[u] = lane < part - 64 * u ? sKeys[cb + 64 * u + lane] : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) hist[lane + 64 * k] = 0;
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < ITEMS; u++) {
+      if (64 * u >= part) continue;
+      if (lane < part - 64 * u) atomicAdd(&hist[(mine[u] >> shift) & 255u], 1u);
+    }
+    __syncthreads();
+    // thread d < 256: keys with a smaller digit, then this digit's keys of the waves in front
+    unsigned c[WAVES], tot = 0, incl = 0;
+    if (tid < 256) {
+#pragma unroll
+      for (int v = 0; v < WAVES; v++) {
+        c[v] = sHist[256 * v + tid];
+        tot += c[v];
+      }
+      incl = wave_inclusive_scan(tot, lane);
+      if (lane == 63) sWaveTot[wave] = incl;
+    }
+    __syncthreads();
+    if (tid < 256) {
+      unsigned run = incl - tot;
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        if (v < wave) run += sWaveTot[v];
+#pragma unroll
+      for (int v = 0; v < WAVES; v++) {
+        sHist[256 * v + tid] = run;
+        run += c[v];
+      }
+    }
+    __syncthreads();
+    if (shift == 0)
+      wave_scatter<ITEMS>(mine, sKeys, hist, part, 0, 8, lane);
+    else
+      wave_scatter_in_order<ITEMS>(mine, sKeys, hist, part, shift, 8, lane);
+  }
+  __syncthreads();
+  // distinct keys: first occurrences, a count with ballots, the waves' totals, then the stores
+  unsigned cnt = 0, first = 0;  // bit u: key 64 u + lane of the part is one
+#pragma unroll
+  for (int u = 0; u < ITEMS; u++) {
+    if (64 * u >= part) continue;
+    const int i = cb + 64 * u + lane;
+    const bool valid = lane < part - 64 * u;
+    mine[u] = valid ? sKeys[i] : 0u;
+    const bool is = valid && (i == 0 || sKeys[i - 1] != mine[u]);
+    first |= is ? 1u << u : 0u;
+    cnt += (unsigned)__popcll(__ballot(is));
+  }
+  if (lane == 0) sWaveTot[wave] = cnt;
+  __syncthreads();
+  unsigned pos = 0, all = 0;
+#pragma unroll
+  for (int v = 0; v < WAVES; v++) {
+    const unsigned x = sWaveTot[v];
+    if (v < wave) pos += x;
+    all += x;
+  }
+#pragma unroll
+  for (int u = 0; u < ITEMS; u++) {
+    if (64 * u >= part) continue;
+    const bool is = (first >> u) & 1u;
+    const unsigned long long bal = __ballot(is);
+    if (is) sKeys[pos + (unsigned)__popcll(bal & ((1ull << lane) - 1ull))] = mine[u];
+    pos += (unsigned)__popcll(bal);
+  }
+  if (tid == 0) *sUniq = (int)all;
+  __syncthreads();
 }
 
 // takes the mid windows of the queue, or (LARGE) the large ones of at most THREADS * ITEMS edges
 template <int W, int ITEMS, int THREADS, bool LARGE>
-__global__ __launch_bounds__(THREADS) void window_rank_sort_kernel(
+__global__ __launch_bounds__(THREADS, LARGE ? 1 : 6) void window_rank_sort_kernel(
     const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
     int colBits, LongQueue queue, int32_t* __restrict__ blockPartition,
     int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
     int* __restrict__ error) {
   constexpr int WAVES = THREADS / 64;
   constexpr int CAP = THREADS * ITEMS;
-  constexpr int BIN_BITS = THREADS == 256 ? 11 : 13;
-  constexpr int U = 4;  // edges of a thread in flight together
+  constexpr int BIN_BITS = THREADS == 256 ? 11 : THREADS == 512 ? 12 : 13;
   static_assert((1 << BIN_BITS) == 8 * THREADS, "eight bins per thread");
   static_assert(THREADS >= 256 && THREADS % 256 == 0, "the first 256 threads own one digit each");
-  // two buffers of CAP keys, then the bins' 16-bit counters or the radix sort's digit counters
-  extern __shared__ __align__(16) uint32_t sBufDyn[];
-  uint32_t* const sBuf0 = sBufDyn;
-  uint32_t* const sBuf1 = sBufDyn + CAP;
-  uint32_t* const sBins = sBufDyn + 2 * CAP;
-  uint32_t (*const sHist)[256] = reinterpret_cast<uint32_t (*)[256]>(sBins);
+  extern __shared__ __align__(16) uint32_t sSort[];
+  uint32_t* sKeys = sSort + kSortPad;  // CAP keys, room for kSortPad on each side
+  uint32_t* sBins = sKeys + CAP + kSortPad;  // 16-bit counters, or the radix sort's digit counters
+  uint32_t* sFirst = sBins + 4 * THREADS;  // bit per key: the first one of its column
+  uint32_t* sBefore = sFirst + CAP / 32;  // such keys in front of a word of bits
   __shared__ int sRow[17];
   __shared__ unsigned sWaveTot[WAVES];
   __shared__ int sCrowded;
+  __shared__ int sUniq;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const unsigned long long ltMask = (1ull << lane) - 1ull;
-  const int shiftBins = colBits > BIN_BITS ? colBits - BIN_BITS : 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // keys are columns plus one: 0 stands for none
+  const int keyBits = colBits + (((int64_t)1 << colBits) <= (int64_t)N ? 1 : 0);
+  const int shiftBins = keyBits > BIN_BITS ? keyBits - BIN_BITS : 0;
+  const uint32_t sameBin = 1u << shiftBins;
   const int listed = queue.size(LARGE);
   for (int taken = blockIdx.x; taken < listed; taken += (int)gridDim.x) {
     const int w = queue.at(LARGE, taken);
@@ -1082,23 +1178,34 @@ __global__ __launch_bounds__(THREADS) void window_rank_sort_kernel(
     if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
     if (tid == 0) sCrowded = 0;
     reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(0, 0, 0, 0);
+    for (int i = tid; i < CAP / 32; i += THREADS) sFirst[i] = 0u;
+    if (tid < kSortPad) sSort[tid] = 0u;
     __syncthreads();
-    const int eS = sRow[0], eE = sRow[16];
-    const int n = eE - eS;
+    const int eS = uniform(sRow[0]);
+    int n = uniform(sRow[16]) - eS;
+    const int32_t* cols = colIdx + eS;
+    int32_t *ranks = edgeToColumn + eS, *rows = edgeToRow + eS;
+    // thread t's keys: of edges t + THREADS u
+    uint32_t key[ITEMS], at[ITEMS];
+#pragma unroll
+    for (int u = 0; u < ITEMS; u++) {
+      if (u * THREADS >= n) continue;
+      key[u] = (uint32_t)cols[min(u * THREADS + tid, n - 1)];
+    }
+    if (tid < kSortPad) sKeys[n + tid] = 0xFFFFFFFFu;
+    asm volatile("" : "+s"(n));
     bool bad = false;
-    for (int i0 = tid; i0 < n; i0 += U * THREADS) {
-      unsigned k[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) k[u] = (unsigned)colIdx[eS + min(i0 + u * THREADS, n - 1)];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (i0 + u * THREADS >= n) break;
-        if (k[u] >= (unsigned)N) {
-          bad = true;
-          k[u] = 0u;
-        }
-        sBuf0[i0 + u * THREADS] = k[u];
-        const unsigned bin = k[u] >> shiftBins;
+    for (int u = 0; u < ITEMS; u++) {
+      if (u * THREADS >= n) continue;
+      if (key[u] >= (uint32_t)N) {
+        bad = true;
+        key[u] = 0u;
+      }
+      key[u] += 1u;
+      const uint32_t bin = key[u] >> shiftBins;
+      if (tid < n - u * THREADS) {
+        rows[u * THREADS + tid] = r0 + row_of_edge(sRow, eS + u * THREADS + tid);
         atomicAdd(&sBins[bin >> 1], 1u << ((bin & 1u) * 16u));
       }
     }
@@ -1128,210 +1235,101 @@ __global__ __launch_bounds__(THREADS) void window_rank_sort_kernel(
         run = mid + (v[k] >> 16);
         v[k] = start;
       }
-      if (!sCrowded) reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(v[0], v[1], v[2], v[3]);
+      reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(v[0], v[1], v[2], v[3]);
     }
     __syncthreads();
-    // the wave's contiguous part of the keys
-    const int chunk = ((n + THREADS - 1) / THREADS) * 64;
-    const int cb = min(n, wave * chunk), ce = min(n, cb + chunk);
-    if (!sCrowded) {
-      // into the bins; afterwards a bin's counter says where it ends
-      for (int i0 = tid; i0 < n; i0 += U * THREADS) {
-        uint32_t col[U], old[U];
+    if (sCrowded) {
+      rank_crowded_keys<ITEMS, THREADS>(key, sKeys, sBins, sWaveTot, n, keyBits, &sUniq);
+      const int nUniq = sUniq;
 #pragma unroll
-        for (int u = 0; u < U; u++) col[u] = sBuf0[min(i0 + u * THREADS, n - 1)];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const uint32_t bin = col[u] >> shiftBins;
-          if (i0 + u * THREADS < n)
-            old[u] = atomicAdd(&sBins[bin >> 1], 1u << ((bin & 1u) * 16u));
+      for (int u = 0; u < ITEMS; u++) {
+        if (u * THREADS >= n) continue;
+        int lo = 0, hi = nUniq - 1;  // the key is one of the window's distinct ones
+        while (lo < hi) {
+          const int mid = (lo + hi) >> 1;
+          if (sKeys[mid] < key[u])
+            lo = mid + 1;
+          else
+            hi = mid;
         }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const uint32_t half = ((col[u] >> shiftBins) & 1u) * 16u;
-          if (i0 + u * THREADS < n) sBuf1[(old[u] >> half) & 0xFFFFu] = col[u];
-        }
+        if (tid < n - u * THREADS) ranks[u * THREADS + tid] = lo;
       }
-      __syncthreads();
-      const uint16_t* binEnd = reinterpret_cast<const uint16_t*>(sBins);
-      for (int i0 = tid; i0 < n; i0 += U * THREADS) {
-        uint32_t key[U];
-        int end[U], at[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) key[u] = sBuf1[min(i0 + u * THREADS, n - 1)];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const uint32_t bin = key[u] >> shiftBins;
-          end[u] = binEnd[bin];
-          at[u] = bin == 0u ? 0 : (int)binEnd[max(bin, 1u) - 1u];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const int i = i0 + u * THREADS;
-          if (i >= n) break;
-          const int begin = at[u];
-          if (end[u] - begin > 1)
-            for (int q = begin; q < end[u]; q++) {
-              const uint32_t other = sBuf1[q];
-              at[u] += (other < key[u] || (other == key[u] && q < i)) ? 1 : 0;
-            }
-          sBuf0[at[u]] = key[u];
-        }
-      }
-      __syncthreads();
-      // ranks of the sorted keys, next to them in the other buffer
-      unsigned cnt = 0;
-      for (int base = cb; base < ce; base += 64) {
-        const int i = base + lane;
-        cnt += (unsigned)__popcll(__ballot(i < ce && (i == 0 || sBuf0[i - 1] != sBuf0[i])));
-      }
-      if (lane == 0) sWaveTot[wave] = cnt;
-      __syncthreads();
-      unsigned rank = 0, nUniq = 0;
-#pragma unroll
-      for (int v = 0; v < WAVES; v++) {
-        const unsigned x = sWaveTot[v];
-        if (v < wave) rank += x;
-        nUniq += x;
-      }
-      for (int base = cb; base < ce; base += 64) {
-        const int i = base + lane;
-        const unsigned long long bal =
-            __ballot(i < ce && (i == 0 || sBuf0[i - 1] != sBuf0[i]));
-        if (i < ce) sBuf1[i] = rank + (unsigned)__popcll(bal & (ltMask | (1ull << lane))) - 1u;
-        rank += (unsigned)__popcll(bal);
-      }
-      __syncthreads();
-      for (int i0 = tid; i0 < n; i0 += U * THREADS) {
-        uint32_t col[U];
-        int end[U], q[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          col[u] = (uint32_t)colIdx[eS + min(i0 + u * THREADS, n - 1)];
-          if (col[u] >= (uint32_t)N) col[u] = 0u;
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const uint32_t bin = col[u] >> shiftBins;
-          end[u] = binEnd[bin];
-          q[u] = bin == 0u ? 0 : (int)binEnd[max(bin, 1u) - 1u];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const int e = eS + i0 + u * THREADS;
-          if (e >= eE) break;
-          // the first of the bin's sorted columns that is not below this one: the column itself
-          while (q[u] < end[u] - 1) {
-            const int mid = (q[u] + end[u] - 1) >> 1;
-            if (sBuf0[mid] < col[u])
-              q[u] = mid + 1;
-            else
-              end[u] = mid + 1;
-          }
-          edgeToColumn[e] = (int)sBuf1[q[u]];
-          edgeToRow[e] = r0 + row_of_edge(sRow, e);
-        }
-      }
-      if (tid == 0) blockPartition[w] = (int)((nUniq + W - 1) / W);
+      if (tid == 0) blockPartition[w] = (nUniq + W - 1) / W;
       continue;
     }
-    // wave v sorts the keys [cb, ce) of every pass's input into their places of its output
-    uint32_t* src = sBuf0;
-    uint32_t* dst = sBuf1;
-    uint32_t* hist = sHist[wave];
-    for (int shift = 0; shift < colBits; shift += 8) {
+    // into the bins (n is hidden from the compiler between the passes: sixteen comparisons with it, kept for
+    // all of them, cost more registers than the keys)
+    asm volatile("" : "+s"(n));
 #pragma unroll
-      for (int k = 0; k < 4; k++) hist[lane + 64 * k] = 0;
-      __syncthreads();  // the keys of this pass are in place, the counters are clear
-      for (int i = cb + lane; i < ce; i += 64) atomicAdd(&hist[(src[i] >> shift) & 255u], 1u);
+    for (int u = 0; u < ITEMS; u++) {
+      if (u * THREADS >= n) continue;
+      const uint32_t bin = key[u] >> shiftBins, half = (bin & 1u) * 16u;
+      at[u] = 0;
+      if (tid < n - u * THREADS) {
+        at[u] = (atomicAdd(&sBins[bin >> 1], 1u << half) >> half) & 0xFFFFu;
+        sKeys[at[u]] = key[u];
+      }
+    }
+    __syncthreads();
+    asm volatile("" : "+s"(n));
+    // Each key's place among the sorted ones: from its place in the bins' order, later keys that are smaller
+    // move it up, earlier ones that are larger move it down, and keys of other bins do neither. An earlier
+    // equal one says that this is not the first of its column.
+#pragma unroll
+    for (int u = 0; u < ITEMS; u++) {
+      if (u * THREADS >= n) continue;
+      const bool valid = tid < n - u * THREADS;
+      const uint32_t* here = sKeys + at[u];
+      uint32_t up = 0, down = 0;
+      int place = (int)at[u];
+      bool again = false;
+#pragma unroll
+      for (int k = 1; k <= kRankNear; k++) {
+        up = here[k];
+        down = here[-k];
+        place += up < key[u] ? 1 : 0;
+        place -= down > key[u] ? 1 : 0;
+        again = again || down == key[u];
+      }
+      for (int k = kRankNear; k < kSortCrowd; k += kRankStep) {
+        const bool more = valid && ((up ^ key[u]) < sameBin || ((down ^ key[u]) < sameBin && down != 0u));
+        if (__ballot(more) == 0ull) break;
+#pragma unroll
+        for (int j = 1; j <= kRankStep; j++) {
+          up = here[k + j];
+          down = here[-k - j];
+          place += up < key[u] ? 1 : 0;
+          place -= down > key[u] ? 1 : 0;
+          again = again || down == key[u];
+        }
+      }
+      at[u] = (uint32_t)place;
+      if (valid && !again) atomicOr(&sFirst[place >> 5], 1u << (place & 31));
+    }
+    __syncthreads();
+    {
+      static_assert(CAP / 32 <= THREADS, "a word of bits per thread");
+      const uint32_t count = tid < CAP / 32 ? __popc(sFirst[tid]) : 0u;
+      const uint32_t incl = wave_inclusive_scan(count, lane);
+      if (lane == 63) sWaveTot[wave] = incl;
       __syncthreads();
-      {
-        // thread d < 256: keys with a smaller digit, then this digit's keys of the waves in front
-        unsigned c[WAVES], tot = 0, incl = 0;
-        if (tid < 256) {
+      uint32_t run = incl - count;
 #pragma unroll
-          for (int v = 0; v < WAVES; v++) {
-            c[v] = sHist[v][tid];
-            tot += c[v];
-          }
-          incl = wave_inclusive_scan(tot, lane);
-          if (lane == 63) sWaveTot[wave] = incl;
-        }
-        __syncthreads();
-        if (tid < 256) {
-          unsigned run = incl - tot;
-#pragma unroll
-          for (int v = 0; v < 4; v++)
-            if (v < wave) run += sWaveTot[v];
-#pragma unroll
-          for (int v = 0; v < WAVES; v++) {
-            sHist[v][tid] = run;
-            run += c[v];
-          }
-        }
-      }
-      __syncthreads();
-      if (shift == 0) {
-        // the first pass need not be stable (equal columns only have to end up next to each
-        // other): a returning LDS atomic hands out the places of the wave's keys
-        for (int i = cb + lane; i < ce; i += 64) {
-          const uint32_t key = src[i];
-          dst[atomicAdd(&hist[key & 255u], 1u)] = key;
-        }
-      } else {
-        wave_scatter_in_order<8>(src + cb, dst, hist, ce - cb, shift, lane);
-      }
-      uint32_t* t = src;
-      src = dst;
-      dst = t;
+      for (int u = 0; u < CAP / 32 / 64; u++)
+        if (u < wave) run += sWaveTot[u];
+      if (tid < CAP / 32) sBefore[tid] = run;
+      if (tid == CAP / 32 - 1) blockPartition[w] = ((int)(run + count) + W - 1) / W;
     }
     __syncthreads();
-    // distinct columns: first occurrences, compacted in order into the other buffer (every wave
-    // on its quarter [cb, ce) again: a count with ballots, the waves' totals, then the stores)
-    uint32_t* uniq = dst;
-    unsigned cnt = 0;
-    for (int base = cb; base < ce; base += 64) {
-      const int i = base + lane;
-      const bool first = i < ce && (i == 0 || src[i - 1] != src[i]);
-      cnt += (unsigned)__popcll(__ballot(first));
-    }
-    if (lane == 0) sWaveTot[wave] = cnt;
-    __syncthreads();
-    unsigned pos = 0, nUniq = 0;
+    asm volatile("" : "+s"(n));
+    // an edge's rank: the first keys at or in front of its place, without the column's own
 #pragma unroll
-    for (int v = 0; v < WAVES; v++) {
-      const unsigned x = sWaveTot[v];
-      if (v < wave) pos += x;
-      nUniq += x;
+    for (int u = 0; u < ITEMS; u++) {
+      if (u * THREADS >= n) continue;
+      if (tid >= n - u * THREADS) continue;
+      const uint32_t bits = sFirst[at[u] >> 5] & ((2u << (at[u] & 31u)) - 1u);
+      ranks[u * THREADS + tid] = (int)(sBefore[at[u] >> 5] + __popc(bits)) - 1;
     }
-    for (int base = cb; base < ce; base += 64) {
-      const int i = base + lane;
-      const bool first = i < ce && (i == 0 || src[i - 1] != src[i]);
-      const unsigned long long bal = __ballot(first);
-      if (first) uniq[pos + (unsigned)__popcll(bal & ltMask)] = src[i];
-      pos += (unsigned)__popcll(bal);
-    }
-    __syncthreads();
-    for (int e = eS + tid; e < eE; e += THREADS) {
-      unsigned col = (unsigned)colIdx[e];
-      if (col >= (unsigned)N) col = 0u;
-      int lo = 0, hi = (int)nUniq - 1, found = 0;
-      while (lo <= hi) {
-        const int mid = (lo + hi) >> 1;
-        const unsigned v = uniq[mid];
-        if (v == col) {
-          found = mid;
-          break;
-        }
-        if (v < col)
-          lo = mid + 1;
-        else
-          hi = mid - 1;
-      }
-      edgeToColumn[e] = found;
-      edgeToRow[e] = r0 + row_of_edge(sRow, e);
-    }
-    if (tid == 0) blockPartition[w] = (int)((nUniq + W - 1) / W);
   }
 }
 

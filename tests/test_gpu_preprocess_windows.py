@@ -170,6 +170,40 @@ def test_waves_of_the_one_launch(oracle_mod, nRW, edges, W):
         assert np.array_equal(got[k].cpu().numpy(), want[k]), k
 
 
+# Above 393 216 nodes a workgroup ranks the windows of 961 to 4096 and of up to 16 384 edges: 512 and 1024
+# edges at a time, bins of 32 edges and more by a radix sort. The last column of a power of two has a bit
+# more than the others
+@pytest.mark.parametrize("N", [1 << 19, (1 << 19) - 1, 500_000])
+def test_windows_of_a_workgroup(oracle_mod, N):
+    from fused3s_amd import capi
+    print("case windows of a workgroup N=%d" % N, flush=True)
+    rng = np.random.default_rng(N)
+    windows = []
+    for n in (961, 1023, 1024, 1025, 1536, 2048, 4095, 4096, 4097, 5000, 16_383, 16_384, 16_385):
+        even = rng.integers(0, N, n)
+        even[:2] = [0, N - 1]
+        windows.append(even)
+        windows.append(np.where(rng.random(n) < 0.2, rng.integers(0, N, n), N // 2 + rng.integers(0, 300, n)))
+        windows.append(np.where(rng.random(n) < 16 / n, N - 1, even))
+        for k in (31, 32, 33):
+            spread = even.copy()
+            spread[2:2 + k] = 0 if k == 33 else N - 1
+            windows.append(spread)
+    degree = np.zeros(N, np.int64)
+    columns = []
+    for w, cols in enumerate(windows):
+        rows = np.sort(rng.integers(0, 16, len(cols)))
+        degree[16 * w:16 * w + 16] = np.bincount(rows, minlength=16)
+        columns.append(cols[np.lexsort((cols, rows))] if w % 4 else cols)
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum(degree)
+    colIdx = np.concatenate(columns).astype(np.int32)
+    want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, 16)
+    got = capi.preprocess(torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda(), N, 16, 16)
+    for k in KEYS:
+        assert np.array_equal(got[k].cpu().numpy(), want[k]), k
+
+
 def split_columns(rng, cols, lengths):
     """16 ascending rows of the given lengths over `cols`, which together name every one of them."""
     cols = np.sort(cols)
