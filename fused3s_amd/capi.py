@@ -20,7 +20,7 @@ EXPORTS = ["f3s_abi_version", "f3s_last_error", "f3s_preprocess_workspace_bytes"
            "f3s_preprocess_static_scratch_bytes", "f3s_preprocess_count_static",
            "f3s_preprocess_capacity", "f3s_preprocess", "f3s_attention_prepare",
            "f3s_attention_heads_workspace_bytes", "f3s_attention_uses_wide_offsets",
-           "f3s_window_order"]
+           "f3s_attention_heads_uses_workspace", "f3s_window_order"]
 
 
 def lib():
@@ -69,6 +69,9 @@ def lib():
         L.f3s_attention_uses_wide_offsets.argtypes = [ctypes.c_int64, ctypes.c_int64, ci]
         L.f3s_attention_uses_workspace.restype = ci
         L.f3s_attention_uses_workspace.argtypes = [ci, ctypes.c_int64, ci, ci]
+        L.f3s_attention_heads_uses_workspace.restype = ci
+        L.f3s_attention_heads_uses_workspace.argtypes = [ci, ctypes.c_int64, ci, ci, ci,
+                                                         ctypes.c_int64]
         L.f3s_attention_fwd_tcb8.restype = ci
         L.f3s_attention_fwd_tcb8.argtypes = [vp, vp, vp, vp, ci, ctypes.c_int64, ci, vp, vp, vp,
                                              ci, vp, vp, vp]
@@ -180,11 +183,14 @@ def preprocess_count_static(rowPtr, colIdx, N, out, H=16, W=16):
 def attention_workspace(N, d, device, nTCB=None, dtype=torch.float16, heads=0):
     """Scratch tensor for attention(..., workspace=...) / attention_heads(..., workspace=...)
     (column-sliced schedule; heads = 0 for the single-head call). With nTCB given, returns None
-    when the library would not use it for this problem."""
+    when the library would not use it for this problem (rows of heads * d elements)."""
     L = lib()
-    if nTCB is not None and not L.f3s_attention_uses_workspace(
-            N, int(nTCB), d, 0 if dtype == torch.float16 else 1):
-        return None
+    if nTCB is not None:
+        code = 0 if dtype == torch.float16 else 1
+        used = (L.f3s_attention_heads_uses_workspace(N, int(nTCB), heads, d, code, heads * d)
+                if heads > 0 else L.f3s_attention_uses_workspace(N, int(nTCB), d, code))
+        if not used:
+            return None
     nbytes = (L.f3s_attention_heads_workspace_bytes(N, heads, d) if heads > 0
               else L.f3s_attention_workspace_bytes(N, d))
     return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)

@@ -42,16 +42,6 @@ bool split_short_windows(const int32_t* windowOrder, int nRW, int64_t nTcb, Head
 // takes 1.54 ms at d = 64 against 2.48 ms for the workgroup-per-window kernel, with 7.1 GB
 // instead of 17.7 GB of traffic beyond L2.
 // Short windows would be cut into units of one or two blocks; they keep the window kernel.
-// F3S_SCHEDULE=window / =sliced in the environment overrides the choice.
-int attention_uses_workspace(int N, int64_t nTcb, int d, int dtype) {
-  const char* e = getenv("F3S_SCHEDULE");  // read per call
-  const int forced = (e && strcmp(e, "sliced") == 0) ? 1 : (e && strcmp(e, "window") == 0) ? -1 : 0;
-  if ((dtype != 0 && dtype != 1) || !head_dim_supported(d) || N <= 0) return 0;
-  if (forced) return forced > 0;
-  const int64_t nRW = ((int64_t)N + kWinRows - 1) / kWinRows;
-  return nRW >= 2048 && nTcb >= 64 * nRW;
-}
-
 // Calls on small structures of narrow rows are over before their slices pay, with or without a workspace
 // (window against sliced, us; nodes, blocks a window). One head, d = 64: 50 000, 76 63 against 83; 70 000,
 // 93 106 against 119; 100 000, 66 120 against 145; 50 000, 178 118 against 121; from 750 000 blocks sliced
@@ -65,6 +55,20 @@ bool windows_suffice(int64_t nTcb, int d, int nHeads) {
   if (nHeads <= 1) return nTcb < (d <= 32 ? 260000 : 450000);
   if (d == 32) return heads_in_pairs(d, nHeads) && nTcb < 600000;
   return nTcb < 250000;
+}
+
+// Whether a call that is given a workspace uses it, that is, takes the column-sliced schedule: the
+// launchers below and the queries that callers allocate by ask this one function. nHeads = 0: the
+// single-head layout; ldIn: row pitch of Q / K / V in elements.
+// F3S_SCHEDULE=window / =sliced in the environment overrides the choice.
+int attention_uses_workspace(int N, int64_t nTcb, int nHeads, int d, int dtype, int64_t ldIn) {
+  const char* e = getenv("F3S_SCHEDULE");  // read per call
+  const int forced = (e && strcmp(e, "sliced") == 0) ? 1 : (e && strcmp(e, "window") == 0) ? -1 : 0;
+  if ((dtype != 0 && dtype != 1) || !head_dim_supported(d) || N <= 0) return 0;
+  if (gather_needs_wide_offsets(N, ldIn * 2, nHeads > 0)) return 0;  // launch_window_wide's
+  if (forced) return forced > 0;
+  const int64_t nRW = ((int64_t)N + kWinRows - 1) / kWinRows;
+  return nRW >= 2048 && nTcb >= 64 * nRW && !windows_suffice(nTcb, d, nHeads);
 }
 
 int launch_attention(const int32_t* rowWindowOffset, const int32_t* windowOrder,
@@ -86,8 +90,7 @@ int launch_attention(const int32_t* rowWindowOffset, const int32_t* windowOrder,
   if (gather_needs_wide_offsets(N, (int64_t)d * 2, false))
     return launch_window_wide(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q,
                               K, V, scaleLog2, applySoftmax, out, cuTimer, 0, d, d, nTcb, stream);
-  if (workspace && !cuTimer && attention_uses_workspace(N, nTcb, d, dtype) &&
-      !windows_suffice(nTcb, d, 0))
+  if (workspace && !cuTimer && attention_uses_workspace(N, nTcb, 0, d, dtype, d))
     return launch_attention_sliced(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, 0, d, d, prepared ? 2 : 0, stream);
@@ -178,7 +181,7 @@ int launch_attention_heads(const int32_t* rowWindowOffset, const int32_t* window
     return launch_window_wide(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q,
                               K, V, scaleLog2, applySoftmax, out, nullptr, nHeads, (int)ldIn,
                               (int)ldOut, nTcb, stream);
-  if (workspace && attention_uses_workspace(N, nTcb, d, dtype) && !windows_suffice(nTcb, d, nHeads))
+  if (workspace && attention_uses_workspace(N, nTcb, nHeads, d, dtype, ldIn))
     return launch_attention_sliced(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, nHeads, (int)ldIn, (int)ldOut, prepared ? 2 : 0, stream);

@@ -142,7 +142,14 @@ size_t f3s_attention_heads_workspace_bytes(int N, int nHeads, int d) {
 }
 
 int f3s_attention_uses_workspace(int N, int64_t nTCB, int d, int dtype) {
-  return f3s::attention_uses_workspace(N, nTCB, d, dtype);
+  return f3s::attention_uses_workspace(N, nTCB, 0, d, dtype, d);
+}
+
+int f3s_attention_heads_uses_workspace(int N, int64_t nTCB, int nHeads, int d, int dtype,
+                                       int64_t ldIn) {
+  if (nHeads < 1 || nHeads > 1024 || ldIn < (int64_t)nHeads * d || ldIn >= ((int64_t)1 << 31))
+    return 0;  // f3s_attention_fwd_heads refuses the call
+  return f3s::attention_uses_workspace(N, nTCB, nHeads, d, dtype, ldIn);
 }
 
 int f3s_attention_uses_wide_offsets(int64_t N, int64_t pitch_bytes, int pitched) {

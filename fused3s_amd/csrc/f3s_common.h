@@ -84,7 +84,8 @@ int launch_attention_tcb8(const int32_t* rowWindowOffset, const int32_t* windowO
                           const void* Q, const void* K, const void* V, int applySoftmax,
                           float* out, float* sddmm, int64_t nTcb8, hipStream_t stream);
 
-int attention_uses_workspace(int N, int64_t nTcb, int d, int dtype);
+// nHeads = 0: contiguous single head; ldIn: row pitch of Q / K / V in elements
+int attention_uses_workspace(int N, int64_t nTcb, int nHeads, int d, int dtype, int64_t ldIn);
 
 // column-sliced schedule (f3s_attention_units.hip)
 // nHeads = 0: contiguous single head. mode 0: attention call; 1: build the slice index only;

@@ -386,7 +386,8 @@ std::vector<torch::Tensor> f3sMultiHeadScaleQK(torch::Tensor rowWindowOffset,
   const int dtype = Q.scalar_type() == torch::kHalf ? F3S_DTYPE_F16 : F3S_DTYPE_BF16;
   // graphs of long windows take the column-sliced schedule here as in the single-head calls
   const bool sliced =
-      f3s_attention_uses_workspace(nNodes, sparseAToXidx.numel() / 16, (int)d, dtype) != 0;
+      f3s_attention_heads_uses_workspace(nNodes, sparseAToXidx.numel() / 16, (int)nHeads, (int)d,
+                                         dtype, Q.stride(0)) != 0;
   const size_t wsBytes =
       sliced ? f3s_attention_heads_workspace_bytes(nNodes, (int)nHeads, (int)d) : 0;
   WorkspaceLease lease(sliced, wsBytes, Q.device());

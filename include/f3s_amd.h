@@ -169,9 +169,9 @@ int f3s_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, i
  *                                  With it, graphs for which f3s_attention_uses_workspace()
  *                                  returns 1 are computed by the column-sliced schedule: per
  *                                  (window, column slice) partial results that a second kernel
- *                                  merges in slice order (small structures at d <= 64 are
- *                                  computed as without it). Results agree with the default
- *                                  schedule within the tolerance of the summation order.
+ *                                  merges in slice order; other calls leave it alone. Results
+ *                                  agree with the default schedule within the tolerance of the
+ *                                  summation order.
  *                                  Ignored with cuTimer. Calls that share a workspace must not
  *                                  overlap. Its contents need not be initialised.
  *   prepared                       0, or 1 when f3s_attention_prepare was called on this workspace
@@ -210,18 +210,26 @@ size_t f3s_attention_heads_workspace_bytes(int N, int nHeads, int d);
  * 0 for f3s_attention_fwd, the head count for f3s_attention_fwd_heads): the caller must not
  * change their contents, nor write to the workspace, while it passes prepared = 1. A call with
  * prepared = 0, or with other arrays, on the same workspace rebuilds the index and ends the
- * preparation. Asynchronous on `stream`.
+ * preparation. Of use only where the queries below return 1: other calls read no index.
+ * Asynchronous on `stream`.
  */
 int f3s_attention_prepare(const int32_t* rowWindowOffset, const int32_t* sparseAToXidx, int N,
                           int64_t nTCB, int d, int nHeads, void* workspace, size_t ws_bytes,
                           void* stream);
 
 /*
- * 1 if f3s_attention_fwd would use a workspace for this problem (at least 2048 row windows with
- * 64 or more TC blocks each on average), else 0: callers can skip the allocation.
- * F3S_SCHEDULE=window or =sliced in the environment (read at every call) forces 0 or 1.
+ * 1 if f3s_attention_fwd / f3s_attention_fwd_heads would use a workspace for this problem, else 0:
+ * callers can skip the allocation and f3s_attention_prepare. It is used for structures of at least
+ * 2048 row windows with 64 or more TC blocks each on average, without cuTimer, unless the structure
+ * is so small at d <= 64 that the slices do not pay (a number of blocks that depends on d and the
+ * heads) or the rows need 64-bit offsets (f3s_attention_uses_wide_offsets). The two entries differ in
+ * the second point, so each has its own query; arguments as in the calls.
+ * F3S_SCHEDULE=window or =sliced in the environment (read at every call) forces 0 or, rows of 64-bit
+ * offsets apart, 1.
  */
 int f3s_attention_uses_workspace(int N, int64_t nTCB, int d, int dtype);
+int f3s_attention_heads_uses_workspace(int N, int64_t nTCB, int nHeads, int d, int dtype,
+                                       int64_t ldIn);
 
 /*
  * 1 if the attention kernels form 64-bit row offsets for K / V arrays of N rows with a row pitch
@@ -240,9 +248,9 @@ int f3s_attention_uses_wide_offsets(int64_t N, int64_t pitch_bytes, int pitched)
  * once per head on contiguous per-head copies and concatenate; this call returns what that loop
  * returns. ldIn % 8 == 0, ldOut % 4 == 0, both below 2^31.
  * workspace, ws_bytes: NULL / 0, or f3s_attention_heads_workspace_bytes(N, nHeads, d) bytes of
- * device scratch (256-byte aligned); with it, graphs for which f3s_attention_uses_workspace()
+ * device scratch (256-byte aligned); with it, graphs for which f3s_attention_heads_uses_workspace()
  * returns 1 take the column-sliced schedule with (window, slice, head) units, as in
- * f3s_attention_fwd; prepared as there. Asynchronous on `stream`.
+ * f3s_attention_fwd; other calls leave it alone; prepared as there. Asynchronous on `stream`.
  */
 int f3s_attention_fwd_heads(const int32_t* rowWindowOffset, const int32_t* windowOrder,
                             const int32_t* sparseAToXidx, const uint64_t* tcbBitMap, int N,

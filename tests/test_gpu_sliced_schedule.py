@@ -253,6 +253,80 @@ def test_wide_offset_rule():
     assert f(3000, 2 << 20, 1) == 1                  # 3000 rows of 2 MiB: 5.9 GiB
 
 
+# (heads, d, blocks from which on the workspace is used); heads = 0: the single-head call
+LINES = [(0, 32, 260_000), (0, 64, 450_000), (0, 96, 0), (1, 64, 450_000), (2, 32, 600_000),
+         (3, 32, 0), (2, 64, 250_000), (4, 64, 250_000), (4, 96, 0)]
+
+
+@pytest.mark.parametrize("heads,d,line", LINES)
+def test_workspace_queries(monkeypatch, heads, d, line):
+    """Host side of the choice between the schedules: both queries around the lines (no GPU needed)."""
+    from fused3s_amd import capi
+    monkeypatch.delenv("F3S_SCHEDULE", raising=False)
+    monkeypatch.delenv("F3S_SLICE_PHASES", raising=False)
+    L, N = capi.lib(), 16 * 2048
+
+    def uses(blocks, pitch=heads * d, n=N):
+        if heads:
+            return L.f3s_attention_heads_uses_workspace(n, blocks, heads, d, 0, pitch)
+        return L.f3s_attention_uses_workspace(n, blocks, d, 0)
+
+    least = 64 * 2048
+    assert uses(least - 1) == 0 and uses(max(line, least)) == 1 and uses(max(line, least) - 1) == 0
+    assert uses(10 * least, n=N - 16) == 0  # 2047 windows
+    if heads:
+        assert uses(10 * least, pitch=heads * d - 1) == 0  # a call that is refused
+        assert uses(10 * least, pitch=1 << 16) == 0  # K spans 4 GiB: 64-bit offsets
+        assert uses(10 * least, pitch=(1 << 16) - 8) == 1
+    else:
+        assert uses(2**40, n=1 << 28) == 0
+    monkeypatch.setenv("F3S_SCHEDULE", "sliced")
+    assert uses(5, n=40) == 1
+    monkeypatch.setenv("F3S_SCHEDULE", "window")
+    assert uses(10 * least) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,d", [(0, 32), (0, 64), (0, 96), (2, 32), (3, 32), (2, 64), (8, 64)])
+def test_calls_and_module_follow_the_queries(monkeypatch, heads, d):
+    """A call uses its workspace exactly where its query says so: one that is too small is refused
+    there and left alone elsewhere; and the module keeps scratch only where it is used."""
+    from fused3s_amd import F3S, capi
+    monkeypatch.delenv("F3S_SCHEDULE", raising=False)
+    monkeypatch.delenv("F3S_SLICE_PHASES", raising=False)
+    nRW = 2048
+    N = 16 * nRW
+    g = torch.Generator(device="cuda").manual_seed(d)
+    Q, K, V = [torch.randn((N, max(heads, 1), d), generator=g, device="cuda").half()
+               for _ in range(3)]
+    if not heads:
+        Q, K, V = [t[:, 0].contiguous() for t in (Q, K, V)]
+    for per in (63, 64, 100, 126, 127, 219, 220, 293):
+        print("case queries heads=%d d=%d blocks=%d" % (heads, d, per * nRW), flush=True)
+        cols = torch.arange(per * 16, device="cuda", dtype=torch.int32) * (N // (per * 16))
+        shift = torch.arange(nRW, device="cuda", dtype=torch.int32) % (N // (per * 16))
+        atox = (cols[None, :] + shift[:, None]).reshape(-1).contiguous()
+        bm = torch.randint(1, 2**62, (nRW * per * 4,), generator=g, device="cuda").view(torch.uint64)
+        rwo = torch.arange(nRW + 1, device="cuda", dtype=torch.int32) * per
+        order = torch.arange(nRW, device="cuda", dtype=torch.int32)
+        ws = capi.attention_workspace(N, d, "cuda", nTCB=nRW * per, heads=heads)
+        call = capi.attention_heads if heads else capi.attention
+        small = torch.full((256,), 0xFF, dtype=torch.uint8, device="cuda")
+        if ws is None:
+            got = call(rwo, order, atox, bm, N, Q, K, V, 8.0, workspace=small)
+            assert bool((small == 0xFF).all())
+            assert torch.equal(got, call(rwo, order, atox, bm, N, Q, K, V, 8.0))
+        else:
+            with pytest.raises(RuntimeError, match="workspace 256 B < required"):
+                call(rwo, order, atox, bm, N, Q, K, V, 8.0, workspace=small)
+        F3S.release_workspace()
+        if heads:
+            F3S.f3s_multihead_scaleQK(rwo, order, atox, bm, N, Q, K, V, 8.0)
+        else:
+            F3S.f3s_1tb1rw_scheduled_permuteV_scaleQK(rwo, order, atox, bm, N, Q, K, V, 8.0, 8)
+        assert F3S.release_workspace() == (0 if ws is None else ws.numel())
+
+
 @pytest.mark.gpu
 def test_rows_beyond_4_gib(oracle_mod):
     """K and V as pitched views whose span exceeds 4 GiB on a small node set (2 304 rows of 2 MiB

@@ -178,7 +178,9 @@ def test_small_single_head_calls_leave_the_workspace(oracle_mod, monkeypatch, d,
     assert pre["blockCount"] >= 64 * 2048
     g = torch.Generator().manual_seed(d)
     Q, K, V = [torch.randn((N, 1, d), generator=g).half().cuda() for _ in range(3)]
-    ws = capi.attention_workspace(N, d, "cuda", nTCB=atox.numel() // 16)
+    assert (capi.attention_workspace(N, d, "cuda", nTCB=atox.numel() // 16) is None) == (
+        pre["blockCount"] < limit)
+    ws = capi.attention_workspace(N, d, "cuda")
     ws.fill_(0xFF)
     got = capi.attention(rwo, order, atox, bm, N, *[t[:, 0].contiguous() for t in (Q, K, V)],
                          float(np.sqrt(d)), workspace=ws)
