@@ -42,19 +42,38 @@ bool split_short_windows(const int32_t* windowOrder, int nRW, int64_t nTcb, Head
 // takes 1.54 ms at d = 64 against 2.48 ms for the workgroup-per-window kernel, with 7.1 GB
 // instead of 17.7 GB of traffic beyond L2.
 // Short windows would be cut into units of one or two blocks; they keep the window kernel.
-// Calls on small structures of narrow rows are over before their slices pay, with or without a workspace
-// (window against sliced, us; nodes, blocks a window). One head, d = 64: 50 000, 76 63 against 83; 70 000,
-// 93 106 against 119; 100 000, 66 120 against 145; 50 000, 178 118 against 121; from 750 000 blocks sliced
-// is faster (100 000, 121: 219 against 193). d = 32: 50 000, 76 47 against 54; 40 000, 100 48 against 54;
-// 100 000, 66 99 against 92. Several heads, d = 64: 40 000, 73: 2 heads 90 against 104, 4 heads 175
-// against 183; 100 000, 66: 241 against 233, 505 against 464. Pairs of 32: 100 000, 61: 4 heads 231
-// against 302, 8 heads 474 against 551; 100 000, 121: 459 against 468, 959 against 879.
+// Calls on small structures of narrow rows are over before their slices pay. What decides is how skewed the
+// graph is, which neither the number of nodes nor of blocks says: the lines are for power-law and R-MAT graphs,
+// whose hot rows stay in the L2s by themselves. Window against sliced, us; nodes, blocks a window:
+// - one head, d = 64, 450 000 blocks. Below: power-law 35 000, 191 81 against 93; 50 000, 118 85 92; 70 000, 93
+//   102 115; 100 000, 68 123 155; R-MAT 60 000, 94 111 155. Beyond, power-law graphs still lose by their
+//   slices, but less and less (50 000, 148 101 107; 178 117 120; 203 131 130; 100 000, 103 182 188; 122 218 204),
+//   and uniform graphs of more rows than an L2 has room for gain more than that, as they do below
+//   (36 000, 193 89 99; 42 000, 147 97 95; 50 000, 129 122 102; 50 000, 148 132 112; 100 000, 91 255 202).
+// - one head, d = 32, 260 000: power-law 35 000, 116 44 57; 50 000, 78 46 51; 50 000, 100 56 60; 70 000, 79 68
+//   69; 100 000, 68 98 87; R-MAT 60 000, 78 71 78; 101 105 89; uniform 36 000, 99 41 47; 50 000, 71 56 49.
+// - two and four heads of 64, 250 000 (bf16): power-law 35 000, 73 75 96 and 148 160; 103 95 106 and 204 205;
+//   133 120 129 and 263 249; 50 000, 87 126 134 and 271 264; 70 000, 77 170 182 and 367 352; R-MAT 40 000, 105
+//   107 183 and 218 255; uniform 36 000, 99 129 108 and 290 220.
+// - pairs of 32-wide heads (bf16), 600 000 for one pair or two: power-law 50 000, 100 76 95 and 148 172; 178 133
+//   149 and 263 278; 100 000, 94 165 200 and 336 358; 122 218 253 and 449 439 (fp16: 50 000, 178 123 126 and 246
+//   231); R-MAT 120 000, 98 180 331 and 333 515; uniform 36 000, 147 87 101 and 173 171; 50 000, 129 134 121 and
+//   267 216. 400 000 for four and eight: power-law 35 000, 133 272 291 and 629 611; 50 000, 100 320 335 and 736
+//   719; 135 431 425 and 970 917; 178 563 537 and 1267 1150 (fp16, four pairs: 135 421 382; 178 552 478);
+//   100 000, 68 524 574 and 1171 1287; 94 721 704 and 1590 1614; R-MAT 60 000, 123 414 474 and 948 955.
+// Eight heads of 64 gain by their slices from the fewest blocks on (35 000, 73 348 347; 103 486 457; 50 000, 87
+// 631 593; R-MAT 40 000, 105 505 493), and so do numbers of heads that leave an XCD several of them to gather
+// (three to sixteen heads of 64, 35 000, 103: 3 212 177, 5 452 314, 6 433 334, 16 1081 829; six of 32, 50 000,
+// 100 325 299; 135 459 370).
 bool windows_suffice(int64_t nTcb, int d, int nHeads) {
   if (getenv("F3S_SCHEDULE") || getenv("F3S_SLICE_PHASES")) return false;  // asked for
   if (d > 64) return false;
   if (nHeads <= 1) return nTcb < (d <= 32 ? 260000 : 450000);
-  if (d == 32) return heads_in_pairs(d, nHeads) && nTcb < 600000;
-  return nTcb < 250000;
+  if (d == 32 && !heads_in_pairs(d, nHeads)) return false;
+  const int units = d == 32 ? nHeads / 2 : nHeads;
+  if (units > head_groups(64, units)) return false;  // several to an XCD
+  if (d == 32) return nTcb < (units <= 2 ? 600000 : 400000);
+  return units <= 4 && nTcb < 250000;
 }
 
 // Whether a call that is given a workspace uses it, that is, takes the column-sliced schedule: the

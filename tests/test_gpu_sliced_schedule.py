@@ -255,7 +255,10 @@ def test_wide_offset_rule():
 
 # (heads, d, blocks from which on the workspace is used); heads = 0: the single-head call
 LINES = [(0, 32, 260_000), (0, 64, 450_000), (0, 96, 0), (1, 64, 450_000), (2, 32, 600_000),
-         (3, 32, 0), (2, 64, 250_000), (4, 64, 250_000), (4, 96, 0)]
+         (3, 32, 0), (2, 64, 250_000), (4, 64, 250_000), (4, 96, 0),
+         # several heads, or pairs of 32-wide ones, left to an XCD, and eight of 64
+         (3, 64, 0), (6, 64, 0), (8, 64, 0), (16, 64, 0), (6, 32, 0), (32, 32, 0),
+         (4, 32, 600_000), (8, 32, 400_000), (16, 32, 400_000)]
 
 
 @pytest.mark.parametrize("heads,d,line", LINES)
