@@ -208,9 +208,9 @@ def test_window_kernel_head_groups(oracle_mod, monkeypatch, heads, d, N):
 
 
 # 32-wide heads two at a time: bit-identical to head by head through every schedule (windows, with and
-# without natural order; short windows with long ones beside them; column slices in both forms), on rows of
-# a pitch that shifts the pairs off the 128-byte lines, scores far above the running maximum in one head
-# of a pair only, and scores that are exactly 0
+# without natural order; short windows with long ones beside them, too few of them for pairs at two and four
+# heads; column slices in both forms), on rows of a pitch that shifts the pairs off the 128-byte lines, scores
+# far above the running maximum in one head of a pair only, and scores that are exactly 0
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("heads", [2, 4, 6, 16])
 @pytest.mark.parametrize("kind", ["window", "short", "sliced", "resident"])
@@ -246,6 +246,40 @@ def test_pairs_of_heads_are_bit_identical(oracle_mod, monkeypatch, kind, heads, 
                                     float(np.sqrt(d)), workspace=scratch(1)) for h in range(heads)]
         assert torch.isfinite(got).all()
         assert torch.equal(got, torch.cat(one, dim=1))
+
+
+# Wave-per-window launches take 32-wide heads in pairs from 50 000 blocks times pairs on, one or two pairs of
+# fewer blocks head by head: both sides of the line, bit-identical to head by head, a few long windows beside
+@pytest.mark.parametrize("missing", [1, 0])
+@pytest.mark.parametrize("heads,blocks", [(2, 50_000), (4, 25_000)])
+def test_pairs_of_heads_in_short_windows(oracle_mod, heads, blocks, missing):
+    from fused3s_amd import capi
+    print("case short pairs heads=%d blocks=%d" % (heads, blocks - missing), flush=True)
+    nRW, d = blocks // 14, 32
+    N = 16 * nRW - 3
+    rng = np.random.default_rng(blocks + missing)
+    counts = np.full(nRW, 14)
+    counts[::701] = 41
+    over = int(counts.sum()) - (blocks - missing)
+    counts[np.setdiff1d(np.arange(nRW), np.arange(0, nRW, 701))[:over]] -= 1
+    rwo = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    assert rwo[-1] == blocks - missing < 16 * nRW
+    step = N // (41 * 16)
+    atox = np.concatenate([np.arange(16 * c) * step for c in counts])
+    atox = (atox + rng.integers(0, step, len(atox))).astype(np.int32)
+    bitmap = rng.integers(0, 2**63, len(atox) // 4, dtype=np.uint64)
+    bitmap &= rng.integers(0, 2**63, len(bitmap), dtype=np.uint64)
+    order = np.argsort(-counts, kind="stable").astype(np.int32)
+    pre = dict(rowWindowOffset=rwo, sparseAToXidx=atox, tcbBitMap=bitmap)
+    dev = lambda a: torch.as_tensor(a).cuda()
+    args = dev(rwo), dev(order), dev(atox), dev(bitmap.view(np.int64)).view(torch.uint64), N
+    g = torch.Generator().manual_seed(heads)
+    Q, K, V = [torch.randn((N, heads, d), generator=g).half().cuda() for _ in range(3)]
+    got = capi.attention_heads(*args, Q, K, V, float(np.sqrt(d)))
+    one = [capi.attention_heads(*args, *[t[:, h:h + 1] for t in (Q, K, V)], float(np.sqrt(d)))
+           for h in range(heads)]
+    assert torch.equal(got, torch.cat(one, dim=1))
+    check(oracle_mod, pre, N, heads, d, Q, K, V, got)
 
 
 # 1025 windows: one more than a whole number of chunks for every number of head groups
