@@ -3421,9 +3421,13 @@ int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
   // average, commonly far fewer): the large workgroups take all of them, which saves a launch
   const bool few = E / kBinsMax <= kFillFewLong && E / nRW <= kBinsMax / 2;
   LongQueue queue = {nullptr, nullptr, 0, 0};
-  if (ws)  // phase 1 has cleared the counts and is done with the keys behind the header
+  const uint16_t* orderRows = nullptr;
+  if (ws) {  // phase 1 has cleared the counts and is done with the keys behind the header
     queue = {&reinterpret_cast<WsHeader*>(ws)->fill, reinterpret_cast<int32_t*>(ws + kWsHeaderBytes), nRW,
              few ? 0 : kFillMid};
+    const size_t seg = align256((size_t)nRW * sizeof(int32_t));
+    orderRows = reinterpret_cast<const uint16_t*>(ws + kWsHeaderBytes + seg);
+  }
   hipLaunchKernelGGL((window_fill_short_kernel<W>), dim3(nRW), dim3(64), 0, stream, rowPtr, colIdx, N,
                      E, nRW, edgeToColumn, rowWindowOffset, queue, tcblockRowid, tcblocktileId,
                      tcblockOffset, sparseAToXidx, bm);
@@ -3441,15 +3445,13 @@ int enqueue_fill(const int32_t* rowPtr, const int32_t* colIdx, int N, int E,
   auto kernel = window_fill_long_kernel<W, 1024, kFillChunkLong, true>;
   constexpr size_t lds = fill_lds_bytes<W>(kFillChunkLong, kFillChunkLong);
   static_assert(lds >= 2 * kOrderRowBins * sizeof(uint32_t), "order_chunk's arrays");
-  const size_t seg = align256((size_t)nRW * sizeof(int32_t));
   if (int rc = allow_lds(kernel, lds)) return rc;
   const unsigned orderGroups =
       sortedRowWindows ? (unsigned)((nRW + kOrderRowWindows - 1) / kOrderRowWindows) : 0;
   hipLaunchKernelGGL(kernel, dim3(orderGroups + long_grid(nRW, E, minEdges, 255)), dim3(1024), lds,
                      stream, rowPtr, colIdx, N, E, nRW, edgeToColumn, rowWindowOffset, queue, minEdges,
-                     0x7FFFFFFF, (int)orderGroups, blockPartition,
-                     reinterpret_cast<const uint16_t*>(ws + kWsHeaderBytes + seg), sortedRowWindows, tcblockRowid,
-                     tcblocktileId, tcblockOffset, sparseAToXidx, bm);
+                     0x7FFFFFFF, (int)orderGroups, blockPartition, orderRows, sortedRowWindows,
+                     tcblockRowid, tcblocktileId, tcblockOffset, sparseAToXidx, bm);
   F3S_HIP_CHECK(hipGetLastError());
   return 0;
 }
