@@ -282,6 +282,31 @@ def test_pairs_of_heads_in_short_windows(oracle_mod, heads, blocks, missing):
     check(oracle_mod, pre, N, heads, d, Q, K, V, got)
 
 
+# The build with 64-bit row offsets takes 32-wide heads in pairs as well: rows of Q, K and V in one array of
+# more than 4 GiB, bit-identical to head by head, on both sides of the lines (one pair 100 000 blocks, four
+# pairs 12 500)
+@pytest.mark.parametrize("heads,deg", [(2, 60), (8, 8), (8, 3)])
+def test_pairs_of_heads_beyond_4_gib(oracle_mod, heads, deg):
+    from fused3s_amd import capi
+    print("case wide pairs heads=%d deg=%d" % (heads, deg), flush=True)
+    N, d, pitch = 33_003, 32, (1 << 16) + 8
+    assert capi.lib().f3s_attention_uses_wide_offsets(N, pitch * 2, 1) == 1
+    rng = np.random.default_rng(deg)
+    pre, (rwo, order, atox, bm) = on_gpu(oracle_mod, *random_csr(rng, N, deg, hub=1999), N)
+    assert (pre["blockCount"] * (heads // 2) >= (100_000 if heads == 2 else 50_000)) == (deg != 3)
+    g = torch.Generator().manual_seed(heads)
+    store = torch.empty((N, pitch), dtype=torch.float16, device="cuda")
+    Q, K, V = [store[:, at:at + heads * d].unflatten(1, (heads, d)) for at in (8, 1024, pitch - heads * d)]
+    for t in (Q, K, V):
+        t.copy_(torch.randn((N, heads, d), generator=g).half())
+    scale = float(np.sqrt(d))
+    got = capi.attention_heads(rwo, order, atox, bm, N, Q, K, V, scale)
+    one = [capi.attention_heads(rwo, order, atox, bm, N, *[t[:, h:h + 1] for t in (Q, K, V)], scale)
+           for h in range(heads)]
+    assert torch.equal(got, torch.cat(one, dim=1))
+    check(oracle_mod, pre, N, heads, d, Q, K, V, got)
+
+
 # 1025 windows: one more than a whole number of chunks for every number of head groups
 @pytest.mark.parametrize("heads,d", [(1, 32), (3, 64), (4, 64), (8, 32), (2, 128)])
 def test_short_windows(oracle_mod, heads, d):
