@@ -111,7 +111,7 @@ def test_split_multi_head_equals_per_head(oracle_mod, dtype):
 
 
 def test_many_long_units_per_workgroup(oracle_mod):
-    """More long (window, head) units than the long-window launch has workgroups (1024): its
+    """More long (window, pair of heads) units than the long-window launch has workgroups (512): its
     workgroups find several units each and compute them one after the other. 40 000 rows, one
     edge per row on average, 310 windows whose rows name 40 columns each; eight heads."""
     from fused3s_amd import capi

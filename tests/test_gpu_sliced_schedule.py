@@ -42,7 +42,7 @@ def to_dev(pre):
 @pytest.fixture(scope="module")
 def long_window_graph(oracle_mod):
     """The 233k-node benchmark generator at 0.145 of its size: 33 779 nodes (N % 16 != 0), 2 112
-    windows of about 130 TC blocks: the library picks the column-sliced schedule by itself."""
+    windows of about 400 TC blocks: the library picks the column-sliced schedule by itself."""
     from fused3s_amd import synth
     rp, ci = synth.make_graph("cfg3_chunglu_233k", scale=0.145)
     N = rp.numel() - 1
