@@ -880,12 +880,12 @@ constexpr int kShortChunk = 16;
 // 32-wide heads are computed one by one where one or two pairs of them make too few waves to fill the CUs: a
 // wave then takes longer for two heads than two waves for one each. Head by head against pairs, us; blocks of
 // the graph. One pair: uniform 10 000 10.7 against 12.0, 19 000 14.1 15.7, 26 000 17.8 16.9, 29 000 18.3 17.2;
-// communities 9 000 9.7 11.1, 31 000 17.1 17.7 or 19.3 18.6, 38 000 23.3 23.1; power-law 24 000 24.1 25.5, 40 000 32.1 33.0; R-MAT 13 000 18.6
-// 22.5, 31 000 28.0 29.2, 37 000 29.6 30.9, 51 000 35.9 35.9, 69 000 44.4 42.7. Two pairs: uniform 10 000 14.7
-// 15.3, 23 000 23.8 20.8; communities 9 000 12.9 14.0, 31 000 26.2 25.9; R-MAT 13 000 23.6 25.5, 23 000 31.9 32.6,
-// 26 000 34.0 34.8, 31 000 41.0 39.0; power-law 24 000 30.0 31.0, 40 000 47.8 45.9. Three and more lose at most
-// 3 % (four: R-MAT 13 000 30.9 31.7) and gain 1 to 25 % (three: communities 9 000 18.5 16.7; eight: uniform 6 000
-// 28.7 26.5).
+// communities 9 000 9.7 11.1, 31 000 17.1 17.7 or 19.3 18.6, 38 000 23.3 23.1; power-law 24 000 24.1 25.5, 40 000
+// 32.1 33.0; R-MAT 13 000 18.6 22.5, 31 000 28.0 29.2, 37 000 29.6 30.9, 51 000 35.9 35.9, 69 000 44.4 42.7. Two
+// pairs: uniform 10 000 14.7 15.3, 23 000 23.8 20.8; communities 9 000 12.9 14.0, 31 000 26.2 25.9; R-MAT 13 000
+// 23.6 25.5, 23 000 31.9 32.6, 26 000 34.0 34.8, 31 000 41.0 39.0; power-law 24 000 30.0 31.0, 40 000 47.8 45.9.
+// Three and more lose at most 3 % (four: R-MAT 13 000 30.9 31.7) and gain 1 to 25 % (three: communities 9 000
+// 18.5 16.7; eight: uniform 6 000 28.7 26.5).
 bool pairs_fill(int64_t nTcb, int pairs) { return pairs >= 3 || nTcb * pairs >= 50000; }
 
 // NH = 2: D = 64 stands for two heads of 32

@@ -1258,7 +1258,9 @@ __global__ __launch_bounds__(THREADS, LARGE ? 1 : 6) void window_rank_sort_kerne
       continue;
     }
     // into the bins (n is hidden from the compiler between the passes: sixteen comparisons with it, kept for
-    // all of them, cost more registers than the keys)
+    // all of them, cost more vector registers than the keys. Within a pass the lane masks of the guarded items
+    // still outnumber the scalar registers: 132 of them in the form of 512 threads and 261 in that of 1 024
+    // go to lanes of vector registers and back. None goes to memory.)
     asm volatile("" : "+s"(n));
 #pragma unroll
     for (int u = 0; u < ITEMS; u++) {
@@ -2619,6 +2621,8 @@ constexpr int rank_fill_bitset_bytes(int range) { return (range / 64 * 10 + 15) 
 // `big`) takes its blocks in chunks of bitmaps and enumerates its ids from the bitset. A window with a
 // repeated or descending column is handed to fill_window_generic once its edgeToColumn entries are
 // written, with the whole of the dynamic LDS as that routine's arrays.
+// Registers: 60 vector ones of the 80 that two workgroups per CU leave; of the scalar ones (pointers, lane
+// masks) about 40 go to lanes of vector registers, none to memory.
 template <int W, int TB>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6, 6)))
 void window_rank_fill_kernel(

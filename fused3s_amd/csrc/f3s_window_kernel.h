@@ -47,16 +47,19 @@ constexpr int waves_per_simd(Team t, int d) {
 // four workgroups fit a CU either way, so the second stage only has to pay for its longer loop.
 // One -> two stages in us, heavy-first order, one head unless stated. It pays
 // - where blocks are few and the longest window of a skewed graph decides. 17 to 30 blocks a window:
-//   R-MAT 65 521 nodes 48.6 -> 40.8, 169 343 nodes 78.9 -> 65.8 and 105 -> 85.7, 600 000 nodes 239 -> 241;
-//   38 to 57: 100 000 nodes 74.0 -> 67.6, 200 000 nodes 224 -> 227; 86 to 90: 30 000 nodes 45.1 -> 41.8,
-//   with 4 heads 143 -> 148; uniform and community graphs of 5 to 20: within 2 %.
+//   R-MAT 65 521 nodes 38.8 -> 32.9, 3 heads 65.1 -> 64.5, 169 343 nodes 71.9 -> 61.1, 3 heads 167 -> 172,
+//   600 000 nodes 268 -> 273; 38 to 57: R-MAT 100 000 nodes 79.1 -> 66.9, 200 000 nodes 146 -> 125; 81 to 90:
+//   30 000 nodes 32.1 -> 28.9; uniform and community graphs of 5 to 21: within 2 %, with 3 and 5 heads 0 to
+//   5 % faster.
 // - where windows are long, many, and the rows come from beyond the L2s (K + V of 20 MB): 100 000 nodes,
-//   423 blocks, 4 heads 3364 -> 2662; 140 000, 274, 4 heads 3194 -> 2897; 180 000, 434 1458 -> 1351;
-//   233 000, 448 2155 -> 2068, 8 heads 23 100 -> 21 200; 400 000, 239, 4 heads 10 168 -> 9 828.
-// In between all CUs are busy to the end, mostly with rows from the L2s: 124 to 132 blocks 52.4 -> 50.8,
-// with 4 heads 196 -> 204; 160 to 180 62.8 -> 63.3 and 127 -> 134; 337 to 387 44.2 -> 47.1 and 108 -> 114;
-// 100 000 nodes, 121 177 -> 188, 4 heads 889 -> 922; 233 000 nodes, 188 882 -> 900; 30 000 nodes, 387,
-// 8 heads 1154 -> 1175.
+//   406 blocks, 3 heads 2463 -> 2136, 5 heads 4628 -> 4441; 35 000, 294, 5 heads 820 -> 749; 140 000, 274, 3
+//   heads 2211 -> 2133, 5 heads 4110 -> 4259; 180 000, 408 1348 -> 1328, 3 heads 4920 -> 4723, 5 heads 10 070 ->
+//   10 170; 233 000, 448 2155 -> 2068, but 188 with 3 heads 2638 -> 2685, 5 heads 4957 -> 5282.
+// In between all CUs are busy to the end, mostly with rows from the L2s: 50 000 nodes, 114 61.3 -> 62.9, 3
+// heads 215 -> 231, 5 heads 420 -> 449; 148 77.2 -> 80.4, 3 heads 292 -> 315; 30 000, 329 90.1 -> 92.7, 3 heads
+// 308 -> 326 (5 heads 736 -> 688); 100 000, 121 164 -> 174, 3 heads 569 -> 607; 233 000, 188 881 -> 902; R-MAT
+// 100 000, 39, 3 heads 147 -> 150, 200 000, 40, 3 heads 345 -> 369.
+// (Even numbers of heads come here only where there is little to do: pairs_pay.)
 // At D = 64 a second stage costs the third workgroup: windows of 160 to 390 blocks 0 to 14 % slower, up
 // to 2 % faster on 100 000 nodes and more; R-MAT of 10 blocks a window up to 25 % slower (169 343 nodes
 // 69 -> 85), uniform graphs 10 to 24 %. Against that, R-MAT of 20 to 29 blocks and up to 100 000 nodes
@@ -97,7 +100,10 @@ __device__ __forceinline__ unsigned cu_key() {
 // group's part of the rows, and whole lines of it. With blockIdx.x = position * nHeads + head the two
 // heads of a line came from two XCDs, each of which fetched all of it (bf16, 200 000 nodes, 48 blocks a
 // window, 4 x 32: 823 -> 472 us; R-MAT of 1 000 000 nodes and 25 blocks, 2 x 32: 1203 -> 836 us; 40 000
-// nodes, 19 blocks, 8 x 32: 111 -> 100 us; wider heads are dealt as before).
+// nodes, 19 blocks, 8 x 32: 111 -> 100 us). 1, 2, 4 and 8 heads of 64 and more come out the same either
+// way; other numbers gain where an XCD's share of the rows shrinks and lose nowhere (graphs of 20 000 to
+// 160 000 nodes and 22 to 92 blocks a window: 3, 5 and 7 heads of 64 0 to 4 %, 12 of 64 2 to 7 %, 16 of 64
+// and 3 of 128 0 to 2 %, 12 of 128 4 to 7 %, 6 of 96 12 to 22 %).
 // W8 = true: the structure comes from preprocessing with 8-column blocks (the reference's
 // 1tb1tcb path, src/F3S_kernel.cu:677-877). Column ids and bitmap words of two consecutive 16x8
 // blocks are laid out exactly like one 16x16 block, so the same pipeline runs over four 16x8

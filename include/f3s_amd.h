@@ -194,7 +194,9 @@ int f3s_attention_fwd(const int32_t* rowWindowOffset, const int32_t* windowOrder
  * 512 * N bytes for copies of K and V with 256-byte rows, which the call makes itself and gathers
  * from instead: rows that start on even 128-byte lines are served faster than rows on the odd lines
  * in between). Room is for as many slices as any structure of N nodes is cut into: two or more, about
- * one per 8 MiB (3 MiB at d = 32) of a group of heads' K + V rows up to sixteen, so the size does not
+ * one per 8 MiB (3 MiB at d = 32 for a single head or an odd number of them, whose rows gain by more and
+ * smaller slices: 317 MB for one head and 1.5 GB for three on 232 965 nodes, 8 MiB slices would take 127 MB
+ * and 1.0 GB) of a group of heads' K + V rows up to sixteen, so the size does not
  * grow with N alone: ask for every N and d. The reference's launchers
  * (src/F3S_kernel.cu:581-671) need no scratch; passing workspace = NULL keeps that behaviour.
  */
