@@ -18,7 +18,7 @@ LIB_PATH = os.path.join(HERE, "libf3s_amd.so")
 EXT_PATH = os.path.join(HERE, "F3S" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 
 HIP_SOURCES = ["f3s_capi.hip", "f3s_attention.hip", "f3s_attention_wide.hip",
-               "f3s_attention_units.hip", "f3s_preprocess.hip"]
+               "f3s_attention_units.hip", "f3s_attention_mixed.hip", "f3s_preprocess.hip"]
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall",
     # packed-fp32 code generation is switched off for every device translation unit

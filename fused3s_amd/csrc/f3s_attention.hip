@@ -15,25 +15,11 @@ using pipe::kLog2e;
 using window::HeadLayout;
 
 
-// Graphs of short windows (a few TC blocks each) leave most of a four-wave workgroup idle and
-// pay its LDS merge for nothing. With a window order such a call is split: windows of at most
-// kShortWindowBlocks blocks go to the wave-per-window kernel, the others, with a heavy-first order
-// a prefix of at most nTcb / kShortWindowBlocks positions, stay with f3s_fwd_kernel, which skips
-// the short ones. An order that is not heavy-first stays correct (a long window outside the
-// prefix is computed by one wave). The two kernels run one after the other, so the split only
-// pays when long windows are rare: it is taken below 16 blocks per window on average (measured:
-// 100k-node 8-head layer 0.164 -> 0.101 ms and 0.248 -> 0.176 ms; an R-MAT graph with 16.6 blocks
-// per window and windows of up to 731 would go from 0.107 to 0.129 ms and is left alone).
-// Without an order nothing is split. F3S_SHORT_WINDOWS=0 in the environment turns it off.
-constexpr int kShortWindowBlocks = 32;
-bool split_short_windows(const int32_t* windowOrder, int nRW, int64_t nTcb, HeadLayout* hl) {
+// Whether a call goes to f3s_attention_mixed.hip. F3S_SHORT_WINDOWS=0 in the environment turns it off.
+bool short_windows(const int32_t* windowOrder, int nRW, int64_t nTcb16, int d, int nHeads) {
   const char* e = getenv("F3S_SHORT_WINDOWS");  // read per call, like every other switch
-  const bool off = e && strcmp(e, "0") == 0;
-  if (off || !windowOrder || nRW < 1024 || nTcb >= (int64_t)16 * nRW) return false;
-  hl->minBlocks = kShortWindowBlocks;
-  const int64_t longMax = nTcb / (kShortWindowBlocks + 1) + 1;
-  hl->gridWindows = (int)(longMax < nRW ? longMax : nRW);
-  return true;
+  if (e && strcmp(e, "0") == 0) return false;
+  return mixed_windows_pay(windowOrder != nullptr, nRW, nTcb16, d, nHeads);
 }
 
 // The column-sliced schedule (f3s_attention_units.hip: (window, column slice) units, every XCD
@@ -114,14 +100,10 @@ int launch_attention(const int32_t* rowWindowOffset, const int32_t* windowOrder,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, 0, d, d, prepared ? 2 : 0, stream);
   const int nRWi = (N + kWinRows - 1) / kWinRows;
-  HeadLayout single = {0, d, d, -1, nRWi, nTcb};
-  if (!cuTimer && split_short_windows(windowOrder, nRWi, nTcb, &single)) {
-    const int rc = launch_attention_short_windows(rowWindowOffset, windowOrder, sparseAToXidx,
-                                                  bitmap, N, d, dtype, Q, K, V, scaleLog2,
-                                                  applySoftmax, out, 0, d, d, kShortWindowBlocks,
-                                                  single.gridWindows, nTcb, stream);
-    if (rc != 0) return rc;
-  }
+  if (!cuTimer && short_windows(windowOrder, nRWi, nTcb, d, 0))
+    return launch_attention_mixed(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q, K, V,
+                                  scaleLog2, applySoftmax, out, 0, d, d, nTcb, stream);
+  const HeadLayout single = {0, d, d, nTcb};
   return dtype == 0 ? window::dispatch_d<_Float16, false>(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N,
                                            d, Q, K, V, scaleLog2, applySoftmax, out, cuTimer,
                                            single, stream)
@@ -155,6 +137,10 @@ int launch_attention_tcb8(const int32_t* rowWindowOffset, const int32_t* windowO
   if (gather_needs_wide_offsets(N, (int64_t)d * 2, false))
     return launch_tcb8_wide(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, Q, K, V,
                             scaleLog2, applySoftmax, out, sddmm, nTcb8, stream);
+  // (at d = 32 the window kernel is the faster one: R-MAT, 150 000 nodes, 15 blocks of 16 a window: 72 against 81 us)
+  if (d > 32 && short_windows(windowOrder, (N + kWinRows - 1) / kWinRows, nTcb8 / 2, d, 0))
+    return launch_tcb8_mixed(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, Q, K, V, scaleLog2,
+                             applySoftmax, out, sddmm, nTcb8, stream);
 #define F3S_DISPATCH(DD)                                                                      \
   if (d == DD)                                                                                \
     return applySoftmax                                                                       \
@@ -204,15 +190,11 @@ int launch_attention_heads(const int32_t* rowWindowOffset, const int32_t* window
     return launch_attention_sliced(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, nHeads, (int)ldIn, (int)ldOut, prepared ? 2 : 0, stream);
-  HeadLayout hl = {nHeads, (int)ldIn, (int)ldOut, -1, (int)nRW, nTcb};
-  if (split_short_windows(windowOrder, (int)nRW, nTcb, &hl)) {
-    const int rc = launch_attention_short_windows(rowWindowOffset, windowOrder, sparseAToXidx,
-                                                  bitmap, N, d, dtype, Q, K, V, scaleLog2,
-                                                  applySoftmax, out, nHeads, (int)ldIn, (int)ldOut,
-                                                  kShortWindowBlocks, hl.gridWindows, nTcb,
-                                                  stream);
-    if (rc != 0) return rc;
-  }
+  if (short_windows(windowOrder, (int)nRW, nTcb, d, nHeads))
+    return launch_attention_mixed(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q, K, V,
+                                  scaleLog2, applySoftmax, out, nHeads, (int)ldIn, (int)ldOut, nTcb,
+                                  stream);
+  const HeadLayout hl = {nHeads, (int)ldIn, (int)ldOut, nTcb};
   return dtype == 0 ? window::dispatch_d<_Float16, false>(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N,
                                            d, Q, K, V, scaleLog2, applySoftmax, out, nullptr, hl,
                                            stream)

@@ -17,9 +17,6 @@
 //     locality is lost). f3s_fwd_resident_kernel: a grid that fits the GPU at once, every
 //     workgroup asks the hardware which XCD it runs on and works through that XCD's units.
 //
-// Wave per window, for graphs of short windows (f3s_fwd_unit_kernel, SLICED = false): a unit is a
-// whole window (of one head); the rows are written straight from the registers.
-//
 // The reference has no counterpart: its kernels (src/F3S_kernel.cu:1371-1583) walk one window
 // per thread block from its first TC block to its last. Its window order (src/utils.cu:400-436)
 // is kept: units are issued heavy windows first.
@@ -27,27 +24,19 @@
 
 #include "f3s_common.h"
 #include "f3s_pair_pipeline.h"
+#include "f3s_wave_units.h"
 
 namespace f3s {
 namespace {
 
-using pipe::float4v;
-using pipe::uniform;
-
 constexpr int kMaxPhases = 16;  // slices that an XCD works through one after the other at most
 constexpr int kUnitWaves = 4;  // waves (= units) per workgroup; they do not cooperate
 
-// Stages of a wave's LDS ring and waves per SIMD the register allocator is held to.
-// Column-sliced units are runs of dozens of blocks: two stages, as many waves as the rings allow
-// (four workgroups of four waves per CU at D = 32, two up to D = 128, one above). Short windows are
-// two to eight steps, so most of a wave's time is the chain order -> block range -> ids -> rows in
-// front of the first step: one stage, and up to D = 64 the LDS that frees goes to more waves
-// (100k-node 8 x 32 layer 130 -> 112 us, 60k-node 4 x 64 layer 69 -> 51 us, both together with the
-// whole-line stores and the XCD chunks below).
-constexpr int unit_stages(int d, bool sliced) { return sliced && d <= 64 ? 2 : 1; }
-constexpr int unit_waves_per_simd(int d, bool sliced) {
-  return d <= 32 ? (sliced ? 4 : 5) : d <= 64 ? (sliced ? 2 : 4) : d <= 128 ? 2 : 1;
-}
+// Stages of a wave's LDS ring and waves per SIMD the register allocator is held to. Units are runs of dozens
+// of blocks: two stages, as many waves as the rings allow (four workgroups of four waves per CU at D = 32,
+// two up to D = 128, one above).
+constexpr int unit_stages(int d) { return d <= 64 ? 2 : 1; }
+constexpr int unit_waves_per_simd(int d) { return d <= 32 ? 4 : d <= 128 ? 2 : 1; }
 
 // Partial result of a unit: the O^T tiles as the lanes hold them, one coalesced 1 KiB row of 16
 // bytes per lane and tile (lane (g, c) holds O[q = c][16j + 4g + i] in o[j][i]), then m[16] and
@@ -55,72 +44,6 @@ constexpr int unit_waves_per_simd(int d, bool sliced) {
 template <int D>
 constexpr int partial_floats() {
   return 16 * D + 32;
-}
-
-template <typename ET, int D, bool HEADS>
-__device__ __forceinline__ pipe::Problem<ET> make_problem(const int32_t* sparseAToXidx,
-                                                          const uint8_t* bitmapBytes, const ET* Q,
-                                                          const ET* K, const ET* V, int N,
-                                                          float scaleLog2, int ldIn,
-                                                          int64_t nTcb, int ldQ = 0) {
-  pipe::Problem<ET> pb;
-  pb.sparseAToXidx = sparseAToXidx;
-  pb.bitmapBytes = bitmapBytes;
-  pb.Q = Q;
-  pb.K = K;
-  pb.V = V;
-  pb.N = N;
-  pb.scaleLog2 = scaleLog2;
-  pb.pitchIn = HEADS ? ldIn : D;
-  pb.pitchQ = (HEADS && ldQ > 0) ? ldQ : pb.pitchIn;  // Q may lie apart from K / V
-  pb.nTcb = nTcb;
-  pb.sddmm = nullptr;
-  return pb;
-}
-
-// How the units of a call are dealt to the XCDs. XCD x works on one column slice of one group of
-// heads at a time, for its share of the order's positions:
-//   x = sg + sliceGroups * (hg + headGroups * wg), slice = phase * sliceGroups + sg,
-//   heads hg * headsPerGroup .. + headsPerGroup - 1,
-//   positions [wg * chunk, (wg + 1) * chunk) of every run of windowGroups * chunk positions.
-struct Unit {
-  int pos, head, slice;
-};
-struct XcdSplit {
-  int phases;         // slices an XCD works through, one after the other
-  int sliceGroups;    // slices in work at a time; sliceGroups * headGroups * windowGroups == 8
-  int headGroups;
-  int windowGroups;
-  int headsPerGroup;
-  int chunk;
-  __host__ __device__ int slices() const { return phases * sliceGroups; }
-  // units of one XCD and phase
-  __host__ __device__ int64_t units(int nRW) const {
-    const int64_t run = (int64_t)windowGroups * chunk;
-    return ((int64_t)nRW + run - 1) / run * chunk * headsPerGroup;
-  }
-  // u-th unit of the XCD in the phase: heads innermost (they share ids, bitmaps and lines)
-  __device__ __forceinline__ Unit unit(int xcd, int phase, unsigned u) const {
-    const int sg = xcd & (sliceGroups - 1);  // the group counts are powers of two
-    const int rest = xcd / sliceGroups;
-    const int hg = rest & (headGroups - 1);
-    const int wg = rest / headGroups;
-    const unsigned p = u / (unsigned)headsPerGroup;
-    const unsigned run = p / (unsigned)chunk;
-    Unit r;
-    r.pos = (int)((run * windowGroups + wg) * chunk + (p - run * chunk));
-    r.head = hg * headsPerGroup + (int)(u - p * headsPerGroup);
-    r.slice = phase * sliceGroups + sg;
-    return r;
-  }
-};
-
-// Head groups come first: an XCD that works on some of the heads gathers only their part of the
-// rows, so its share of K + V shrinks without cutting windows into more units. The part stays at
-// least a line of 128 bytes.
-inline XcdSplit split_heads(int d, int heads) {
-  const int groups = head_groups(d, heads);
-  return {1, 1, groups, kXcds / groups, heads / groups, 1};
 }
 
 // probe builds: the partials through the caches instead of past them
@@ -152,68 +75,29 @@ __device__ __forceinline__ void store_partial(const PipeT& pp, float* __restrict
   }
 }
 
-// A window's 16 rows of D floats from the lanes' O^T tiles (already normalised) to memory, through
-// `lds` of the wave (rows_lds_floats<D>() floats): stored as the lanes hold them, a row would leave
-// in pieces of 64 bytes; this way a store instruction fills whole lines.
-template <int D>
-constexpr int rows_lds_floats() {
-  return 16 * (D + 4);
-}
-template <int D>
-__device__ __forceinline__ void store_rows(const float4v (&o)[D / 16], float* lds, int w, int N,
-                                           float* __restrict__ out, int ldOut) {
-  constexpr int LPR = D / 4;  // lanes per row, 16 bytes each
-  const int lane = threadIdx.x & 63;
-  const int g = lane >> 4, c = lane & 15;
-#pragma unroll
-  for (int j = 0; j < D / 16; j++)
-    *reinterpret_cast<float4v*>(lds + c * (D + 4) + 16 * j + 4 * g) = o[j];
-  __builtin_amdgcn_wave_barrier();
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-  for (int k = 0; k < 16 * LPR / 64; k++) {
-    const int q = (k * 64 + lane) / LPR, cv = (k * 64 + lane) % LPR;
-    const int64_t row = (int64_t)w * 16 + q;
-    if (row < N)
-      store_out(out + row * ldOut + cv * 4,
-                *reinterpret_cast<const float4v*>(lds + q * (D + 4) + cv * 4));
-  }
-}
-
-// One wave per unit, kUnitWaves independent units per workgroup. A unit is
-//   SLICED:  the TC blocks of one (window, column slice[, head]); the result is a partial
-//            (m, l, O). Workgroup b: XCD b % 8, then (phase, group of kUnitWaves consecutive
-//            units of that XCD and phase); which position, head and slice a unit is: XcdSplit.
-//   !SLICED: one whole window (of one head, if HEADS); the result is the window's output rows.
-//            Windows of more than maxBlocks TC blocks among the first longPrefix positions of
-//            the order are left to f3s_fwd_kernel, whose waves share a window and whose grid looks
-//            through exactly those positions (with a heavy-first order no long window lies beyond
-//            them; with any other order such a window is simply computed here). XcdSplit deals
-//            head groups and chunks of the order to the XCDs.
+// One wave per unit, kUnitWaves independent units per workgroup. A unit is the TC blocks of one (window,
+// column slice[, head]); the result is a partial (m, l, O). Workgroup b: XCD b % 8, then (phase, group of
+// kUnitWaves consecutive units of that XCD and phase); which position, head and slice a unit is: XcdSplit.
 // NH = 2: D = 64 stands for two heads of 32; split counts such pairs, nHeads heads.
-template <typename ET, int D, bool SOFTMAX, bool SLICED, bool HEADS, int NH = 1>
+template <typename ET, int D, bool SOFTMAX, bool HEADS, int NH = 1>
 __global__ __launch_bounds__(kUnitWaves * 64)
-__attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D, SLICED),
-                                   unit_waves_per_simd(D, SLICED)))) void
+__attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D), unit_waves_per_simd(D)))) void
 f3s_fwd_unit_kernel(const int32_t* __restrict__ windowOrder,
-                    const int32_t* __restrict__ rowWindowOffset,
                     const int32_t* __restrict__ sparseAToXidx,
                     const uint8_t* __restrict__ bitmapBytes,
                     const int32_t* __restrict__ sliceStart, XcdSplit split, int nGroups, int N,
                     int nRW, int64_t nTcb, const ET* __restrict__ Q, const ET* __restrict__ K,
                     const ET* __restrict__ V, float scaleLog2, float* __restrict__ partial,
-                    float* __restrict__ out, int nHeads, int ldIn, int ldOut, int maxBlocks,
-                    int longPrefix, int ldQ) {
-  constexpr int STAGES = unit_stages(D, SLICED);
+                    int nHeads, int ldIn, int ldQ) {
+  constexpr int STAGES = unit_stages(D);
   typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false, STAGES, false, NH> Pipe;
-  constexpr int TH = D / NH / 16;
   extern __shared__ __align__(1024) unsigned char smem[];
 
   const int wave = uniform(threadIdx.x >> 6);
 
   // Workgroup b runs on XCD b % 8; its waves take consecutive units of that XCD's list.
   const int j = blockIdx.x / kXcds;
-  const int phase = j / nGroups;  // 0 if not SLICED
+  const int phase = j / nGroups;
 #ifdef F3S_PROBE_SAME_UNIT
   // probe: the four waves of a workgroup all compute its first unit, at the same time
   const unsigned u = (unsigned)(j - phase * nGroups) * kUnitWaves;
@@ -226,17 +110,10 @@ f3s_fwd_unit_kernel(const int32_t* __restrict__ windowOrder,
   if (pos >= nRW) return;
   const int w = uniform(windowOrder ? windowOrder[pos] : pos);
   if ((unsigned)w >= (unsigned)nRW) return;  // a corrupt order entry must not index out of range
-  int t0, t1;
-  if constexpr (SLICED) {
-    const int64_t at = (int64_t)w * (split.slices() + 1) + un.slice;
-    t0 = uniform(sliceStart[at]);
-    t1 = uniform(sliceStart[at + 1]);
-    if (t1 <= t0) return;  // empty unit: nothing is written, the merge skips it
-  } else {
-    t0 = uniform(rowWindowOffset[w]);
-    t1 = uniform(rowWindowOffset[w + 1]);
-    if (t1 - t0 > maxBlocks && pos < longPrefix) return;  // f3s_fwd_kernel's
-  }
+  const int64_t at = (int64_t)w * (split.slices() + 1) + un.slice;
+  const int t0 = uniform(sliceStart[at]);
+  const int t1 = uniform(sliceStart[at + 1]);
+  if (t1 <= t0) return;  // empty unit: nothing is written, the merge skips it
   // block ranges that do not fit the structure (a mismatched rowWindowOffset) are not followed;
   // the slice index never holds one (sliced_setup_kernel makes such a window empty)
   if (t0 < 0 || (int64_t)t1 > nTcb) return;
@@ -249,27 +126,9 @@ f3s_fwd_unit_kernel(const int32_t* __restrict__ windowOrder,
   pp.init(pb, w, ringAddr, head);
   pp.run(pb, t0, t1);
 
-  if constexpr (SLICED) {
-    const int64_t wh = (int64_t)w * (HEADS ? nHeads : 1) + head * NH;
-    const int64_t stride = (int64_t)split.slices() * partial_floats<D / NH>();
-    store_partial<D, NH>(pp, partial + wh * stride + un.slice * partial_floats<D / NH>(), stride);
-  } else {
-#pragma unroll
-    for (int h = 0; h < NH; h++) {
-      float inv = 1.0f;
-      if constexpr (SOFTMAX) {
-        const float lAll = pipe::row_sum4(pp.l[h]);
-        inv = (lAll == 0.0f) ? 0.0f : 1.0f / lAll;
-      }
-#pragma unroll
-      for (int jj = 0; jj < TH; jj++) pp.o[h * TH + jj] *= inv;
-    }
-    // the wave's ring is free now
-    static_assert(rows_lds_floats<D>() * 4 <= pipe::Geo<D, STAGES>::WAVE_BYTES, "rows fit the ring");
-    store_rows<D>(pp.o,
-                  reinterpret_cast<float*>(smem + (unsigned)wave * pipe::Geo<D, STAGES>::WAVE_BYTES),
-                  w, N, out + (HEADS ? head * D : 0), HEADS ? ldOut : D);
-  }
+  const int64_t wh = (int64_t)w * (HEADS ? nHeads : 1) + head * NH;
+  const int64_t stride = (int64_t)split.slices() * partial_floats<D / NH>();
+  store_partial<D, NH>(pp, partial + wh * stride + un.slice * partial_floats<D / NH>(), stride);
 }
 
 // ---- workspace of the column-sliced schedule (f3s_attention_workspace_bytes) ------------------
@@ -400,8 +259,7 @@ __global__ __launch_bounds__(256) void sliced_setup_kernel(
 // every unit's path.
 template <typename ET, int D, bool SOFTMAX, bool HEADS, int NW, int NH = 1>
 __global__ __launch_bounds__(NW * 64)
-__attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D, true),
-                                   unit_waves_per_simd(D, true)))) void
+__attribute__((amdgpu_waves_per_eu(unit_waves_per_simd(D), unit_waves_per_simd(D)))) void
 f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
                         const int32_t* __restrict__ sliceStart, XcdSplit split, int nRW, int N,
                         int64_t nTcb, int32_t* __restrict__ tickets,
@@ -409,7 +267,7 @@ f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
                         const uint8_t* __restrict__ bitmapBytes, const ET* __restrict__ Q,
                         const ET* __restrict__ K, const ET* __restrict__ V, float scaleLog2,
                         float* __restrict__ partial, int nHeads, int ldIn) {
-  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false, unit_stages(D, true), false, NH> Pipe;
+  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, false, unit_stages(D), false, NH> Pipe;
   extern __shared__ __align__(1024) unsigned char smem[];
   __shared__ int sCtl[2];  // slot of this workgroup; next unit of its sequence
 
@@ -442,7 +300,7 @@ f3s_fwd_resident_kernel(const int32_t* __restrict__ windowOrder,
   const pipe::Problem<ET> pb = make_problem<ET, D, HEADS>(sparseAToXidx, bitmapBytes, Q, K, V, N,
                                                           scaleLog2, ldIn, nTcb);
   const unsigned ringAddr =
-      (unsigned)(uintptr_t)(F3S_LDS unsigned char*)smem + (unsigned)wave * pipe::Geo<D, unit_stages(D, true)>::WAVE_BYTES;
+      (unsigned)(uintptr_t)(F3S_LDS unsigned char*)smem + (unsigned)wave * pipe::Geo<D, unit_stages(D)>::WAVE_BYTES;
 
   // k-th unit of this workgroup's sequence -> index in the XCD's unit space, -1 past its end,
   // -2 when the sequence is over
@@ -642,7 +500,7 @@ XcdSplit choose_split(int N, int d, int heads, int64_t nTcb) {
   // start when the first phase's light ones should fill the end (60k nodes, d = 32: 188 -> 206 us).
   // The slices at a time are a power of two, the nearest one rather than the next (50k nodes, d = 96:
   // 123 us with 4 slices, 146 with 8).
-  const int64_t waves = 32 * 4 * unit_waves_per_simd(dUnit, true);  // of one XCD
+  const int64_t waves = 32 * 4 * unit_waves_per_simd(dUnit);  // of one XCD
   if (s.units(nRW) < 2 * waves) {
     while (s.windowGroups > 1 && (nTcb < 0 ? s.sliceGroups < need : 3 * s.sliceGroups <= 2 * need)) {
       s.sliceGroups *= 2;
@@ -715,9 +573,9 @@ int resident_grid(int* grid) {
     if (dev >= 0 && dev < kMaxDev) cusOf[dev] = cus;
   }
   // the rings plus the 1 KiB the two control words cost in front of the 1 KiB-aligned rings
-  constexpr size_t lds = (size_t)NW * pipe::Geo<D, unit_stages(D, true)>::WAVE_BYTES + 1024;
+  constexpr size_t lds = (size_t)NW * pipe::Geo<D, unit_stages(D)>::WAVE_BYTES + 1024;
   int perCu = (int)((160 * 1024) / lds);
-  const int byWaves = unit_waves_per_simd(D, true) * 4 / NW;
+  const int byWaves = unit_waves_per_simd(D) * 4 / NW;
   if (perCu > byWaves) perCu = byWaves;
   if (perCu < 1) perCu = 1;
   int gsz = cus * perCu / kXcds * kXcds;
@@ -737,7 +595,7 @@ int launch_sliced_units(const int32_t* rwo, const int32_t* order, const int32_t*
                         float scaleLog2, float* out, int32_t* tickets, int32_t* sliceStart,
                         float* partial, const SlicedLayout& L, int heads, int ldIn, int ldOut,
                         int64_t nTcb, hipStream_t stream, int ldQ = 0) {
-  constexpr size_t lds = (size_t)kUnitWaves * pipe::Geo<D, unit_stages(D, true)>::WAVE_BYTES;
+  constexpr size_t lds = (size_t)kUnitWaves * pipe::Geo<D, unit_stages(D)>::WAVE_BYTES;
   if (resident_requested()) {
     auto kernel = f3s_fwd_resident_kernel<ET, D, SOFTMAX, HEADS, kUnitWaves, NH>;
     if (int rc = allow_lds(kernel, lds)) return rc;
@@ -747,15 +605,15 @@ int launch_sliced_units(const int32_t* rwo, const int32_t* order, const int32_t*
                        sliceStart, resident_split(L.split), nRW, N, nTcb, tickets, atox, bm, Q, K, V, scaleLog2,
                        partial, heads, ldIn);
   } else {
-    auto kernel = f3s_fwd_unit_kernel<ET, D, SOFTMAX, true, HEADS, NH>;
+    auto kernel = f3s_fwd_unit_kernel<ET, D, SOFTMAX, HEADS, NH>;
     if (int rc = allow_lds(kernel, lds)) return rc;
     const int64_t nGroups = (L.split.units(nRW) + kUnitWaves - 1) / kUnitWaves;
     const int64_t grid = L.split.phases * nGroups * kXcds;
     if (grid >= ((int64_t)1 << 31))
       return fail(-2, "f3s_attention: too many (window, slice, head) units for one launch");
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kUnitWaves * 64), lds, stream, order, rwo,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kUnitWaves * 64), lds, stream, order,
                        atox, bm, sliceStart, L.split, (int)nGroups, N, nRW, nTcb, Q, K, V, scaleLog2,
-                       partial, out, heads, ldIn, ldOut, 0, 0, ldQ);
+                       partial, heads, ldIn, ldQ);
   }
   F3S_HIP_CHECK(hipGetLastError());
   return 0;
@@ -865,100 +723,6 @@ int launch_attention_sliced(const int32_t* rowWindowOffset, const int32_t* windo
   }
   F3S_FOR_EACH_HEAD_DIM(F3S_SLICED)
 #undef F3S_SLICED
-  return fail(-2, "f3s_attention: head dim %d unsupported (a multiple of 32 up to 256)", d);
-}
-
-namespace {
-
-// Positions of the order an XCD takes in a row: windows that follow each other in the order (equal
-// block counts are in window order) often name the same rows, which then come from one L2
-// (60k-node community graph, 4 x 64: 69 -> 52 us; 8, 16 and 64 windows are alike, 256 leave the
-// XCDs unevenly loaded). Only short windows are dealt in chunks: of long ones in heavy-first order
-// the first XCD would get the sixteen heaviest.
-constexpr int kShortChunk = 16;
-
-// 32-wide heads are computed one by one where one or two pairs of them make too few waves to fill the CUs: a
-// wave then takes longer for two heads than two waves for one each. Head by head against pairs, us; blocks of
-// the graph. One pair: uniform 10 000 10.7 against 12.0, 19 000 14.1 15.7, 26 000 17.8 16.9, 29 000 18.3 17.2;
-// communities 9 000 9.7 11.1, 31 000 17.1 17.7 or 19.3 18.6, 38 000 23.3 23.1; power-law 24 000 24.1 25.5, 40 000
-// 32.1 33.0; R-MAT 13 000 18.6 22.5, 31 000 28.0 29.2, 37 000 29.6 30.9, 51 000 35.9 35.9, 69 000 44.4 42.7. Two
-// pairs: uniform 10 000 14.7 15.3, 23 000 23.8 20.8; communities 9 000 12.9 14.0, 31 000 26.2 25.9; R-MAT 13 000
-// 23.6 25.5, 23 000 31.9 32.6, 26 000 34.0 34.8, 31 000 41.0 39.0; power-law 24 000 30.0 31.0, 40 000 47.8 45.9.
-// Three and more lose at most 3 % (four: R-MAT 13 000 30.9 31.7) and gain 1 to 25 % (three: communities 9 000
-// 18.5 16.7; eight: uniform 6 000 28.7 26.5).
-bool pairs_fill(int64_t nTcb, int pairs) { return pairs >= 3 || nTcb * pairs >= 50000; }
-
-// NH = 2: D = 64 stands for two heads of 32
-template <typename ET, int D, bool SOFTMAX, int NH = 1>
-int launch_short_d(const int32_t* rwo, const int32_t* order, const int32_t* atox,
-                   const uint64_t* bitmap, int N, const void* Q, const void* K, const void* V,
-                   float scaleLog2, float* out, int nHeads, int ldIn, int ldOut, int maxBlocks,
-                   int longPrefix, int64_t nTcb, hipStream_t stream) {
-  if constexpr (D == 32) {
-    if (heads_in_pairs(D, nHeads) && pairs_fill(nTcb, nHeads / 2))
-      return launch_short_d<ET, 64, SOFTMAX, 2>(rwo, order, atox, bitmap, N, Q, K, V, scaleLog2, out,
-                                                nHeads, ldIn, ldOut, maxBlocks, longPrefix, nTcb, stream);
-  }
-  const int nRW = (N + kWinRows - 1) / kWinRows;
-  XcdSplit split = split_heads(D, nHeads > 0 ? nHeads / NH : 1);
-  split.chunk = kShortChunk;
-  const int64_t nGroups = (split.units(nRW) + kUnitWaves - 1) / kUnitWaves;
-  if (nGroups * kXcds >= ((int64_t)1 << 31))
-    return fail(-2, "f3s_attention: too many (window, head) units for one launch");
-  const dim3 grid((unsigned)(nGroups * kXcds)), block(kUnitWaves * 64);
-  const auto* bm = reinterpret_cast<const uint8_t*>(bitmap);
-  const auto* q = static_cast<const ET*>(Q);
-  const auto* k = static_cast<const ET*>(K);
-  const auto* v = static_cast<const ET*>(V);
-  constexpr size_t lds = (size_t)kUnitWaves * pipe::Geo<D, unit_stages(D, false)>::WAVE_BYTES;
-  if (NH > 1 || nHeads > 0) {
-    auto kernel = f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, true, NH>;
-    if (int rc = allow_lds(kernel, lds)) return rc;
-    hipLaunchKernelGGL(kernel, grid, block, lds,
-                       stream, order, rwo, atox, bm, nullptr, split, (int)nGroups, N, nRW, nTcb, q, k, v,
-                       scaleLog2, nullptr, out, nHeads, ldIn, ldOut, maxBlocks, longPrefix, 0);
-  } else if constexpr (NH == 1) {
-    if (int rc = allow_lds(f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, false>, lds)) return rc;
-    hipLaunchKernelGGL((f3s_fwd_unit_kernel<ET, D, SOFTMAX, false, false>), grid, block, lds,
-                       stream, order, rwo, atox, bm, nullptr, split, (int)nGroups, N, nRW, nTcb, q, k, v,
-                       scaleLog2, nullptr, out, 1, D, D, maxBlocks, longPrefix, 0);
-  }
-  F3S_HIP_CHECK(hipGetLastError());
-  return 0;
-}
-
-}  // namespace
-
-// One wave per window, for every window except those of more than maxBlocks TC blocks among the
-// first longPrefix positions of the order (nHeads = 0: contiguous single head).
-int launch_attention_short_windows(const int32_t* rowWindowOffset, const int32_t* windowOrder,
-                                   const int32_t* sparseAToXidx, const uint64_t* bitmap, int N,
-                                   int d, int dtype, const void* Q, const void* K, const void* V,
-                                   float scaleLog2, int applySoftmax, float* out, int nHeads,
-                                   int ldIn, int ldOut, int maxBlocks, int longPrefix,
-                                   int64_t nTcb, hipStream_t stream) {
-#define F3S_SHORT(DD)                                                                          \
-  if (d == DD) {                                                                               \
-    if (dtype == 0)                                                                            \
-      return applySoftmax ? launch_short_d<_Float16, DD, true>(                                \
-                                rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, Q, K,  \
-                                V, scaleLog2, out, nHeads, ldIn, ldOut, maxBlocks,       \
-                                longPrefix, nTcb, stream)                                      \
-                          : launch_short_d<_Float16, DD, false>(                               \
-                                rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, Q, K,  \
-                                V, scaleLog2, out, nHeads, ldIn, ldOut, maxBlocks,       \
-                                longPrefix, nTcb, stream);                                     \
-    return applySoftmax ? launch_short_d<__bf16, DD, true>(                                    \
-                              rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, Q, K, V, \
-                              scaleLog2, out, nHeads, ldIn, ldOut, maxBlocks,            \
-                              longPrefix, nTcb, stream)                                        \
-                        : launch_short_d<__bf16, DD, false>(                                   \
-                              rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, Q, K, V, \
-                              scaleLog2, out, nHeads, ldIn, ldOut, maxBlocks,            \
-                              longPrefix, nTcb, stream);                                       \
-  }
-  F3S_FOR_EACH_HEAD_DIM(F3S_SHORT)
-#undef F3S_SHORT
   return fail(-2, "f3s_attention: head dim %d unsupported (a multiple of 32 up to 256)", d);
 }
 

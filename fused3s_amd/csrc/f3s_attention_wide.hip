@@ -14,8 +14,7 @@ int launch_window_wide(const int32_t* rowWindowOffset, const int32_t* windowOrde
                        int dtype, const void* Q, const void* K, const void* V, float scaleLog2,
                        int applySoftmax, float* out, unsigned long long* cuTimer, int nHeads,
                        int ldIn, int ldOut, int64_t nTcb, hipStream_t stream) {
-  const int nRW = (N + kWinRows - 1) / kWinRows;
-  const window::HeadLayout hl = {nHeads, ldIn, ldOut, -1, nRW, nTcb};
+  const window::HeadLayout hl = {nHeads, ldIn, ldOut, nTcb};
   return dtype == 0
              ? window::dispatch_d<_Float16, true>(rowWindowOffset, windowOrder, sparseAToXidx,
                                                   bitmap, N, d, Q, K, V, scaleLog2, applySoftmax,

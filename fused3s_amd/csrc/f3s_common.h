@@ -98,12 +98,19 @@ int launch_attention_sliced(const int32_t* rowWindowOffset, const int32_t* windo
                             size_t wsBytes, int64_t nTcb, int nHeads, int ldIn, int ldOut,
                             int mode, hipStream_t stream);
 
-int launch_attention_short_windows(const int32_t* rowWindowOffset, const int32_t* windowOrder,
-                                   const int32_t* sparseAToXidx, const uint64_t* bitmap, int N,
-                                   int d, int dtype, const void* Q, const void* K, const void* V,
-                                   float scaleLog2, int applySoftmax, float* out, int nHeads,
-                                   int ldIn, int ldOut, int maxBlocks, int longPrefix,
-                                   int64_t nTcb, hipStream_t stream);
+// graphs of short windows (f3s_attention_mixed.hip): a wave per window, workgroups for the long ones
+// nHeads = 0: contiguous single head; windowOrder may be null; nTcb16: blocks of 16 columns
+bool mixed_windows_pay(bool ordered, int nRW, int64_t nTcb16, int d, int nHeads);
+int launch_attention_mixed(const int32_t* rowWindowOffset, const int32_t* windowOrder,
+                           const int32_t* sparseAToXidx, const uint64_t* bitmap, int N, int d, int dtype,
+                           const void* Q, const void* K, const void* V, float scaleLog2,
+                           int applySoftmax, float* out, int nHeads, int ldIn, int ldOut,
+                           int64_t nTcb, hipStream_t stream);
+int launch_tcb8_mixed(const int32_t* rowWindowOffset, const int32_t* windowOrder,
+                      const int32_t* sparseAToXidx, const uint64_t* bitmap, int N, int d,
+                      const void* Q, const void* K, const void* V, float scaleLog2,
+                      int applySoftmax, float* out, float* sddmm, int64_t nTcb8,
+                      hipStream_t stream);
 
 // The workgroup-per-window kernel built with 64-bit row offsets in its gathers, for K / V of
 // 4 GiB and more (f3s_attention_wide.hip). nHeads = 0: contiguous single head.

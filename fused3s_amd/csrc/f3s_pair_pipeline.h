@@ -737,5 +737,114 @@ struct PairPipeline {
   }
 };
 
+// ---- epilogue of workgroups whose waves share a window. Every thread of the workgroup calls these three; the
+// buffers lie at the start of smem, where the rings were.
+
+// The waves' partial (m, l, O) into smem: m and l [NH][NWAVES][16], O [NWAVES][16][D + 4].
+template <int D, int NWAVES, bool SOFTMAX, int NH, typename PipeT>
+__device__ __forceinline__ void put_partials(const PipeT& pp, unsigned char* smem, int wave) {
+  int lane = threadIdx.x & 63;
+  pin(lane);  // nothing below is computed in front of the caller's loop and kept in registers
+  const int g = lane >> 4, c = lane & 15;
+  __syncthreads();
+  float* sM = reinterpret_cast<float*>(smem);
+  float* sL = sM + NH * NWAVES * 16;
+  float* sO = sL + NH * NWAVES * 16;
+#pragma unroll
+  for (int h = 0; h < NH; h++) {
+    float l = pp.l[h];
+    if constexpr (SOFTMAX) l = row_sum4(l);
+    if (g == 0) {
+      sM[(h * NWAVES + wave) * 16 + c] = pp.m[h];
+      sL[(h * NWAVES + wave) * 16 + c] = l;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < D / 16; j++)
+    *reinterpret_cast<float4v*>(&sO[(wave * 16 + c) * (D + 4) + 16 * j + 4 * g]) = pp.o[j];
+  __syncthreads();
+}
+
+// The window's rows (16 bytes of a row per element, dealt to the threads) from the partials of four
+// waves, first .. first + 3: log-sum-exp, not yet divided by l.
+template <int D, int NWAVES, bool SOFTMAX, int NH>
+struct MergedRows {
+  static constexpr int VEC_PER_ROW = D / 4, THREADS = NWAVES * 64;
+  static constexpr int N = (16 * VEC_PER_ROW + THREADS - 1) / THREADS;  // elements of a thread
+  float4v acc[N];
+  float m[N], l[N];
+  __device__ __forceinline__ static bool has(int tid, int i) {
+    return 16 * VEC_PER_ROW % THREADS == 0 || i * THREADS + tid < 16 * VEC_PER_ROW;
+  }
+  __device__ __forceinline__ void merge(const unsigned char* smem, int first) {
+    int tid = threadIdx.x;
+    pin(tid);
+    const float* sM = reinterpret_cast<const float*>(smem);
+    const float* sL = sM + NH * NWAVES * 16;
+    const float* sO = sL + NH * NWAVES * 16;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      if (!has(tid, i)) continue;
+      const int q = (i * THREADS + tid) / VEC_PER_ROW, cv = (i * THREADS + tid) % VEC_PER_ROW;
+      const int h = NH > 1 ? cv / (VEC_PER_ROW / NH) : 0;
+      const float* mOf = sM + (h * NWAVES + first) * 16 + q;
+      const float* lOf = sL + (h * NWAVES + first) * 16 + q;
+      const float* oOf = sO + (first * 16 + q) * (D + 4) + cv * 4;
+      acc[i] = float4v{0.f, 0.f, 0.f, 0.f};
+      m[i] = mOf[0];
+      l[i] = 0.0f;
+      if constexpr (SOFTMAX) {
+#pragma unroll
+        for (int v = 1; v < 4; v++) m[i] = fmaxf(m[i], mOf[v * 16]);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const float4v o = *reinterpret_cast<const float4v*>(oOf + v * 16 * (D + 4));
+        if constexpr (SOFTMAX) {
+          const float f = fast_exp2(mOf[v * 16] - m[i]);
+          l[i] = fmaf(f, lOf[v * 16], l[i]);
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[i][e] = fmaf(f, o[e], acc[i][e]);
+        } else {
+          acc[i] += o;
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void add(const MergedRows& b) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      if constexpr (SOFTMAX) {
+        const float both = fmaxf(m[i], b.m[i]);
+        const float fa = fast_exp2(m[i] - both), fb = fast_exp2(b.m[i] - both);
+        m[i] = both;
+        l[i] = fmaf(fb, b.l[i], fa * l[i]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[i][e] = fmaf(fb, b.acc[i][e], fa * acc[i][e]);
+      } else {
+        acc[i] += b.acc[i];
+      }
+    }
+  }
+  // out points at the first column, rows are pitchOut floats apart
+  __device__ __forceinline__ void store(int w, int rows, float* __restrict__ out, int pitchOut) const {
+    int tid = threadIdx.x;
+    pin(tid);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      if (!has(tid, i)) continue;
+      const int q = (i * THREADS + tid) / VEC_PER_ROW, cv = (i * THREADS + tid) % VEC_PER_ROW;
+      const int64_t row = (int64_t)w * 16 + q;
+      if (row >= rows) continue;
+      float4v r = acc[i];
+      if constexpr (SOFTMAX) {
+        const float inv = (l[i] == 0.0f) ? 0.0f : 1.0f / l[i];
+        r *= inv;
+      }
+      store_out(out + row * pitchOut + cv * 4, out_vec{r[0], r[1], r[2], r[3]});
+    }
+  }
+};
+
 }  // namespace pipe
 }  // namespace f3s

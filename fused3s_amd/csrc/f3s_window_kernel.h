@@ -32,16 +32,11 @@ using pipe::kLog2e;
 //   TEAM_SHORT  one workgroup for every window: four waves of one stage. Four workgroups per CU at
 //               D = 32, three at D = 64 (two stages allow two), two up to D = 128, one above.
 //   TEAM_PAIRS  the same with two stages at D = 32, where they cost no workgroup (see two_stages).
-//   TEAM_LONG   the few long windows of a graph of short ones, one workgroup after the other per CU:
-//               as many bytes in flight as one CU's LDS holds, eight waves of two stages up to
-//               D = 64, eight of one stage up to D = 128, four above.
-enum Team { TEAM_SHORT, TEAM_PAIRS, TEAM_LONG };
-constexpr int team_waves(Team t, int d) { return t == TEAM_LONG && d <= 128 ? 8 : 4; }
-constexpr int team_stages(Team t, int d) { return t != TEAM_SHORT && d <= 64 ? 2 : 1; }
-constexpr int waves_per_simd(Team t, int d) {
-  if (d > 128) return 1;
-  return t == TEAM_LONG || d > 64 ? 2 : d > 32 ? 3 : 4;
-}
+// Graphs of short windows take f3s_fwd_mixed_kernel instead (f3s_attention_units.hip).
+enum Team { TEAM_SHORT, TEAM_PAIRS };
+constexpr int kTeamWaves = 4;  // MergedRows takes four
+constexpr int team_stages(Team t) { return t == TEAM_SHORT ? 1 : 2; }
+constexpr int waves_per_simd(int d) { return d > 128 ? 1 : d > 64 ? 2 : d > 32 ? 3 : 4; }
 
 // Whether TEAM_PAIRS takes the windows rather than TEAM_SHORT (nTcb16: blocks of 16 columns). At D = 32
 // four workgroups fit a CU either way, so the second stage only has to pay for its longer loop.
@@ -76,7 +71,7 @@ inline bool two_stages(int d, int64_t nTcb16, int heads, int N) {
 // LDS of a workgroup: its waves' rings
 constexpr size_t team_lds(Team t, int d) {
   const int dp = d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : 256;
-  return (size_t)team_waves(t, d) * (team_stages(t, d) * 128 * dp + 2 * 768);
+  return (size_t)kTeamWaves * (team_stages(t) * 128 * dp + 2 * 768);
 }
 
 // Constant-rate (100 MHz) timestamp shared by all CUs, and an id of the CU this wave runs on:
@@ -128,21 +123,19 @@ __global__ void reset_window_cursor_kernel() {
 // NH = 2: D = 64 stands for two heads of 32; nHeads and headGroups count such pairs.
 template <typename ET, int D, Team TEAM, bool SOFTMAX, bool CLOCKED, bool HEADS, bool W8,
           bool WIDE, bool PERSIST = false, int NH = 1>
-__global__ __launch_bounds__(team_waves(TEAM, D) * 64)
-__attribute__((amdgpu_waves_per_eu(waves_per_simd(TEAM, D), waves_per_simd(TEAM, D)))) void
+__global__ __launch_bounds__(kTeamWaves * 64)
+__attribute__((amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D)))) void
 f3s_fwd_kernel(
     const int32_t* __restrict__ rowWindowOffset, const int32_t* __restrict__ windowOrder,
     const int32_t* __restrict__ sparseAToXidx, const uint8_t* __restrict__ bitmapBytes, int N,
     int nRW, int64_t nTcb, const ET* __restrict__ Q, const ET* __restrict__ K,
     const ET* __restrict__ V, float scaleLog2, float* __restrict__ out,
     unsigned long long* __restrict__ cuTimer, int nHeads, int headGroups, int ldIn, int ldOut,
-    float* __restrict__ sddmm, int minBlocks, int nPositions) {
-  constexpr int NWAVES = team_waves(TEAM, D);
-  constexpr int WAVE_BYTES = pipe::Geo<D, team_stages(TEAM, D)>::WAVE_BYTES;
+    float* __restrict__ sddmm) {
+  constexpr int NWAVES = kTeamWaves;
+  constexpr int WAVE_BYTES = pipe::Geo<D, team_stages(TEAM)>::WAVE_BYTES;
   static_assert(team_lds(TEAM, D) == (size_t)NWAVES * WAVE_BYTES, "what the launch asks for");
-  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, W8, team_stages(TEAM, D), WIDE, NH> Pipe;
-  constexpr int T = D / 16;
-  constexpr int OSTRIDE = D + 4;
+  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, W8, team_stages(TEAM), WIDE, NH> Pipe;
   constexpr int BPS = W8 ? 4 : 2;  // blocks of the structure per pipeline step
   extern __shared__ __align__(1024) unsigned char smem[];
   unsigned long long tBegin = 0;
@@ -150,59 +143,20 @@ f3s_fwd_kernel(
 
   static_assert(!PERSIST || (!CLOCKED && !HEADS && !W8), "the persistent form is single-head");
   __shared__ int sNextPos[2];
-  constexpr bool scan = TEAM == TEAM_LONG;
-  __shared__ int sUnitCount;
-  __shared__ int sUnitList[scan ? NWAVES * 64 : 1];
   int pos = (int)blockIdx.x, head = 0;
-  if constexpr (HEADS && !scan) {
+  if constexpr (HEADS) {
     const unsigned perGroup = (unsigned)nHeads / (unsigned)headGroups;
     const unsigned xcd = blockIdx.x % kXcds, u = blockIdx.x / kXcds, p = u / perGroup;
     const unsigned shares = kXcds / (unsigned)headGroups;  // of the positions
     pos = (int)(p * shares + xcd / (unsigned)headGroups);
     head = (int)(xcd % (unsigned)headGroups * perGroup + (u - p * perGroup));
-    if (pos >= nPositions) return;
-  }
-  // A launch that shares the windows with the wave-per-window kernel (TEAM_LONG, minBlocks >= 0)
-  // covers the (position, head) units of the order's first nPositions positions with a grid of its
-  // own size: thread t of workgroup b looks at unit b + t * gridDim.x, and the workgroup computes
-  // the units it finds long, one after the other. When no window is long, which is the usual
-  // case on a graph of short windows, the launch is a few hundred workgroups that read a count each
-  // and leave, instead of one workgroup per unit; in a heavy-first order the long units are the
-  // first ones and are dealt out round-robin.
-  int nMine = 1;
-  if constexpr (scan) {
-    if (threadIdx.x == 0) sUnitCount = 0;
-    __syncthreads();
-    const int heads = HEADS ? nHeads : 1;
-    const int64_t nUnits = (int64_t)nPositions * heads;
-    const int64_t u = (int64_t)blockIdx.x + (int64_t)threadIdx.x * (int64_t)gridDim.x;
-    if (u < nUnits) {
-      const int p = (int)(u / heads);
-      const int w = windowOrder ? windowOrder[p] : p;
-      if ((unsigned)w < (unsigned)nRW) {
-        const int t0 = rowWindowOffset[w];
-        const int t1 = rowWindowOffset[w + 1];
-        if (t0 >= 0 && (int64_t)t1 <= nTcb && t1 - t0 > minBlocks)
-          sUnitList[atomicAdd(&sUnitCount, 1)] = (int)u;
-      }
-    }
-    __syncthreads();
-    nMine = sUnitCount;
+    if (pos >= nRW) return;
   }
   const int pitchOut = HEADS ? ldOut : D;
-  const int lane = threadIdx.x & 63;
   const int wave = pipe::uniform(threadIdx.x >> 6);
-  const int g = lane >> 4;
-  const int c = lane & 15;
   for (int iter = 0;; iter++) {
-  if constexpr (scan) {
-    if (iter >= nMine) break;
-    const int u = sUnitList[iter];
-    pos = HEADS ? u / nHeads : u;
-    head = HEADS ? u - pos * nHeads : 0;
-  }
   if constexpr (PERSIST) {
-    if (pos >= nPositions) break;
+    if (pos >= nRW) break;
     // position of the window after this one; read at the end of this iteration
     if (threadIdx.x == 0) sNextPos[iter & 1] = atomicAdd(&g_windowCursor, 1) + (int)gridDim.x;
   }
@@ -215,9 +169,6 @@ f3s_fwd_kernel(
   // block ranges that do not fit the structure (a mismatched rowWindowOffset) are not followed:
   // the window is treated as empty
   if (t0 < 0 || (int64_t)t1 > nTcb || t1 < t0) t1 = t0;
-  // windows of at most minBlocks blocks belong to the wave-per-window kernel of the same call
-  // (f3s_fwd_unit_kernel); -1 when this kernel computes every window
-  if (t1 - t0 <= minBlocks) break;
   const int nSteps = (t1 - t0 + BPS - 1) / BPS;
 
   pipe::Problem<ET> pb;
@@ -245,70 +196,13 @@ f3s_fwd_kernel(
     if (re > rb) pp.run(pb, rb, re);
   }
 
-  // ---- merge the waves' partial (m, l, O) and write the window's rows. The merge buffers reuse
-  // the rings' memory once every wave has left its loop.
-  __syncthreads();
-  float* sM = reinterpret_cast<float*>(smem);                    // [NH][NWAVES][16]
-  float* sL = sM + NH * NWAVES * 16;                             // [NH][NWAVES][16]
-  float* sO = sL + NH * NWAVES * 16;                             // [NWAVES][16][OSTRIDE]
-#pragma unroll
-  for (int h = 0; h < NH; h++) {
-    float l = pp.l[h];
-    if constexpr (SOFTMAX) l = pipe::row_sum4(l);
-    if (g == 0) {
-      sM[(h * NWAVES + wave) * 16 + c] = pp.m[h];
-      sL[(h * NWAVES + wave) * 16 + c] = l;
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < T; j++)
-    *reinterpret_cast<float4v*>(&sO[(wave * 16 + c) * OSTRIDE + 16 * j + 4 * g]) = pp.o[j];
-  __syncthreads();
-
-  constexpr int VEC_PER_ROW = D / 4;
-  for (int idx = threadIdx.x; idx < 16 * VEC_PER_ROW; idx += NWAVES * 64) {
-    const int q = idx / VEC_PER_ROW;
-    const int cv = idx % VEC_PER_ROW;
-    const int64_t row = (int64_t)w * 16 + q;
-    if (row >= N) continue;
-    float4 acc = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (SOFTMAX) {
-      const int ml = (NH > 1 ? cv / (VEC_PER_ROW / NH) * NWAVES * 16 : 0) + q;  // of this head and row
-      float mAll = sM[ml];
-#pragma unroll
-      for (int v = 1; v < NWAVES; v++) mAll = fmaxf(mAll, sM[v * 16 + ml]);
-      float lAll = 0.0f;
-#pragma unroll
-      for (int v = 0; v < NWAVES; v++) {
-        const float f = pipe::fast_exp2(sM[v * 16 + ml] - mAll);
-        lAll = fmaf(f, sL[v * 16 + ml], lAll);
-        const float4 ov = *reinterpret_cast<const float4*>(&sO[(v * 16 + q) * OSTRIDE + cv * 4]);
-        acc.x = fmaf(f, ov.x, acc.x);
-        acc.y = fmaf(f, ov.y, acc.y);
-        acc.z = fmaf(f, ov.z, acc.z);
-        acc.w = fmaf(f, ov.w, acc.w);
-      }
-      const float inv = (lAll == 0.0f) ? 0.0f : 1.0f / lAll;
-      acc.x *= inv;
-      acc.y *= inv;
-      acc.z *= inv;
-      acc.w *= inv;
-    } else {
-#pragma unroll
-      for (int v = 0; v < NWAVES; v++) {
-        const float4 ov = *reinterpret_cast<const float4*>(&sO[(v * 16 + q) * OSTRIDE + cv * 4]);
-        acc.x += ov.x;
-        acc.y += ov.y;
-        acc.z += ov.z;
-        acc.w += ov.w;
-      }
-    }
-    store_out(out + row * pitchOut + head * D + cv * 4, out_vec{acc.x, acc.y, acc.z, acc.w});
-  }
+  // one LDS merge per window; the buffers reuse the rings' memory once every wave has left its loop
+  pipe::put_partials<D, NWAVES, SOFTMAX, NH>(pp, smem, wave);
+  pipe::MergedRows<D, NWAVES, SOFTMAX, NH> rows;
+  rows.merge(smem, 0);
+  rows.store(w, N, out + head * D, pitchOut);
   } while (false);
-  if constexpr (!PERSIST) {
-    if constexpr (!scan) break;
-  }
+  if constexpr (!PERSIST) break;
   __syncthreads();  // the merge buffers are free again, the next position has arrived
   if constexpr (PERSIST) pos = sNextPos[iter & 1];
   }
@@ -344,8 +238,6 @@ struct HeadLayout {
   int nHeads;       // 0: contiguous [N, d] single head
   int ldIn;         // row pitch of Q/K/V in elements
   int ldOut;        // row pitch of out in floats
-  int minBlocks;    // this kernel skips windows of at most minBlocks blocks (-1: none)
-  int gridWindows;  // positions of the window order this launch covers (<= nRW)
   int64_t nTcb;     // TC blocks of the structure (bounds every window's block range)
 };
 
@@ -377,10 +269,8 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
   const auto* q = static_cast<const ET*>(Q);
   const auto* k = static_cast<const ET*>(K);
   const auto* v = static_cast<const ET*>(V);
-  const unsigned gw = (unsigned)(hl.gridWindows < nRW ? hl.gridWindows : nRW);
-  if (gw == 0) return 0;
+  const unsigned gw = (unsigned)nRW;
   const int heads = hl.nHeads > 0 ? hl.nHeads : 1;
-  const unsigned units = gw * (unsigned)heads;
   const int headGroups = head_groups(D, heads);
   const unsigned shares = kXcds / (unsigned)headGroups;
   const unsigned headGrid = (gw + shares - 1) / shares * (heads / headGroups) * kXcds;
@@ -390,25 +280,13 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
                                  HEADS_ ? NH : 1>;                                             \
     constexpr size_t lds = team_lds(TEAM_, D);                                                 \
     if (int rc = allow_lds(kernel, lds)) return rc;                                            \
-    hipLaunchKernelGGL(kernel, dim3(GRID), dim3(team_waves(TEAM_, D) * 64), lds, stream, rwo,  \
+    hipLaunchKernelGGL(kernel, dim3(GRID), dim3(kTeamWaves * 64), lds, stream, rwo,            \
                        order, atox, bm, N, nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer,     \
                        heads, headGroups, hl.nHeads > 0 ? hl.ldIn : D,                         \
                        hl.nHeads > 0 ? hl.ldOut : D,                                           \
-                       (float*)nullptr, hl.minBlocks, (int)gw);                                \
+                       (float*)nullptr);                                                       \
   }
-  if (hl.minBlocks >= 0) {
-    // a launch next to the wave-per-window kernel looks for its units itself (see the kernel): one
-    // unit per thread at most, two workgroups per CU (one at a time) when that is enough
-    if constexpr (WIDE) {
-      return fail(-2, "f3s_attention: windows are not shared in the 64-bit form");
-    } else {
-      const unsigned threads = (unsigned)team_waves(TEAM_LONG, D) * 64;
-      unsigned grid = (units + threads - 1) / threads;
-      if (grid < 512u) grid = units < 512u ? units : 512u;
-      if (NH > 1 || hl.nHeads > 0) F3S_LAUNCH(TEAM_LONG, false, true, grid)
-      else if constexpr (NH == 1) F3S_LAUNCH(TEAM_LONG, false, false, grid)
-    }
-  } else if (NH > 1) {
+  if (NH > 1) {
     F3S_LAUNCH(TEAM_SHORT, false, true, headGrid)
   } else if (!WIDE && hl.nHeads == 0 && !cuTimer && window_cursor_requested()) {
     // F3S_WINDOW_PERSISTENT=1: as many workgroups as the GPU holds at once, windows drawn from
@@ -416,7 +294,7 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
     if constexpr (!WIDE && NH == 1) {
       auto kernel = f3s_fwd_kernel<ET, D, TEAM_SHORT, SOFTMAX, false, false, false, false, true>;
       constexpr size_t lds = team_lds(TEAM_SHORT, D);
-      constexpr int threads = team_waves(TEAM_SHORT, D) * 64;
+      constexpr int threads = kTeamWaves * 64;
       if (int rc = allow_lds(kernel, lds)) return rc;
       int dev = 0, nCu = 0, perCu = 0;
       F3S_HIP_CHECK(hipGetDevice(&dev));
@@ -427,8 +305,8 @@ int launch_d(const int32_t* rwo, const int32_t* order, const int32_t* atox, cons
       if (grid > gw) grid = gw;
       hipLaunchKernelGGL(reset_window_cursor_kernel<0>, dim3(1), dim3(1), 0, stream);
       hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream, rwo, order, atox, bm, N,
-                         nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer, 1, 1, D, D, (float*)nullptr,
-                         hl.minBlocks, (int)gw);
+                         nRW, hl.nTcb, q, k, v, scaleLog2, out, cuTimer, 1, 1, D, D,
+                         (float*)nullptr);
     }
   } else if constexpr (NH == 1) {
     constexpr Team kPairs = D <= 32 ? TEAM_PAIRS : TEAM_SHORT;  // no second kernel above D = 32
@@ -460,13 +338,11 @@ int launch_tcb8(const int32_t* rwo, const int32_t* order, const int32_t* atox,
   const size_t lds = pairs ? team_lds(kPairs, D) : team_lds(TEAM_SHORT, D);
   auto kernel = pairs ? f3s_fwd_kernel<_Float16, D, kPairs, SOFTMAX, false, false, true, WIDE>
                       : f3s_fwd_kernel<_Float16, D, TEAM_SHORT, SOFTMAX, false, false, true, WIDE>;
-  static_assert(team_waves(kPairs, D) == team_waves(TEAM_SHORT, D), "one launch for both");
   if (int rc = allow_lds(kernel, lds)) return rc;
-  hipLaunchKernelGGL(kernel, dim3(nRW), dim3(team_waves(TEAM_SHORT, D) * 64), lds, stream, rwo, order, atox,
+  hipLaunchKernelGGL(kernel, dim3(nRW), dim3(kTeamWaves * 64), lds, stream, rwo, order, atox,
                      reinterpret_cast<const uint8_t*>(bitmap), N, nRW, nTcb8,
                      static_cast<const _Float16*>(Q), static_cast<const _Float16*>(K),
-                     static_cast<const _Float16*>(V), scaleLog2, out, nullptr, 1, 1, D, D, sddmm, -1,
-                     nRW);
+                     static_cast<const _Float16*>(V), scaleLog2, out, nullptr, 1, 1, D, D, sddmm);
   F3S_HIP_CHECK(hipGetLastError());
   return 0;
 }

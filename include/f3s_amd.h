@@ -146,8 +146,10 @@ int f3s_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, i
  * f3sKernel1tb1rwScheduledPermutedQKV[ScaleQK] :1371-1800, f2sKernel1tb1rw :2186-2327).
  *
  *   rowWindowOffset [nRW+1], sparseAToXidx [nTCB*16], tcbBitMap [nTCB*4]   from preprocessing
- *   windowOrder [nRW] or NULL      launch order of the row windows: sortedRowWindows for the
- *                                  heavy-first schedule, NULL for natural order
+ *   windowOrder [nRW] or NULL      launch order of the row windows, a permutation of them:
+ *                                  sortedRowWindows for the heavy-first schedule, NULL for natural
+ *                                  order. On a graph of short windows whose first one in the order is
+ *                                  not a long one, windows start in natural order whatever it says
  *   N, nTCB, d                     nodes; TC blocks (rowWindowOffset[nRW]); head dimension: a
  *                                  multiple of 32 up to 256 (the reference takes embeddingDim
  *                                  at run time, src/F3S_kernel.cu:601-604,1424,1522)

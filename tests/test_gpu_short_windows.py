@@ -159,3 +159,96 @@ def test_many_long_units_per_workgroup(oracle_mod):
     capi.attention(rwo, heavy_first, atox, bm, N, q1, k1, v1, scale, out=out1)
     torch.cuda.synchronize()
     assert np.abs(out1.cpu().numpy() - want[0]).max() < MAX_ABS
+
+
+# A wave per window and a workgroup per long one, at the edges of what decides between them: windows all alike (the
+# waves then go by window number), one window just long or just not (32 blocks, or 9/4 of the mean), means on both
+# sides of 16 and 32 blocks; four and eight waves to a workgroup, all of a head dimension's forms; 1 024 windows,
+# the fewest, and a last one of a single row. Every row is compared with the oracle (fp32 sums of 16-bit
+# probabilities), orders with each other in the places of the rows.
+def _structure(rng, nRW, counts):
+    N = 16 * nRW - 15
+    rwo = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    most = int(counts.max()) * 16
+    step = N // most
+    atox = np.concatenate([np.arange(16 * c) * step for c in counts])
+    atox = (atox + rng.integers(0, step, len(atox))).astype(np.int32)
+    bitmap = rng.integers(0, 2**63, len(atox) // 4, dtype=np.uint64)
+    bitmap &= rng.integers(0, 2**63, len(bitmap), dtype=np.uint64)
+    return N, dict(rowWindowOffset=rwo, sparseAToXidx=atox, tcbBitMap=bitmap)
+
+
+@pytest.mark.parametrize("heads,d,dtype", [
+    (1, 32, torch.float16), (1, 64, torch.bfloat16), (4, 64, torch.float16), (2, 32, torch.bfloat16),
+    (8, 32, torch.float16), (1, 96, torch.float16), (3, 128, torch.bfloat16), (1, 192, torch.float16)])
+@pytest.mark.parametrize("kind", ["alike", "one_not_long", "one_long", "many_long", "mean_30"])
+def test_waves_and_teams(oracle_mod, kind, heads, d, dtype):
+    from fused3s_amd import capi
+    print("case waves and teams %s %dx%d %s" % (kind, heads, d, dtype), flush=True)
+    rng = np.random.default_rng(heads * d)
+    nRW = 1024 + (7 if heads == 1 else 0)
+    counts = rng.integers(0, 6, nRW)
+    if kind == "one_not_long":
+        counts[700] = 32
+    elif kind == "one_long":
+        counts[700] = 33
+    elif kind == "many_long":
+        counts[::9] = 34 + np.arange(len(counts[::9])) % 9
+    elif kind == "mean_30":
+        counts[:] = 28 + counts % 4
+        counts[11::50] = 69  # 9/4 of the mean and a block more
+    N, pre = _structure(rng, nRW, counts)
+    dev = lambda a: torch.as_tensor(a).cuda()
+    rwo, atox, bm = dev(pre["rowWindowOffset"]), dev(pre["sparseAToXidx"]), dev(
+        pre["tcbBitMap"].view(np.int64)).view(torch.uint64)
+    heavy = np.argsort(-counts, kind="stable").astype(np.int32)
+    g = torch.Generator().manual_seed(d)
+    Q, K, V = [(torch.randn((N, heads, d), generator=g) * d ** -0.25).to(dtype).cuda() for _ in range(3)]
+    scale = float(np.sqrt(d))
+    outs = []
+    for order in (heavy, rng.permutation(heavy)):
+        out = torch.full((N, heads * d), float("nan"), device="cuda")
+        capi.attention_heads(rwo, dev(order), atox, bm, N, Q, K, V, scale, out=out)
+        outs.append(out.cpu().numpy())
+    for h in range(heads):
+        want = oracle_mod.attention_ref(pre["rowWindowOffset"], pre["sparseAToXidx"], pre["tcbBitMap"], N,
+                                        bits(Q[:, h]), bits(K[:, h]), bits(V[:, h]), scale,
+                                        dtype=0 if dtype == torch.float16 else 1)
+        for got in outs:
+            gh = got[:, h * d:(h + 1) * d]
+            assert np.isfinite(gh).all()
+            assert np.abs(gh - want).max() < MAX_ABS
+            assert np.abs(gh - want).mean() / np.abs(want).mean() < MEAN_REL[dtype]
+
+
+@pytest.mark.parametrize("d", [64, 128, 160])
+@pytest.mark.parametrize("longest", [9, 65])
+def test_waves_and_teams_of_narrow_blocks(oracle_mod, longest, d):
+    """16x8 blocks with their scores: odd block counts, so that windows and their shared runs end inside a
+    step; `longest` 9: windows all alike, 65: one window of one block more than a wave takes."""
+    from fused3s_amd import capi
+    print("case waves and teams 16x8 longest=%d d=%d" % (longest, d), flush=True)
+    rng = np.random.default_rng(d + longest)
+    nRW = 1030
+    counts = rng.integers(0, 10, nRW)
+    counts[5::400] = longest
+    N = 16 * nRW - 3
+    rwo = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    step = N // (8 * 65)
+    atox = np.concatenate([np.arange(8 * c) * step for c in counts])
+    atox = (atox + rng.integers(0, step, len(atox))).astype(np.int32)
+    bitmap = rng.integers(0, 2**63, len(atox) // 4, dtype=np.uint64)
+    bitmap &= rng.integers(0, 2**63, len(bitmap), dtype=np.uint64)
+    g = torch.Generator().manual_seed(d)
+    Q, K, V = [(torch.randn((N, d), generator=g) * d ** -0.5).half() for _ in range(3)]
+    want, scores = oracle_mod.attention_tcb8(rwo, atox, bitmap, N, Q.numpy(), K.numpy(), V.numpy(),
+                                             save_sddmm=True)
+    order = np.argsort(-counts, kind="stable").astype(np.int32)
+    got, got_scores = capi.attention_tcb8(
+        torch.as_tensor(rwo).cuda(), torch.as_tensor(order).cuda(), torch.as_tensor(atox).cuda(),
+        torch.as_tensor(bitmap.view(np.int64)).cuda().view(torch.uint64), N, Q.cuda(), K.cuda(), V.cuda(),
+        save_sddmm=True)
+    got, got_scores = got.cpu().numpy(), got_scores.cpu().numpy()
+    assert np.isfinite(got).all()
+    assert np.abs(got - want).max() < MAX_ABS
+    assert np.abs(got_scores.reshape(-1) - np.asarray(scores).reshape(-1)).max() < 2e-2
