@@ -10,8 +10,8 @@
 //                        bins of LDS counters, ranks of the distinct columns back to the edges.
 //                        Larger graphs, <= 1024 edges: bitonic sort of the column ids, ballot /
 //                        popcount compaction of the distinct ones, rank by binary search.
-//   window_rank_sort_kernel
-//                        windows of up to 16 384 edges where the columns take several bitset
+//   window_rank_mid_kernel, window_rank_rest_kernel
+//                        longer windows of up to 16 384 edges where the columns take several bitset
 //                        passes, one workgroup per window: sorted by bins as well.
 //   window_rank_kernel   larger windows, one workgroup per window. Column ids are OR-ed into an
 //                        LDS bitset (a column range per pass when N exceeds the LDS range), a
@@ -483,11 +483,13 @@ struct EdgeRows {
 
 // EdgeRows where only the rows are asked for: bit i - 1 is set where a row that is not empty starts at edge
 // i > 0, so that the set bits below a lane are the rows that started before its edge, without the first one.
+// Where no row is empty (every node has its own diagonal entry, for one) that number is the row.
 template <int MAX>
 struct RowMarks {
   uint32_t words;  // lane l holds word l of the marks
   unsigned long long names;
   int rows;
+  bool named;  // some rows are empty
 
   // rowStart, mark: as for EdgeRows
   __device__ __forceinline__ void init(uint32_t* mark, int rowStart, int lane) {
@@ -496,10 +498,11 @@ struct RowMarks {
     wave_lds_sync();
     const int next = __shfl_down(rowStart, 1);
     const unsigned filled = (unsigned)__ballot(lane < 16 && next > rowStart);
+    named = filled != 0xFFFFu;
     if (lane < 16 && ((filled >> lane) & 1u)) {
       const int k = __popc(filled & ((1u << lane) - 1u));
       if (k > 0) atomicOr(&mark[(rowStart - 1) >> 5], 1u << ((rowStart - 1) & 31));
-      atomicOr(&mark[MAX / 32 + (k >> 3)], (uint32_t)lane << (4 * (k & 7)));
+      if (named) atomicOr(&mark[MAX / 32 + (k >> 3)], (uint32_t)lane << (4 * (k & 7)));
     }
     wave_lds_sync();
     words = mark[min(lane, MAX / 32 + 1)];
@@ -511,9 +514,10 @@ struct RowMarks {
   __device__ __forceinline__ int next_group(int u) {
     const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)words, 2 * u);
     const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)words, 2 * u + 1);
-    const int k = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, rows));
+    int k = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, rows));
     rows += __popc(lo) + __popc(hi);
-    return (int)(names >> (4 * k)) & 15;
+    if (named) k = (int)(names >> (4 * k)) & 15;
+    return k;
   }
 };
 
@@ -551,6 +555,19 @@ struct alignas(16) RankBinsLds {  // of one wave
 
 constexpr int kRankIdxBits = 10;
 static_assert(kBinsMax <= (1 << kRankIdxBits), "edge position must fit kRankIdxBits");
+
+// Adjacency matrices commonly hold the diagonal: sixteen neighbouring columns in every window, of one bin, where
+// every one of them compares itself with the others. So a window's own columns are spread over bins of their
+// own: each moves a bin further than the one before, and the columns above all sixteen with them. The columns'
+// order stays. (61M edges: 199 -> 176 us for the short windows, 77 -> 70 us for those of up to 4 096 edges.)
+// Returns the window's first column, or one past all columns where the bins (1 << bits columns in all) have no
+// room for that.
+__device__ __forceinline__ int own_columns(int w, int64_t N, int shift, int bits) {
+  return N + (17ll << shift) < (1ll << bits) ? w * 16 : 0x7FFFFFFF;
+}
+__device__ __forceinline__ uint32_t spread_column(uint32_t col, int own, int shift) {
+  return col + ((uint32_t)min(max((int)col - own + 1, 0), 17) << shift);
+}
 
 // Ranks of the distinct columns of n sorted words, collected in edge order and written as whole lines. Here and
 // in rank_window_groups 64 (G - P) < n <= 64 G: the first G - P groups of 64 edges are whole, and only the
@@ -618,39 +635,65 @@ __device__ __forceinline__ bool rank_bin_starts(uint32_t* hist, int lane) {
   return crowded;
 }
 
-// Place of word i of the words that are in their bins' order: inside its bin, later ones that are smaller move
-// it up, earlier ones that are larger move it down, and words of other bins do neither. Three neighbours on
-// each side are enough for bins of four; a group with a fuller bin goes on until no lane's next neighbour is
-// of its bin. sameBin: words of one bin differ by less in their exclusive or. WHOLE: the group and the one
-// before it are all words of the window, and the one behind it is not its end.
-template <bool WHOLE>
-__device__ __forceinline__ int rank_place(const uint32_t* buf, int u, int lane, int n, uint32_t word,
-                                          uint32_t sameBin) {
-  uint32_t up = 0, down = 0;
-  int place = 64 * u + lane;
-  const uint32_t* at = buf + place;
+// Places of the words of groups u0 .. u0 + B - 1 (those before `groups`) of the words that are in their bins'
+// order: inside its bin, later ones that are smaller move a word up, earlier ones that are larger move it
+// down, and words of other bins do neither. Three neighbours on each side are enough for bins of four; a group with
+// a fuller bin goes on until no lane's next neighbour is of its bin. The groups' first neighbours are read
+// together, as what a wave waits for here is one round of LDS reads after the other. sameBin: words of one
+// bin differ by less in their exclusive or. wholeGroups: groups from 1 up to there are all words of the window, and so
+// are the one before and the one behind.
+template <int B>
+__device__ __forceinline__ void rank_places(const uint32_t* buf, int u0, int groups, int wholeGroups, int lane,
+                                            int n, uint32_t sameBin, uint32_t (&word)[B], uint32_t (&place)[B]) {
+  uint32_t up[B][kRankNear], down[B][kRankNear];
 #pragma unroll
-  for (int k = 1; k <= kRankNear; k++) {
-    up = at[k];
-    down = at[-k];
-    place += up < word ? 1 : 0;
-    place -= down > word ? 1 : 0;
-  }
-  for (int k = kRankNear; k < kRankCrowd; k += kRankStep) {
-    bool more = (up ^ word) < sameBin || (down ^ word) < sameBin;
-    if constexpr (!WHOLE)
-      more = ((up ^ word) < sameBin && lane < n - 64 * u - k) ||
-             ((down ^ word) < sameBin && lane >= k - 64 * u && lane < n - 64 * u);
-    if (__ballot(more) == 0ull) break;
+  for (int b = 0; b < B; b++) {
+    if (u0 + b >= groups) continue;
+    const uint32_t* at = buf + 64 * (u0 + b) + lane;
+    word[b] = at[0];
 #pragma unroll
-    for (int j = 1; j <= kRankStep; j++) {
-      up = at[k + j];
-      down = at[-k - j];
-      place += up < word ? 1 : 0;
-      place -= down > word ? 1 : 0;
+    for (int k = 0; k < kRankNear; k++) {
+      up[b][k] = at[k + 1];
+      down[b][k] = at[-k - 1];
     }
   }
-  return place;
+  const auto more_in_bin = [&](int b, int k, uint32_t u, uint32_t d) {
+    const int g = u0 + b;
+    if (g > 0 && g < wholeGroups) return (u ^ word[b]) < sameBin || (d ^ word[b]) < sameBin;
+    return ((u ^ word[b]) < sameBin && lane < n - 64 * g - k) ||
+           ((d ^ word[b]) < sameBin && lane >= k - 64 * g && lane < n - 64 * g);
+  };
+  bool more = false;
+#pragma unroll
+  for (int b = 0; b < B; b++) {
+    if (u0 + b >= groups) continue;
+    int p = 64 * (u0 + b) + lane;
+#pragma unroll
+    for (int k = 0; k < kRankNear; k++) {
+      p += up[b][k] < word[b] ? 1 : 0;
+      p -= down[b][k] > word[b] ? 1 : 0;
+    }
+    place[b] = (uint32_t)p;
+    more = more || more_in_bin(b, kRankNear, up[b][kRankNear - 1], down[b][kRankNear - 1]);
+  }
+  if (__ballot(more) != 0ull) {
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      if (u0 + b >= groups) continue;
+      const uint32_t* at = buf + 64 * (u0 + b) + lane;
+      uint32_t u = up[b][kRankNear - 1], d = down[b][kRankNear - 1];
+      for (int k = kRankNear; k < kRankCrowd; k += kRankStep) {
+        if (__ballot(more_in_bin(b, k, u, d)) == 0ull) break;
+#pragma unroll
+        for (int j = 1; j <= kRankStep; j++) {
+          u = at[k + j];
+          d = at[-k - j];
+          place[b] += u < word[b] ? 1u : 0u;
+          place[b] -= d > word[b] ? 1u : 0u;
+        }
+      }
+    }
+  }
 }
 
 // False where columns crowd into few bins: the rows are written, the unsorted words are in lds.words and the
@@ -694,6 +737,9 @@ __device__ __forceinline__ bool rank_window_groups(
 #pragma unroll
     for (int u = 0; u < G; u++) col[u] = col[u] < (uint32_t)N ? col[u] : 0u;
   }
+  const int own = own_columns(w, N, shift, colBits);
+#pragma unroll
+  for (int u = 0; u < G; u++) col[u] = spread_column(col[u], own, shift);
   const uint32_t upper = 512u << shift;  // first column of the bins in high halves
 #pragma unroll
   for (int u = 0; u < G; u++)
@@ -708,23 +754,28 @@ __device__ __forceinline__ bool rank_window_groups(
     return false;
   }
   // ---- into the bins
-#pragma unroll
-  for (int u = 0; u < G; u++) {
-    const uint32_t half = col[u] < upper ? 0u : 16u;
-    if (valid(u)) {
-      const uint32_t old = atomicAdd(&hist[(col[u] >> shift) & 511u], 1u << half);
-      buf[(old >> half) & 0xFFFFu] = (col[u] << kRankIdxBits) | (uint32_t)(64 * u + lane);
-    }
-  }
-  wave_lds_sync();
-  // ---- from the bins' order to the columns'
-  const uint32_t sameBin = 1u << (kRankIdxBits + shift);
   uint32_t at[G];
 #pragma unroll
   for (int u = 0; u < G; u++) {
-    col[u] = buf[64 * u + lane];
-    at[u] = (uint32_t)(u > 0 && u < G - P - 1 ? rank_place<true>(buf, u, lane, n, col[u], sameBin)
-                                              : rank_place<false>(buf, u, lane, n, col[u], sameBin));
+    const uint32_t half = col[u] < upper ? 0u : 16u;
+    if (valid(u)) at[u] = (atomicAdd(&hist[(col[u] >> shift) & 511u], 1u << half) >> half) & 0xFFFFu;
+  }
+#pragma unroll
+  for (int u = 0; u < G; u++)
+    if (valid(u)) buf[at[u]] = (col[u] << kRankIdxBits) | (uint32_t)(64 * u + lane);
+  wave_lds_sync();
+  // ---- from the bins' order to the columns'
+  constexpr int B = 2;
+#pragma unroll
+  for (int u = 0; u < G; u += B) {
+    uint32_t word[B], place[B];
+    rank_places<B>(buf, u, G, G - P - 1, lane, n, 1u << (kRankIdxBits + shift), word, place);
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      if (u + b >= G) continue;
+      col[u + b] = word[b];
+      at[u + b] = place[b];
+    }
   }
   wave_lds_sync();
 #pragma unroll
@@ -791,10 +842,11 @@ __device__ __forceinline__ void rank_crowded_window(int w, int n, int colBits, R
 #pragma unroll
     for (int u = 0; u < G; u++) {
       if (64 * u >= n) continue;
-      word[u] = buf[64 * u + lane];
-      const bool middleBin = (word[u] >> kRankIdxBits) - from < span;
-      const uint32_t sameBin = 1u << (kRankIdxBits + (middleBin ? fine : shift + 2));
-      at[u] = (uint32_t)rank_place<false>(buf, u, lane, n, word[u], sameBin);
+      const bool middleBin = (buf[64 * u + lane] >> kRankIdxBits) - from < span;
+      uint32_t one[1], place[1];
+      rank_places<1>(buf, u, G, 0, lane, n, 1u << (kRankIdxBits + (middleBin ? fine : shift + 2)), one, place);
+      word[u] = one[0];
+      at[u] = place[0];
     }
     wave_lds_sync();
 #pragma unroll
@@ -1019,20 +1071,19 @@ __global__ __launch_bounds__(TB) void window_rank_all_kernel(
 // a 48 KiB bitset that such a window fills with a few thousand bits. The columns go into eight bins per
 // thread, as in rank_window_groups; a thread keeps its columns and where it put them, finds their places
 // among the sorted ones from their neighbours and marks the first of every column in a bitset of places, in
-// which a rank is a count. Bound by latency, so by the waves that LDS and registers leave: 24 per CU, where
-// the sorted columns in a second buffer, searched again by every edge, allowed 16 (4 272 such windows of a
-// 61M-edge graph: preprocessing 635 -> 615 us). Windows whose columns crowd into few bins
-// take an LSD radix sort, eight bits per pass, and a binary search per edge.
-// The windows come from the lists that the kernel for short windows has made: where every workgroup looked
-// for its own, some met five and some none (4 272 windows dealt to 8 192 workgroups: 133 instead of
-// 96 us; window_fill_long_kernel 68 instead of 45 us).
-// Two sizes: windows of up to kMedMax edges (512 threads, 26 KiB of LDS; 256 threads of 16 edges
-// do not fit 80 registers), and the handful of windows of up to kLargeMax edges (1024
-// threads, 85 KiB), which would otherwise each walk the bitset passes alone at the end of the phase.
-constexpr int kMedThreads = 512;
-constexpr int kMedItems = 8;
-constexpr int kMedMax = kMedThreads * kMedItems;
+// which a rank is a count. Bound by the issue of vector instructions, and by latency where windows are few.
+// Windows whose columns crowd into few bins take an LSD radix sort, eight bits per pass, and a binary search
+// per edge. 256 threads for up to kMidMax edges, 24 waves per CU: most such windows have less than half of the 4 096
+// edges that 512 threads hold, and each wave pays for the clearing, the scans and the guards of eight items
+// (5 000 of 960 to 2 048 edges in a 61M-edge graph: 70 -> 54 us. A wave each, its state in LDS or in registers
+// over thirty unrolled groups, took 63 to 97: too few waves, or code that the instruction cache does not hold.)
+// 1024 threads for up to kFourMax and kLargeMax edges.
+constexpr int kMidThreads = 256;
+constexpr int kMidItems = 8;
+constexpr int kMidMax = kMidThreads * kMidItems;
 constexpr int kLargeThreads = 1024;
+constexpr int kFourItems = 4;
+constexpr int kFourMax = kLargeThreads * kFourItems;
 constexpr int kLargeItems = 16;
 constexpr int kLargeMax = kLargeThreads * kLargeItems;
 constexpr int kSortCrowd = 32;  // a fuller bin sends the window to the radix sort
@@ -1141,19 +1192,17 @@ __device__ __forceinline__ void rank_crowded_keys(const uint32_t (&key)[ITEMS], 
   __syncthreads();
 }
 
-// takes the mid windows of the queue, or (LARGE) the large ones of at most THREADS * ITEMS edges
-template <int W, int ITEMS, int THREADS, bool LARGE>
-__global__ __launch_bounds__(THREADS, LARGE ? 1 : 6) void window_rank_sort_kernel(
-    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
-    int colBits, LongQueue queue, int32_t* __restrict__ blockPartition,
-    int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
-    int* __restrict__ error) {
+// One window of at most THREADS * ITEMS edges by the whole workgroup; every thread calls this.
+template <int W, int ITEMS, int THREADS>
+__device__ __forceinline__ void rank_window_by_sort(
+    int w, const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int colBits,
+    uint32_t* sSort, int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
+    int32_t* __restrict__ edgeToRow, int* __restrict__ error) {
   constexpr int WAVES = THREADS / 64;
   constexpr int CAP = THREADS * ITEMS;
   constexpr int BIN_BITS = THREADS == 256 ? 11 : THREADS == 512 ? 12 : 13;
   static_assert((1 << BIN_BITS) == 8 * THREADS, "eight bins per thread");
   static_assert(THREADS >= 256 && THREADS % 256 == 0, "the first 256 threads own one digit each");
-  extern __shared__ __align__(16) uint32_t sSort[];
   uint32_t* sKeys = sSort + kSortPad;  // CAP keys, room for kSortPad on each side
   uint32_t* sBins = sKeys + CAP + kSortPad;  // 16-bit counters, or the radix sort's digit counters
   uint32_t* sFirst = sBins + 4 * THREADS;  // bit per key: the first one of its column
@@ -1169,169 +1218,210 @@ __global__ __launch_bounds__(THREADS, LARGE ? 1 : 6) void window_rank_sort_kerne
   const int keyBits = colBits + (((int64_t)1 << colBits) <= (int64_t)N ? 1 : 0);
   const int shiftBins = keyBits > BIN_BITS ? keyBits - BIN_BITS : 0;
   const uint32_t sameBin = 1u << shiftBins;
-  const int listed = queue.size(LARGE);
-  for (int taken = blockIdx.x; taken < listed; taken += (int)gridDim.x) {
-    const int w = queue.at(LARGE, taken);
-    const int r0 = w * 16;
-    if (LARGE && rowPtr[min(r0 + 16, N)] - rowPtr[r0] > CAP) continue;  // window_rank_kernel's
-    __syncthreads();  // the window before this one has left the LDS arrays
-    if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
-    if (tid == 0) sCrowded = 0;
-    reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(0, 0, 0, 0);
-    for (int i = tid; i < CAP / 32; i += THREADS) sFirst[i] = 0u;
-    if (tid < kSortPad) sSort[tid] = 0u;
+  const int r0 = w * 16;
+  __syncthreads();  // the window before this one has left the LDS arrays
+  if (tid < 17) sRow[tid] = rowPtr[min(r0 + tid, N)];
+  if (tid == 0) sCrowded = 0;
+  reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(0, 0, 0, 0);
+  for (int i = tid; i < CAP / 32; i += THREADS) sFirst[i] = 0u;
+  if (tid < kSortPad) sSort[tid] = 0u;
+  __syncthreads();
+  const int eS = uniform(sRow[0]);
+  int n = uniform(sRow[16]) - eS;
+  const int32_t* cols = colIdx + eS;
+  int32_t *ranks = edgeToColumn + eS, *rows = edgeToRow + eS;
+  // thread t's keys: of edges t + THREADS u
+  uint32_t key[ITEMS], at[ITEMS];
+#pragma unroll
+  for (int u = 0; u < ITEMS; u++) {
+    if (u * THREADS >= n) continue;
+    key[u] = (uint32_t)cols[min(u * THREADS + tid, n - 1)];
+  }
+  if (tid < kSortPad) sKeys[n + tid] = 0xFFFFFFFFu;
+  asm volatile("" : "+s"(n));
+  const int own = own_columns(w, (int64_t)N + 1, shiftBins, keyBits);
+  bool bad = false;
+#pragma unroll
+  for (int u = 0; u < ITEMS; u++) {
+    if (u * THREADS >= n) continue;
+    if (key[u] >= (uint32_t)N) {
+      bad = true;
+      key[u] = 0u;
+    }
+    key[u] = spread_column(key[u], own, shiftBins) + 1u;
+    const uint32_t bin = key[u] >> shiftBins;
+    if (tid < n - u * THREADS) {
+      rows[u * THREADS + tid] = r0 + row_of_edge(sRow, eS + u * THREADS + tid);
+      atomicAdd(&sBins[bin >> 1], 1u << ((bin & 1u) * 16u));
+    }
+  }
+  if (bad) *error = 1;
+  __syncthreads();
+  {
+    const uint4 x = reinterpret_cast<const uint4*>(sBins)[tid];
+    uint32_t v[4] = {x.x, x.y, x.z, x.w};
+    uint32_t total = 0, most = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      total += (v[k] & 0xFFFFu) + (v[k] >> 16);
+      most = max(most, max(v[k] & 0xFFFFu, v[k] >> 16));
+    }
+    if (most > (uint32_t)kSortCrowd) sCrowded = 1;
+    const unsigned incl = wave_inclusive_scan(total, lane);
+    if (lane == 63) sWaveTot[wave] = incl;
     __syncthreads();
-    const int eS = uniform(sRow[0]);
-    int n = uniform(sRow[16]) - eS;
-    const int32_t* cols = colIdx + eS;
-    int32_t *ranks = edgeToColumn + eS, *rows = edgeToRow + eS;
-    // thread t's keys: of edges t + THREADS u
-    uint32_t key[ITEMS], at[ITEMS];
+    unsigned run = incl - total;
+#pragma unroll
+    for (int u = 0; u < WAVES; u++)
+      if (u < wave) run += sWaveTot[u];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t mid = run + (v[k] & 0xFFFFu);
+      const uint32_t start = run | (mid << 16);
+      run = mid + (v[k] >> 16);
+      v[k] = start;
+    }
+    reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(v[0], v[1], v[2], v[3]);
+  }
+  __syncthreads();
+  if (sCrowded) {
+    rank_crowded_keys<ITEMS, THREADS>(key, sKeys, sBins, sWaveTot, n, keyBits, &sUniq);
+    const int nUniq = sUniq;
 #pragma unroll
     for (int u = 0; u < ITEMS; u++) {
       if (u * THREADS >= n) continue;
-      key[u] = (uint32_t)cols[min(u * THREADS + tid, n - 1)];
+      int lo = 0, hi = nUniq - 1;  // the key is one of the window's distinct ones
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (sKeys[mid] < key[u])
+          lo = mid + 1;
+        else
+          hi = mid;
+      }
+      if (tid < n - u * THREADS) ranks[u * THREADS + tid] = lo;
     }
-    if (tid < kSortPad) sKeys[n + tid] = 0xFFFFFFFFu;
-    asm volatile("" : "+s"(n));
-    bool bad = false;
+    if (tid == 0) blockPartition[w] = (nUniq + W - 1) / W;
+    return;
+  }
+  // into the bins (n is hidden from the compiler between the passes: sixteen comparisons with it, kept for
+  // all of them, cost more vector registers than the keys. Within a pass the lane masks of the guarded items
+  // still outnumber the scalar registers: 132 of them in the form of 512 threads and 261 in that of 1 024
+  // go to lanes of vector registers and back. None goes to memory.)
+  asm volatile("" : "+s"(n));
 #pragma unroll
-    for (int u = 0; u < ITEMS; u++) {
-      if (u * THREADS >= n) continue;
-      if (key[u] >= (uint32_t)N) {
-        bad = true;
-        key[u] = 0u;
-      }
-      key[u] += 1u;
-      const uint32_t bin = key[u] >> shiftBins;
-      if (tid < n - u * THREADS) {
-        rows[u * THREADS + tid] = r0 + row_of_edge(sRow, eS + u * THREADS + tid);
-        atomicAdd(&sBins[bin >> 1], 1u << ((bin & 1u) * 16u));
-      }
+  for (int u = 0; u < ITEMS; u++) {
+    if (u * THREADS >= n) continue;
+    const uint32_t bin = key[u] >> shiftBins, half = (bin & 1u) * 16u;
+    at[u] = 0;
+    if (tid < n - u * THREADS) {
+      at[u] = (atomicAdd(&sBins[bin >> 1], 1u << half) >> half) & 0xFFFFu;
+      sKeys[at[u]] = key[u];
     }
-    if (bad) *error = 1;
-    __syncthreads();
-    {
-      const uint4 x = reinterpret_cast<const uint4*>(sBins)[tid];
-      uint32_t v[4] = {x.x, x.y, x.z, x.w};
-      uint32_t total = 0, most = 0;
+  }
+  __syncthreads();
+  asm volatile("" : "+s"(n));
+  // Each key's place among the sorted ones: from its place in the bins' order, later keys that are smaller
+  // move it up, earlier ones that are larger move it down, and keys of other bins do neither. An earlier
+  // equal one says that this is not the first of its column.
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        total += (v[k] & 0xFFFFu) + (v[k] >> 16);
-        most = max(most, max(v[k] & 0xFFFFu, v[k] >> 16));
-      }
-      if (most > (uint32_t)kSortCrowd) sCrowded = 1;
-      const unsigned incl = wave_inclusive_scan(total, lane);
-      if (lane == 63) sWaveTot[wave] = incl;
-      __syncthreads();
-      unsigned run = incl - total;
+  for (int u = 0; u < ITEMS; u++) {
+    if (u * THREADS >= n) continue;
+    const bool valid = tid < n - u * THREADS;
+    const uint32_t* here = sKeys + at[u];
+    uint32_t up = 0, down = 0;
+    int place = (int)at[u];
+    bool again = false;
 #pragma unroll
-      for (int u = 0; u < WAVES; u++)
-        if (u < wave) run += sWaveTot[u];
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const uint32_t mid = run + (v[k] & 0xFFFFu);
-        const uint32_t start = run | (mid << 16);
-        run = mid + (v[k] >> 16);
-        v[k] = start;
-      }
-      reinterpret_cast<uint4*>(sBins)[tid] = make_uint4(v[0], v[1], v[2], v[3]);
+    for (int k = 1; k <= kRankNear; k++) {
+      up = here[k];
+      down = here[-k];
+      place += up < key[u] ? 1 : 0;
+      place -= down > key[u] ? 1 : 0;
+      again = again || down == key[u];
     }
-    __syncthreads();
-    if (sCrowded) {
-      rank_crowded_keys<ITEMS, THREADS>(key, sKeys, sBins, sWaveTot, n, keyBits, &sUniq);
-      const int nUniq = sUniq;
+    for (int k = kRankNear; k < kSortCrowd; k += kRankStep) {
+      const bool more = valid && ((up ^ key[u]) < sameBin || ((down ^ key[u]) < sameBin && down != 0u));
+      if (__ballot(more) == 0ull) break;
 #pragma unroll
-      for (int u = 0; u < ITEMS; u++) {
-        if (u * THREADS >= n) continue;
-        int lo = 0, hi = nUniq - 1;  // the key is one of the window's distinct ones
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (sKeys[mid] < key[u])
-            lo = mid + 1;
-          else
-            hi = mid;
-        }
-        if (tid < n - u * THREADS) ranks[u * THREADS + tid] = lo;
-      }
-      if (tid == 0) blockPartition[w] = (nUniq + W - 1) / W;
-      continue;
-    }
-    // into the bins (n is hidden from the compiler between the passes: sixteen comparisons with it, kept for
-    // all of them, cost more vector registers than the keys. Within a pass the lane masks of the guarded items
-    // still outnumber the scalar registers: 132 of them in the form of 512 threads and 261 in that of 1 024
-    // go to lanes of vector registers and back. None goes to memory.)
-    asm volatile("" : "+s"(n));
-#pragma unroll
-    for (int u = 0; u < ITEMS; u++) {
-      if (u * THREADS >= n) continue;
-      const uint32_t bin = key[u] >> shiftBins, half = (bin & 1u) * 16u;
-      at[u] = 0;
-      if (tid < n - u * THREADS) {
-        at[u] = (atomicAdd(&sBins[bin >> 1], 1u << half) >> half) & 0xFFFFu;
-        sKeys[at[u]] = key[u];
-      }
-    }
-    __syncthreads();
-    asm volatile("" : "+s"(n));
-    // Each key's place among the sorted ones: from its place in the bins' order, later keys that are smaller
-    // move it up, earlier ones that are larger move it down, and keys of other bins do neither. An earlier
-    // equal one says that this is not the first of its column.
-#pragma unroll
-    for (int u = 0; u < ITEMS; u++) {
-      if (u * THREADS >= n) continue;
-      const bool valid = tid < n - u * THREADS;
-      const uint32_t* here = sKeys + at[u];
-      uint32_t up = 0, down = 0;
-      int place = (int)at[u];
-      bool again = false;
-#pragma unroll
-      for (int k = 1; k <= kRankNear; k++) {
-        up = here[k];
-        down = here[-k];
+      for (int j = 1; j <= kRankStep; j++) {
+        up = here[k + j];
+        down = here[-k - j];
         place += up < key[u] ? 1 : 0;
         place -= down > key[u] ? 1 : 0;
         again = again || down == key[u];
       }
-      for (int k = kRankNear; k < kSortCrowd; k += kRankStep) {
-        const bool more = valid && ((up ^ key[u]) < sameBin || ((down ^ key[u]) < sameBin && down != 0u));
-        if (__ballot(more) == 0ull) break;
-#pragma unroll
-        for (int j = 1; j <= kRankStep; j++) {
-          up = here[k + j];
-          down = here[-k - j];
-          place += up < key[u] ? 1 : 0;
-          place -= down > key[u] ? 1 : 0;
-          again = again || down == key[u];
-        }
-      }
-      at[u] = (uint32_t)place;
-      if (valid && !again) atomicOr(&sFirst[place >> 5], 1u << (place & 31));
     }
+    at[u] = (uint32_t)place;
+    if (valid && !again) atomicOr(&sFirst[place >> 5], 1u << (place & 31));
+  }
+  __syncthreads();
+  {
+    static_assert(CAP / 32 <= THREADS, "a word of bits per thread");
+    const uint32_t count = tid < CAP / 32 ? __popc(sFirst[tid]) : 0u;
+    const uint32_t incl = wave_inclusive_scan(count, lane);
+    if (lane == 63) sWaveTot[wave] = incl;
     __syncthreads();
-    {
-      static_assert(CAP / 32 <= THREADS, "a word of bits per thread");
-      const uint32_t count = tid < CAP / 32 ? __popc(sFirst[tid]) : 0u;
-      const uint32_t incl = wave_inclusive_scan(count, lane);
-      if (lane == 63) sWaveTot[wave] = incl;
-      __syncthreads();
-      uint32_t run = incl - count;
+    uint32_t run = incl - count;
 #pragma unroll
-      for (int u = 0; u < CAP / 32 / 64; u++)
-        if (u < wave) run += sWaveTot[u];
-      if (tid < CAP / 32) sBefore[tid] = run;
-      if (tid == CAP / 32 - 1) blockPartition[w] = ((int)(run + count) + W - 1) / W;
-    }
+    for (int u = 0; u < CAP / 32 / 64; u++)
+      if (u < wave) run += sWaveTot[u];
+    if (tid < CAP / 32) sBefore[tid] = run;
+    if (tid == CAP / 32 - 1) blockPartition[w] = ((int)(run + count) + W - 1) / W;
+  }
+  __syncthreads();
+  asm volatile("" : "+s"(n));
+  // an edge's rank: the first keys at or in front of its place, without the column's own
+#pragma unroll
+  for (int u = 0; u < ITEMS; u++) {
+    if (u * THREADS >= n) continue;
+    if (tid >= n - u * THREADS) continue;
+    const uint32_t bits = sFirst[at[u] >> 5] & ((2u << (at[u] & 31u)) - 1u);
+    ranks[u * THREADS + tid] = (int)(sBefore[at[u] >> 5] + __popc(bits)) - 1;
+  }
+}
+
+// The mid windows of the queue.
+template <int W>
+__global__ __launch_bounds__(kMidThreads, 6) void window_rank_mid_kernel(
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int colBits,
+    LongQueue queue, int32_t* __restrict__ blockPartition, int32_t* __restrict__ edgeToColumn,
+    int32_t* __restrict__ edgeToRow, int* __restrict__ error) {
+  extern __shared__ __align__(16) uint32_t smem[];
+  const int listed = queue.size(false);
+  for (int k = blockIdx.x; k < listed; k += (int)gridDim.x)
+    rank_window_by_sort<W, kMidItems, kMidThreads>(queue.at(false, k), rowPtr, colIdx, N, colBits, smem,
+                                                   blockPartition, edgeToColumn, edgeToRow, error);
+}
+
+// The large windows of the queue, those of more than kLargeMax edges by the bitset in several passes. One launch:
+// the handful of windows of thousands of edges would each keep a launch of its own waiting (61M edges, 414
+// windows of 1 921 to 11 001 edges: 18 + 25 + 5 us as three launches, 29 as one).
+template <int W>
+constexpr size_t rank_rest_lds(size_t bitset) {
+  constexpr size_t sort = rank_sort_lds<kLargeItems, kLargeThreads>();
+  return bitset > sort ? bitset : sort;
+}
+template <int W>
+__global__ __launch_bounds__(kLargeThreads) void window_rank_rest_kernel(
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
+    int colBits, int range, int nPasses, LongQueue queue, int32_t* __restrict__ blockPartition,
+    int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
+    int* __restrict__ error) {
+  extern __shared__ __align__(16) uint32_t smem[];
+  const int listed = queue.size(true);
+  for (int k = blockIdx.x; k < listed; k += (int)gridDim.x) {
+    const int w = uniform(queue.at(true, k));
+    const int n = rowPtr[min(w * 16 + 16, N)] - rowPtr[w * 16];
     __syncthreads();
-    asm volatile("" : "+s"(n));
-    // an edge's rank: the first keys at or in front of its place, without the column's own
-#pragma unroll
-    for (int u = 0; u < ITEMS; u++) {
-      if (u * THREADS >= n) continue;
-      if (tid >= n - u * THREADS) continue;
-      const uint32_t bits = sFirst[at[u] >> 5] & ((2u << (at[u] & 31u)) - 1u);
-      ranks[u * THREADS + tid] = (int)(sBefore[at[u] >> 5] + __popc(bits)) - 1;
-    }
+    if (n > kLargeMax)
+      rank_window_by_bitset<W, kLargeThreads>(w, rowPtr, colIdx, N, range, nPasses, 0, smem, blockPartition,
+                                              edgeToColumn, edgeToRow, error);
+    else if (n > kFourMax)
+      rank_window_by_sort<W, kLargeItems, kLargeThreads>(w, rowPtr, colIdx, N, colBits, smem, blockPartition,
+                                                         edgeToColumn, edgeToRow, error);
+    else
+      rank_window_by_sort<W, kFourItems, kLargeThreads>(w, rowPtr, colIdx, N, colBits, smem, blockPartition,
+                                                       edgeToColumn, edgeToRow, error);
   }
 }
 
@@ -2140,13 +2230,13 @@ __device__ __forceinline__ void fill_short_window(
   if (nb < 1) return;  // no block to write: every column of the window lay outside [0, N)
   unsigned long long* bm = lds.bm;
   uint32_t* ids = lds.ids;
-  EdgeRows<kBinsMax> edgeRows;
-  edgeRows.init(lds.mark, rowStart, lane);
+  RowMarks<kBinsMax> marks;
+  marks.init(lds.mark, rowStart, lane);
   for (int i = lane; i < nb * WPT / 2; i += 64)
     reinterpret_cast<uint4*>(bm)[i] = make_uint4(0, 0, 0, 0);
   for (int i = nb * W - W + lane; i < nb * W; i += 64) ids[i] = 0u;  // unused slots hold 0
   wave_lds_sync();
-  bool rough = false;  // some row's columns do not strictly ascend
+  bool rough = false;  // some row's columns do not strictly ascend: nor do its (row, rank) pairs
   int before = -1;
   for (int e0 = 0; e0 < n; e0 += 64 * U) {
     int rank[U], col[U];
@@ -2157,19 +2247,22 @@ __device__ __forceinline__ void fill_short_window(
       col[u] = colIdx[eS + i];
     }
 #pragma unroll
+    for (int u = 0; u < U; u++)  // all of them in flight before the first one is used
+      asm volatile("" : "+v"(rank[u]), "+v"(col[u]));
+#pragma unroll
     for (int u = 0; u < U; u++) {
       if (e0 + 64 * u >= n) break;
-      bool starts;
-      const int row = edgeRows.next_group(e0 + 64 * u, lane, &starts);
-      const int left = __builtin_amdgcn_update_dpp(before, col[u], 0x138, 0xf, 0xf, false);
-      before = __builtin_amdgcn_readlane(col[u], 63);
+      const int row = marks.next_group((e0 >> 6) + u);
+      const int pair = (row << 16) | rank[u];
+      const int left = __builtin_amdgcn_update_dpp(before, pair, 0x138, 0xf, 0xf, false);
+      before = __builtin_amdgcn_readlane(pair, 63);
       if (e0 + 64 * u + lane < n && (unsigned)rank[u] < (unsigned)(nb * W)) {
-        rough = rough || (!starts && left >= col[u]);
+        rough = rough || left >= pair;
         ids[rank[u]] = (uint32_t)col[u];
-        // word and bit of (rank, row): see window_rank_fill_kernel
-        const int byte = 7 - (row & 7);
-        atomicOr(&reinterpret_cast<unsigned*>(bm)[(rank[u] >> 3) * 4 + (row >> 3) * 2 + (byte >> 2)],
-                 (0x80u << (8 * (byte & 3))) >> (rank[u] & 7));
+        // Byte 7 - row % 8 of word 2 (rank >> 3) + (row >> 3) is the row, MSB first (see window_rank_fill_kernel):
+        // in dwords, the halves of a word change places.
+        atomicOr(&reinterpret_cast<unsigned*>(bm)[((rank[u] & ~7) >> 1) + ((row >> 2) ^ 1)],
+                 0x80000000u >> ((((unsigned)row << 3) | ((unsigned)rank[u] & 7u)) & 31u));
       }
     }
   }
@@ -2221,9 +2314,10 @@ __device__ __forceinline__ void fill_short_window(
   // into places and the rows replayed in order (src/utils.cu:173-224).
   uint32_t* cnt = ids;
   wave_lds_sync();
+  EdgeRows<kBinsMax> edgeRows;
+  edgeRows.init(lds.mark, rowStart, lane);
   for (int i = lane; i < nb * 8; i += 64) cnt[i] = 0u;
   wave_lds_sync();
-  edgeRows.rows = 0;
   for (int e0 = 0; e0 < n; e0 += 64) {
     bool starts;
     const int row = edgeRows.next_group(e0, lane, &starts);
@@ -2290,7 +2384,8 @@ __global__ __launch_bounds__(64) void window_fill_short_kernel(
     int32_t* __restrict__ tcblockOffset, int32_t* __restrict__ sparseAToXidx,
     unsigned long long* __restrict__ bitmap) {
   __shared__ FillShortLds<W> lds;
-  const int w = blockIdx.x;
+  // the last windows first: what the ranking wrote last is still in the memory-side cache (61M edges: 204 -> 198 us)
+  const int w = nRW - 1 - (int)blockIdx.x;
   const int base = __builtin_amdgcn_readfirstlane(rowWindowOffset[w]);
   const int nb = __builtin_amdgcn_readfirstlane(rowWindowOffset[w + 1]) - base;
   if (w == nRW - 1 && threadIdx.x == 0) tcblockOffset[base + nb] = E;
@@ -3170,7 +3265,7 @@ int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, cha
   WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
   LongQueue queue = {nullptr, nullptr, 0, 0};
   if (!long_windows(nRW, E)) {
-    queue = {&hdr->rank, sortedRowWindows, nRW, nPasses >= 2 ? kMedMax : 0};
+    queue = {&hdr->rank, sortedRowWindows, nRW, nPasses >= 2 ? kMidMax : 0};
     hipLaunchKernelGGL(clear_header_kernel, dim3(1), dim3(1), 0, stream, hdr);
   }
   if (colBits <= 22) {
@@ -3192,27 +3287,24 @@ int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, cha
   // The longer ones, from the lists. On a graph that needs several bitset passes,
   // windows of a few thousand edges are sorted instead of walking every pass: up to kMedMax edges
   // with four workgroups per CU, then the few windows up to kLargeMax with one.
-  int minEdges = shortMax;
   if (nPasses >= 2) {
-    auto med = window_rank_sort_kernel<W, kMedItems, kMedThreads, false>;
-    auto large = window_rank_sort_kernel<W, kLargeItems, kLargeThreads, true>;
-    constexpr size_t medLds = rank_sort_lds<kMedItems, kMedThreads>();
-    constexpr size_t largeLds = rank_sort_lds<kLargeItems, kLargeThreads>();
-    if (int rc = allow_lds(med, medLds)) return rc;
-    if (int rc = allow_lds(large, largeLds)) return rc;
-    hipLaunchKernelGGL(med, dim3(long_grid(nRW, E, minEdges, 8192)), dim3(kMedThreads), medLds,
-                       stream, rowPtr, colIdx, N, nRW, colBits, queue, blockPartition, edgeToColumn,
+    auto rest = window_rank_rest_kernel<W>;
+    const size_t restLds = rank_rest_lds<W>(lds);
+    if (int rc = allow_lds(rest, restLds)) return rc;
+    constexpr size_t midLds = rank_sort_lds<kMidItems, kMidThreads>();
+    hipLaunchKernelGGL(window_rank_mid_kernel<W>, dim3(long_grid(nRW, E, shortMax, 8192)), dim3(kMidThreads),
+                       midLds, stream, rowPtr, colIdx, N, colBits, queue, blockPartition, edgeToColumn,
                        edgeToRow, error);
-    hipLaunchKernelGGL(large, dim3(long_grid(nRW, E, kMedMax, 1024)), dim3(kLargeThreads),
-                       largeLds, stream, rowPtr, colIdx, N, nRW, colBits, queue, blockPartition,
-                       edgeToColumn, edgeToRow, error);
+    hipLaunchKernelGGL(rest, dim3(long_grid(nRW, E, kMidMax, 1024)), dim3(kLargeThreads), restLds, stream,
+                       rowPtr, colIdx, N, nRW, colBits, range, nPasses, queue, blockPartition, edgeToColumn,
+                       edgeToRow, error);
     F3S_HIP_CHECK(hipGetLastError());
-    minEdges = kLargeMax;
+    return 0;
   }
   // sixteen waves per window: what counts is how soon the longest one is done (169k-node R-MAT graph,
   // windows of up to 12 500 edges: 31 us with four)
-  hipLaunchKernelGGL((window_rank_kernel<W, 1024, true>), dim3(long_grid(nRW, E, minEdges, 512)),
-                     dim3(1024), lds, stream, rowPtr, colIdx, N, nRW, range, nPasses, minEdges, queue,
+  hipLaunchKernelGGL((window_rank_kernel<W, 1024, true>), dim3(long_grid(nRW, E, shortMax, 512)),
+                     dim3(1024), lds, stream, rowPtr, colIdx, N, nRW, range, nPasses, shortMax, queue,
                      blockPartition, edgeToColumn, edgeToRow, error);
   F3S_HIP_CHECK(hipGetLastError());
   return 0;

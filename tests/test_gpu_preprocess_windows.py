@@ -204,6 +204,39 @@ def test_windows_of_a_workgroup(oracle_mod, N):
         assert np.array_equal(got[k].cpu().numpy(), want[k]), k
 
 
+# A window's own sixteen columns (the diagonal of an adjacency matrix) get bins of their own where the bins have
+# room for that: the most columns for which they do, one more, and powers of two on either side; windows of a wave
+# (ten bits of bins), of 256 threads and of 1024 (eleven and thirteen) with all, some and none of their own columns,
+# own columns in every row, and neighbours on both sides of them; the last window, whose columns are the last ones
+@pytest.mark.parametrize("W", [16, 8])
+@pytest.mark.parametrize("N", [1024, 1025, (1 << 15) - 17 * 32 - 1, (1 << 15) - 17 * 32, 1 << 15,
+                               (1 << 19) - 17 * 256 - 2, (1 << 19) - 17 * 256 - 1, (1 << 19) - 17 * 512])
+def test_own_columns(oracle_mod, N, W):
+    from fused3s_amd import capi
+    print("case own columns N=%d W=%d" % (N, W), flush=True)
+    rng = np.random.default_rng(N + W)
+    nRW = (N + 15) // 16
+    rows = [np.zeros(0, np.int32)] * N
+    sizes = [40, 400, 900] + ([1500, 2047, 2049, 3000, 5000] if N > 393_216 else [])
+    picked = np.concatenate([[0, nRW - 1], rng.choice(np.arange(1, nRW - 1), 3 * len(sizes) - 2, replace=False)])
+    for k, w in enumerate(picked):
+        own = np.arange(16 * w, min(16 * w + 16, N))
+        for r in own:
+            cols = rng.choice(N, size=min(sizes[k % len(sizes)] // 16, N // 2), replace=False)
+            near = np.clip(16 * w + rng.integers(-40, 56, 6), 0, N - 1)
+            extra = {0: [r], 1: own, 2: near}[k % 3]
+            rows[r] = np.unique(np.concatenate([cols, extra])).astype(np.int32)
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum([len(r) for r in rows])
+    colIdx = np.concatenate(rows).astype(np.int32)
+    want = oracle_mod.preprocess(rowPtr, colIdx, N, 16, W)
+    rp, ci = torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda()
+    got = capi.preprocess(rp, ci, N, W=W)
+    for key in KEYS:
+        assert np.array_equal(got[key].cpu().numpy(), want[key]), key
+    assert np.array_equal(got["tcbBitMap"].cpu().view(torch.int64).numpy().view(np.uint64), want["tcbBitMap"])
+
+
 def split_columns(rng, cols, lengths):
     """16 ascending rows of the given lengths over `cols`, which together name every one of them."""
     cols = np.sort(cols)
