@@ -155,24 +155,33 @@ __device__ __forceinline__ void vm_wait() {
 
 // ---- geometry of the per-wave LDS ring
 // D: head dimension, any multiple of 32 up to 256 (the reference takes embeddingDim at run time,
-// src/F3S_kernel.cu:601-604,1424,1522). The ring is laid out for DP, the next power of two: a row
-// of the LDS tile is DP elements wide, of which the first D hold data; lanes whose chunk does not
-// exist fetch nothing.
+// src/F3S_kernel.cu:601-604,1424,1522). A tile is the 32 rows of a pair, D elements each, one behind the
+// other: a gather instruction's 64 lanes fetch 64 chunks of 16 bytes that follow each other in it. At
+// the powers of two those are whole rows. At 96, 160, 192 and 224 a row may begin in one instruction and
+// end in the next; the ring holds no unused bytes and every lane of every gather works: 6, 10, 12, 14
+// instructions a tile. Rows at the pitch of the next power of two, the lanes beyond the row idle, need 8, 16, 16,
+// 16 and rings a third larger. What bounds such calls is the vector memory path, in instructions as well as
+// lines; us a call, that pitch -> rows one behind the other (blocks a window in brackets):
+//   sliced, 50 000 nodes (109)             d =  96 165 -> 154, 160 328 -> 255, 192 347 -> 280, 224 390 -> 363
+//   sliced, 233 000 nodes, bf16 (188)      1352 -> 1324, 2611 -> 2371, 2804 -> 2577, 3565 -> 3436
+//   mixed, R-MAT 100 000 nodes (22)        98.5 -> 96.0, 167 -> 151, 173 -> 158, 203 -> 200
+//   mixed, 40 000 nodes (39)               73.8 -> 70.8, 115 -> 103, 120 -> 111, 146 -> 140
+//   windows, 20 000 nodes, bf16 (6)        27.6 -> 27.1, 39.8 -> 37.2, 42.0 -> 39.3, 45.0 -> 43.3
+//   16x8 blocks, R-MAT 100 000 nodes (12)  83.9 -> 81.9, 139 -> 122
+// (More waves in what the smaller rings leave free, units in workgroups of one or two waves: sliced calls at
+// d = 96 1 to 2 % faster or slower, at 160 up to 14 % slower: the rows of more units at a time
+// do not stay in the L2s.)
 // STAGES: pairs of the ring in flight per wave (the kernels choose: two stages where a wave is alone
 // with a long run of blocks, one stage and more waves where runs are short and what has to be
 // hidden is the chain of loads in front of the first gather).
 template <int D, int STAGES>
 struct Geo {
   static_assert(D % 32 == 0 && D >= 32 && D <= 256, "head dimension: a multiple of 32 up to 256");
-  static constexpr int DP = D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256;
   static constexpr int T = D / 16;         // output tiles
   static constexpr int KS = D / 32;        // k-steps of the score product
-  static constexpr int TG = DP / 16;       // gather instructions per 32-row tile
-  static constexpr int ROW = DP * 2;       // bytes of a K / V row in LDS
-  static constexpr int GROW = D * 2;       // bytes of a contiguous K / V row in memory
-  static constexpr int CHUNKS = D / 8;     // 16-byte chunks of a row that exist
-  static constexpr int CPR = DP / 8;       // 16-byte chunks per LDS row == lanes per gathered row
-  static constexpr int RPI = 64 / CPR;     // rows per gather instruction
+  static constexpr int TG = D / 16;        // gather instructions per 32-row tile
+  static constexpr int ROW = D * 2;        // bytes of a K / V row, in memory and in LDS
+  static constexpr int CPR = D / 8;        // 16-byte chunks per row
   static constexpr int TILE = 32 * ROW;    // K (or V) rows of one pair
   static constexpr int STAGE = 2 * TILE;   // one pair: K tile, then V tile
   static constexpr int NS = STAGES;  // stages of the ring
@@ -181,81 +190,163 @@ struct Geo {
   static constexpr int WAVE_BYTES = NS * STAGE + META;
 };
 
-// Which of the pair's 32 key slots lane-row rho of gather instruction i fetches, and its inverse
-// (the row of the LDS tile a slot lands in: row i * RPI + rho). Chosen so that the slots a lane
-// fetches are groups of four consecutive dwords of the metadata (one 16-byte LDS read yields four
-// of its row ids). DP >= 64: slot = 4 * (rho + RPI * (i / 4)) + i % 4.
-template <int DP>
-__device__ __forceinline__ constexpr int slot_of(int i, int rho) {
-  if constexpr (DP == 32) return 4 * (rho >> 1) + 2 * i + (rho & 1);
-  constexpr int RPI = 512 / DP;
+// rows that straddle gather instructions (above), and the number of rows after which a row starts where
+// an instruction does again: that many rows, and instructions, later a lane's chunk has the same place in its row
+template <int D>
+constexpr bool straddling() {
+  return (D & (D - 1)) != 0;
+}
+template <int D>
+constexpr int rows_of_period() {
+  return D % 64 == 0 ? 8 : 16;
+}
+template <int D>
+constexpr int gathers_of_period() {
+  return rows_of_period<D>() * D / 512;
+}
+// Row of the tile that lane `lane` fetches a chunk of in gather instruction i, and the chunk's place in it.
+template <int D>
+__device__ __forceinline__ constexpr int gather_row(int i, int lane) {
+  return (i * 64 + lane) / (D / 8);
+}
+template <int D>
+__device__ __forceinline__ constexpr int gather_pos(int i, int lane) {
+  return (i * 64 + lane) % (D / 8);
+}
+// Which of the pair's 32 key slots lies in which row of the tile, and the inverse. Powers of two: such that
+// the slots a lane fetches are groups of four consecutive dwords of the metadata (one 16-byte LDS read
+// yields four of its row ids); D >= 64: slot = 4 * (rho + RPI * (i / 4)) + i % 4 in lane-row rho of instruction
+// i, RPI rows an instruction. Straddling rows: slot by slot.
+template <int D>
+__device__ __forceinline__ constexpr int slot_of_row(int row) {
+  if constexpr (straddling<D>()) return row;
+  if constexpr (D == 32) return 4 * ((row & 15) >> 1) + 2 * (row >> 4) + (row & 1);
+  constexpr int RPI = 512 / D;
+  const int i = row / RPI, rho = row % RPI;
   return 4 * (rho + RPI * (i >> 2)) + (i & 3);
 }
-template <int DP>
+template <int D>
 __device__ __forceinline__ constexpr int lds_row_of(int s) {
-  if constexpr (DP == 32) return ((s & 3) >> 1) * 16 + 2 * (s >> 2) + (s & 1);
-  constexpr int RPI = 512 / DP;
+  if constexpr (straddling<D>()) return s;
+  if constexpr (D == 32) return ((s & 3) >> 1) * 16 + 2 * (s >> 2) + (s & 1);
+  constexpr int RPI = 512 / D;
   const int rho = (s >> 2) & (RPI - 1);
   const int q = (s >> 2) / RPI;
   return ((s & 3) + 4 * q) * RPI + rho;
 }
 // XOR applied to the 16-byte chunk index of slot s inside its LDS row: the K tile is read with
 // one 16-byte read per lane (16 consecutive slots by 4 chunks), the V tile with transposing
-// 8-byte reads (4 consecutive slots by 32 bytes); each pattern wants its rows on different banks.
-template <int DP>
+// 8-byte reads (8 consecutive slots by 32 bytes in each half of the lanes); each pattern wants its 256
+// bytes on different banks.
+template <int D>
 __device__ __forceinline__ constexpr int swz_k(int s) {
   const int c = s & 15;
-  if constexpr (DP == 64) return (c & 3) | ((((c >> 2) ^ (c >> 3)) & 1) << 2);
-  if constexpr (DP >= 128) return c;
-  return ((c >> 1) & 1) | ((((c >> 2) ^ (c >> 3)) & 1) << 1);  // DP == 32
+  if constexpr (D == 32) return ((c >> 1) & 1) | ((((c >> 2) ^ (c >> 3)) & 1) << 1);
+  if constexpr (D == 64) return (c & 3) | ((((c >> 2) ^ (c >> 3)) & 1) << 2);
+  if constexpr (D == 192) return c >> 1;  // every other row begins on the same bank
+  if constexpr (straddling<D>()) return c >> 2;  // every fourth row
+  return c;
 }
-template <int DP>
+template <int D>
 __device__ __forceinline__ constexpr int swz_v(int s) {
-  if constexpr (DP == 32) return ((s >> 1) & 1) << 1;
-  return (s & 3) << 1;
+  if constexpr (D == 32) return ((s >> 1) & 1) << 1;
+  if constexpr (D == 64) return (s & 3) << 1;
+  if constexpr (D == 192) return ((s >> 1) & 3) << 1;
+  if constexpr (straddling<D>()) return ((s >> 2) & 1) << 1;
+  return (s & 7) << 1;
 }
 // The chunk a lane fetches in gather instruction i depends on i only through i % NK (K) and
 // i % NV (V), so that many byte offsets are kept per lane.
-template <int DP>
+template <int D>
 constexpr int distinct_k_offsets() {
-  return DP == 32 ? 2 : DP == 256 ? 8 : 4;
+  if (D == 192) return 2 * gathers_of_period<D>();
+  if (straddling<D>()) return gathers_of_period<D>();
+  return D == 32 ? 2 : D == 256 ? 8 : 4;
 }
-template <int DP>
+template <int D>
 constexpr int distinct_v_offsets() {
-  return DP == 32 ? 2 : 4;
+  if (straddling<D>()) return gathers_of_period<D>();
+  return D == 32 ? 2 : 4;
 }
-template <int DP>
+// Likewise the operand reads: k-step i reads at address i % KA plus i / KA of its stride, tile j at j % VA
+// plus j / VA. KA k-steps (64 bytes each) and VA tiles (32 bytes each) span the chunks an XOR moves within.
+template <int D>
+constexpr int distinct_k_reads() {
+  if (D == 192) return 2;
+  if (straddling<D>()) return 1;
+  return D / 32 < 4 ? D / 32 : 4;
+}
+template <int D>
+constexpr int distinct_v_reads() {
+  if (D == 192) return 4;
+  if (straddling<D>()) return 2;
+  return D / 16 < 8 ? (D == 32 ? 2 : 4) : 8;
+}
+template <int D>
 constexpr bool gather_offsets_periodic() {
-  constexpr int RPI = 512 / DP, TG = DP / 16;
-  for (int i = 0; i < TG; i++)
-    for (int rho = 0; rho < RPI; rho++) {
-      if (swz_k<DP>(slot_of<DP>(i, rho)) !=
-          swz_k<DP>(slot_of<DP>(i % distinct_k_offsets<DP>(), rho)))
+  for (int i = 0; i < D / 16; i++)
+    for (int lane = 0; lane < 64; lane++) {
+      const int s = slot_of_row<D>(gather_row<D>(i, lane));
+      const int ik = i % distinct_k_offsets<D>(), iv = i % distinct_v_offsets<D>();
+      if (gather_pos<D>(i, lane) != gather_pos<D>(ik, lane) || gather_pos<D>(i, lane) != gather_pos<D>(iv, lane))
         return false;
-      if (swz_v<DP>(slot_of<DP>(i, rho)) !=
-          swz_v<DP>(slot_of<DP>(i % distinct_v_offsets<DP>(), rho)))
+      if (swz_k<D>(s) != swz_k<D>(slot_of_row<D>(gather_row<D>(ik, lane)))) return false;
+      if (swz_v<D>(s) != swz_v<D>(slot_of_row<D>(gather_row<D>(iv, lane)))) return false;
+      if ((gather_pos<D>(i, lane) ^ swz_k<D>(s)) >= D / 8 || (gather_pos<D>(i, lane) ^ swz_v<D>(s)) >= D / 8)
         return false;
     }
   return true;
 }
-static_assert(gather_offsets_periodic<32>() && gather_offsets_periodic<64>() &&
-                  gather_offsets_periodic<128>() && gather_offsets_periodic<256>(),
-              "gather offsets must repeat with the stated periods");
-
-// the two maps are inverse to each other for every power-of-two width
-template <int DP>
+// the two maps of rows and slots are inverse to each other, and the second half of a tile lies a fixed
+// distance behind the first
+template <int D>
 constexpr bool slot_maps_consistent() {
-  constexpr int RPI = 512 / DP, TG = DP / 16;
-  for (int i = 0; i < TG; i++)
-    for (int rho = 0; rho < RPI; rho++) {
-      const int s = slot_of<DP>(i, rho);
-      if (s < 0 || s >= 32 || lds_row_of<DP>(s) != i * RPI + rho) return false;
+  for (int row = 0; row < 32; row++) {
+    const int s = slot_of_row<D>(row);
+    if (s < 0 || s >= 32 || lds_row_of<D>(s) != row) return false;
+  }
+  for (int s = 0; s < 16; s++)
+    if (lds_row_of<D>(s + 16) - lds_row_of<D>(s) != lds_row_of<D>(16) - lds_row_of<D>(0) ||
+        swz_k<D>(s + 16) != swz_k<D>(s) || swz_v<D>(s + 16) != swz_v<D>(s))
+      return false;
+  return true;
+}
+// what the lanes of one group (K: 16 slots, V: 8 slots by two chunks) read lies in different chunks of the
+// 256 bytes that the banks span, and each k-step and tile where its address and stride say
+template <int D>
+constexpr bool operand_reads_consistent() {
+  constexpr int KA = distinct_k_reads<D>(), VA = distinct_v_reads<D>(), C = D / 8;
+  for (int i = 0; i < D / 32; i++)
+    for (int g = 0; g < 4; g++) {
+      unsigned banks = 0;
+      for (int s = 0; s < 16; s++) {
+        const int chunk = (4 * i + g) ^ swz_k<D>(s);
+        banks |= 1u << ((lds_row_of<D>(s) * C + chunk) & 15);
+        if (chunk >= C || chunk != ((4 * (i % KA) + g) ^ swz_k<D>(s)) + i / KA * KA * 4) return false;
+      }
+      if (banks != 0xFFFFu) return false;
+    }
+  for (int j = 0; j < D / 16; j++)
+    for (int s0 = 0; s0 < 16; s0 += 8) {
+      unsigned banks = 0;
+      for (int s = s0; s < s0 + 8; s++)
+        for (int x = 0; x < 2; x++) {
+          const int chunk = (2 * j + x) ^ swz_v<D>(s);
+          banks |= 1u << ((lds_row_of<D>(s) * C + chunk) & 15);
+          if (chunk >= C || chunk != ((2 * (j % VA) + x) ^ swz_v<D>(s)) + j / VA * VA * 2) return false;
+        }
+      if (banks != 0xFFFFu) return false;
     }
   return true;
 }
-static_assert(slot_maps_consistent<32>() && slot_maps_consistent<64>() &&
-                  slot_maps_consistent<128>() && slot_maps_consistent<256>(),
-              "slot_of and lds_row_of must be inverse");
+template <int D>
+constexpr bool maps_consistent() {
+  return gather_offsets_periodic<D>() && slot_maps_consistent<D>() && operand_reads_consistent<D>();
+}
+static_assert(maps_consistent<32>() && maps_consistent<64>() && maps_consistent<96>() &&
+                  maps_consistent<128>() && maps_consistent<160>() && maps_consistent<192>() &&
+                  maps_consistent<224>() && maps_consistent<256>(),
+              "tile maps");
 
 // Problem description shared by every kernel.
 template <typename ET>
@@ -295,11 +386,11 @@ struct PairPipeline {
   static constexpr int KS = G::KS;
   static constexpr int NS = G::NS;
   static constexpr int TG = G::TG;
-  static constexpr int DP = G::DP;
-  static constexpr int NK = distinct_k_offsets<DP>();
-  static constexpr int NV = distinct_v_offsets<DP>();
-  static constexpr int NVA = T < 4 ? T : 4;  // V read addresses kept: tile j reads at
-                                             // vReadAddr[j % 4] + (j / 4) * 128
+  static constexpr int NK = distinct_k_offsets<D>();
+  static constexpr int NV = distinct_v_offsets<D>();
+  static constexpr int KA = distinct_k_reads<D>();
+  static constexpr int VA = distinct_v_reads<D>();
+  static constexpr int NI = straddling<D>() ? gathers_of_period<D>() : 1;
   static constexpr int BPS = W8 ? 4 : 2;  // blocks of the structure per step
   static constexpr bool SPLIT_P = sizeof(ET) == 2 && !__is_same(ET, _Float16);  // bf16
 
@@ -311,13 +402,12 @@ struct PairPipeline {
   half8 qf[KS];
   unsigned ring;        // LDS byte address of this wave's ring
   unsigned metaBase;    // LDS byte address of this wave's two metadata slots
-  unsigned kReadAddr[2][KS];  // K tile: slot 16b + c, chunk 4i + g (swizzled)
-  unsigned vReadAddr[NVA];  // V tile: transposing read of tiles 0..3, first key half
-  unsigned idReadAddr;     // metadata: this lane's row ids
+  unsigned kReadAddr[KA];  // K tile: slot c, chunk 4i + g (swizzled)
+  unsigned vReadAddr[VA];  // V tile: transposing read of tiles 0.., first key half
+  unsigned idReadAddr[NI];  // metadata: this lane's row ids
   unsigned maskReadAddr;   // metadata: the bitmap dword with this lane's bits of block A
   int keepPos[4];          // bit position of element i in that dword
   uint32_t gatherOffK[NK], gatherOffV[NV];  // byte offset inside the row this lane fetches
-  uint32_t gatherLive;  // D < DP: bit i / bit 16 + i: the chunk of K / V instruction i exists
   int lane, g, c;
 
   __device__ __forceinline__ void init(const Problem<ET>& pb, int w, unsigned ringAddr, int head) {
@@ -343,43 +433,31 @@ struct PairPipeline {
         for (int i = 0; i < KS; i++) qf[i] = __builtin_bit_cast(half8, zero16);
       }
     }
-    // gather: in instruction i this lane fetches chunk (lane % CPR) ^ swizzle of slot
-    // slot_of(i, lane / CPR); the chunk lands at ring + i * 1024 + lane * 16
-    const int rho = lane / G::CPR;
-    const int pos = lane % G::CPR;
-    gatherLive = 0;
+    // gather: in instruction i this lane fetches chunk gather_pos ^ swizzle of the slot in row gather_row;
+    // the chunk lands at ring + i * 1024 + lane * 16
 #pragma unroll
     for (int i = 0; i < TG; i++) {
-      const int s = slot_of<DP>(i, rho);
-      const int ck = pos ^ swz_k<DP>(s), cv = pos ^ swz_v<DP>(s);
-      if (i < NK) gatherOffK[i] = (uint32_t)(ck * 16 + (HEADS ? head * D * 2 : 0));
-      if (i < NV) gatherOffV[i] = (uint32_t)(cv * 16 + (HEADS ? head * D * 2 : 0));
-      if (ck < G::CHUNKS) gatherLive |= 1u << i;
-      if (cv < G::CHUNKS) gatherLive |= 1u << (16 + i);
+      const int s = slot_of_row<D>(gather_row<D>(i, lane)), pos = gather_pos<D>(i, lane);
+      if (i < NK) gatherOffK[i] = (uint32_t)((pos ^ swz_k<D>(s)) * 16 + (HEADS ? head * D * 2 : 0));
+      if (i < NV) gatherOffV[i] = (uint32_t)((pos ^ swz_v<D>(s)) * 16 + (HEADS ? head * D * 2 : 0));
     }
     // score product: lane (g, c) reads, for block b and k-step i, chunk 4i + g of slot 16b + c
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
-      const int s = 16 * b + c;
-#pragma unroll
-      for (int i = 0; i < KS; i++)
-        kReadAddr[b][i] = ring + lds_row_of<DP>(s) * G::ROW + (((4 * i + g) ^ swz_k<DP>(s)) * 16);
-    }
+    for (int i = 0; i < KA; i++)
+      kReadAddr[i] = ring + lds_row_of<D>(c) * G::ROW + (((4 * i + g) ^ swz_k<D>(c)) * 16);
     // P V product: lane (g, c = 4e + x) addresses slot 16h + 4g + e, columns 16j + 4x .. +3:
     // chunk 2j + x/2 (swizzled), byte (x % 2) * 8 inside it. h = 1 is a fixed distance away.
     {
       const int e = c >> 2, x = c & 3;
       const int s = 4 * g + e;
 #pragma unroll
-      for (int j = 0; j < NVA; j++)
-        vReadAddr[j] = ring + G::TILE + lds_row_of<DP>(s) * G::ROW +
-                       (((2 * j + (x >> 1)) ^ swz_v<DP>(s)) * 16) + (x & 1) * 8;
+      for (int j = 0; j < VA; j++)
+        vReadAddr[j] = ring + G::TILE + lds_row_of<D>(s) * G::ROW +
+                       (((2 * j + (x >> 1)) ^ swz_v<D>(s)) * 16) + (x & 1) * 8;
     }
     // metadata slot: ids of step q at q * 128, bitmaps at 512 + q * 64
-    if constexpr (DP == 32)
-      idReadAddr = metaBase + (4 * (rho >> 1) + (rho & 1)) * 4;
-    else
-      idReadAddr = metaBase + rho * 16;
+#pragma unroll
+    for (int i = 0; i < NI; i++) idReadAddr[i] = metaBase + slot_of_row<D>(gather_row<D>(i, lane)) * 4;
     const int maskByte = ((g >> 1) * 2 + (c >> 3)) * 8 + 7 - (c & 7);
     maskReadAddr = metaBase + 512 + (maskByte >> 2) * 4;
 #pragma unroll
@@ -417,22 +495,36 @@ struct PairPipeline {
   // position in its metadata slot is the compile-time Q4 plus the run-time q (one of them 0).
   template <int STAGE_IDX, int Q4>
   __device__ __forceinline__ void issue_gather(const Problem<ET>& pb, int metaSlot, int q) {
-    // row ids of this lane's TG slots: groups of four consecutive dwords of the step's 32 ids
     int rows[TG];
-    const unsigned ida = idReadAddr + (unsigned)(metaSlot * G::META_SLOT + q * 128);
-    if constexpr (DP == 32) {
-      const int2v r = lds_read2_b32<Q4 * 32, Q4 * 32 + 2>(ida);
+    const unsigned at = (unsigned)(metaSlot * G::META_SLOT + q * 128);
+    if constexpr (straddling<D>()) {
+      // slot i of this lane, and the ones as many rows further as a period has
+      constexpr int P = rows_of_period<D>(), HALVES = 32 / P / 2;
+      int2v r[NI][HALVES];
+#pragma unroll
+      for (int i = 0; i < NI; i++) {
+        r[i][0] = lds_read2_b32<Q4 * 32, Q4 * 32 + P>(idReadAddr[i] + at);
+        if constexpr (HALVES == 2)
+          r[i][1] = lds_read2_b32<Q4 * 32 + 2 * P, Q4 * 32 + 3 * P>(idReadAddr[i] + at);
+      }
+      lds_wait();
+#pragma unroll
+      for (int i = 0; i < TG; i++) rows[i] = r[i % NI][i / NI / 2][i / NI % 2];
+    } else if constexpr (D == 32) {
+      const int2v r = lds_read2_b32<Q4 * 32, Q4 * 32 + 2>(idReadAddr[0] + at);
       lds_wait();
       rows[0] = r[0];
       rows[1] = r[1];
     } else {
-      // group q of four slots starts RPI * 4 slots (RPI * 16 bytes) after group q - 1
+      // groups of four consecutive dwords; group q of four slots starts 64 / CPR * 4 slots after group q - 1
+      const unsigned ida = idReadAddr[0] + at;
+      constexpr int RPI = 64 / G::CPR;
       int4v r[TG / 4];
       r[0] = lds_read_b128<Q4 * 128>(ida);
-      if constexpr (TG >= 8) r[1] = lds_read_b128<Q4 * 128 + 1 * G::RPI * 16>(ida);
+      if constexpr (TG >= 8) r[1] = lds_read_b128<Q4 * 128 + 1 * RPI * 16>(ida);
       if constexpr (TG >= 16) {
-        r[2] = lds_read_b128<Q4 * 128 + 2 * G::RPI * 16>(ida);
-        r[3] = lds_read_b128<Q4 * 128 + 3 * G::RPI * 16>(ida);
+        r[2] = lds_read_b128<Q4 * 128 + 2 * RPI * 16>(ida);
+        r[3] = lds_read_b128<Q4 * 128 + 3 * RPI * 16>(ida);
       }
       lds_wait();
 #pragma unroll
@@ -442,7 +534,7 @@ struct PairPipeline {
     }
     const char* Kb = reinterpret_cast<const char*>(pb.K);
     const char* Vb = reinterpret_cast<const char*>(pb.V);
-    const uint32_t rowBytes = HEADS ? (uint32_t)pb.pitchIn * 2u : (uint32_t)G::GROW;
+    const uint32_t rowBytes = HEADS ? (uint32_t)pb.pitchIn * 2u : (uint32_t)G::ROW;
     const int ringU = uniform((int)ring);
 #pragma unroll
     for (int i = 0; i < TG; i++) {
@@ -452,39 +544,32 @@ struct PairPipeline {
 #endif
     }
     // one gather instruction: 64 lanes x 16 bytes of K (V) rows into 1 KiB of the stage
-    auto gather = [&](const char* src, bool live, int ldsOffset) {
+    auto gather = [&](const char* src, int ldsOffset) {
       F3S_LDS int4v* dst = (F3S_LDS int4v*)(uintptr_t)(ringU + ldsOffset);
-      if constexpr (D == DP) {
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const int4v*>(src), dst, 16, 0, 0);
-      } else {
-        if (live)
-          __builtin_amdgcn_global_load_lds(reinterpret_cast<const int4v*>(src), dst, 16, 0, 0);
-      }
+      __builtin_amdgcn_global_load_lds(reinterpret_cast<const int4v*>(src), dst, 16, 0, 0);
     };
     if constexpr (WIDE) {
       // the reference indexes rows with int64_t (src/F3S_kernel.cu:1422-1423)
 #pragma unroll
       for (int i = 0; i < TG; i++)
         gather(Kb + ((uint64_t)(uint32_t)rows[i] * rowBytes + gatherOffK[i % NK]),
-               (gatherLive >> i) & 1u, STAGE_IDX * G::STAGE + i * 1024);
+               STAGE_IDX * G::STAGE + i * 1024);
 #pragma unroll
       for (int i = 0; i < TG; i++)
         gather(Vb + ((uint64_t)(uint32_t)rows[i] * rowBytes + gatherOffV[i % NV]),
-               (gatherLive >> (16 + i)) & 1u, STAGE_IDX * G::STAGE + G::TILE + i * 1024);
+               STAGE_IDX * G::STAGE + G::TILE + i * 1024);
     } else {
 #pragma unroll
       for (int i = 0; i < TG; i++) {
         const uint32_t ro = HEADS ? __umul24((uint32_t)rows[i], rowBytes)
                                   : (uint32_t)rows[i] * rowBytes;
-        gather(Kb + (ro + gatherOffK[i % NK]), (gatherLive >> i) & 1u,
-               STAGE_IDX * G::STAGE + i * 1024);
+        gather(Kb + (ro + gatherOffK[i % NK]), STAGE_IDX * G::STAGE + i * 1024);
       }
 #pragma unroll
       for (int i = 0; i < TG; i++) {
         const uint32_t ro = HEADS ? __umul24((uint32_t)rows[i], rowBytes)
                                   : (uint32_t)rows[i] * rowBytes;
-        gather(Vb + (ro + gatherOffV[i % NV]), (gatherLive >> (16 + i)) & 1u,
-               STAGE_IDX * G::STAGE + G::TILE + i * 1024);
+        gather(Vb + (ro + gatherOffV[i % NV]), STAGE_IDX * G::STAGE + G::TILE + i * 1024);
       }
     }
   }
@@ -499,25 +584,28 @@ struct PairPipeline {
   template <int STAGE_IDX, int Q4>
   __device__ __forceinline__ void read_operands(int metaSlot, int q, Operands& op) {
     constexpr int SO = STAGE_IDX * G::STAGE;
-#pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int i = 0; i < KS; i++) op.k[b][i] = lds_read_b128<SO>(kReadAddr[b][i]);
+    read_k_step<SO, 0>(op);
     read_v_tile<SO, 0>(op);
     op.words = lds_read2_b32<Q4 * 16, Q4 * 16 + 8>(
         maskReadAddr + (unsigned)(metaSlot * G::META_SLOT + q * 64));
   }
-  // tile J of the V operand: 128 bytes (eight chunks) per four tiles beyond tile J % 4
+  template <int SO, int I>
+  __device__ __forceinline__ void read_k_step(Operands& op) {
+    constexpr int OFF = SO + I / KA * KA * 64;
+    op.k[0][I] = lds_read_b128<OFF>(kReadAddr[I % KA]);
+    op.k[1][I] = lds_read_b128<OFF + half_distance()>(kReadAddr[I % KA]);
+    if constexpr (I + 1 < KS) read_k_step<SO, I + 1>(op);
+  }
   template <int SO, int J>
   __device__ __forceinline__ void read_v_tile(Operands& op) {
-    constexpr int OFF = SO + (J / 4) * 128;
-    op.v[J][0] = lds_read_tr16_b64<OFF>(vReadAddr[J % 4]);
-    op.v[J][1] = lds_read_tr16_b64<OFF + v_half_distance()>(vReadAddr[J % 4]);
+    constexpr int OFF = SO + J / VA * VA * 32;
+    op.v[J][0] = lds_read_tr16_b64<OFF>(vReadAddr[J % VA]);
+    op.v[J][1] = lds_read_tr16_b64<OFF + half_distance()>(vReadAddr[J % VA]);
     if constexpr (J + 1 < T) read_v_tile<SO, J + 1>(op);
   }
   // LDS distance between the rows of slot s and slot s + 16 of a tile
-  static __device__ __forceinline__ constexpr int v_half_distance() {
-    return (lds_row_of<DP>(16) - lds_row_of<DP>(0)) * G::ROW;
+  static __device__ __forceinline__ constexpr int half_distance() {
+    return (lds_row_of<D>(16) - lds_row_of<D>(0)) * G::ROW;
   }
 
   __device__ __forceinline__ void consume(Operands& op) {

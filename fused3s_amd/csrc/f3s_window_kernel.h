@@ -32,7 +32,7 @@ using pipe::kLog2e;
 //   TEAM_SHORT  one workgroup for every window: four waves of one stage. Four workgroups per CU at
 //               D = 32, three at D = 64 (two stages allow two), two up to D = 128, one above.
 //   TEAM_PAIRS  the same with two stages at D = 32, where they cost no workgroup (see two_stages).
-// Graphs of short windows take f3s_fwd_mixed_kernel instead (f3s_attention_units.hip).
+// Graphs of short windows take f3s_fwd_mixed_kernel instead (f3s_attention_mixed.hip).
 enum Team { TEAM_SHORT, TEAM_PAIRS };
 constexpr int kTeamWaves = 4;  // MergedRows takes four
 constexpr int team_stages(Team t) { return t == TEAM_SHORT ? 1 : 2; }
@@ -70,8 +70,7 @@ inline bool two_stages(int d, int64_t nTcb16, int heads, int N) {
 
 // LDS of a workgroup: its waves' rings
 constexpr size_t team_lds(Team t, int d) {
-  const int dp = d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : 256;
-  return (size_t)kTeamWaves * (team_stages(t) * 128 * dp + 2 * 768);
+  return (size_t)kTeamWaves * (team_stages(t) * 128 * d + 2 * 768);
 }
 
 // Constant-rate (100 MHz) timestamp shared by all CUs, and an id of the CU this wave runs on:
