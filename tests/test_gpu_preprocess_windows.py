@@ -237,6 +237,39 @@ def test_own_columns(oracle_mod, N, W):
     assert np.array_equal(got["tcbBitMap"].cpu().view(torch.int64).numpy().view(np.uint64), want["tcbBitMap"])
 
 
+# Columns that crowd into few bins are binned again, by what they are, around the window's middle edge: communities
+# around the window's own columns, below, above, and across the ends of the range, narrower and wider than the
+# 512 columns (or four bins) that half of the bins then cover, alone and with edges elsewhere
+@pytest.mark.parametrize("N", [1025, 100_000, (1 << 17) - 17 * 128 - 1, (1 << 17) - 17 * 128, 500_000])
+def test_communities_around_own_columns(oracle_mod, N):
+    from fused3s_amd import capi
+    print("case communities N=%d" % N, flush=True)
+    rng = np.random.default_rng(N)
+    nRW = (N + 15) // 16
+    rows = [np.zeros(0, np.int32)] * N
+    kinds = [(reach, shift, size) for reach in (40, 120, 300, 700, 3000) for shift in (-1, 0, 1) for size in (150, 500, 940)]
+    picked = np.unique(np.concatenate([[0, 1, nRW - 2, nRW - 1],
+                                       rng.choice(nRW, min(nRW - 4, len(kinds) + 10), replace=False)]))
+    for k, w in enumerate(rng.permutation(picked)):
+        reach, shift, size = kinds[k % len(kinds)]
+        own = np.arange(16 * w, min(16 * w + 16, N))
+        near = np.arange(max(16 * w + shift * reach - reach, 0), min(16 * w + 16 + shift * reach + reach, N))
+        if len(near) == 0:
+            near = own
+        for r in own:
+            cols = rng.choice(near, size=min(size // 16 - 1, len(near)), replace=False)
+            far = rng.integers(0, N, k % 2)
+            rows[r] = np.unique(np.concatenate([cols, far, [r]])).astype(np.int32)
+    rowPtr = np.zeros(N + 1, np.int32)
+    rowPtr[1:] = np.cumsum([len(r) for r in rows])
+    colIdx = np.concatenate(rows).astype(np.int32)
+    want = oracle_mod.preprocess(rowPtr, colIdx, N)
+    got = capi.preprocess(torch.as_tensor(rowPtr).cuda(), torch.as_tensor(colIdx).cuda(), N)
+    for key in KEYS:
+        assert np.array_equal(got[key].cpu().numpy(), want[key]), key
+    assert np.array_equal(got["tcbBitMap"].cpu().view(torch.int64).numpy().view(np.uint64), want["tcbBitMap"])
+
+
 def split_columns(rng, cols, lengths):
     """16 ascending rows of the given lengths over `cols`, which together name every one of them."""
     cols = np.sort(cols)
