@@ -1,7 +1,7 @@
 // The inner loop of the fused SDDMM -> online softmax -> SpMM kernels for gfx950 (MI355X),
 // wave64: one wave walks a run of consecutive TC blocks of one 16-row window, two 16x16 blocks
 // (a "pair", 32 keys) per step, with running (m, l, O) in registers. Every kernel of the library
-// (workgroup per window, wave per (window, column slice) unit, wave per short window, 16x8
+// (workgroup per window, wave per (window, column slice) unit, waves and workgroups mixed, 16x8
 // blocks, multi-head, timed) is this loop plus its own prologue and epilogue.
 //
 // Replaces the loop bodies of f3sKernel1tb1rw / ...Scheduled / ...ScheduledPermutedQKV[ScaleQK],

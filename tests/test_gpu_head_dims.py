@@ -83,8 +83,8 @@ def test_single_head_entry(oracle_mod, d, dtype):
 @pytest.mark.parametrize("d", NEW_DIMS)
 def test_heads_entry_and_short_window_split(oracle_mod, d):
     """f3s_attention_fwd_heads on pitched [N, 2, d] inputs: bit-identical to per-head launches.
-    The graph has more than 1024 windows of a few blocks each, so with an order the call is split
-    into the wave-per-window kernel and the workgroup-per-window kernel."""
+    The graph has more than 1024 windows of a few blocks each, so with an order the short
+    ones are computed by waves and the long ones by workgroups of the same launch."""
     from fused3s_amd import capi
     print("case head_dim heads d=%d" % d, flush=True)
     N, heads, pad = 20_000, 2, 8

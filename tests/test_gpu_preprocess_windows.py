@@ -170,7 +170,7 @@ def test_waves_of_the_one_launch(oracle_mod, nRW, edges, W):
         assert np.array_equal(got[k].cpu().numpy(), want[k]), k
 
 
-# Above 393 216 nodes a workgroup ranks the windows of 961 to 4096 and of up to 16 384 edges: 512 and 1024
+# Above 393 216 nodes a workgroup ranks the windows of 961 to 2048 and of up to 16 384 edges: 256 and 1024
 # edges at a time, bins of 32 edges and more by a radix sort. The last column of a power of two has a bit
 # more than the others
 @pytest.mark.parametrize("N", [1 << 19, (1 << 19) - 1, 500_000])

@@ -1,7 +1,7 @@
-"""Graphs of short windows: the call is split between the wave-per-window kernel and the
-four-wave kernel (long windows). Checked against the reference-emulating oracle for fp16 and
-bf16, single head and multi-head, with the heavy-first order, a shuffled order (a long window may
-then lie outside the four-wave kernel's grid) and natural order (no split)."""
+"""Graphs of short windows: one launch computes the short windows by waves and the long ones by
+workgroups. Checked against the reference-emulating oracle for fp16 and bf16, single head and
+multi-head, with the heavy-first order, a shuffled order (a long window may then lie outside the
+workgroups' share) and natural order (a workgroup for every window)."""
 import numpy as np
 import pytest
 import torch

@@ -1,5 +1,5 @@
 """How units are dealt to the XCDs: head groups, slice groups, phases and window groups of the
-column-sliced schedule, and the chunks of the wave-per-window launches, at head counts and window
+column-sliced schedule, and the chunks of the launches with waves for short windows, at head counts and window
 counts that do not divide evenly. Every (window, head) has to be computed exactly once."""
 import numpy as np
 import pytest
