@@ -90,8 +90,10 @@ f3s_fwd_mixed_kernel(const int32_t* __restrict__ windowOrder,
   const int wave = uniform(threadIdx.x >> 6);
   const int pitchOut = HEADS ? ldOut : D;
   // block ranges that do not fit the structure (a mismatched rowWindowOffset) are not followed: such a window
-  // is treated as empty, and so is one that does not exist (a corrupt order entry must not index out of range)
-  const auto is_long = [&](int t0, int t1) { return t0 >= 0 && (int64_t)t1 <= nTcb && t1 - t0 > maxBlocks; };
+  // is treated as empty, and so is one that does not exist (a corrupt order entry must not index out of range).
+  // An end in front of the begin is looked at before the two are subtracted: the difference may not fit.
+  const auto fits = [&](int t0, int t1) { return t0 >= 0 && t1 >= t0 && (int64_t)t1 <= nTcb; };
+  const auto is_long = [&](int t0, int t1) { return fits(t0, t1) && t1 - t0 > maxBlocks; };
 
   // Where this wave stands in the given and in natural order, and what it will ask for, in two rounds of loads.
   const int waveGroups = (int)gridDim.x - teamGroups;
@@ -155,7 +157,7 @@ f3s_fwd_mixed_kernel(const int32_t* __restrict__ windowOrder,
       if constexpr (HEADS) head = even ? natural.head : given.head;
       if ((even ? natural.pos : given.pos) >= nRW || (unsigned)w >= (unsigned)nRW) return;
       if (!even && given.pos < longPrefix && is_long(t0, t1)) return;  // a team's
-      if (t0 < 0 || (int64_t)t1 > nTcb) t1 = t0;
+      if (!fits(t0, t1)) t1 = t0;
     }
     Pipe pp;
     pp.init(pb, w, (unsigned)(uintptr_t)(F3S_LDS unsigned char*)ring, head);

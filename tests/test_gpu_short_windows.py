@@ -252,3 +252,33 @@ def test_waves_and_teams_of_narrow_blocks(oracle_mod, longest, d):
     assert np.isfinite(got).all()
     assert np.abs(got - want).max() < MAX_ABS
     assert np.abs(got_scores.reshape(-1) - np.asarray(scores).reshape(-1)).max() < 2e-2
+
+
+# Offsets that do not belong to the structure: a window whose end lies so far in front of its begin that the
+# difference of the two does not fit 32 bits is empty, and so is the one that begins there
+@pytest.mark.parametrize("heads", [1, 4])
+def test_ends_far_in_front_of_begins(heads):
+    from fused3s_amd import capi
+    print("case ends far in front of begins heads=%d" % heads, flush=True)
+    rng = np.random.default_rng(heads)
+    nRW, d = 1030, 64
+    counts = rng.integers(1, 6, nRW)
+    counts[::90] = 40
+    N, pre = _structure(rng, nRW, counts)
+    dev = lambda a: torch.as_tensor(a).cuda()
+    atox, bm = dev(pre["sparseAToXidx"]), dev(pre["tcbBitMap"].view(np.int64)).view(torch.uint64)
+    order = dev(np.argsort(-counts, kind="stable").astype(np.int32))
+    g = torch.Generator().manual_seed(heads)
+    Q, K, V = [torch.randn((N, heads, d), generator=g).half().cuda() for _ in range(3)]
+    whole = capi.attention_heads(dev(pre["rowWindowOffset"]), order, atox, bm, N, Q, K, V, 8.0)
+    rwo = pre["rowWindowOffset"].copy()
+    bad = [89, 200, 359, 1000]  # 89 and 359 in front of long windows
+    rwo[np.array(bad) + 1] = [-2**31, -2**31 + 7, -2**31 + 1, -2**31 + 1000]
+    got = capi.attention_heads(dev(rwo), order, atox, bm, N, Q, K, V, 8.0)
+    torch.cuda.synchronize()
+    rows = torch.zeros(16 * nRW, dtype=torch.bool, device="cuda")
+    for w in bad:
+        rows[16 * w:16 * w + 32] = True
+    rows = rows[:N]
+    assert not got[rows].any()
+    assert torch.equal(got[~rows], whole[~rows])
