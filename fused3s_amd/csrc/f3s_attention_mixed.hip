@@ -54,18 +54,21 @@ struct WaveSplit {
 };
 
 // Workgroups of two kinds.
-//   teams   teamGroups of them look through the first longPrefix positions of the order, a thread per (position,
+//   teams   the first teamGroups of the grid look through all positions of the order, a thread per (position,
 //           head) unit, and compute the windows of more than maxBlocks TC blocks that they find, one after the
 //           other with all of their waves. In a heavy-first order those are its first positions, and they
-//           are dealt round-robin.
-//   others  a wave takes a whole window (of one head, or of NH) and writes its rows from its registers.
-//           A long window beyond longPrefix (the order is not heavy-first) is computed by one as well.
-// Where the order's first window is not a long one nobody is: the teams then come last and leave at once, and the
-// waves take the windows in natural order instead of the given one, 1 << evenShift in a row to an XCD. Windows
-// that follow each other in a graph of communities name the same rows, of which a heavy-first order makes
-// as many visits as there are block counts; and when the longest window is little more than twice the
-// mean, it does not matter which one starts last.
-// Without an order the teams look through all windows (longPrefix is their number).
+//           are dealt round-robin; in any other they start first all the same. (Looked for among as many positions
+//           as there can be long windows, those of other orders were left to single waves: d = 64, R-MAT 169 343
+//           nodes, 17 blocks a window, longest 759, natural order given as the order: 218 us, now 86.)
+//   others  a wave takes a whole window (of one head, or of NH) that is not a long one and writes its rows from
+//           its registers.
+// Where the order's first window is not a long one, none is if the order is heavy-first: evenTeams are then
+// enough to look, the other teams leave, and the waves take the windows in natural order instead of the given
+// one, 1 << evenShift in a row to an XCD. Windows that follow each other in a graph of communities name the same
+// rows, of which a heavy-first order makes as many visits as there are block counts (100 000 nodes, 6 blocks a
+// window, 8 x 32: 74 us in the given order, 58); and when the longest window is little more than twice the mean, it
+// does not matter which one starts last. An order that ends in an entry out of range, or twice in the same
+// one, names some of the windows and is filled up: it is followed as it stands.
 // W8: 16x8 blocks, with the scores to sddmm if it is not null; maxBlocks and nTcb then count such blocks.
 template <typename ET, int D, int NWAVES, bool SOFTMAX, bool HEADS, bool W8, int NH = 1>
 __global__ __launch_bounds__(NWAVES * 64)
@@ -74,7 +77,7 @@ f3s_fwd_mixed_kernel(const int32_t* __restrict__ windowOrder,
                      const int32_t* __restrict__ rowWindowOffset,
                      const int32_t* __restrict__ sparseAToXidx,
                      const uint8_t* __restrict__ bitmapBytes, WaveSplit split, int evenShift,
-                     int teamGroups, int longPrefix, int maxBlocks, int N, int nRW, int64_t nTcb,
+                     int teamGroups, int evenTeams, int maxBlocks, int N, int nRW, int64_t nTcb,
                      const ET* __restrict__ Q, const ET* __restrict__ K, const ET* __restrict__ V,
                      float scaleLog2, float* __restrict__ out, int nHeads, int ldIn, int ldOut,
                      float* __restrict__ sddmm) {
@@ -97,35 +100,39 @@ f3s_fwd_mixed_kernel(const int32_t* __restrict__ windowOrder,
 
   // Where this wave stands in the given and in natural order, and what it will ask for, in two rounds of loads.
   const int waveGroups = (int)gridDim.x - teamGroups;
-  const int givenGroup = (int)blockIdx.x - teamGroups;  // negative: a team
-  const Unit given = split.unit(max(givenGroup, 0), NWAVES, wave);
+  const Unit given = split.unit(max((int)blockIdx.x - teamGroups, 0), NWAVES, wave);
   WaveSplit evenSplit = split;
   evenSplit.chunkShift = evenShift;
-  const Unit natural = evenSplit.unit((int)blockIdx.x, NWAVES, wave);
-  int firstWindow = -1, givenWindow = given.pos;
+  const Unit natural = evenSplit.unit(max((int)blockIdx.x - evenTeams, 0), NWAVES, wave);
+  int firstWindow = -1, nextToLast = -1, lastWindow = -1, givenWindow = given.pos;
   if (windowOrder) {
     firstWindow = windowOrder[0];
+    nextToLast = windowOrder[nRW - 2];
+    lastWindow = windowOrder[nRW - 1];
     givenWindow = windowOrder[min(given.pos, nRW - 1)];
   }
   const int natural0 = rowWindowOffset[min(natural.pos, nRW - 1)];
   const int natural1 = rowWindowOffset[min(natural.pos, nRW - 1) + 1];
-  asm volatile("" : : "s"(firstWindow), "s"(givenWindow), "s"(natural0), "s"(natural1));
+  asm volatile("" : : "s"(firstWindow), "s"(nextToLast), "s"(lastWindow), "s"(givenWindow), "s"(natural0), "s"(natural1));
   const int first = (unsigned)firstWindow < (unsigned)nRW ? firstWindow : 0;
   const int most = rowWindowOffset[first + 1] - rowWindowOffset[first];
   const int ask = (unsigned)givenWindow < (unsigned)nRW ? givenWindow : 0;
   const int given0 = rowWindowOffset[ask], given1 = rowWindowOffset[ask + 1];
   asm volatile("" : : "s"(most), "s"(given0), "s"(given1));
-  const bool even = firstWindow == first && most <= maxBlocks;
-  const bool team = !even && givenGroup < 0;
-  if (even && (int)blockIdx.x >= waveGroups) return;
+  const bool filledUp =
+      (unsigned)nextToLast >= (unsigned)nRW || (unsigned)lastWindow >= (unsigned)nRW || nextToLast == lastWindow;
+  const bool even = firstWindow == first && most <= maxBlocks && !filledUp;
+  const int teams = even ? evenTeams : teamGroups;
+  const bool team = (int)blockIdx.x < teams;
+  if (even && (int)blockIdx.x >= evenTeams + waveGroups) return;
 
   int found = 0;  // units of a team in sList
   if (team) {
     if (threadIdx.x == 0) sFound = 0;
     __syncthreads();
-    const int64_t u = (int64_t)blockIdx.x + (int64_t)threadIdx.x * teamGroups;
-    if (u < (int64_t)longPrefix * nHeads) {
-      const int pos = (int)(u / nHeads), w = windowOrder ? windowOrder[pos] : pos;
+    const int64_t u = (int64_t)blockIdx.x + (int64_t)threadIdx.x * teams;
+    if (u < (int64_t)nRW * nHeads) {
+      const int pos = (int)(u / nHeads), w = windowOrder && !even ? windowOrder[pos] : pos;
       if ((unsigned)w < (unsigned)nRW && is_long(rowWindowOffset[w], rowWindowOffset[w + 1]))
         sList[atomicAdd(&sFound, 1)] = (int)u;
     }
@@ -144,7 +151,7 @@ f3s_fwd_mixed_kernel(const int32_t* __restrict__ windowOrder,
       const int u = uniform(sList[k / TURNS]);
       const int pos = HEADS ? u / nHeads : u;
       if constexpr (HEADS) head = u - pos * nHeads;
-      w = uniform(windowOrder ? windowOrder[pos] : pos);
+      w = uniform(windowOrder && !even ? windowOrder[pos] : pos);
       const int from = rowWindowOffset[w], to = rowWindowOffset[w + 1];
       // run r: steps [r * nSteps / RUNS, (r + 1) * nSteps / RUNS)
       const int nSteps = (to - from + BPS - 1) / BPS, r = k % TURNS * NWAVES + wave;
@@ -156,7 +163,7 @@ f3s_fwd_mixed_kernel(const int32_t* __restrict__ windowOrder,
       t1 = even ? natural1 : given1;
       if constexpr (HEADS) head = even ? natural.head : given.head;
       if ((even ? natural.pos : given.pos) >= nRW || (unsigned)w >= (unsigned)nRW) return;
-      if (!even && given.pos < longPrefix && is_long(t0, t1)) return;  // a team's
+      if (is_long(t0, t1)) return;  // a team's
       if (!fits(t0, t1)) t1 = t0;
     }
     Pipe pp;
@@ -249,7 +256,6 @@ int launch_mixed_waves(const MixedCall& c) {
   const int64_t longer = (9 * c.nTcb + 4 * (int64_t)nRW - 1) / (4 * (int64_t)nRW);
   const int maxBlocks = (int)(longer > (W8 ? 64 : 32) ? longer : (W8 ? 64 : 32));
   const int64_t longMax = c.order ? c.nTcb / (maxBlocks + 1) + 1 : nRW;
-  const int longPrefix = (int)(longMax < nRW ? longMax : nRW);
   WaveSplit split;
   split.headGroups = head_groups(D, heads);
   split.windowGroups = kXcds / split.headGroups;
@@ -264,22 +270,27 @@ int launch_mixed_waves(const MixedCall& c) {
     evenSplit.chunkShift--;
   const int64_t given = split.units(nRW), natural = evenSplit.units(nRW);
   const int64_t waveGroups = ((given > natural ? given : natural) + NWAVES - 1) / NWAVES * kXcds;
-  // a quarter of the long windows that there can be, 256 to 2048, and at least a thread for each (256, 512, 1024, 2048
-  // teams, us, d = 64: R-MAT 40 000 nodes, 12 blocks a window: 32, 36, 35, 36; 19: 41, 37, 38, 44; 169 343, 17: 93, 84, 78,
-  // 76; d = 32, 600 000, 15: 238, 222, 208, 195)
-  const int64_t units = (int64_t)longPrefix * heads;
-  int64_t teams = units / 4 < 256 ? 256 : units / 4 > 2048 ? 2048 : units / 4;
-  if (teams > units) teams = units;
-  if (teams * NWAVES * 64 < units) teams = (units + NWAVES * 64 - 1) / (NWAVES * 64);
-  teams = (teams + kXcds - 1) / kXcds * kXcds;
+  // a quarter of the long windows that there can be, 256 to 2048, and at least a thread for each unit (256, 512, 1024,
+  // 2048 teams, us, d = 64: R-MAT 40 000 nodes, 12 blocks a window: 32, 36, 35, 36; 19: 41, 37, 38, 44; 169 343, 17: 93, 84, 78,
+  // 76; d = 32, 600 000, 15: 238, 222, 208, 195). 256 of them, or a thread for each unit, where the order names no
+  // long window first (64, 128, 256, as many as ever, us: communities, 8 x 32 58.3, 58.1, 58.3, 60.1; R-MAT 169 343
+  // in a shuffled order 183, 119, 86, 68).
+  const int64_t units = (int64_t)nRW * heads;
+  const int64_t longUnits = (longMax < nRW ? longMax : nRW) * heads;
+  const auto at_least = [&](int64_t n) {
+    const int64_t look = (units + NWAVES * 64 - 1) / (NWAVES * 64);
+    return ((n > look ? n : look) + kXcds - 1) / kXcds * kXcds;
+  };
+  const int64_t teams = at_least(longUnits / 4 < 256 ? 256 : longUnits / 4 > 2048 ? 2048 : longUnits / 4);
+  const int64_t evenTeams = at_least(256);
   if (waveGroups + teams >= ((int64_t)1 << 31))
     return fail(-2, "f3s_attention: too many (window, head) units for one launch");
   auto kernel = f3s_fwd_mixed_kernel<ET, D, NWAVES, SOFTMAX, HEADS, W8, NH>;
   constexpr size_t lds = (size_t)NWAVES * pipe::Geo<D, 1>::WAVE_BYTES;
   if (int rc = allow_lds(kernel, lds)) return rc;
   hipLaunchKernelGGL(kernel, dim3((unsigned)(waveGroups + teams)), dim3(NWAVES * 64), lds, c.stream, c.order,
-                     c.rwo, c.atox, c.bitmap, split, evenSplit.chunkShift, (int)teams, longPrefix, maxBlocks, c.N,
-                     nRW, c.nTcb, static_cast<const ET*>(c.Q), static_cast<const ET*>(c.K),
+                     c.rwo, c.atox, c.bitmap, split, evenSplit.chunkShift, (int)teams, (int)evenTeams, maxBlocks,
+                     c.N, nRW, c.nTcb, static_cast<const ET*>(c.Q), static_cast<const ET*>(c.K),
                      static_cast<const ET*>(c.V), c.scaleLog2, c.out, heads, HEADS ? c.ldIn : D,
                      HEADS ? c.ldOut : D, c.sddmm);
   F3S_HIP_CHECK(hipGetLastError());

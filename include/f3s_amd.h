@@ -148,8 +148,10 @@ int f3s_preprocess(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, i
  *   rowWindowOffset [nRW+1], sparseAToXidx [nTCB*16], tcbBitMap [nTCB*4]   from preprocessing
  *   windowOrder [nRW] or NULL      launch order of the row windows, a permutation of them:
  *                                  sortedRowWindows for the heavy-first schedule, NULL for natural
- *                                  order. On a graph of short windows whose first one in the order is
- *                                  not a long one, windows start in natural order whatever it says
+ *                                  order. It is a matter of time only: rows are the same in any order.
+ *                                  On a graph of short windows the long ones start first, and where
+ *                                  the order begins with a short one, the others in natural order. An
+ *                                  entry that is no window is passed over
  *   N, nTCB, d                     nodes; TC blocks (rowWindowOffset[nRW]); head dimension: a
  *                                  multiple of 32 up to 256 (the reference takes embeddingDim
  *                                  at run time, src/F3S_kernel.cu:601-604,1424,1522)
@@ -270,7 +272,8 @@ int f3s_attention_fwd_heads(const int32_t* rowWindowOffset, const int32_t* windo
  *
  *   rowWindowOffset [nRW+1], sparseAToXidx [nTCB*8], tcbBitMap [nTCB*2]   from preprocessing
  *                                  with H = 16, W = 8
- *   windowOrder [nRW] or NULL      launch order (the reference launches in natural order)
+ *   windowOrder [nRW] or NULL      launch order, as in f3s_attention_fwd (the reference launches in
+ *                                  natural order)
  *   Q, K, V [N*d]                  fp16, row-major, contiguous; d a multiple of 32 up to 256
  *   applySoftmax                   0 = SDDMM -> SpMM only; scores are never scaled on this path
  *   out [N*d] float                fully written

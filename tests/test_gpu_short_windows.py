@@ -282,3 +282,66 @@ def test_ends_far_in_front_of_begins(heads):
     rows = rows[:N]
     assert not got[rows].any()
     assert torch.equal(got[~rows], whole[~rows])
+
+
+# A long window is a workgroup's whatever the order: its rows come out as in heavy-first order, bit for bit, where
+# the order begins with a short window, where it begins with a long one and has others at its very end, and where
+# it is natural; above d = 128 and for pairs of heads a workgroup has four runs, else eight, in one turn or two
+@pytest.mark.parametrize("heads,d", [(1, 32), (1, 64), (4, 64), (2, 128), (8, 32), (1, 160), (3, 224)])
+def test_long_windows_of_any_order(heads, d):
+    from fused3s_amd import capi
+    print("case long windows of any order %dx%d" % (heads, d), flush=True)
+    rng = np.random.default_rng(heads * d)
+    nRW = 1100
+    counts = rng.integers(0, 6, nRW)
+    counts[np.concatenate([[7, 8], np.arange(20, nRW, 83), [nRW - 1]])] = 34 + rng.integers(0, 40)
+    N, pre = _structure(rng, nRW, counts)
+    dev = lambda a: torch.as_tensor(a).cuda()
+    args = dev(pre["rowWindowOffset"]), dev(pre["sparseAToXidx"]), dev(pre["tcbBitMap"].view(np.int64)).view(torch.uint64)
+    g = torch.Generator().manual_seed(d)
+    Q, K, V = [torch.randn((N, heads, d), generator=g).to(torch.bfloat16).cuda() for _ in range(3)]
+
+    def call(order):
+        out = torch.full((N, heads * d), float("nan"), device="cuda")
+        return capi.attention_heads(args[0], dev(order.astype(np.int32)), *args[1:], N, Q, K, V, d ** 0.5, out=out)
+
+    heavy = np.argsort(-counts, kind="stable")
+    want = call(heavy)
+    assert torch.isfinite(want).all()
+    longFirst = rng.permutation(heavy[1:])
+    ends = np.concatenate([[heavy[0]], longFirst[counts[longFirst] <= 33], longFirst[counts[longFirst] > 33]])
+    orders = [np.arange(nRW), heavy[::-1], rng.permutation(heavy), ends]
+    assert [counts[o[0]] > 33 for o in orders] == [False, False, counts[orders[2][0]] > 33, True]
+    assert counts[ends[counts.sum() // 33 + 1:]].max() > 33  # beyond as many positions as can be long ones
+    for k, order in enumerate(orders):
+        assert torch.equal(call(order), want), k
+
+
+# An order that names some of the windows and is filled up with what is no window, or with one again and again: the
+# other windows' rows are left as they are, also where all windows are alike
+@pytest.mark.parametrize("fill", [-1, 1 << 30, "last"])
+@pytest.mark.parametrize("longest", [7, 60])
+def test_filled_up_orders(longest, fill):
+    from fused3s_amd import capi
+    print("case filled up orders longest=%d %s" % (longest, fill), flush=True)
+    rng = np.random.default_rng(longest)
+    nRW, heads, d = 1050, 4, 64
+    counts = 4 + rng.integers(0, 3, nRW)
+    counts[333::100] = longest
+    N, pre = _structure(rng, nRW, counts)
+    dev = lambda a: torch.as_tensor(a).cuda()
+    args = dev(pre["rowWindowOffset"]), dev(pre["sparseAToXidx"]), dev(pre["tcbBitMap"].view(np.int64)).view(torch.uint64)
+    g = torch.Generator().manual_seed(longest)
+    Q, K, V = [torch.randn((N, heads, d), generator=g).half().cuda() for _ in range(3)]
+    heavy = np.argsort(-counts, kind="stable").astype(np.int32)
+    whole = capi.attention_heads(args[0], dev(heavy), *args[1:], N, Q, K, V, 8.0)
+    some = heavy[rng.random(nRW) < 0.4]
+    order = np.full(nRW, some[-1] if fill == "last" else fill, np.int32)
+    order[:len(some)] = some
+    named = np.zeros(nRW, bool)
+    named[some] = True
+    rows = torch.as_tensor(np.repeat(named, 16)[:N]).cuda()
+    out = torch.full((N, heads * d), float("nan"), device="cuda")
+    capi.attention_heads(args[0], dev(order), *args[1:], N, Q, K, V, 8.0, out=out)
+    assert torch.equal(out[rows], whole[rows])
+    assert torch.isnan(out[~rows]).all()
