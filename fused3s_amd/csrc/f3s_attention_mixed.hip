@@ -16,18 +16,23 @@ constexpr int mixed_waves_per_simd(int d) { return d <= 32 ? 5 : d <= 64 ? 4 : d
 
 // Waves of a workgroup, four or eight. Eight compute a long window in half the time, and the longest one decides a
 // call of one or two heads on a skewed graph. A wave that has finished its own window keeps its ring until the
-// workgroup ends, which costs less with four, so those take calls of more heads and, above D = 64, large
-// ones. Eight -> four, us (heads x d, blocks a window): R-MAT 40 000 nodes, 12: 1 x 64 34 -> 38, 2 x 64 40 -> 43,
+// workgroup ends, which costs less with four, so those take calls of more heads and, above D = 64, of two, large
+// ones and those of less than 16 blocks of 16 columns a window. Eight -> four, us (heads x d, blocks a window): R-MAT 40 000 nodes, 12: 1 x 64 34 -> 38, 2 x 64 40 -> 43,
 // 4 x 64 57 -> 52, 8 x 64 100 -> 93, 4 x 128 106 -> 92; 169 343 nodes, 17: 1 x 64 76 -> 95; 200 000, 27: 1 x 64 111
 // -> 143, 1 x 128 241 -> 253, 8 x 64 1063 -> 1050; 600 000, 20: 1 x 64 294 -> 326, 1 x 128 648 -> 628; uniform
-// 25 000, 9: 1 x 64 25.7 -> 25.5, 8 x 64 70 -> 66; 30 000, 21: 1 x 128 45.7 -> 46.1, 8 x 64 128 -> 133.
+// 25 000, 9: 1 x 64 25.7 -> 25.5, 8 x 64 70 -> 66; 30 000, 21: 1 x 128 45.7 -> 46.1, 8 x 64 128 -> 133. Below 16
+// blocks, d = 128: uniform 33 000, 15: one head 40.3 -> 32.9, two 66.2 -> 58.7; communities 400 000, 14: 230 -> 209;
+// R-MAT 65 000, 9: 36.9 -> 40.2; power-law 65 000, 11: 44.5 -> 52.1 (a launch for either kind of window: 33.2, 58.5, 258,
+// 50.3, 61.7). 16x8 blocks of the same graphs, power-law 65 000, 7: 38.1 -> 46.3, where a workgroup for every
+// window takes 41.4.
 // A long window is cut into as many runs of blocks whether four or eight waves compute them, so that a head's
 // rows do not depend on how many heads the call has. At D = 32 and with two heads of 32 to a wave there are always
 // four of each: what four waves keep of the first four runs would not fit the registers there.
 constexpr int mixed_runs(int d, int nh) { return d == 32 || nh == 2 || d > 128 ? 4 : 8; }
-inline int mixed_waves(int d, int64_t nTcb16, int heads) {
+inline int mixed_waves(int d, bool w8, int nRW, int64_t nTcb16, int heads) {
   if (heads >= 3) return 4;
-  return d > 64 && nTcb16 * heads >= 500000 ? 4 : 8;
+  if (d <= 64) return 8;
+  return heads == 2 || (!w8 && nTcb16 < 16 * (int64_t)nRW) || nTcb16 >= 500000 ? 4 : 8;
 }
 
 // How the (position, head) units of a call are dealt to the XCDs: XcdSplit with one slice and with shifts in the
@@ -300,7 +305,8 @@ int launch_mixed_waves(const MixedCall& c) {
 template <typename ET, int D, bool SOFTMAX, bool HEADS, bool W8, int NH = 1>
 int launch_mixed_kernel(const MixedCall& c) {
   if constexpr (mixed_runs(D, NH) == 8) {
-    if (mixed_waves(D, W8 ? c.nTcb / 2 : c.nTcb, HEADS ? c.nHeads / NH : 1) == 8)
+    const int nRW = (c.N + kWinRows - 1) / kWinRows;
+    if (mixed_waves(D, W8, nRW, W8 ? c.nTcb / 2 : c.nTcb, HEADS ? c.nHeads / NH : 1) == 8)
       return launch_mixed_waves<ET, D, 8, SOFTMAX, HEADS, W8, NH>(c);
   }
   return launch_mixed_waves<ET, D, 4, SOFTMAX, HEADS, W8, NH>(c);
