@@ -67,13 +67,14 @@ struct WaveSplit {
 //           nodes, 17 blocks a window, longest 759, natural order given as the order: 218 us, now 86.)
 //   others  a wave takes a whole window (of one head, or of NH) that is not a long one and writes its rows from
 //           its registers.
-// Where the order's first window is not a long one, none is if the order is heavy-first: evenTeams are then
+// Where the order's first window has at most evenBlocks, all have if the order is heavy-first: evenTeams are then
 // enough to look, the other teams leave, and the waves take the windows in natural order instead of the given
 // one, 1 << evenShift in a row to an XCD. Windows that follow each other in a graph of communities name the same
 // rows, of which a heavy-first order makes as many visits as there are block counts (100 000 nodes, 6 blocks a
 // window, 8 x 32: 74 us in the given order, 58); and when the longest window is little more than twice the mean, it
-// does not matter which one starts last. An order that ends in an entry out of range, or twice in the same
-// one, names some of the windows and is filled up: it is followed as it stands.
+// does not matter which one starts last. It does where one of four times the mean is short all the same (R-MAT
+// 33 000 nodes, 7 blocks, longest 32, d = 256: 48 us, heavy-first 40). An order that ends in an entry out of range, or
+// twice in the same one, names some of the windows and is filled up: it is followed as it stands.
 // W8: 16x8 blocks, with the scores to sddmm if it is not null; maxBlocks and nTcb then count such blocks.
 template <typename ET, int D, int NWAVES, bool SOFTMAX, bool HEADS, bool W8, int NH = 1>
 __global__ __launch_bounds__(NWAVES * 64)
@@ -82,7 +83,7 @@ f3s_fwd_mixed_kernel(const int32_t* __restrict__ windowOrder,
                      const int32_t* __restrict__ rowWindowOffset,
                      const int32_t* __restrict__ sparseAToXidx,
                      const uint8_t* __restrict__ bitmapBytes, WaveSplit split, int evenShift,
-                     int teamGroups, int evenTeams, int maxBlocks, int N, int nRW, int64_t nTcb,
+                     int teamGroups, int evenTeams, int evenBlocks, int maxBlocks, int N, int nRW, int64_t nTcb,
                      const ET* __restrict__ Q, const ET* __restrict__ K, const ET* __restrict__ V,
                      float scaleLog2, float* __restrict__ out, int nHeads, int ldIn, int ldOut,
                      float* __restrict__ sddmm) {
@@ -126,7 +127,7 @@ f3s_fwd_mixed_kernel(const int32_t* __restrict__ windowOrder,
   asm volatile("" : : "s"(most), "s"(given0), "s"(given1));
   const bool filledUp =
       (unsigned)nextToLast >= (unsigned)nRW || (unsigned)lastWindow >= (unsigned)nRW || nextToLast == lastWindow;
-  const bool even = firstWindow == first && most <= maxBlocks && !filledUp;
+  const bool even = firstWindow == first && most <= evenBlocks && !filledUp;
   const int teams = even ? evenTeams : teamGroups;
   const bool team = (int)blockIdx.x < teams;
   if (even && (int)blockIdx.x >= evenTeams + waveGroups) return;
@@ -260,6 +261,7 @@ int launch_mixed_waves(const MixedCall& c) {
   // 200 000, 27: 121, 116, 109, 109, 111; d = 192 alike)
   const int64_t longer = (9 * c.nTcb + 4 * (int64_t)nRW - 1) / (4 * (int64_t)nRW);
   const int maxBlocks = (int)(longer > (W8 ? 64 : 32) ? longer : (W8 ? 64 : 32));
+  const int evenBlocks = (int)(longer > (W8 ? 32 : 16) ? longer : (W8 ? 32 : 16));
   const int64_t longMax = c.order ? c.nTcb / (maxBlocks + 1) + 1 : nRW;
   WaveSplit split;
   split.headGroups = head_groups(D, heads);
@@ -279,7 +281,8 @@ int launch_mixed_waves(const MixedCall& c) {
   // 2048 teams, us, d = 64: R-MAT 40 000 nodes, 12 blocks a window: 32, 36, 35, 36; 19: 41, 37, 38, 44; 169 343, 17: 93, 84, 78,
   // 76; d = 32, 600 000, 15: 238, 222, 208, 195). 256 of them, or a thread for each unit, where the order names no
   // long window first (64, 128, 256, as many as ever, us: communities, 8 x 32 58.3, 58.1, 58.3, 60.1; R-MAT 169 343
-  // in a shuffled order 183, 119, 86, 68).
+  // in a shuffled order 183, 119, 86, 68), and half as many above D = 128, where they would keep every CU from its
+  // first waves (R-MAT 100 000, 25 blocks, d = 160, shuffled: 191, 192, 192, 189).
   const int64_t units = (int64_t)nRW * heads;
   const int64_t longUnits = (longMax < nRW ? longMax : nRW) * heads;
   const auto at_least = [&](int64_t n) {
@@ -287,15 +290,15 @@ int launch_mixed_waves(const MixedCall& c) {
     return ((n > look ? n : look) + kXcds - 1) / kXcds * kXcds;
   };
   const int64_t teams = at_least(longUnits / 4 < 256 ? 256 : longUnits / 4 > 2048 ? 2048 : longUnits / 4);
-  const int64_t evenTeams = at_least(256);
+  const int64_t evenTeams = at_least(D > 128 ? 128 : 256);
   if (waveGroups + teams >= ((int64_t)1 << 31))
     return fail(-2, "f3s_attention: too many (window, head) units for one launch");
   auto kernel = f3s_fwd_mixed_kernel<ET, D, NWAVES, SOFTMAX, HEADS, W8, NH>;
   constexpr size_t lds = (size_t)NWAVES * pipe::Geo<D, 1>::WAVE_BYTES;
   if (int rc = allow_lds(kernel, lds)) return rc;
   hipLaunchKernelGGL(kernel, dim3((unsigned)(waveGroups + teams)), dim3(NWAVES * 64), lds, c.stream, c.order,
-                     c.rwo, c.atox, c.bitmap, split, evenSplit.chunkShift, (int)teams, (int)evenTeams, maxBlocks,
-                     c.N, nRW, c.nTcb, static_cast<const ET*>(c.Q), static_cast<const ET*>(c.K),
+                     c.rwo, c.atox, c.bitmap, split, evenSplit.chunkShift, (int)teams, (int)evenTeams, evenBlocks,
+                     maxBlocks, c.N, nRW, c.nTcb, static_cast<const ET*>(c.Q), static_cast<const ET*>(c.K),
                      static_cast<const ET*>(c.V), c.scaleLog2, c.out, heads, HEADS ? c.ldIn : D,
                      HEADS ? c.ldOut : D, c.sddmm);
   F3S_HIP_CHECK(hipGetLastError());
