@@ -10,9 +10,15 @@
 namespace f3s {
 namespace {
 
-// Waves per SIMD the register allocator is held to: as many as the rings (one stage each) leave room for in a
-// CU's LDS, 16 at D = 64, eight up to D = 128, four above; and 20 at D = 32, where 24 would spill registers.
-constexpr int mixed_waves_per_simd(int d) { return d <= 32 ? 5 : d <= 64 ? 4 : d <= 128 ? 2 : 1; }
+// Stages of a wave's LDS ring, and waves per SIMD the register allocator is held to: as many as the rings leave room
+// for in a CU's LDS, 16 up to D = 64, eight up to D = 128, four above. Two stages fit 16 waves at D = 32, where 20
+// of one stage leave a long window's four waves waiting for every step's rows. One head, d = 32, 20 waves of one
+// stage -> 16 of two (a launch for each kind of window), us; nodes, blocks a window: power-law 110 000, 15 49 -> 41
+// (47), 200 000, 7 69 -> 55 (64), 11 81 -> 67 (74); R-MAT 46 000, 12 20 -> 17 (24), 200 000, 13 66 -> 54 (64), 600 000, 15 220
+// -> 187 (221); communities 200 000, 9 28 -> 27 (35); uniform 110 000, 11 34 -> 36 (36), 15 42 -> 46 (43); three heads of
+// 200 000 nodes, power-law, 11 142 -> 130 (151), R-MAT, 9 93 -> 97 (108), uniform, 11 171 -> 172 (171).
+constexpr int mixed_stages(int d) { return d == 32 ? 2 : 1; }
+constexpr int mixed_waves_per_simd(int d) { return d <= 64 ? 4 : d <= 128 ? 2 : 1; }
 
 // Waves of a workgroup, four or eight. Eight compute a long window in half the time, and the longest one decides a
 // call of one or two heads on a skewed graph. A wave that has finished its own window keeps its ring until the
@@ -26,8 +32,9 @@ constexpr int mixed_waves_per_simd(int d) { return d <= 32 ? 5 : d <= 64 ? 4 : d
 // 50.3, 61.7). 16x8 blocks of the same graphs, power-law 65 000, 7: 38.1 -> 46.3, where a workgroup for every
 // window takes 41.4.
 // A long window is cut into as many runs of blocks whether four or eight waves compute them, so that a head's
-// rows do not depend on how many heads the call has. At D = 32 and with two heads of 32 to a wave there are always
-// four of each: what four waves keep of the first four runs would not fit the registers there.
+// rows do not depend on how many heads the call has. With two heads of 32 to a wave there are always four of
+// each, as what four waves keep of the first four runs would not fit the registers there, and so at D = 32, whose
+// rows are those of the pairs.
 constexpr int mixed_runs(int d, int nh) { return d == 32 || nh == 2 || d > 128 ? 4 : 8; }
 inline int mixed_waves(int d, bool w8, int nRW, int64_t nTcb16, int heads) {
   if (heads >= 3) return 4;
@@ -87,8 +94,8 @@ f3s_fwd_mixed_kernel(const int32_t* __restrict__ windowOrder,
                      const ET* __restrict__ Q, const ET* __restrict__ K, const ET* __restrict__ V,
                      float scaleLog2, float* __restrict__ out, int nHeads, int ldIn, int ldOut,
                      float* __restrict__ sddmm) {
-  constexpr int WAVE_BYTES = pipe::Geo<D, 1>::WAVE_BYTES;
-  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, W8, 1, false, NH> Pipe;
+  constexpr int WAVE_BYTES = pipe::Geo<D, mixed_stages(D)>::WAVE_BYTES;
+  typedef pipe::PairPipeline<ET, D, SOFTMAX, HEADS, W8, mixed_stages(D), false, NH> Pipe;
   constexpr int TH = D / NH / 16;
   constexpr int BPS = W8 ? 4 : 2;  // blocks of the structure per step
   // four waves take eight runs in two turns
@@ -294,7 +301,7 @@ int launch_mixed_waves(const MixedCall& c) {
   if (waveGroups + teams >= ((int64_t)1 << 31))
     return fail(-2, "f3s_attention: too many (window, head) units for one launch");
   auto kernel = f3s_fwd_mixed_kernel<ET, D, NWAVES, SOFTMAX, HEADS, W8, NH>;
-  constexpr size_t lds = (size_t)NWAVES * pipe::Geo<D, 1>::WAVE_BYTES;
+  constexpr size_t lds = (size_t)NWAVES * pipe::Geo<D, mixed_stages(D)>::WAVE_BYTES;
   if (int rc = allow_lds(kernel, lds)) return rc;
   hipLaunchKernelGGL(kernel, dim3((unsigned)(waveGroups + teams)), dim3(NWAVES * 64), lds, c.stream, c.order,
                      c.rwo, c.atox, c.bitmap, split, evenSplit.chunkShift, (int)teams, (int)evenTeams, evenBlocks,
