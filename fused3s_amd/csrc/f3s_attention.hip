@@ -16,10 +16,10 @@ using window::HeadLayout;
 
 
 // Whether a call goes to f3s_attention_mixed.hip. F3S_SHORT_WINDOWS=0 in the environment turns it off.
-bool short_windows(const int32_t* windowOrder, int nRW, int64_t nTcb16, int d, int nHeads) {
+bool short_windows(const int32_t* windowOrder, int nRW, int64_t nTcb16, int d, int nHeads, bool w8) {
   const char* e = getenv("F3S_SHORT_WINDOWS");  // read per call, like every other switch
   if (e && strcmp(e, "0") == 0) return false;
-  return mixed_windows_pay(windowOrder != nullptr, nRW, nTcb16, d, nHeads);
+  return mixed_windows_pay(windowOrder != nullptr, nRW, nTcb16, d, nHeads, w8);
 }
 
 // The column-sliced schedule (f3s_attention_units.hip: (window, column slice) units, every XCD
@@ -100,7 +100,7 @@ int launch_attention(const int32_t* rowWindowOffset, const int32_t* windowOrder,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, 0, d, d, prepared ? 2 : 0, stream);
   const int nRWi = (N + kWinRows - 1) / kWinRows;
-  if (!cuTimer && short_windows(windowOrder, nRWi, nTcb, d, 0))
+  if (!cuTimer && short_windows(windowOrder, nRWi, nTcb, d, 0, false))
     return launch_attention_mixed(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q, K, V,
                                   scaleLog2, applySoftmax, out, 0, d, d, nTcb, stream);
   const HeadLayout single = {0, d, d, nTcb};
@@ -138,7 +138,7 @@ int launch_attention_tcb8(const int32_t* rowWindowOffset, const int32_t* windowO
     return launch_tcb8_wide(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, Q, K, V,
                             scaleLog2, applySoftmax, out, sddmm, nTcb8, stream);
   // (at d = 32 the window kernel is the faster one: R-MAT, 150 000 nodes, 15 blocks of 16 a window: 72 against 81 us)
-  if (d > 32 && short_windows(windowOrder, (N + kWinRows - 1) / kWinRows, nTcb8 / 2, d, 0))
+  if (d > 32 && short_windows(windowOrder, (N + kWinRows - 1) / kWinRows, nTcb8 / 2, d, 0, true))
     return launch_tcb8_mixed(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, Q, K, V, scaleLog2,
                              applySoftmax, out, sddmm, nTcb8, stream);
 #define F3S_DISPATCH(DD)                                                                      \
@@ -190,7 +190,7 @@ int launch_attention_heads(const int32_t* rowWindowOffset, const int32_t* window
     return launch_attention_sliced(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, nHeads, (int)ldIn, (int)ldOut, prepared ? 2 : 0, stream);
-  if (short_windows(windowOrder, (int)nRW, nTcb, d, nHeads))
+  if (short_windows(windowOrder, (int)nRW, nTcb, d, nHeads, false))
     return launch_attention_mixed(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q, K, V,
                                   scaleLog2, applySoftmax, out, nHeads, (int)ldIn, (int)ldOut, nTcb,
                                   stream);

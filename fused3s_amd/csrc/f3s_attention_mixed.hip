@@ -334,30 +334,51 @@ int launch_mixed_d(const MixedCall& c) {
 
 }  // namespace
 
-// Where this kernel takes a call (nTcb16: blocks of 16 columns). Against a workgroup of four waves for every
-// window, us, one head, with an order; nodes, blocks a window:
-// - d = 64: R-MAT 40 000, 12 38 -> 33, 19 46 -> 38; 60 000, 28 66 -> 57; 200 000, 17 97 -> 84, 27 132 -> 111; 600 000, 13
-//   259 -> 208; uniform 30 000, 21 34 -> 30, 60 000, 60 106 -> 76; but power-law 20 000, 46 35 -> 41; 50 000, 47 57 ->
-//   68, 100 000, 57 119 -> 120. 96 and 128 alike (d = 128: R-MAT 60 000, 28 90 -> 78; 600 000, 13 536 -> 450; uniform 30 000,
-//   21 56 -> 44; power-law 20 000, 46 49 -> 62; 100 000, 57 262 -> 257). Nothing on the host tells uniform from
-//   power-law graphs, which is why these stop at 32 blocks.
-// - d > 128, where four waves were all that a CU held and a window's last step kept three of them waiting: d = 192, R-MAT
-//   40 000, 12 86 -> 63; 200 000, 27 521 -> 400; uniform 60 000, 60 (d = 224) 443 -> 273; power-law 20 000, 46 90 -> 91;
-//   60 000, 52 257 -> 213; 180 000, 48 762 -> 644.
-// - d = 32, where four workgroups of four waves fit a CU, two stages each: R-MAT 40 000, 12 30 -> 30; 600 000, 13 190 -> 166;
-//   but 200 000, 17 76 -> 79, 27 103 -> 106. Pairs of 32-wide heads are 64 wide (4 x 32: R-MAT 200 000, 27 230 -> 204;
-//   power-law 20 000, 46 50 -> 73).
-// - several heads: R-MAT 200 000, 17 4 x 64 388 -> 319, 4 x 128 812 -> 732; uniform 30 000, 21 8 x 64 138 -> 133, 4 x 128 166 ->
-//   136; power-law 20 000, 46 2 x 64 48 -> 58, 8 x 64 138 -> 135.
-// - K + V of 1 GiB and more, which come from HBM as fast as it gives them: R-MAT 2 449 029, 25, d = 128 4428 -> 4398.
+// Where this kernel takes a call (nTcb16: blocks of 16 columns; w8: of a structure of 16x8 blocks). Against a workgroup
+// of four waves for every window, us, with an order, one head unless heads are given; nodes, blocks a window:
+// - blocks of 16 columns, less than 16 a window, d <= 128: here. Communities 200 000, 14 d = 64 97 -> 57, d = 32 61 -> 32;
+//   uniform 65 000, 7 d = 64 21 -> 19; R-MAT 110 000, 9 d = 128 68 -> 64; power-law 110 000, 15 d = 32 37 -> 41.
+// - more of them and 16x8 blocks, d = 64 to 128: up to 32 a window, and where windows times heads (or pairs of 32-wide
+//   heads) are 11/8 of the waves that fit the chip at a time. Below that line a window that one wave computes
+//   lasts longer than all of the rest. d = 64, 5 632 of them: power-law 24 000, 16 15 -> 21, 27 18 -> 29; 46 000, 28 28 -> 32;
+//   72 000, 27 42 -> 47; flat R-MAT 24 000, 28 15 -> 27; 72 000, 28 44 -> 48; but R-MAT 46 000, 17 30 -> 24; 72 000, 17 38 -> 31;
+//   uniform 46 000, 17 27 -> 25. Beyond: power-law 90 000, 17 44 -> 41, 27 55 -> 54, 30 57 -> 58; 200 000, 28 132 -> 127; flat
+//   R-MAT 90 000, 28 57 -> 57; R-MAT 90 000, 18 47 -> 37; 200 000, 31 132 -> 105; uniform 90 000, 28 81 -> 70. d = 128, 2 816:
+//   power-law 24 000, 27 29 -> 45; 33 000, 17 30 -> 34; but R-MAT 33 000, 16 33 -> 31. Beyond: power-law 48 000, 17 43 -> 42,
+//   27 57 -> 59; 200 000, 28 296 -> 287; uniform 200 000, 18 247 -> 254; 90 000, 28 177 -> 151; R-MAT 48 000, 26 59 -> 50.
+//   16x8 blocks of the same graphs: d = 64, power-law 24 000, 7 13 -> 19; 110 000, 7 42 -> 35, 28 68 -> 72. Three heads and
+//   more have workgroups of four waves here, which end sooner: all the waves that fit are enough (4 x 64: power-law
+//   17 000, 16 28 -> 22, 27 36 -> 30; flat R-MAT 17 000, 28 35 -> 31). Nothing on the host tells uniform from power-law
+//   graphs, which is why these stop at 32 blocks (power-law 20 000, 46 35 -> 41; 50 000, 47 57 -> 68; 100 000, 57 119 ->
+//   120; but uniform 60 000, 60 106 -> 76).
+// - the same at d = 32: pairs of heads, which are 64 wide, from two on (4 x 32: power-law 45 000, 17 39 -> 32; R-MAT 45 000, 29
+//   48 -> 51; 110 000, 18 92 -> 73). One pair takes longer than window by window head for head (2 x 32: power-law 110 000, 17 53
+//   -> 62; R-MAT 110 000, 26 70 -> 75; 33 000, 22 1.35 times), and so do single heads.
+// - d > 128, where four waves were all that a CU held and a window's last step kept three of them waiting: up to 64
+//   blocks a window. d = 192, R-MAT 40 000, 12 86 -> 63; 200 000, 27 521 -> 400; uniform 60 000, 60 (d = 224) 443 -> 273;
+//   power-law 20 000, 46 90 -> 91; 60 000, 52 257 -> 213; 180 000, 48 762 -> 644. From 16 blocks on not the few windows above
+//   d = 192 (1 025 windows, d = 256: power-law 54 blocks 74 -> 83, R-MAT 25 45 -> 47; 1 250: power-law 55 95 -> 96).
+// - K + V of 1 GiB and more, which come from HBM as fast as it gives them, window by window: R-MAT 2 449 029, 25, d = 128
+//   4398 against 4428.
 // - without an order, on graphs of more windows than f3s_window_order takes: d = 192, flat R-MAT 1 000 000, 26 3300 -> 2820,
 //   R-MAT 800 000, 15 2000 -> 1533, uniform 300 000, 17 670 -> 576; but d = 64, R-MAT 800 000, 15 466 -> 344, flat 300 000,
 //   18 184 -> 195, 1 000 000, 26 904 -> 926, uniform 197 -> 204, d = 128 900 -> 729, 369 -> 394, 1780 -> 1820, 377 -> 388.
-bool mixed_windows_pay(bool ordered, int nRW, int64_t nTcb16, int d, int nHeads) {
-  const int most = d > 128 ? 64 : d > 32 || heads_in_pairs(d, nHeads) ? 32 : 16;
-  if (nRW < 1024 || nTcb16 >= (int64_t)most * nRW) return false;
-  if (d > 128) return ordered || nRW > 16384;
-  return ordered && (int64_t)nRW * kWinRows * d * (nHeads > 0 ? nHeads : 1) * 4 < (int64_t)1 << 30;
+bool mixed_windows_pay(bool ordered, int nRW, int64_t nTcb16, int d, int nHeads, bool w8) {
+  if (nRW < 1024) return false;
+  const int heads = nHeads > 0 ? nHeads : 1;
+  const bool pairs = heads_in_pairs(d, nHeads);
+  const int64_t units = (int64_t)nRW * (pairs ? heads / 2 : heads);
+  const bool below16 = nTcb16 < 16 * (int64_t)nRW;
+  if (d > 128) {
+    if (d > 192 && !below16 && units < 1200) return false;
+    return nTcb16 < 64 * (int64_t)nRW && (ordered || nRW > 16384);
+  }
+  if (!ordered || (int64_t)nRW * kWinRows * d * heads * 4 >= (int64_t)1 << 30) return false;
+  if (below16 && !w8) return true;
+  if (d == 32 && !(pairs && heads >= 4)) return false;
+  const int64_t fit = 256 * 4 * mixed_waves_per_simd(d);
+  const bool fourWaves = (pairs ? heads / 2 : heads) >= 3;
+  return nTcb16 < 32 * (int64_t)nRW && units >= (fourWaves ? fit : fit * 11 / 8);
 }
 
 int launch_attention_mixed(const int32_t* rowWindowOffset, const int32_t* windowOrder,

@@ -100,7 +100,7 @@ int launch_attention_sliced(const int32_t* rowWindowOffset, const int32_t* windo
 
 // graphs of short windows (f3s_attention_mixed.hip): a wave per window, workgroups for the long ones
 // nHeads = 0: contiguous single head; windowOrder may be null; nTcb16: blocks of 16 columns
-bool mixed_windows_pay(bool ordered, int nRW, int64_t nTcb16, int d, int nHeads);
+bool mixed_windows_pay(bool ordered, int nRW, int64_t nTcb16, int d, int nHeads, bool w8);
 int launch_attention_mixed(const int32_t* rowWindowOffset, const int32_t* windowOrder,
                            const int32_t* sparseAToXidx, const uint64_t* bitmap, int N, int d, int dtype,
                            const void* Q, const void* K, const void* V, float scaleLog2,

@@ -345,3 +345,41 @@ def test_filled_up_orders(longest, fill):
     capi.attention_heads(args[0], dev(order), *args[1:], N, Q, K, V, 8.0, out=out)
     assert torch.equal(out[rows], whole[rows])
     assert torch.isnan(out[~rows]).all()
+
+
+# From 16 blocks a window on, and with 16x8 blocks, what takes a call depends on windows times heads: one window fewer
+# than the line and the call is the workgroup-per-window kernel's, bit for bit; at the line it is not, and its rows
+# are the same to the rounding of 16-bit probabilities. One pair of 32-wide heads and single ones have no such line.
+@pytest.mark.parametrize("heads,d,W,line", [
+    (1, 64, 16, 5632), (2, 64, 16, 2816), (3, 64, 16, 1366), (1, 96, 16, 2816), (1, 128, 16, 2816), (2, 128, 16, 1408),
+    (4, 32, 16, 2816), (6, 32, 16, 1366), (2, 32, 16, None), (1, 32, 16, None), (1, 256, 16, 1200), (1, 64, 8, 5632),
+    (1, 96, 8, 2816), (1, 128, 8, 2816)])
+def test_line_in_windows_and_heads(monkeypatch, heads, d, W, line):
+    from fused3s_amd import capi
+    print("case line in windows and heads %dx%d W=%d" % (heads, d, W), flush=True)
+    for nRW, mixed in [(6000, False)] if line is None else [(line - 1, False), (line, True)]:
+        rng = np.random.default_rng(nRW)
+        counts = 16 + rng.integers(0, 3, nRW)
+        counts[5::97] = 70 + rng.integers(0, 9)
+        rwo = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+        N = 16 * nRW - 3
+        step = N // (W * int(counts.max()))
+        atox = np.concatenate([np.arange(W * c) * step for c in counts])
+        atox = (atox + rng.integers(0, step, len(atox))).astype(np.int32)
+        bitmap = rng.integers(0, 2**63, len(atox) // 4, dtype=np.uint64)
+        bitmap &= rng.integers(0, 2**63, len(bitmap), dtype=np.uint64)
+        dev = lambda a: torch.as_tensor(a).cuda()
+        args = [dev(rwo), dev(np.argsort(-counts, kind="stable").astype(np.int32)), dev(atox),
+                dev(bitmap.view(np.int64)).view(torch.uint64), N]
+        g = torch.Generator().manual_seed(d)
+        args += [(torch.randn((N, heads, d), generator=g) * d ** -0.25).half().cuda() for _ in range(3)]
+        if W == 8:
+            args[5:] = [t[:, 0].contiguous() for t in args[5:]]
+        call = capi.attention_tcb8 if W == 8 else capi.attention_heads
+        got = call(*args)
+        monkeypatch.setenv("F3S_SHORT_WINDOWS", "0")
+        want = call(*args)
+        monkeypatch.delenv("F3S_SHORT_WINDOWS")
+        assert torch.equal(got, want) != mixed, nRW
+        assert (got - want).abs().max().item() < MAX_ABS
+        assert ((got - want).abs().mean() / want.abs().mean()).item() < MEAN_REL[torch.float16]
