@@ -224,25 +224,21 @@ std::vector<torch::Tensor> timed_launch(const char* what, const torch::Tensor& o
 // are shared out between single waves and workgroups (which needs an order). Neither the
 // number of windows nor of blocks says how skewed a graph is, so the lines are where no measured
 // graph lost more than 3 % (natural -> own order, in us):
-// - windows below 32 blocks of 16 columns on average, 1024 to 8192 of them, d = 64 to 128, from 64M products of
-//   block columns and d: d = 64, R-MAT 60k nodes, 28 blocks 84 -> 62, 100k, 12 63 -> 55; flatter R-MAT 100k, 20
-//   70 -> 72; below, 24k, 19 38 -> 45, uniform 20k, 20 29 -> 34; above 8192 windows, flatter R-MAT 200k, 12 95 -> 104,
-//   but R-MAT 250k, 31 197 -> 164. d = 128: R-MAT 40k, 19 64 -> 58, 60k, 28 128 -> 88, flatter 100k, 20 132 -> 127,
-//   14 104 -> 107, uniform 30k, 21 58 -> 51; 24k, 19 48 -> 53; 200k, 12 178 -> 186.
-//   d > 128, from 32M products and for any number of windows: d = 192, R-MAT 24k, 19 90 -> 71, 150k, 25 468 -> 303,
-//   flatter 100k, 20 272 -> 197, uniform 20k, 20 70 -> 66.
+// - d > 128, windows below 32 blocks of 16 columns on average, from 1024 windows and 32M products of block columns and
+//   d: d = 192, R-MAT 24k nodes, 19 blocks 90 -> 71, 150k, 25 468 -> 303, flatter 100k, 20 272 -> 197, uniform 20k, 14
+//   58 -> 57, 40k, 14 100 -> 84, power-law 20k, 9 61 -> 47, communities 20k, 7 48 -> 46.
 // - longer windows of 16 columns (50k nodes, 4.1M edges, d = 96: 192 -> 148; 180k nodes, 40M edges,
 //   d = 64: 842 -> 647), from 1024 windows and 128M products (35k nodes, 3M edges, d = 64, 192M: 106 -> 92;
-//   12k nodes, 3M edges, 750 windows: 49 -> 50); at d = 32 windows of 32 blocks and more only.
-// - blocks of 8 columns, by a workgroup per window: from 64M products (R-MAT, 65k nodes, d = 128:
-//   122 -> 90; 149k nodes, d = 64: 137 -> 105; below, 24k nodes, d = 128: 53 -> 55).
+//   12k nodes, 3M edges, 750 windows: 49 -> 50). Not shorter ones up to d = 128, which gain where they are skewed (d = 64,
+//   R-MAT 60k, 28 84 -> 62; d = 128, 60k, 28 128 -> 88) and lose where they are not: uniform 70k, 19 d = 64 60 -> 66, d = 128 107
+//   -> 116, 120k, 14 d = 64 76 -> 85; 70k, 14 d = 96 81 -> 87; flatter R-MAT 70k, 29 d = 64 64 -> 71.
+// - blocks of 8 columns: from 64M products (R-MAT, 65k nodes, d = 128: 122 -> 90; 149k nodes, d = 64: 137 -> 105;
+//   below, 24k nodes, d = 128: 53 -> 55).
 bool order_pays(int64_t nRW, int64_t nTCB, int W, int64_t d) {
   if (nRW > 16384) return false;  // more than f3s_window_order takes
   const int64_t products = nTCB * W * d;
-  const bool shortWindows = nRW >= 1024 && nTCB * W < 16 * 32 * nRW;
-  if (shortWindows && d > 128) return products >= (32ll << 20);
+  if (d > 128 && nRW >= 1024 && nTCB * W < 16 * 32 * nRW) return products >= (32ll << 20);
   if (W == 8) return products >= (64ll << 20);
-  if (shortWindows) return d > 32 && nRW <= 8192 && products >= (64ll << 20);
   return nRW >= 1024 && nTCB >= 32 * nRW && products >= (128ll << 20);
 }
 

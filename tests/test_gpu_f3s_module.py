@@ -288,3 +288,30 @@ def test_calls_without_a_window_order(oracle_mod, W, edges, ordered):
             p = np.exp(s - s.max())
             want = (p / p.sum()) @ Vh[c]
         np.testing.assert_allclose(out[r].cpu().numpy(), want, atol=MAX_ABS, rtol=1e-2)
+
+
+# Calls without an order on graphs of short windows: up to d = 128 they are computed window by window as they stand,
+# above it in an order of their own (from 32M products of block columns and d on)
+@pytest.mark.parametrize("d,nRW,ordered", [(64, 5700, False), (128, 2900, False), (160, 2900, True), (160, 700, False)])
+def test_short_windows_without_a_window_order(d, nRW, ordered):
+    from fused3s_amd import F3S, capi
+    print("case short windows without an order d=%d" % d, flush=True)
+    rng = np.random.default_rng(d)
+    N = 16 * nRW - 5
+    counts = 17 + rng.integers(0, 4, nRW)
+    counts[nRW // 2::211] = 70
+    assert (int(counts.sum()) * 16 * d >= (64 if d <= 128 else 32) << 20) == (nRW > 1024)
+    step = N // (16 * 70)
+    atox = np.concatenate([np.arange(16 * c) * step for c in counts])
+    atox = torch.as_tensor((atox + rng.integers(0, step, len(atox))).astype(np.int32)).cuda()
+    rwo = torch.as_tensor(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)).cuda()
+    bits = rng.integers(0, 2**63, len(atox) // 4) & rng.integers(0, 2**63, len(atox) // 4)
+    bm = torch.as_tensor(bits).cuda().view(torch.uint64)
+    order = torch.as_tensor(np.argsort(-counts, kind="stable").astype(np.int32)).cuda()
+    Q, K, V = (torch.rand((N, d), device="cuda", generator=torch.Generator("cuda").manual_seed(i))
+               .half() for i in range(3))
+    got = F3S.f3s_1tb1rw(rwo, atox, bm, N, Q, K, V, 8, True, False)[1]
+    natural = capi.attention(rwo, None, atox, bm, N, Q, K, V)
+    heavy = capi.attention(rwo, order, atox, bm, N, Q, K, V)
+    assert torch.equal(got, heavy if ordered else natural)
+    assert (nRW < 1024) == torch.equal(natural, heavy)  # other sums, other rounding
