@@ -100,7 +100,9 @@ int launch_attention(const int32_t* rowWindowOffset, const int32_t* windowOrder,
                                    Q, K, V, scaleLog2, applySoftmax, out, workspace, wsBytes,
                                    nTcb, 0, d, d, prepared ? 2 : 0, stream);
   const int nRWi = (N + kWinRows - 1) / kWinRows;
-  if (!cuTimer && short_windows(windowOrder, nRWi, nTcb, d, 0, false))
+  // the timed form is the window kernel's, and from 16 blocks a window on so is the one that draws windows from a cursor
+  const bool cursor = window::window_cursor_requested() && nTcb >= 16 * (int64_t)nRWi;
+  if (!cuTimer && !cursor && short_windows(windowOrder, nRWi, nTcb, d, 0, false))
     return launch_attention_mixed(rowWindowOffset, windowOrder, sparseAToXidx, bitmap, N, d, dtype, Q, K, V,
                                   scaleLog2, applySoftmax, out, 0, d, d, nTcb, stream);
   const HeadLayout single = {0, d, d, nTcb};

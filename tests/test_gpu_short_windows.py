@@ -383,3 +383,27 @@ def test_line_in_windows_and_heads(monkeypatch, heads, d, W, line):
         assert torch.equal(got, want) != mixed, nRW
         assert (got - want).abs().max().item() < MAX_ABS
         assert ((got - want).abs().mean() / want.abs().mean()).item() < MEAN_REL[torch.float16]
+
+
+# F3S_WINDOW_PERSISTENT=1 asks for the cursor form of the workgroup-per-window kernel, also where an ordered call of
+# 16 blocks a window and more would go to the kernel for short windows
+@pytest.mark.parametrize("d,nRW", [(64, 5700), (160, 1100)])
+def test_cursor_form_is_asked_for(monkeypatch, d, nRW):
+    from fused3s_amd import capi
+    print("case cursor form d=%d" % d, flush=True)
+    rng = np.random.default_rng(d)
+    counts = 16 + rng.integers(0, 5, nRW)
+    counts[11::300] = 65
+    N, pre = _structure(rng, nRW, counts)
+    dev = lambda a: torch.as_tensor(a).cuda()
+    args = [dev(pre["rowWindowOffset"]), dev(np.argsort(-counts, kind="stable").astype(np.int32)),
+            dev(pre["sparseAToXidx"]), dev(pre["tcbBitMap"].view(np.int64)).view(torch.uint64), N]
+    g = torch.Generator().manual_seed(d)
+    args += [torch.randn((N, d), generator=g).half().cuda() for _ in range(3)]
+    plain = capi.attention(*args, 8.0)
+    monkeypatch.setenv("F3S_WINDOW_PERSISTENT", "1")
+    cursor = capi.attention(*args, 8.0)
+    monkeypatch.setenv("F3S_WINDOW_PERSISTENT", "0")
+    monkeypatch.setenv("F3S_SHORT_WINDOWS", "0")
+    windows = capi.attention(*args, 8.0)
+    assert torch.equal(cursor, windows) and not torch.equal(plain, windows)
