@@ -234,9 +234,8 @@ def run_config(name, args, dev, headline):
         # the schedule's index depends on the structure only: built once, like the structure
         capi.attention_prepare(pre["rowWindowOffset"], pre["sparseAToXidx"], N, d,
                                workspace, heads=0 if heads == 1 else heads)
-    schedule = "column-sliced" if workspace is not None else "window"
-    log("attention schedule: %s" % ("column-sliced (%.0f MB workspace)" % (workspace.numel() / 1e6)
-                                    if workspace is not None else "workgroup per window"))
+    if workspace is not None:
+        log("attention schedule: column-sliced (%.0f MB workspace)" % (workspace.numel() / 1e6))
 
     layout = getattr(args, "kv_layout", "") if headline else ""
     if heads == 1 and layout:
@@ -310,6 +309,21 @@ def run_config(name, args, dev, headline):
     torch.cuda.synchronize()
     has = (deg > 0).unsqueeze(1).to(o1.dtype)
     rowsum_err = float((o1 - has).abs().max())
+    # which kernel that was: with F3S_SHORT_WINDOWS=0 every window has a workgroup, and rows that single waves
+    # computed come out with other last bits
+    schedule = "column-sliced"
+    if workspace is None:
+        switch = os.environ.get("F3S_SHORT_WINDOWS")
+        os.environ["F3S_SHORT_WINDOWS"] = "0"
+        step(V, o1)
+        torch.cuda.synchronize()
+        if switch is None:
+            del os.environ["F3S_SHORT_WINDOWS"]
+        else:
+            os.environ["F3S_SHORT_WINDOWS"] = switch
+        schedule = "window" if torch.equal(out, o1) else "mixed"
+        log("attention schedule: %s" % ("workgroup per window" if schedule == "window"
+                                        else "waves for short windows, workgroups for long ones"))
     del ones, o1
     sanity = {"finite": finite, "rowsum_max_err": rowsum_err, "ok": finite and rowsum_err < 2e-3}
 
