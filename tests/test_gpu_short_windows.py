@@ -1,7 +1,7 @@
 """Graphs of short windows: one launch computes the short windows by waves and the long ones by
 workgroups. Checked against the reference-emulating oracle for fp16 and bf16, single head and
-multi-head, with the heavy-first order, a shuffled order (a long window may then lie outside the
-workgroups' share) and natural order (a workgroup for every window)."""
+multi-head, with the heavy-first order, a shuffled order (where its first window is short, the short ones
+are then taken in natural order) and without an order (a workgroup for every window)."""
 import numpy as np
 import pytest
 import torch
@@ -163,9 +163,10 @@ def test_many_long_units_per_workgroup(oracle_mod):
 
 # A wave per window and a workgroup per long one, at the edges of what decides between them: windows all alike (the
 # waves then go by window number), one window just long or just not (32 blocks, or 9/4 of the mean), means on both
-# sides of 16 and 32 blocks; four and eight waves to a workgroup, all of a head dimension's forms; 1 024 windows,
+# sides of 16 and 32 blocks (of those above 16 the fewest windows are a workgroup's each up to d = 128 with less than
+# three heads); four and eight waves to a workgroup, all of a head dimension's forms; 1 024 windows,
 # the fewest, and a last one of a single row. Every row is compared with the oracle (fp32 sums of 16-bit
-# probabilities), orders with each other in the places of the rows.
+# probabilities), in heavy-first and in shuffled order.
 def _structure(rng, nRW, counts):
     N = 16 * nRW - 15
     rwo = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
@@ -221,15 +222,15 @@ def test_waves_and_teams(oracle_mod, kind, heads, d, dtype):
             assert np.abs(gh - want).mean() / np.abs(want).mean() < MEAN_REL[dtype]
 
 
-@pytest.mark.parametrize("d", [64, 128, 160])
+@pytest.mark.parametrize("d,nRW", [(64, 5632), (64, 1030), (128, 2816), (128, 1030), (160, 1030)])
 @pytest.mark.parametrize("longest", [9, 65])
-def test_waves_and_teams_of_narrow_blocks(oracle_mod, longest, d):
+def test_waves_and_teams_of_narrow_blocks(oracle_mod, longest, d, nRW):
     """16x8 blocks with their scores: odd block counts, so that windows and their shared runs end inside a
-    step; `longest` 9: windows all alike, 65: one window of one block more than a wave takes."""
+    step; `longest` 9: windows all alike, 65: one window of one block more than a wave takes. Up to d = 128
+    1030 windows are a workgroup's each."""
     from fused3s_amd import capi
-    print("case waves and teams 16x8 longest=%d d=%d" % (longest, d), flush=True)
+    print("case waves and teams 16x8 longest=%d d=%d windows=%d" % (longest, d, nRW), flush=True)
     rng = np.random.default_rng(d + longest)
-    nRW = 1030
     counts = rng.integers(0, 10, nRW)
     counts[5::400] = longest
     N = 16 * nRW - 3
@@ -407,3 +408,64 @@ def test_cursor_form_is_asked_for(monkeypatch, d, nRW):
     monkeypatch.setenv("F3S_SHORT_WINDOWS", "0")
     windows = capi.attention(*args, 8.0)
     assert torch.equal(cursor, windows) and not torch.equal(plain, windows)
+
+
+# Calls without an order above d = 128 on more windows than an order is made for: the workgroups look for long windows
+# in natural order. The rows are those of a call in heavy-first order.
+@pytest.mark.parametrize("heads,d", [(1, 160), (2, 256)])
+def test_many_windows_without_an_order(heads, d):
+    from fused3s_amd import capi
+    print("case many windows without an order %dx%d" % (heads, d), flush=True)
+    rng = np.random.default_rng(d)
+    nRW = 16_385
+    counts = rng.integers(0, 5, nRW)
+    counts[np.array([0, 3, 7000, 7001, nRW - 1])] = [33, 40, 64, 34, 51]
+    N, pre = _structure(rng, nRW, counts)
+    dev = lambda a: torch.as_tensor(a).cuda()
+    rwo, atox, bm = dev(pre["rowWindowOffset"]), dev(pre["sparseAToXidx"]), dev(
+        pre["tcbBitMap"].view(np.int64)).view(torch.uint64)
+    order = dev(np.argsort(-counts, kind="stable").astype(np.int32))
+    g = torch.Generator(device="cuda").manual_seed(d)
+    Q, K, V = [torch.randn((N, heads, d), generator=g, device="cuda").bfloat16() for _ in range(3)]
+    outs = []
+    for o in (None, order):
+        out = torch.full((N, heads * d), float("nan"), device="cuda")
+        outs.append(capi.attention_heads(rwo, o, atox, bm, N, Q, K, V, d ** 0.5, out=out))
+    assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+    if heads == 1:
+        assert torch.equal(capi.attention(rwo, None, atox, bm, N, *[t[:, 0].contiguous() for t in (Q, K, V)], d ** 0.5),
+                           outs[0])
+
+
+# The forms of a single head of 96 and 128: eight waves to a workgroup, and four that take the same eight runs in two
+# turns, from 500 000 blocks on or with three heads. A head's rows are the same in all of them; those of the
+# window kernel differ by the rounding of 16-bit probabilities.
+@pytest.mark.parametrize("W", [16, 8])
+@pytest.mark.parametrize("d,nRW,mean", [(96, 2900, 17), (128, 2900, 17), (96, 17_000, 30), (128, 17_000, 30)])
+def test_eight_and_four_waves_of_single_heads(monkeypatch, d, nRW, mean, W):
+    from fused3s_amd import capi
+    print("case eight and four waves W=%d d=%d windows=%d" % (W, d, nRW), flush=True)
+    rng = np.random.default_rng(d + W)
+    counts = mean * (16 // W) - 1 + rng.integers(0, 3, nRW)
+    counts[::nRW // 17] = 140 + rng.integers(0, 60)
+    assert (counts.sum() * W // 16 >= 500_000) == (nRW > 10_000)
+    rwo = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    N = 16 * nRW - 9
+    step = N // (W * int(counts.max()))
+    atox = (np.arange(rwo[-1] * W) - np.repeat(rwo[:-1] * W, counts * W)) * step + rng.integers(0, step, rwo[-1] * W)
+    bits = [rng.integers(0, 2**63, len(atox) // 4) for _ in range(2)]
+    dev = lambda a: torch.as_tensor(a).cuda()
+    args = [dev(rwo), dev(np.argsort(-counts, kind="stable").astype(np.int32)), dev(atox.astype(np.int32)),
+            dev(bits[0] & bits[1]).view(torch.uint64), N]
+    g = torch.Generator(device="cuda").manual_seed(d)
+    Q, K, V = [(torch.randn((N, 3, d), generator=g, device="cuda") * d ** -0.25).half() for _ in range(3)]
+    one = [t[:, 1].contiguous() for t in (Q, K, V)]
+    call = capi.attention if W == 16 else capi.attention_tcb8
+    got = call(*args, *one)
+    monkeypatch.setenv("F3S_SHORT_WINDOWS", "0")
+    want = call(*args, *one)
+    monkeypatch.delenv("F3S_SHORT_WINDOWS")
+    assert not torch.equal(got, want) and (got - want).abs().max().item() < MAX_ABS
+    assert ((got - want).abs().mean() / want.abs().mean()).item() < MEAN_REL[torch.float16]
+    if W == 16:
+        assert torch.equal(capi.attention_heads(*args, Q, K, V)[:, d:2 * d], got)
