@@ -2,7 +2,7 @@
 // its K / V gathers: for arrays of 4 GiB and more, and for pitched multi-head layouts whose row
 // count or pitch exceeds the 24-bit multiply of the narrow kernels. The reference indexes rows
 // with int64_t throughout (src/F3S_kernel.cu:1422-1423). Every window of such a problem is
-// computed by this kernel (no column-sliced units, no wave-per-window split): a translation unit
+// computed by this kernel (no column-sliced units, no waves for short windows): a translation unit
 // of its own, so that the common kernels do not carry a second address form.
 #include "f3s_common.h"
 #include "f3s_window_kernel.h"

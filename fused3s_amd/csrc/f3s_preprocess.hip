@@ -11,8 +11,8 @@
 //                        Larger graphs, <= 1024 edges: bitonic sort of the column ids, ballot /
 //                        popcount compaction of the distinct ones, rank by binary search.
 //   window_rank_mid_kernel, window_rank_rest_kernel
-//                        longer windows of up to 16 384 edges where the columns take several bitset
-//                        passes, one workgroup per window: sorted by bins as well.
+//                        longer windows where the columns take several bitset passes, one workgroup
+//                        per window: sorted by bins as well, above 16 384 edges by the bitset.
 //   window_rank_kernel   larger windows, one workgroup per window. Column ids are OR-ed into an
 //                        LDS bitset (a column range per pass when N exceeds the LDS range), a
 //                        wave64 popcount prefix scan turns the bitset into ranks, and every edge
@@ -1212,7 +1212,7 @@ __device__ __forceinline__ void rank_window_by_sort(
     int32_t* __restrict__ edgeToRow, int* __restrict__ error) {
   constexpr int WAVES = THREADS / 64;
   constexpr int CAP = THREADS * ITEMS;
-  constexpr int BIN_BITS = THREADS == 256 ? 11 : THREADS == 512 ? 12 : 13;
+  constexpr int BIN_BITS = THREADS == 256 ? 11 : 13;
   static_assert((1 << BIN_BITS) == 8 * THREADS, "eight bins per thread");
   static_assert(THREADS >= 256 && THREADS % 256 == 0, "the first 256 threads own one digit each");
   uint32_t* sKeys = sSort + kSortPad;  // CAP keys, room for kSortPad on each side
@@ -1317,8 +1317,8 @@ __device__ __forceinline__ void rank_window_by_sort(
   }
   // into the bins (n is hidden from the compiler between the passes: sixteen comparisons with it, kept for
   // all of them, cost more vector registers than the keys. Within a pass the lane masks of the guarded items
-  // still outnumber the scalar registers: 132 of them in the form of 512 threads and 261 in that of 1 024
-  // go to lanes of vector registers and back. None goes to memory.)
+  // still outnumber the scalar registers: 120 of them in window_rank_mid_kernel and 382 in the two forms of
+  // window_rank_rest_kernel go to lanes of vector registers and back. None goes to memory.)
   asm volatile("" : "+s"(n));
 #pragma unroll
   for (int u = 0; u < ITEMS; u++) {
@@ -1408,14 +1408,13 @@ __global__ __launch_bounds__(kMidThreads, 6) void window_rank_mid_kernel(
 // The large windows of the queue, those of more than kLargeMax edges by the bitset in several passes. One launch:
 // the handful of windows of thousands of edges would each keep a launch of its own waiting (61M edges, 414
 // windows of 1 921 to 11 001 edges: 18 + 25 + 5 us as three launches, 29 as one).
-template <int W>
 constexpr size_t rank_rest_lds(size_t bitset) {
   constexpr size_t sort = rank_sort_lds<kLargeItems, kLargeThreads>();
   return bitset > sort ? bitset : sort;
 }
 template <int W>
 __global__ __launch_bounds__(kLargeThreads) void window_rank_rest_kernel(
-    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N, int nRW,
+    const int32_t* __restrict__ rowPtr, const int32_t* __restrict__ colIdx, int N,
     int colBits, int range, int nPasses, LongQueue queue, int32_t* __restrict__ blockPartition,
     int32_t* __restrict__ edgeToColumn, int32_t* __restrict__ edgeToRow,
     int* __restrict__ error) {
@@ -3296,19 +3295,19 @@ int enqueue_rank(const int32_t* rowPtr, const int32_t* colIdx, int N, int E, cha
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
   }
-  // The longer ones, from the lists. On a graph that needs several bitset passes,
-  // windows of a few thousand edges are sorted instead of walking every pass: up to kMedMax edges
-  // with four workgroups per CU, then the few windows up to kLargeMax with one.
+  // The longer ones, from the lists. On a graph that needs several bitset passes, windows of a few thousand edges
+  // are sorted instead of walking every pass: up to kMidMax edges by 256 threads each, and those of up to kLargeMax
+  // by 1024, in one launch with the longer ones, which do walk the passes.
   if (nPasses >= 2) {
     auto rest = window_rank_rest_kernel<W>;
-    const size_t restLds = rank_rest_lds<W>(lds);
+    const size_t restLds = rank_rest_lds(lds);
     if (int rc = allow_lds(rest, restLds)) return rc;
     constexpr size_t midLds = rank_sort_lds<kMidItems, kMidThreads>();
     hipLaunchKernelGGL(window_rank_mid_kernel<W>, dim3(long_grid(nRW, E, shortMax, 8192)), dim3(kMidThreads),
                        midLds, stream, rowPtr, colIdx, N, colBits, queue, blockPartition, edgeToColumn,
                        edgeToRow, error);
     hipLaunchKernelGGL(rest, dim3(long_grid(nRW, E, kMidMax, 1024)), dim3(kLargeThreads), restLds, stream,
-                       rowPtr, colIdx, N, nRW, colBits, range, nPasses, queue, blockPartition, edgeToColumn,
+                       rowPtr, colIdx, N, colBits, range, nPasses, queue, blockPartition, edgeToColumn,
                        edgeToRow, error);
     F3S_HIP_CHECK(hipGetLastError());
     return 0;
