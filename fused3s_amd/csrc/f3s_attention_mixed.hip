@@ -23,14 +23,16 @@ constexpr int mixed_waves_per_simd(int d) { return d <= 64 ? 4 : d <= 128 ? 2 : 
 // Waves of a workgroup, four or eight. Eight compute a long window in half the time, and the longest one decides a
 // call of one or two heads on a skewed graph. A wave that has finished its own window keeps its ring until the
 // workgroup ends, which costs less with four, so those take calls of more heads and, above D = 64, of two, large
-// ones and those of less than 16 blocks of 16 columns a window. Eight -> four, us (heads x d, blocks a window): R-MAT 40 000 nodes, 12: 1 x 64 34 -> 38, 2 x 64 40 -> 43,
-// 4 x 64 57 -> 52, 8 x 64 100 -> 93, 4 x 128 106 -> 92; 169 343 nodes, 17: 1 x 64 76 -> 95; 200 000, 27: 1 x 64 111
-// -> 143, 1 x 128 241 -> 253, 8 x 64 1063 -> 1050; 600 000, 20: 1 x 64 294 -> 326, 1 x 128 648 -> 628; uniform
-// 25 000, 9: 1 x 64 25.7 -> 25.5, 8 x 64 70 -> 66; 30 000, 21: 1 x 128 45.7 -> 46.1, 8 x 64 128 -> 133. Below 16
-// blocks, d = 128: uniform 33 000, 15: one head 40.3 -> 32.9, two 66.2 -> 58.7; communities 400 000, 14: 230 -> 209;
-// R-MAT 65 000, 9: 36.9 -> 40.2; power-law 65 000, 11: 44.5 -> 52.1 (a launch for either kind of window: 33.2, 58.5, 258,
-// 50.3, 61.7). 16x8 blocks of the same graphs, power-law 65 000, 7: 38.1 -> 46.3, where a workgroup for every
-// window takes 41.4.
+// ones and those whose last round of waves would be less than half full. Eight -> four, us (heads x d, blocks a
+// window): R-MAT 40 000 nodes, 12: 1 x 64 34 -> 38, 2 x 64 40 -> 43, 4 x 64 57 -> 52, 8 x 64 100 -> 93, 4 x 128 106 -> 92;
+// 169 343 nodes, 17: 1 x 64 76 -> 95; 200 000, 27: 1 x 64 111 -> 143, 1 x 128 241 -> 253, 8 x 64 1063 -> 1050; 600 000, 20: 1 x 64
+// 294 -> 326, 1 x 128 648 -> 628; uniform 25 000, 9: 1 x 64 25.7 -> 25.5, 8 x 64 70 -> 66; 30 000, 21: 1 x 128 45.7 -> 46.1, 8 x 64
+// 128 -> 133; 33 000, 15: 2 x 128 66 -> 59; R-MAT 65 000, 14: 2 x 128 78 -> 71.
+// Rounds: at D = 96 and 128 a workgroup of eight waves fills a CU and 2 048 windows the chip. One window more, and a
+// uniform graph takes another round of which a CU or two do anything. Below 16 blocks a window, 1 x 128: uniform 33 000
+// nodes (2 063 windows), 15: 40 -> 33 (with a launch for either kind of window 33); 66 000 (4 125), 11: 0.89 of those two
+// launches -> 1.01; 46 000 (2 875), 15: 0.92 -> 1.01; 50 000 (3 125): 1.01 -> 1.01; R-MAT 33 000, 14 1.50 -> 1.32, 54 000, 11 1.47 -> 1.19;
+// power-law 66 000, 11 1.39 -> 1.19.
 // A long window is cut into as many runs of blocks whether four or eight waves compute them, so that a head's
 // rows do not depend on how many heads the call has. With two heads of 32 to a wave there are always four of
 // each, as what four waves keep of the first four runs would not fit the registers there, and so at D = 32, whose
@@ -39,7 +41,10 @@ constexpr int mixed_runs(int d, int nh) { return d == 32 || nh == 2 || d > 128 ?
 inline int mixed_waves(int d, bool w8, int nRW, int64_t nTcb16, int heads) {
   if (heads >= 3) return 4;
   if (d <= 64) return 8;
-  return heads == 2 || (!w8 && nTcb16 < 16 * (int64_t)nRW) || nTcb16 >= 500000 ? 4 : 8;
+  if (heads == 2 || nTcb16 >= 500000) return 4;
+  constexpr int kRound = 256 * 8;
+  const bool below16 = !w8 && nTcb16 < 16 * (int64_t)nRW;
+  return below16 && nRW > kRound && nRW < 3 * kRound && (nRW - 1) % kRound < kRound / 2 ? 4 : 8;
 }
 
 // How the (position, head) units of a call are dealt to the XCDs: XcdSplit with one slice and with shifts in the
